@@ -999,6 +999,8 @@ hipError_t host_err_word(int** dev) {
 
 }  // namespace
 
+hipError_t ring_cluster_host_err(int** dev) { return host_err_word(dev); }
+
 bool ring_cluster_applicable(int N, int k) { return N == 512 && k == 2; }
 
 size_t ring_cluster_workspace_bytes(int nbt) {

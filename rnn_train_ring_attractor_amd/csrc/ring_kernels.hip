@@ -998,13 +998,13 @@ __global__ __launch_bounds__(256) void ring_dw_reduce_kernel(RingDwArgs p, int N
   const int it = (int)(v % NT);
   const int mm = (int)(v / NT);
   const int q = lane >> 4, n = lane & 15;
-  const int j = 16 * NC * (jt / NC) + NC * n + (jt % NC);
+  const int j = p.linear_tiles ? 16 * jt + n : 16 * NC * (jt / NC) + NC * n + (jt % NC);
   if (j >= p.N) return;
   float* out = (mm == 0) ? p.grad_Wo : p.grad_Wa + (size_t)(mm - 1) * p.N * p.N;
   const float scale = (mm == 0) ? p.J1 : 1.f;
 #pragma unroll
   for (int e = 0; e < 4; ++e) {
-    const int i = 16 * NC * (it / NC) + NC * (4 * q + e) + (it % NC);
+    const int i = p.linear_tiles ? 16 * it + 4 * q + e : 16 * NC * (it / NC) + NC * (4 * q + e) + (it % NC);
     if (i < p.N) {
       float* o = out + (size_t)i * p.N + j;
       *o = p.accumulate ? *o + scale * s[e] : scale * s[e];
@@ -1319,6 +1319,17 @@ hipError_t ring_launch_rebuild(const RingFwdArgs& a, int NCv, hipStream_t st) {
   RING_DISPATCH_NC(NCv, RING_DISPATCH_ACT(a.act, RING_DISPATCH_RT(rt,
       e = launch_stream(ring_rebuild_saved_kernel<NC, ACT, RT>, dim3((a.nbt + RT - 1) / RT, a.T), 0, st, a))));
   return e;
+}
+
+// Team launches under their profiling slots.
+hipError_t ring_run_team_fwd(const RingFwdArgs& a, const float* Wo, const float* Wa, bool folded, int cts, void* ws, hipStream_t st,
+                             bool rebuild) {
+  ProfScope prof(rebuild ? 2 : 1, st);
+  return ring_team_fwd(a, Wo, Wa, folded, cts, ws, st);
+}
+hipError_t ring_run_team_bptt(const RingBpttArgs& a, const float* Wo, const float* Wa, bool folded, int cts, void* ws, hipStream_t st) {
+  ProfScope prof(3, st);
+  return ring_team_bptt(a, Wo, Wa, folded, cts, ws, st);
 }
 
 template <int NC, bool GA, int RT, bool WL>

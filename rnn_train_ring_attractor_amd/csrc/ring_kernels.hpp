@@ -55,6 +55,7 @@ struct RingDwArgs {
   float J1;
   int accumulate;        // non-zero: += into grad_Wo / grad_Wa (the caller zeroed them); zero: overwrite
   int N, k, T, B, nbt, nz;
+  int linear_tiles = 0;  // operand copies with tile = neuron / 16 (team kernels) instead of the common tile order
 };
 
 // matrix 0 is packed as scale0 * Wo + shift0 (see ring_pack_weights_kernel)
@@ -195,3 +196,37 @@ int ring_dw_tiled_segments(int nbt, int T, int nz);   // launches per matrix gro
 void ring_profile_set(int stride);
 bool ring_profile_on();
 hipError_t ring_profile_collect(double* ms, long long* launches);
+
+// Teams of workgroups that keep the weights on chip and exchange the state through L2 (ring_team*.hip).
+struct RingTeamArgs {
+  void* xchg;            // [slots][batch tiles][K chunks][1280 bytes], all 0xFF at launch
+  unsigned xchg_bytes;
+  int* host_err;         // word in pinned host memory, RING_CLUSTER_ERR_WAIT when a wait ran out
+  const float *Wo, *Wa;  // fp32 weights; matrix 0 is taken as scale0 * Wo + shift0
+  const float* A;
+  float* ga_part;        // dL/dA partials [member][T][k][B]
+  float scale0, shift0, J0, J1;
+  int N, k, T, B, nbt, KC, G, nteams, nt, slots, cts, transposed, spin_max;
+};
+struct RingTeamShape { int kpw, c16, mr, wk, lds_mats, grid; };
+struct RingTeamPlan {
+  bool ok;
+  RingTeamShape shape;
+  int KC, G, nteams, nt, slots;
+  size_t xchg_bytes, ga_bytes;
+  float step_cycles;     // what the cost model expects of one time step
+};
+RingTeamPlan ring_team_plan(int N, int k, int T, int B, bool bptt, bool ga);
+bool ring_uses_team(int N, int k, int T, int B);
+size_t ring_team_fwd_bytes(int N, int k, int T, int B);   // scratch of one launch (0 where teams do not apply)
+size_t ring_team_bptt_bytes(int N, int k, int T, int B);
+// J1 * Wo + J0 as one operand (folded) or kept apart; `ws` is ring_team_fwd_bytes / ring_team_bptt_bytes large
+hipError_t ring_team_fwd(const RingFwdArgs& a, const float* Wo, const float* Wa, bool folded, int cts, void* ws, hipStream_t st);
+hipError_t ring_team_bptt(const RingBpttArgs& a, const float* Wo, const float* Wa, bool folded, int cts, void* ws, hipStream_t st);
+hipError_t ring_launch_team_fwd(const RingFwdArgs& a, const RingTeamArgs& c, const RingTeamShape& sh, hipStream_t st);
+hipError_t ring_launch_team_bptt(const RingBpttArgs& a, const RingTeamArgs& c, const RingTeamShape& sh, hipStream_t st);
+hipError_t ring_launch_team_bptt_ga(const RingBpttArgs& a, const RingTeamArgs& c, const RingTeamShape& sh, hipStream_t st);
+hipError_t ring_cluster_host_err(int** dev);              // the error word both exchange families report through
+hipError_t ring_run_team_fwd(const RingFwdArgs& a, const float* Wo, const float* Wa, bool folded, int cts, void* ws, hipStream_t st,
+                             bool rebuild = false);       // the same under the profiling slots
+hipError_t ring_run_team_bptt(const RingBpttArgs& a, const float* Wo, const float* Wa, bool folded, int cts, void* ws, hipStream_t st);

@@ -1,0 +1,253 @@
+// Team kernels: choice of shape, scratch area, launch order between streams (kernels: ring_team.hpp).
+#include "ring_team.hpp"
+
+// Sum of the members' dL/dA partials in member order.
+__global__ __launch_bounds__(256) void ring_team_ga_reduce_kernel(const float* __restrict__ part, float* __restrict__ grad_A,
+                                                                  int G, int T, int k, int B) {
+  const size_t n = (size_t)T * k * B, u = (size_t)blockIdx.x * 256 + threadIdx.x;
+  if (u >= n) return;
+  float v = 0.f;
+  for (int g = 0; g < G; ++g) v += part[(size_t)g * n + u];
+  const int b = (int)(u % B);
+  const size_t tc = u / B;
+  const int ch = (int)(tc % k), t = (int)(tc / k);
+  grad_A[((size_t)b * T + t) * k + ch] = v;
+}
+
+__global__ __launch_bounds__(256) void ring_team_fill_kernel(u32x4* p, unsigned n) {
+  for (unsigned i = blockIdx.x * 256 + threadIdx.x; i < n; i += gridDim.x * 256) p[i] = u32x4{EMPTY, EMPTY, EMPTY, EMPTY};
+}
+
+#include <stdlib.h>
+#include <algorithm>
+#include <mutex>
+
+namespace {
+
+constexpr int XCDS = 8, CUS_PER_XCD = 32;
+constexpr size_t LDS_MAX = 160 * 1024;
+
+size_t up256(size_t n) { return (n + 255) & ~(size_t)255; }
+
+// One team launch at a time per device.  Two of them dispatched together could each hold compute units the other's
+// missing members need.  Launches of one stream follow each other anyway; when another stream comes along it is made
+// to wait for the last one (an event recorded there and then, so single-stream programs pay nothing).  Streams under
+// graph capture are left alone: a replayed graph is ordered by whoever launches it.
+std::mutex g_guard_mu;
+struct GuardState {
+  bool used = false;
+  hipStream_t last = nullptr;
+  hipEvent_t ev = nullptr;
+} g_guard[64];
+
+bool capturing(hipStream_t st) {
+  hipStreamCaptureStatus s = hipStreamCaptureStatusNone;
+  return hipStreamIsCapturing(st, &s) == hipSuccess && s != hipStreamCaptureStatusNone;
+}
+
+template <int C16, int WK>
+size_t plan_lds(const RingTeamShape& s, int k, int nt, int KC, bool bptt, bool ga) {
+  return lds_plan<C16, WK>(k, nt, s.lds_mats, KC, parked_bytes(s.kpw, s.c16, s.mr, s.wk), bptt, ga).total;
+}
+
+size_t shape_lds(const RingTeamShape& s, int k, int nt, int KC, bool bptt, bool ga) {
+  if (s.wk == 4) {
+    return s.c16 == 1 ? plan_lds<1, 4>(s, k, nt, KC, bptt, ga)
+                      : (s.c16 == 2 ? plan_lds<2, 4>(s, k, nt, KC, bptt, ga) : plan_lds<4, 4>(s, k, nt, KC, bptt, ga));
+  }
+  return s.c16 == 1 ? plan_lds<1, 8>(s, k, nt, KC, bptt, ga)
+                    : (s.c16 == 2 ? plan_lds<2, 8>(s, k, nt, KC, bptt, ga) : plan_lds<4, 8>(s, k, nt, KC, bptt, ga));
+}
+
+const RingTeamShape kShapes[] = {
+#define RING_TEAM_ROW(KPW, C16, MR, WK) {KPW, C16, MR, WK, 0, 0},
+    RING_TEAM_SHAPES(RING_TEAM_ROW)
+#undef RING_TEAM_ROW
+};
+
+int device_cus() {
+  int dev = 0, cus = 0;
+  if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
+    return 0;
+  return cus;
+}
+
+}  // namespace
+
+hipError_t ring_team_guard_enter(hipStream_t st) {
+  g_guard_mu.lock();
+  int dev = 0;
+  if (capturing(st) || hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return hipSuccess;
+  GuardState& g = g_guard[dev];
+  if (g.used && g.last != st && !capturing(g.last)) {
+    hipError_t e = g.ev ? hipSuccess : hipEventCreateWithFlags(&g.ev, hipEventDisableTiming);
+    if (e == hipSuccess) e = hipEventRecord(g.ev, g.last);
+    if (e == hipSuccess) e = hipStreamWaitEvent(st, g.ev, 0);
+    if (e != hipSuccess) {                 // the other stream is gone: whatever ran there is waited for
+      (void)hipGetLastError();
+      e = hipDeviceSynchronize();
+      if (e != hipSuccess) {
+        g_guard_mu.unlock();
+        return e;
+      }
+    }
+  }
+  g.used = true;
+  g.last = st;
+  return hipSuccess;
+}
+
+void ring_team_guard_leave() { g_guard_mu.unlock(); }
+
+// The shape of a team for this problem: the cheapest of the built ones by a model of one time step in cycles.
+//   products of an item  M c16 KC 16 / 4 (four matrix pipes) + reading the fragments kept in LDS + what a wave spends around them
+//   epilogue of an item  grows with the outputs per auxiliary thread
+//   one tile per team:   products + epilogue + hand-over through L2, one after the other
+//   more tiles:          products and epilogue of neighbouring items overlap
+RingTeamPlan ring_team_plan(int N, int k, int T, int B, bool bptt, bool ga) {
+  RingTeamPlan best{};
+  best.ok = false;
+  if (N < 17 || N > 1024 || k < 1 || k > 16 || T < 1 || B < 1) return best;
+  const int KC = (N + 31) / 32, nbt = (B + 15) / 16;
+  for (const RingTeamShape& s0 : kShapes) {
+    RingTeamShape s = s0;
+    if (s.wk == 4 ? KC > 4 : KC <= 4) continue;
+    if (s.kpw != (KC + s.wk - 1) / s.wk) continue;
+    s.lds_mats = std::max(0, k + 1 - s.mr);
+    const int G = (2 * KC + s.c16 - 1) / s.c16;
+    if (G > CUS_PER_XCD) continue;
+    const int nteams = std::min(nbt, XCDS * (CUS_PER_XCD / G)), nt = (nbt + nteams - 1) / nteams;
+    const int slots = nt == 1 ? 8 : (nt < 4 ? 6 : 4);
+    const size_t xbytes = (size_t)slots * nbt * KC * CHUNK_BYTES;
+    if (xbytes >= ((size_t)1 << 30)) continue;     // (offsets past the buffer say 'nowhere')
+    if (shape_lds(s, k, nt, KC, bptt, ga) > LDS_MAX) continue;
+    s.grid = XCDS * G * ((nteams + XCDS - 1) / XCDS);
+    const float npt = s.c16 == 4 ? 4.f : 2.f;
+    const float prod = 4.4f * (float)(std::max(s.mr, k + 1) * s.c16 * s.kpw * s.wk) + 4.f * (float)(s.lds_mats * s.c16 * KC) + 250.f;
+    const float epi = 350.f + 110.f * npt;
+    const float one = prod + epi + 650.f;
+    const float step = nt == 1 ? one : std::max(one, (float)nt * (std::max(prod, epi) + 60.f));
+    if (!best.ok || step < best.step_cycles) {
+      best.ok = true;
+      best.shape = s;
+      best.KC = KC;
+      best.G = G;
+      best.nteams = nteams;
+      best.nt = nt;
+      best.slots = slots;
+      best.xchg_bytes = up256(xbytes);
+      best.ga_bytes = ga ? up256((size_t)G * T * k * B * sizeof(float)) : 0;
+      best.step_cycles = step;
+    }
+  }
+  return best;
+}
+
+static bool forced() {
+  const char* v = getenv("RINGATTR_TEAM");
+  return v && v[0] == '1';
+}
+
+// whether a shape is left to the weight-resident kernels
+static bool resident_only(int N, int k, int B) { return ring_res256_applicable(N, k) && ((N == 256 && B % 16 == 0) || B > 256); }
+
+// Where teams run (us per time step, measured with T = 60, gelu; forward for inference / forward + backward):
+//   N = 120, a_dim 2:  B = 64: 2.5 -> 0.9 / 5.8 -> 2.3    B = 4096: 2.7 -> 1.9 / 9.6 -> 8.0
+//   N = 360, a_dim 2:  B = 64: 8.2 -> 1.5 / 30.6 -> 3.4   B = 1024: 12.9 -> 3.3 / 31.9 -> 7.8   B = 4096: 15.6 -> 8.0 / 37 -> 23
+//   N = 512, a_dim 2:  B = 64: 8.9 -> 1.6 / 29.1 -> 3.7   B = 2048: 14.3 -> 5.5 / 32.4 -> 14.8
+//   N = 1024, a_dim 2: B = 64: 17.8 -> 3.3 / 43 -> 6.9    B = 2048: 40 -> 19 / 104 -> 52
+// against the streaming and step-per-launch kernels.  The exceptions:
+//   * the weight-resident kernels (N = 256, a_dim 2, whole tiles) take 1.5 us per step at any batch up to 4096 rows.
+//     They keep that shape at every batch, also below 257 rows where teams are faster: a slice of a batch reproduces its
+//     rows bit for bit, and the two families sum in a different order.  On ragged shapes (128 < N < 256, or a last tile
+//     that is not full) their masked variants are slower and teams take the batches up to 256 rows.  The rule does not
+//     ask whether a record is wanted: a history is the same with and without one;
+//   * with many tiles per team (more than eight at N <= 512) a compute unit's epilogue work is what bounds a step, and
+//     the kernels that have a batch tile to themselves, or the N = 512 clusters, are as fast or faster.
+bool ring_uses_team(int N, int k, int T, int B) {
+  const char* v = getenv("RINGATTR_TEAM");
+  const bool force = v && v[0] == '1';
+  if ((v && v[0] == '0') || (!force && resident_only(N, k, B)) || ring_cluster_error()) return false;
+  // a switch that asks for one of the other families by name is obeyed
+  for (const char* name : {"RINGATTR_STREAMING", "RINGATTR_ROW_TILES", "RINGATTR_BLOCK", "RINGATTR_WIDE", "RINGATTR_SPLIT_FORWARD",
+                           "RINGATTR_LDS_WEIGHTS", "RINGATTR_BLOCK_SHAPE", "RINGATTR_CLUSTER", "RINGATTR_CLUSTER_BPTT"})
+    if (getenv(name)) return false;
+  if (device_cus() != XCDS * CUS_PER_XCD) return false;
+  const RingTeamPlan f = ring_team_plan(N, k, T, B, false, false);
+  if (!f.ok || !ring_team_plan(N, k, T, B, true, true).ok) return false;
+  return force || ring_res256_applicable(N, k) || N > 512 || f.nt <= 8;
+}
+
+// (no exchange area where no call of this shape comes here)
+size_t ring_team_fwd_bytes(int N, int k, int T, int B) {
+  if (resident_only(N, k, B) && !forced()) return 0;
+  const RingTeamPlan p = ring_team_plan(N, k, T, B, false, false);
+  return p.ok ? p.xchg_bytes : 0;
+}
+
+size_t ring_team_bptt_bytes(int N, int k, int T, int B) {
+  if (resident_only(N, k, B) && !forced()) return 0;
+  const RingTeamPlan p = ring_team_plan(N, k, T, B, true, false), g = ring_team_plan(N, k, T, B, true, true);
+  return std::max(p.ok ? p.xchg_bytes : 0, g.ok ? g.xchg_bytes + g.ga_bytes : 0);
+}
+
+static hipError_t team_args(const RingTeamPlan& p, const float* Wo, const float* Wa, const float* A, float J0, float J1,
+                            bool folded, int N, int k, int T, int B, int cts, bool transposed, void* ws, RingTeamArgs& c,
+                            hipStream_t st) {
+  hipError_t e = ring_cluster_host_err(&c.host_err);
+  if (e != hipSuccess) return e;
+  c.xchg = ws;
+  c.xchg_bytes = (unsigned)p.xchg_bytes;
+  c.Wo = Wo;
+  c.Wa = Wa;
+  c.A = A;
+  c.ga_part = reinterpret_cast<float*>(static_cast<char*>(ws) + p.xchg_bytes);
+  c.scale0 = folded ? J1 : 1.f;
+  c.shift0 = folded ? J0 : 0.f;
+  c.J0 = folded ? 0.f : J0;
+  c.J1 = folded ? 1.f : J1;
+  c.N = N;
+  c.k = k;
+  c.T = T;
+  c.B = B;
+  c.nbt = (B + 15) / 16;
+  c.KC = p.KC;
+  c.G = p.G;
+  c.nteams = p.nteams;
+  c.nt = p.nt;
+  c.slots = p.slots;
+  c.cts = cts;
+  c.transposed = transposed ? 1 : 0;
+  c.spin_max = 16000000;   // some seconds of polling
+  if (const char* v = getenv("RINGATTR_CLUSTER_SPIN")) {
+    const long s = atol(v);
+    if (s >= -1 && s <= 100000000L) c.spin_max = (int)s;
+  }
+  const unsigned n = (unsigned)(p.xchg_bytes / 16);
+  hipLaunchKernelGGL(ring_team_fill_kernel, dim3(std::min(1024u, (n + 255) / 256)), dim3(256), 0, st, reinterpret_cast<u32x4*>(ws), n);
+  return hipGetLastError();
+}
+
+hipError_t ring_team_fwd(const RingFwdArgs& a, const float* Wo, const float* Wa, bool folded, int cts, void* ws, hipStream_t st) {
+  const RingTeamPlan p = ring_team_plan(a.N, a.k, a.T, a.B, false, false);
+  if (!p.ok || !ws || (a.dfrag != nullptr) != (a.rfrag != nullptr)) return hipErrorInvalidValue;
+  RingTeamArgs c;
+  hipError_t e = team_args(p, Wo, Wa, a.A, a.J0, a.J1, folded, a.N, a.k, a.T, a.B, cts, false, ws, c, st);
+  if (e != hipSuccess) return e;
+  return ring_launch_team_fwd(a, c, p.shape, st);
+}
+
+hipError_t ring_team_bptt(const RingBpttArgs& a, const float* Wo, const float* Wa, bool folded, int cts, void* ws, hipStream_t st) {
+  const bool ga = a.grad_A != nullptr;
+  const RingTeamPlan p = ring_team_plan(a.N, a.k, a.T, a.B, true, ga);
+  if (!p.ok || !ws) return hipErrorInvalidValue;
+  RingTeamArgs c;
+  hipError_t e = team_args(p, Wo, Wa, a.A, a.J0, a.J1, folded, a.N, a.k, a.T, a.B, cts, true, ws, c, st);
+  if (e != hipSuccess) return e;
+  if (!ga) return ring_launch_team_bptt(a, c, p.shape, st);
+  e = ring_launch_team_bptt_ga(a, c, p.shape, st);
+  if (e != hipSuccess) return e;
+  const size_t n = (size_t)a.T * a.k * a.B;
+  hipLaunchKernelGGL(ring_team_ga_reduce_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, c.ga_part, a.grad_A, p.G, a.T, a.k, a.B);
+  return hipGetLastError();
+}

@@ -105,7 +105,7 @@ int hip_fail(hipError_t e, const char* what) {
 constexpr int kSavedNotes = 256;
 struct SavedNote {
   const void* ptr;
-  int family;   // 1 streaming, 2 weight-resident, 3 step-per-launch
+  int family;   // 1 streaming, 2 weight-resident, 3 step-per-launch, 4 team
   int N, k, T, B;
   float J0, J1;
   const void *Wo, *Wa;
@@ -176,7 +176,15 @@ size_t ringattr_fwd_workspace_bytes(int N, int a_dim, int seq_len, int batch_siz
   Geo g;
   if (make_geo(N, a_dim, seq_len, batch_size, g) != RINGATTR_OK) return 0;
   // (the cluster forward's exchange area is asked for wherever its shape applies, switched on or not)
-  return g.wpack_bytes + (ring_cluster_applicable(N, a_dim) ? ring_cluster_workspace_bytes(g.nbt) : 0);
+  const size_t packed = g.wpack_bytes + (ring_cluster_applicable(N, a_dim) ? ring_cluster_workspace_bytes(g.nbt) : 0);
+  const size_t team = ring_team_fwd_bytes(N, a_dim, seq_len, batch_size);   // (used instead of the packed weights)
+  return packed > team ? packed : team;
+}
+
+// The tail of a backward's workspace that the team kernels use: the exchange of the BPTT, or of the rebuild before it.
+static size_t team_area(int N, int a_dim, int seq_len, int batch_size) {
+  const size_t f = ring_team_fwd_bytes(N, a_dim, seq_len, batch_size), b = ring_team_bptt_bytes(N, a_dim, seq_len, batch_size);
+  return f > b ? f : b;
 }
 
 size_t ringattr_bwd_workspace_bytes(int N, int a_dim, int seq_len, int batch_size, int have_saved) {
@@ -186,7 +194,7 @@ size_t ringattr_bwd_workspace_bytes(int N, int a_dim, int seq_len, int batch_siz
   if (!have_saved) s += g.wpack_bytes + g.side_bytes + g.pair_bytes;
   // (the cluster BPTT's scratch area is asked for wherever its shape applies, switched on or not)
   if (ring_cluster_applicable(N, a_dim)) s += ring_cluster_bptt_workspace_bytes(g.nbt);
-  return s;
+  return s + team_area(N, a_dim, seq_len, batch_size);
 }
 
 // loss_stats != null: the forward kernel that can do so also leaves the loss head's per-row sums there; *stats_done
@@ -226,6 +234,27 @@ int ringattr_fwd_loss(const void* A, const void* Wa, float J0, float J1, const v
   return RINGATTR_OK;
 }
 
+static RingFwdArgs fwd_args(const void* A, const void* Wpack, const void* r_init, void* bump_history, void* saved, const Geo& g,
+                            float J0, float J1, float alpha, int act) {
+  RingFwdArgs a;
+  a.A = (const float*)A;
+  a.Wpack = Wpack;
+  a.r_init = (const float*)r_init;
+  a.hist = (float*)bump_history;
+  a.dfrag = saved ? (_Float16*)saved : nullptr;
+  a.rfrag = saved ? (__bf16*)((char*)saved + g.side_bytes) : nullptr;
+  a.J0 = J0;
+  a.J1 = J1;
+  a.alpha = alpha;
+  a.N = g.N;
+  a.k = g.k;
+  a.T = g.T;
+  a.B = g.B;
+  a.nbt = g.nbt;
+  a.act = act;
+  return a;
+}
+
 static int fwd_impl(const void* A, const void* Wa, float J0, float J1, const void* Wo, const void* r_init,
                     void* bump_history, float alpha, int N, int a_dim, int seq_len, int batch_size, int activation_type,
                     void* saved, void* workspace, size_t workspace_bytes, ring_f32x4* loss_stats, bool* stats_done,
@@ -249,6 +278,15 @@ static int fwd_impl(const void* A, const void* Wa, float J0, float J1, const voi
                 "invalid; this is reported once, and the streaming kernels run N = 512 from here on",
                 ce);
 
+  if (ring_uses_team(N, a_dim, seq_len, batch_size) && workspace_bytes >= ring_team_fwd_bytes(N, a_dim, seq_len, batch_size)) {
+    RingFwdArgs a = fwd_args(A, nullptr, r_init, bump_history, saved, g, J0, J1, alpha, activation_type);
+    if (saved) saved_note_put(SavedNote{saved, 4, N, a_dim, seq_len, batch_size, J0, J1, Wo, Wa});
+    if (stats_done) *stats_done = false;
+    const hipError_t e = ring_run_team_fwd(a, (const float*)Wo, (const float*)Wa, ring_res256_applicable(N, a_dim), 4 * g.NC, workspace, st);
+    if (e != hipSuccess) return hip_fail(e, "team forward launch");
+    return RINGATTR_OK;
+  }
+
   // With a saved buffer the same launch also writes the transposed copy the backward will need behind the saved
   // activations.  The weight-resident kernels take Wo as J1 * Wo + J0 in both copies; the cluster forward takes it so
   // in its own copy and leaves the plain transposed one the streaming BPTT expects.
@@ -267,22 +305,7 @@ static int fwd_impl(const void* A, const void* Wa, float J0, float J1, const voi
     saved_note_put(SavedNote{saved, ring_uses_step_kernels(N, a_dim, g.NC, g.nbt) ? 3 : (resident ? 2 : 1), N, a_dim,
                              seq_len, batch_size, J0, J1, Wo, Wa});
 
-  RingFwdArgs a;
-  a.A = (const float*)A;
-  a.Wpack = workspace;
-  a.r_init = (const float*)r_init;
-  a.hist = (float*)bump_history;
-  a.dfrag = saved ? (_Float16*)saved : nullptr;
-  a.rfrag = saved ? (__bf16*)((char*)saved + g.side_bytes) : nullptr;
-  a.J0 = J0;
-  a.J1 = J1;
-  a.alpha = alpha;
-  a.N = N;
-  a.k = a_dim;
-  a.T = seq_len;
-  a.B = batch_size;
-  a.nbt = g.nbt;
-  a.act = activation_type;
+  RingFwdArgs a = fwd_args(A, workspace, r_init, bump_history, saved, g, J0, J1, alpha, activation_type);
   a.cluster_ws = cluster ? (char*)workspace + g.wpack_bytes : nullptr;
   // the persistent forward kernels form the loss head's row sums themselves
   a.loss_stats = ring_fwd_forms_loss_sums(a, g.NC) ? loss_stats : nullptr;
@@ -360,10 +383,14 @@ static int bwd_impl(const char* who, const void* grad_output, const void* loss_w
   if ((rc = check_act(activation_type))) return rc;
   if (!A || !Wa || !Wo || !bump_history || !r_init || !grad_Wa || !grad_Wo)
     return fail(RINGATTR_ERR_INVALID, "%s: null tensor pointer", who);
-  const bool step_family = ring_uses_step_kernels(N, a_dim, g.NC, g.nbt);
+  // a record is read by the family that wrote it; without a note (or a record) the choice is the forward's
+  const SavedNote note = saved ? saved_note_get(saved) : SavedNote{};
+  const bool noted_shape = note.family != 0 && note.N == N && note.k == a_dim && note.T == seq_len && note.B == batch_size;
+  const bool team = noted_shape ? note.family == 4 : ring_uses_team(N, a_dim, seq_len, batch_size);
+  const bool step_family = !team && ring_uses_step_kernels(N, a_dim, g.NC, g.nbt);
   // the persistent streaming BPTT kernel stages the per-channel shares of dL/dA in 24 KiB of LDS; the
   // step-per-launch families form dL/dA in a pass of their own that has no such stage
-  if (grad_A && !step_family && !ring_uses_resident(N, a_dim) && (size_t)2 * a_dim * 64 * sizeof(float) > 24 * 1024)
+  if (grad_A && !team && !step_family && !ring_uses_resident(N, a_dim) && (size_t)2 * a_dim * 64 * sizeof(float) > 24 * 1024)
     return fail(RINGATTR_ERR_INVALID, "%s: grad_A on the persistent streaming kernels (N <= 512 at this batch) is "
                 "supported for a_dim <= 48 (got %d)", who, a_dim);
   if (step_family && grad_A && seq_len > 65535)
@@ -376,6 +403,9 @@ static int bwd_impl(const char* who, const void* grad_output, const void* loss_w
   if (!workspace || workspace_bytes < need)
     return fail(RINGATTR_ERR_WORKSPACE, "%s: workspace of %zu bytes needed, %zu given", who, need,
                 workspace ? workspace_bytes : (size_t)0);
+  if (team && ring_team_bptt_bytes(N, a_dim, seq_len, batch_size) == 0)
+    return fail(RINGATTR_ERR_INVALID, "%s: the saved buffer was filled by the team kernels, which RINGATTR_TEAM no longer asks for; run "
+                "forward and backward under the same setting", who);
   hipStream_t st = static_cast<hipStream_t>(stream);
 
   char* ws = (char*)workspace;
@@ -390,6 +420,7 @@ static int bwd_impl(const char* who, const void* grad_output, const void* loss_w
   float* trig = g.trig_bytes ? (float*)ws : nullptr;
   ws += g.trig_bytes;
 
+  void* const team_ws = (char*)workspace + need - team_area(N, a_dim, seq_len, batch_size);
   const _Float16* dfrag;
   const __bf16* rfrag;
   if (saved) {
@@ -402,8 +433,9 @@ static int bwd_impl(const char* who, const void* grad_output, const void* loss_w
     ws += g.side_bytes;
     __bf16* r = (__bf16*)ws;
     const bool res = ring_uses_resident(N, a_dim);
-    hipError_t e = ring_launch_pack((const float*)Wo, (const float*)Wa, wf, N, a_dim, g.NC, 0, res ? 1 : 0, res ? J1 : 1.f,
-                                    res ? J0 : 0.f, st);
+    hipError_t e = team ? hipSuccess
+                        : ring_launch_pack((const float*)Wo, (const float*)Wa, wf, N, a_dim, g.NC, 0, res ? 1 : 0, res ? J1 : 1.f,
+                                           res ? J0 : 0.f, st);
     if (e != hipSuccess) return hip_fail(e, "pack weights");
     RingFwdArgs f;
     f.A = (const float*)A;
@@ -421,7 +453,12 @@ static int bwd_impl(const char* who, const void* grad_output, const void* loss_w
     f.B = batch_size;
     f.nbt = g.nbt;
     f.act = activation_type;
-    e = ring_launch_rebuild(f, g.NC, st);
+    if (team) {   // the recurrence again, without its history stores
+      f.hist = nullptr;
+      e = ring_run_team_fwd(f, (const float*)Wo, (const float*)Wa, ring_res256_applicable(N, a_dim), 4 * g.NC, team_ws, st, true);
+    } else {
+      e = ring_launch_rebuild(f, g.NC, st);
+    }
     if (e != hipSuccess) return hip_fail(e, "rebuild launch");
     dfrag = d;
     rfrag = r;
@@ -429,20 +466,21 @@ static int bwd_impl(const char* who, const void* grad_output, const void* loss_w
 
   // The cluster BPTT (N = 512, where ring_uses_cluster_bptt says so; no dL/dA, no fused loss head) packs its own
   // transposed copy, in its column order with J1 * Wo^T + J0 as matrix 0; its scratch area is the workspace's tail.
-  const bool bptt_cluster = !step_family && !grad_A && !loss_workspace && ring_uses_cluster_bptt(N, a_dim, batch_size, seq_len) &&
+  const bool bptt_cluster = !team && !step_family && !grad_A && !loss_workspace && ring_uses_cluster_bptt(N, a_dim, batch_size, seq_len) &&
                             !ring_uses_resident(N, a_dim);
-  void* const cluster_ws = bptt_cluster ? (char*)workspace + need - ring_cluster_bptt_workspace_bytes(g.nbt) : nullptr;
+  void* const cluster_ws = bptt_cluster ? (char*)team_ws - ring_cluster_bptt_workspace_bytes(g.nbt) : nullptr;
   // the weight-resident BPTT kernel takes J1 * Wo + J0 in the transposed Wo fragments
   const bool resident = ring_uses_resident(N, a_dim);
   const bool bptt_resident = resident;
   hipError_t e = hipSuccess;
-  const int family = step_family ? 3 : (bptt_resident ? 2 : 1);
-  const SavedNote note = saved ? saved_note_get(saved) : SavedNote{};
+  const int family = team ? 4 : (step_family ? 3 : (bptt_resident ? 2 : 1));
   const int noted = note.family;
-  if (noted != 0 && (noted == 3) != (family == 3))
+  if (!team && noted != 0 && (noted == 3) != (family == 3))
     return fail(RINGATTR_ERR_INVALID, "%s: the saved buffer was filled by the other kernel family (its derivative record "
                 "has a different layout); run forward and backward under the same RINGATTR_BLOCK setting", who);
-  if (bptt_cluster) {
+  if (team) {
+    // (the team kernels read the fp32 weights)
+  } else if (bptt_cluster) {
     e = ring_launch_pack((const float*)Wo, (const float*)Wa, wb, N, a_dim, g.NC, 1,
                          ring_cluster_pack_order(N, batch_size, seq_len), J1, J0, st);
     if (e != hipSuccess) return hip_fail(e, "pack transposed weights");
@@ -485,7 +523,8 @@ static int bwd_impl(const char* who, const void* grad_output, const void* loss_w
   b.B = batch_size;
   b.nbt = g.nbt;
   b.cluster_ws = cluster_ws;
-  e = ring_launch_bptt(b, g.NC, st);
+  e = team ? ring_run_team_bptt(b, (const float*)Wo, (const float*)Wa, ring_res256_applicable(N, a_dim), 4 * g.NC, team_ws, st)
+           : ring_launch_bptt(b, g.NC, st);
   if (e != hipSuccess) return hip_fail(e, "BPTT launch");
   if (step_family && grad_A) {
     // forward-orientation fragments, packed into the split-K partial area (not yet in use, and never smaller)
@@ -511,6 +550,7 @@ static int bwd_impl(const char* who, const void* grad_output, const void* loss_w
   d.B = batch_size;
   d.nbt = g.nbt;
   d.nz = g.nz;
+  d.linear_tiles = team ? 1 : 0;
   e = ring_launch_dw(d, g.NC, st);
   if (e != hipSuccess) return hip_fail(e, "weight-gradient launch");
   return RINGATTR_OK;

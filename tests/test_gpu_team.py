@@ -1,0 +1,171 @@
+"""GPU tests of the team kernels (several workgroups of one XCD keep the weights on chip and exchange the state through
+L2): parity with the fp64 oracle over the shapes they are built in, every output of the backward, the rebuilt record,
+the fused loss head, run-to-run reproducibility (a read of state that was not complete would differ between runs), two
+streams at once, and the exit taken when a wait runs out."""
+import os
+import subprocess
+import sys
+
+import numpy as np
+import pytest
+import torch
+
+from oracle import ring_oracle as O
+from tests.ring_cases import make_problem
+
+pytestmark = pytest.mark.gpu
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+ACTS = {"relu": 0, "gelu": 1, "tanh": 2, "silu": 3}
+TRAJ_TOL = 1e-2      # bf16 operands against fp64, as in the parity tests of the other families
+GRAD_COS, GRAD_TOL = 0.999, 2e-2
+
+# B, T, k, N, act: K chunks 1 to 32 over four and eight compute waves (even and uneven splits), one to four column tiles
+# per member, one to several batch tiles per team, ragged rows and widths (N odd, 2 mod 4), one matrix to sixteen channels
+# (matrices in LDS), single step, odd and even lengths
+CASES = [
+    (9, 4, 1, 17, "tanh"), (33, 1, 2, 33, "gelu"), (20, 7, 2, 100, "silu"), (700, 4, 2, 120, "tanh"), (2300, 3, 3, 126, "gelu"),
+    (50, 6, 2, 131, "gelu"), (1, 9, 2, 256, "tanh"), (40, 5, 16, 256, "silu"), (300, 4, 9, 250, "tanh"), (600, 3, 3, 230, "gelu"),
+    (24, 6, 2, 257, "silu"), (100, 5, 3, 360, "tanh"), (1100, 3, 2, 500, "gelu"), (260, 3, 16, 512, "silu"), (30, 4, 12, 511, "tanh"),
+    (48, 5, 2, 513, "gelu"), (150, 3, 2, 768, "tanh"), (290, 3, 2, 1000, "silu"), (17, 4, 3, 1024, "gelu"),
+]
+
+
+def _t(x, dev):
+    return torch.tensor(x, device=dev)
+
+
+def _run(p, act, J0, J1, dev, saved=True, ga=True):
+    from rnn_train_ring_attractor_amd import rnn_cuda, _lib
+    A, Wa, Wo, r0, G = (_t(p[x], dev) for x in ("A", "Wa", "Wo", "r0", "G"))
+    B, T, k = p["A"].shape
+    N = p["Wo"].shape[0]
+    hist = torch.full((T, B, N), float("nan"), device=dev)
+    sv = torch.empty(rnn_cuda.saved_nbytes(N, k, T, B), dtype=torch.uint8, device=dev).fill_(0xFF) if saved else None
+    rnn_cuda.fwd_cuda.fwd(A=A, Wa=Wa, J0=J0, J1=J1, Wo=Wo, r_init=r0, bump_history=hist, alpha=0.15,
+                          activation_type=ACTS[act], saved=sv)
+    gWa, gWo, gr = torch.full_like(Wa, float("nan")), torch.full_like(Wo, float("nan")), torch.full_like(r0, float("nan"))
+    gA = torch.full_like(A, float("nan")) if ga else None
+    rnn_cuda.bwd_cuda.bwd(grad_output=G, A=A, Wa=Wa, J0=J0, J1=J1, Wo=Wo, bump_history=hist, r_init=r0, grad_Wa=gWa,
+                          grad_Wo=gWo, alpha=0.15, activation_type=ACTS[act], saved=sv, grad_r_init=gr, grad_A=gA,
+                          accumulate=False)
+    torch.cuda.synchronize()
+    names = _lib.last_kernel_names()
+    assert "ring_team_bptt" in names["bptt"] and ("ring_team_fwd" in names["fwd"] or not saved)
+    return dict(hist=hist, grad_Wa=gWa, grad_Wo=gWo, grad_r_init=gr, **({"grad_A": gA} if ga else {}))
+
+
+@pytest.fixture
+def teams(monkeypatch):
+    for v in ("RINGATTR_STREAMING", "RINGATTR_ROW_TILES", "RINGATTR_BLOCK", "RINGATTR_WIDE", "RINGATTR_SPLIT_FORWARD",
+              "RINGATTR_LDS_WEIGHTS", "RINGATTR_BLOCK_SHAPE", "RINGATTR_CLUSTER", "RINGATTR_CLUSTER_BPTT"):
+        monkeypatch.delenv(v, raising=False)
+    monkeypatch.setenv("RINGATTR_TEAM", "1")
+
+
+@pytest.mark.parametrize("B,T,k,N,act", CASES, ids=[f"b{c[0]}_t{c[1]}_k{c[2]}_n{c[3]}" for c in CASES])
+def test_team_kernels_against_the_oracle(B, T, k, N, act, gpu_device, teams):
+    print(f"[case] team B={B} T={T} k={k} N={N} {act}", flush=True)
+    J0, J1 = -1.0 / N, 0.6
+    p = make_problem(900 + N + k, B, T, k, N, action="dense")
+    if k > 3:
+        p["A"][:, :, k // 2] = 0.0         # one silent channel among the driven ones
+    got = _run(p, act, J0, J1, gpu_device)
+    again = _run(p, act, J0, J1, gpu_device)
+    assert all(torch.equal(got[x], again[x]) for x in got)
+    rebuilt = _run(p, act, J0, J1, gpu_device, saved=False)
+    plain = _run(p, act, J0, J1, gpu_device, ga=False)
+    assert all(torch.equal(got[x], rebuilt[x]) for x in got if x != "hist")     # the same recurrence, run again
+    assert all(torch.equal(got[x], plain[x]) for x in plain)
+    ref, _ = O.forward_dense(p["A"], p["Wa"], J0, J1, p["Wo"], p["r0"], 0.15, act)
+    assert O.max_rel_err(got["hist"].cpu().numpy(), ref) <= TRAJ_TOL
+    g = O.backward_dense(p["G"], p["A"], p["Wa"], J0, J1, p["Wo"], ref, p["r0"], 0.15, act)
+    for name in ("grad_Wo", "grad_Wa", "grad_r_init", "grad_A"):
+        x = got[name].cpu().numpy()
+        assert np.isfinite(x).all(), name
+        assert O.cosine(x, g[name]) >= GRAD_COS and O.max_rel_err(x, g[name]) <= GRAD_TOL, name
+
+
+@pytest.mark.parametrize("B,T,k,N", [(40, 5, 2, 120), (70, 6, 3, 361)])
+def test_fused_loss_head_on_teams(B, T, k, N, gpu_device, teams):
+    """The objective's gradient formed inside the team BPTT against the loss head's own backward through the plain one."""
+    from rnn_train_ring_attractor_amd import ring_rnn_cuda_func, ring_rnn_loss_func, ring_loss_pair
+    print(f"[case] team loss B={B} T={T} k={k} N={N}", flush=True)
+    p = make_problem(77, B, T, k, N, action="dense")
+    A, r0 = _t(p["A"], gpu_device), _t(p["r0"], gpu_device)
+    angle = torch.rand(B, T, device=gpu_device) * 6.28
+    grads = []
+    for fused in (True, False):
+        Wa, Wo = _t(p["Wa"], gpu_device).requires_grad_(True), _t(p["Wo"], gpu_device).requires_grad_(True)
+        if fused:
+            total = ring_rnn_loss_func(A, Wa, -1.0 / N, 0.6, Wo, r0, 0.15, "gelu", angle, 0.2)[0]
+        else:
+            total = ring_loss_pair(ring_rnn_cuda_func(A, Wa, -1.0 / N, 0.6, Wo, r0, 0.15, "gelu"), angle, 0.2)[0]
+        total.backward()
+        grads.append((float(total), Wa.grad.cpu().numpy(), Wo.grad.cpu().numpy()))
+    assert abs(grads[0][0] - grads[1][0]) <= 1e-5 * abs(grads[1][0])
+    # fp32 differences in the loss gradient can flip the bf16 rounding of g: one part in 2^8 of single contributions
+    assert O.max_rel_err(grads[0][1], grads[1][1]) <= 4e-3 and O.max_rel_err(grads[0][2], grads[1][2]) <= 4e-3
+
+
+def test_teams_on_two_streams(gpu_device, teams):
+    """Two launches that each want compute units of the whole device, issued on two streams: the second waits for the
+    first instead of sharing the device with it half and half, and both give the sequential result."""
+    B, T, k, N = 600, 24, 2, 512
+    print(f"[case] teams on two streams B={B} T={T} N={N}", flush=True)
+    from rnn_train_ring_attractor_amd import rnn_cuda
+    p = make_problem(78, B, T, k, N, action="dense")
+    A, Wa, Wo, r0 = (_t(p[x], gpu_device) for x in ("A", "Wa", "Wo", "r0"))
+
+    def fwd(out):
+        rnn_cuda.fwd_cuda.fwd(A=A, Wa=Wa, J0=-1.0 / N, J1=0.6, Wo=Wo, r_init=r0, bump_history=out, alpha=0.15, activation_type=2)
+
+    ref = torch.empty(T, B, N, device=gpu_device)
+    fwd(ref)
+    torch.cuda.synchronize()
+    streams = [torch.cuda.Stream(device=gpu_device) for _ in range(2)]
+    outs = [torch.full((T, B, N), float("nan"), device=gpu_device) for _ in range(6)]
+    torch.cuda.synchronize()
+    for i, o in enumerate(outs):
+        with torch.cuda.stream(streams[i % 2]):
+            fwd(o)
+    torch.cuda.synchronize()
+    assert all(torch.equal(o, ref) for o in outs)
+    fwd(ref)                       # (a wait that had run out would be reported by this call)
+
+
+_GIVE_UP_SCRIPT = r"""
+import os, sys
+sys.path.insert(0, {root!r})
+os.environ["RINGATTR_TEAM"] = "1"
+os.environ["RINGATTR_CLUSTER_SPIN"] = "-1"      # every wave gives up its waits at once
+import torch
+from tests.ring_cases import make_problem
+from rnn_train_ring_attractor_amd import rnn_cuda, _lib
+dev = torch.device("cuda:0")
+p = make_problem(315, 64, 6, 2, 360, action="dense")
+A, Wa, Wo, r0 = (torch.tensor(p[k], device=dev) for k in ("A", "Wa", "Wo", "r0"))
+def fwd():
+    hist = torch.full((6, 64, 360), float("nan"), device=dev)
+    rnn_cuda.fwd_cuda.fwd(A=A, Wa=Wa, J0=-0.01, J1=0.5, Wo=Wo, r_init=r0, bump_history=hist, alpha=0.15, activation_type=2)
+    torch.cuda.synchronize()
+    return hist
+print("[case] team forward whose waves give up", flush=True)
+fwd()                                             # the launch goes through its steps without waiting and ends
+assert "team" in _lib.last_kernel_names()["fwd"]
+try:
+    fwd()
+    sys.exit(1)
+except Exception as e:                            # reported once, by the next call
+    assert "gave up waiting" in str(e), str(e)
+h = fwd()                                         # from here on the other kernels do the work
+assert "team" not in _lib.last_kernel_names()["fwd"] and torch.isfinite(h).all()
+print("give-up path ok")
+"""
+
+
+def test_a_wait_that_runs_out_is_reported_once_and_the_other_kernels_take_over(gpu_device):
+    proc = subprocess.run([sys.executable, "-c", _GIVE_UP_SCRIPT.format(root=ROOT)], capture_output=True, text=True, timeout=300,
+                          cwd=ROOT)
+    print(proc.stdout[-1500:], proc.stderr[-1500:], flush=True)
+    assert proc.returncode == 0 and "give-up path ok" in proc.stdout
