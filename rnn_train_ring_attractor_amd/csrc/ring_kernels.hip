@@ -20,8 +20,8 @@
 //   column n of tile c for neuron 64*w + 32*(c/2) + 2*n + c%2: the pipelined weight-resident forward's order.
 //   split_k = 2 (NC = 8 only): the same column order (neuron 128*w + 32*(c/2) + 2*n + c%2) with the contraction in
 //   neuron order: the cluster forward's (four waves).
-//   split_k = 3 (NC = 8 only): tile c of wave group w holds the 16 consecutive neurons 128*w + 16*c + n, contraction
-//   in neuron order: the eight-wave cluster forward's.
+//   split_k = 3: tile c of wave group w holds the 16 consecutive neurons 16*(NC*w + c) + n, contraction in neuron
+//   order: the eight-wave cluster forward's (NC = 8) and the panel kernels' (NC >= 16).
 // ------------------------------------------------------------------------------------------------
 __device__ __forceinline__ bf16x8 pack_fragment(const float* __restrict__ Wo, const float* __restrict__ Wa, size_t u,
                                                 int N, int NC, int transposed, int split_k, float scale0, float shift0) {
@@ -41,7 +41,7 @@ __device__ __forceinline__ bf16x8 pack_fragment(const float* __restrict__ Wo, co
   const int k0 = 32 * kc + 8 * q;
   const float* W = (mm == 0) ? Wo : Wa + (size_t)(mm - 1) * N * N;
   bf16x8 pk;
-  if (!transposed && !split_k && (N & 3) == 0 && col < N && k0 + 8 <= N) {
+  if (!transposed && (split_k == 0 || split_k == 3) && (N & 3) == 0 && col < N && k0 + 8 <= N) {
     // forward orientation away from the padding: the fragment's eight values lie side by side in one row
     const f32x4* src = reinterpret_cast<const f32x4*>(W + (size_t)col * N + k0);
     const f32x4 a = src[0], b = src[1];
@@ -1146,7 +1146,7 @@ hipError_t ring_profile_collect(double* ms, long long* launches) {
 hipError_t ring_launch_pack2(const float* Wo, const float* Wa, int N, int k, int NC, void* out, int transposed,
                              int split_k, float scale0, float shift0, void* out2, int transposed2, int split_k2,
                              float scale2, float shift2, hipStream_t st) {
-  auto order_ok = [&](int sk) { return sk == 0 || (sk == 1 && NC == 4) || ((sk == 2 || sk == 3) && NC == 8); };
+  auto order_ok = [&](int sk) { return sk == 0 || (sk == 1 && NC == 4) || (sk == 2 && NC == 8) || (sk == 3 && NC >= 8); };
   if (!order_ok(split_k) || (out2 && !order_ok(split_k2))) return hipErrorInvalidValue;
   const size_t total = (size_t)(1 + k) * 4 * NC * 2 * NC * 64 * (out2 ? 2 : 1);
   const int blocks = (int)((total + 255) / 256 < 4096 ? (total + 255) / 256 : 4096);
@@ -1253,6 +1253,7 @@ hipError_t ring_launch_fwd(const RingFwdArgs& a, int NCv, hipStream_t st) {
   // the kernels write the derivative record and the operand copy together: both or neither
   if ((a.dfrag != nullptr) != (a.rfrag != nullptr)) return hipErrorInvalidValue;
   ProfScope prof(1, st);
+  if (a.panel_ws) return ring_launch_panel_fwd(a, NCv, st);   // (the caller's choice: ring_uses_panel)
   if (ring_uses_step_kernels(a.N, a.k, NCv, a.nbt))
     return step_prefers_wide(NCv, a.nbt, a.k) ? ring_launch_wide_fwd(a, NCv, false, 4, st) : ring_launch_block_fwd(a, NCv, false, st);
   if (a.cluster_ws) return ring_launch_fwd_cluster(a, st);   // (the caller's choice: ring_uses_cluster)

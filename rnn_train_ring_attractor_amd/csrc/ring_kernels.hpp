@@ -20,6 +20,9 @@ struct RingFwdArgs {
   // Non-null: run the four-compute-unit cluster kernel (ring_cluster.hip) with this scratch area of
   // ring_cluster_workspace_bytes(nbt) bytes; Wpack is then in that kernel's column order with J1 * Wo + J0 as matrix 0.
   void* cluster_ws = nullptr;
+  // Non-null: run the panel kernels (ring_panel.hip) with this scratch area of ring_panel_workspace_bytes; Wpack is then
+  // in their column order (3).
+  void* panel_ws = nullptr;
 };
 
 struct RingBpttArgs {
@@ -116,6 +119,12 @@ hipError_t ring_launch_trig_table(float* out, int N, int NPAD, hipStream_t st);
 hipError_t ring_launch_block_grad_A(const RingBpttArgs& a, const void* Wf, int NC, hipStream_t st);
 // which kernel family runs a problem with a saved record: 0 persistent, 1 step-per-launch (wide or block)
 bool ring_uses_step_kernels(int N, int k, int NC, int nbt);
+
+// Step-per-launch forward without a saved record, wide rings (ring_panel.hip).
+bool ring_panel_applicable(int NC, int k);
+bool ring_uses_panel(int N, int k, int NC, int nbt);
+size_t ring_panel_workspace_bytes(int NC, int nbt);
+hipError_t ring_launch_panel_fwd(const RingFwdArgs& a, int NC, hipStream_t st);
 
 // LDS-tiled weight-gradient contraction for NC in {4, 8, 16, 24, 32} (ring_dw.hip).
 bool ring_dw_tiled_applicable(int NC);

@@ -1,0 +1,371 @@
+// One launch per time step for wide rings, forward without a saved record ("panel" kernels).
+//
+// What bounds a step here is how often the weights travel from the caches into the compute units: at N = 2048 with 16
+// channels they are 143 MB, far more than the L2s hold, and ring_block.hip pulls every fragment into eight compute
+// units (32 rows x 64 neurons each): 1.1 GB per step at B = 256.  A workgroup here takes a panel of up to 128 rows x 16
+// neurons and ALL (1 + a_dim) matrices of it at once: a fragment is fetched by B / 128 workgroups and feeds eight MFMAs,
+// and the operand rows, which no longer fit LDS as a whole, stream through it in stages of four K chunks.
+//   * A (matrix, column tile) pair is a virtual column; the four waves share out a workgroup's virtual columns in
+//     contiguous runs of at most five.  A wave holds the products of its run with every row tile (up to 160
+//     accumulators), so weight fragments go straight from global memory to the one wave that needs them (eight chunks
+//     ahead), and operand fragments are read from LDS once per wave.
+//   * Per K chunk a workgroup with R row tiles and V virtual columns loads (R + V) KiB for R * V MFMAs: 8 + 17 KiB
+//     against 544 matrix-pipe cycles at B = 256 and 16 channels.  What is left is the rate at which a compute unit takes
+//     in lines that miss its L2; see panel_shape.
+//   * The operand arrives as bf16 MFMA fragments: a small launch before each step converts the state and takes its
+//     row sums (in ring_block.hip's order), 5 us at B = 256.
+// us per step, before (ring_block.hip / ring_bign.hip) -> here, T = 20 with the packing launch:
+//   N = 2048, 16 channels: B = 1: 120 -> 39   B = 256: 102 -> 64 (the step kernel itself 97 -> 57)   B = 1024: 286 -> 189
+//   N = 2048,  2 channels: B = 16: 31 -> 13   B = 256:  35 -> 22                                     B = 1024:  73 -> 47
+//   N = 1100,  2 channels: B = 16: 22 -> 12   B = 200:  29 -> 18     N = 1500, 6 channels, B = 64: 49 -> 16
+// Products, gates and activation are the arithmetic of ring_block.hip in the same order (a product's contraction is
+// never split), so the two families agree bit for bit: tests/test_gpu_panel.py.
+#include "ring_step_common.hpp"
+
+namespace {
+
+constexpr int PANEL_NV = 5;        // virtual columns per wave
+constexpr int PANEL_S = 4;         // K chunks per LDS stage; weights are fetched two stages ahead
+
+// What a pass over the contraction works on.  (All of it the same in every lane.)
+struct PanelPass {
+  __amdgpu_buffer_rsrc_t x, w;        // operand fragments, packed weights
+  unsigned wat[PANEL_NV];             // byte offset of the wave's virtual columns, chunk 0
+  int mat[PANEL_NV], col[PANEL_NV];   // their matrix and column tile
+  const float* gl;       // gates [16 R][k]
+  float J1;
+  int KCH, k, nv, wv;
+};
+
+// A fragment per lane from a scalar byte offset.  (Buffer loads: every address but the lane's own 16 bytes is scalar, which
+// leaves the registers to the fragments in flight.)
+__device__ __forceinline__ bf16x8 panel_load(__amdgpu_buffer_rsrc_t r, unsigned at, int lane) {
+  return __builtin_bit_cast(bf16x8, __builtin_amdgcn_raw_buffer_load_b128(r, lane * 16, (int)at, 0));
+}
+
+// The products X_i @ W_v of a wave's NV virtual columns with all row tiles, then gates and the sum over the matrices in
+// their order, one wave after the other, into sums [C][R][64].
+template <int R, int NV>
+__device__ __forceinline__ void panel_pass(const PanelPass& p, const unsigned (&xrow)[R], bf16x8* xs, f32x4* sums, int lane) {
+  const int KCH = p.KCH, nst = KCH / PANEL_S, wv = p.wv;
+  auto stage = [&](int buf, int i, int d) { return xs + ((buf * R + i) * PANEL_S + d) * 64 + lane; };
+  f32x4 acc[NV][R];
+#pragma unroll
+  for (int v = 0; v < NV; ++v)
+#pragma unroll
+    for (int i = 0; i < R; ++i) {
+      acc[v][i] = f32x4{0.f, 0.f, 0.f, 0.f};
+      asm volatile("" : "+a"(acc[v][i]));                 // products live in the accumulation-register half
+    }
+  bf16x8 x0[R], xr[R], wf[2 * PANEL_S][NV], xa[2][R];
+  // wave d carries chunk d of every row tile of a stage into LDS.  (The second stage's loads go out before the weights',
+  // as in the loop: its wait at the top of the loop then leaves the weights in flight on both ways in.)
+#pragma unroll
+  for (int i = 0; i < R; ++i) x0[i] = panel_load(p.x, xrow[i] + wv * 1024, lane);
+#pragma unroll
+  for (int i = 0; i < R; ++i) xr[i] = panel_load(p.x, xrow[i] + (PANEL_S + wv) * 1024, lane);
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int d = 0; d < 2 * PANEL_S; ++d)
+#pragma unroll
+    for (int v = 0; v < NV; ++v) wf[d][v] = panel_load(p.w, p.wat[v] + d * 1024, lane);
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int i = 0; i < R; ++i) {
+    *stage(0, i, wv) = x0[i];
+    asm volatile("" : "+v"(xr[i]));      // (used here, or the compiler moves the loads behind the weights')
+  }
+  lds_barrier();
+#pragma unroll
+  for (int i = 0; i < R; ++i) xa[0][i] = *stage(0, i, 0);
+#pragma unroll 1
+  for (int s0 = 0; s0 < nst; s0 += 2)                     // (the number of stages is a multiple of four)
+#pragma unroll
+    for (int cur = 0; cur < 2; ++cur) {
+      const int s = s0 + cur, nxt = cur ^ 1;
+      // (the barrier of the stage before: nobody reads that buffer any more)
+#pragma unroll
+      for (int i = 0; i < R; ++i) *stage(nxt, i, wv) = xr[i];
+      const int sx = s + 2 < nst ? s + 2 : nst - 1;       // past the end: a re-read, unused
+#pragma unroll
+      for (int i = 0; i < R; ++i) xr[i] = panel_load(p.x, xrow[i] + (PANEL_S * sx + wv) * 1024, lane);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int d = 0; d < PANEL_S; ++d) {
+        if (d + 1 < PANEL_S) {
+#pragma unroll
+          for (int i = 0; i < R; ++i) xa[(d + 1) & 1][i] = *stage(cur, i, d + 1);
+        } else {
+          lds_barrier();                                  // the next stage is in LDS; all reads of this one have landed
+#pragma unroll
+          for (int i = 0; i < R; ++i) xa[(d + 1) & 1][i] = *stage(nxt, i, 0);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        bf16x8(&w)[NV] = wf[PANEL_S * cur + d];
+#pragma unroll
+        for (int v = 0; v < NV; ++v)
+#pragma unroll
+          for (int i = 0; i < R; ++i) acc[v][i] = mfma16(xa[d & 1][i], w[v], acc[v][i]);
+        const int kp = PANEL_S * (s + 2) + d < KCH ? PANEL_S * (s + 2) + d : KCH - 1;
+#pragma unroll
+        for (int v = 0; v < NV; ++v) w[v] = panel_load(p.w, p.wat[v] + kp * 1024, lane);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+#pragma unroll 1
+  for (int r = 0; r < 4; ++r) {
+    if (wv == r && p.nv > 0) {
+#pragma unroll
+      for (int v = 0; v < NV; ++v) {
+        const int m = p.mat[v];
+#pragma unroll
+        for (int i = 0; i < R; ++i) {
+          f32x4* dst = sums + (p.col[v] * R + i) * 64 + lane;
+          f32x4 s = *dst;
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            const float g = p.gl[(16 * i + 4 * (lane >> 4) + e) * p.k + (m > 0 ? m - 1 : 0)];
+            s[e] = fmaf(m > 0 ? g : p.J1, acc[v][i][e], s[e]);
+          }
+          *dst = s;
+        }
+      }
+    }
+    lds_barrier();
+  }
+}
+
+}  // namespace
+
+// Operand fragments [batch tile][K chunk][lane][8] and fp32 row sums of one step's rows; four rows per wave.  The sums
+// run in the order of ring_block.hip's stage_tiles.
+__global__ __launch_bounds__(64) void ring_panel_operand_kernel(const float* __restrict__ prev, bf16x8* __restrict__ xfrag,
+                                                                float* __restrict__ rs, int N, int B, int NPAD) {
+  const int lane = threadIdx.x, row = 4 * (blockIdx.x & 3) + (lane >> 4), sub = lane & 15, bt = blockIdx.x >> 2;
+  char* base = reinterpret_cast<char*>(xfrag + (size_t)bt * (NPAD >> 5) * 64);
+  float sum = 0.f;
+  auto put = [&](int j, f32x4 v) {
+    sum += (v[0] + v[1]) + (v[2] + v[3]);
+    const bf16x4 pk = {(__bf16)v[0], (__bf16)v[1], (__bf16)v[2], (__bf16)v[3]};
+    *reinterpret_cast<bf16x4*>(base + (size_t)((j >> 5) * 64 + ((j >> 3) & 3) * 16 + row) * 16 + (j & 7) * 2) = pk;
+  };
+  const int b = 16 * bt + row;
+  const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+  if ((N & 3) == 0) {
+    // sixteen loads in flight (addresses clamped into the row): one at a time this launch is all latency, 12.7 us
+    const float* src = prev + (size_t)(b < B ? b : B - 1) * N;
+    for (int j0 = 4 * sub; j0 < NPAD; j0 += 16 * 64) {      // (NPAD is a multiple of 512; what lies past it is skipped)
+      f32x4 v[16];
+#pragma unroll
+      for (int i = 0; i < 16; ++i) v[i] = *reinterpret_cast<const f32x4*>(src + (j0 + 64 * i < N ? j0 + 64 * i : 0));
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        const int j = j0 + 64 * i;
+        if (j < NPAD) put(j, b < B && j < N ? v[i] : zero);
+      }
+    }
+  } else {
+    for (int j = 4 * sub; j < NPAD; j += 64) put(j, load4_masked(prev, N, B, b, j));
+  }
+  sum = row16_sum_dpp(sum);
+  if (sub == 0) rs[16 * bt + row] = sum;
+}
+
+// One step for R row tiles x C column tiles (16 consecutive neurons each).  Wpack: order 3 of ring_pack_weights_kernel.
+template <int ACT, int R>
+__global__ __launch_bounds__(256) void ring_panel_fwd_kernel(RingFwdArgs p, const bf16x8* __restrict__ xfrag,
+                                                             const float* __restrict__ rs, int NC, int C, int t, int xcd_map) {
+  extern __shared__ __attribute__((aligned(16))) char panel_lds[];
+  __shared__ int list[BN_GATE_KMAX + 1];
+  const int tid = threadIdx.x, wv = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+  const int N = p.N, B = p.B, T = p.T, k = p.k, KCH = 2 * NC;
+  bf16x8* const xs = reinterpret_cast<bf16x8*>(panel_lds);                                  // [2][R][PANEL_S][64]
+  f32x4* const sums = reinterpret_cast<f32x4*>(xs + (size_t)2 * R * PANEL_S * 64);          // [C][R][64]
+  float* const gl = reinterpret_cast<float*>(sums + (size_t)C * R * 64);                    // [16 R][k]
+  int rg, cb;
+  step_block_coords(xcd_map, rg, cb);
+  const int bt0 = rg * R;
+
+  for (int idx = tid; idx < R * 16 * k; idx += 256) {
+    const int row = idx / k, c = idx - row * k, b = 16 * bt0 + row;
+    gl[idx] = b < B ? p.A[((size_t)b * T + t) * k + c] : 0.f;
+  }
+  for (int i = tid; i < C * R * 64; i += 256) sums[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+  lds_barrier();
+  // matrices worth multiplying: Wo, and the channels that are not zero in all of the workgroup's rows
+  int nact = 1;
+  {
+    unsigned long long m = 0;
+    for (int c0 = 0; c0 < k; c0 += 4) {
+      const int c = c0 + (lane >> 4);
+      bool nz = false;
+#pragma unroll
+      for (int i = 0; i < R; ++i) nz |= c < k && gl[(16 * i + (lane & 15)) * k + (c < k ? c : 0)] != 0.f;
+      const unsigned long long bal = __ballot(nz);
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        if ((bal >> (16 * j)) & 0xffffull) m |= 1ull << (c0 + j);
+    }
+    if (tid == 0) list[0] = 0;
+    for (int c = 0; c < k; ++c)
+      if ((m >> c) & 1ull) {
+        if (tid == 0) list[nact] = c + 1;
+        ++nact;
+      }
+  }
+  nact = __builtin_amdgcn_readfirstlane(nact);
+  lds_barrier();
+
+  unsigned xrow[R];
+#pragma unroll
+  for (int i = 0; i < R; ++i) xrow[i] = (unsigned)(bt0 + i < p.nbt ? bt0 + i : p.nbt - 1) * (unsigned)KCH * 1024u;   // (past the end: a re-read)
+  PanelPass ps;
+  ps.x = __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16x8*>(xfrag), 0, (int)((unsigned)p.nbt * (unsigned)KCH * 1024u), 0x00020000);
+  ps.w = __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p.Wpack), 0, (int)((unsigned)(k + 1) * 4u * NC * KCH * 1024u), 0x00020000);
+  ps.gl = gl;
+  ps.J1 = p.J1;
+  ps.KCH = KCH;
+  ps.k = k;
+  ps.wv = wv;
+  const int per_pass = (4 * PANEL_NV) / C;                // matrices per pass over the contraction
+  for (int m0 = 0; m0 < nact; m0 += per_pass) {
+    const int nm = nact - m0 < per_pass ? nact - m0 : per_pass, V = nm * C;
+    const int v0 = wv * V / 4;
+    ps.nv = (wv + 1) * V / 4 - v0;                        // this wave's run; matrices ascending
+#pragma unroll
+    for (int v = 0; v < PANEL_NV; ++v) {
+      const int u = v < ps.nv ? v0 + v : (ps.nv > 0 ? v0 : 0);
+      ps.mat[v] = __builtin_amdgcn_readfirstlane(list[m0 + u / C]);
+      ps.col[v] = u % C;
+      ps.wat[v] = ((unsigned)ps.mat[v] * 4u * NC + (unsigned)(cb * C + ps.col[v])) * (unsigned)KCH * 1024u;
+    }
+    // (every variant passes the same number of barriers; a wave without a column of its own helps with the staging)
+    switch (ps.nv) {
+      case 5: panel_pass<R, 5>(ps, xrow, xs, sums, lane); break;
+      case 4: panel_pass<R, 4>(ps, xrow, xs, sums, lane); break;
+      case 3: panel_pass<R, 3>(ps, xrow, xs, sums, lane); break;
+      case 2: panel_pass<R, 2>(ps, xrow, xs, sums, lane); break;
+      default: panel_pass<R, 1>(ps, xrow, xs, sums, lane); break;
+    }
+  }
+
+  // activation and leak; a thread takes four consecutive neurons of a row
+  const float* prev = (t == 0) ? p.r_init : p.hist + (size_t)(t - 1) * B * N;
+  float* out = p.hist + (size_t)t * B * N;
+  const float oma = 1.f - p.alpha;
+  const float* sf = reinterpret_cast<const float*>(sums);
+  for (int idx = tid; idx < R * 16 * 4 * C; idx += 256) {
+    const int row = idx / (4 * C), j4 = 4 * (idx % (4 * C)), cc = j4 >> 4, n = j4 & 15;
+    const int b = 16 * bt0 + row, j = 16 * C * cb + j4, i = row >> 4;
+    if (b >= B || j >= N) continue;
+    const f32x4 rp = load4_masked(prev, N, B, b, j);
+    const float js = p.J0 * rs[b];
+    f32x4 rn;
+#pragma unroll
+    for (int x = 0; x < 4; ++x) {
+      const float s = sf[((size_t)(cc * R + i) * 64 + ((row & 15) >> 2) * 16 + n + x) * 4 + (row & 3)];
+      float F, D;
+      act_fast<ACT>(s + js, F, D);
+      rn[x] = fmaf(p.alpha, F, oma * rp[x]);
+    }
+    store4_masked(out, N, B, b, j, rn);
+  }
+}
+
+// ------------------------------------------------------------------------------------------------
+// Launchers
+// ------------------------------------------------------------------------------------------------
+static size_t panel_lds_bytes(int R, int C, int k) {
+  return (size_t)2 * R * PANEL_S * 1024 + (size_t)C * R * 1024 + (size_t)R * 16 * k * sizeof(float);
+}
+
+// Row tiles and column tiles of a workgroup.  Per K chunk a workgroup needs the longer of its matrix-pipe time
+// (16 cycles an MFMA, the fullest wave's share) and its loads: a compute unit takes in some 16 bytes per cycle from the
+// memory side of its L2, whatever is in flight (measured: 18 KiB a chunk on 128 compute units and 25 KiB on 256 both run
+// at 15 to 17).  Workgroups beyond one per compute unit queue.  us per step, N = 2048, by (row tiles, column tiles):
+//   16 channels, B = 256:  (8,1) 64  (4,1) 71  (4,2) 66  (8,2) 98      B = 1:  (1,1) 39  (4,1) 45  (8,1) 57
+//   16 channels, B = 1024: (8,1) 208 (8,2) 195 (8,4) 189               2 channels, B = 256:  (4,2) 22  (8,1) 27  (8,4) 43
+static void panel_shape(int NC, int nbt, int k, int* R_out, int* C_out) {
+  float best = 0.f;
+  for (int R = 1; R <= 8; R *= 2)
+    for (int C = 1; C <= 4; C *= 2) {
+      const int V = (k + 1) * C;
+      if (R > 1 && R / 2 >= nbt) continue;
+      if (panel_lds_bytes(R, C, k) > 150 * 1024) continue;
+      const int passes = (V + 4 * PANEL_NV - 1) / (4 * PANEL_NV), Vp = (V + passes - 1) / passes;
+      const long wgs = (long)((nbt + R - 1) / R) * (4 * NC / C), rounds = (wgs + 255) / 256;
+      const float mfma = 16.f * (float)(((Vp + 3) / 4) * R), load = 1024.f * (float)(R + Vp) / 16.f;
+      const float cost = (float)(rounds * passes) * (mfma > load ? mfma : load);
+      if (best == 0.f || cost <= best) {      // (a tie goes to the wider panel: fewer workgroups fetch the same rows)
+        best = cost;
+        *R_out = R;
+        *C_out = C;
+      }
+    }
+}
+
+bool ring_panel_applicable(int NC, int k) { return NC >= 16 && NC % 8 == 0 && k <= BN_GATE_KMAX; }
+
+size_t ring_panel_workspace_bytes(int NC, int nbt) { return (size_t)nbt * 2 * NC * 1024 + (size_t)nbt * 16 * sizeof(float); }
+
+// RINGATTR_PANEL=0: never; a switch that asks for one of the other step-per-launch families is obeyed.
+bool ring_uses_panel(int N, int k, int NC, int nbt) {
+  if (!ring_panel_applicable(NC, k)) return false;
+  const char* v = getenv("RINGATTR_PANEL");
+  if (v && v[0] == '0') return false;
+  for (const char* name : {"RINGATTR_WIDE", "RINGATTR_BLOCK", "RINGATTR_BLOCK_SHAPE"})
+    if (getenv(name)) return false;
+  (void)N;
+  return ring_panel_workspace_bytes(NC, nbt) < ((size_t)1 << 30);   // (32-bit offsets; the weights are 0.6 GB at most)
+}
+
+template <int ACT, int R>
+static hipError_t panel_run(const RingFwdArgs& a, int NC, int C, hipStream_t st) {
+  const size_t dyn = panel_lds_bytes(R, C, a.k);
+  hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&ring_panel_fwd_kernel<ACT, R>),
+                                     hipFuncAttributeMaxDynamicSharedMemorySize, (int)dyn);
+  if (e != hipSuccess) return e;
+  bf16x8* xfrag = reinterpret_cast<bf16x8*>(a.panel_ws);
+  float* rs = reinterpret_cast<float*>(xfrag + (size_t)a.nbt * 2 * NC * 64);
+  const dim3 grid((a.nbt + R - 1) / R, 4 * NC / C);
+  const int xm = step_xcd_map();
+  for (int t = 0; t < a.T; ++t) {
+    const float* prev = t == 0 ? a.r_init : a.hist + (size_t)(t - 1) * a.B * a.N;
+    RING_LAUNCH(ring_panel_operand_kernel, dim3(4 * a.nbt), dim3(64), 0, st, prev, xfrag, rs, a.N, a.B, 64 * NC);
+    RING_LAUNCH((ring_panel_fwd_kernel<ACT, R>), grid, dim3(256), dyn, st, a, xfrag, rs, NC, C, t, xm);
+    e = hipGetLastError();
+    if (e != hipSuccess) return e;
+  }
+  return hipSuccess;
+}
+
+template <int ACT>
+static hipError_t panel_act(const RingFwdArgs& a, int NC, hipStream_t st) {
+  int R = 1, C = 1;
+  panel_shape(NC, a.nbt, a.k, &R, &C);
+  if (const char* v = getenv("RINGATTR_PANEL_SHAPE")) {   // <R><C>, e.g. 81 (cross-checks)
+    const int r = v[0] - '0', c = v[0] ? v[1] - '0' : 0;
+    if ((r == 1 || r == 2 || r == 4 || r == 8) && (c == 1 || c == 2 || c == 4) && panel_lds_bytes(r, c, a.k) <= 150 * 1024) {
+      R = r;
+      C = c;
+    }
+  }
+  switch (R) {
+    case 8: return panel_run<ACT, 8>(a, NC, C, st);
+    case 4: return panel_run<ACT, 4>(a, NC, C, st);
+    case 2: return panel_run<ACT, 2>(a, NC, C, st);
+    default: return panel_run<ACT, 1>(a, NC, C, st);
+  }
+}
+
+// a.panel_ws: ring_panel_workspace_bytes; a.Wpack in order 3 of ring_pack_weights_kernel
+hipError_t ring_launch_panel_fwd(const RingFwdArgs& a, int NC, hipStream_t st) {
+  if (!ring_panel_applicable(NC, a.k) || !a.panel_ws || !a.hist || a.dfrag || a.rfrag) return hipErrorInvalidValue;
+  switch (a.act) {
+    case ACT_RELU: return panel_act<ACT_RELU>(a, NC, st);
+    case ACT_GELU: return panel_act<ACT_GELU>(a, NC, st);
+    case ACT_TANH: return panel_act<ACT_TANH>(a, NC, st);
+    case ACT_SILU: return panel_act<ACT_SILU>(a, NC, st);
+    default: return hipErrorInvalidValue;
+  }
+}

@@ -176,7 +176,8 @@ size_t ringattr_fwd_workspace_bytes(int N, int a_dim, int seq_len, int batch_siz
   Geo g;
   if (make_geo(N, a_dim, seq_len, batch_size, g) != RINGATTR_OK) return 0;
   // (the cluster forward's exchange area is asked for wherever its shape applies, switched on or not)
-  const size_t packed = g.wpack_bytes + (ring_cluster_applicable(N, a_dim) ? ring_cluster_workspace_bytes(g.nbt) : 0);
+  const size_t packed = g.wpack_bytes + (ring_cluster_applicable(N, a_dim) ? ring_cluster_workspace_bytes(g.nbt) : 0) +
+                        (ring_panel_applicable(g.NC, a_dim) ? align_up(ring_panel_workspace_bytes(g.NC, g.nbt)) : 0);
   const size_t team = ring_team_fwd_bytes(N, a_dim, seq_len, batch_size);   // (used instead of the packed weights)
   return packed > team ? packed : team;
 }
@@ -294,11 +295,13 @@ static int fwd_impl(const void* A, const void* Wa, float J0, float J1, const voi
   const size_t cluster_bytes = ring_cluster_applicable(N, a_dim) ? ring_cluster_workspace_bytes(g.nbt) : 0;
   const bool cluster = !resident && ring_uses_cluster(N, a_dim, batch_size, seq_len) && !ring_uses_step_kernels(N, a_dim, g.NC, g.nbt) &&
                        workspace_bytes >= g.wpack_bytes + cluster_bytes;
+  const bool panel = !saved && ring_uses_step_kernels(N, a_dim, g.NC, g.nbt) && ring_uses_panel(N, a_dim, g.NC, g.nbt) &&
+                     workspace_bytes >= g.wpack_bytes + ring_panel_workspace_bytes(g.NC, g.nbt);
   void* wpack_t = saved ? (char*)saved + g.side_bytes + g.pair_bytes : nullptr;
   const float s0 = (resident || cluster) ? J1 : 1.f, h0 = (resident || cluster) ? J0 : 0.f;
   const float s2 = resident ? J1 : 1.f, h2 = resident ? J0 : 0.f;
   hipError_t e = ring_launch_pack2((const float*)Wo, (const float*)Wa, N, a_dim, g.NC, workspace, 0,
-                                   cluster ? ring_cluster_pack_order(N, batch_size, seq_len) : resident,
+                                   cluster ? ring_cluster_pack_order(N, batch_size, seq_len) : (panel ? 3 : resident),
                                    s0, h0, wpack_t, 1, 0, s2, h2, st);
   if (e != hipSuccess) return hip_fail(e, "pack weights");
   if (saved)
@@ -307,6 +310,7 @@ static int fwd_impl(const void* A, const void* Wa, float J0, float J1, const voi
 
   RingFwdArgs a = fwd_args(A, workspace, r_init, bump_history, saved, g, J0, J1, alpha, activation_type);
   a.cluster_ws = cluster ? (char*)workspace + g.wpack_bytes : nullptr;
+  a.panel_ws = panel ? (char*)workspace + g.wpack_bytes : nullptr;
   // the persistent forward kernels form the loss head's row sums themselves
   a.loss_stats = ring_fwd_forms_loss_sums(a, g.NC) ? loss_stats : nullptr;
   if (stats_done) *stats_done = a.loss_stats != nullptr;
