@@ -155,7 +155,7 @@ static bool resident_only(int N, int k, int B) { return ring_res256_applicable(N
 //   N = 120, a_dim 2:  B = 64: 2.5 -> 0.9 / 5.8 -> 2.3    B = 4096: 2.7 -> 1.9 / 9.6 -> 8.0
 //   N = 360, a_dim 2:  B = 64: 8.2 -> 1.5 / 30.6 -> 3.4   B = 1024: 12.9 -> 3.3 / 31.9 -> 7.8   B = 4096: 15.6 -> 8.0 / 37 -> 23
 //   N = 512, a_dim 2:  B = 64: 8.9 -> 1.6 / 29.1 -> 3.7   B = 2048: 14.3 -> 5.5 / 32.4 -> 14.8
-//   N = 1024, a_dim 2: B = 64: 17.8 -> 3.3 / 43 -> 6.9    B = 2048: 40 -> 19 / 104 -> 52
+//   N = 1024, a_dim 2: B = 64: 17.8 -> 3.3 / 43 -> 6.9    B = 2048: 40 -> 19 / 104 -> 50
 // against the streaming and step-per-launch kernels.  The exceptions:
 //   * the weight-resident kernels (N = 256, a_dim 2, whole tiles) take 1.5 us per step at any batch up to 4096 rows.
 //     They keep that shape at every batch, also below 257 rows where teams are faster: a slice of a batch reproduces its
