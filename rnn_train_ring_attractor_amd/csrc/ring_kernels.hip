@@ -1146,7 +1146,7 @@ hipError_t ring_profile_collect(double* ms, long long* launches) {
 hipError_t ring_launch_pack2(const float* Wo, const float* Wa, int N, int k, int NC, void* out, int transposed,
                              int split_k, float scale0, float shift0, void* out2, int transposed2, int split_k2,
                              float scale2, float shift2, hipStream_t st) {
-  auto order_ok = [&](int sk) { return sk == 0 || (sk == 1 && NC == 4) || (sk == 2 && NC == 8) || (sk == 3 && NC >= 8); };
+  auto order_ok = [&](int sk) { return sk == 0 || (sk == 1 && NC == 4) || (sk == 2 && NC == 8) || sk == 3; };
   if (!order_ok(split_k) || (out2 && !order_ok(split_k2))) return hipErrorInvalidValue;
   const size_t total = (size_t)(1 + k) * 4 * NC * 2 * NC * 64 * (out2 ? 2 : 1);
   const int blocks = (int)((total + 255) / 256 < 4096 ? (total + 255) / 256 : 4096);
@@ -1323,10 +1323,13 @@ hipError_t ring_launch_rebuild(const RingFwdArgs& a, int NCv, hipStream_t st) {
 }
 
 // Team launches under their profiling slots.
-hipError_t ring_run_team_fwd(const RingFwdArgs& a, const float* Wo, const float* Wa, bool folded, int cts, void* ws, hipStream_t st,
-                             bool rebuild) {
-  ProfScope prof(rebuild ? 2 : 1, st);
+hipError_t ring_run_team_fwd(const RingFwdArgs& a, const float* Wo, const float* Wa, bool folded, int cts, void* ws, hipStream_t st) {
+  ProfScope prof(1, st);
   return ring_team_fwd(a, Wo, Wa, folded, cts, ws, st);
+}
+hipError_t ring_run_team_rebuild(const RingFwdArgs& a, bool folded, int cts, hipStream_t st) {
+  ProfScope prof(2, st);
+  return ring_team_rebuild(a, folded, cts, st);
 }
 hipError_t ring_run_team_bptt(const RingBpttArgs& a, const float* Wo, const float* Wa, bool folded, int cts, void* ws, hipStream_t st) {
   ProfScope prof(3, st);

@@ -232,10 +232,14 @@ size_t ring_team_bptt_bytes(int N, int k, int T, int B);
 // J1 * Wo + J0 as one operand (folded) or kept apart; `ws` is ring_team_fwd_bytes / ring_team_bptt_bytes large
 hipError_t ring_team_fwd(const RingFwdArgs& a, const float* Wo, const float* Wa, bool folded, int cts, void* ws, hipStream_t st);
 hipError_t ring_team_bptt(const RingBpttArgs& a, const float* Wo, const float* Wa, bool folded, int cts, void* ws, hipStream_t st);
+// the record from a.hist; a.Wpack: forward fragments in order 3, with J1 * Wo + J0 as matrix 0 when folded
+hipError_t ring_team_rebuild(const RingFwdArgs& a, bool folded, int cts, hipStream_t st);
+hipError_t ring_launch_team_rebuild(const RingFwdArgs& a, const RingTeamArgs& c, int wk, hipStream_t st);
 hipError_t ring_launch_team_fwd(const RingFwdArgs& a, const RingTeamArgs& c, const RingTeamShape& sh, hipStream_t st);
 hipError_t ring_launch_team_bptt(const RingBpttArgs& a, const RingTeamArgs& c, const RingTeamShape& sh, hipStream_t st);
 hipError_t ring_launch_team_bptt_ga(const RingBpttArgs& a, const RingTeamArgs& c, const RingTeamShape& sh, hipStream_t st);
 hipError_t ring_cluster_host_err(int** dev);              // the error word both exchange families report through
-hipError_t ring_run_team_fwd(const RingFwdArgs& a, const float* Wo, const float* Wa, bool folded, int cts, void* ws, hipStream_t st,
-                             bool rebuild = false);       // the same under the profiling slots
+// the same under the profiling slots
+hipError_t ring_run_team_fwd(const RingFwdArgs& a, const float* Wo, const float* Wa, bool folded, int cts, void* ws, hipStream_t st);
+hipError_t ring_run_team_rebuild(const RingFwdArgs& a, bool folded, int cts, hipStream_t st);
 hipError_t ring_run_team_bptt(const RingBpttArgs& a, const float* Wo, const float* Wa, bool folded, int cts, void* ws, hipStream_t st);

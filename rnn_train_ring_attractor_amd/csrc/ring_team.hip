@@ -237,6 +237,19 @@ hipError_t ring_team_fwd(const RingFwdArgs& a, const float* Wo, const float* Wa,
   return ring_launch_team_fwd(a, c, p.shape, st);
 }
 
+hipError_t ring_team_rebuild(const RingFwdArgs& a, bool folded, int cts, hipStream_t st) {
+  const RingTeamPlan p = ring_team_plan(a.N, a.k, a.T, a.B, false, false);
+  if (!p.ok) return hipErrorInvalidValue;
+  RingTeamArgs c = {};
+  c.A = a.A;
+  c.J0 = folded ? 0.f : a.J0;
+  c.J1 = folded ? 1.f : a.J1;
+  c.k = a.k;
+  c.KC = p.KC;
+  c.cts = cts;
+  return ring_launch_team_rebuild(a, c, p.shape.wk, st);
+}
+
 hipError_t ring_team_bptt(const RingBpttArgs& a, const float* Wo, const float* Wa, bool folded, int cts, void* ws, hipStream_t st) {
   const bool ga = a.grad_A != nullptr;
   const RingTeamPlan p = ring_team_plan(a.N, a.k, a.T, a.B, true, ga);

@@ -28,7 +28,8 @@
 // an auxiliary wave waits for the loads of an item within three items of issuing them, vector-memory operations
 // complete in order, and three items are fewer than slots - 3 rounds (8 slots with one tile per team, 6 with two or
 // three, 4 from four tiles up).
-// Besides the bf16 state a chunk carries fp32 row sums of the unrounded state (groups of eight neurons) for the J0 term.
+// Besides the bf16 state a chunk carries fp32 row sums of the unrounded state (groups of eight neurons, always summed in
+// the order of row_sum8, so that a row's bits do not depend on how wide the members are) for the J0 term.
 //
 // Placement: workgroups go to XCDs round robin by workgroup index, members of a team are 8 indices apart; every
 // workgroup has a compute unit of its own (the grid never exceeds the device).  Every wait is bounded: a wave whose wait
@@ -70,7 +71,10 @@ __device__ __forceinline__ float dpp_ror(float x) {
   return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), CTRL, 0xF, 0xF, false));
 }
 
-// Sum over the four lanes of a 16-lane row that differ in lane bits 2-3.
+// Sum of eight neurons from the sums of their four pairs.
+__device__ __forceinline__ float row_sum8(float s0, float s1, float s2, float s3) { return (s0 + s3) + (s2 + s1); }
+
+// Sum over the four lanes of a 16-lane row that differ in lane bits 2-3; in the first of them the order of row_sum8.
 __device__ __forceinline__ float sum_bits23(float v) {
   v += dpp_ror<0x124>(v);   // row_ror:4
   v += dpp_ror<0x128>(v);   // row_ror:8
@@ -468,9 +472,10 @@ struct TeamAux {
     tile_ok = map.active && ct < 2 * c.KC;
     const unsigned kc = (unsigned)j0 >> 5;
     x_off = kc * CHUNK_BYTES + ((((unsigned)j0 >> 3) & 3) * 16 + map.b) * 16 + (j0 & 7) * 2;
-    rs_off = kc * CHUNK_BYTES + 1024 + map.b * 16 + (NPT == 4 ? (ct & 1) * 8 : (((unsigned)j0 >> 3) & 3) * 4);
+    rs_off = kc * CHUNK_BYTES + 1024 + map.b * 16 + (((unsigned)j0 >> 3) & 3) * 4;
     if (!tile_ok) x_off = NOWHERE;
-    if (!tile_ok || ((lane >> 2) & 3) != 0) rs_off = NOWHERE;      // one lane of the four that share a row writes its sum
+    // one lane of those that share a row's eight neurons (four lanes of two, or two of four) writes their sum
+    if (!tile_ok || ((lane >> 2) & (NPT == 4 ? 1 : 3)) != 0) rs_off = NOWHERE;
     row_off = tile_ok && j0 < c.N ? (unsigned)(map.b * c.N + j0) * 4 : NOWHERE;
     d_off = tile_ok ? (unsigned)(ct * 256 + (map.q * 16 + map.b) * 4 + 2 * map.p) * 2 : NOWHERE;
     // one 16-byte slot per neuron and row quad (see pair_offset; tile = neuron / 16): after the quad transpose a lane has
@@ -485,11 +490,10 @@ struct TeamAux {
   __device__ __forceinline__ void put(__amdgpu_buffer_rsrc_t rsrc, unsigned base, const unsigned (&x)[NPT / 2], unsigned r) {
     if constexpr (NPT == 4) {
       __builtin_amdgcn_raw_buffer_store_b64(u32x2{x[0], x[1]}, rsrc, (int)x_off, (int)base, ST);
-      __builtin_amdgcn_raw_buffer_store_b64(u32x2{r, r == EMPTY ? EMPTY : 0u}, rsrc, (int)rs_off, (int)base, ST);
     } else {
       __builtin_amdgcn_raw_buffer_store_b32(x[0], rsrc, (int)x_off, (int)base, ST);
-      __builtin_amdgcn_raw_buffer_store_b32(r, rsrc, (int)rs_off, (int)base, ST);
     }
+    __builtin_amdgcn_raw_buffer_store_b32(r, rsrc, (int)rs_off, (int)base, ST);
   }
   // publish the thread's NPT values of a tile's state in `slot`
   __device__ __forceinline__ void publish(const RingTeamArgs& c, __amdgpu_buffer_rsrc_t rsrc, int slot, int bt, const float (&v)[NPT]) {
@@ -497,8 +501,14 @@ struct TeamAux {
 #pragma unroll
     for (int i = 0; i < NPT / 2; ++i) x[i] = not_empty(pack_bf16(v[2 * i], v[2 * i + 1]));
     float s = v[0] + v[1];
-    if constexpr (NPT == 4) s += v[2] + v[3];
-    if (c.J0 != 0.f) s = sum_bits23(s);
+    if (c.J0 != 0.f) {
+      if constexpr (NPT == 4) {
+        const float u = v[2] + v[3];
+        s = row_sum8(s, u, dpp_ror<0x12C>(s), dpp_ror<0x12C>(u));    // (row_ror:12: the next four neurons' lane)
+      } else {
+        s = sum_bits23(s);
+      }
+    }
     const unsigned r = not_empty(__builtin_bit_cast(unsigned, s));
     const unsigned base = (unsigned)slot * slot_bytes + (unsigned)bt * tile_bytes;
     put<ST_LOCAL>(rsrc, base, x, r);
@@ -558,10 +568,10 @@ struct TeamAux {
 #pragma unroll
     for (int i = 0; i < NPT; ++i) v[i] = (16 * bt + map.b < B && map.active && j0 + i < N) ? v[i] : 0.f;
   }
-  // into row block bt of an fp32 [B][N] slab (null: nowhere)
+  // into row block bt of an fp32 [B][N] slab
   __device__ __forceinline__ void row_store(float* slab, int N, int B, int bt, const float (&v)[NPT]) const {
     const int rows = B - 16 * bt < 16 ? B - 16 * bt : 16;
-    const __amdgpu_buffer_rsrc_t r = team_buffer(slab + (size_t)16 * bt * N, slab ? (size_t)rows * N * 4 : 0);
+    const __amdgpu_buffer_rsrc_t r = team_buffer(slab + (size_t)16 * bt * N, (size_t)rows * N * 4);
     if (N % NPT == 0) {
       if constexpr (NPT == 4)
         __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, f32x4{v[0], v[1], v[2], v[3]}), r, (int)row_off, 0, 0);

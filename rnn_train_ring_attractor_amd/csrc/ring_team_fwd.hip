@@ -2,7 +2,7 @@
 #include "ring_team.hpp"
 
 // ------------------------------------------------------------------------------------------------
-// Forward.  p.hist may be null (rebuild of the record), p.dfrag / p.rfrag null together (inference).
+// Forward.  p.dfrag / p.rfrag may be null together (inference).
 // ------------------------------------------------------------------------------------------------
 template <int KPW, int C16, int MR, int WK, bool EX, int ACT>
 __global__ __launch_bounds__(64 * (WK + AUX)) void ring_team_fwd_kernel(RingFwdArgs p, RingTeamArgs c) {
@@ -78,7 +78,7 @@ __global__ __launch_bounds__(64 * (WK + AUX)) void ring_team_fwd_kernel(RingFwdA
       for (int i = 0; i < NPT; ++i) state[(size_t)j * C16 * 256 + i] = rn[i];
     }
     aux.refill(c, rsrc, slot == 0 ? c.slots - 1 : slot - 1, bt);
-    aux.row_store(p.hist ? p.hist + (size_t)t * B * N : nullptr, N, B, bt, rn);
+    aux.row_store(p.hist + (size_t)t * B * N, N, B, bt, rn);
     aux.dact_store(p.dfrag, t, nbt, bt, c.cts, aD);
     if (save && (t & 1) == 0) {        // this step's operand and the next one's are both in hand: one 16-byte slot
       unsigned lo[NPT / 2], hi[NPT / 2];

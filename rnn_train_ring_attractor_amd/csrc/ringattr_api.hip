@@ -182,11 +182,8 @@ size_t ringattr_fwd_workspace_bytes(int N, int a_dim, int seq_len, int batch_siz
   return packed > team ? packed : team;
 }
 
-// The tail of a backward's workspace that the team kernels use: the exchange of the BPTT, or of the rebuild before it.
-static size_t team_area(int N, int a_dim, int seq_len, int batch_size) {
-  const size_t f = ring_team_fwd_bytes(N, a_dim, seq_len, batch_size), b = ring_team_bptt_bytes(N, a_dim, seq_len, batch_size);
-  return f > b ? f : b;
-}
+// The tail of a backward's workspace that the team BPTT uses.
+static size_t team_area(int N, int a_dim, int seq_len, int batch_size) { return ring_team_bptt_bytes(N, a_dim, seq_len, batch_size); }
 
 size_t ringattr_bwd_workspace_bytes(int N, int a_dim, int seq_len, int batch_size, int have_saved) {
   Geo g;
@@ -436,10 +433,9 @@ static int bwd_impl(const char* who, const void* grad_output, const void* loss_w
     _Float16* d = (_Float16*)ws;
     ws += g.side_bytes;
     __bf16* r = (__bf16*)ws;
-    const bool res = ring_uses_resident(N, a_dim);
-    hipError_t e = team ? hipSuccess
-                        : ring_launch_pack((const float*)Wo, (const float*)Wa, wf, N, a_dim, g.NC, 0, res ? 1 : 0, res ? J1 : 1.f,
-                                           res ? J0 : 0.f, st);
+    const bool res = team ? ring_res256_applicable(N, a_dim) : ring_uses_resident(N, a_dim);
+    hipError_t e = ring_launch_pack((const float*)Wo, (const float*)Wa, wf, N, a_dim, g.NC, 0, team ? 3 : (res ? 1 : 0), res ? J1 : 1.f,
+                                    res ? J0 : 0.f, st);
     if (e != hipSuccess) return hip_fail(e, "pack weights");
     RingFwdArgs f;
     f.A = (const float*)A;
@@ -457,12 +453,7 @@ static int bwd_impl(const char* who, const void* grad_output, const void* loss_w
     f.B = batch_size;
     f.nbt = g.nbt;
     f.act = activation_type;
-    if (team) {   // the recurrence again, without its history stores
-      f.hist = nullptr;
-      e = ring_run_team_fwd(f, (const float*)Wo, (const float*)Wa, ring_res256_applicable(N, a_dim), 4 * g.NC, team_ws, st, true);
-    } else {
-      e = ring_launch_rebuild(f, g.NC, st);
-    }
+    e = team ? ring_run_team_rebuild(f, res, 4 * g.NC, st) : ring_launch_rebuild(f, g.NC, st);
     if (e != hipSuccess) return hip_fail(e, "rebuild launch");
     dfrag = d;
     rfrag = r;

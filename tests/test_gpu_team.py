@@ -86,6 +86,35 @@ def test_team_kernels_against_the_oracle(B, T, k, N, act, gpu_device, teams):
         assert O.cosine(x, g[name]) >= GRAD_COS and O.max_rel_err(x, g[name]) <= GRAD_TOL, name
 
 
+# two and four items per workgroup of the rebuild, odd and even lengths, ragged rows and widths, channels that are silent
+@pytest.mark.parametrize("B,T,k,N,act", [(9, 1, 1, 17, "gelu"), (700, 48, 2, 120, "tanh"), (530, 65, 3, 131, "silu"),
+                                         (100, 9, 3, 360, "gelu"), (1030, 32, 16, 250, "tanh"), (40, 6, 2, 1000, "silu")])
+def test_backward_without_a_record_differentiates_the_history_it_is_given(B, T, k, N, act, gpu_device, teams):
+    """The reference's boundary hands the backward a history and no record; the record follows from that history whoever
+    made it, so every gradient is the given trajectory's."""
+    from rnn_train_ring_attractor_amd import rnn_cuda, _lib
+    print(f"[case] team rebuild B={B} T={T} k={k} N={N} {act}", flush=True)
+    J0, J1 = -1.0 / N, 0.6
+    p = make_problem(500 + N + k, B, T, k, N, action="dense")
+    if k > 3:
+        p["A"][:, :, 2:] = 0.0
+    hist, _ = O.forward_dense(p["A"], p["Wa"], J0, J1, p["Wo"], p["r0"], 0.15, act)
+    rng = np.random.default_rng(B + T)
+    hist = (hist * (1.0 + 0.3 * rng.standard_normal(hist.shape)) + 0.02 * rng.standard_normal(hist.shape)).astype(np.float32)
+    A, Wa, Wo, r0, G, H = (_t(x, gpu_device) for x in (p["A"], p["Wa"], p["Wo"], p["r0"], p["G"], hist))
+    got = {n: torch.full_like(x, float("nan")) for n, x in (("grad_Wa", Wa), ("grad_Wo", Wo), ("grad_r_init", r0), ("grad_A", A))}
+    rnn_cuda.bwd_cuda.bwd(grad_output=G, A=A, Wa=Wa, J0=J0, J1=J1, Wo=Wo, bump_history=H, r_init=r0, alpha=0.15,
+                          activation_type=ACTS[act], accumulate=False, **got)
+    torch.cuda.synchronize()
+    want = O.backward_dense(p["G"], p["A"], p["Wa"], J0, J1, p["Wo"], hist.astype(np.float64), p["r0"], 0.15, act)
+    for name, x in got.items():
+        x = x.cpu().numpy()
+        assert np.isfinite(x).all(), name
+        assert O.cosine(x, want[name]) >= GRAD_COS and O.max_rel_err(x, want[name]) <= GRAD_TOL, name
+    names = _lib.last_kernel_names()
+    assert "ring_team_rebuild" in names["rebuild_saved"] and "ring_team_bptt" in names["bptt"], names
+
+
 @pytest.mark.parametrize("B,T,k,N", [(40, 5, 2, 120), (70, 6, 3, 361)])
 def test_fused_loss_head_on_teams(B, T, k, N, gpu_device, teams):
     """The objective's gradient formed inside the team BPTT against the loss head's own backward through the plain one."""
