@@ -210,19 +210,22 @@ hipError_t ring_profile_collect(double* ms, long long* launches);
 struct RingTeamArgs {
   void* xchg;            // [slots][batch tiles][K chunks][1280 bytes], all 0xFF at launch
   unsigned xchg_bytes;
+  unsigned long long* gather;   // a word per team, 0 at launch: members that are resident, a byte per XCD; top bit: given up
   int* host_err;         // word in pinned host memory, RING_CLUSTER_ERR_WAIT when a wait ran out
   const float *Wo, *Wa;  // fp32 weights; matrix 0 is taken as scale0 * Wo + shift0
   const float* A;
   float* ga_part;        // dL/dA partials [member][T][k][B]
   float scale0, shift0, J0, J1;
   int N, k, T, B, nbt, KC, G, nteams, nt, slots, cts, transposed, spin_max;
+  int gather_ticks;      // how long the members of a team wait for each other, in 10 ns (negative: not at all)
+  int c16, mr, wk;       // the shape, for the single workgroups that take over
 };
 struct RingTeamShape { int kpw, c16, mr, wk, lds_mats, grid; };
 struct RingTeamPlan {
   bool ok;
   RingTeamShape shape;
   int KC, G, nteams, nt, slots;
-  size_t xchg_bytes, ga_bytes;
+  size_t xchg_bytes, gather_bytes, ga_bytes;
   float step_cycles;     // what the cost model expects of one time step
 };
 RingTeamPlan ring_team_plan(int N, int k, int T, int B, bool bptt, bool ga);
@@ -238,6 +241,9 @@ hipError_t ring_launch_team_rebuild(const RingFwdArgs& a, const RingTeamArgs& c,
 hipError_t ring_launch_team_fwd(const RingFwdArgs& a, const RingTeamArgs& c, const RingTeamShape& sh, hipStream_t st);
 hipError_t ring_launch_team_bptt(const RingBpttArgs& a, const RingTeamArgs& c, const RingTeamShape& sh, hipStream_t st);
 hipError_t ring_launch_team_bptt_ga(const RingBpttArgs& a, const RingTeamArgs& c, const RingTeamShape& sh, hipStream_t st);
+// the teams that did not gather, a workgroup per batch tile (ring_team_solo.hip)
+hipError_t ring_launch_team_solo_fwd(const RingFwdArgs& a, const RingTeamArgs& c, hipStream_t st);
+hipError_t ring_launch_team_solo_bptt(const RingBpttArgs& a, const RingTeamArgs& c, hipStream_t st);
 hipError_t ring_cluster_host_err(int** dev);              // the error word both exchange families report through
 // the same under the profiling slots
 hipError_t ring_run_team_fwd(const RingFwdArgs& a, const float* Wo, const float* Wa, bool folded, int cts, void* ws, hipStream_t st);

@@ -14,8 +14,12 @@ __global__ __launch_bounds__(256) void ring_team_ga_reduce_kernel(const float* _
   grad_A[((size_t)b * T + t) * k + ch] = v;
 }
 
-__global__ __launch_bounds__(256) void ring_team_fill_kernel(u32x4* p, unsigned n) {
-  for (unsigned i = blockIdx.x * 256 + threadIdx.x; i < n; i += gridDim.x * 256) p[i] = u32x4{EMPTY, EMPTY, EMPTY, EMPTY};
+// The exchange area empty, the teams' words behind it zero.
+__global__ __launch_bounds__(256) void ring_team_fill_kernel(u32x4* p, unsigned nx, unsigned n) {
+  for (unsigned i = blockIdx.x * 256 + threadIdx.x; i < n; i += gridDim.x * 256) {
+    const unsigned v = i < nx ? EMPTY : 0u;
+    p[i] = u32x4{v, v, v, v};
+  }
 }
 
 #include <stdlib.h>
@@ -136,6 +140,7 @@ RingTeamPlan ring_team_plan(int N, int k, int T, int B, bool bptt, bool ga) {
       best.nt = nt;
       best.slots = slots;
       best.xchg_bytes = up256(xbytes);
+      best.gather_bytes = up256((size_t)nteams * sizeof(unsigned long long));
       best.ga_bytes = ga ? up256((size_t)G * T * k * B * sizeof(float)) : 0;
       best.step_cycles = step;
     }
@@ -182,13 +187,13 @@ bool ring_uses_team(int N, int k, int T, int B) {
 size_t ring_team_fwd_bytes(int N, int k, int T, int B) {
   if (resident_only(N, k, B) && !forced()) return 0;
   const RingTeamPlan p = ring_team_plan(N, k, T, B, false, false);
-  return p.ok ? p.xchg_bytes : 0;
+  return p.ok ? p.xchg_bytes + p.gather_bytes : 0;
 }
 
 size_t ring_team_bptt_bytes(int N, int k, int T, int B) {
   if (resident_only(N, k, B) && !forced()) return 0;
   const RingTeamPlan p = ring_team_plan(N, k, T, B, true, false), g = ring_team_plan(N, k, T, B, true, true);
-  return std::max(p.ok ? p.xchg_bytes : 0, g.ok ? g.xchg_bytes + g.ga_bytes : 0);
+  return std::max(p.ok ? p.xchg_bytes + p.gather_bytes : 0, g.ok ? g.xchg_bytes + g.gather_bytes + g.ga_bytes : 0);
 }
 
 static hipError_t team_args(const RingTeamPlan& p, const float* Wo, const float* Wa, const float* A, float J0, float J1,
@@ -201,7 +206,8 @@ static hipError_t team_args(const RingTeamPlan& p, const float* Wo, const float*
   c.Wo = Wo;
   c.Wa = Wa;
   c.A = A;
-  c.ga_part = reinterpret_cast<float*>(static_cast<char*>(ws) + p.xchg_bytes);
+  c.gather = reinterpret_cast<unsigned long long*>(static_cast<char*>(ws) + p.xchg_bytes);
+  c.ga_part = reinterpret_cast<float*>(static_cast<char*>(ws) + p.xchg_bytes + p.gather_bytes);
   c.scale0 = folded ? J1 : 1.f;
   c.shift0 = folded ? J0 : 0.f;
   c.J0 = folded ? 0.f : J0;
@@ -223,8 +229,17 @@ static hipError_t team_args(const RingTeamPlan& p, const float* Wo, const float*
     const long s = atol(v);
     if (s >= -1 && s <= 100000000L) c.spin_max = (int)s;
   }
-  const unsigned n = (unsigned)(p.xchg_bytes / 16);
-  hipLaunchKernelGGL(ring_team_fill_kernel, dim3(std::min(1024u, (n + 255) / 256)), dim3(256), 0, st, reinterpret_cast<u32x4*>(ws), n);
+  // A team whose compute units are busy waits about as long as the way round it takes (some 50 ms at N = 1024, T = 120).
+  c.gather_ticks = 5000000;
+  if (const char* v = getenv("RINGATTR_TEAM_GATHER_US")) {
+    const long us = atol(v);
+    if (us >= -1 && us <= 10000000L) c.gather_ticks = us < 0 ? -1 : (int)us * 100;
+  }
+  c.c16 = p.shape.c16;
+  c.mr = p.shape.mr;
+  c.wk = p.shape.wk;
+  const unsigned nx = (unsigned)(p.xchg_bytes / 16), n = (unsigned)((p.xchg_bytes + p.gather_bytes) / 16);
+  hipLaunchKernelGGL(ring_team_fill_kernel, dim3(std::min(1024u, (n + 255) / 256)), dim3(256), 0, st, reinterpret_cast<u32x4*>(ws), nx, n);
   return hipGetLastError();
 }
 
@@ -234,7 +249,8 @@ hipError_t ring_team_fwd(const RingFwdArgs& a, const float* Wo, const float* Wa,
   RingTeamArgs c;
   hipError_t e = team_args(p, Wo, Wa, a.A, a.J0, a.J1, folded, a.N, a.k, a.T, a.B, cts, false, ws, c, st);
   if (e != hipSuccess) return e;
-  return ring_launch_team_fwd(a, c, p.shape, st);
+  e = ring_launch_team_fwd(a, c, p.shape, st);
+  return e == hipSuccess ? ring_launch_team_solo_fwd(a, c, st) : e;
 }
 
 hipError_t ring_team_rebuild(const RingFwdArgs& a, bool folded, int cts, hipStream_t st) {
@@ -257,9 +273,9 @@ hipError_t ring_team_bptt(const RingBpttArgs& a, const float* Wo, const float* W
   RingTeamArgs c;
   hipError_t e = team_args(p, Wo, Wa, a.A, a.J0, a.J1, folded, a.N, a.k, a.T, a.B, cts, true, ws, c, st);
   if (e != hipSuccess) return e;
-  if (!ga) return ring_launch_team_bptt(a, c, p.shape, st);
-  e = ring_launch_team_bptt_ga(a, c, p.shape, st);
-  if (e != hipSuccess) return e;
+  e = ga ? ring_launch_team_bptt_ga(a, c, p.shape, st) : ring_launch_team_bptt(a, c, p.shape, st);
+  if (e == hipSuccess) e = ring_launch_team_solo_bptt(a, c, st);
+  if (e != hipSuccess || !ga) return e;
   const size_t n = (size_t)a.T * a.k * a.B;
   hipLaunchKernelGGL(ring_team_ga_reduce_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, c.ga_part, a.grad_A, p.G, a.T, a.k, a.B);
   return hipGetLastError();

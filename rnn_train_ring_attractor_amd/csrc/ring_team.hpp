@@ -32,9 +32,16 @@
 // the order of row_sum8, so that a row's bits do not depend on how wide the members are) for the J0 term.
 //
 // Placement: workgroups go to XCDs round robin by workgroup index, members of a team are 8 indices apart; every
-// workgroup has a compute unit of its own (the grid never exceeds the device).  Every wait is bounded: a wave whose wait
-// runs out leaves a word in host memory, waits for nothing from then on and goes through the remaining steps on whatever
-// it finds, so the launch ends by itself; the library reports the word on its next call.
+// workgroup has a compute unit of its own (the grid never exceeds the device).  That the members of a team are resident
+// together and share an XCD is checked, not assumed: other work may hold compute units (another stream's or process's
+// team launch whose members are as incomplete), or a stream may be kept to some of them.  Every member counts itself in
+// the team's word before the time loop.  When all have, they stay until the end and nothing can keep them from finishing;
+// a team that does not get there within gather_ticks, or meets on different XCDs, gives up as a whole (one atomic word, so
+// all members see the same) and leaves its compute units.  A small launch behind this one (ring_team_solo.hip) does the
+// tiles of the teams that gave up, a workgroup each and with the same bits, whatever else runs.
+// The waits inside the time loop are bounded too: a wave whose wait runs out leaves a word in host memory, waits for
+// nothing from then on and goes through the remaining steps on whatever it finds, so the launch ends by itself; the
+// library reports the word on its next call.
 #pragma once
 #include "ring_common.hpp"
 #include "ring_kernels.hpp"
@@ -173,7 +180,7 @@ constexpr int parked_fragments() { return KPW * C16 * MR < 24 ? 0 : (GA ? 4 : 2)
 inline __host__ __device__ int parked_bytes(int kpw, int c16, int mr, int wk) { return kpw * c16 * mr < 24 ? 0 : wk * 4 * 1024; }
 
 struct LdsPlan {       // byte offsets into dynamic LDS
-  unsigned share, state, held, gates, rows, ga, parked, weights, total;
+  unsigned share, state, held, gates, gathered, rows, ga, parked, weights, total;
 };
 
 // k: channels; nt: tiles of the fullest team; lds_mats: matrices kept in LDS; KC: K chunks
@@ -189,6 +196,7 @@ __host__ __device__ inline LdsPlan lds_plan(int k, int nt, int lds_mats, int KC,
   at += bptt ? (unsigned)nt * C16 * 256 * 2 : 0;
   p.gates = at;
   at += ((unsigned)3 * k * 16 + 64) * 4;                  // two buffers, and the spare words of TeamGates::put
+  p.gathered = at - 64;
   p.rows = at;                                            // dL/dA: r_prev of the item's rows, this member's neurons
   at += ga ? (unsigned)2 * C16 * 256 * 4 : 0;
   p.ga = at;                                              // dL/dA: shares [2][WK][k][16]
@@ -367,6 +375,51 @@ __device__ __forceinline__ void team_products(const TeamCompute<KPW, C16, MR, WK
   }
 }
 
+// Residence of the whole team (see the top of this file).  The first auxiliary wave counts its workgroup in with
+// team_arrive, waits in team_gather and leaves the verdict in LDS for all waves to read behind the next barrier (team_go).
+constexpr unsigned long long TEAM_GAVE_UP = 1ull << 63;
+
+__device__ __forceinline__ int xcc_id() { return __builtin_amdgcn_s_getreg(20 | (0 << 6) | (3 << 11)) & 7; }
+__device__ __forceinline__ unsigned team_arrived(unsigned long long v) { return (unsigned)((v * 0x0101010101010101ull) >> 56); }
+__device__ __forceinline__ bool team_complete(unsigned long long v, int G, int xcc) {
+  return !(v & TEAM_GAVE_UP) && (int)((v >> (8 * xcc)) & 255) == G;
+}
+
+__device__ __forceinline__ void team_arrive(const RingTeamArgs& c, int team, int at) {
+  if (at != 0) return;
+  if (c.gather_ticks < 0) __hip_atomic_fetch_or(c.gather + team, TEAM_GAVE_UP, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  else __hip_atomic_fetch_add(c.gather + team, 1ull << (8 * xcc_id()), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+__device__ __forceinline__ void team_gather(const RingTeamArgs& c, char* lds, const LdsPlan& L, int team, int at) {
+  if (at != 0) return;
+  const int xcc = xcc_id();
+  const long long start = wall_clock64();
+  bool ok = false;
+  unsigned long long v = __hip_atomic_load(c.gather + team, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  while (!(v & TEAM_GAVE_UP)) {
+    if ((int)team_arrived(v) == c.G) {
+      ok = team_complete(v, c.G, xcc);
+      if (!ok) __hip_atomic_fetch_or(c.gather + team, TEAM_GAVE_UP, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      break;
+    }
+    if (wall_clock64() - start > c.gather_ticks) {
+      // (fails, and leaves the new value in v, if another member has arrived meanwhile)
+      if (__hip_atomic_compare_exchange_strong(c.gather + team, &v, v | TEAM_GAVE_UP, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
+                                               __HIP_MEMORY_SCOPE_AGENT))
+        break;
+      continue;
+    }
+    __builtin_amdgcn_s_sleep(1);
+    v = __hip_atomic_load(c.gather + team, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+  *reinterpret_cast<int*>(lds + L.gathered) = ok;
+}
+
+__device__ __forceinline__ bool team_go(const char* lds, const LdsPlan& L) {
+  return __builtin_amdgcn_readfirstlane(*reinterpret_cast<const int*>(lds + L.gathered)) != 0;
+}
+
 // The compute waves' loop: `steps` rounds over the team's my_nt tiles, operand number s of round s.
 template <int KPW, int C16, int MR, int WK, bool EX, bool GA>
 __device__ __forceinline__ void team_compute_loop(const RingTeamArgs& c, const LdsPlan& L, char* lds,
@@ -384,6 +437,7 @@ __device__ __forceinline__ void team_compute_loop(const RingTeamArgs& c, const L
   const unsigned tile_bytes = (unsigned)c.KC * CHUNK_BYTES;
   const unsigned slot_bytes = tile_bytes * (unsigned)c.nbt;
   lds_barrier();                                          // the auxiliary waves' first gates (and rows) are in LDS
+  if (!team_go(lds, L)) return;
   TeamOperand<KPW> opA, opB;
   int slot = 0, it = 0, s = 0, j = 0;
   bool dead = c.spin_max < 0;      // (a negative limit gives up at once: the host's way to exercise this exit)

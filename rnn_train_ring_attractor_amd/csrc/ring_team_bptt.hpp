@@ -27,6 +27,7 @@ __global__ __launch_bounds__(64 * (WK + AUX)) void ring_team_bptt_kernel(RingBpt
   using TA = TeamAux<C16>;
   constexpr int NPT = TA::NPT;
   TA aux(c, mem, tid - 64 * WK);
+  team_arrive(c, team, aux.at);
   const int at = aux.at, N = p.N, B = p.B, nbt = p.nbt;
   float* const share = reinterpret_cast<float*>(lds + L.share);
   float* const state = reinterpret_cast<float*>(lds + L.state) + at * NPT;         // (1 - alpha) G
@@ -175,7 +176,11 @@ __global__ __launch_bounds__(64 * (WK + AUX)) void ring_team_bptt_kernel(RingBpt
     aux.publish(c, rsrc, 0, team + c.nteams * j, gg);
     keep_g(G, x, T - 1, j);
   }
-  if (steps == 0) { lds_barrier(); return; }
+  if (steps == 0) {
+    team_gather(c, lds, L, team, at);
+    lds_barrier();
+    return;
+  }
   // Register set A serves the even items, B the odd ones.  At item `it` a set holds that item's grad_output and
   // derivative record, and the gates (and r_prev rows) of item it + 1, all fetched two items earlier.
   In inA, inB;
@@ -189,7 +194,9 @@ __global__ __launch_bounds__(64 * (WK + AUX)) void ring_team_bptt_kernel(RingBpt
   far.advance(my_nt, steps);
   fetch(near, inB);
   fetch_side(far, inB);
+  team_gather(c, lds, L, team, at);
   lds_barrier();
+  if (!team_go(lds, L)) return;
 
   int slot = 0, it = 0, s = 0, j = 0;
   bool done = false;

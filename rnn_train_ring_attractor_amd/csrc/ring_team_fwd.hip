@@ -24,6 +24,7 @@ __global__ __launch_bounds__(64 * (WK + AUX)) void ring_team_fwd_kernel(RingFwdA
   using TA = TeamAux<C16>;
   constexpr int NPT = TA::NPT;
   TA aux(c, mem, tid - 64 * WK);
+  team_arrive(c, team, aux.at);
   const int at = aux.at, N = p.N, B = p.B, nbt = p.nbt;
   float* const share = reinterpret_cast<float*>(lds + L.share);
   float* const state = reinterpret_cast<float*>(lds + L.state) + at * NPT;
@@ -50,7 +51,9 @@ __global__ __launch_bounds__(64 * (WK + AUX)) void ring_team_fwd_kernel(RingFwdA
   float gA = gates_of(cur);               // items 1 and 2
   cur.advance(my_nt, T);
   float gB = gates_of(cur);
+  team_gather(c, lds, L, team, at);
   lds_barrier();
+  if (!team_go(lds, L)) return;
 
   int slot = 0, it = 0, t = 0, j = 0;
   bool done = false;

@@ -1,7 +1,8 @@
 // The team kernels' arithmetic (ring_team.hpp) by single workgroups, which need no other workgroup to be resident.
 //
 // ring_team_rebuild_kernel makes the saved record out of a given state history: every (step, batch tile) stands alone, so
-// nothing is handed over.
+// nothing is handed over.  ring_team_solo_fwd_kernel and ring_team_solo_bptt_kernel run the time loops of the teams whose
+// members did not become resident together.
 //
 // The order of every sum is that of the team kernels (K chunks by compute wave, matrices one after the other, the waves'
 // shares in wave order), so the bits are the same.
@@ -225,4 +226,313 @@ hipError_t ring_launch_team_rebuild(const RingFwdArgs& a, const RingTeamArgs& c,
     case 4: return launch_rebuild<2, 4>(a, c, wk, st);
     default: return hipErrorInvalidValue;
   }
+}
+
+// ------------------------------------------------------------------------------------------------
+// Forward and BPTT of the teams that did not gather, a workgroup per batch tile that goes through the team's members one
+// after the other.  The weights are read in fp32 from memory every step: tens of times slower than a team, and hardly
+// ever needed.  Workgroups of gathered teams leave at once: the launch and the wait for the members cost a call 3 to 4 us
+// (N = 256, B = 1, T = 100: 127 -> 130; N = 120, B = 64, T = 120, forward and backward: 238 -> 242).
+// ------------------------------------------------------------------------------------------------
+namespace {
+
+constexpr int SOLO_WAVES = 8, SOLO_C16 = 4;
+
+struct SoloLds {       // byte offsets into dynamic LDS
+  unsigned x, rs, state, gates, ga, trig, total;
+};
+__host__ __device__ inline SoloLds solo_lds(int KC, int k, bool ga, bool trig) {
+  SoloLds l;
+  unsigned at = 0;
+  l.x = at;
+  at += 2u * KC * 1024;                          // two operands, this step's and the next one's
+  l.rs = at;
+  at += 2u * KC * 256;
+  l.state = at;
+  at += 2u * KC * 1024;                          // [column tile][64 lanes] x 4 neurons: the state, or (1 - alpha) G
+  l.gates = at;
+  at += (unsigned)k * 64;
+  l.ga = at;
+  at += ga ? SOLO_WAVES * (unsigned)k * 64 : 0;
+  l.trig = at;
+  at += trig ? (unsigned)KC * 256 : 0;           // (cos, sin) of every neuron's angle
+  l.total = at;
+  return l;
+}
+
+__device__ __forceinline__ bool solo_needed(const RingTeamArgs& c, int bt) {
+  const unsigned long long v = c.gather[bt % c.nteams];      // (written by the launch in front)
+  for (int x = 0; x < 8; ++x)
+    if (team_complete(v, c.G, x)) return false;
+  return true;
+}
+
+template <bool TR>
+__device__ __forceinline__ bf16x8 solo_weight(const RingTeamArgs& c, int m, int ct, int kc, int lane) {
+  const int out = 16 * ct + (lane & 15), k0 = 32 * kc + 8 * (lane >> 4);
+  const float* W = m == 0 ? c.Wo : c.Wa + (size_t)(m - 1) * c.N * c.N;
+  WeightLoad l;
+  if (!TR && k0 + 8 <= c.N) {
+    const float* src = W + (size_t)(out < c.N ? out : c.N - 1) * c.N + k0;
+    const f32x4 lo = *reinterpret_cast<const f32x4u*>(src), hi = *reinterpret_cast<const f32x4u*>(src + 4);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) { l.v[i] = lo[i]; l.v[4 + i] = hi[i]; }
+  } else {
+    weight_load(l, W, c.N, out, k0, TR);
+  }
+  return weight_fragment(l, c.N, out, k0, m == 0 ? c.scale0 : 1.f, m == 0 ? c.shift0 : 0.f);
+}
+
+// What member `mem` of the team adds up for its column tiles: tot[cc], lane (q, row) with neurons 4q .. 4q + 3 of tile
+// mem * c16 + cc.  GA: also the member's dL/dA shares, from r_prev in rp, into ga[k][16].
+template <bool TR, bool GA>
+__device__ __forceinline__ void solo_products(const RingTeamArgs& c, const SoloOperand& o, const float* gates,
+                                              const f32x4 (&rp)[SOLO_C16], float* ga, int mem, int lane, f32x4 (&tot)[SOLO_C16]) {
+  const int b = lane & 15;
+  for (int cw = 0; cw < c.wk && cw < c.KC; ++cw) {
+    f32x4 acc[SOLO_C16];
+    float sum = 0.f;
+    for (int kc = cw; kc < c.KC; kc += c.wk) sum += o.rs[kc * 64 + lane];
+    const float j0r = c.J0 * sum_bits45(sum);
+    for (int m = 0; m <= c.k; ++m) {
+      const float g = m == 0 ? 0.f : gates[(m - 1) * 16 + b];
+      if (!GA && m >= c.mr && __ballot(g != 0.f) == 0) continue;
+      float d = 0.f;
+#pragma unroll
+      for (int cc = 0; cc < SOLO_C16; ++cc) {
+        if (cc >= c.c16) continue;
+        f32x4 P = {0.f, 0.f, 0.f, 0.f};
+        for (int kc = cw; kc < c.KC; kc += c.wk) P = mfma16(solo_weight<TR>(c, m, mem * c.c16 + cc, kc, lane), o.x[kc * 64 + lane], P);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          acc[cc][i] = m == 0 ? fmaf(c.J1, P[i], j0r) : fmaf(g, P[i], acc[cc][i]);
+          if (GA) d = fmaf(P[i], rp[cc][i], d);
+        }
+      }
+      if (GA && m > 0) {
+        d = sum_bits45(d);
+        if (lane < 16) ga[(m - 1) * 16 + b] = (cw == 0 ? 0.f : ga[(m - 1) * 16 + b]) + d;
+      }
+    }
+#pragma unroll
+    for (int cc = 0; cc < SOLO_C16; ++cc)
+      if (cc < c.c16) tot[cc] = cw == 0 ? acc[cc] : tot[cc] + acc[cc];
+  }
+}
+
+// Four neurons of a row from neuron j on; zero past the row's or the batch's end.
+__device__ __forceinline__ f32x4 solo_row4(const float* __restrict__ slab, int N, int B, int b, int j) {
+  f32x4 v;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) v[i] = b < B && j + i < N ? slab[(size_t)b * N + j + i] : 0.f;
+  return v;
+}
+__device__ __forceinline__ void solo_row4_store(float* __restrict__ slab, int N, int B, int b, int j, const f32x4& v) {
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+    if (b < B && j + i < N) slab[(size_t)b * N + j + i] = v[i];
+}
+
+// The lane's four neurons of column tile ct into the operand (all lanes of the wave).
+__device__ __forceinline__ void solo_put4(const SoloOperand& o, int ct, int lane, const f32x4& v) {
+  const int q = lane >> 4, b = lane & 15, j = 16 * ct + 4 * q, at = (j >> 5) * 64 + ((j >> 3) & 3) * 16 + b;
+  const u32x2 x = {not_empty(pack_bf16(v[0], v[1])), not_empty(pack_bf16(v[2], v[3]))};
+  *reinterpret_cast<u32x2*>(reinterpret_cast<char*>(o.x + at) + (j & 7) * 2) = x;
+  const float s = v[0] + v[1], u = v[2] + v[3], s2 = __shfl_xor(s, 16), u2 = __shfl_xor(u, 16);
+  if (!(q & 1)) o.rs[at] = row_sum8(s, u, s2, u2);
+}
+
+// A pair of steps of the copy for the weight gradients (hi null: zeros).
+__device__ __forceinline__ void solo_pair(__bf16* base, int t, int nbt, int bt, int cts, int KC, int tid, const bf16x8* lo, const bf16x8* hi) {
+  for (int u = tid; u < 2 * KC * 64; u += 64 * SOLO_WAVES) {
+    const int ct = u >> 6, rq = u >> 4 & 3, j = 16 * ct + (u & 15);
+    const size_t at = ((size_t)(j >> 5) * 64 + ((j >> 3) & 3) * 16 + 4 * rq) * 8 + (j & 7);
+    bf16x8 o;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      o[i] = reinterpret_cast<const __bf16*>(lo)[at + i * 8];
+      o[4 + i] = hi ? reinterpret_cast<const __bf16*>(hi)[at + i * 8] : (__bf16)0.f;
+    }
+    *reinterpret_cast<bf16x8*>(base + ((((size_t)(t >> 1) * nbt + bt) * cts + ct) * 64 + (u & 63)) * 8) = o;
+  }
+}
+
+__device__ __forceinline__ void solo_gates(const RingTeamArgs& c, float* gates, int t, int bt, int tid) {
+  for (int u = tid; u < c.k * 16; u += 64 * SOLO_WAVES) {
+    const int row = 16 * bt + (u & 15);
+    gates[u] = row < c.B ? c.A[((size_t)row * c.T + t) * c.k + (u >> 4)] : 0.f;
+  }
+}
+
+}  // namespace
+
+template <int ACT>
+__global__ __launch_bounds__(64 * SOLO_WAVES) void ring_team_solo_fwd_kernel(RingFwdArgs p, RingTeamArgs c) {
+  extern __shared__ __attribute__((aligned(16))) char lds[];
+  const int bt = blockIdx.x;
+  if (!solo_needed(c, bt)) return;
+  const int KC = c.KC, N = p.N, B = p.B, T = p.T, tid = threadIdx.x, lane = tid & 63, q = lane >> 4, b = 16 * bt + (lane & 15);
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const SoloLds L = solo_lds(KC, c.k, false, false);
+  auto operand = [&](int i) {
+    return SoloOperand{reinterpret_cast<bf16x8*>(lds + L.x) + (size_t)i * KC * 64, reinterpret_cast<float*>(lds + L.rs) + (size_t)i * KC * 64};
+  };
+  f32x4* const state = reinterpret_cast<f32x4*>(lds + L.state) + lane;
+  float* const gates = reinterpret_cast<float*>(lds + L.gates);
+  const float oma = 1.f - p.alpha;
+  const ActScale asc = act_scale_make(p.alpha);
+
+  for (int ct = w; ct < 2 * KC; ct += SOLO_WAVES) {
+    const f32x4 r = solo_row4(p.r_init, N, B, b, 16 * ct + 4 * q);
+    state[ct * 64] = r;
+    solo_put4(operand(0), ct, lane, r);
+  }
+  for (int t = 0; t < T; ++t) {
+    const SoloOperand cur = operand(t & 1), next = operand((t + 1) & 1);
+    solo_gates(c, gates, t, bt, tid);
+    lds_barrier();
+    for (int mem = w; mem < c.G; mem += SOLO_WAVES) {
+      f32x4 x[SOLO_C16];
+      const f32x4 none[SOLO_C16] = {};
+      solo_products<false, false>(c, cur, gates, none, nullptr, mem, lane, x);
+#pragma unroll
+      for (int cc = 0; cc < SOLO_C16; ++cc) {
+        const int ct = mem * c.c16 + cc, j = 16 * ct + 4 * q;
+        if (cc >= c.c16 || ct >= 2 * KC) continue;
+        const f32x4 r = state[ct * 64];
+        f32x4 rn;
+        f16x4 d;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          float aF, aD;
+          act_scaled<ACT>(x[cc][i], asc, aF, aD);
+          rn[i] = j + i < N ? fmaf(oma, r[i], aF) : 0.f;
+          d[i] = (_Float16)aD;
+        }
+        state[ct * 64] = rn;
+        solo_put4(next, ct, lane, rn);
+        solo_row4_store(p.hist + (size_t)t * B * N, N, B, b, j, rn);
+        if (p.dfrag) *reinterpret_cast<f16x4*>(p.dfrag + (((size_t)t * p.nbt + bt) * c.cts + ct) * 256 + lane * 4) = d;
+      }
+    }
+    lds_barrier();
+    if (p.rfrag && (t & 1) == 0) solo_pair(p.rfrag, t, p.nbt, bt, c.cts, KC, tid, cur.x, t + 1 < T ? next.x : nullptr);
+  }
+}
+
+template <bool GA>
+__global__ __launch_bounds__(64 * SOLO_WAVES) void ring_team_solo_bptt_kernel(RingBpttArgs p, RingTeamArgs c) {
+  extern __shared__ __attribute__((aligned(16))) char lds[];
+  const int bt = blockIdx.x;
+  if (!solo_needed(c, bt)) return;
+  const int KC = c.KC, N = p.N, B = p.B, T = p.T, k = c.k, tid = threadIdx.x, lane = tid & 63, q = lane >> 4, b = 16 * bt + (lane & 15);
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const bool loss = p.loss_coef != nullptr;
+  const SoloLds L = solo_lds(KC, k, GA, loss);
+  auto operand = [&](int i) {
+    return SoloOperand{reinterpret_cast<bf16x8*>(lds + L.x) + (size_t)i * KC * 64, reinterpret_cast<float*>(lds + L.rs) + (size_t)i * KC * 64};
+  };
+  f32x4* const state = reinterpret_cast<f32x4*>(lds + L.state) + lane;
+  float* const gates = reinterpret_cast<float*>(lds + L.gates);
+  float* const ga = reinterpret_cast<float*>(lds + L.ga) + (size_t)w * k * 16;
+  f32x2* const trig = reinterpret_cast<f32x2*>(lds + L.trig);
+  const float oma = 1.f - p.alpha;
+  float up = 0.f;
+  if (loss) {
+    for (int j = tid; j < 32 * KC; j += 64 * SOLO_WAVES) {
+      const float phi = 6.2831853071795864769f * (float)j / (float)N;
+      trig[j] = f32x2{cosf(phi), sinf(phi)};
+    }
+    up = (p.loss_upstream ? p.loss_upstream[0] : 1.f) * p.loss_inv_rows;
+    lds_barrier();
+  }
+
+  // g of step t from what is carried into it, into an operand; keeps (1 - alpha) G
+  auto form_g = [&](int t, int ct, const f32x4& carry, const SoloOperand& o) {
+    const int j = 16 * ct + 4 * q;
+    const f32x4 in = solo_row4((loss ? p.hist : p.grad_out) + (size_t)t * B * N, N, B, b, j);
+    const f16x4 d = *reinterpret_cast<const f16x4*>(p.dfrag + (((size_t)t * p.nbt + bt) * c.cts + ct) * 256 + lane * 4);
+    float kc = 0.f, ks = 0.f, beta = 0.f;
+    if (loss && b < B) {
+      const ring_f32x4 cf = p.loss_coef[(size_t)t * B + b];
+      kc = cf[0] * up;
+      ks = cf[1] * up;
+      beta = cf[2] * up;
+    }
+    f32x4 gg, keep;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      float go = in[i];
+      if (loss) {
+        const float r = go;
+        const f32x2 a = trig[j + i];
+        go = fmaf(kc, a[0], fmaf(ks, a[1], r > 0.f ? beta : (r < 0.f ? -beta : 0.f)));
+      }
+      const bool ok = b < B && j + i < N;
+      const float G = ok ? go + carry[i] : 0.f;
+      gg[i] = ok ? (float)d[i] * G : 0.f;
+      keep[i] = oma * G;
+    }
+    state[ct * 64] = keep;
+    solo_put4(o, ct, lane, gg);
+  };
+
+  for (int ct = w; ct < 2 * KC; ct += SOLO_WAVES) form_g(T - 1, ct, f32x4{0.f, 0.f, 0.f, 0.f}, operand(0));
+  lds_barrier();
+  if (((T - 1) & 1) == 0) solo_pair(p.gfrag, T - 1, p.nbt, bt, c.cts, KC, tid, operand(0).x, nullptr);
+  const int steps = (p.grad_r_init || GA) ? T : T - 1;
+  for (int s = 0; s < steps; ++s) {
+    const SoloOperand cur = operand(s & 1), next = operand((s + 1) & 1);
+    const int t = T - 1 - s;                     // the products' step
+    solo_gates(c, gates, t, bt, tid);
+    lds_barrier();
+    for (int mem = w; mem < c.G; mem += SOLO_WAVES) {
+      f32x4 x[SOLO_C16], rp[SOLO_C16] = {};
+      if constexpr (GA) {
+#pragma unroll
+        for (int cc = 0; cc < SOLO_C16; ++cc)
+          if (cc < c.c16) rp[cc] = solo_row4(t == 0 ? p.r_init : p.hist + (size_t)(t - 1) * B * N, N, B, b, 16 * (mem * c.c16 + cc) + 4 * q);
+      }
+      solo_products<true, GA>(c, cur, gates, rp, ga, mem, lane, x);
+      if constexpr (GA) {
+        if (lane < 16 && b < B)
+          for (int ch = 0; ch < k; ++ch) c.ga_part[(((size_t)mem * T + t) * k + ch) * B + b] = ga[ch * 16 + lane];
+      }
+#pragma unroll
+      for (int cc = 0; cc < SOLO_C16; ++cc) {
+        const int ct = mem * c.c16 + cc;
+        if (cc >= c.c16 || ct >= 2 * KC) continue;
+        const f32x4 carry = state[ct * 64] + x[cc];
+        if (t > 0) form_g(t - 1, ct, carry, next);
+        else if (p.grad_r_init) solo_row4_store(p.grad_r_init, N, B, b, 16 * ct + 4 * q, carry);
+      }
+    }
+    lds_barrier();
+    if (t > 0 && ((t - 1) & 1) == 0) solo_pair(p.gfrag, t - 1, p.nbt, bt, c.cts, KC, tid, next.x, cur.x);
+  }
+}
+
+// (launched past RING_LAUNCH: the slot's kernel is the team kernel in front)
+template <typename K, typename Args>
+static hipError_t launch_solo(K kern, const Args& a, const RingTeamArgs& c, unsigned lds, hipStream_t st) {
+  const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+  if (e != hipSuccess) return e;
+  hipLaunchKernelGGL(kern, dim3((unsigned)c.nbt), dim3(64 * SOLO_WAVES), lds, st, a, c);
+  return hipGetLastError();
+}
+
+hipError_t ring_launch_team_solo_fwd(const RingFwdArgs& a, const RingTeamArgs& c, hipStream_t st) {
+  const unsigned lds = solo_lds(c.KC, c.k, false, false).total;
+  switch (a.act) {
+    case ACT_RELU: return launch_solo(ring_team_solo_fwd_kernel<ACT_RELU>, a, c, lds, st);
+    case ACT_GELU: return launch_solo(ring_team_solo_fwd_kernel<ACT_GELU>, a, c, lds, st);
+    case ACT_TANH: return launch_solo(ring_team_solo_fwd_kernel<ACT_TANH>, a, c, lds, st);
+    case ACT_SILU: return launch_solo(ring_team_solo_fwd_kernel<ACT_SILU>, a, c, lds, st);
+    default: return hipErrorInvalidValue;
+  }
+}
+
+hipError_t ring_launch_team_solo_bptt(const RingBpttArgs& a, const RingTeamArgs& c, hipStream_t st) {
+  const unsigned lds = solo_lds(c.KC, c.k, a.grad_A != nullptr, a.loss_coef != nullptr).total;
+  return a.grad_A ? launch_solo(ring_team_solo_bptt_kernel<true>, a, c, lds, st) : launch_solo(ring_team_solo_bptt_kernel<false>, a, c, lds, st);
 }

@@ -35,7 +35,7 @@ def _t(x, dev):
     return torch.tensor(x, device=dev)
 
 
-def _run(p, act, J0, J1, dev, saved=True, ga=True):
+def _run(p, act, J0, J1, dev, saved=True, ga=True, keep_record=False):
     from rnn_train_ring_attractor_amd import rnn_cuda, _lib
     A, Wa, Wo, r0, G = (_t(p[x], dev) for x in ("A", "Wa", "Wo", "r0", "G"))
     B, T, k = p["A"].shape
@@ -52,7 +52,8 @@ def _run(p, act, J0, J1, dev, saved=True, ga=True):
     torch.cuda.synchronize()
     names = _lib.last_kernel_names()
     assert "ring_team_bptt" in names["bptt"] and ("ring_team_fwd" in names["fwd"] or not saved)
-    return dict(hist=hist, grad_Wa=gWa, grad_Wo=gWo, grad_r_init=gr, **({"grad_A": gA} if ga else {}))
+    return dict(hist=hist, grad_Wa=gWa, grad_Wo=gWo, grad_r_init=gr, **({"grad_A": gA} if ga else {}),
+                **({"saved": sv} if saved and keep_record else {}))
 
 
 @pytest.fixture
@@ -160,6 +161,76 @@ def test_teams_on_two_streams(gpu_device, teams):
             fwd(o)
     torch.cuda.synchronize()
     assert all(torch.equal(o, ref) for o in outs)
+    fwd(ref)                       # (a wait that had run out would be reported by this call)
+
+
+@pytest.mark.parametrize("B,T,k,N,act", CASES + [(40, 5, 2, 120, "relu")], ids=[f"b{c[0]}_t{c[1]}_k{c[2]}_n{c[3]}" for c in CASES] + ["relu"])
+def test_teams_that_do_not_gather_are_done_by_single_workgroups_with_the_same_bits(B, T, k, N, act, gpu_device, teams, monkeypatch):
+    """A team whose members do not become resident together (another team launch may hold the compute units they lack)
+    gives up before the time loop, and a launch behind does its tiles.  Here the host lets every team give up at once, and
+    then after no wait at all, when some teams are complete and others are not."""
+    print(f"[case] ungathered teams B={B} T={T} k={k} N={N} {act}", flush=True)
+    p = make_problem(900 + N + k, B, T, k, N, action="dense")
+    if k > 3:
+        p["A"][:, :, k // 2] = 0.0
+    for ga in (True, False):
+        want = _run(p, act, -1.0 / N, 0.6, gpu_device, ga=ga, keep_record=True)
+        for wait_us in ("-1", "0", "2"):
+            monkeypatch.setenv("RINGATTR_TEAM_GATHER_US", wait_us)
+            got = _run(p, act, -1.0 / N, 0.6, gpu_device, ga=ga, keep_record=True)
+            monkeypatch.delenv("RINGATTR_TEAM_GATHER_US")
+            assert all(torch.equal(got[x], want[x]) for x in want), [x for x in want if not torch.equal(got[x], want[x])]
+
+
+def test_objective_of_teams_that_do_not_gather(gpu_device, teams, monkeypatch):
+    from rnn_train_ring_attractor_amd import ring_rnn_loss_func
+    B, T, k, N = 70, 6, 3, 361
+    print(f"[case] ungathered teams, objective B={B} T={T} k={k} N={N}", flush=True)
+    p = make_problem(77, B, T, k, N, action="dense")
+    r0 = _t(p["r0"], gpu_device)
+    angle = torch.rand(B, T, device=gpu_device) * 6.28
+    for want_a in (False, True):
+        runs = []
+        for wait_us in ("50000", "-1"):
+            monkeypatch.setenv("RINGATTR_TEAM_GATHER_US", wait_us)
+            leaves = [_t(p[x], gpu_device).requires_grad_(x != "A" or want_a) for x in ("A", "Wa", "Wo")]
+            total = ring_rnn_loss_func(leaves[0], leaves[1], -1.0 / N, 0.6, leaves[2], r0, 0.15, "gelu", angle, 0.2)[0]
+            total.backward()
+            runs.append([total.detach()] + [x.grad for x in leaves if x.grad is not None])
+        assert len(runs[0]) == (4 if want_a else 3) and all(torch.equal(x, y) for x, y in zip(*runs))
+
+
+def test_graphs_replayed_on_two_streams(gpu_device, teams):
+    """Nothing on the host orders the team launches of two replayed graphs.  Each of these wants every compute unit for its
+    teams of 32; whichever teams starve give up and are done by single workgroups."""
+    from rnn_train_ring_attractor_amd import rnn_cuda, _lib
+    B, T, k, N = 128, 12, 2, 1000
+    print(f"[case] two graphs of team forwards on two streams B={B} T={T} N={N}", flush=True)
+    p = make_problem(81, B, T, k, N, action="dense")
+    A, Wa, Wo, r0 = (_t(p[x], gpu_device) for x in ("A", "Wa", "Wo", "r0"))
+
+    def fwd(out):
+        rnn_cuda.fwd_cuda.fwd(A=A, Wa=Wa, J0=-1.0 / N, J1=0.6, Wo=Wo, r_init=r0, bump_history=out, alpha=0.15, activation_type=2)
+
+    ref = torch.empty(T, B, N, device=gpu_device)
+    fwd(ref)
+    assert "ring_team_fwd" in _lib.last_kernel_names()["fwd"]
+    outs = [torch.empty_like(ref) for _ in range(2)]
+    graphs = [torch.cuda.CUDAGraph() for _ in range(2)]
+    for g, o in zip(graphs, outs):
+        torch.cuda.synchronize()
+        with torch.cuda.graph(g):
+            fwd(o)
+    streams = [torch.cuda.Stream(device=gpu_device) for _ in range(2)]
+    for _ in range(4):
+        for o in outs:
+            o.fill_(float("nan"))
+        torch.cuda.synchronize()
+        for st, g in zip(streams, graphs):
+            with torch.cuda.stream(st):
+                g.replay()
+        torch.cuda.synchronize()
+        assert all(torch.equal(o, ref) for o in outs)
     fwd(ref)                       # (a wait that had run out would be reported by this call)
 
 
