@@ -1075,6 +1075,7 @@ static hipError_t launch_fwd_cluster_act(const RingFwdArgs& a, const RingCluster
     hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
                                        (int)C8_LDS_BYTES);
     if (e != hipSuccess) return e;
+    const RingLaunchGuard::Launch order(ring_launch_guard(), st, 3);     // (clusters of four, on the way to being resident)
     RING_LAUNCH(kern, dim3(grid), dim3(512), C8_LDS_BYTES, st, a, c);
     return hipGetLastError();
   };
@@ -1118,6 +1119,7 @@ hipError_t ring_launch_bptt_cluster(const RingBpttArgs& a, hipStream_t st) {
     hipError_t e2 = hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
                                         (int)C8_LDS_BYTES);
     if (e2 != hipSuccess) return e2;
+    const RingLaunchGuard::Launch order(ring_launch_guard(), st, 3);     // (clusters of four, on the way to being resident)
     RING_LAUNCH(kern, dim3(grid), dim3(512), C8_LDS_BYTES, st, a, c);
     return hipGetLastError();
   };

@@ -1322,6 +1322,38 @@ hipError_t ring_launch_rebuild(const RingFwdArgs& a, int NCv, hipStream_t st) {
   return e;
 }
 
+unsigned long RingGuardHip::owner(hipStream_t st) {
+  static std::atomic<unsigned long> threads{0};
+  static thread_local const unsigned long id = ++threads;
+  return st == hipStreamPerThread ? id : 0;
+}
+bool RingGuardHip::capturing(hipStream_t st) {
+  hipStreamCaptureStatus s = hipStreamCaptureStatusNone;
+  return hipStreamIsCapturing(st, &s) == hipSuccess && s != hipStreamCaptureStatusNone;
+}
+bool RingGuardHip::record(hipEvent_t& ev, hipStream_t st) {
+  if ((ev || hipEventCreateWithFlags(&ev, hipEventDisableTiming) == hipSuccess) && hipEventRecord(ev, st) == hipSuccess) return true;
+  (void)hipGetLastError();
+  return false;
+}
+bool RingGuardHip::wait(hipStream_t st, hipEvent_t ev) { return hipStreamWaitEvent(st, ev, 0) == hipSuccess; }
+bool RingGuardHip::done(hipEvent_t ev) {
+  if (hipEventQuery(ev) == hipSuccess) return true;
+  (void)hipGetLastError();
+  return false;
+}
+
+RingLaunchGuard& ring_launch_guard() {
+  constexpr int DEVICES = 64, CUS_PER_XCD = 32;
+  static std::vector<RingLaunchGuard*> guards = [] {
+    std::vector<RingLaunchGuard*> v(DEVICES);
+    for (auto& g : v) g = new RingLaunchGuard(CUS_PER_XCD);     // (for the life of the process)
+    return v;
+  }();
+  int dev = 0;
+  return *guards[hipGetDevice(&dev) == hipSuccess && dev >= 0 && dev < DEVICES ? dev : 0];
+}
+
 // Team launches under their profiling slots.
 hipError_t ring_run_team_fwd(const RingFwdArgs& a, const float* Wo, const float* Wa, bool folded, int cts, void* ws, hipStream_t st) {
   ProfScope prof(1, st);

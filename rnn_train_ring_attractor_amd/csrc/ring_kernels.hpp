@@ -3,6 +3,8 @@
 #include <hip/hip_runtime.h>
 #include <stddef.h>
 
+#include "ring_guard.hpp"
+
 typedef float ring_f32x4 __attribute__((ext_vector_type(4)));
 
 struct RingFwdArgs {
@@ -205,6 +207,24 @@ int ring_dw_tiled_segments(int nbt, int T, int nz);   // launches per matrix gro
 void ring_profile_set(int stride);
 bool ring_profile_on();
 hipError_t ring_profile_collect(double* ms, long long* launches);
+
+// The HIP side of ring_guard.hpp.  A handle of hipStreamPerThread means another stream in every thread.
+struct RingGuardHip {
+  using Stream = hipStream_t;
+  using Event = hipEvent_t;
+  static unsigned long owner(Stream st);
+  static bool capturing(Stream st);
+  static bool record(Event& ev, Stream st);
+  static bool wait(Stream st, Event ev);
+  static bool done(Event ev);
+  struct Quiet {
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    Quiet() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+    ~Quiet() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+  };
+};
+using RingLaunchGuard = ResidencyGuard<RingGuardHip>;
+RingLaunchGuard& ring_launch_guard();     // the current device's
 
 // Teams of workgroups that keep the weights on chip and exchange the state through L2 (ring_team*.hip).
 struct RingTeamArgs {

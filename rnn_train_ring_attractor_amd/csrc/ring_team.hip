@@ -1,4 +1,4 @@
-// Team kernels: choice of shape, scratch area, launch order between streams (kernels: ring_team.hpp).
+// Team kernels: choice of shape and scratch area (kernels: ring_team.hpp).
 #include "ring_team.hpp"
 
 // Sum of the members' dL/dA partials in member order.
@@ -24,7 +24,6 @@ __global__ __launch_bounds__(256) void ring_team_fill_kernel(u32x4* p, unsigned 
 
 #include <stdlib.h>
 #include <algorithm>
-#include <mutex>
 
 namespace {
 
@@ -32,22 +31,6 @@ constexpr int XCDS = 8, CUS_PER_XCD = 32;
 constexpr size_t LDS_MAX = 160 * 1024;
 
 size_t up256(size_t n) { return (n + 255) & ~(size_t)255; }
-
-// One team launch at a time per device.  Two of them dispatched together could each hold compute units the other's
-// missing members need.  Launches of one stream follow each other anyway; when another stream comes along it is made
-// to wait for the last one (an event recorded there and then, so single-stream programs pay nothing).  Streams under
-// graph capture are left alone: a replayed graph is ordered by whoever launches it.
-std::mutex g_guard_mu;
-struct GuardState {
-  bool used = false;
-  hipStream_t last = nullptr;
-  hipEvent_t ev = nullptr;
-} g_guard[64];
-
-bool capturing(hipStream_t st) {
-  hipStreamCaptureStatus s = hipStreamCaptureStatusNone;
-  return hipStreamIsCapturing(st, &s) == hipSuccess && s != hipStreamCaptureStatusNone;
-}
 
 template <int C16, int WK>
 size_t plan_lds(const RingTeamShape& s, int k, int nt, int KC, bool bptt, bool ga) {
@@ -77,31 +60,6 @@ int device_cus() {
 }
 
 }  // namespace
-
-hipError_t ring_team_guard_enter(hipStream_t st) {
-  g_guard_mu.lock();
-  int dev = 0;
-  if (capturing(st) || hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return hipSuccess;
-  GuardState& g = g_guard[dev];
-  if (g.used && g.last != st && !capturing(g.last)) {
-    hipError_t e = g.ev ? hipSuccess : hipEventCreateWithFlags(&g.ev, hipEventDisableTiming);
-    if (e == hipSuccess) e = hipEventRecord(g.ev, g.last);
-    if (e == hipSuccess) e = hipStreamWaitEvent(st, g.ev, 0);
-    if (e != hipSuccess) {                 // the other stream is gone: whatever ran there is waited for
-      (void)hipGetLastError();
-      e = hipDeviceSynchronize();
-      if (e != hipSuccess) {
-        g_guard_mu.unlock();
-        return e;
-      }
-    }
-  }
-  g.used = true;
-  g.last = st;
-  return hipSuccess;
-}
-
-void ring_team_guard_leave() { g_guard_mu.unlock(); }
 
 // The shape of a team for this problem: the cheapest of the built ones by a model of one time step in cycles.
 //   products of an item  M c16 KC 16 / 4 (four matrix pipes) + reading the fragments kept in LDS + what a wave spends around them

@@ -712,18 +712,13 @@ __device__ __forceinline__ bool team_coords(const RingTeamArgs& c, int& team, in
   X(3, 1, 3, 8) X(3, 2, 3, 8) X(4, 1, 3, 8) X(4, 2, 3, 8)
 // (each once with all matrices in registers and once with further ones in LDS)
 
-// Launches one team kernel: one launch of this family at a time per device (see ring_team.hip).
-hipError_t ring_team_guard_enter(hipStream_t st);
-void ring_team_guard_leave();
+// Launches one team kernel.
 template <typename F>
-hipError_t ring_team_start(const void* kernel, const RingTeamShape& sh, unsigned lds, hipStream_t st, F&& go) {
+hipError_t ring_team_start(const void* kernel, const RingTeamShape& sh, int G, unsigned lds, hipStream_t st, F&& go) {
   hipError_t e = hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
   if (e != hipSuccess) return e;
-  e = ring_team_guard_enter(st);
-  if (e != hipSuccess) return e;
+  const RingLaunchGuard::Launch order(ring_launch_guard(), st, G - 1);
   go(dim3((unsigned)sh.grid), dim3(64u * (unsigned)(sh.wk + AUX)), lds);
-  e = hipGetLastError();
-  ring_team_guard_leave();
-  return e;
+  return hipGetLastError();
 }
 

@@ -108,7 +108,7 @@ __global__ __launch_bounds__(64 * (WK + AUX)) void ring_team_fwd_kernel(RingFwdA
 
 hipError_t ring_launch_team_fwd(const RingFwdArgs& a, const RingTeamArgs& c, const RingTeamShape& sh, hipStream_t st) {
 #define RING_TEAM_ACT(KPW, C16, MR, WK, EX, ACT)                                                                    \
-  return ring_team_start(reinterpret_cast<const void*>(&ring_team_fwd_kernel<KPW, C16, MR, WK, EX, ACT>), sh,       \
+  return ring_team_start(reinterpret_cast<const void*>(&ring_team_fwd_kernel<KPW, C16, MR, WK, EX, ACT>), sh, c.G,       \
                          lds_plan<C16, WK>(c.k, c.nt, sh.lds_mats, c.KC, parked_bytes(KPW, C16, MR, WK), false, false).total, st,               \
                          [&](dim3 g, dim3 b, unsigned lds) {                                                    \
                            RING_LAUNCH((ring_team_fwd_kernel<KPW, C16, MR, WK, EX, ACT>), g, b, lds, st, a, c);     \

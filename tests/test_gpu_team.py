@@ -200,6 +200,34 @@ def test_objective_of_teams_that_do_not_gather(gpu_device, teams, monkeypatch):
         assert len(runs[0]) == (4 if want_a else 3) and all(torch.equal(x, y) for x, y in zip(*runs))
 
 
+def test_cluster_and_team_launches_on_two_streams(gpu_device, teams, monkeypatch):
+    """Teams of 32 on one stream and the N = 512 clusters on another, launched in turn: between them they could fill an XCD
+    with workgroups that wait for others, so they run one after the other."""
+    from rnn_train_ring_attractor_amd import rnn_cuda, _lib
+    monkeypatch.delenv("RINGATTR_TEAM")
+    jobs = []
+    for B, T, N, kernel in ((8192, 16, 512, "ring_fwd_cluster8"), (128, 40, 1000, "ring_team_fwd")):
+        p = make_problem(82, B, T, 2, N, action="dense")
+        A, Wa, Wo, r0 = (_t(p[x], gpu_device) for x in ("A", "Wa", "Wo", "r0"))
+
+        def fwd(out, A=A, Wa=Wa, Wo=Wo, r0=r0, N=N):
+            rnn_cuda.fwd_cuda.fwd(A=A, Wa=Wa, J0=-1.0 / N, J1=0.6, Wo=Wo, r_init=r0, bump_history=out, alpha=0.15, activation_type=2)
+
+        ref = torch.empty(T, B, N, device=gpu_device)
+        fwd(ref)
+        assert kernel in _lib.last_kernel_names()["fwd"]
+        jobs.append((fwd, ref, torch.cuda.Stream(device=gpu_device), [torch.full_like(ref, float("nan")) for _ in range(3)]))
+    print("[case] clusters and teams on two streams", flush=True)
+    torch.cuda.synchronize()
+    for i in range(3):
+        for fwd, _, st, outs in jobs:
+            with torch.cuda.stream(st):
+                fwd(outs[i])
+    torch.cuda.synchronize()
+    assert all(torch.equal(o, ref) for _, ref, _, outs in jobs for o in outs)
+    jobs[0][0](jobs[0][1])         # (a wait that had run out would be reported by this call)
+
+
 def test_graphs_replayed_on_two_streams(gpu_device, teams):
     """Nothing on the host orders the team launches of two replayed graphs.  Each of these wants every compute unit for its
     teams of 32; whichever teams starve give up and are done by single workgroups."""
