@@ -68,9 +68,14 @@ RINGATTR_API size_t ringattr_saved_bytes(int N, int a_dim, int seq_len, int batc
  * least the packed weights) runs the weight-streaming kernel instead.
  * The backward's figure at that width includes the scratch area of the BPTT on the same clusters
  * (switched on by RINGATTR_CLUSTER_BPTT=1), whether it is on or not.
+ * ringattr_bwd_workspace_bytes is enough with and without grad_A.  A backward that is not asked for dL/dA may need
+ * much less (the team kernels keep a share of it per member, up to 4 * N * seq_len * batch_size bytes):
+ * ringattr_bwd_workspace_bytes_for tells the two apart, and ringattr_bwd asks for no more than its own arguments need.
  * Replaces the fixed workspace list of cpp/ring_rnn_cuda.py:108-114. */
 RINGATTR_API size_t ringattr_fwd_workspace_bytes(int N, int a_dim, int seq_len, int batch_size);
 RINGATTR_API size_t ringattr_bwd_workspace_bytes(int N, int a_dim, int seq_len, int batch_size, int have_saved);
+RINGATTR_API size_t ringattr_bwd_workspace_bytes_for(int N, int a_dim, int seq_len, int batch_size, int have_saved,
+                                                     int want_grad_A);
 
 /* Forward recurrence over all T steps in one persistent launch.
  * Replaces fwd_cuda (cpp/fwd.cu:21-50) and the pybind shim cpp/fwd.cpp:20-47.

@@ -27,6 +27,7 @@ PROTOTYPES = {
     "ringattr_saved_bytes": (c_size_t, [c_int] * 4),
     "ringattr_fwd_workspace_bytes": (c_size_t, [c_int] * 4),
     "ringattr_bwd_workspace_bytes": (c_size_t, [c_int] * 5),
+    "ringattr_bwd_workspace_bytes_for": (c_size_t, [c_int] * 6),
     "ringattr_fwd": (c_int, [c_void_p, c_void_p, c_float, c_float, c_void_p, c_void_p, c_void_p, c_float,
                              c_int, c_int, c_int, c_int, c_int, c_void_p, c_void_p, c_size_t, c_void_p]),
     "ringattr_fwd_loss": (c_int, [c_void_p, c_void_p, c_float, c_float, c_void_p, c_void_p, c_void_p, c_float,

@@ -251,7 +251,7 @@ struct RingTeamPlan {
 RingTeamPlan ring_team_plan(int N, int k, int T, int B, bool bptt, bool ga);
 bool ring_uses_team(int N, int k, int T, int B);
 size_t ring_team_fwd_bytes(int N, int k, int T, int B);   // scratch of one launch (0 where teams do not apply)
-size_t ring_team_bptt_bytes(int N, int k, int T, int B);
+size_t ring_team_bptt_bytes(int N, int k, int T, int B, bool ga);
 // J1 * Wo + J0 as one operand (folded) or kept apart; `ws` is ring_team_fwd_bytes / ring_team_bptt_bytes large
 hipError_t ring_team_fwd(const RingFwdArgs& a, const float* Wo, const float* Wa, bool folded, int cts, void* ws, hipStream_t st);
 hipError_t ring_team_bptt(const RingBpttArgs& a, const float* Wo, const float* Wa, bool folded, int cts, void* ws, hipStream_t st);

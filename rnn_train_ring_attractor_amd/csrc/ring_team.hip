@@ -127,32 +127,31 @@ static bool resident_only(int N, int k, int B) { return ring_res256_applicable(N
 //     ask whether a record is wanted: a history is the same with and without one;
 //   * with many tiles per team (more than eight at N <= 512) a compute unit's epilogue work is what bounds a step, and
 //     the kernels that have a batch tile to themselves, or the N = 512 clusters, are as fast or faster.
+static bool team_shape(int N, int k, int T, int B) {
+  if (resident_only(N, k, B) && !forced()) return false;
+  const RingTeamPlan f = ring_team_plan(N, k, T, B, false, false);
+  if (!f.ok || !ring_team_plan(N, k, T, B, true, true).ok) return false;
+  return forced() || ring_res256_applicable(N, k) || N > 512 || f.nt <= 8;
+}
+
 bool ring_uses_team(int N, int k, int T, int B) {
   const char* v = getenv("RINGATTR_TEAM");
-  const bool force = v && v[0] == '1';
-  if ((v && v[0] == '0') || (!force && resident_only(N, k, B)) || ring_cluster_error()) return false;
+  if ((v && v[0] == '0') || ring_cluster_error()) return false;
   // a switch that asks for one of the other families by name is obeyed
   for (const char* name : {"RINGATTR_STREAMING", "RINGATTR_ROW_TILES", "RINGATTR_BLOCK", "RINGATTR_WIDE", "RINGATTR_SPLIT_FORWARD",
                            "RINGATTR_LDS_WEIGHTS", "RINGATTR_BLOCK_SHAPE", "RINGATTR_CLUSTER", "RINGATTR_CLUSTER_BPTT"})
     if (getenv(name)) return false;
-  if (device_cus() != XCDS * CUS_PER_XCD) return false;
-  const RingTeamPlan f = ring_team_plan(N, k, T, B, false, false);
-  if (!f.ok || !ring_team_plan(N, k, T, B, true, true).ok) return false;
-  return force || ring_res256_applicable(N, k) || N > 512 || f.nt <= 8;
+  return device_cus() == XCDS * CUS_PER_XCD && team_shape(N, k, T, B);
 }
 
-// (no exchange area where no call of this shape comes here)
-size_t ring_team_fwd_bytes(int N, int k, int T, int B) {
-  if (resident_only(N, k, B) && !forced()) return 0;
-  const RingTeamPlan p = ring_team_plan(N, k, T, B, false, false);
-  return p.ok ? p.xchg_bytes + p.gather_bytes : 0;
+// Scratch of one launch; none where no call of this shape comes here.
+static size_t plan_bytes(int N, int k, int T, int B, bool bptt, bool ga) {
+  if (!team_shape(N, k, T, B)) return 0;
+  const RingTeamPlan p = ring_team_plan(N, k, T, B, bptt, ga);
+  return p.xchg_bytes + p.gather_bytes + p.ga_bytes;
 }
-
-size_t ring_team_bptt_bytes(int N, int k, int T, int B) {
-  if (resident_only(N, k, B) && !forced()) return 0;
-  const RingTeamPlan p = ring_team_plan(N, k, T, B, true, false), g = ring_team_plan(N, k, T, B, true, true);
-  return std::max(p.ok ? p.xchg_bytes + p.gather_bytes : 0, g.ok ? g.xchg_bytes + g.gather_bytes + g.ga_bytes : 0);
-}
+size_t ring_team_fwd_bytes(int N, int k, int T, int B) { return plan_bytes(N, k, T, B, false, false); }
+size_t ring_team_bptt_bytes(int N, int k, int T, int B, bool ga) { return plan_bytes(N, k, T, B, true, ga); }
 
 static hipError_t team_args(const RingTeamPlan& p, const float* Wo, const float* Wa, const float* A, float J0, float J1,
                             bool folded, int N, int k, int T, int B, int cts, bool transposed, void* ws, RingTeamArgs& c,

@@ -182,17 +182,39 @@ size_t ringattr_fwd_workspace_bytes(int N, int a_dim, int seq_len, int batch_siz
   return packed > team ? packed : team;
 }
 
-// The tail of a backward's workspace that the team BPTT uses.
-static size_t team_area(int N, int a_dim, int seq_len, int batch_size) { return ring_team_bptt_bytes(N, a_dim, seq_len, batch_size); }
+// A backward's workspace.  Most families: packed weights, operand copy of g, split-K partials, the small areas, and
+// without a saved record a second packed copy, the record and the clusters' scratch.  The team kernels read the fp32
+// weights and use neither of the small areas; their packed copy for the rebuild, their BPTT's scratch and the split-K
+// partials are needed one after the other and share one area behind the operand copy and the record.
+static size_t team_shared_bytes(const Geo& g, bool have_saved, bool grad_A) {
+  const size_t bptt = ring_team_bptt_bytes(g.N, g.k, g.T, g.B, grad_A), packed = have_saved ? 0 : g.wpack_bytes;
+  const size_t most = bptt > packed ? bptt : packed;
+  return most > g.partial_bytes ? most : g.partial_bytes;
+}
+static size_t bwd_bytes(const Geo& g, bool have_saved, bool team, bool grad_A) {
+  const size_t record = have_saved ? 0 : g.side_bytes + g.pair_bytes;
+  if (team) return g.pair_bytes + record + team_shared_bytes(g, have_saved, grad_A);
+  size_t s = g.wpack_bytes + g.pair_bytes + g.partial_bytes + g.carry_bytes + g.trig_bytes + record;
+  if (!have_saved) s += g.wpack_bytes;
+  // (the cluster BPTT's scratch area is asked for wherever its shape applies, switched on or not)
+  if (ring_cluster_applicable(g.N, g.k)) s += ring_cluster_bptt_workspace_bytes(g.nbt);
+  return s;
+}
+
+size_t ringattr_bwd_workspace_bytes_for(int N, int a_dim, int seq_len, int batch_size, int have_saved, int want_grad_A) {
+  Geo g;
+  if (make_geo(N, a_dim, seq_len, batch_size, g) != RINGATTR_OK) return 0;
+  // (whichever family runs: a switch in the environment may change that between the query and the call)
+  const size_t s = bwd_bytes(g, have_saved != 0, false, want_grad_A != 0), t = bwd_bytes(g, have_saved != 0, true, want_grad_A != 0);
+  return s > t ? s : t;
+}
 
 size_t ringattr_bwd_workspace_bytes(int N, int a_dim, int seq_len, int batch_size, int have_saved) {
   Geo g;
   if (make_geo(N, a_dim, seq_len, batch_size, g) != RINGATTR_OK) return 0;
-  size_t s = g.wpack_bytes + g.pair_bytes + g.partial_bytes + g.carry_bytes + g.trig_bytes;
-  if (!have_saved) s += g.wpack_bytes + g.side_bytes + g.pair_bytes;
-  // (the cluster BPTT's scratch area is asked for wherever its shape applies, switched on or not)
-  if (ring_cluster_applicable(N, a_dim)) s += ring_cluster_bptt_workspace_bytes(g.nbt);
-  return s + team_area(N, a_dim, seq_len, batch_size);
+  const size_t a = ringattr_bwd_workspace_bytes_for(N, a_dim, seq_len, batch_size, have_saved, 0);
+  const size_t b = ringattr_bwd_workspace_bytes_for(N, a_dim, seq_len, batch_size, have_saved, 1);
+  return a > b ? a : b;
 }
 
 // loss_stats != null: the forward kernel that can do so also leaves the loss head's per-row sums there; *stats_done
@@ -400,39 +422,40 @@ static int bwd_impl(const char* who, const void* grad_output, const void* loss_w
       !aligned16(r_init) || !aligned16(grad_Wa) || !aligned16(grad_Wo) || !aligned16(saved) ||
       !aligned16(grad_r_init) || !aligned16(grad_A) || !aligned16(workspace))
     return fail(RINGATTR_ERR_INVALID, "%s: every pointer must be 16-byte aligned", who);
-  const size_t need = ringattr_bwd_workspace_bytes(N, a_dim, seq_len, batch_size, saved != nullptr);
+  const size_t need = bwd_bytes(g, saved != nullptr, team, grad_A != nullptr);
   if (!workspace || workspace_bytes < need)
     return fail(RINGATTR_ERR_WORKSPACE, "%s: workspace of %zu bytes needed, %zu given", who, need,
                 workspace ? workspace_bytes : (size_t)0);
-  if (team && ring_team_bptt_bytes(N, a_dim, seq_len, batch_size) == 0)
+  if (team && ring_team_bptt_bytes(N, a_dim, seq_len, batch_size, grad_A != nullptr) == 0)
     return fail(RINGATTR_ERR_INVALID, "%s: the saved buffer was filled by the team kernels, which RINGATTR_TEAM no longer asks for; run "
                 "forward and backward under the same setting", who);
   hipStream_t st = static_cast<hipStream_t>(stream);
 
   char* ws = (char*)workspace;
-  void* wb = ws;
-  ws += g.wpack_bytes;
-  __bf16* gfrag = (__bf16*)ws;
-  ws += g.pair_bytes;
-  ring_f32x4* partial = (ring_f32x4*)ws;
-  ws += g.partial_bytes;
-  float* carry = g.carry_bytes ? (float*)ws : nullptr;
-  ws += g.carry_bytes;
-  float* trig = g.trig_bytes ? (float*)ws : nullptr;
-  ws += g.trig_bytes;
-
-  void* const team_ws = (char*)workspace + need - team_area(N, a_dim, seq_len, batch_size);
+  auto take = [&ws](size_t bytes) {
+    char* const p = ws;
+    ws += bytes;
+    return p;
+  };
+  void* wb = team ? nullptr : take(g.wpack_bytes);
+  __bf16* gfrag = (__bf16*)take(g.pair_bytes);
+  ring_f32x4* partial = team ? nullptr : (ring_f32x4*)take(g.partial_bytes);
+  float* carry = !team && g.carry_bytes ? (float*)take(g.carry_bytes) : nullptr;
+  float* trig = !team && g.trig_bytes ? (float*)take(g.trig_bytes) : nullptr;
+  void* team_ws = nullptr;
+  if (team) {
+    team_ws = (char*)workspace + need - team_shared_bytes(g, saved != nullptr, grad_A != nullptr);
+    partial = (ring_f32x4*)team_ws;
+  }
   const _Float16* dfrag;
   const __bf16* rfrag;
   if (saved) {
     dfrag = (const _Float16*)saved;
     rfrag = (const __bf16*)((const char*)saved + g.side_bytes);
   } else {
-    void* wf = ws;
-    ws += g.wpack_bytes;
-    _Float16* d = (_Float16*)ws;
-    ws += g.side_bytes;
-    __bf16* r = (__bf16*)ws;
+    void* wf = team ? team_ws : take(g.wpack_bytes);
+    _Float16* d = (_Float16*)take(g.side_bytes);
+    __bf16* r = (__bf16*)take(g.pair_bytes);
     const bool res = team ? ring_res256_applicable(N, a_dim) : ring_uses_resident(N, a_dim);
     hipError_t e = ring_launch_pack((const float*)Wo, (const float*)Wa, wf, N, a_dim, g.NC, 0, team ? 3 : (res ? 1 : 0), res ? J1 : 1.f,
                                     res ? J0 : 0.f, st);
@@ -463,7 +486,7 @@ static int bwd_impl(const char* who, const void* grad_output, const void* loss_w
   // transposed copy, in its column order with J1 * Wo^T + J0 as matrix 0; its scratch area is the workspace's tail.
   const bool bptt_cluster = !team && !step_family && !grad_A && !loss_workspace && ring_uses_cluster_bptt(N, a_dim, batch_size, seq_len) &&
                             !ring_uses_resident(N, a_dim);
-  void* const cluster_ws = bptt_cluster ? (char*)team_ws - ring_cluster_bptt_workspace_bytes(g.nbt) : nullptr;
+  void* const cluster_ws = bptt_cluster ? (char*)workspace + need - ring_cluster_bptt_workspace_bytes(g.nbt) : nullptr;
   // the weight-resident BPTT kernel takes J1 * Wo + J0 in the transposed Wo fragments
   const bool resident = ring_uses_resident(N, a_dim);
   const bool bptt_resident = resident;

@@ -204,7 +204,7 @@ class _Bwd:
             if loss_workspace.dtype != torch.uint8 or loss_workspace.numel() < need or loss_workspace.device != dev:
                 raise ValueError(f"loss_workspace must be a uint8 tensor of at least {need} bytes on {dev}")
             with torch.cuda.device(dev):
-                ws_bytes = lib.ringattr_bwd_workspace_bytes(N, k, T, B, 1 if saved is not None else 0)
+                ws_bytes = lib.ringattr_bwd_workspace_bytes_for(N, k, T, B, int(saved is not None), int(grad_A is not None))
                 if ws_bytes == 0:
                     _lib.check(1)
                 ws = _workspace(ws_bytes, dev, stream)
@@ -215,7 +215,7 @@ class _Bwd:
             _lib.check(rc)
             return None
         with torch.cuda.device(dev):
-            ws_bytes = lib.ringattr_bwd_workspace_bytes(N, k, T, B, 1 if saved is not None else 0)
+            ws_bytes = lib.ringattr_bwd_workspace_bytes_for(N, k, T, B, int(saved is not None), int(grad_A is not None))
             if ws_bytes == 0:
                 _lib.check(1)
             ws = _workspace(ws_bytes, dev, stream)

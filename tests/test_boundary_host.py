@@ -48,6 +48,24 @@ def test_size_queries():
     assert lib.ringattr_saved_bytes(2049, 2, 7, 64) == 0 and "2048" in _lib.last_error()
 
 
+def test_backward_workspace_holds_no_team_scratch_that_is_not_used():
+    """Exchange areas and dL/dA shares of the team kernels are asked for only where these kernels run, the shares only
+    with grad_A, and they lie where the split-K partials go afterwards: without grad_A a backward takes no more than the
+    streaming and step-per-launch kernels need for the same shape (bytes below: packed weights, operand copy of g,
+    partials, and without a record the rebuilt one and its weights)."""
+    lib = _lib.load()
+    for (N, k, T, B, saved), size in {(512, 2, 512, 8192, 1): 4430926848, (256, 16, 120, 4096, 1): 547489792,
+                                      (500, 12, 300, 4096, 1): 1499992064}.items():      # not team shapes
+        assert lib.ringattr_bwd_workspace_bytes(N, k, T, B, saved) == size
+    for (N, k, T, B, saved), size in {(360, 3, 75, 100, 1): 78385152, (512, 16, 60, 256, 1): 310906880,
+                                      (240, 16, 512, 1024, 1): 557975552, (1024, 2, 120, 2048, 1): 576724992,
+                                      (120, 16, 512, 8192, 1): 1170112512, (360, 2, 60, 1024, 0): 246419456,
+                                      (700, 2, 60, 500, 0): 255860736}.items():
+        without, with_a = (lib.ringattr_bwd_workspace_bytes_for(N, k, T, B, saved, a) for a in (0, 1))
+        assert without <= size, (N, k, T, B)
+        assert lib.ringattr_bwd_workspace_bytes(N, k, T, B, saved) == max(without, with_a)
+
+
 def test_c_abi_rejects_bad_arguments_with_codes_not_exit():
     lib = _lib.load()
     buf = (ctypes.c_char * 4096)()

@@ -116,6 +116,38 @@ def test_backward_without_a_record_differentiates_the_history_it_is_given(B, T, 
     assert "ring_team_rebuild" in names["rebuild_saved"] and "ring_team_bptt" in names["bptt"], names
 
 
+@pytest.mark.parametrize("B,T,k,N", [(40, 7, 2, 120), (20, 6, 16, 100), (100, 5, 3, 360), (300, 4, 2, 700)])
+def test_backward_stays_inside_the_workspace_it_asks_for(B, T, k, N, gpu_device, teams):
+    """The areas that take turns in the workspace, against the workspace's end and against each other: same bits as with
+    room to spare, nothing written behind the end."""
+    from rnn_train_ring_attractor_amd import _lib, rnn_cuda
+    print(f"[case] team workspace B={B} T={T} k={k} N={N}", flush=True)
+    lib = _lib.load()
+    p = make_problem(83, B, T, k, N, action="dense")
+    A, Wa, Wo, r0, G = (_t(p[x], gpu_device) for x in ("A", "Wa", "Wo", "r0", "G"))
+    hist = torch.empty(T, B, N, device=gpu_device)
+    record = torch.empty(rnn_cuda.saved_nbytes(N, k, T, B), dtype=torch.uint8, device=gpu_device)
+    rnn_cuda.fwd_cuda.fwd(A=A, Wa=Wa, J0=-0.01, J1=0.6, Wo=Wo, r_init=r0, bump_history=hist, alpha=0.15, activation_type=1, saved=record)
+    for saved in (record, None):
+        for ga in (False, True):
+            need = lib.ringattr_bwd_workspace_bytes_for(N, k, T, B, int(saved is not None), int(ga))
+
+            def bwd(space, nbytes):
+                out = [torch.full_like(x, float("nan")) for x in (Wa, Wo, r0)] + ([torch.full_like(A, float("nan"))] if ga else [])
+                ptr = lambda x: None if x is None else x.data_ptr()
+                rc = lib.ringattr_bwd(ptr(G), ptr(A), ptr(Wa), -0.01, 0.6, ptr(Wo), ptr(hist), ptr(r0), ptr(out[0]), ptr(out[1]), 0.15,
+                                      N, k, T, B, 1, 0, ptr(saved), ptr(out[3]) if ga else None, ptr(out[2]), ptr(space), nbytes,
+                                      torch.cuda.current_stream().cuda_stream)
+                torch.cuda.synchronize()
+                return rc, out
+
+            roomy = torch.zeros(2 * need + (1 << 20), dtype=torch.uint8, device=gpu_device)
+            tight = torch.full((need + 4096,), 0xAB, dtype=torch.uint8, device=gpu_device)
+            (rc0, want), (rc1, got) = bwd(roomy, roomy.numel()), bwd(tight, need)
+            assert rc0 == 0 and rc1 == 0 and "ring_team_bptt" in _lib.last_kernel_names()["bptt"]
+            assert all(torch.equal(x, y) for x, y in zip(got, want)) and bool((tight[need:] == 0xAB).all())
+
+
 @pytest.mark.parametrize("B,T,k,N", [(40, 5, 2, 120), (70, 6, 3, 361)])
 def test_fused_loss_head_on_teams(B, T, k, N, gpu_device, teams):
     """The objective's gradient formed inside the team BPTT against the loss head's own backward through the plain one."""
