@@ -111,27 +111,28 @@ static bool forced() {
   return v && v[0] == '1';
 }
 
-// whether a shape is left to the weight-resident kernels
-static bool resident_only(int N, int k, int B) { return ring_res256_applicable(N, k) && ((N == 256 && B % 16 == 0) || B > 256); }
-
 // Where teams run (us per time step, measured with T = 60, gelu; forward for inference / forward + backward):
 //   N = 120, a_dim 2:  B = 64: 2.5 -> 0.9 / 5.8 -> 2.3    B = 4096: 2.7 -> 1.9 / 9.6 -> 8.0
 //   N = 360, a_dim 2:  B = 64: 8.2 -> 1.5 / 30.6 -> 3.4   B = 1024: 12.9 -> 3.3 / 31.9 -> 7.8   B = 4096: 15.6 -> 8.0 / 37 -> 23
 //   N = 512, a_dim 2:  B = 64: 8.9 -> 1.6 / 29.1 -> 3.7   B = 2048: 14.3 -> 5.5 / 32.4 -> 14.8
 //   N = 1024, a_dim 2: B = 64: 17.8 -> 3.3 / 43 -> 6.9    B = 2048: 40 -> 19 / 104 -> 50
 // against the streaming and step-per-launch kernels.  The exceptions:
-//   * the weight-resident kernels (N = 256, a_dim 2, whole tiles) take 1.5 us per step at any batch up to 4096 rows.
-//     They keep that shape at every batch, also below 257 rows where teams are faster: a slice of a batch reproduces its
-//     rows bit for bit, and the two families sum in a different order.  On ragged shapes (128 < N < 256, or a last tile
-//     that is not full) their masked variants are slower and teams take the batches up to 256 rows.  The rule does not
-//     ask whether a record is wanted: a history is the same with and without one;
+//   * 128 < N <= 256 with two channels belongs to the weight-resident kernels at every batch, whole tiles or not, also
+//     where teams are faster (N = 256, B = 1: 1.6 against 1.1 us per step forward; N = 200, B = 64, forward and backward:
+//     4.9 against 3.0), because they are far ahead on large batches (N = 200, B = 4096: 7.4 against 10.5) and a slice of a
+//     batch has to reproduce its rows bit for bit: the two families sum in a different order, so one of them has to have
+//     all batches;
 //   * with many tiles per team (more than eight at N <= 512) a compute unit's epilogue work is what bounds a step, and
-//     the kernels that have a batch tile to themselves, or the N = 512 clusters, are as fast or faster.
+//     the kernels that have a batch tile to themselves, or the N = 512 clusters, are faster (N = 360, B = 6000, forward
+//     and backward: 49 against 43 us per step with nine tiles, B = 8192: 53 against 68 with thirteen; N = 512, B = 4608:
+//     46 against 37, B = 6016: 49 against 54).  Rows reproduce between batches on the same side of this line: members of
+//     any width sum a row alike.
+// The rule does not ask whether a record is wanted: a history is the same with and without one.
 static bool team_shape(int N, int k, int T, int B) {
-  if (resident_only(N, k, B) && !forced()) return false;
+  if (ring_res256_applicable(N, k) && !forced()) return false;
   const RingTeamPlan f = ring_team_plan(N, k, T, B, false, false);
   if (!f.ok || !ring_team_plan(N, k, T, B, true, true).ok) return false;
-  return forced() || ring_res256_applicable(N, k) || N > 512 || f.nt <= 8;
+  return forced() || N > 512 || f.nt <= 8;
 }
 
 bool ring_uses_team(int N, int k, int T, int B) {

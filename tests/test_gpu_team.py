@@ -116,6 +116,41 @@ def test_backward_without_a_record_differentiates_the_history_it_is_given(B, T, 
     assert "ring_team_rebuild" in names["rebuild_saved"] and "ring_team_bptt" in names["bptt"], names
 
 
+# the kernels of 128 < N <= 256 with two channels, whole and ragged widths; teams with members of different width per batch
+@pytest.mark.parametrize("N,k,B,kernel", [(256, 2, 4096, "res256"), (200, 2, 1500, "res256"), (120, 2, 4096, "team"),
+                                          (360, 2, 2048, "team"), (333, 3, 1000, "team"), (700, 2, 1024, "team")])
+def test_rows_do_not_depend_on_the_batch_they_are_in(N, k, B, kernel, gpu_device, teams, monkeypatch):
+    """A slice of a batch run alone reproduces its rows of the full batch bit for bit, whatever its size.  (At N = 256 the
+    weight-resident BPTT of ragged batches is another variant than that of whole tiles: dL/dr_init is compared there for
+    whole tiles.)"""
+    from rnn_train_ring_attractor_amd import ring_rnn_cuda_func, _lib
+    monkeypatch.delenv("RINGATTR_TEAM")
+    T = 9
+    print(f"[case] rows across batches N={N} k={k} B={B}", flush=True)
+    p = make_problem(84, B, T, k, N, action="dense")
+    G = torch.randn(T, B, N, device=gpu_device, generator=torch.Generator(device=gpu_device).manual_seed(5))
+    Wa, Wo = _t(p["Wa"], gpu_device).requires_grad_(True), _t(p["Wo"], gpu_device).requires_grad_(True)
+
+    def run(rows):
+        A, r0 = _t(p["A"][rows], gpu_device), _t(p["r0"][rows], gpu_device).requires_grad_(True)
+        hist = ring_rnn_cuda_func(A, Wa, -1.0 / N, 0.6, Wo, r0, 0.15, "gelu")
+        hist.backward(G[:, rows].contiguous())
+        names = _lib.last_kernel_names()
+        assert kernel in names["fwd"] and kernel in names["bptt"], names
+        with torch.no_grad():
+            again = ring_rnn_cuda_func(A, Wa, -1.0 / N, 0.6, Wo, r0, 0.15, "gelu")
+        if kernel in _lib.last_kernel_names()["fwd"]:
+            assert torch.equal(again, hist)
+        return hist.detach(), r0.grad
+
+    full = run(slice(0, B))
+    for lo, n in ((5, 1), (16, 16), (3, 100), (128, 128), (0, B // 2), (0, 1000 if B > 1000 else 500)):
+        part = run(slice(lo, lo + n))
+        assert torch.equal(part[0], full[0][:, lo:lo + n]), (lo, n)
+        if N != 256 or n % 16 == 0:
+            assert torch.equal(part[1], full[1][lo:lo + n]), (lo, n)
+
+
 @pytest.mark.parametrize("B,T,k,N", [(40, 7, 2, 120), (20, 6, 16, 100), (100, 5, 3, 360), (300, 4, 2, 700)])
 def test_backward_stays_inside_the_workspace_it_asks_for(B, T, k, N, gpu_device, teams):
     """The areas that take turns in the workspace, against the workspace's end and against each other: same bits as with
