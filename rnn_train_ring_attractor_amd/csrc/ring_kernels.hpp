@@ -239,6 +239,7 @@ struct RingTeamArgs {
   int N, k, T, B, nbt, KC, G, nteams, nt, slots, cts, transposed, spin_max;
   int gather_ticks;      // how long the members of a team wait for each other, in 10 ns (negative: not at all)
   int c16, mr, wk;       // the shape, for the single workgroups that take over
+  int rows;              // non-zero: one wave sums the whole contraction, chunks in the order of rows_chunk (ring_team_rows.hip)
 };
 struct RingTeamShape { int kpw, c16, mr, wk, lds_mats, grid; };
 struct RingTeamPlan {
@@ -255,6 +256,12 @@ size_t ring_team_bptt_bytes(int N, int k, int T, int B, bool ga);
 // J1 * Wo + J0 as one operand (folded) or kept apart; `ws` is ring_team_fwd_bytes / ring_team_bptt_bytes large
 hipError_t ring_team_fwd(const RingFwdArgs& a, const float* Wo, const float* Wa, bool folded, int cts, void* ws, hipStream_t st);
 hipError_t ring_team_bptt(const RingBpttArgs& a, const float* Wo, const float* Wa, bool folded, int cts, void* ws, hipStream_t st);
+// small batches of 128 < N <= 256 with two channels, without a record (ring_team_rows.hip)
+RingTeamPlan ring_team_rows_plan(int N, int k, int B);
+bool ring_uses_team_rows(int N, int k, int B);
+size_t ring_team_rows_bytes(int N, int k, int B);
+hipError_t ring_team_rows(const RingFwdArgs& a, const float* Wo, const float* Wa, void* ws, hipStream_t st);
+hipError_t ring_launch_team_rows(const RingFwdArgs& a, const RingTeamArgs& c, const RingTeamShape& sh, hipStream_t st);
 // the record from a.hist; a.Wpack: forward fragments in order 3, with J1 * Wo + J0 as matrix 0 when folded
 hipError_t ring_team_rebuild(const RingFwdArgs& a, bool folded, int cts, hipStream_t st);
 hipError_t ring_launch_team_rebuild(const RingFwdArgs& a, const RingTeamArgs& c, int wk, hipStream_t st);
@@ -267,5 +274,6 @@ hipError_t ring_launch_team_solo_bptt(const RingBpttArgs& a, const RingTeamArgs&
 hipError_t ring_cluster_host_err(int** dev);              // the error word both exchange families report through
 // the same under the profiling slots
 hipError_t ring_run_team_fwd(const RingFwdArgs& a, const float* Wo, const float* Wa, bool folded, int cts, void* ws, hipStream_t st);
+hipError_t ring_run_team_rows(const RingFwdArgs& a, const float* Wo, const float* Wa, void* ws, hipStream_t st);
 hipError_t ring_run_team_rebuild(const RingFwdArgs& a, bool folded, int cts, hipStream_t st);
 hipError_t ring_run_team_bptt(const RingBpttArgs& a, const float* Wo, const float* Wa, bool folded, int cts, void* ws, hipStream_t st);

@@ -118,10 +118,10 @@ static bool forced() {
 //   N = 1024, a_dim 2: B = 64: 17.8 -> 3.3 / 43 -> 6.9    B = 2048: 40 -> 19 / 104 -> 50
 // against the streaming and step-per-launch kernels.  The exceptions:
 //   * 128 < N <= 256 with two channels belongs to the weight-resident kernels at every batch, whole tiles or not, also
-//     where teams are faster (N = 256, B = 1: 1.6 against 1.1 us per step forward; N = 200, B = 64, forward and backward:
-//     4.9 against 3.0), because they are far ahead on large batches (N = 200, B = 4096: 7.4 against 10.5) and a slice of a
-//     batch has to reproduce its rows bit for bit: the two families sum in a different order, so one of them has to have
-//     all batches;
+//     where teams are faster (N = 200, B = 64, forward and backward: 4.9 against 3.0), because they are far ahead on large
+//     batches (N = 200, B = 4096: 7.4 against 10.5) and a slice of a batch has to reproduce its rows bit for bit: the two
+//     families sum in a different order, so one of them has to have all batches (small ones without a record run on
+//     teams that sum in the weight-resident order: ring_team_rows.hip);
 //   * with many tiles per team (more than eight at N <= 512) a compute unit's epilogue work is what bounds a step, and
 //     the kernels that have a batch tile to themselves, or the N = 512 clusters, are faster (N = 360, B = 6000, forward
 //     and backward: 49 against 43 us per step with nine tiles, B = 8192: 53 against 68 with thirteen; N = 512, B = 4608:
@@ -135,14 +135,23 @@ static bool team_shape(int N, int k, int T, int B) {
   return forced() || N > 512 || f.nt <= 8;
 }
 
-bool ring_uses_team(int N, int k, int T, int B) {
+static bool teams_allowed() {
   const char* v = getenv("RINGATTR_TEAM");
   if ((v && v[0] == '0') || ring_cluster_error()) return false;
   // a switch that asks for one of the other families by name is obeyed
   for (const char* name : {"RINGATTR_STREAMING", "RINGATTR_ROW_TILES", "RINGATTR_BLOCK", "RINGATTR_WIDE", "RINGATTR_SPLIT_FORWARD",
                            "RINGATTR_LDS_WEIGHTS", "RINGATTR_BLOCK_SHAPE", "RINGATTR_CLUSTER", "RINGATTR_CLUSTER_BPTT"})
     if (getenv(name)) return false;
-  return device_cus() == XCDS * CUS_PER_XCD && team_shape(N, k, T, B);
+  return device_cus() == XCDS * CUS_PER_XCD;
+}
+
+bool ring_uses_team(int N, int k, int T, int B) { return teams_allowed() && team_shape(N, k, T, B); }
+
+// Same bits as the weight-resident forward, so the batch may decide: wherever every batch tile gets a team.
+bool ring_uses_team_rows(int N, int k, int B) { return !forced() && teams_allowed() && ring_team_rows_plan(N, k, B).ok; }
+size_t ring_team_rows_bytes(int N, int k, int B) {
+  const RingTeamPlan p = ring_team_rows_plan(N, k, B);
+  return p.ok ? p.xchg_bytes + p.gather_bytes : 0;
 }
 
 // Scratch of one launch; none where no call of this shape comes here.
@@ -196,6 +205,7 @@ static hipError_t team_args(const RingTeamPlan& p, const float* Wo, const float*
   c.c16 = p.shape.c16;
   c.mr = p.shape.mr;
   c.wk = p.shape.wk;
+  c.rows = 0;
   const unsigned nx = (unsigned)(p.xchg_bytes / 16), n = (unsigned)((p.xchg_bytes + p.gather_bytes) / 16);
   hipLaunchKernelGGL(ring_team_fill_kernel, dim3(std::min(1024u, (n + 255) / 256)), dim3(256), 0, st, reinterpret_cast<u32x4*>(ws), nx, n);
   return hipGetLastError();
@@ -208,6 +218,17 @@ hipError_t ring_team_fwd(const RingFwdArgs& a, const float* Wo, const float* Wa,
   hipError_t e = team_args(p, Wo, Wa, a.A, a.J0, a.J1, folded, a.N, a.k, a.T, a.B, cts, false, ws, c, st);
   if (e != hipSuccess) return e;
   e = ring_launch_team_fwd(a, c, p.shape, st);
+  return e == hipSuccess ? ring_launch_team_solo_fwd(a, c, st) : e;
+}
+
+hipError_t ring_team_rows(const RingFwdArgs& a, const float* Wo, const float* Wa, void* ws, hipStream_t st) {
+  const RingTeamPlan p = ring_team_rows_plan(a.N, a.k, a.B);
+  if (!p.ok || !ws || !a.hist || a.dfrag || a.rfrag) return hipErrorInvalidValue;
+  RingTeamArgs c;
+  hipError_t e = team_args(p, Wo, Wa, a.A, a.J0, a.J1, true, a.N, a.k, a.T, a.B, 0, false, ws, c, st);
+  if (e != hipSuccess) return e;
+  c.wk = c.rows = 1;
+  e = ring_launch_team_rows(a, c, p.shape, st);
   return e == hipSuccess ? ring_launch_team_solo_fwd(a, c, st) : e;
 }
 

@@ -169,6 +169,9 @@ struct AuxMap {
   }
 };
 
+// K chunk number i in the order of the weight-resident forward's contraction (split_k_neuron): even ones, odd ones.
+__host__ __device__ __forceinline__ int rows_chunk(int i) { return 2 * (i & 3) + (i >> 2); }
+
 template <int C16, int WK>
 constexpr size_t share_floats() { return (size_t)2 * WK * C16 * AuxMap<C16>::SHARE; }
 

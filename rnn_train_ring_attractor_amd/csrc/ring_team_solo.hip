@@ -292,7 +292,13 @@ __device__ __forceinline__ void solo_products(const RingTeamArgs& c, const SoloO
   for (int cw = 0; cw < c.wk && cw < c.KC; ++cw) {
     f32x4 acc[SOLO_C16];
     float sum = 0.f;
-    for (int kc = cw; kc < c.KC; kc += c.wk) sum += o.rs[kc * 64 + lane];
+    auto chunks = [&](auto&& use) {              // the wave's K chunks in its order
+      for (int i = 0; i < (c.rows ? 8 : c.KC); i += c.wk) {
+        const int kc = c.rows ? rows_chunk(i) : cw + i;
+        if (kc < c.KC) use(kc);
+      }
+    };
+    chunks([&](int kc) { sum += o.rs[kc * 64 + lane]; });
     const float j0r = c.J0 * sum_bits45(sum);
     for (int m = 0; m <= c.k; ++m) {
       const float g = m == 0 ? 0.f : gates[(m - 1) * 16 + b];
@@ -302,7 +308,7 @@ __device__ __forceinline__ void solo_products(const RingTeamArgs& c, const SoloO
       for (int cc = 0; cc < SOLO_C16; ++cc) {
         if (cc >= c.c16) continue;
         f32x4 P = {0.f, 0.f, 0.f, 0.f};
-        for (int kc = cw; kc < c.KC; kc += c.wk) P = mfma16(solo_weight<TR>(c, m, mem * c.c16 + cc, kc, lane), o.x[kc * 64 + lane], P);
+        chunks([&](int kc) { P = mfma16(solo_weight<TR>(c, m, mem * c.c16 + cc, kc, lane), o.x[kc * 64 + lane], P); });
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
           acc[cc][i] = m == 0 ? fmaf(c.J1, P[i], j0r) : fmaf(g, P[i], acc[cc][i]);

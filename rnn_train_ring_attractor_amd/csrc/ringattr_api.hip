@@ -178,8 +178,10 @@ size_t ringattr_fwd_workspace_bytes(int N, int a_dim, int seq_len, int batch_siz
   // (the cluster forward's exchange area is asked for wherever its shape applies, switched on or not)
   const size_t packed = g.wpack_bytes + (ring_cluster_applicable(N, a_dim) ? ring_cluster_workspace_bytes(g.nbt) : 0) +
                         (ring_panel_applicable(g.NC, a_dim) ? align_up(ring_panel_workspace_bytes(g.NC, g.nbt)) : 0);
-  const size_t team = ring_team_fwd_bytes(N, a_dim, seq_len, batch_size);   // (used instead of the packed weights)
-  return packed > team ? packed : team;
+  // (used instead of the packed weights)
+  const size_t team = ring_team_fwd_bytes(N, a_dim, seq_len, batch_size), rows = ring_team_rows_bytes(N, a_dim, batch_size);
+  const size_t most = team > rows ? team : rows;
+  return packed > most ? packed : most;
 }
 
 // A backward's workspace.  Most families: packed weights, operand copy of g, split-K partials, the small areas, and
@@ -303,6 +305,14 @@ static int fwd_impl(const void* A, const void* Wa, float J0, float J1, const voi
     if (saved) saved_note_put(SavedNote{saved, 4, N, a_dim, seq_len, batch_size, J0, J1, Wo, Wa});
     if (stats_done) *stats_done = false;
     const hipError_t e = ring_run_team_fwd(a, (const float*)Wo, (const float*)Wa, ring_res256_applicable(N, a_dim), 4 * g.NC, workspace, st);
+    if (e != hipSuccess) return hip_fail(e, "team forward launch");
+    return RINGATTR_OK;
+  }
+
+  // (the loss head's row sums come from the weight-resident forward, whatever the batch)
+  if (!saved && !loss_stats && ring_uses_team_rows(N, a_dim, batch_size) && workspace_bytes >= ring_team_rows_bytes(N, a_dim, batch_size)) {
+    const RingFwdArgs a = fwd_args(A, nullptr, r_init, bump_history, nullptr, g, J0, J1, alpha, activation_type);
+    const hipError_t e = ring_run_team_rows(a, (const float*)Wo, (const float*)Wa, workspace, st);
     if (e != hipSuccess) return hip_fail(e, "team forward launch");
     return RINGATTR_OK;
   }

@@ -116,6 +116,34 @@ def test_backward_without_a_record_differentiates_the_history_it_is_given(B, T, 
     assert "ring_team_rebuild" in names["rebuild_saved"] and "ring_team_bptt" in names["bptt"], names
 
 
+@pytest.mark.parametrize("N,B,T,act", [(256, 1, 100, "gelu"), (256, 512, 21, "tanh"), (256, 100, 2, "relu"), (129, 16, 40, "silu"),
+                                       (131, 9, 1, "gelu"), (200, 257, 33, "gelu"), (250, 300, 12, "tanh"), (222, 64, 17, "relu")])
+def test_small_batches_without_a_record_have_the_weight_resident_forwards_bits(N, B, T, act, gpu_device, teams, monkeypatch):
+    from rnn_train_ring_attractor_amd import rnn_cuda, _lib
+    print(f"[case] team rows N={N} B={B} T={T} {act}", flush=True)
+    p = make_problem(85, B, T, 2, N, action="dense")
+    A, Wa, Wo, r0 = (_t(p[x], gpu_device) for x in ("A", "Wa", "Wo", "r0"))
+
+    def fwd(kernel, **env):
+        monkeypatch.delenv("RINGATTR_TEAM", raising=False)
+        for name, value in env.items():
+            monkeypatch.setenv(name, value)
+        out = torch.full((T, B, N), float("nan"), device=gpu_device)
+        rnn_cuda.fwd_cuda.fwd(A=A, Wa=Wa, J0=-0.05, J1=0.7, Wo=Wo, r_init=r0, bump_history=out, alpha=0.15, activation_type=ACTS[act])
+        torch.cuda.synchronize()
+        for name in env:
+            monkeypatch.delenv(name)
+        assert kernel in _lib.last_kernel_names()["fwd"]
+        return out
+
+    want = fwd("ring_fwd_res256", RINGATTR_TEAM="0")
+    assert torch.isfinite(want).all()
+    for wait_us in (None, "-1", "0"):
+        for _ in range(3):
+            got = fwd("ring_team_rows", **({} if wait_us is None else {"RINGATTR_TEAM_GATHER_US": wait_us}))
+            assert torch.equal(got, want), wait_us
+
+
 # the kernels of 128 < N <= 256 with two channels, whole and ragged widths; teams with members of different width per batch
 @pytest.mark.parametrize("N,k,B,kernel", [(256, 2, 4096, "res256"), (200, 2, 1500, "res256"), (120, 2, 4096, "team"),
                                           (360, 2, 2048, "team"), (333, 3, 1000, "team"), (700, 2, 1024, "team")])
@@ -138,9 +166,7 @@ def test_rows_do_not_depend_on_the_batch_they_are_in(N, k, B, kernel, gpu_device
         names = _lib.last_kernel_names()
         assert kernel in names["fwd"] and kernel in names["bptt"], names
         with torch.no_grad():
-            again = ring_rnn_cuda_func(A, Wa, -1.0 / N, 0.6, Wo, r0, 0.15, "gelu")
-        if kernel in _lib.last_kernel_names()["fwd"]:
-            assert torch.equal(again, hist)
+            assert torch.equal(ring_rnn_cuda_func(A, Wa, -1.0 / N, 0.6, Wo, r0, 0.15, "gelu"), hist)     # and without a record
         return hist.detach(), r0.grad
 
     full = run(slice(0, B))
