@@ -25,9 +25,13 @@
 // state s - 1 is refilled by its owner in the epilogue of step s: by then every member has published state s, i.e.
 // has read all of state s - 1.  It is written again as state s + slots - 1; a reader polls for that only after it has
 // read state s + slots - 2 from the same owner, which must have been published after the refill reached L2.  It was:
-// an auxiliary wave waits for the loads of an item within three items of issuing them, vector-memory operations
-// complete in order, and three items are fewer than slots - 3 rounds (8 slots with one tile per team, 6 with two or
-// three, 4 from four tiles up).
+// an auxiliary wave issues the refill of an item (step s) before the loads of the next one, waits for those in the third
+// item after the refill's, before it publishes anything there, and vector-memory operations complete in order.  In
+// rounds of the team's tiles that third item is at most step s + 3 with one tile per team, s + 2 with two, s + 1 from
+// three up, and what it publishes is state s + 4, s + 3 or s + 2 at the latest: no later than state s + slots - 2, the
+// one that has to come behind the refill, with 8 slots where every team has one tile, 6 where the fullest have two or
+// three and others one less, 4 from four tiles up (three in some).  Six slots with one tile and four with three are
+// exact: one slot less would not do.
 // Besides the bf16 state a chunk carries fp32 row sums of the unrounded state (groups of eight neurons, always summed in
 // the order of row_sum8, so that a row's bits do not depend on how wide the members are) for the J0 term.
 //

@@ -209,6 +209,36 @@ def test_backward_stays_inside_the_workspace_it_asks_for(B, T, k, N, gpu_device,
             assert all(torch.equal(x, y) for x, y in zip(got, want)) and bool((tight[need:] == 0xAB).all())
 
 
+# Sequences that go through the exchange slots many times: one tile per team (8 slots), teams of one and two tiles and of
+# two (6 slots), of three and four (4 slots, the fullest and the others), sixteen; the sizes of ordinary calls among them
+@pytest.mark.parametrize("B,T,k,N", [(64, 120, 2, 120), (100, 75, 3, 360), (150, 50, 2, 600), (1000, 45, 2, 360), (256, 20, 16, 512),
+                                     (400, 44, 2, 1000), (2048, 120, 2, 1024)])
+def test_slots_are_reused_many_times(B, T, k, N, gpu_device, teams, monkeypatch):
+    """A slot of the exchange area is emptied and published again every 8, 6 or 4 steps.  Single workgroups, which exchange
+    nothing, give the same bits; row-wise outputs are held to the fp64 oracle on rows of the first tile, the last one and
+    one of a team with fewest tiles."""
+    print(f"[case] team slots B={B} T={T} k={k} N={N}", flush=True)
+    J0, J1 = -1.0 / N, 0.6
+    p = make_problem(86, B, T, k, N, action="dense")
+    # (dL/dA of the largest shape would need a share per member of all its steps)
+    got = _run(p, "tanh", J0, J1, gpu_device, ga=B < 2048)
+    monkeypatch.setenv("RINGATTR_TEAM_GATHER_US", "-1")
+    alone = _run(p, "tanh", J0, J1, gpu_device, ga=B < 2048)
+    monkeypatch.delenv("RINGATTR_TEAM_GATHER_US")
+    assert all(torch.equal(got[x], alone[x]) for x in got), [x for x in got if not torch.equal(got[x], alone[x])]
+    del alone
+    again = _run(p, "tanh", J0, J1, gpu_device, ga=B < 2048)
+    assert all(torch.equal(got[x], again[x]) for x in got)
+    del again
+    rows = np.array(sorted({0, 7, B // 2, B - 1} | {r for r in (16 * 7 + 3, 16 * 15 + 9, 16 * 39 + 1) if r < B}))
+    ref, _ = O.forward_dense(p["A"][rows], p["Wa"], J0, J1, p["Wo"], p["r0"][rows], 0.15, "tanh")
+    assert O.max_rel_err(got["hist"][:, torch.as_tensor(rows, device=gpu_device)].cpu().numpy(), ref) <= TRAJ_TOL
+    g = O.backward_dense(p["G"][:, rows], p["A"][rows], p["Wa"], J0, J1, p["Wo"], ref, p["r0"][rows], 0.15, "tanh")
+    for name in [x for x in ("grad_r_init", "grad_A") if x in got]:
+        x = got[name][torch.as_tensor(rows, device=gpu_device)].cpu().numpy()
+        assert O.cosine(x, g[name]) >= GRAD_COS and O.max_rel_err(x, g[name]) <= GRAD_TOL, name
+
+
 @pytest.mark.parametrize("B,T,k,N", [(40, 5, 2, 120), (70, 6, 3, 361)])
 def test_fused_loss_head_on_teams(B, T, k, N, gpu_device, teams):
     """The objective's gradient formed inside the team BPTT against the loss head's own backward through the plain one."""
