@@ -124,7 +124,7 @@ bool ring_uses_step_kernels(int N, int k, int NC, int nbt);
 
 // Step-per-launch forward without a saved record, wide rings (ring_panel.hip).
 bool ring_panel_applicable(int NC, int k);
-bool ring_uses_panel(int N, int k, int NC, int nbt);
+bool ring_uses_panel(int k, int NC, int nbt);
 size_t ring_panel_workspace_bytes(int NC, int nbt);
 hipError_t ring_launch_panel_fwd(const RingFwdArgs& a, int NC, hipStream_t st);
 

@@ -329,13 +329,12 @@ bool ring_panel_applicable(int NC, int k) { return NC >= 16 && NC % 8 == 0 && k 
 size_t ring_panel_workspace_bytes(int NC, int nbt) { return (size_t)nbt * 2 * NC * 1024 + (size_t)nbt * 16 * sizeof(float); }
 
 // RINGATTR_PANEL=0: never; a switch that asks for one of the other step-per-launch families is obeyed.
-bool ring_uses_panel(int N, int k, int NC, int nbt) {
+bool ring_uses_panel(int k, int NC, int nbt) {
   if (!ring_panel_applicable(NC, k)) return false;
   const char* v = getenv("RINGATTR_PANEL");
   if (v && v[0] == '0') return false;
   for (const char* name : {"RINGATTR_WIDE", "RINGATTR_BLOCK", "RINGATTR_BLOCK_SHAPE"})
     if (getenv(name)) return false;
-  (void)N;
   return ring_panel_workspace_bytes(NC, nbt) < ((size_t)1 << 30);   // (32-bit offsets; the weights are 0.6 GB at most)
 }
 

@@ -710,14 +710,16 @@ __device__ __forceinline__ bool team_coords(const RingTeamArgs& c, int& team, in
 
 }  // namespace
 
-// Shapes that are built: K chunks per compute wave, column tiles per member, matrices in registers, compute waves.
-// (kpw * wk chunks cover the contraction; c16 * kpw * mr weight fragments of four registers per wave.)
-#define RING_TEAM_SHAPES(X)                                                     \
-  X(1, 1, 3, 4) X(1, 2, 3, 4) X(1, 4, 3, 4)                                     \
-  X(1, 1, 3, 8) X(1, 2, 3, 8) X(1, 4, 3, 8) X(1, 1, 9, 8) X(1, 2, 13, 8)        \
-  X(2, 1, 3, 8) X(2, 2, 3, 8) X(2, 4, 3, 8) X(2, 1, 9, 8) X(2, 1, 13, 8)        \
-  X(3, 1, 3, 8) X(3, 2, 3, 8) X(4, 1, 3, 8) X(4, 2, 3, 8)
-// (each once with all matrices in registers and once with further ones in LDS)
+// Shapes that are built: K chunks per compute wave, column tiles per member, matrices in registers, compute waves, and
+// whether also with further matrices in LDS.  (kpw * wk chunks cover the contraction; c16 * kpw * mr weight fragments of
+// four registers per wave.  Past N = 512 one column tile per member would make teams of more than an XCD's 32 compute
+// units; four at 256 < N <= 512 leave LDS room for a further matrix only up to N = 288, where two are as fast: N = 257,
+// a_dim 3, B = 1395, T = 60 forward 235 us with four, 233 with two.)
+#define RING_TEAM_SHAPES(X)                                                                              \
+  X(1, 1, 3, 4, true) X(1, 2, 3, 4, true) X(1, 4, 3, 4, true)                                            \
+  X(1, 1, 3, 8, true) X(1, 2, 3, 8, true) X(1, 4, 3, 8, true) X(1, 1, 9, 8, true) X(1, 2, 13, 8, true)   \
+  X(2, 1, 3, 8, true) X(2, 2, 3, 8, true) X(2, 4, 3, 8, false) X(2, 1, 9, 8, true) X(2, 1, 13, 8, true)  \
+  X(3, 2, 3, 8, true) X(4, 2, 3, 8, true)
 
 // Launches one team kernel.
 template <typename F>

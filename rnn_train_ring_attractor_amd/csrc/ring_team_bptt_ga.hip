@@ -9,10 +9,10 @@ hipError_t ring_launch_team_bptt_ga(const RingBpttArgs& a, const RingTeamArgs& c
                          [&](dim3 g, dim3 b, unsigned lds) {                                                          \
                            RING_LAUNCH((ring_team_bptt_kernel<KPW, C16, MR, WK, EX, GA>), g, b, lds, st, a, c);       \
                          })
-#define RING_TEAM_CASE(KPW, C16, MR, WK)                                                                              \
+#define RING_TEAM_CASE(KPW, C16, MR, WK, EX)                                                                          \
   if (sh.kpw == KPW && sh.c16 == C16 && sh.mr == MR && sh.wk == WK) {                                                 \
-    if (sh.lds_mats) RING_TEAM_RUN(KPW, C16, MR, WK, true);                                                           \
-    RING_TEAM_RUN(KPW, C16, MR, WK, false);                                                                           \
+    if (sh.lds_mats == 0) RING_TEAM_RUN(KPW, C16, MR, WK, false);                                                     \
+    if constexpr (EX) RING_TEAM_RUN(KPW, C16, MR, WK, true);                                                          \
   }
   RING_TEAM_SHAPES(RING_TEAM_CASE)
 #undef RING_TEAM_CASE

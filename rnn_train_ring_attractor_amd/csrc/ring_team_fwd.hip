@@ -121,10 +121,10 @@ hipError_t ring_launch_team_fwd(const RingFwdArgs& a, const RingTeamArgs& c, con
     case ACT_SILU: RING_TEAM_ACT(KPW, C16, MR, WK, EX, ACT_SILU);             \
     default: return hipErrorInvalidValue;                                     \
   }
-#define RING_TEAM_CASE(KPW, C16, MR, WK)                                      \
+#define RING_TEAM_CASE(KPW, C16, MR, WK, EX)                                  \
   if (sh.kpw == KPW && sh.c16 == C16 && sh.mr == MR && sh.wk == WK) {         \
-    if (sh.lds_mats) { RING_TEAM_ACTS(KPW, C16, MR, WK, true) }               \
-    else { RING_TEAM_ACTS(KPW, C16, MR, WK, false) }                          \
+    if (sh.lds_mats == 0) { RING_TEAM_ACTS(KPW, C16, MR, WK, false) }         \
+    if constexpr (EX) { RING_TEAM_ACTS(KPW, C16, MR, WK, true) }              \
   }
   RING_TEAM_SHAPES(RING_TEAM_CASE)
 #undef RING_TEAM_CASE

@@ -324,7 +324,7 @@ static int fwd_impl(const void* A, const void* Wa, float J0, float J1, const voi
   const size_t cluster_bytes = ring_cluster_applicable(N, a_dim) ? ring_cluster_workspace_bytes(g.nbt) : 0;
   const bool cluster = !resident && ring_uses_cluster(N, a_dim, batch_size, seq_len) && !ring_uses_step_kernels(N, a_dim, g.NC, g.nbt) &&
                        workspace_bytes >= g.wpack_bytes + cluster_bytes;
-  const bool panel = !saved && ring_uses_step_kernels(N, a_dim, g.NC, g.nbt) && ring_uses_panel(N, a_dim, g.NC, g.nbt) &&
+  const bool panel = !saved && ring_uses_step_kernels(N, a_dim, g.NC, g.nbt) && ring_uses_panel(a_dim, g.NC, g.nbt) &&
                      workspace_bytes >= g.wpack_bytes + ring_panel_workspace_bytes(g.NC, g.nbt);
   void* wpack_t = saved ? (char*)saved + g.side_bytes + g.pair_bytes : nullptr;
   const float s0 = (resident || cluster) ? J1 : 1.f, h0 = (resident || cluster) ? J0 : 0.f;
