@@ -99,7 +99,7 @@ RingTeamPlan ring_team_plan(int N, int k, int T, int B, bool bptt, bool ga) {
       best.nt = nt;
       best.slots = slots;
       best.xchg_bytes = up256(xbytes);
-      best.gather_bytes = up256((size_t)nteams * sizeof(unsigned long long));
+      best.gather_bytes = (size_t)nteams * RING_TEAM_WORD * sizeof(unsigned long long);
       best.ga_bytes = ga ? up256((size_t)G * T * k * B * sizeof(float)) : 0;
       best.step_cycles = step;
     }

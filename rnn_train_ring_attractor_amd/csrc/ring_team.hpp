@@ -386,6 +386,7 @@ __device__ __forceinline__ void team_products(const TeamCompute<KPW, C16, MR, WK
 // team_arrive, waits in team_gather and leaves the verdict in LDS for all waves to read behind the next barrier (team_go).
 constexpr unsigned long long TEAM_GAVE_UP = 1ull << 63;
 
+__device__ __forceinline__ unsigned long long* team_word(const RingTeamArgs& c, int team) { return c.gather + (size_t)team * RING_TEAM_WORD; }
 __device__ __forceinline__ int xcc_id() { return __builtin_amdgcn_s_getreg(20 | (0 << 6) | (3 << 11)) & 7; }
 __device__ __forceinline__ unsigned team_arrived(unsigned long long v) { return (unsigned)((v * 0x0101010101010101ull) >> 56); }
 __device__ __forceinline__ bool team_complete(unsigned long long v, int G, int xcc) {
@@ -394,8 +395,8 @@ __device__ __forceinline__ bool team_complete(unsigned long long v, int G, int x
 
 __device__ __forceinline__ void team_arrive(const RingTeamArgs& c, int team, int at) {
   if (at != 0) return;
-  if (c.gather_ticks < 0) __hip_atomic_fetch_or(c.gather + team, TEAM_GAVE_UP, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  else __hip_atomic_fetch_add(c.gather + team, 1ull << (8 * xcc_id()), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  if (c.gather_ticks < 0) __hip_atomic_fetch_or(team_word(c, team), TEAM_GAVE_UP, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  else __hip_atomic_fetch_add(team_word(c, team), 1ull << (8 * xcc_id()), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
 __device__ __forceinline__ void team_gather(const RingTeamArgs& c, char* lds, const LdsPlan& L, int team, int at) {
@@ -403,22 +404,22 @@ __device__ __forceinline__ void team_gather(const RingTeamArgs& c, char* lds, co
   const int xcc = xcc_id();
   const long long start = wall_clock64();
   bool ok = false;
-  unsigned long long v = __hip_atomic_load(c.gather + team, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  unsigned long long v = __hip_atomic_load(team_word(c, team), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   while (!(v & TEAM_GAVE_UP)) {
     if ((int)team_arrived(v) == c.G) {
       ok = team_complete(v, c.G, xcc);
-      if (!ok) __hip_atomic_fetch_or(c.gather + team, TEAM_GAVE_UP, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      if (!ok) __hip_atomic_fetch_or(team_word(c, team), TEAM_GAVE_UP, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       break;
     }
     if (wall_clock64() - start > c.gather_ticks) {
       // (fails, and leaves the new value in v, if another member has arrived meanwhile)
-      if (__hip_atomic_compare_exchange_strong(c.gather + team, &v, v | TEAM_GAVE_UP, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
+      if (__hip_atomic_compare_exchange_strong(team_word(c, team), &v, v | TEAM_GAVE_UP, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
                                                __HIP_MEMORY_SCOPE_AGENT))
         break;
       continue;
     }
     __builtin_amdgcn_s_sleep(1);
-    v = __hip_atomic_load(c.gather + team, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    v = __hip_atomic_load(team_word(c, team), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
   *reinterpret_cast<int*>(lds + L.gathered) = ok;
 }

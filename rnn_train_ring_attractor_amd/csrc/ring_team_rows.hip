@@ -171,7 +171,7 @@ RingTeamPlan ring_team_rows_plan(int N, int k, int B) {
   p.ok = p.nteams <= 8 * (32 / p.G);                       // (8 XCDs of 32 compute units)
   p.shape = RingTeamShape{ROWS_CHUNKS, ROWS_TILES, ROWS_MATS, ROWS_TILES, 0, 8 * p.G * ((p.nteams + 7) / 8)};
   p.xchg_bytes = (size_t)ROWS_SLOTS * p.nteams * p.KC * CHUNK_BYTES;
-  p.gather_bytes = ((size_t)p.nteams * sizeof(unsigned long long) + 255) & ~(size_t)255;
+  p.gather_bytes = (size_t)p.nteams * RING_TEAM_WORD * sizeof(unsigned long long);
   return p;
 }
 

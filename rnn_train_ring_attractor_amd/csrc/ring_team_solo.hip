@@ -261,7 +261,7 @@ __host__ __device__ inline SoloLds solo_lds(int KC, int k, bool ga, bool trig) {
 }
 
 __device__ __forceinline__ bool solo_needed(const RingTeamArgs& c, int bt) {
-  const unsigned long long v = c.gather[bt % c.nteams];      // (written by the launch in front)
+  const unsigned long long v = *team_word(c, bt % c.nteams);      // (written by the launch in front)
   for (int x = 0; x < 8; ++x)
     if (team_complete(v, c.G, x)) return false;
   return true;
