@@ -105,12 +105,14 @@ RINGATTR_API int ringattr_fwd_noalloc(const void* A, const void* Wa, float J0, f
  * `saved` may be NULL: the saved record is then recomputed, from bump_history
  * or (weight-resident geometry: a_dim == 2, 128 < N <= 256) by running the
  * recurrence again from r_init, which reproduces the forward's own numbers.
+ * (From bump_history means: of the trajectory it is handed, whoever made it.)
  * grad_A [B,T,k] and grad_r_init [B,N] are optional outputs (NULL = skip), written
  * rather than accumulated; the reference returns None for both
  * (cpp/ring_rnn_cuda.py:144).  grad_A comes out of the BPTT kernel itself up to N = 512 (the
  * weight-resident kernel reads the bf16 operand copy of r_prev with the step's other inputs; the persistent
  * streaming kernel stages its per-channel shares in LDS, which limits it to a_dim <= 48) and from a pass of its own
- * after the BPTT steps on the step-per-launch kernels (wide rings and small batches; any a_dim, seq_len <= 65535).
+ * after the BPTT steps on the step-per-launch kernels (wide rings; any a_dim, seq_len <= 65535); the team kernels
+ * (csrc/ring_team.hip, up to N = 1024) form it inside, from fp32 r_prev.
  * With a saved buffer, the buffer must be the one the forward filled, at the address it filled it, and the
  * weights must be unchanged since (the forward's transposed weight copy inside it is reused on an exact match of
  * shape, J0, J1 and weight addresses; anything else is repacked).
@@ -144,9 +146,9 @@ RINGATTR_API int ringattr_loss_bwd(const void* bump_history, const void* target_
 
 /* ringattr_fwd followed by ringattr_loss_fwd in one call (same arguments, the time loop's first): the forward of
  *   total = loss_pair(bump_history),  bump_history = forward(...)
- * The persistent forward kernels (N <= 512, except small-batch forwards that are split over workgroups) form the loss
- * head's three sums per history row themselves, right after the activation, and the loss needs no pass of its own
- * over the history (-4N bytes read per sample-step); other shapes run the two stages back to back.  Either way loss_workspace ends up
+ * The weight-resident and the streaming forward kernels form the loss head's three sums per history row themselves,
+ * right after the activation, and the loss needs no pass of its own over the history (-4N bytes read per sample-step);
+ * other shapes (teams, clusters, one launch per step) run the two stages back to back.  Either way loss_workspace ends up
  * as ringattr_loss_fwd leaves it (for ringattr_loss_bwd / ringattr_bwd_loss).  No counterpart in the reference. */
 RINGATTR_API int ringattr_fwd_loss(const void* A, const void* Wa, float J0, float J1, const void* Wo, const void* r_init,
                       void* bump_history, float alpha, int N, int a_dim, int seq_len, int batch_size,

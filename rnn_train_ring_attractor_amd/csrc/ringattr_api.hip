@@ -295,9 +295,9 @@ static int fwd_impl(const void* A, const void* Wa, float J0, float J1, const voi
   hipStream_t st = static_cast<hipStream_t>(stream);
   if (const int ce = ring_cluster_take_error())
     return fail(RINGATTR_ERR_HIP,
-                "an earlier cluster forward gave up waiting for a sibling workgroup (code %d: 1 members on different "
-                "XCDs, 2 members not resident together, 3 a published state never arrived) and its results are "
-                "invalid; this is reported once, and the streaming kernels run N = 512 from here on",
+                "an earlier launch on clusters or teams of workgroups gave up waiting for a sibling (code %d: 1 members "
+                "on different XCDs, 2 members not resident together, 3 a published state never arrived) and its results "
+                "are invalid; this is reported once, and the kernels whose workgroups wait for none run from here on",
                 ce);
 
   if (ring_uses_team(N, a_dim, seq_len, batch_size) && workspace_bytes >= ring_team_fwd_bytes(N, a_dim, seq_len, batch_size)) {
