@@ -69,7 +69,8 @@ RINGATTR_API size_t ringattr_saved_bytes(int N, int a_dim, int seq_len, int batc
  * The backward's figure at that width includes the scratch area of the BPTT on the same clusters
  * (switched on by RINGATTR_CLUSTER_BPTT=1), whether it is on or not.
  * ringattr_bwd_workspace_bytes is enough with and without grad_A.  A backward that is not asked for dL/dA may need
- * much less (the team kernels keep a share of it per member, up to 4 * N * seq_len * batch_size bytes):
+ * much less (the team kernels keep a share of it per member, up to 4 * seq_len * batch_size bytes times N
+ * rounded up to 32):
  * ringattr_bwd_workspace_bytes_for tells the two apart, and ringattr_bwd asks for no more than its own arguments need.
  * Replaces the fixed workspace list of cpp/ring_rnn_cuda.py:108-114. */
 RINGATTR_API size_t ringattr_fwd_workspace_bytes(int N, int a_dim, int seq_len, int batch_size);

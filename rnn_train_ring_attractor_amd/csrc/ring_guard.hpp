@@ -105,6 +105,7 @@ class ResidencyGuard {
 
   void leave(Stream st) {
     if (entries_.size() < 2 && Rt::owner(st) == 0) return;
+    typename Rt::Quiet quiet;
     for (Entry& e : entries_)
       if (mine(e, st)) e.marked = Rt::record(e.ev, st);
   }

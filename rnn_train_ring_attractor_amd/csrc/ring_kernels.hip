@@ -1329,7 +1329,9 @@ unsigned long RingGuardHip::owner(hipStream_t st) {
 }
 bool RingGuardHip::capturing(hipStream_t st) {
   hipStreamCaptureStatus s = hipStreamCaptureStatusNone;
-  return hipStreamIsCapturing(st, &s) == hipSuccess && s != hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(st, &s) == hipSuccess) return s != hipStreamCaptureStatusNone;
+  (void)hipGetLastError();       // (the legacy stream beside another stream's capture: the launch itself reports that)
+  return false;
 }
 bool RingGuardHip::record(hipEvent_t& ev, hipStream_t st) {
   if ((ev || hipEventCreateWithFlags(&ev, hipEventDisableTiming) == hipSuccess) && hipEventRecord(ev, st) == hipSuccess) return true;

@@ -30,6 +30,7 @@ struct Fake {
   static bool capturing(Stream st) { return capture.count(real(st)) != 0; }
   static bool record(Event& ev, Stream st) {
     ++records;
+    if (quiet == 0) std::exit(2);
     if (gone.count(st)) return false;
     ev = Ev{real(st), queued[real(st)]};
     return true;
