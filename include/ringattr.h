@@ -215,6 +215,13 @@ RINGATTR_API int ringattr_generate_inputs(unsigned long long seed, int N, int a_
                       int spread_action, int bump_kind, float bump_param,
                       void* av, void* angle, void* action_signal, void* r_init, void* stream);
 
+/* The two driven channels c0 < c1 of a zero-padded action signal (root train_general_ring_no_gain.py:52-66):
+ * A_out [B,T,2] and Wa_out [2,N,N] from A [B,T,a_dim] and Wa [a_dim,N,N].  The other channels are checked on the device: if
+ * one of them is not zero everywhere, A_out is NaN throughout.  The workspace's size does not depend on the shape. */
+RINGATTR_API size_t ringattr_compact_workspace_bytes(void);
+RINGATTR_API int ringattr_compact_channels(const void* A, const void* Wa, void* A_out, void* Wa_out, int N, int a_dim,
+                      int seq_len, int batch_size, int c0, int c1, void* workspace, size_t workspace_bytes, void* stream);
+
 /* Optimizer tail of a training step: torch.nn.utils.clip_grad_norm_(parameters, max_norm) followed by
  * torch.optim.Adam.step() (root train_general_ring_no_gain.py:333-336), for up to 16 fp32 tensors in three launches.
  * The gradient norm is summed in a fixed order (repeatable).  params / grads / exp_avg / exp_avg_sq are HOST arrays of

@@ -55,6 +55,8 @@ PROTOTYPES = {
     "ringattr_generate_inputs": (c_int, [ctypes.c_ulonglong, c_int, c_int, c_int, c_int, ctypes.c_double,
                                          ctypes.POINTER(c_float), c_int, c_float, c_int, c_int, c_float,
                                          c_void_p, c_void_p, c_void_p, c_void_p, c_void_p]),
+    "ringattr_compact_workspace_bytes": (c_size_t, []),
+    "ringattr_compact_channels": (c_int, [c_void_p] * 4 + [c_int] * 6 + [c_void_p, c_size_t, c_void_p]),
     "ringattr_clip_adam_workspace_bytes": (c_size_t, [c_int, ctypes.POINTER(c_size_t)]),
     "ringattr_clip_adam": (c_int, [c_int, ctypes.POINTER(c_void_p), ctypes.POINTER(c_void_p), ctypes.POINTER(c_void_p),
                                    ctypes.POINTER(c_void_p), ctypes.POINTER(c_size_t), c_float, c_float, c_float,

@@ -15,6 +15,9 @@
 // Optimizer tail (root train_general_ring_no_gain.py:333-336: clip_grad_norm_(parameters, max_norm) then Adam.step()):
 // the squared gradient norm over all tensors in a fixed order (two launches), then one launch that scales the
 // gradients by min(1, max_norm / (norm + 1e-6)) and applies the Adam update to every tensor.
+//
+// Compaction of a zero-padded action signal (root train_general_ring_no_gain.py:52-66): the two driven channels and
+// their matrices side by side, and the check that the others are zero.
 #include "ring_common.hpp"
 #include "ring_kernels.hpp"
 
@@ -156,6 +159,76 @@ hipError_t ring_launch_generate(const RingGenArgs& a, hipStream_t st) {
   hipError_t e = hipGetLastError();
   if (e != hipSuccess || !a.r_init) return e;
   hipLaunchKernelGGL(ring_generate_bump_kernel, dim3(a.B), dim3(256), 0, st, a);
+  return hipGetLastError();
+}
+
+// ------------------------------------------------------------------------------------------------
+// Compaction of the action signal
+// ------------------------------------------------------------------------------------------------
+// out[s] = (A[s][c0], A[s][c1]); Wout = (Wa[c0], Wa[c1]); violated[workgroup]: one of its samples has another channel that is
+// not zero.  The first `signal` workgroups go through the samples, a thread each, the others copy the matrices.
+// Bound by launches at the sizes of a training step: with the launch behind it 6 us where a chain of thirteen tensor
+// operations took 33 (k = 16, B = 1, T = 100, N = 256).
+constexpr int COMPACT_BLOCK = 256, COMPACT_SIGNAL_MAX = RING_COMPACT_FLAGS, COMPACT_COPY = 512;
+__global__ __launch_bounds__(COMPACT_BLOCK) void ring_compact_kernel(const float* __restrict__ A, const float* __restrict__ Wa,
+                                                                     f32x2* __restrict__ out, float* __restrict__ Wout, int* violated,
+                                                                     size_t samples, size_t nn, int k, int c0, int c1, int signal) {
+  if ((int)blockIdx.x >= signal) {
+    const size_t stride = (size_t)(gridDim.x - signal) * COMPACT_BLOCK;
+    for (size_t i = (size_t)(blockIdx.x - signal) * COMPACT_BLOCK + threadIdx.x; i < nn; i += stride) {
+      const float a = Wa[c0 * nn + i], b = Wa[c1 * nn + i];
+      Wout[i] = a;
+      Wout[nn + i] = b;
+    }
+    return;
+  }
+  bool bad = false;
+  const bool wide = (k & 3) == 0 && (reinterpret_cast<uintptr_t>(A) & 15) == 0;      // (a slice may start anywhere)
+  for (size_t s = (size_t)blockIdx.x * COMPACT_BLOCK + threadIdx.x; s < samples; s += (size_t)signal * COMPACT_BLOCK) {
+    const float* row = A + s * k;
+    f32x2 v = {0.f, 0.f};
+    if (wide) {
+      for (int c = 0; c < k; c += 4) {
+        const f32x4 x = *reinterpret_cast<const f32x4*>(row + c);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          if (c + i == c0) v[0] = x[i];
+          else if (c + i == c1) v[1] = x[i];
+          else bad |= x[i] != 0.f;
+        }
+      }
+    } else {
+      for (int c = 0; c < k; ++c) {
+        const float x = row[c];
+        if (c == c0) v[0] = x;
+        else if (c == c1) v[1] = x;
+        else bad |= x != 0.f;
+      }
+    }
+    out[s] = v;
+  }
+  const int any = __syncthreads_or(bad);
+  if (threadIdx.x == 0) violated[blockIdx.x] = any;
+}
+
+// The whole signal NaN if any workgroup found a violation.  (A launch of its own: the verdict is the whole signal's.)
+__global__ __launch_bounds__(COMPACT_SIGNAL_MAX) void ring_compact_verdict_kernel(const int* violated, int n, float* out, size_t values) {
+  const int any = __syncthreads_or((int)threadIdx.x < n && violated[threadIdx.x]);
+  if (!any) return;
+  for (size_t i = threadIdx.x; i < values; i += COMPACT_SIGNAL_MAX) out[i] = __builtin_nanf("");
+}
+
+hipError_t ring_launch_compact(const float* A, const float* Wa, float* out, float* Wout, int* violated, int N, int k, size_t samples,
+                               int c0, int c1, hipStream_t st) {
+  const size_t nn = (size_t)N * N;
+  const size_t blocks = (samples + COMPACT_BLOCK - 1) / COMPACT_BLOCK, copies = (nn + COMPACT_BLOCK - 1) / COMPACT_BLOCK;
+  const int signal = (int)(blocks < COMPACT_SIGNAL_MAX ? blocks : COMPACT_SIGNAL_MAX);
+  const int copy = (int)(copies < COMPACT_COPY ? copies : COMPACT_COPY);
+  hipLaunchKernelGGL(ring_compact_kernel, dim3(signal + copy), dim3(COMPACT_BLOCK), 0, st, A, Wa, reinterpret_cast<f32x2*>(out), Wout,
+                     violated, samples, nn, k, c0, c1, signal);
+  const hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return e;
+  hipLaunchKernelGGL(ring_compact_verdict_kernel, dim3(1), dim3(COMPACT_SIGNAL_MAX), 0, st, violated, signal, out, 2 * samples);
   return hipGetLastError();
 }
 

@@ -169,6 +169,11 @@ struct RingGenArgs {
 };
 hipError_t ring_launch_generate(const RingGenArgs& a, hipStream_t st);
 
+// The two driven channels of a zero-padded action signal and their matrices (ring_aux.hip); violated: RING_COMPACT_FLAGS ints.
+constexpr int RING_COMPACT_FLAGS = 1024;
+hipError_t ring_launch_compact(const float* A, const float* Wa, float* out, float* Wout, int* violated, int N, int k, size_t samples,
+                               int c0, int c1, hipStream_t st);
+
 constexpr int RING_OPT_MAX_TENSORS = 16;
 struct RingOptArgs {
   float* param[RING_OPT_MAX_TENSORS];

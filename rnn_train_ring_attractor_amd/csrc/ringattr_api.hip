@@ -716,6 +716,28 @@ int ringattr_generate_inputs(unsigned long long seed, int N, int a_dim, int seq_
   return RINGATTR_OK;
 }
 
+size_t ringattr_compact_workspace_bytes(void) { return RING_COMPACT_FLAGS * sizeof(int); }
+
+int ringattr_compact_channels(const void* A, const void* Wa, void* A_out, void* Wa_out, int N, int a_dim, int seq_len,
+                              int batch_size, int c0, int c1, void* workspace, size_t workspace_bytes, void* stream) {
+  if (N <= 0 || a_dim <= 0 || seq_len <= 0 || batch_size <= 0)
+    return fail(RINGATTR_ERR_INVALID, "N, a_dim, seq_len, batch_size must be positive (got %d, %d, %d, %d)", N, a_dim,
+                seq_len, batch_size);
+  if (c0 < 0 || c0 >= c1 || c1 >= a_dim)
+    return fail(RINGATTR_ERR_INVALID, "ringattr_compact_channels: channels must be 0 <= c0 < c1 < a_dim (got %d, %d)", c0, c1);
+  if (!A || !Wa || !A_out || !Wa_out) return fail(RINGATTR_ERR_INVALID, "ringattr_compact_channels: null tensor pointer");
+  if (!aligned16(A_out) || !aligned16(Wa_out) || !aligned16(workspace))
+    return fail(RINGATTR_ERR_INVALID, "ringattr_compact_channels: the outputs and the workspace must be 16-byte aligned");
+  const size_t need = ringattr_compact_workspace_bytes();
+  if (!workspace || workspace_bytes < need)
+    return fail(RINGATTR_ERR_WORKSPACE, "ringattr_compact_channels: workspace of %zu bytes needed, %zu given", need,
+                workspace ? workspace_bytes : (size_t)0);
+  hipError_t e = ring_launch_compact((const float*)A, (const float*)Wa, (float*)A_out, (float*)Wa_out, (int*)workspace, N, a_dim,
+                                     (size_t)seq_len * batch_size, c0, c1, static_cast<hipStream_t>(stream));
+  if (e != hipSuccess) return hip_fail(e, "channel compaction launch");
+  return RINGATTR_OK;
+}
+
 size_t ringattr_clip_adam_workspace_bytes(int n_tensors, const size_t* numel) {
   if (n_tensors < 1 || n_tensors > RING_OPT_MAX_TENSORS || !numel) {
     fail(RINGATTR_ERR_INVALID, "between 1 and %d tensors are supported (got %d)", RING_OPT_MAX_TENSORS, n_tensors);

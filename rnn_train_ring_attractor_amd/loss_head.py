@@ -93,13 +93,17 @@ class RingRnnLossFunc(Function):
 
     @staticmethod
     def forward(ctx, action_signal, Wa, J0, J1, Wo, r_init, alpha, activation_name, target_angle, bump_weight,
-                target_amplitude, grad_mode=None):
-        from .ring_rnn_cuda import _activation_id
+                target_amplitude, grad_mode=None, pair=None):
+        from .ring_rnn_cuda import _activation_id, _compact
         act = _activation_id(activation_name)
         B, T, k = action_signal.shape
         N = Wa.shape[1]
         dev = action_signal.device
         A, Wa_c, Wo_c, r0 = action_signal.contiguous(), Wa.contiguous(), Wo.contiguous(), r_init.contiguous()
+        ctx.pair, ctx.Wa_shape = pair, Wa.shape
+        if pair is not None:
+            A, Wa_c = _compact(A, Wa_c, pair)
+            k = 2
         angle = target_angle.contiguous()
         _check("target_angle", angle, (B, T), dev)
         amp = None
@@ -109,7 +113,7 @@ class RingRnnLossFunc(Function):
         hist = torch.empty(T, B, N, device=dev, dtype=A.dtype)
         # autograd switches gradient mode off in here and needs_input_grad stays True under no_grad(): the wrapper says
         needs_grad = grad_mode is not False and any(ctx.needs_input_grad[i] for i in (0, 1, 4, 5))
-        ctx.extra_inputs = 0 if grad_mode is None else 1
+        ctx.extra_inputs = 0 if grad_mode is None else 2
         saved = torch.empty(saved_nbytes(N, k, T, B), dtype=torch.uint8, device=dev) if needs_grad else None
         lib = _lib.load()
         with torch.cuda.device(dev):
@@ -130,7 +134,9 @@ class RingRnnLossFunc(Function):
     @staticmethod
     def backward(ctx, grad_total, _grad_parts, _grad_hist):
         A, Wa, Wo, hist, r0, saved, lws, angle, amp = ctx.saved_tensors
-        grad_Wa, grad_Wo = torch.empty_like(Wa), torch.empty_like(Wo)    # written, not accumulated into
+        from .ring_rnn_cuda import _grad_buffers, _grad_gather
+        grad_Wa, part = _grad_buffers(Wa, ctx.Wa_shape, ctx.pair)         # written, not accumulated into
+        grad_Wo = torch.empty_like(Wo)
         grad_A = torch.empty_like(A) if ctx.needs_input_grad[0] else None
         grad_r0 = torch.empty_like(r0) if ctx.needs_input_grad[5] else None
         if grad_total is None:                   # (gradients are not materialised: the total went unused)
@@ -147,13 +153,13 @@ class RingRnnLossFunc(Function):
                                                  ctx.bump_weight, up.data_ptr(), grad_hist.data_ptr(), N, T, B,
                                                  lws.data_ptr(), lws.numel(), torch.cuda.current_stream(dev).cuda_stream))
             bwd_cuda.bwd(grad_output=grad_hist, A=A, Wa=Wa, J0=ctx.J0, J1=ctx.J1, Wo=Wo, bump_history=hist, r_init=r0,
-                         grad_Wa=grad_Wa, grad_Wo=grad_Wo, alpha=ctx.alpha, activation_type=ctx.act, saved=saved,
+                         grad_Wa=part, grad_Wo=grad_Wo, alpha=ctx.alpha, activation_type=ctx.act, saved=saved,
                          grad_A=grad_A, grad_r_init=grad_r0, accumulate=False)
-            return (grad_A, grad_Wa, None, None, grad_Wo, grad_r0, None, None, None, None, None) + (None,) * ctx.extra_inputs
+            return (grad_A, _grad_gather(grad_Wa, part, ctx.pair), None, None, grad_Wo, grad_r0, None, None, None, None, None) + (None,) * ctx.extra_inputs
         bwd_cuda.bwd(grad_output=None, A=A, Wa=Wa, J0=ctx.J0, J1=ctx.J1, Wo=Wo, bump_history=hist, r_init=r0,
-                     grad_Wa=grad_Wa, grad_Wo=grad_Wo, alpha=ctx.alpha, activation_type=ctx.act, saved=saved,
+                     grad_Wa=part, grad_Wo=grad_Wo, alpha=ctx.alpha, activation_type=ctx.act, saved=saved,
                      grad_A=grad_A, grad_r_init=grad_r0, loss_workspace=lws, loss_upstream=up, accumulate=False)
-        return (grad_A, grad_Wa, None, None, grad_Wo, grad_r0, None, None, None, None, None) + (None,) * ctx.extra_inputs
+        return (grad_A, _grad_gather(grad_Wa, part, ctx.pair), None, None, grad_Wo, grad_r0, None, None, None, None, None) + (None,) * ctx.extra_inputs
 
 
 def ring_rnn_loss_func(action_signal, Wa, J0, J1, Wo, r_init, alpha, activation, target_angle, bump_weight=0.2,
@@ -162,10 +168,8 @@ def ring_rnn_loss_func(action_signal, Wa, J0, J1, Wo, r_init, alpha, activation,
 
     Returns (total, cos_loss, amp_loss, bump_history); only `total` is differentiable (w.r.t. Wa, Wo and, when they
     require it, action_signal and r_init); bump_history [T,B,N] is returned detached for decoding and logging."""
-    from .ring_rnn_cuda import _silent_channel_view
-    compact = _silent_channel_view(action_signal, Wa, driven_channels)
-    if compact is not None:
-        action_signal, Wa = compact
+    from .ring_rnn_cuda import _driven_pair
+    pair = _driven_pair(action_signal, Wa, driven_channels)
     total, parts, hist = RingRnnLossFunc.apply(action_signal, Wa, J0, J1, Wo, r_init, alpha, activation, target_angle,
-                                               bump_weight, target_amplitude, torch.is_grad_enabled())
+                                               bump_weight, target_amplitude, torch.is_grad_enabled(), pair)
     return total, parts[1], parts[2], hist

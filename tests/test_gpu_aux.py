@@ -121,3 +121,48 @@ def test_fused_clip_adam_matches_torch(max_norm, gpu_device):
         o.step()
     torch.cuda.synchronize()
     assert all(torch.equal(x, y) for x, y in zip(opt2.params, opt3.params))
+
+
+# k a multiple of four and not, a slice that starts off a 16-byte boundary, one sample, more samples than one pass of the grid
+@pytest.mark.parametrize("B,T,k,N,pair,offset", [(1, 1, 3, 17, (0, 2), 0), (5, 7, 16, 33, (0, 1), 0), (40, 9, 6, 130, (2, 5), 3),
+                                                 (700, 513, 4, 20, (1, 3), 1)])
+def test_compacted_channels_are_the_named_ones_and_the_rest_is_checked(B, T, k, N, pair, offset, gpu_device):
+    from rnn_train_ring_attractor_amd.ring_rnn_cuda import _compact
+    print(f"[case] compaction B={B} T={T} k={k} N={N} {pair}", flush=True)
+    A = torch.zeros(B * T * k + offset, device=gpu_device)[offset:].view(B, T, k)
+    for c in pair:
+        A[..., c] = torch.randn(B, T, device=gpu_device)
+    Wa = torch.randn(k, N, N, device=gpu_device)
+    a2, w2 = _compact(A, Wa, pair)
+    assert torch.equal(a2, A[..., list(pair)]) and torch.equal(w2, Wa[list(pair)])
+    silent = [c for c in range(k) if c not in pair]
+    for b, t, c, v in ((B - 1, T - 1, silent[-1], 1e-30), (0, 0, silent[0], float("nan"))):
+        A[b, t, c] = v
+        assert torch.isnan(_compact(A, Wa, pair)[0]).all()
+        A[b, t, c] = 0.0
+
+
+@pytest.mark.parametrize("N,k", [(60, 16), (300, 5), (600, 6)])
+def test_a_padded_signal_runs_on_its_driven_channels_at_every_width(N, k, gpu_device):
+    """The helper's statement is acted on outside the weight-resident widths too, unless the tensor has been written to."""
+    from rnn_train_ring_attractor_amd import host, ring_rnn_cuda_func
+    from rnn_train_ring_attractor_amd.ring_rnn_cuda import _driven_pair
+    B, T = 20, 6
+    print(f"[case] padded signal N={N} k={k}", flush=True)
+    g = torch.Generator(device=gpu_device).manual_seed(3)
+    r = lambda *s: torch.randn(*s, device=gpu_device, generator=g)
+    A, r0, G = host.av_to_action_signal_ND(r(B, T) * 0.2, k), r(B, N).abs() * 0.1, r(T, B, N)
+    wa, wo, outs = r(k, N, N) / N ** 0.5, r(N, N) / N ** 0.5, []
+    for signal in (A, A.clone()):                      # (a copy carries no statement)
+        Wa, Wo = wa.clone().requires_grad_(True), wo.clone().requires_grad_(True)
+        h = ring_rnn_cuda_func(signal, Wa, -0.05, 0.5, Wo, r0, 0.15, "tanh")
+        h.backward(G)
+        outs.append((h.detach(), Wa.grad, Wo.grad))
+    assert _driven_pair(A, Wa) == (0, 1) and _driven_pair(A.clone(), Wa) is None
+    assert torch.count_nonzero(outs[0][1][2:]) == 0
+    for x, y in zip(*outs):                             # two kernel families: other row-sum roundings
+        assert float((x - y).abs().max()) <= 5e-3 * float(y.abs().max())
+    A[0, 0, 2] = 0.1
+    assert _driven_pair(A, Wa) is None
+    want = ring_rnn_cuda_func(A.clone(), Wa, -0.05, 0.5, Wo, r0, 0.15, "tanh")
+    assert torch.equal(ring_rnn_cuda_func(A, Wa, -0.05, 0.5, Wo, r0, 0.15, "tanh"), want)
