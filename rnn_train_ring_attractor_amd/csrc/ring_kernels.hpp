@@ -244,7 +244,7 @@ struct RingTeamArgs {
   const float* A;
   float* ga_part;        // dL/dA partials [member][T][k][B]
   float scale0, shift0, J0, J1;
-  int N, k, T, B, nbt, KC, G, nteams, nt, slots, cts, transposed, spin_max;
+  int N, k, T, B, nbt, KC, G, nteams, nt, slots, cts, spin_max;
   int gather_ticks;      // how long the members of a team wait for each other, in 10 ns (negative: not at all)
   int c16, mr, wk;       // the shape, for the single workgroups that take over
   int rows;              // non-zero: one wave sums the whole contraction, chunks in the order of rows_chunk (ring_team_rows.hip)

@@ -165,7 +165,7 @@ size_t ring_team_fwd_bytes(int N, int k, int T, int B) { return plan_bytes(N, k,
 size_t ring_team_bptt_bytes(int N, int k, int T, int B, bool ga) { return plan_bytes(N, k, T, B, true, ga); }
 
 static hipError_t team_args(const RingTeamPlan& p, const float* Wo, const float* Wa, const float* A, float J0, float J1,
-                            bool folded, int N, int k, int T, int B, int cts, bool transposed, void* ws, RingTeamArgs& c,
+                            bool folded, int N, int k, int T, int B, int cts, void* ws, RingTeamArgs& c,
                             hipStream_t st) {
   hipError_t e = ring_cluster_host_err(&c.host_err);
   if (e != hipSuccess) return e;
@@ -191,7 +191,6 @@ static hipError_t team_args(const RingTeamPlan& p, const float* Wo, const float*
   c.nt = p.nt;
   c.slots = p.slots;
   c.cts = cts;
-  c.transposed = transposed ? 1 : 0;
   c.spin_max = 16000000;   // some seconds of polling
   if (const char* v = getenv("RINGATTR_CLUSTER_SPIN")) {
     const long s = atol(v);
@@ -216,7 +215,7 @@ hipError_t ring_team_fwd(const RingFwdArgs& a, const float* Wo, const float* Wa,
   const RingTeamPlan p = ring_team_plan(a.N, a.k, a.T, a.B, false, false);
   if (!p.ok || !ws || (a.dfrag != nullptr) != (a.rfrag != nullptr)) return hipErrorInvalidValue;
   RingTeamArgs c;
-  hipError_t e = team_args(p, Wo, Wa, a.A, a.J0, a.J1, folded, a.N, a.k, a.T, a.B, cts, false, ws, c, st);
+  hipError_t e = team_args(p, Wo, Wa, a.A, a.J0, a.J1, folded, a.N, a.k, a.T, a.B, cts, ws, c, st);
   if (e != hipSuccess) return e;
   e = ring_launch_team_fwd(a, c, p.shape, st);
   return e == hipSuccess ? ring_launch_team_solo_fwd(a, c, st) : e;
@@ -226,7 +225,7 @@ hipError_t ring_team_rows(const RingFwdArgs& a, const float* Wo, const float* Wa
   const RingTeamPlan p = ring_team_rows_plan(a.N, a.k, a.B);
   if (!p.ok || !ws || !a.hist || a.dfrag || a.rfrag) return hipErrorInvalidValue;
   RingTeamArgs c;
-  hipError_t e = team_args(p, Wo, Wa, a.A, a.J0, a.J1, true, a.N, a.k, a.T, a.B, 0, false, ws, c, st);
+  hipError_t e = team_args(p, Wo, Wa, a.A, a.J0, a.J1, true, a.N, a.k, a.T, a.B, 0, ws, c, st);
   if (e != hipSuccess) return e;
   c.wk = c.rows = 1;
   e = ring_launch_team_rows(a, c, p.shape, st);
@@ -251,7 +250,7 @@ hipError_t ring_team_bptt(const RingBpttArgs& a, const float* Wo, const float* W
   const RingTeamPlan p = ring_team_plan(a.N, a.k, a.T, a.B, true, ga);
   if (!p.ok || !ws) return hipErrorInvalidValue;
   RingTeamArgs c;
-  hipError_t e = team_args(p, Wo, Wa, a.A, a.J0, a.J1, folded, a.N, a.k, a.T, a.B, cts, true, ws, c, st);
+  hipError_t e = team_args(p, Wo, Wa, a.A, a.J0, a.J1, folded, a.N, a.k, a.T, a.B, cts, ws, c, st);
   if (e != hipSuccess) return e;
   e = ga ? ring_launch_team_bptt_ga(a, c, p.shape, st) : ring_launch_team_bptt(a, c, p.shape, st);
   if (e == hipSuccess) e = ring_launch_team_solo_bptt(a, c, st);

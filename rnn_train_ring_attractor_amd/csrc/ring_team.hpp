@@ -123,16 +123,26 @@ __device__ __forceinline__ u32x2 quad_rows2(unsigned x, int lane) {
 
 // Eight consecutive weights of one output neuron `out`, contraction indices k0 .. k0 + 7, from an fp32 [N][N] matrix.
 // Loads and arithmetic are apart so that several fragments' loads can be in flight; addresses are clamped into the
-// matrix and the padding is zeroed afterwards.
+// matrix and the padding is zeroed afterwards.  ROWS4 (rows that start on 16-byte boundaries): two 16-byte loads, eight
+// fragments at a time; a call of T = 20 steps falls from 181 to 128 us at N = 512, 16 channels, B = 256, from 105 to 70 at
+// N = 1024, two channels, B = 1 (all on their way at once into one XCD: 12.6 MB).  Other rows are slower so than a word at a
+// time (N = 1023, B = 100: 140 against 98 us).
 struct WeightLoad { float v[8]; };
 typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));
 typedef float f32x2u __attribute__((ext_vector_type(2), aligned(4)));
+enum : int { WEIGHT_ROWS, WEIGHT_ROWS4, WEIGHT_COLUMNS };      // COLUMNS: the transposed matrix
 
-__device__ __forceinline__ void weight_load(WeightLoad& l, const float* __restrict__ W, int N, int out, int k0, bool transposed) {
+template <int HOW>
+__device__ __forceinline__ void weight_load(WeightLoad& l, const float* __restrict__ W, int N, int out, int k0) {
   const int o = out < N ? out : N - 1;
-  if (transposed) {
+  if constexpr (HOW == WEIGHT_COLUMNS) {
 #pragma unroll
     for (int x = 0; x < 8; ++x) l.v[x] = W[(size_t)(k0 + x < N ? k0 + x : N - 1) * N + o];
+  } else if constexpr (HOW == WEIGHT_ROWS4) {      // (N is a multiple of four: a group of four is in the row or past it)
+    const float* src = W + (size_t)o * N;
+    const f32x4 lo = *reinterpret_cast<const f32x4*>(src + (k0 < N ? k0 : 0)), hi = *reinterpret_cast<const f32x4*>(src + (k0 + 4 < N ? k0 + 4 : 0));
+#pragma unroll
+    for (int x = 0; x < 4; ++x) { l.v[x] = lo[x]; l.v[4 + x] = hi[x]; }
   } else {
 #pragma unroll
     for (int x = 0; x < 8; ++x) l.v[x] = W[(size_t)o * N + (k0 + x < N ? k0 + x : N - 1)];
@@ -228,10 +238,29 @@ struct TeamCompute {
   // offsets).  Only the last one can lie past the contraction: its lanes then point past the buffer and read zero.
   unsigned x_lane, rs_lane, x_last, rs_last;
 
-  template <bool TR>
-  __device__ __forceinline__ void load_resident(const RingTeamArgs& c, int mem, int w, int lane) {
+  template <int HOW>
+  __device__ __forceinline__ void load_matrices(const RingTeamArgs& c, bf16x8* wl, int mem, int w, int lane) {
     const int q = lane >> 4, n = lane & 15;
-    constexpr int BATCH = 4;          // (four fragments' fp32 values at a time: registers are short)
+    constexpr int BATCH = HOW == WEIGHT_ROWS4 ? 8 : 4;      // fragments on their way at a time
+    // into LDS: the matrices past the registers', this wave's own chunks
+    if constexpr (EX) {
+      const int total = (c.k + 1 - MR) * C16 * KPW;
+      for (int f0 = 0; f0 < total; f0 += BATCH) {
+        WeightLoad l[BATCH];
+#pragma unroll
+        for (int i = 0; i < BATCH; ++i) {
+          const int f = f0 + i < total ? f0 + i : total - 1, mm = MR + f / (C16 * KPW), cc = f / KPW % C16, kc = w + WK * (f % KPW);
+          weight_load<HOW>(l[i], c.Wa + (size_t)(mm - 1) * c.N * c.N, c.N, 16 * (mem * C16 + cc) + n, 32 * kc + 8 * q);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int i = 0; i < BATCH; ++i) {
+          const int f = f0 + i, mm = MR + f / (C16 * KPW), cc = f / KPW % C16, kc = w + WK * (f % KPW);
+          if (f < total && kc < c.KC)
+            wl[((size_t)((mm - MR) * C16 + cc) * c.KC + kc) * 64 + lane] = weight_fragment(l[i], c.N, 16 * (mem * C16 + cc) + n, 32 * kc + 8 * q, 1.f, 0.f);
+        }
+      }
+    }
 #pragma unroll
     for (int f0 = 0; f0 < F; f0 += BATCH) {
       WeightLoad l[BATCH];
@@ -240,7 +269,7 @@ struct TeamCompute {
         const int f = f0 + i, mm = f / (C16 * KPW), cc = f / KPW % C16, kc = w + WK * (f % KPW);
         if (f < F) {
           const float* W = mm == 0 || mm > c.k ? c.Wo : c.Wa + (size_t)(mm - 1) * c.N * c.N;
-          weight_load(l[i], W, c.N, 16 * (mem * C16 + cc) + n, 32 * kc + 8 * q, TR);
+          weight_load<HOW>(l[i], W, c.N, 16 * (mem * C16 + cc) + n, 32 * kc + 8 * q);
         }
       }
       __builtin_amdgcn_sched_barrier(0);
@@ -257,29 +286,18 @@ struct TeamCompute {
       __builtin_amdgcn_sched_barrier(0);
     }
   }
+  template <bool TR>
   __device__ __forceinline__ void load_weights(const RingTeamArgs& c, bf16x8* wl, bf16x8* parked_area, int mem, int w, int lane) {
     parked = parked_area + (size_t)w * (F - FR) * 64 + lane;
-    const int q = lane >> 4, n = lane & 15;
     const unsigned first = (unsigned)w * CHUNK_BYTES;
     x_lane = first + lane * 16;
     rs_lane = first + 1024 + (lane & 15) * 16 + (lane >> 4) * 4;
     const bool whole = w + WK * (KPW - 1) < c.KC;
     x_last = whole ? x_lane : NOWHERE;
     rs_last = whole ? rs_lane : NOWHERE;
-    if constexpr (EX)
-    for (int mm = MR; mm <= c.k; ++mm)                    // into LDS: this wave's own chunks
-      for (int kc = w; kc < c.KC; kc += WK) {
-        const float* W = c.Wa + (size_t)(mm - 1) * c.N * c.N;
-        WeightLoad l[C16];
-#pragma unroll
-        for (int cc = 0; cc < C16; ++cc) weight_load(l[cc], W, c.N, 16 * (mem * C16 + cc) + n, 32 * kc + 8 * q, c.transposed != 0);
-#pragma unroll
-        for (int cc = 0; cc < C16; ++cc)
-          wl[((size_t)((mm - MR) * C16 + cc) * c.KC + kc) * 64 + lane] =
-              weight_fragment(l[cc], c.N, 16 * (mem * C16 + cc) + n, 32 * kc + 8 * q, 1.f, 0.f);
-      }
-    if (c.transposed) load_resident<true>(c, mem, w, lane);
-    else load_resident<false>(c, mem, w, lane);
+    if constexpr (TR) load_matrices<WEIGHT_COLUMNS>(c, wl, mem, w, lane);
+    else if ((c.N & 3) == 0) load_matrices<WEIGHT_ROWS4>(c, wl, mem, w, lane);
+    else load_matrices<WEIGHT_ROWS>(c, wl, mem, w, lane);
   }
 };
 
@@ -429,14 +447,15 @@ __device__ __forceinline__ bool team_go(const char* lds, const LdsPlan& L) {
 }
 
 // The compute waves' loop: `steps` rounds over the team's my_nt tiles, operand number s of round s.
-template <int KPW, int C16, int MR, int WK, bool EX, bool GA>
+// (TR: with the transposed matrices)
+template <bool TR, int KPW, int C16, int MR, int WK, bool EX, bool GA>
 __device__ __forceinline__ void team_compute_loop(const RingTeamArgs& c, const LdsPlan& L, char* lds,
                                                   __amdgpu_buffer_rsrc_t rsrc, int mem, int team, int my_nt, int steps, int w,
                                                   int lane) {
   using AM = AuxMap<C16>;
   TeamCompute<KPW, C16, MR, WK, EX, GA> tc;
   bf16x8* const wl = reinterpret_cast<bf16x8*>(lds + L.weights);
-  tc.load_weights(c, wl, reinterpret_cast<bf16x8*>(lds + L.parked), mem, w, lane);
+  tc.template load_weights<TR>(c, wl, reinterpret_cast<bf16x8*>(lds + L.parked), mem, w, lane);
   const int q = lane >> 4, b = lane & 15;
   float* const share = reinterpret_cast<float*>(lds + L.share) + (size_t)w * C16 * AM::SHARE + q * AM::QS + b * 4;
   const float* const gates = reinterpret_cast<const float*>(lds + L.gates);

@@ -19,7 +19,7 @@ __global__ __launch_bounds__(64 * (WK + AUX)) void ring_team_bptt_kernel(RingBpt
   const int steps = (p.grad_r_init || GA) ? T : T - 1;
 
   if (w < WK) {
-    team_compute_loop<KPW, C16, MR, WK, EX, GA>(c, L, lds, rsrc, mem, team, my_nt, steps, w, lane);
+    team_compute_loop<true, KPW, C16, MR, WK, EX, GA>(c, L, lds, rsrc, mem, team, my_nt, steps, w, lane);
     return;
   }
 

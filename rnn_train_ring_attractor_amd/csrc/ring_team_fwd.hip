@@ -16,7 +16,7 @@ __global__ __launch_bounds__(64 * (WK + AUX)) void ring_team_fwd_kernel(RingFwdA
   const int T = p.T;
 
   if (w < WK) {
-    team_compute_loop<KPW, C16, MR, WK, EX, false>(c, L, lds, rsrc, mem, team, my_nt, T, w, lane);
+    team_compute_loop<false, KPW, C16, MR, WK, EX, false>(c, L, lds, rsrc, mem, team, my_nt, T, w, lane);
     return;
   }
 

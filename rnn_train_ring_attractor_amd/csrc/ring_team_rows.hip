@@ -57,23 +57,28 @@ __global__ __launch_bounds__(64 * (ROWS_TILES + AUX)) void ring_team_rows_kernel
       const int kc = rows_chunk(i);
       at[i] = kc < c.KC ? (unsigned)kc * CHUNK_BYTES + lane * 16 : NOWHERE;        // (past the contraction: zeros)
     }
+    auto load = [&](auto how) {
+      constexpr int HOW = decltype(how)::value, BATCH = HOW == WEIGHT_ROWS4 ? 8 : 4;
 #pragma unroll
-    for (int m = 0; m < ROWS_MATS; ++m)
+      for (int m = 0; m < ROWS_MATS; ++m)
 #pragma unroll
-      for (int i0 = 0; i0 < ROWS_CHUNKS; i0 += 4) {
-        WeightLoad l[4];
-        const float* W = m == 0 ? c.Wo : c.Wa + (size_t)(m - 1) * c.N * c.N;
+        for (int i0 = 0; i0 < ROWS_CHUNKS; i0 += BATCH) {
+          WeightLoad l[BATCH];
+          const float* W = m == 0 ? c.Wo : c.Wa + (size_t)(m - 1) * c.N * c.N;
 #pragma unroll
-        for (int i = 0; i < 4; ++i) weight_load(l[i], W, c.N, out, 32 * rows_chunk(i0 + i) + 8 * q, false);
-        __builtin_amdgcn_sched_barrier(0);
+          for (int i = 0; i < BATCH; ++i) weight_load<HOW>(l[i], W, c.N, out, 32 * rows_chunk(i0 + i) + 8 * q);
+          __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          bf16x8 f = weight_fragment(l[i], c.N, out, 32 * rows_chunk(i0 + i) + 8 * q, m == 0 ? c.scale0 : 1.f, m == 0 ? c.shift0 : 0.f);
-          asm volatile("" : "+v"(f));              // (here, not at its first use: twice the registers until then)
-          wt[m][i0 + i] = f;
+          for (int i = 0; i < BATCH; ++i) {
+            bf16x8 f = weight_fragment(l[i], c.N, out, 32 * rows_chunk(i0 + i) + 8 * q, m == 0 ? c.scale0 : 1.f, m == 0 ? c.shift0 : 0.f);
+            asm volatile("" : "+v"(f));              // (here, not at its first use: twice the registers until then)
+            wt[m][i0 + i] = f;
+          }
+          __builtin_amdgcn_sched_barrier(0);
         }
-        __builtin_amdgcn_sched_barrier(0);
-      }
+    };
+    if ((c.N & 3) == 0) load(std::integral_constant<int, WEIGHT_ROWS4>{});
+    else load(std::integral_constant<int, WEIGHT_ROWS>{});
     lds_barrier();                                        // the first gates are in LDS
     if (!team_go(lds, L)) return;
     float* const dst = share + w * AM::SHARE + q * AM::QS + b * 4;

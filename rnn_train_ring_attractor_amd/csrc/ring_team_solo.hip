@@ -272,14 +272,9 @@ __device__ __forceinline__ bf16x8 solo_weight(const RingTeamArgs& c, int m, int 
   const int out = 16 * ct + (lane & 15), k0 = 32 * kc + 8 * (lane >> 4);
   const float* W = m == 0 ? c.Wo : c.Wa + (size_t)(m - 1) * c.N * c.N;
   WeightLoad l;
-  if (!TR && k0 + 8 <= c.N) {
-    const float* src = W + (size_t)(out < c.N ? out : c.N - 1) * c.N + k0;
-    const f32x4 lo = *reinterpret_cast<const f32x4u*>(src), hi = *reinterpret_cast<const f32x4u*>(src + 4);
-#pragma unroll
-    for (int i = 0; i < 4; ++i) { l.v[i] = lo[i]; l.v[4 + i] = hi[i]; }
-  } else {
-    weight_load(l, W, c.N, out, k0, TR);
-  }
+  if constexpr (TR) weight_load<WEIGHT_COLUMNS>(l, W, c.N, out, k0);
+  else if ((c.N & 3) == 0) weight_load<WEIGHT_ROWS4>(l, W, c.N, out, k0);
+  else weight_load<WEIGHT_ROWS>(l, W, c.N, out, k0);
   return weight_fragment(l, c.N, out, k0, m == 0 ? c.scale0 : 1.f, m == 0 ? c.shift0 : 0.f);
 }
 
