@@ -1,4 +1,4 @@
-// Weight-gradient contraction, register-tiled variant for NPAD >= 256 (NC = 4 or 8).
+// Weight-gradient contraction, register-tiled, for NPAD >= 128.
 //
 //   dW_mm[i][j] = sum over samples (b,t) of coef_mm(b,t) * g[t,b,i] * r_prev[t,b,j]
 //
@@ -223,17 +223,25 @@ __global__ __launch_bounds__(256) void ring_dw_direct_kernel(RingDwArgs p, int m
   }
 }
 
-bool ring_dw_tiled_applicable(int NC) { return NC == 4 || NC == 8 || NC == 16 || NC == 24 || NC == 32; }
+bool ring_dw_tiled_applicable(int NC) { return NC == 2 || NC == 4 || NC == 8 || NC == 16 || NC == 24 || NC == 32; }
 
 // K splits: one workgroup per CU, a multiple of 8 when possible (XCD grouping).  One launch per
 // group of three matrices, so the grid of a launch does not depend on a_dim.
+// N <= 128 (one block): a split's partial sums are 64 KiB a matrix, as much to write and to sum up as some four chunks take to
+// contract, so none gets fewer, and with more than five channels there are at most 80 splits.  us of contraction and
+// reduction against a wave per 32 x 128 block without an LDS stage: N = 120, a_dim 2, T = 240, B = 64 33 -> 25, B = 4096
+// 932 -> 123.
 int ring_dw_tiled_nz(int NC, int k, long nchunk) {
-  (void)k;
   const int NB = 4 * NC / 8;
   const long tiles = (long)NB * NB;
   long nz = (256 + tiles - 1) / tiles;
   if (nz >= 8) nz = (nz + 7) / 8 * 8;
-  if (nz > 128) nz = 128;
+  if (NC == 2) {
+    if (k > 5) nz = 80;
+    if (nz > nchunk / 4) nz = nchunk / 4 >= 8 ? nchunk / 32 * 8 : nchunk / 4;
+  } else if (nz > 128) {
+    nz = 128;
+  }
   if (nz > nchunk) nz = nchunk;
   if (nz < 1) nz = 1;
   return (int)nz;
@@ -298,6 +306,7 @@ hipError_t ring_launch_dw_tiled(const RingDwArgs& a, int NC, hipStream_t st) {
       const int b = (int)(p0 * a.nbt), e_ = (int)(p1 * a.nbt), add = p0 > 0 ? 1 : 0;
       hipError_t e = hipErrorInvalidValue;
       switch (NC) {
+        case 2: e = launch_group<2>(a, mg, blocks, b, e_, add, st); break;
         case 4: e = launch_group<4>(a, mg, blocks, b, e_, add, st); break;
         case 8: e = launch_group<8>(a, mg, blocks, b, e_, add, st); break;
         case 16: e = launch_group<16>(a, mg, blocks, b, e_, add, st); break;

@@ -68,8 +68,8 @@ int make_geo(int N, int k, int T, int B, Geo& g) {
   g.wpack_bytes = align_up((size_t)(1 + k) * g.NPAD * g.NPAD * 2);
   g.side_bytes = align_up((size_t)T * g.nbt * 16 * g.NPAD * 2);
   g.pair_bytes = align_up((size_t)((T + 1) / 2) * 2 * g.nbt * 16 * g.NPAD * 2);
-  const int NT = 4 * nc, TJ = nc == 1 ? 4 : 8;
-  const long per_z = (long)(NT / 2) * (NT / TJ) * ((k + 3) / 3);  // wave work items per K split
+  const int NT = 4 * nc;
+  const long per_z = (long)(NT / 2) * (NT / 4) * ((k + 3) / 3);  // wave work items per K split (of the kernel for N <= 64)
   const long nchunk = (long)g.nbt * ((T + 1) / 2);
   if (nchunk > 0x7fffffffL) return fail(RINGATTR_ERR_INVALID, "batch_size * seq_len is too large");
   long nz = (2048 + per_z - 1) / per_z;
