@@ -270,6 +270,11 @@ bool ring_uses_team_rows(int N, int k, int B);
 size_t ring_team_rows_bytes(int N, int k, int B);
 hipError_t ring_team_rows(const RingFwdArgs& a, const float* Wo, const float* Wa, void* ws, hipStream_t st);
 hipError_t ring_launch_team_rows(const RingFwdArgs& a, const RingTeamArgs& c, const RingTeamShape& sh, hipStream_t st);
+// 17 <= N <= 128 with up to six channels: a workgroup per batch tile (ring_team_one.hip)
+bool ring_team_one_applicable(int N, int k);
+bool ring_uses_team_one(int N, int k);
+hipError_t ring_launch_team_one_fwd(const RingFwdArgs& a, const RingTeamArgs& c, hipStream_t st);
+hipError_t ring_launch_team_one_bptt(const RingBpttArgs& a, const RingTeamArgs& c, hipStream_t st);
 // the record from a.hist; a.Wpack: forward fragments in order 3, with J1 * Wo + J0 as matrix 0 when folded
 hipError_t ring_team_rebuild(const RingFwdArgs& a, bool folded, int cts, hipStream_t st);
 hipError_t ring_launch_team_rebuild(const RingFwdArgs& a, const RingTeamArgs& c, int wk, hipStream_t st);

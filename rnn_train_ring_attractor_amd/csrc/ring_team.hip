@@ -129,7 +129,11 @@ static bool forced() {
 //     46 against 37, B = 6016: 49 against 54).  Rows reproduce between batches on the same side of this line: members of
 //     any width sum a row alike.
 // The rule does not ask whether a record is wanted: a history is the same with and without one.
+// Whether a workgroup per batch tile does it; RINGATTR_TEAM=1 asks for the exchange through L2.
+bool ring_uses_team_one(int N, int k) { return ring_team_one_applicable(N, k) && !forced(); }
+
 static bool team_shape(int N, int k, int T, int B) {
+  if (ring_uses_team_one(N, k)) return true;
   if (ring_res256_applicable(N, k) && !forced()) return false;
   const RingTeamPlan f = ring_team_plan(N, k, T, B, false, false);
   if (!f.ok || !ring_team_plan(N, k, T, B, true, true).ok) return false;
@@ -157,7 +161,7 @@ size_t ring_team_rows_bytes(int N, int k, int B) {
 
 // Scratch of one launch; none where no call of this shape comes here.
 static size_t plan_bytes(int N, int k, int T, int B, bool bptt, bool ga) {
-  if (!team_shape(N, k, T, B)) return 0;
+  if (!team_shape(N, k, T, B) || ring_uses_team_one(N, k)) return 0;
   const RingTeamPlan p = ring_team_plan(N, k, T, B, bptt, ga);
   return p.xchg_bytes + p.gather_bytes + p.ga_bytes;
 }
@@ -211,7 +215,24 @@ static hipError_t team_args(const RingTeamPlan& p, const float* Wo, const float*
   return hipGetLastError();
 }
 
+// (the fields that a workgroup on its own needs)
+static RingTeamArgs one_args(const float* Wo, const float* Wa, const float* A, float J0, float J1, int N, int k, int T, int B, int cts) {
+  RingTeamArgs c = {};
+  c.Wo = Wo;
+  c.Wa = Wa;
+  c.A = A;
+  c.J0 = J0;
+  c.J1 = J1;
+  c.N = N;
+  c.k = k;
+  c.T = T;
+  c.B = B;
+  c.cts = cts;
+  return c;
+}
+
 hipError_t ring_team_fwd(const RingFwdArgs& a, const float* Wo, const float* Wa, bool folded, int cts, void* ws, hipStream_t st) {
+  if (ring_uses_team_one(a.N, a.k)) return ring_launch_team_one_fwd(a, one_args(Wo, Wa, a.A, a.J0, a.J1, a.N, a.k, a.T, a.B, cts), st);
   const RingTeamPlan p = ring_team_plan(a.N, a.k, a.T, a.B, false, false);
   if (!p.ok || !ws || (a.dfrag != nullptr) != (a.rfrag != nullptr)) return hipErrorInvalidValue;
   RingTeamArgs c;
@@ -233,20 +254,22 @@ hipError_t ring_team_rows(const RingFwdArgs& a, const float* Wo, const float* Wa
 }
 
 hipError_t ring_team_rebuild(const RingFwdArgs& a, bool folded, int cts, hipStream_t st) {
-  const RingTeamPlan p = ring_team_plan(a.N, a.k, a.T, a.B, false, false);
-  if (!p.ok) return hipErrorInvalidValue;
+  const bool one = ring_uses_team_one(a.N, a.k);           // (sums in the order of a single compute wave)
+  const RingTeamPlan p = one ? RingTeamPlan{} : ring_team_plan(a.N, a.k, a.T, a.B, false, false);
+  if (!one && !p.ok) return hipErrorInvalidValue;
   RingTeamArgs c = {};
   c.A = a.A;
   c.J0 = folded ? 0.f : a.J0;
   c.J1 = folded ? 1.f : a.J1;
   c.k = a.k;
-  c.KC = p.KC;
+  c.KC = (a.N + 31) / 32;
   c.cts = cts;
-  return ring_launch_team_rebuild(a, c, p.shape.wk, st);
+  return ring_launch_team_rebuild(a, c, one ? 1 : p.shape.wk, st);
 }
 
 hipError_t ring_team_bptt(const RingBpttArgs& a, const float* Wo, const float* Wa, bool folded, int cts, void* ws, hipStream_t st) {
   const bool ga = a.grad_A != nullptr;
+  if (ring_uses_team_one(a.N, a.k)) return ring_launch_team_one_bptt(a, one_args(Wo, Wa, a.A, a.J0, a.J1, a.N, a.k, a.T, a.B, cts), st);
   const RingTeamPlan p = ring_team_plan(a.N, a.k, a.T, a.B, true, ga);
   if (!p.ok || !ws) return hipErrorInvalidValue;
   RingTeamArgs c;

@@ -75,6 +75,13 @@ __device__ __forceinline__ unsigned pack_bf16(float lo, float hi) {
   return __builtin_bit_cast(unsigned, v);
 }
 
+// The derivative record's fp16.  (The value is rounded to fp32 first: left alone the compiler forms it in one fused operation
+// in some kernels and not in others, and a row's record would depend on the kernel.)
+__device__ __forceinline__ _Float16 record_value(float d) {
+  asm("" : "+v"(d));
+  return (_Float16)d;
+}
+
 __device__ __forceinline__ unsigned dpp_xor1(unsigned x) { return (unsigned)__builtin_amdgcn_update_dpp(0, (int)x, 0xB1, 0xF, 0xF, false); }
 __device__ __forceinline__ unsigned dpp_xor2(unsigned x) { return (unsigned)__builtin_amdgcn_update_dpp(0, (int)x, 0x4E, 0xF, 0xF, false); }
 template <int CTRL>
@@ -134,18 +141,19 @@ enum : int { WEIGHT_ROWS, WEIGHT_ROWS4, WEIGHT_COLUMNS };      // COLUMNS: the t
 
 template <int HOW>
 __device__ __forceinline__ void weight_load(WeightLoad& l, const float* __restrict__ W, int N, int out, int k0) {
-  const int o = out < N ? out : N - 1;
+  const unsigned o = out < N ? out : N - 1;          // (offsets in 32 bits: one register an address, not two)
   if constexpr (HOW == WEIGHT_COLUMNS) {
 #pragma unroll
-    for (int x = 0; x < 8; ++x) l.v[x] = W[(size_t)(k0 + x < N ? k0 + x : N - 1) * N + o];
+    for (int x = 0; x < 8; ++x) l.v[x] = W[(unsigned)(k0 + x < N ? k0 + x : N - 1) * (unsigned)N + o];
   } else if constexpr (HOW == WEIGHT_ROWS4) {      // (N is a multiple of four: a group of four is in the row or past it)
-    const float* src = W + (size_t)o * N;
-    const f32x4 lo = *reinterpret_cast<const f32x4*>(src + (k0 < N ? k0 : 0)), hi = *reinterpret_cast<const f32x4*>(src + (k0 + 4 < N ? k0 + 4 : 0));
+    const unsigned at = o * (unsigned)N;
+    const f32x4 lo = *reinterpret_cast<const f32x4*>(W + (at + (unsigned)(k0 < N ? k0 : 0))),
+                hi = *reinterpret_cast<const f32x4*>(W + (at + (unsigned)(k0 + 4 < N ? k0 + 4 : 0)));
 #pragma unroll
     for (int x = 0; x < 4; ++x) { l.v[x] = lo[x]; l.v[4 + x] = hi[x]; }
   } else {
 #pragma unroll
-    for (int x = 0; x < 8; ++x) l.v[x] = W[(size_t)o * N + (k0 + x < N ? k0 + x : N - 1)];
+    for (int x = 0; x < 8; ++x) l.v[x] = W[o * (unsigned)N + (unsigned)(k0 + x < N ? k0 + x : N - 1)];
   }
 }
 __device__ __forceinline__ bf16x8 weight_fragment(const WeightLoad& l, int N, int out, int k0, float scale, float shift) {
@@ -673,8 +681,8 @@ struct TeamAux {
     const __amdgpu_buffer_rsrc_t r = team_buffer(base + ((size_t)t * nbt + bt) * cts * 256, base ? (size_t)cts * 512 : 0);
     if constexpr (NPT == 4)
       __builtin_amdgcn_raw_buffer_store_b64(
-          __builtin_bit_cast(u32x2, f16x4{(_Float16)d[0], (_Float16)d[1], (_Float16)d[2], (_Float16)d[3]}), r, (int)d_off, 0, 0);
-    else __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, f16x2{(_Float16)d[0], (_Float16)d[1]}), r, (int)d_off, 0, 0);
+          __builtin_bit_cast(u32x2, f16x4{record_value(d[0]), record_value(d[1]), record_value(d[2]), record_value(d[3])}), r, (int)d_off, 0, 0);
+    else __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, f16x2{record_value(d[0]), record_value(d[1])}), r, (int)d_off, 0, 0);
   }
   // operand copy for the weight gradients: steps 2j (lo) and 2j + 1 (hi) of a neuron's four rows side by side
   __device__ __forceinline__ void pair_put(__bf16* base, int t, int nbt, int bt, int cts, const unsigned (&lo)[NPT / 2],

@@ -186,7 +186,7 @@ __global__ __launch_bounds__(512) void ring_team_rebuild_kernel(RingFwdArgs p, R
         for (int i = 0; i < 4; ++i) {
           float aF, aD;
           act_scaled<ACT>(tot[cc][r][i], asc, aF, aD);
-          d[i] = (_Float16)aD;
+          d[i] = record_value(aD);
         }
         *reinterpret_cast<f16x4*>(p.dfrag + ((((size_t)t0 + (r & 1)) * p.nbt + tile(r)) * c.cts + 2 * pair + cc) * 256 + (q * 16 + b) * 4) = d;
       }
@@ -408,7 +408,7 @@ __global__ __launch_bounds__(64 * SOLO_WAVES) void ring_team_solo_fwd_kernel(Rin
           float aF, aD;
           act_scaled<ACT>(x[cc][i], asc, aF, aD);
           rn[i] = j + i < N ? fmaf(oma, r[i], aF) : 0.f;
-          d[i] = (_Float16)aD;
+          d[i] = record_value(aD);
         }
         state[ct * 64] = rn;
         solo_put4(next, ct, lane, rn);

@@ -436,7 +436,7 @@ static int bwd_impl(const char* who, const void* grad_output, const void* loss_w
   if (!workspace || workspace_bytes < need)
     return fail(RINGATTR_ERR_WORKSPACE, "%s: workspace of %zu bytes needed, %zu given", who, need,
                 workspace ? workspace_bytes : (size_t)0);
-  if (team && ring_team_bptt_bytes(N, a_dim, seq_len, batch_size, grad_A != nullptr) == 0)
+  if (team && !ring_uses_team_one(N, a_dim) && ring_team_bptt_bytes(N, a_dim, seq_len, batch_size, grad_A != nullptr) == 0)
     return fail(RINGATTR_ERR_INVALID, "%s: the saved buffer was filled by the team kernels, which RINGATTR_TEAM no longer asks for; run "
                 "forward and backward under the same setting", who);
   hipStream_t st = static_cast<hipStream_t>(stream);
