@@ -215,6 +215,24 @@ RINGATTR_API int ringattr_generate_inputs(unsigned long long seed, int N, int a_
                       int spread_action, int bump_kind, float bump_param,
                       void* av, void* angle, void* action_signal, void* r_init, void* stream);
 
+/* The gain operator with the networks' parameters where the modules keep them: nets is a HOST array of 4 a_dim device
+ * pointers, w1 [hidden], b1 [hidden], w2 [hidden], b2 [1] of every channel (a_dim <= 16).  halves: the signal is an angular
+ * velocity [B,T] and the two channels are relu(-av) and relu(av) (train/train_ring_attractor.py:136-146); otherwise it is
+ * [B,T,a_dim].  grad_params comes packed, [a_dim, 3 hidden + 1]; the workspace is ringattr_gain_workspace_bytes large. */
+RINGATTR_API int ringattr_gain_nets_fwd(const void* signal, int halves, const void* const* nets, void* action_signal, int a_dim,
+                      int hidden, int seq_len, int batch_size, void* stream);
+RINGATTR_API int ringattr_gain_nets_bwd(const void* signal, int halves, const void* const* nets, const void* grad_action_signal,
+                      void* grad_params, int a_dim, int hidden, int seq_len, int batch_size, void* workspace,
+                      size_t workspace_bytes, void* stream);
+
+/* Action signal [B,T,a_dim] of an angular velocity [B,T]: relu(-av), relu(av), zeros (root
+ * train_general_ring_no_gain.py:52-66). */
+RINGATTR_API int ringattr_action_signal(const void* av, void* action_signal, int a_dim, int seq_len, int batch_size, void* stream);
+/* r_init [B,N]: exp(-d^2 / two_var) over its Euclidean norm, d the circular distance in neurons to angle[b * angle_stride]
+ * N / (2 pi) (train/train_ring_attractor.py:21-52). */
+RINGATTR_API int ringattr_initial_bump(const void* angle, size_t angle_stride, void* r_init, int N, int batch_size, float two_var,
+                      void* stream);
+
 /* The two driven channels c0 < c1 of a zero-padded action signal (root train_general_ring_no_gain.py:52-66):
  * A_out [B,T,2] and Wa_out [2,N,N] from A [B,T,a_dim] and Wa [a_dim,N,N].  The other channels are checked on the device: if
  * one of them is not zero everywhere, A_out is NaN throughout.  The workspace's size does not depend on the shape. */

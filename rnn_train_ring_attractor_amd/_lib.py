@@ -55,6 +55,11 @@ PROTOTYPES = {
     "ringattr_generate_inputs": (c_int, [ctypes.c_ulonglong, c_int, c_int, c_int, c_int, ctypes.c_double,
                                          ctypes.POINTER(c_float), c_int, c_float, c_int, c_int, c_float,
                                          c_void_p, c_void_p, c_void_p, c_void_p, c_void_p]),
+    "ringattr_gain_nets_fwd": (c_int, [c_void_p, c_int, ctypes.POINTER(c_void_p), c_void_p, c_int, c_int, c_int, c_int, c_void_p]),
+    "ringattr_gain_nets_bwd": (c_int, [c_void_p, c_int, ctypes.POINTER(c_void_p), c_void_p, c_void_p, c_int, c_int, c_int, c_int,
+                                       c_void_p, c_size_t, c_void_p]),
+    "ringattr_action_signal": (c_int, [c_void_p, c_void_p, c_int, c_int, c_int, c_void_p]),
+    "ringattr_initial_bump": (c_int, [c_void_p, c_size_t, c_void_p, c_int, c_int, c_float, c_void_p]),
     "ringattr_compact_workspace_bytes": (c_size_t, []),
     "ringattr_compact_channels": (c_int, [c_void_p] * 4 + [c_int] * 6 + [c_void_p, c_size_t, c_void_p]),
     "ringattr_clip_adam_workspace_bytes": (c_size_t, [c_int, ctypes.POINTER(c_size_t)]),
@@ -142,3 +147,16 @@ def profile_read():
     cnt = (ctypes.c_longlong * n)()
     check(load().ringattr_profile_read(ms, cnt))
     return {KERNEL_NAMES[i]: (ms[i], cnt[i]) for i in range(n)}
+
+
+def plain_gpu_tensor(t) -> bool:
+    """Whether a helper may hand t's memory to a kernel in place of a chain of torch operations: an fp32 GPU tensor that no
+    derivative is wanted of, and nothing that watches or transforms the operations (autograd, forward mode, functorch,
+    tracing, compilation, a dispatch or function mode) to miss them."""
+    if type(t) is not torch.Tensor or not t.is_cuda or t.dtype != torch.float32 or t.layout != torch.strided:
+        return False
+    if (t.requires_grad and torch.is_grad_enabled()) or torch.compiler.is_compiling() or torch.jit.is_tracing():
+        return False
+    if torch._C._functorch.maybe_current_level() is not None or torch.autograd.forward_ad._current_level >= 0:
+        return False
+    return torch._C._len_torch_dispatch_stack() == 0 and torch._C._len_torch_function_stack() == 0 and not t.is_neg() and t.numel() > 0

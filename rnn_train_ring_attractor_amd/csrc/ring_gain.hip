@@ -10,13 +10,27 @@
 // summed over B*T samples in a fixed order (per-thread partial sums, fixed tree inside a workgroup, per-workgroup
 // partials summed in a fixed order by a second launch), and optionally dL/dx.
 //
-// Parameters are packed per channel as [w1[0..h) | b1[0..h) | w2[0..h) | b2]; gradients use the same packing.
+// Parameters are packed per channel as [w1[0..h) | b1[0..h) | w2[0..h) | b2]; gradients use the same packing.  They may
+// also be given as the networks' own tensors, and the signal as the angular velocity whose two halves (relu(-av), relu(av))
+// are the channels: at N = 120, B = 128, T = 120 packing, splitting and their way back were sixteen of a training pass's launches.
 #include "ring_common.hpp"
 #include "ring_kernels.hpp"
 
 namespace {
 
 constexpr int GAIN_THREADS = 256;
+
+// Parameter o of channel c, o = 0 .. 3h: w1, b1, w2, b2.
+__device__ __forceinline__ float gain_param(const RingGainParams& p, int h, int c, int part, int j) {
+  if (p.packed) return p.packed[(size_t)c * (3 * h + 1) + part * h + j];
+  return p.part[4 * c + part][j];
+}
+// Channel c of sample s: its own value, or half of the angular velocity.
+__device__ __forceinline__ float gain_input(const RingGainParams& p, const float* x, long s, int k, int c) {
+  if (!p.halves) return x[s * k + c];
+  const float v = c == 0 ? -x[s] : x[s];
+  return v <= 0.f ? 0.f : v;
+}
 
 __device__ __forceinline__ void gelu_pair(float x, float& F, float& D) { act_fast<ACT_GELU>(x, F, D); }
 
@@ -34,7 +48,7 @@ __device__ __forceinline__ void softplus_pair(float z, float& s, float& ds) {
 // One thread per element (b, t, c) of the [B,T,k] signal.
 template <int H>
 __global__ __launch_bounds__(GAIN_THREADS) void ring_gain_fwd_kernel(const float* __restrict__ x,
-                                                                     const float* __restrict__ params,
+                                                                     RingGainParams params,
                                                                      float* __restrict__ out, int k, int h, long total) {
   extern __shared__ float prm[];                           // [k][3H+1], zero padded past h
   constexpr int PS = 3 * H + 1;
@@ -42,15 +56,15 @@ __global__ __launch_bounds__(GAIN_THREADS) void ring_gain_fwd_kernel(const float
     const int c = i / PS, o = i % PS;
     const int part = o / H, j = o % H;
     float v = 0.f;
-    if (o == 3 * H) v = params[(size_t)c * (3 * h + 1) + 3 * h];
-    else if (j < h) v = params[(size_t)c * (3 * h + 1) + part * h + j];
+    if (o == 3 * H) v = gain_param(params, h, c, 3, 0);
+    else if (j < h) v = gain_param(params, h, c, part, j);
     prm[i] = v;
   }
   __syncthreads();
   for (long idx = (long)blockIdx.x * GAIN_THREADS + threadIdx.x; idx < total; idx += (long)gridDim.x * GAIN_THREADS) {
     const int c = (int)(idx % k);
     const float* pc = prm + c * PS;
-    const float xv = x[idx], m = fabsf(xv);
+    const float xv = gain_input(params, x, idx / k, k, c), m = fabsf(xv);
     float z = pc[3 * H];
 #pragma unroll
     for (int j = 0; j < H; ++j) {
@@ -69,7 +83,7 @@ __global__ __launch_bounds__(GAIN_THREADS) void ring_gain_fwd_kernel(const float
 // partial[blk][c][3H+1].  grad_x (optional) receives dL/dx = dL/dA * (s + x * s' * sign(x)).
 template <int H>
 __global__ __launch_bounds__(GAIN_THREADS) void ring_gain_bwd_kernel(const float* __restrict__ x,
-                                                                     const float* __restrict__ params,
+                                                                     RingGainParams params,
                                                                      const float* __restrict__ grad_A,
                                                                      float* __restrict__ grad_x,
                                                                      float* __restrict__ partial, int k, int h,
@@ -81,8 +95,8 @@ __global__ __launch_bounds__(GAIN_THREADS) void ring_gain_bwd_kernel(const float
   for (int o = tid; o < PS; o += GAIN_THREADS) {
     const int part = o / H, j = o % H;
     float v = 0.f;
-    if (o == 3 * H) v = params[(size_t)c * (3 * h + 1) + 3 * h];
-    else if (j < h) v = params[(size_t)c * (3 * h + 1) + part * h + j];
+    if (o == 3 * H) v = gain_param(params, h, c, 3, 0);
+    else if (j < h) v = gain_param(params, h, c, part, j);
     prm[o] = v;
   }
   __syncthreads();
@@ -91,7 +105,7 @@ __global__ __launch_bounds__(GAIN_THREADS) void ring_gain_bwd_kernel(const float
   for (int j = 0; j < H; ++j) gw1[j] = gb1[j] = gw2[j] = 0.f;
   for (long sidx = (long)blockIdx.x * GAIN_THREADS + tid; sidx < samples; sidx += (long)gridDim.x * GAIN_THREADS) {
     const long idx = sidx * k + c;
-    const float xv = x[idx], m = fabsf(xv), go = grad_A[idx];
+    const float xv = gain_input(params, x, sidx, k, c), m = fabsf(xv), go = grad_A[idx];
     float a[H], da[H];
     float z = prm[3 * H];
 #pragma unroll
@@ -179,7 +193,7 @@ size_t ring_gain_workspace_bytes(int k, int h, long samples) {
   return (size_t)ring_gain_blocks(samples) * k * (3 * H + 1) * sizeof(float);
 }
 
-hipError_t ring_launch_gain_fwd(const float* x, const float* params, float* out, int k, int h, long samples,
+hipError_t ring_launch_gain_fwd(const float* x, const RingGainParams& params, float* out, int k, int h, long samples,
                                 hipStream_t st) {
   const int H = gain_pad(h);
   if (H == 0) return hipErrorInvalidValue;
@@ -196,7 +210,7 @@ hipError_t ring_launch_gain_fwd(const float* x, const float* params, float* out,
   return hipGetLastError();
 }
 
-hipError_t ring_launch_gain_bwd(const float* x, const float* params, const float* grad_A, float* grad_params,
+hipError_t ring_launch_gain_bwd(const float* x, const RingGainParams& params, const float* grad_A, float* grad_params,
                                 float* grad_x, int k, int h, long samples, void* workspace, hipStream_t st) {
   const int H = gain_pad(h);
   if (H == 0) return hipErrorInvalidValue;

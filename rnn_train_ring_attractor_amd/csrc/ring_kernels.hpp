@@ -148,8 +148,14 @@ const ring_f32x4* ring_loss_row_coefficients(const void* workspace);
 
 // Gain networks of the action signal (ring_gain.hip): params / grad_params are [k][3h+1] = [w1 | b1 | w2 | b2] per channel.
 size_t ring_gain_workspace_bytes(int k, int h, long samples);
-hipError_t ring_launch_gain_fwd(const float* x, const float* params, float* out, int k, int h, long samples, hipStream_t st);
-hipError_t ring_launch_gain_bwd(const float* x, const float* params, const float* grad_A, float* grad_params, float* grad_x,
+constexpr int RING_GAIN_NETS = 16;
+struct RingGainParams {
+  const float* packed;                          // [k][3h+1], or null:
+  const float* part[4 * RING_GAIN_NETS];        // w1 [h], b1 [h], w2 [h], b2 [1] of every channel
+  int halves;                                   // non-zero: the signal is an angular velocity, channels relu(-av) and relu(av)
+};
+hipError_t ring_launch_gain_fwd(const float* x, const RingGainParams& params, float* out, int k, int h, long samples, hipStream_t st);
+hipError_t ring_launch_gain_bwd(const float* x, const RingGainParams& params, const float* grad_A, float* grad_params, float* grad_x,
                                 int k, int h, long samples, void* workspace, hipStream_t st);
 
 // Synthetic input generator and optimizer tail (ring_aux.hip).
@@ -168,6 +174,10 @@ struct RingGenArgs {
   int N, k, T, B;
 };
 hipError_t ring_launch_generate(const RingGenArgs& a, hipStream_t st);
+
+// Action signal and initial bump of given trials (ring_aux.hip).
+hipError_t ring_launch_action_signal(const float* av, float* out, int k, size_t samples, hipStream_t st);
+hipError_t ring_launch_initial_bump(const float* angle, size_t stride, float* out, int N, int B, float two_var, hipStream_t st);
 
 // The two driven channels of a zero-padded action signal and their matrices (ring_aux.hip); violated: RING_COMPACT_FLAGS ints.
 constexpr int RING_COMPACT_FLAGS = 1024;

@@ -650,7 +650,9 @@ int ringattr_gain_fwd(const void* base_signal, const void* params, void* action_
                       int batch_size, void* stream) {
   if (ringattr_gain_workspace_bytes(a_dim, hidden, seq_len, batch_size) == 0) return RINGATTR_ERR_INVALID;
   if (!base_signal || !params || !action_signal) return fail(RINGATTR_ERR_INVALID, "ringattr_gain_fwd: null tensor pointer");
-  hipError_t e = ring_launch_gain_fwd((const float*)base_signal, (const float*)params, (float*)action_signal, a_dim, hidden,
+  RingGainParams prm = {};
+  prm.packed = (const float*)params;
+  hipError_t e = ring_launch_gain_fwd((const float*)base_signal, prm, (float*)action_signal, a_dim, hidden,
                                       (long)seq_len * batch_size, static_cast<hipStream_t>(stream));
   if (e != hipSuccess) return hip_fail(e, "gain network forward launch");
   return RINGATTR_OK;
@@ -666,10 +668,81 @@ int ringattr_gain_bwd(const void* base_signal, const void* params, const void* g
   if (!workspace || workspace_bytes < need)
     return fail(RINGATTR_ERR_WORKSPACE, "ringattr_gain_bwd: workspace of %zu bytes needed, %zu given", need,
                 workspace ? workspace_bytes : (size_t)0);
-  hipError_t e = ring_launch_gain_bwd((const float*)base_signal, (const float*)params, (const float*)grad_action_signal,
+  RingGainParams prm = {};
+  prm.packed = (const float*)params;
+  hipError_t e = ring_launch_gain_bwd((const float*)base_signal, prm, (const float*)grad_action_signal,
                                       (float*)grad_params, (float*)grad_base_signal, a_dim, hidden,
                                       (long)seq_len * batch_size, workspace, static_cast<hipStream_t>(stream));
   if (e != hipSuccess) return hip_fail(e, "gain network backward launch");
+  return RINGATTR_OK;
+}
+
+// The networks' own tensors; false with a message if something is missing.
+static bool gain_nets(const char* who, const void* const* nets, int halves, int a_dim, RingGainParams& prm) {
+  prm = {};
+  if (a_dim > RING_GAIN_NETS || (halves && a_dim != 2)) {
+    fail(RINGATTR_ERR_INVALID, "%s: up to %d channels, and two where the signal is an angular velocity (got %d)", who, RING_GAIN_NETS, a_dim);
+    return false;
+  }
+  prm.halves = halves ? 1 : 0;
+  for (int i = 0; i < 4 * a_dim; ++i) {
+    if (!nets || !nets[i]) {
+      fail(RINGATTR_ERR_INVALID, "%s: null parameter pointer", who);
+      return false;
+    }
+    prm.part[i] = (const float*)nets[i];
+  }
+  return true;
+}
+
+int ringattr_gain_nets_fwd(const void* signal, int halves, const void* const* nets, void* action_signal, int a_dim, int hidden,
+                           int seq_len, int batch_size, void* stream) {
+  if (ringattr_gain_workspace_bytes(a_dim, hidden, seq_len, batch_size) == 0) return RINGATTR_ERR_INVALID;
+  if (!signal || !action_signal) return fail(RINGATTR_ERR_INVALID, "ringattr_gain_nets_fwd: null tensor pointer");
+  RingGainParams prm;
+  if (!gain_nets("ringattr_gain_nets_fwd", nets, halves, a_dim, prm)) return RINGATTR_ERR_INVALID;
+  hipError_t e = ring_launch_gain_fwd((const float*)signal, prm, (float*)action_signal, a_dim, hidden, (long)seq_len * batch_size,
+                                      static_cast<hipStream_t>(stream));
+  if (e != hipSuccess) return hip_fail(e, "gain network forward launch");
+  return RINGATTR_OK;
+}
+
+int ringattr_gain_nets_bwd(const void* signal, int halves, const void* const* nets, const void* grad_action_signal,
+                           void* grad_params, int a_dim, int hidden, int seq_len, int batch_size, void* workspace,
+                           size_t workspace_bytes, void* stream) {
+  const size_t need = ringattr_gain_workspace_bytes(a_dim, hidden, seq_len, batch_size);
+  if (need == 0) return RINGATTR_ERR_INVALID;
+  if (!signal || !grad_action_signal || !grad_params)
+    return fail(RINGATTR_ERR_INVALID, "ringattr_gain_nets_bwd: null tensor pointer");
+  if (!workspace || workspace_bytes < need)
+    return fail(RINGATTR_ERR_WORKSPACE, "ringattr_gain_nets_bwd: workspace of %zu bytes needed, %zu given", need,
+                workspace ? workspace_bytes : (size_t)0);
+  RingGainParams prm;
+  if (!gain_nets("ringattr_gain_nets_bwd", nets, halves, a_dim, prm)) return RINGATTR_ERR_INVALID;
+  hipError_t e = ring_launch_gain_bwd((const float*)signal, prm, (const float*)grad_action_signal, (float*)grad_params, nullptr,
+                                      a_dim, hidden, (long)seq_len * batch_size, workspace, static_cast<hipStream_t>(stream));
+  if (e != hipSuccess) return hip_fail(e, "gain network backward launch");
+  return RINGATTR_OK;
+}
+
+int ringattr_action_signal(const void* av, void* action_signal, int a_dim, int seq_len, int batch_size, void* stream) {
+  if (a_dim < 2 || seq_len <= 0 || batch_size <= 0)
+    return fail(RINGATTR_ERR_INVALID, "ringattr_action_signal: at least two channels, seq_len and batch_size positive (got %d, %d, %d)",
+                a_dim, seq_len, batch_size);
+  if (!av || !action_signal) return fail(RINGATTR_ERR_INVALID, "ringattr_action_signal: null tensor pointer");
+  hipError_t e = ring_launch_action_signal((const float*)av, (float*)action_signal, a_dim, (size_t)seq_len * batch_size,
+                                           static_cast<hipStream_t>(stream));
+  if (e != hipSuccess) return hip_fail(e, "action signal launch");
+  return RINGATTR_OK;
+}
+
+int ringattr_initial_bump(const void* angle, size_t angle_stride, void* r_init, int N, int batch_size, float two_var, void* stream) {
+  if (N <= 0 || batch_size <= 0)
+    return fail(RINGATTR_ERR_INVALID, "ringattr_initial_bump: N and batch_size must be positive (got %d, %d)", N, batch_size);
+  if (!angle || !r_init) return fail(RINGATTR_ERR_INVALID, "ringattr_initial_bump: null tensor pointer");
+  hipError_t e = ring_launch_initial_bump((const float*)angle, angle_stride, (float*)r_init, N, batch_size, two_var,
+                                          static_cast<hipStream_t>(stream));
+  if (e != hipSuccess) return hip_fail(e, "initial bump launch");
   return RINGATTR_OK;
 }
 

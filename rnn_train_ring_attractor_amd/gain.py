@@ -4,9 +4,12 @@
 nn.Sequential(Linear(1,h), GELU, Linear(h,1), Softplus) on |x| and returns x * gain (train/train_ring_attractor.py:70-79,
 136-146; train/train_general_ring_attractor.py:38-46, 99-109).  `params` is [k, 3h+1] = per channel [w1 | b1 | w2 | b2];
 `pack_gain_nets` builds it from the nn.Sequential modules with differentiable torch ops, so autograd carries the
-operator's parameter gradients back into the modules.
+operator's parameter gradients back into the modules.  `ring_gain_nets` and `ring_gain_halves` take the modules: the kernels
+then read the parameters where they are, and their gradients are slices of one buffer.
 """
 from __future__ import annotations
+
+import ctypes
 
 import torch
 from torch.autograd import Function
@@ -76,3 +79,76 @@ class RingGainFunc(Function):
 def ring_gain_func(base_signal, params):
     """[B,T,k] base signal, [k,3h+1] packed gain-network parameters -> [B,T,k] gated action signal."""
     return RingGainFunc.apply(base_signal, params)
+
+
+class RingGainNetsFunc(Function):
+    """The same operator with the modules' own parameter tensors (four per channel) as inputs, for a signal that needs no
+    gradient; halves: the signal is an angular velocity [B,T] and the channels are relu(-av) and relu(av)."""
+
+    @staticmethod
+    def forward(ctx, signal, halves, *params):
+        B, T = signal.shape[:2]
+        k, h = len(params) // 4, params[0].numel()
+        ctx.save_for_backward(signal, *params)
+        ctx.dims = (B, T, k, h, halves)
+        out = torch.empty(B, T, k, dtype=signal.dtype, device=signal.device)
+        with torch.cuda.device(signal.device):
+            _lib.check(_lib.load().ringattr_gain_nets_fwd(signal.data_ptr(), int(halves), _pointers(params), out.data_ptr(), k, h, T, B,
+                                                          torch.cuda.current_stream(signal.device).cuda_stream))
+        return out
+
+    @staticmethod
+    def backward(ctx, grad_out):
+        signal, *params = ctx.saved_tensors
+        B, T, k, h, halves = ctx.dims
+        lib = _lib.load()
+        g = grad_out.contiguous()
+        grad = torch.empty(k, 3 * h + 1, dtype=signal.dtype, device=signal.device)
+        with torch.cuda.device(signal.device):
+            nbytes = lib.ringattr_gain_workspace_bytes(k, h, T, B)
+            if nbytes == 0:
+                _lib.check(1)
+            ws = torch.empty(nbytes, dtype=torch.uint8, device=signal.device)
+            _lib.check(lib.ringattr_gain_nets_bwd(signal.data_ptr(), int(halves), _pointers(params), g.data_ptr(), grad.data_ptr(), k, h,
+                                                  T, B, ws.data_ptr(), nbytes, torch.cuda.current_stream(signal.device).cuda_stream))
+        parts = []
+        for row in grad:
+            w1, b1, w2, b2 = row.split((h, h, h, 1))
+            parts += [w1.view(h, 1), b1, w2.view(1, h), b2]
+        return (None, None, *parts)
+
+
+def _pointers(tensors):
+    return (ctypes.c_void_p * len(tensors))(*[t.data_ptr() for t in tensors])
+
+
+def _net_parameters(nets, signal):
+    """The parameter tensors as RingGainNetsFunc takes them, or None if these networks or this signal are not its case."""
+    if not 1 <= len(nets) <= 16 or signal.dtype != torch.float32 or signal.requires_grad or signal.numel() == 0:
+        return None
+    h = nets[0][0].weight.shape[0]
+    params = []
+    for net in nets:
+        shaped = ((net[0].weight, (h, 1)), (net[0].bias, (h,)), (net[2].weight, (1, h)), (net[2].bias, (1,)))
+        for t, shape in shaped:
+            if t is None or tuple(t.shape) != shape or t.dtype != torch.float32 or t.device != signal.device or not t.is_contiguous():
+                return None
+            params.append(t)
+    return params if 1 <= h <= 32 else None
+
+
+def ring_gain_nets(base_signal, nets):
+    """[B,T,k] base signal through its channels' gain networks (nn.Sequential modules) -> [B,T,k] action signal."""
+    params = _net_parameters(nets, base_signal) if base_signal.dim() == 3 and base_signal.shape[2] == len(nets) else None
+    if params is None:
+        return ring_gain_func(base_signal, pack_gain_nets(nets))
+    return RingGainNetsFunc.apply(base_signal.contiguous(), False, *params)
+
+
+def ring_gain_halves(av_signal, nets):
+    """[B,T] angular velocity -> [B,T,2] action signal: relu(-av) and relu(av) through the two networks."""
+    params = _net_parameters(nets, av_signal) if av_signal.dim() == 2 and len(nets) == 2 else None
+    if params is None:
+        base = torch.cat([torch.relu(-av_signal).unsqueeze(2), torch.relu(av_signal).unsqueeze(2)], dim=2)
+        return ring_gain_func(base, pack_gain_nets(nets))
+    return RingGainNetsFunc.apply(av_signal.contiguous(), True, *params)

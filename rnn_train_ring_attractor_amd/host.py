@@ -1,6 +1,7 @@
 """Host-side companions of the operator: the helpers the reference training script imports next to
 `ring_rnn_cuda_func` (initial bump, losses, decoders, action-signal builders, the AV dataset) and the
-nn.Module that wraps the operator.  All plain torch; they run on whatever device their inputs are on.
+nn.Module that wraps the operator.  Plain torch on whatever device their inputs are on; the initial bump and the action
+signal of a GPU tensor nobody differentiates are one HIP launch each.
 
 Counterparts (reference paths): train/train_ring_attractor.py:10-52, 190-298;
 utils/generate_av_integration_data.py:11-58, 111-215; train_general_ring_no_gain.py:21-118, 176-229.
@@ -11,6 +12,8 @@ import math
 
 import torch
 import torch.nn as nn
+
+from ._lib import check, load, plain_gpu_tensor
 
 
 def non_linear(x, activation_name):
@@ -23,6 +26,13 @@ def non_linear(x, activation_name):
 def create_initial_bump(initial_angles, num_neurons, bump_width_factor=10, device="cpu"):
     """Gaussian bump on the ring (circular index distance, sigma = N / factor), unit L2 norm per row."""
     ang = initial_angles.to(device)
+    if type(num_neurons) is int and num_neurons > 0 and type(bump_width_factor) in (int, float) and ang.dim() == 1 and plain_gpu_tensor(ang):
+        sigma = num_neurons / bump_width_factor
+        with torch.cuda.device(ang.device):
+            out = torch.empty(ang.shape[0], num_neurons, dtype=torch.float32, device=ang.device)
+            check(load().ringattr_initial_bump(ang.data_ptr(), ang.stride(0), out.data_ptr(), num_neurons, ang.shape[0],
+                                               2 * sigma * sigma, torch.cuda.current_stream(ang.device).cuda_stream))
+        return out
     centre = (ang * num_neurons / (2 * math.pi)).unsqueeze(1)
     idx = torch.arange(num_neurons, device=device).unsqueeze(0)
     dist = (idx - centre).abs()
@@ -68,15 +78,32 @@ def plot_ring_matrices(ring_rnn, title_prefix=""):
     return None
 
 
+def _action_signal(av_signal, action_dim):
+    """(L, R, 0, ...) of a plain GPU tensor in one launch, else None."""
+    if action_dim < 2 or av_signal.dim() != 2 or not av_signal.is_contiguous() or not plain_gpu_tensor(av_signal):
+        return None
+    B, T = av_signal.shape
+    with torch.cuda.device(av_signal.device):
+        out = torch.empty(B, T, action_dim, dtype=torch.float32, device=av_signal.device)
+        check(load().ringattr_action_signal(av_signal.data_ptr(), out.data_ptr(), action_dim, T, B,
+                                            torch.cuda.current_stream(av_signal.device).cuda_stream))
+    return out
+
+
 def av_to_action_signal(av_signal):
+    out = _action_signal(av_signal, 2)
+    if out is not None:
+        return out
     return torch.stack([torch.relu(-av_signal), torch.relu(av_signal)], dim=2)
 
 
 def av_to_action_signal_ND(av_signal, action_dim=16, zero_padding=True):
     if zero_padding:
-        out = torch.zeros(*av_signal.shape, action_dim, device=av_signal.device, dtype=av_signal.dtype)
-        out[:, :, 0] = torch.relu(-av_signal)
-        out[:, :, 1] = torch.relu(av_signal)
+        out = _action_signal(av_signal, action_dim) if type(action_dim) is int else None
+        if out is None:
+            out = torch.zeros(*av_signal.shape, action_dim, device=av_signal.device, dtype=av_signal.dtype)
+            out[:, :, 0] = torch.relu(-av_signal)
+            out[:, :, 1] = torch.relu(av_signal)
         if action_dim > 2:
             # what this construction guarantees, for the operator: channels 2.. are identically zero
             from .ring_rnn_cuda import state_driven_channels
@@ -244,8 +271,8 @@ class GeneralizedRingAttractor(nn.Module):
         """[B,T,k] action signal -> action * gain(|action|) per channel.  On the GPU all gain networks run as one HIP
         operator (forward and backward); on the CPU (tests of the module itself) as the torch modules they are."""
         if action_signal.is_cuda:
-            from .gain import pack_gain_nets, ring_gain_func
-            return ring_gain_func(action_signal, pack_gain_nets(list(self.gain_nets)))
+            from .gain import ring_gain_nets
+            return ring_gain_nets(action_signal, list(self.gain_nets))
         gains = [net(action_signal[:, :, c:c + 1].abs()) for c, net in enumerate(self.gain_nets)]
         return action_signal * torch.cat(gains, dim=2)
 
@@ -323,12 +350,12 @@ class LeakyRingAttractor(nn.Module):
     def action_signal(self, av_signal):
         """[B,T] angular velocity -> [B,T,2] gated (L, R) channels.  On the GPU both gain networks run as one HIP
         operator (forward and backward); on the CPU (tests of the module itself) as the torch modules they are."""
+        if self.gain_l_net is not None and av_signal.is_cuda:
+            from .gain import ring_gain_halves
+            return ring_gain_halves(av_signal, [self.gain_l_net, self.gain_r_net])
         left, right = torch.relu(-av_signal).unsqueeze(2), torch.relu(av_signal).unsqueeze(2)
         if self.gain_l_net is None:
             return torch.cat([left, right], dim=2)
-        if av_signal.is_cuda:
-            from .gain import pack_gain_nets, ring_gain_func
-            return ring_gain_func(torch.cat([left, right], dim=2), pack_gain_nets([self.gain_l_net, self.gain_r_net]))
         return torch.cat([self.gain_l_net(left) * left, self.gain_r_net(right) * right], dim=2)
 
     def forward_history(self, av_signal, r_init=None):

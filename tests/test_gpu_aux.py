@@ -166,3 +166,41 @@ def test_a_padded_signal_runs_on_its_driven_channels_at_every_width(N, k, gpu_de
     assert _driven_pair(A, Wa) is None
     want = ring_rnn_cuda_func(A.clone(), Wa, -0.05, 0.5, Wo, r0, 0.15, "tanh")
     assert torch.equal(ring_rnn_cuda_func(A, Wa, -0.05, 0.5, Wo, r0, 0.15, "tanh"), want)
+
+
+@pytest.mark.parametrize("B,T,k", [(1, 1, 2), (5, 7, 3), (33, 20, 16), (700, 513, 5)])
+def test_action_signal_in_one_launch_equals_the_tensor_operations(B, T, k, gpu_device):
+    from rnn_train_ring_attractor_amd import host
+    print(f"[case] action signal B={B} T={T} k={k}", flush=True)
+    av = torch.randn(B, T, device=gpu_device)
+    av[0, 0] = float("nan")
+    av[-1, -1] = 0.0
+    for fast, slow in ((host.av_to_action_signal_ND(av, k), host.av_to_action_signal_ND(av.clone().requires_grad_(True), k)),
+                       (host.av_to_action_signal(av), host.av_to_action_signal(av.cpu()).to(gpu_device))):
+        assert fast.shape == slow.shape and torch.equal(torch.nan_to_num(fast, 7.0), torch.nan_to_num(slow.detach(), 7.0))
+
+
+@pytest.mark.parametrize("B,N,width", [(1, 1, 10), (3, 17, 10), (130, 256, 7.5), (9, 2048, 10)])
+def test_initial_bump_in_one_launch_equals_the_tensor_operations(B, N, width, gpu_device):
+    from rnn_train_ring_attractor_amd import host
+    print(f"[case] initial bump B={B} N={N}", flush=True)
+    angle = torch.rand(B, 5, device=gpu_device, dtype=torch.float32) * 6.283
+    angle[0, 0] = 0.0
+    got = host.create_initial_bump(angle[:, 0], N, width, device=gpu_device)
+    want = host.create_initial_bump(angle[:, 0].double().cpu(), N, width)
+    # the centre is N times a rounded angle: 2^-24 N neurons, against a width of N / width ones
+    assert float((got.cpu().double() - want).abs().max()) <= 4 * 2.0 ** -22 * width * float(want.max())
+    with_grad = host.create_initial_bump(angle[:, 0].clone().requires_grad_(True), N, width, device=gpu_device)
+    assert with_grad.requires_grad and float((with_grad - got).abs().max()) <= 1e-5 * float(want.max())
+
+
+def test_helpers_keep_to_tensor_operations_where_something_watches_them(gpu_device):
+    """vmap, forward mode and tracing see the operations themselves."""
+    from rnn_train_ring_attractor_amd import host
+    av = torch.randn(3, 4, 5, device=gpu_device)
+    assert torch.equal(torch.func.vmap(host.av_to_action_signal)(av), torch.stack([host.av_to_action_signal(a) for a in av]))
+    angle = torch.rand(4, device=gpu_device)
+    _, tangent = torch.func.jvp(lambda a: host.create_initial_bump(a, 32, device=gpu_device), (angle,), (torch.ones_like(angle),))
+    assert float(tangent.abs().max()) > 0
+    traced = torch.jit.trace(lambda a: host.av_to_action_signal(a), av[0])
+    assert torch.equal(traced(av[1]), host.av_to_action_signal(av[1]))

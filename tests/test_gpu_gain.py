@@ -66,3 +66,27 @@ def test_gain_gradients_are_repeatable_and_additive_at_full_size(gpu_device):
     assert O.max_rel_err(c(part[0]), O.gain_forward(c(x[sl]), c(params))) <= 1e-5
     gp, _ = O.gain_backward(c(x[sl]), c(params), c(g[sl]))
     assert O.max_rel_err(c(part[1]), gp) <= 1e-4
+
+
+@pytest.mark.parametrize("B,T,h,k", [(1, 1, 1, 1), (7, 5, 3, 2), (300, 40, 16, 2), (20, 9, 32, 16)])
+def test_networks_read_in_place_equal_the_packed_operator(B, T, h, k, gpu_device):
+    """Same kernels, parameters by pointer: the same bits, forward and every parameter's gradient; the angular velocity's
+    halves likewise."""
+    from rnn_train_ring_attractor_amd import gain
+    print(f"[case] gain networks in place B={B} T={T} h={h} k={k}", flush=True)
+    torch.manual_seed(2)
+    nets = [torch.nn.Sequential(torch.nn.Linear(1, h), torch.nn.GELU(), torch.nn.Linear(h, 1), torch.nn.Softplus()).to(gpu_device)
+            for _ in range(k)]
+    params = [p for net in nets for p in net.parameters()]
+
+    def grads(out, g):
+        return [out.detach()] + list(torch.autograd.grad(out, params, g))
+
+    x, av = torch.randn(B, T, k, device=gpu_device), torch.randn(B, T, device=gpu_device)
+    g = torch.randn(B, T, k, device=gpu_device)
+    for a, b in zip(grads(gain.ring_gain_nets(x, nets), g), grads(gain.ring_gain_func(x, gain.pack_gain_nets(nets)), g)):
+        assert a.shape == b.shape and torch.equal(a, b)
+    if k == 2:
+        base = torch.stack([torch.relu(-av), torch.relu(av)], dim=2)
+        for a, b in zip(grads(gain.ring_gain_halves(av, nets), g), grads(gain.ring_gain_func(base, gain.pack_gain_nets(nets)), g)):
+            assert torch.equal(a, b)
