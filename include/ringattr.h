@@ -228,10 +228,9 @@ RINGATTR_API int ringattr_gain_nets_bwd(const void* signal, int halves, const vo
 /* Action signal [B,T,a_dim] of an angular velocity [B,T]: relu(-av), relu(av), zeros (root
  * train_general_ring_no_gain.py:52-66). */
 RINGATTR_API int ringattr_action_signal(const void* av, void* action_signal, int a_dim, int seq_len, int batch_size, void* stream);
-/* r_init [B,N]: exp(-d^2 / two_var) over its Euclidean norm, d the circular distance in neurons to angle[b * angle_stride]
- * N / (2 pi) (train/train_ring_attractor.py:21-52). */
-RINGATTR_API int ringattr_initial_bump(const void* angle, size_t angle_stride, void* r_init, int N, int batch_size, float two_var,
-                      void* stream);
+/* bump [B,N]: exp(-d^2 / two_var), d the circular distance in neurons to angle[b * angle_stride] N / (2 pi)
+ * (train/train_ring_attractor.py:21-52, before the normalisation). */
+RINGATTR_API int ringattr_bump(const void* angle, size_t angle_stride, void* bump, int N, int batch_size, float two_var, void* stream);
 
 /* The two driven channels c0 < c1 of a zero-padded action signal (root train_general_ring_no_gain.py:52-66):
  * A_out [B,T,2] and Wa_out [2,N,N] from A [B,T,a_dim] and Wa [a_dim,N,N].  The other channels are checked on the device: if

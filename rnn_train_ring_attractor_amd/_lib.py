@@ -59,7 +59,7 @@ PROTOTYPES = {
     "ringattr_gain_nets_bwd": (c_int, [c_void_p, c_int, ctypes.POINTER(c_void_p), c_void_p, c_void_p, c_int, c_int, c_int, c_int,
                                        c_void_p, c_size_t, c_void_p]),
     "ringattr_action_signal": (c_int, [c_void_p, c_void_p, c_int, c_int, c_int, c_void_p]),
-    "ringattr_initial_bump": (c_int, [c_void_p, c_size_t, c_void_p, c_int, c_int, c_float, c_void_p]),
+    "ringattr_bump": (c_int, [c_void_p, c_size_t, c_void_p, c_int, c_int, c_float, c_void_p]),
     "ringattr_compact_workspace_bytes": (c_size_t, []),
     "ringattr_compact_channels": (c_int, [c_void_p] * 4 + [c_int] * 6 + [c_void_p, c_size_t, c_void_p]),
     "ringattr_clip_adam_workspace_bytes": (c_size_t, [c_int, ctypes.POINTER(c_size_t)]),

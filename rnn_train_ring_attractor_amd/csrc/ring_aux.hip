@@ -163,9 +163,9 @@ hipError_t ring_launch_generate(const RingGenArgs& a, hipStream_t st) {
 }
 
 // ------------------------------------------------------------------------------------------------
-// The host helpers' action signal and initial bump of given trials, a launch each.  Their chains of tensor operations (six
-// and thirteen launches of 2 to 5 us, and as much on the host's side) were 40 of the 483 us of the training script's step at
-// N = 256, B = 128, T = 100.
+// The host helpers' action signal and initial bump (before its normalisation) of given trials, a launch each.  As chains of
+// six and eleven tensor operations (2 to 5 us each, and as much on the host's side) they were 40 of the 483 us of the training
+// script's step at N = 256, B = 128, T = 100.
 // ------------------------------------------------------------------------------------------------
 // out[s][c] = relu(-av[s]), relu(av[s]), 0, 0, ...  (NaN stays NaN)
 __global__ __launch_bounds__(256) void ring_action_signal_kernel(const float* __restrict__ av, float* __restrict__ out, int k, size_t n) {
@@ -187,35 +187,24 @@ hipError_t ring_launch_action_signal(const float* av, float* out, int k, size_t 
   return hipGetLastError();
 }
 
-// out[b][i] = exp(-d^2 / two_var) / (the row's Euclidean norm), d the circular distance in neurons to angle[b * stride] N / (2 pi).
-// One workgroup per row.
-__global__ __launch_bounds__(256) void ring_initial_bump_kernel(const float* __restrict__ angle, size_t stride, float* __restrict__ out,
-                                                                int N, float two_var) {
-  __shared__ float red[4];
-  const int tid = threadIdx.x;
-  const float centre = angle[blockIdx.x * stride] * (float)N / 6.283185307179586f;
-  float* row = out + (size_t)blockIdx.x * N;
-  auto bump = [&](int i) {
-    const float d0 = fabsf((float)i - centre), d = fminf(d0, (float)N - d0);
-    return expf(-(d * d) / two_var);
-  };
-  float ss = 0.f;
-  for (int i = tid; i < N; i += 256) {
-    const float v = bump(i);
-    ss = fmaf(v, v, ss);
+// out[b][i] = exp(-d^2 / two_var), d the circular distance in neurons to angle[b * stride] N / (2 pi).  Every operation and
+// rounding is the chain's own (a division by a number is a product with its reciprocal there).
+__global__ __launch_bounds__(256) void ring_bump_kernel(const float* __restrict__ angle, size_t stride, float* __restrict__ out, int N,
+                                                        float inv_two_pi, float inv_two_var, size_t n) {
+#pragma clang fp contract(off)
+  for (size_t u = (size_t)blockIdx.x * 256 + threadIdx.x; u < n; u += (size_t)gridDim.x * 256) {
+    const size_t b = u / N;
+    const int i = (int)(u - b * N);
+    const float centre = (angle[b * stride] * (float)N) * inv_two_pi;
+    const float d0 = fabsf((float)i - centre), d1 = (float)N - d0, d = d1 < d0 ? d1 : d0;       // (an angle that is NaN stays NaN)
+    out[u] = expf(-(d * d) * inv_two_var);
   }
-  ss = row16_sum_dpp(ss);
-  const int si = __builtin_bit_cast(int, ss);
-  ss = (__builtin_bit_cast(float, __builtin_amdgcn_readlane(si, 0)) + __builtin_bit_cast(float, __builtin_amdgcn_readlane(si, 16))) +
-       (__builtin_bit_cast(float, __builtin_amdgcn_readlane(si, 32)) + __builtin_bit_cast(float, __builtin_amdgcn_readlane(si, 48)));
-  if ((tid & 63) == 0) red[tid >> 6] = ss;
-  __syncthreads();
-  const float norm = sqrtf((red[0] + red[1]) + (red[2] + red[3]));
-  for (int i = tid; i < N; i += 256) row[i] = bump(i) / norm;
 }
 
-hipError_t ring_launch_initial_bump(const float* angle, size_t stride, float* out, int N, int B, float two_var, hipStream_t st) {
-  hipLaunchKernelGGL(ring_initial_bump_kernel, dim3((unsigned)B), dim3(256), 0, st, angle, stride, out, N, two_var);
+hipError_t ring_launch_bump(const float* angle, size_t stride, float* out, int N, int B, float two_var, hipStream_t st) {
+  const size_t n = (size_t)B * N, blocks = (n + 255) / 256;
+  hipLaunchKernelGGL(ring_bump_kernel, dim3((unsigned)(blocks < 8192 ? blocks : 8192)), dim3(256), 0, st, angle, stride, out, N,
+                     1.f / 6.283185307179586f, 1.f / two_var, n);
   return hipGetLastError();
 }
 

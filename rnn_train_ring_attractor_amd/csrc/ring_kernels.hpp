@@ -177,7 +177,7 @@ hipError_t ring_launch_generate(const RingGenArgs& a, hipStream_t st);
 
 // Action signal and initial bump of given trials (ring_aux.hip).
 hipError_t ring_launch_action_signal(const float* av, float* out, int k, size_t samples, hipStream_t st);
-hipError_t ring_launch_initial_bump(const float* angle, size_t stride, float* out, int N, int B, float two_var, hipStream_t st);
+hipError_t ring_launch_bump(const float* angle, size_t stride, float* out, int N, int B, float two_var, hipStream_t st);
 
 // The two driven channels of a zero-padded action signal and their matrices (ring_aux.hip); violated: RING_COMPACT_FLAGS ints.
 constexpr int RING_COMPACT_FLAGS = 1024;

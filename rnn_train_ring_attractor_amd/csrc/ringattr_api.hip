@@ -736,11 +736,11 @@ int ringattr_action_signal(const void* av, void* action_signal, int a_dim, int s
   return RINGATTR_OK;
 }
 
-int ringattr_initial_bump(const void* angle, size_t angle_stride, void* r_init, int N, int batch_size, float two_var, void* stream) {
+int ringattr_bump(const void* angle, size_t angle_stride, void* r_init, int N, int batch_size, float two_var, void* stream) {
   if (N <= 0 || batch_size <= 0)
-    return fail(RINGATTR_ERR_INVALID, "ringattr_initial_bump: N and batch_size must be positive (got %d, %d)", N, batch_size);
-  if (!angle || !r_init) return fail(RINGATTR_ERR_INVALID, "ringattr_initial_bump: null tensor pointer");
-  hipError_t e = ring_launch_initial_bump((const float*)angle, angle_stride, (float*)r_init, N, batch_size, two_var,
+    return fail(RINGATTR_ERR_INVALID, "ringattr_bump: N and batch_size must be positive (got %d, %d)", N, batch_size);
+  if (!angle || !r_init) return fail(RINGATTR_ERR_INVALID, "ringattr_bump: null tensor pointer");
+  hipError_t e = ring_launch_bump((const float*)angle, angle_stride, (float*)r_init, N, batch_size, two_var,
                                           static_cast<hipStream_t>(stream));
   if (e != hipSuccess) return hip_fail(e, "initial bump launch");
   return RINGATTR_OK;

@@ -29,10 +29,10 @@ def create_initial_bump(initial_angles, num_neurons, bump_width_factor=10, devic
     if type(num_neurons) is int and num_neurons > 0 and type(bump_width_factor) in (int, float) and ang.dim() == 1 and plain_gpu_tensor(ang):
         sigma = num_neurons / bump_width_factor
         with torch.cuda.device(ang.device):
-            out = torch.empty(ang.shape[0], num_neurons, dtype=torch.float32, device=ang.device)
-            check(load().ringattr_initial_bump(ang.data_ptr(), ang.stride(0), out.data_ptr(), num_neurons, ang.shape[0],
-                                               2 * sigma * sigma, torch.cuda.current_stream(ang.device).cuda_stream))
-        return out
+            bump = torch.empty(ang.shape[0], num_neurons, dtype=torch.float32, device=ang.device)
+            check(load().ringattr_bump(ang.data_ptr(), ang.stride(0), bump.data_ptr(), num_neurons, ang.shape[0],
+                                       2 * sigma * sigma, torch.cuda.current_stream(ang.device).cuda_stream))
+        return bump / bump.norm(dim=1, keepdim=True)
     centre = (ang * num_neurons / (2 * math.pi)).unsqueeze(1)
     idx = torch.arange(num_neurons, device=device).unsqueeze(0)
     dist = (idx - centre).abs()
