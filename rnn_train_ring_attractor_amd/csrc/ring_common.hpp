@@ -152,6 +152,75 @@ __device__ __forceinline__ void act_scaled(float x, const ActScale& k, float& aF
   }
 }
 
+// The derivative record is fp16, and a row's record must not depend on the kernel that made it.  Left alone the compiler
+// rounds the last operation of alpha * F' once, fused with the conversion, in some kernels and twice in others.  Here a
+// kernel says which: record_pair rounds twice, ActRecord's pair and value round gelu's and tanh's once where `once` is set.
+// Once: the team kernels, and the late role (columns with bit 5 set, but for the last step) of the weight-resident forward
+// of whole tiles, with the small batches that stand in for it.  Twice: everything else.
+__device__ __forceinline__ _Float16 record_value(float d) {
+  asm("" : "+v"(d));
+  return (_Float16)d;
+}
+__device__ __forceinline__ unsigned record_pair(float d0, float d1) {
+  typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
+  return __builtin_bit_cast(unsigned, f16x2{record_value(d0), record_value(d1)});
+}
+
+// alpha * F(x), by act_scaled's operations, and what alpha * F'(x) is a single operation away from (relu and silu: itself).
+template <int ACT>
+struct ActRecord {
+  static constexpr bool FUSED = ACT == ACT_GELU || ACT == ACT_TANH;
+  float s, u;
+  __device__ __forceinline__ float apply(float x, const ActScale& k) {
+    float aF;
+    if constexpr (ACT == ACT_GELU) {
+      const float t = __builtin_amdgcn_rcpf(fmaf(fabsf(x), 0.3275911f * 0.70710678f, 1.f));
+      const float e = __builtin_amdgcn_exp2f(x * x * -0.72134752f);
+      float poly = fmaf(t, k.g4, k.g3);
+      poly = fmaf(t, poly, k.g2);
+      poly = fmaf(t, poly, k.g1);
+      poly = fmaf(t, poly, k.g0);
+      const float h = poly * t * e;
+      u = x >= 0.f ? k.a - h : h;
+      s = x * e;
+      aF = x * u;
+    } else if constexpr (ACT == ACT_TANH) {
+      const float xc = __builtin_amdgcn_fmed3f(x, -15.f, 15.f);
+      const float e2 = __builtin_amdgcn_exp2f(xc * 2.88539008f);
+      s = fmaf(-2.f, __builtin_amdgcn_rcpf(e2 + 1.f), 1.f);
+      aF = k.a * s;
+      u = aF;
+    } else {
+      act_scaled<ACT>(x, k, aF, s);
+      u = 0.f;
+    }
+    return aF;
+  }
+  __device__ __forceinline__ float derivative(const ActScale& k) const {
+    return ACT == ACT_GELU ? fmaf(s, k.gd, u) : ACT == ACT_TANH ? fmaf(-s, u, k.a) : s;
+  }
+  __device__ __forceinline__ _Float16 once(const ActScale& k) const {
+    unsigned r = 0u;
+    if constexpr (ACT == ACT_GELU) asm("v_fma_mixlo_f16 %0, %1, %2, %3" : "+v"(r) : "v"(s), "v"(k.gd), "v"(u));
+    else if constexpr (ACT == ACT_TANH) asm("v_fma_mixlo_f16 %0, -%1, %2, %3" : "+v"(r) : "v"(s), "v"(u), "v"(k.a));
+    else return record_value(s);
+    return __builtin_bit_cast(_Float16, (unsigned short)r);
+  }
+  static __device__ __forceinline__ unsigned pair_once(const ActScale& k, const ActRecord& a, const ActRecord& b) {
+    unsigned r;
+    if constexpr (ACT == ACT_GELU)
+      asm("v_fma_mixlo_f16 %0, %1, %3, %4\n\tv_fma_mixhi_f16 %0, %2, %3, %5" : "=&v"(r) : "v"(a.s), "v"(b.s), "v"(k.gd), "v"(a.u), "v"(b.u));
+    else if constexpr (ACT == ACT_TANH)
+      asm("v_fma_mixlo_f16 %0, -%1, %3, %5\n\tv_fma_mixhi_f16 %0, -%2, %4, %5" : "=&v"(r) : "v"(a.s), "v"(b.s), "v"(a.u), "v"(b.u), "v"(k.a));
+    else r = record_pair(a.s, b.s);
+    return r;
+  }
+  static __device__ __forceinline__ unsigned pair(const ActScale& k, const ActRecord& a, const ActRecord& b, bool once) {
+    const unsigned twice = record_pair(a.derivative(k), b.derivative(k));
+    return FUSED && once ? pair_once(k, a, b) : twice;
+  }
+};
+
 // Sum over the 16 lanes that share q (one MFMA column group); every lane gets the total.
 __device__ __forceinline__ float row16_sum(float v) {
   v += __shfl_xor(v, 1, 16);

@@ -1365,6 +1365,10 @@ hipError_t ring_run_team_rows(const RingFwdArgs& a, const float* Wo, const float
   ProfScope prof(1, st);
   return ring_team_rows(a, Wo, Wa, ws, st);
 }
+hipError_t ring_run_team_rows_bptt(const RingBpttArgs& a, const float* Wo, const float* Wa, void* ws, hipStream_t st) {
+  ProfScope prof(3, st);
+  return ring_team_rows_bptt(a, Wo, Wa, ws, st);
+}
 hipError_t ring_run_team_rebuild(const RingFwdArgs& a, bool folded, int cts, hipStream_t st) {
   ProfScope prof(2, st);
   return ring_team_rebuild(a, folded, cts, st);

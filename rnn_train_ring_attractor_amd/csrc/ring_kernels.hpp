@@ -140,6 +140,8 @@ hipError_t ring_launch_loss_fwd(const float* hist, const float* angle, const flo
                                 hipStream_t st);
 // where the forward kernel leaves the per-row sums for ring_launch_loss_fwd(..., have_row_sums = true)
 ring_f32x4* ring_loss_row_sums(void* workspace);
+// the three sums of every history row for 128 < N <= 256, with the bits of the weight-resident forward
+hipError_t ring_launch_row_sums256(const float* hist, ring_f32x4* stats, int N, int T, int B, hipStream_t st);
 hipError_t ring_launch_loss_bwd(const float* hist, const float* angle, const float* target_amp, float bump_weight,
                                 const float* upstream, float* grad_hist, int N, int T, int B, const void* workspace,
                                 hipStream_t st);
@@ -257,7 +259,8 @@ struct RingTeamArgs {
   int N, k, T, B, nbt, KC, G, nteams, nt, slots, cts, spin_max;
   int gather_ticks;      // how long the members of a team wait for each other, in 10 ns (negative: not at all)
   int c16, mr, wk;       // the shape, for the single workgroups that take over
-  int rows;              // non-zero: one wave sums the whole contraction, chunks in the order of rows_chunk (ring_team_rows.hip)
+  int rows;              // non-zero: one wave sums the whole contraction, in the weight-resident order (ring_team_rows.hip);
+                         // 2: the record rounded as the whole-tile kernel does (ActRecord)
 };
 struct RingTeamShape { int kpw, c16, mr, wk, lds_mats, grid; };
 struct RingTeamPlan {
@@ -274,12 +277,18 @@ size_t ring_team_bptt_bytes(int N, int k, int T, int B, bool ga);
 // J1 * Wo + J0 as one operand (folded) or kept apart; `ws` is ring_team_fwd_bytes / ring_team_bptt_bytes large
 hipError_t ring_team_fwd(const RingFwdArgs& a, const float* Wo, const float* Wa, bool folded, int cts, void* ws, hipStream_t st);
 hipError_t ring_team_bptt(const RingBpttArgs& a, const float* Wo, const float* Wa, bool folded, int cts, void* ws, hipStream_t st);
-// small batches of 128 < N <= 256 with two channels, without a record (ring_team_rows.hip)
-RingTeamPlan ring_team_rows_plan(int N, int k, int B);
-bool ring_uses_team_rows(int N, int k, int B);
-size_t ring_team_rows_bytes(int N, int k, int B);
+// small batches of 128 < N <= 256 with two channels, in the weight-resident kernels' order (ring_team_rows.hip); record: with
+// a record, and the BPTT
+RingTeamPlan ring_team_rows_plan(int N, int k, int B, bool record);
+bool ring_uses_team_rows(int N, int k, int B, bool record);
+size_t ring_team_rows_bytes(int N, int k, int B, bool record);
+size_t ring_team_rows_bptt_bytes(int N, int k, int T, int B, bool ga);
+size_t ring_team_rows_ga_bytes(int T, int B);
 hipError_t ring_team_rows(const RingFwdArgs& a, const float* Wo, const float* Wa, void* ws, hipStream_t st);
+hipError_t ring_team_rows_bptt(const RingBpttArgs& a, const float* Wo, const float* Wa, void* ws, hipStream_t st);
 hipError_t ring_launch_team_rows(const RingFwdArgs& a, const RingTeamArgs& c, const RingTeamShape& sh, hipStream_t st);
+hipError_t ring_launch_team_rows_bptt(const RingBpttArgs& a, const RingTeamArgs& c, const RingTeamShape& sh, hipStream_t st);
+hipError_t ring_launch_team_rows_ga(const float* part, float* grad_A, int T, int B, hipStream_t st);
 // 17 <= N <= 128 with up to six channels: a workgroup per batch tile (ring_team_one.hip)
 bool ring_team_one_applicable(int N, int k);
 bool ring_uses_team_one(int N, int k);
@@ -298,5 +307,6 @@ hipError_t ring_cluster_host_err(int** dev);              // the error word both
 // the same under the profiling slots
 hipError_t ring_run_team_fwd(const RingFwdArgs& a, const float* Wo, const float* Wa, bool folded, int cts, void* ws, hipStream_t st);
 hipError_t ring_run_team_rows(const RingFwdArgs& a, const float* Wo, const float* Wa, void* ws, hipStream_t st);
+hipError_t ring_run_team_rows_bptt(const RingBpttArgs& a, const float* Wo, const float* Wa, void* ws, hipStream_t st);
 hipError_t ring_run_team_rebuild(const RingFwdArgs& a, bool folded, int cts, hipStream_t st);
 hipError_t ring_run_team_bptt(const RingBpttArgs& a, const float* Wo, const float* Wa, bool folded, int cts, void* ws, hipStream_t st);

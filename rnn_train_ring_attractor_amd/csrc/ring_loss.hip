@@ -120,6 +120,39 @@ __global__ __launch_bounds__(256) void ring_loss_stats_kernel(const float* __res
   }
 }
 
+// The same sums in the order of the weight-resident forward (ring_res256.hip: eight waves of 32 columns, two to a lane, the
+// waves in turn), for the teams that stand in for it on small batches: a loss and its gradients then keep their bits.  One
+// wave per row; lane (g, n) has columns 64 g + 2 n, + 1 of wave g and those 32 further on of wave 4 + g.
+__global__ __launch_bounds__(256) void ring_row_sums256_kernel(const float* __restrict__ hist, f32x4* __restrict__ stats, int N,
+                                                               int rows) {
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, i0 = 64 * (lane >> 4) + 2 * (lane & 15);
+  float sn[2][2], cs[2][2];
+#pragma unroll
+  for (int h = 0; h < 2; ++h)
+#pragma unroll
+    for (int x = 0; x < 2; ++x) sincosf(6.283185307179586f * (float)(i0 + 32 * h + x) / (float)N, &sn[h][x], &cs[h][x]);
+  for (int row = blockIdx.x * L_ROWS_PER_BLOCK + wv; row < rows; row += gridDim.x * L_ROWS_PER_BLOCK) {
+    const float* src = hist + (size_t)row * N;
+    float r[2][2], sum[3] = {0.f, 0.f, 0.f};
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+      for (int x = 0; x < 2; ++x) r[h][x] = i0 + 32 * h + x < N ? src[i0 + 32 * h + x] : 0.f;
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const float part[3] = {row16_sum_dpp(fmaf(r[h][1], cs[h][1], r[h][0] * cs[h][0])),
+                             row16_sum_dpp(fmaf(r[h][1], sn[h][1], r[h][0] * sn[h][0])),
+                             row16_sum_dpp(fabsf(r[h][0]) + fabsf(r[h][1]))};
+#pragma unroll
+      for (int g = 0; g < 4; ++g)
+#pragma unroll
+        for (int i = 0; i < 3; ++i)
+          sum[i] += __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, part[i]), 16 * g));
+    }
+    if (lane == 0) stats[row] = f32x4{sum[0], sum[1], sum[2], 0.f};
+  }
+}
+
 // Per batch row, then per (t, b), in one launch.  A workgroup takes 16 batch rows at a time (sixteen threads per row
 // stride over t):
 //  1. target amplitude of the row, sum over t of the deviations (what flows into the target) and of their squares,
@@ -344,6 +377,12 @@ hipError_t ring_launch_loss_fwd(const float* hist, const float* angle, const flo
                      bump_weight, T, B);
   hipLaunchKernelGGL(ring_loss_final_kernel, dim3(1), dim3(256), 0, st, w.partial, dgrid, w.sq, B, 1.f / (float)rows,
                      bump_weight, loss_out);
+  return hipGetLastError();
+}
+
+hipError_t ring_launch_row_sums256(const float* hist, ring_f32x4* stats, int N, int T, int B, hipStream_t st) {
+  const int rows = T * B, blocks = (rows + L_ROWS_PER_BLOCK - 1) / L_ROWS_PER_BLOCK;
+  hipLaunchKernelGGL(ring_row_sums256_kernel, dim3(blocks < 2048 ? blocks : 2048), dim3(256), 0, st, hist, stats, N, rows);
   return hipGetLastError();
 }
 

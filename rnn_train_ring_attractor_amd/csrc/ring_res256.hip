@@ -131,6 +131,8 @@ __device__ __forceinline__ void write_half(bf16x8* half, const float (&v)[4][2],
 // sum_i |r_i|, phi_i = 2 pi i / N) in p.loss_stats[t * B + b], so that the loss needs no pass of its own over the
 // history.  Each wave reduces its 32 neurons' share over the row group's 16 lanes right after the activation, the
 // eight shares meet in LDS (buffer by step parity) and wave 0 adds them in wave order behind the next barrier.
+struct NoStores {};
+
 template <int ACT, bool SAVE, bool FULL, bool STATS>
 __global__ __launch_bounds__(512) void ring_fwd_res256_kernel(RingFwdArgs p) {
   extern __shared__ __attribute__((aligned(16))) char smem[];
@@ -157,7 +159,13 @@ __global__ __launch_bounds__(512) void ring_fwd_res256_kernel(RingFwdArgs p) {
   bf16x8* wl = wlds + (size_t)(w8 * 2 * R_KCH) * 64 + lane;
   load_resident8(reinterpret_cast<const bf16x8*>(p.Wpack), wl, wreg, w, h, lane);
 
-  float r[4][2], okf[4][2], d[4][2];
+  float r[4][2], okf[4][2];
+  // alpha F', or what it is made of (late role of whole tiles), until it is stored.  With the row sums the registers are not
+  // there: the finished fp16 pairs of rows 0, 1 and 2, 3.
+  using Record = ActRecord<ACT>;
+  float d[4][2];
+  Record late[4][2];
+  unsigned dp[2][2];
 #pragma unroll
   for (int e = 0; e < 4; ++e)
 #pragma unroll
@@ -250,7 +258,7 @@ __global__ __launch_bounds__(512) void ring_fwd_res256_kernel(RingFwdArgs p) {
   const unsigned hist_lane = (unsigned)((4 * q * 256 + 2 * n) * sizeof(float));           // + row e * 1 KiB
   const unsigned d_lane = (unsigned)((lc * 4 * R_NC + 4 * ct0) * sizeof(_Float16));        // + tile cc * 8 B
   const unsigned r_lane = (unsigned)((ct0 * 64 + lc) * 16);                                // + tile cc * 1 KiB
-  auto emit_store = [&](int t, int slot) {
+  auto emit_store = [&](int t, int slot, auto once) {
     __builtin_amdgcn_sched_barrier(0);
     if (slot < 4) {
       if (p.hist == nullptr) return;   // recompute of the saved record only: the history already exists
@@ -268,11 +276,17 @@ __global__ __launch_bounds__(512) void ring_fwd_res256_kernel(RingFwdArgs p) {
       // lane pair; two 8-byte stores would each write every other 8 bytes, and a store of partial sectors costs the
       // wave several times what a whole one costs
       if (SAVE && slot == 4) {
-        typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
         char* base = reinterpret_cast<char*>(p.dfrag + side_offset<R_NC>(t, p.nbt, bt, wu, 0));
-        const f16x8 pk = {(_Float16)d[0][0], (_Float16)d[1][0], (_Float16)d[2][0], (_Float16)d[3][0],
-                          (_Float16)d[0][1], (_Float16)d[1][1], (_Float16)d[2][1], (_Float16)d[3][1]};
-        *reinterpret_cast<f16x8*>(base + d_lane) = pk;
+        typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
+        u32x4 pk;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const int e = 2 * (i & 1), cc = i >> 1;
+          if constexpr (STATS) pk[i] = dp[cc][e / 2];
+          else if constexpr (decltype(once)::value) pk[i] = Record::pair_once(asc, late[e][cc], late[e + 1][cc]);
+          else pk[i] = record_pair(d[e][cc], d[e + 1][cc]);
+        }
+        *reinterpret_cast<u32x4*>(base + d_lane) = pk;
       }
     } else if (SAVE) {
       const int cc = slot - 6;   // r after step t is the operand of step t+1
@@ -322,7 +336,7 @@ __global__ __launch_bounds__(512) void ring_fwd_res256_kernel(RingFwdArgs p) {
     __builtin_amdgcn_s_setprio(3);
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-      if constexpr (decltype(emit)::value) emit_store(ts, 4 * ph + j);
+      if constexpr (!std::is_same<decltype(emit), NoStores>::value) emit_store(ts, 4 * ph + j, emit);
       mfma_unit(4 * ph + j, af);
     }
     __builtin_amdgcn_s_setprio(0);
@@ -340,24 +354,32 @@ __global__ __launch_bounds__(512) void ring_fwd_res256_kernel(RingFwdArgs p) {
       }
     }
   };
-  auto activate = [&](const float (&x)[4][2]) {
+  // once: round the record's last operation once (ActRecord)
+  auto activate = [&](const float (&x)[4][2], auto once) {
 #pragma unroll
     for (int e = 0; e < 4; ++e)
 #pragma unroll
       for (int cc = 0; cc < 2; ++cc) {
-        float aF, aD;
-        act_scaled<ACT>(x[e][cc], asc, aF, aD);
+        float aF;
+        if constexpr (decltype(once)::value) aF = late[e][cc].apply(x[e][cc], asc);
+        else act_scaled<ACT>(x[e][cc], asc, aF, d[e][cc]);
         float rn = fmaf(oma, r[e][cc], aF);
         if constexpr (!FULL) {
           rn *= okf[e][cc];
-          aD *= okf[e][cc];
+          d[e][cc] *= okf[e][cc];                  // (never `once`)
         }
         r[e][cc] = rn;
-        d[e][cc] = aD;          // the saved record is alpha * F'(re)
+        if constexpr (SAVE && STATS) {
+          if (e & 1) {
+            if constexpr (decltype(once)::value) dp[cc][e / 2] = Record::pair_once(asc, late[e - 1][cc], late[e][cc]);
+            else dp[cc][e / 2] = record_pair(d[e - 1][cc], d[e][cc]);
+          }
+        }
       }
   };
-  constexpr std::true_type with_stores{};
-  constexpr std::false_type no_stores{};
+  constexpr std::bool_constant<SAVE && FULL && Record::FUSED> late_once{};
+  constexpr std::false_type with_stores{};
+  constexpr NoStores no_stores{};
   if (h == 0) {
     // ---------------- role E ----------------
     auto e_step = [&](int t, auto emit) {
@@ -371,7 +393,7 @@ __global__ __launch_bounds__(512) void ring_fwd_res256_kernel(RingFwdArgs p) {
       contract_half(1, xL, t - 1, emit);
       float x[4][2];
       preactivation(t, x);
-      activate(x);
+      activate(x, std::false_type{});
       if constexpr (STATS) stat_share(t);
       if (t + 1 < T) write_half(xE + ((t + 1) & 1) * R8_HALF_SLOTS, r, w, q, n);
       // the next chunk's gates are first read after barrier B of its first step
@@ -389,16 +411,16 @@ __global__ __launch_bounds__(512) void ring_fwd_res256_kernel(RingFwdArgs p) {
     preactivation(0, x);
     lds_barrier();   // A_1
     for (int t = 1; t < T; ++t) {
-      activate(x);   // step t-1 -> r^L_t
+      activate(x, late_once);   // step t-1 -> r^L_t
       if constexpr (STATS) stat_share(t - 1);
       write_half(xL, r, w, q, n);
       lds_barrier();   // B_t
-      contract_half(0, xE + (t & 1) * R8_HALF_SLOTS, t - 1, with_stores);
-      contract_half(1, xL, t - 1, with_stores);
+      contract_half(0, xE + (t & 1) * R8_HALF_SLOTS, t - 1, late_once);
+      contract_half(1, xL, t - 1, late_once);
       preactivation(t, x);
       lds_barrier();   // A_{t+1}
     }
-    activate(x);
+    activate(x, std::false_type{});
     if constexpr (STATS) stat_share(T - 1);
   }
   if constexpr (STATS) {
@@ -407,7 +429,7 @@ __global__ __launch_bounds__(512) void ring_fwd_res256_kernel(RingFwdArgs p) {
   }
   // stores of the last step (its state is not an operand of any further step)
 #pragma unroll
-  for (int slot = 0; slot < 6; ++slot) emit_store(T - 1, slot);
+  for (int slot = 0; slot < 6; ++slot) emit_store(T - 1, slot, std::false_type{});
 }
 
 // ------------------------------------------------------------------------------------------------

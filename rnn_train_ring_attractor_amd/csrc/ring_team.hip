@@ -118,11 +118,10 @@ static bool forced() {
 //   N = 512, a_dim 2:  B = 64: 8.9 -> 1.6 / 29.1 -> 3.7   B = 2048: 14.3 -> 5.5 / 32.4 -> 14.8
 //   N = 1024, a_dim 2: B = 64: 17.8 -> 3.3 / 43 -> 6.9    B = 2048: 40 -> 19 / 104 -> 50
 // against the streaming and step-per-launch kernels.  The exceptions:
-//   * 128 < N <= 256 with two channels belongs to the weight-resident kernels at every batch, whole tiles or not, also
-//     where teams are faster (N = 200, B = 64, forward and backward: 4.9 against 3.0), because they are far ahead on large
-//     batches (N = 200, B = 4096: 7.4 against 10.5) and a slice of a batch has to reproduce its rows bit for bit: the two
-//     families sum in a different order, so one of them has to have all batches (small ones without a record run on
-//     teams that sum in the weight-resident order: ring_team_rows.hip);
+//   * 128 < N <= 256 with two channels belongs to the weight-resident kernels, which are far ahead on large batches (N = 200,
+//     B = 4096, forward and backward: 7.4 against 10.5).  A slice of a batch has to reproduce its rows bit for bit and the two
+//     families sum in a different order, so batches of up to 512 rows run on teams that sum in the weight-resident order
+//     (ring_team_rows.hip; N = 200, B = 64: 2.0 against 3.8 on the weight-resident kernels and 3.0 on these teams);
 //   * with many tiles per team (more than eight at N <= 512) a compute unit's epilogue work is what bounds a step, and
 //     the kernels that have a batch tile to themselves, or the N = 512 clusters, are faster (N = 360, B = 6000, forward
 //     and backward: 49 against 43 us per step with nine tiles, B = 8192: 53 against 68 with thirteen; N = 512, B = 4608:
@@ -152,11 +151,16 @@ static bool teams_allowed() {
 
 bool ring_uses_team(int N, int k, int T, int B) { return teams_allowed() && team_shape(N, k, T, B); }
 
-// Same bits as the weight-resident forward, so the batch may decide: wherever every batch tile gets a team.
-bool ring_uses_team_rows(int N, int k, int B) { return !forced() && teams_allowed() && ring_team_rows_plan(N, k, B).ok; }
-size_t ring_team_rows_bytes(int N, int k, int B) {
-  const RingTeamPlan p = ring_team_rows_plan(N, k, B);
+// Same bits and record as the weight-resident kernels, so the batch may decide: wherever every batch tile gets a team.
+bool ring_uses_team_rows(int N, int k, int B, bool record) {
+  return !forced() && teams_allowed() && ring_uses_resident(N, k) && ring_team_rows_plan(N, k, B, record).ok;
+}
+size_t ring_team_rows_bytes(int N, int k, int B, bool record) {
+  const RingTeamPlan p = ring_team_rows_plan(N, k, B, record);
   return p.ok ? p.xchg_bytes + p.gather_bytes : 0;
+}
+size_t ring_team_rows_bptt_bytes(int N, int k, int T, int B, bool ga) {
+  return ring_team_rows_bytes(N, k, B, true) + (ga ? ring_team_rows_ga_bytes(T, B) : 0);
 }
 
 // Scratch of one launch; none where no call of this shape comes here.
@@ -243,14 +247,29 @@ hipError_t ring_team_fwd(const RingFwdArgs& a, const float* Wo, const float* Wa,
 }
 
 hipError_t ring_team_rows(const RingFwdArgs& a, const float* Wo, const float* Wa, void* ws, hipStream_t st) {
-  const RingTeamPlan p = ring_team_rows_plan(a.N, a.k, a.B);
-  if (!p.ok || !ws || !a.hist || a.dfrag || a.rfrag) return hipErrorInvalidValue;
+  const bool record = a.dfrag != nullptr;
+  const RingTeamPlan p = ring_team_rows_plan(a.N, a.k, a.B, record);
+  if (!p.ok || !ws || !a.hist || record != (a.rfrag != nullptr)) return hipErrorInvalidValue;
   RingTeamArgs c;
-  hipError_t e = team_args(p, Wo, Wa, a.A, a.J0, a.J1, true, a.N, a.k, a.T, a.B, 0, ws, c, st);
+  hipError_t e = team_args(p, Wo, Wa, a.A, a.J0, a.J1, true, a.N, a.k, a.T, a.B, 16, ws, c, st);
+  if (e != hipSuccess) return e;
+  c.wk = 1;
+  c.rows = a.N == 256 && a.B % 16 == 0 ? 2 : 1;
+  e = ring_launch_team_rows(a, c, p.shape, st);
+  if (e == hipSuccess) e = ring_launch_team_solo_fwd(a, c, st);
+  return e == hipSuccess && a.loss_stats ? ring_launch_row_sums256(a.hist, a.loss_stats, a.N, a.T, a.B, st) : e;
+}
+
+hipError_t ring_team_rows_bptt(const RingBpttArgs& a, const float* Wo, const float* Wa, void* ws, hipStream_t st) {
+  const RingTeamPlan p = ring_team_rows_plan(a.N, a.k, a.B, true);
+  if (!p.ok || !ws) return hipErrorInvalidValue;
+  RingTeamArgs c;
+  hipError_t e = team_args(p, Wo, Wa, a.A, a.J0, a.J1, true, a.N, a.k, a.T, a.B, 16, ws, c, st);
   if (e != hipSuccess) return e;
   c.wk = c.rows = 1;
-  e = ring_launch_team_rows(a, c, p.shape, st);
-  return e == hipSuccess ? ring_launch_team_solo_fwd(a, c, st) : e;
+  e = ring_launch_team_rows_bptt(a, c, p.shape, st);
+  if (e == hipSuccess) e = ring_launch_team_solo_bptt(a, c, st);
+  return e == hipSuccess && a.grad_A ? ring_launch_team_rows_ga(c.ga_part, a.grad_A, a.T, a.B, st) : e;
 }
 
 hipError_t ring_team_rebuild(const RingFwdArgs& a, bool folded, int cts, hipStream_t st) {

@@ -75,13 +75,6 @@ __device__ __forceinline__ unsigned pack_bf16(float lo, float hi) {
   return __builtin_bit_cast(unsigned, v);
 }
 
-// The derivative record's fp16.  (The value is rounded to fp32 first: left alone the compiler forms it in one fused operation
-// in some kernels and not in others, and a row's record would depend on the kernel.)
-__device__ __forceinline__ _Float16 record_value(float d) {
-  asm("" : "+v"(d));
-  return (_Float16)d;
-}
-
 __device__ __forceinline__ unsigned dpp_xor1(unsigned x) { return (unsigned)__builtin_amdgcn_update_dpp(0, (int)x, 0xB1, 0xF, 0xF, false); }
 __device__ __forceinline__ unsigned dpp_xor2(unsigned x) { return (unsigned)__builtin_amdgcn_update_dpp(0, (int)x, 0x4E, 0xF, 0xF, false); }
 template <int CTRL>
@@ -677,12 +670,10 @@ struct TeamAux {
   __device__ __forceinline__ size_t dact_offset(int t, int nbt, int bt, int cts) const {
     return (((size_t)t * nbt + bt) * cts + (ct < cts ? ct : cts - 1)) * 256 + (map.q * 16 + map.b) * 4 + 2 * map.p;
   }
-  __device__ __forceinline__ void dact_store(_Float16* base, int t, int nbt, int bt, int cts, const float (&d)[NPT]) const {
+  __device__ __forceinline__ void dact_store(_Float16* base, int t, int nbt, int bt, int cts, const unsigned (&d)[NPT / 2]) const {
     const __amdgpu_buffer_rsrc_t r = team_buffer(base + ((size_t)t * nbt + bt) * cts * 256, base ? (size_t)cts * 512 : 0);
-    if constexpr (NPT == 4)
-      __builtin_amdgcn_raw_buffer_store_b64(
-          __builtin_bit_cast(u32x2, f16x4{record_value(d[0]), record_value(d[1]), record_value(d[2]), record_value(d[3])}), r, (int)d_off, 0, 0);
-    else __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, f16x2{record_value(d[0]), record_value(d[1])}), r, (int)d_off, 0, 0);
+    if constexpr (NPT == 4) __builtin_amdgcn_raw_buffer_store_b64(u32x2{d[0], d[1]}, r, (int)d_off, 0, 0);
+    else __builtin_amdgcn_raw_buffer_store_b32(d[0], r, (int)d_off, 0, 0);
   }
   // operand copy for the weight gradients: steps 2j (lo) and 2j + 1 (hi) of a neuron's four rows side by side
   __device__ __forceinline__ void pair_put(__bf16* base, int t, int nbt, int bt, int cts, const unsigned (&lo)[NPT / 2],

@@ -65,10 +65,11 @@ __global__ __launch_bounds__(64 * (WK + AUX)) void ring_team_fwd_kernel(RingFwdA
     for (int i = 0; i < NPT; ++i) r[i] = state[(size_t)j * C16 * 256 + i];
     tg.put(gl + ((it + 1) & 1) * c.k * 16, g);              // the next item's gates, fetched two items ago
     lds_barrier();                                          // the item's shares are complete
-    float x[NPT], aF[NPT], aD[NPT], rn[NPT];
+    float x[NPT], aF[NPT], rn[NPT];
+    ActRecord<ACT> rd[NPT];
     aux.template sum_shares<WK>(share, it & 1, x);
 #pragma unroll
-    for (int i = 0; i < NPT; ++i) act_scaled<ACT>(x[i], asc, aF[i], aD[i]);
+    for (int i = 0; i < NPT; ++i) aF[i] = rd[i].apply(x[i], asc);
     // Rows past B need no mask: their operand, row sum and initial state are zero and every F(0) is zero.  Neurons past N
     // see the J0 term.
 #pragma unroll
@@ -82,7 +83,10 @@ __global__ __launch_bounds__(64 * (WK + AUX)) void ring_team_fwd_kernel(RingFwdA
     }
     aux.refill(c, rsrc, slot == 0 ? c.slots - 1 : slot - 1, bt);
     aux.row_store(p.hist + (size_t)t * B * N, N, B, bt, rn);
-    aux.dact_store(p.dfrag, t, nbt, bt, c.cts, aD);
+    unsigned d[NPT / 2];
+#pragma unroll
+    for (int i = 0; i < NPT / 2; ++i) d[i] = ActRecord<ACT>::pair_once(asc, rd[2 * i], rd[2 * i + 1]);
+    aux.dact_store(p.dfrag, t, nbt, bt, c.cts, d);
     if (save && (t & 1) == 0) {        // this step's operand and the next one's are both in hand: one 16-byte slot
       unsigned lo[NPT / 2], hi[NPT / 2];
 #pragma unroll

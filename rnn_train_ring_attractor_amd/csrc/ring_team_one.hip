@@ -337,11 +337,11 @@ __global__ __launch_bounds__(128 * KCT, 2) void ring_team_one_fwd_kernel(RingFwd
     o.own(all, pre);
 #pragma unroll
     for (int i = 0; i < EPL; ++i) {
-      float aF, aD;
-      act_scaled<ACT>(pre[i], asc, aF, aD);
+      ActRecord<ACT> rd;
+      const float aF = rd.apply(pre[i], asc);
       before[i] = r[i];
       r[i] = o.j0 + i < N ? fmaf(oma, r[i], aF) : 0.f;       // (rows past B stay zero by themselves)
-      d[i] = record_value(aD);
+      d[i] = rd.once(asc);
     }
     one_put(L, even ? 1 : 0, o, sums, r);
     lds_barrier();

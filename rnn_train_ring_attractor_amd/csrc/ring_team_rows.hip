@@ -1,17 +1,23 @@
-// Forward without a record over small teams for 128 < N <= 256 with two channels (protocol and pieces: ring_team.hpp),
-// with the bits of the weight-resident forward (ring_res256.hip), so that a row comes out the same in any batch.
+// Time loops over small teams for 128 < N <= 256 with two channels (protocol and pieces: ring_team.hpp), with the bits and
+// the record of the weight-resident kernels (ring_res256.hip), so that a row comes out the same in any batch and either
+// family's backward reads either one's record.
 //
-// That forward gives one compute unit the whole ring, 24 products for each of its 16 column tiles, and B = 1 pays the same
-// step as B = 4096.  Here a member of a team has two column tiles and a compute wave the 24 products of one: it
-// sums the whole contraction in the resident kernel's order, its K chunks first the even and then the odd ones, every
-// matrix in an accumulator of its own, the gates afterwards.  One batch tile per team, so up to 32 tiles.
-// us per call, T = 100, gelu: N = 256, B = 1: 142 -> 105; N = 256, B = 512: 137 -> 120; N = 200, B = 64: 142 -> 108.
+// Those kernels give one compute unit the whole ring, 24 products for each of its 16 column tiles, and B = 1 pays the same
+// step as B = 4096.  Here a member of a team has two column tiles and a compute wave the 24 products of one: it sums the
+// whole contraction in the resident kernel's order (forward: its K chunks first the even and then the odd ones; BPTT: one
+// after the other, the ungated sum starting from (1 - alpha) G), every matrix in an accumulator of its own, the gates
+// afterwards.  One batch tile per team, so up to 32 tiles.
+// us per call, T = 100, weight-resident kernels -> here.  With a record: N = 256, B = 128, gelu: forward 143 -> 117, BPTT
+// 138 -> 130; N = 200, B = 64: 156 -> 110 and 245 -> 120; N = 256, B = 128, relu, with the loss's gradient and dL/dA:
+// 165 -> 114 (its row sums by a pass of their own included) and 222 -> 149.  Without: N = 256, B = 1: 142 -> 99.
 // What bounds it is the hand-over's latency and the chain of 24 products (some 400 cycles).
 #include "ring_team.hpp"
 
 namespace {
 
 constexpr int ROWS_TILES = 2, ROWS_CHUNKS = 8, ROWS_MATS = 3, ROWS_SLOTS = 8;
+// (the plan has room for one column tile's dL/dA shares, behind everything else)
+constexpr unsigned ROWS_GA_MORE = 2 * 2 * (ROWS_TILES - 1) * 16 * sizeof(float);
 
 struct RowsOperand {
   u32x4 x[ROWS_CHUNKS];
@@ -29,11 +35,83 @@ struct RowsOperand {
   }
 };
 
-}  // namespace
+// The weight fragments of one column tile, K chunk number i in the direction's order.
+template <bool TR>
+__device__ __forceinline__ void rows_weights(const RingTeamArgs& c, int out, int q, bf16x8 (&wt)[ROWS_MATS][ROWS_CHUNKS]) {
+  auto load = [&](auto how) {
+    constexpr int HOW = decltype(how)::value, BATCH = HOW == WEIGHT_ROWS4 ? 8 : 4;
+#pragma unroll
+    for (int m = 0; m < ROWS_MATS; ++m)
+#pragma unroll
+      for (int i0 = 0; i0 < ROWS_CHUNKS; i0 += BATCH) {
+        WeightLoad l[BATCH];
+        const float* W = m == 0 ? c.Wo : c.Wa + (size_t)(m - 1) * c.N * c.N;
+#pragma unroll
+        for (int i = 0; i < BATCH; ++i) weight_load<HOW>(l[i], W, c.N, out, 32 * (TR ? i0 + i : rows_chunk(i0 + i)) + 8 * q);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int i = 0; i < BATCH; ++i) {
+          bf16x8 f = weight_fragment(l[i], c.N, out, 32 * (TR ? i0 + i : rows_chunk(i0 + i)) + 8 * q, m == 0 ? c.scale0 : 1.f, m == 0 ? c.shift0 : 0.f);
+          asm volatile("" : "+v"(f));              // (here, not at its first use: twice the registers until then)
+          wt[m][i0 + i] = f;
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      }
+  };
+  if constexpr (TR) load(std::integral_constant<int, WEIGHT_COLUMNS>{});
+  else if ((c.N & 3) == 0) load(std::integral_constant<int, WEIGHT_ROWS4>{});
+  else load(std::integral_constant<int, WEIGHT_ROWS>{});
+}
 
-template <int ACT>
-__global__ __launch_bounds__(64 * (ROWS_TILES + AUX)) void ring_team_rows_kernel(RingFwdArgs p, RingTeamArgs c) {
-  extern __shared__ __attribute__((aligned(16))) char lds[];
+// A compute wave's place in the exchange: its operand's chunks in the direction's order.  Rows past the batch are not there.
+template <bool TR>
+__device__ __forceinline__ void rows_places(const RingTeamArgs& c, int lane, int rows, unsigned (&at)[ROWS_CHUNKS]) {
+#pragma unroll
+  for (int i = 0; i < ROWS_CHUNKS; ++i) {
+    const int kc = TR ? i : rows_chunk(i);
+    at[i] = kc < c.KC && (lane & 15) < rows ? (unsigned)kc * CHUNK_BYTES + lane * 16 : NOWHERE;        // (past the contraction: zeros)
+  }
+}
+
+// Waits until the operand under `base` is complete.
+__device__ __forceinline__ void rows_wait(RowsOperand& op, const RingTeamArgs& c, __amdgpu_buffer_rsrc_t rsrc, const unsigned (&at)[ROWS_CHUNKS],
+                                          unsigned base, bool& dead, int lane) {
+  int spins = 0;
+  while (!dead && !op.ready()) {
+    if (++spins > c.spin_max) {
+      dead = true;
+      if (lane == 0) *c.host_err = RING_CLUSTER_ERR_WAIT;
+    }
+    op.issue(rsrc, at, base);
+  }
+  __builtin_amdgcn_s_waitcnt(0x0F70);    // vmcnt(0), for the compiler's books: this operand has landed on every path
+}
+
+// Where an auxiliary thread's two neurons go in the weight-resident kernels' record (split tile order: neuron j is in tile
+// 4 (j / 64) + j % 4, column j % 64 / 4), byte offsets inside a batch tile.  After the quad exchange a lane has all four
+// rows of neuron j0 + (lane & 1).
+struct RowsRecord {
+  unsigned d_off, p_off;
+  bool row_ok;
+  __device__ __forceinline__ RowsRecord(const TeamAux<ROWS_TILES>& aux, int rows) {
+    const int lane = aux.lane, j = aux.j0 + (lane & 1), rq = aux.map.b >> 2, w = j >> 6, n = (j & 63) >> 2, cc = j & 3;
+    d_off = (lane & 2) ? NOWHERE : (unsigned)((w * 64 + rq * 16 + n) * 32 + cc * 8);
+    p_off = (unsigned)(((w * 4 + cc) * 64 + rq * 16 + n) * 16 + (lane & 2) * 4);
+    row_ok = aux.map.b < rows;
+  }
+  __device__ __forceinline__ void dact_store(_Float16* base, int t, int nbt, int bt, int lane, unsigned d) const {
+    const u32x2 x = quad_rows2(d, lane);
+    __builtin_amdgcn_raw_buffer_store_b64(x, team_buffer(base + ((size_t)t * nbt + bt) * 4096, 8192), (int)d_off, 0, 0);
+  }
+  // steps t (even; otherwise nothing is stored) and t + 1
+  __device__ __forceinline__ void pair_store(__bf16* base, int t, bool even, int nbt, int bt, int lane, unsigned lo, unsigned hi) const {
+    const u32x2 a = quad_rows2(lo, lane), d = quad_rows2(hi, lane);
+    __builtin_amdgcn_raw_buffer_store_b64((lane & 2) ? d : a, team_buffer(base + ((size_t)(t >> 1) * nbt + bt) * 8192, even ? 16384 : 0), (int)p_off, 0, 0);
+  }
+};
+
+template <int ACT, bool SAVE>
+__device__ __forceinline__ void rows_forward(const RingFwdArgs& p, const RingTeamArgs& c, char* lds) {
   using TA = TeamAux<ROWS_TILES>;
   using AM = typename TA::AM;
   constexpr int NPT = TA::NPT;
@@ -46,39 +124,14 @@ __global__ __launch_bounds__(64 * (ROWS_TILES + AUX)) void ring_team_rows_kernel
   const unsigned tile_at = (unsigned)team * tile_bytes;
   float* const share = reinterpret_cast<float*>(lds + L.share);
   float* const gl = reinterpret_cast<float*>(lds + L.gates);
-  const int T = p.T;
+  const int T = p.T, rows = p.B - 16 * team;
 
   if (w < ROWS_TILES) {
-    const int q = lane >> 4, b = lane & 15, out = 16 * (mem * ROWS_TILES + w) + b;
+    const int q = lane >> 4, b = lane & 15;
     unsigned at[ROWS_CHUNKS];
+    rows_places<false>(c, lane, rows, at);
     bf16x8 wt[ROWS_MATS][ROWS_CHUNKS];
-#pragma unroll
-    for (int i = 0; i < ROWS_CHUNKS; ++i) {
-      const int kc = rows_chunk(i);
-      at[i] = kc < c.KC ? (unsigned)kc * CHUNK_BYTES + lane * 16 : NOWHERE;        // (past the contraction: zeros)
-    }
-    auto load = [&](auto how) {
-      constexpr int HOW = decltype(how)::value, BATCH = HOW == WEIGHT_ROWS4 ? 8 : 4;
-#pragma unroll
-      for (int m = 0; m < ROWS_MATS; ++m)
-#pragma unroll
-        for (int i0 = 0; i0 < ROWS_CHUNKS; i0 += BATCH) {
-          WeightLoad l[BATCH];
-          const float* W = m == 0 ? c.Wo : c.Wa + (size_t)(m - 1) * c.N * c.N;
-#pragma unroll
-          for (int i = 0; i < BATCH; ++i) weight_load<HOW>(l[i], W, c.N, out, 32 * rows_chunk(i0 + i) + 8 * q);
-          __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-          for (int i = 0; i < BATCH; ++i) {
-            bf16x8 f = weight_fragment(l[i], c.N, out, 32 * rows_chunk(i0 + i) + 8 * q, m == 0 ? c.scale0 : 1.f, m == 0 ? c.shift0 : 0.f);
-            asm volatile("" : "+v"(f));              // (here, not at its first use: twice the registers until then)
-            wt[m][i0 + i] = f;
-          }
-          __builtin_amdgcn_sched_barrier(0);
-        }
-    };
-    if ((c.N & 3) == 0) load(std::integral_constant<int, WEIGHT_ROWS4>{});
-    else load(std::integral_constant<int, WEIGHT_ROWS>{});
+    rows_weights<false>(c, 16 * (mem * ROWS_TILES + w) + b, q, wt);
     lds_barrier();                                        // the first gates are in LDS
     if (!team_go(lds, L)) return;
     float* const dst = share + w * AM::SHARE + q * AM::QS + b * 4;
@@ -90,15 +143,7 @@ __global__ __launch_bounds__(64 * (ROWS_TILES + AUX)) void ring_team_rows_kernel
     for (int t = 0; t < T; ++t) {
       const float* g = gl + (t & 1) * c.k * 16 + b;
       const float g1 = g[0], g2 = g[16];
-      int spins = 0;
-      while (!dead && !op.ready()) {
-        if (++spins > c.spin_max) {
-          dead = true;
-          if (lane == 0) *c.host_err = RING_CLUSTER_ERR_WAIT;
-        }
-        op.issue(rsrc, at, (unsigned)slot * slot_bytes + tile_at);
-      }
-      __builtin_amdgcn_s_waitcnt(0x0F70);    // vmcnt(0), for the compiler's books: this operand has landed on every path
+      rows_wait(op, c, rsrc, at, (unsigned)slot * slot_bytes + tile_at, dead, lane);
       f32x4 P0 = {0.f, 0.f, 0.f, 0.f}, P1 = P0, P2 = P0;
 #pragma unroll
       for (int i = 0; i < ROWS_CHUNKS; ++i) {
@@ -121,13 +166,18 @@ __global__ __launch_bounds__(64 * (ROWS_TILES + AUX)) void ring_team_rows_kernel
   __builtin_amdgcn_s_setprio(3);
   TA aux(c, mem, tid - 64 * ROWS_TILES);
   team_arrive(c, team, aux.at);
+  const RowsRecord rec(aux, rows);
   const int N = p.N, B = p.B;
   const float oma = 1.f - p.alpha;
   const ActScale asc = act_scale_make(p.alpha);
-  auto put = [&](int slot, unsigned x) { __builtin_amdgcn_raw_buffer_store_b32(x, rsrc, (int)aux.x_off, (int)((unsigned)slot * slot_bytes + tile_at), ST_LOCAL); };
+  const unsigned d_mask = rec.row_ok ? (aux.j0 < N ? 0xFFFFu : 0u) | (aux.j0 + 1 < N ? 0xFFFF0000u : 0u) : 0u;
+  const bool late_once = c.rows == 2 && (aux.j0 & 32);
+  const unsigned x_off = rec.row_ok ? aux.x_off : NOWHERE;
+  auto put = [&](int slot, unsigned x) { __builtin_amdgcn_raw_buffer_store_b32(x, rsrc, (int)x_off, (int)((unsigned)slot * slot_bytes + tile_at), ST_LOCAL); };
   float r[NPT];
   aux.row_load(p.r_init, N, B, team, r);
-  put(0, not_empty(pack_bf16(r[0], r[1])));
+  unsigned before = pack_bf16(r[0], r[1]);
+  put(0, not_empty(before));
   const TeamGates tg(c, aux.at);
   auto gates_of = [&](int t) { return tg.fetch(c, t < T ? t : T - 1, team); };
   tg.put(gl, gates_of(0));
@@ -137,38 +187,286 @@ __global__ __launch_bounds__(64 * (ROWS_TILES + AUX)) void ring_team_rows_kernel
   if (!team_go(lds, L)) return;
 
   int slot = 0, t = 0;
-  auto step = [&](float& g) {
+  auto step = [&](bool even, float& g) {
     tg.put(gl + ((t + 1) & 1) * c.k * 16, g);               // the next step's gates, fetched two steps ago
     lds_barrier();                                          // the step's products are complete
-    float x[NPT], rn[NPT];
+    float x[NPT], rn[NPT], aF[NPT];
     aux.template sum_shares<1>(share, t & 1, x);
+    ActRecord<ACT> rd[NPT];
 #pragma unroll
-    for (int i = 0; i < NPT; ++i) {
-      float aF, aD;
-      act_scaled<ACT>(x[i], asc, aF, aD);
-      rn[i] = aux.j0 + i < N ? fmaf(oma, r[i], aF) : 0.f;
-    }
+    for (int i = 0; i < NPT; ++i) aF[i] = rd[i].apply(x[i], asc);
+#pragma unroll
+    for (int i = 0; i < NPT; ++i) rn[i] = aux.j0 + i < N ? fmaf(oma, r[i], aF[i]) : 0.f;
     const int next_slot = slot + 1 == ROWS_SLOTS ? 0 : slot + 1;
-    put(next_slot, not_empty(pack_bf16(rn[0], rn[1])));     // (after the last step: nobody looks)
+    const unsigned now = pack_bf16(rn[0], rn[1]);
+    put(next_slot, not_empty(now));                         // (after the last step: nobody looks)
     g = gates_of(t + 3);
     put(slot == 0 ? ROWS_SLOTS - 1 : slot - 1, EMPTY);
     aux.row_store(p.hist + (size_t)t * B * N, N, B, team, rn);
+    if constexpr (SAVE) {
+      rec.dact_store(p.dfrag, t, p.nbt, team, lane, ActRecord<ACT>::pair(asc, rd[0], rd[1], late_once && t + 1 < T) & d_mask);
+      if (even) rec.pair_store(p.rfrag, t, true, p.nbt, team, lane, before, t + 1 < T ? now : 0u);
+      before = now;
+    }
 #pragma unroll
     for (int i = 0; i < NPT; ++i) r[i] = rn[i];
     slot = next_slot;
     ++t;
   };
   while (t < T) {
-    step(gA);
+    step(true, gA);
     if (t >= T) return;
-    step(gB);
+    step(false, gB);
   }
 }
 
-RingTeamPlan ring_team_rows_plan(int N, int k, int B) {
+}  // namespace
+
+template <int ACT>
+__global__ __launch_bounds__(64 * (ROWS_TILES + AUX)) void ring_team_rows_kernel(RingFwdArgs p, RingTeamArgs c) {
+  extern __shared__ __attribute__((aligned(16))) char lds[];
+  rows_forward<ACT, false>(p, c, lds);
+}
+
+// With the weight-resident kernels' record.
+template <int ACT>
+__global__ __launch_bounds__(64 * (ROWS_TILES + AUX)) void ring_team_res256_fwd_kernel(RingFwdArgs p, RingTeamArgs c) {
+  extern __shared__ __attribute__((aligned(16))) char lds[];
+  rows_forward<ACT, true>(p, c, lds);
+}
+
+// ------------------------------------------------------------------------------------------------
+// BPTT.  Operand number s is g of step T - 1 - s, the products of round s give the carry into step T - 2 - s.  The ungated
+// sum starts from (1 - alpha) G: the auxiliary waves leave it in LDS before they publish g, so a wave that has seen all of g
+// finds it there.
+// ------------------------------------------------------------------------------------------------
+template <bool GA>
+__global__ __launch_bounds__(64 * (ROWS_TILES + AUX)) void ring_team_res256_bptt_kernel(RingBpttArgs p, RingTeamArgs c) {
+  extern __shared__ __attribute__((aligned(16))) char lds[];
+  using TA = TeamAux<ROWS_TILES>;
+  using AM = typename TA::AM;
+  constexpr int NPT = TA::NPT;
+  int team, mem;
+  if (!team_coords(c, team, mem)) return;
+  const LdsPlan L = lds_plan<ROWS_TILES, 1>(c.k, 1, 0, c.KC, 0, true, GA);
+  const int tid = threadIdx.x, w = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+  const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(c.xchg, 0, (int)c.xchg_bytes, 0x00020000);
+  const unsigned tile_bytes = (unsigned)c.KC * CHUNK_BYTES, slot_bytes = tile_bytes * (unsigned)c.nbt;
+  const unsigned tile_at = (unsigned)team * tile_bytes;
+  float* const share = reinterpret_cast<float*>(lds + L.share);
+  float* const keep = reinterpret_cast<float*>(lds + L.state);        // (1 - alpha) G: [tile][q][row] x 4 neurons
+  float* const gl = reinterpret_cast<float*>(lds + L.gates);
+  float* const prev = reinterpret_cast<float*>(lds + L.rows);         // r_prev of a round's step, two buffers, likewise
+  float* const ga = reinterpret_cast<float*>(lds + L.ga);             // dL/dA shares [2][channel][tile][row]
+  const int T = p.T, rows = p.B - 16 * team;
+  const int steps = (p.grad_r_init || GA) ? T : T - 1;
+
+  if (w < ROWS_TILES) {
+    const int q = lane >> 4, b = lane & 15;
+    unsigned at[ROWS_CHUNKS];
+    rows_places<true>(c, lane, rows, at);
+    bf16x8 wt[ROWS_MATS][ROWS_CHUNKS];
+    rows_weights<true>(c, 16 * (mem * ROWS_TILES + w) + b, q, wt);
+    lds_barrier();                                        // the first gates (and r_prev) are in LDS
+    if (!team_go(lds, L)) return;
+    float* const dst = share + w * AM::SHARE + q * AM::QS + b * 4;
+    RowsOperand op;
+    int slot = 0;
+    bool dead = c.spin_max < 0;
+    if (dead && lane == 0) *c.host_err = RING_CLUSTER_ERR_WAIT;
+    op.issue(rsrc, at, tile_at);
+    for (int s = 0; s < steps; ++s) {
+      const float* g = gl + (s & 1) * c.k * 16 + b;
+      const float g1 = g[0], g2 = g[16];
+      rows_wait(op, c, rsrc, at, (unsigned)slot * slot_bytes + tile_at, dead, lane);
+      asm volatile("" ::: "memory");                       // (what follows is read behind the wait)
+      f32x4 P0 = *reinterpret_cast<const f32x4*>(keep + (w * 64 + lane) * 4);
+      f32x4 P1 = {0.f, 0.f, 0.f, 0.f}, P2 = P1;
+#pragma unroll
+      for (int i = 0; i < ROWS_CHUNKS; ++i) {
+        const bf16x8 x = __builtin_bit_cast(bf16x8, op.x[i]);
+        P1 = mfma16(wt[1][i], x, P1);
+        P2 = mfma16(wt[2][i], x, P2);
+      }
+#pragma unroll
+      for (int i = 0; i < ROWS_CHUNKS; ++i) P0 = mfma16(wt[0][i], __builtin_bit_cast(bf16x8, op.x[i]), P0);
+      slot = slot + 1 == ROWS_SLOTS ? 0 : slot + 1;
+      op.issue(rsrc, at, (unsigned)slot * slot_bytes + tile_at);      // (the first look at the next one)
+      f32x4 v;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) v[i] = fmaf(g2, P2[i], fmaf(g1, P1[i], P0[i]));
+      *reinterpret_cast<f32x4*>(dst + (s & 1) * (ROWS_TILES * AM::SHARE)) = v;
+      if constexpr (GA) {
+        const f32x4 rp = *reinterpret_cast<const f32x4*>(prev + ((s & 1) * ROWS_TILES * 64 + w * 64 + lane) * 4);
+        float d1 = 0.f, d2 = 0.f;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          d1 = fmaf(P1[i], rp[i], d1);
+          d2 = fmaf(P2[i], rp[i], d2);
+        }
+        d1 = sum_bits45(d1);
+        d2 = sum_bits45(d2);
+        float* const gp = ga + ((s & 1) * 2 * ROWS_TILES + w) * 16 + b;
+        if (lane < 16) {
+          gp[0] = d1;
+          gp[ROWS_TILES * 16] = d2;
+        }
+      }
+      lds_barrier();
+    }
+    return;
+  }
+
+  __builtin_amdgcn_s_setprio(3);
+  TA aux(c, mem, tid - 64 * ROWS_TILES);
+  team_arrive(c, team, aux.at);
+  const RowsRecord rec(aux, rows);
+  const int N = p.N, B = p.B, nbt = p.nbt;
+  const float oma = 1.f - p.alpha;
+  const bool loss = p.loss_coef != nullptr;
+  const unsigned x_off = rec.row_ok ? aux.x_off : NOWHERE;
+  auto put = [&](int slot, unsigned x) { __builtin_amdgcn_raw_buffer_store_b32(x, rsrc, (int)x_off, (int)((unsigned)slot * slot_bytes + tile_at), ST_LOCAL); };
+  const TeamGates tg(c, aux.at);
+  float cs[NPT] = {0.f, 0.f}, sn[NPT] = {0.f, 0.f}, up = 0.f;
+  if (loss) {
+#pragma unroll
+    for (int i = 0; i < NPT; ++i) {
+      const float phi = 6.2831853071795864769f * (float)(aux.j0 + i) / (float)N;
+      cs[i] = cosf(phi);
+      sn[i] = sinf(phi);
+    }
+    up = (p.loss_upstream ? p.loss_upstream[0] : 1.f) * p.loss_inv_rows;
+  }
+  const float* const grads = loss ? p.hist : p.grad_out;
+  const int at_row = 16 * team + (rec.row_ok ? aux.map.b : rows - 1);
+  const char* const coef = loss ? reinterpret_cast<const char*>(p.loss_coef + at_row) : reinterpret_cast<const char*>(c.Wo);
+  const int j = aux.j0, dw = j >> 6, dn = (j & 63) >> 2;
+  const unsigned d_at = (unsigned)((dw * 64 + (aux.map.b >> 2) * 16 + dn) * 16 + (j & 3) * 4 + (aux.map.b & 3));     // fp16 values
+  const int at4 = (aux.map.c * 64 + aux.map.q * 16 + aux.map.b) * 4 + 2 * aux.map.p;        // of the thread's values in keep and prev
+  struct In {                          // of a step: grad_output or history, record, loss coefficients, r_prev, gate
+    float go[NPT];
+    _Float16 d[NPT];
+    f32x3 cf;
+    float rp[GA ? NPT : 1];
+    float g;
+  };
+  auto fetch = [&](int t, In& in) {
+    const int tc = t < 0 ? 0 : t;
+    aux.row_load_raw(grads + (size_t)tc * B * N, N, B, team, in.go);
+    const _Float16* src = p.dfrag + ((size_t)tc * nbt + team) * 4096 + d_at;
+    in.d[0] = src[0];
+    in.d[1] = src[4];
+    in.cf = *reinterpret_cast<const f32x3*>(coef + (loss ? (size_t)tc * B * 16 : 0));      // (without the loss head: unused)
+    in.g = tg.fetch(c, tc, team);
+    if constexpr (GA) aux.row_load_raw(tc == 0 ? p.r_init : p.hist + (size_t)(tc - 1) * B * N, N, B, team, in.rp);
+  };
+  auto put_side = [&](int buf, const In& in) {
+    tg.put(gl + buf * c.k * 16, in.g);
+    if constexpr (GA) {
+      float v[NPT] = {in.rp[0], in.rp[1]};
+      aux.align(N, v);
+#pragma unroll
+      for (int i = 0; i < NPT; ++i) prev[buf * ROWS_TILES * 256 + at4 + i] = rec.row_ok && j + i < N ? (float)(__bf16)v[i] : 0.f;
+    }
+  };
+  const bool ok[NPT] = {rec.row_ok && j < N, rec.row_ok && j + 1 < N};
+  // what is carried into the step -> g's bf16 pair; (1 - alpha) G into LDS, where it is before this returns
+  auto form_g = [&](const In& in, const float (&carry)[NPT]) {
+    float gin[NPT] = {in.go[0], in.go[1]};
+    aux.align(N, gin);
+    const float kc = in.cf[0] * up, ks = in.cf[1] * up, beta = in.cf[2] * up;
+    float gg[NPT];
+#pragma unroll
+    for (int i = 0; i < NPT; ++i) {
+      const float r = gin[i], of_loss = fmaf(kc, cs[i], fmaf(ks, sn[i], r > 0.f ? beta : (r < 0.f ? -beta : 0.f)));
+      const float all = (loss ? of_loss : r) + carry[i];
+      const float G = ok[i] ? all : 0.f, g = (float)in.d[i] * G;
+      keep[at4 + i] = oma * G;
+      gg[i] = ok[i] ? g : 0.f;                    // the record carries alpha
+    }
+    const unsigned x = pack_bf16(gg[0], gg[1]);
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    return x;
+  };
+  // dL/dA of round s: one partial per column tile
+  auto flush = [&](int s) {
+    if constexpr (GA) {
+      const int at = aux.at, tile = at >> 5 & 1, ch = at >> 4 & 1, row = at & 15, t = T - 1 - s;
+      const float v = ga[((s & 1) * 2 * ROWS_TILES + (ch * ROWS_TILES + tile)) * 16 + row];
+      const __amdgpu_buffer_rsrc_t r = team_buffer(c.ga_part + ((size_t)mem * ROWS_TILES * T + t) * 2 * B, ((size_t)T + 1) * 2 * B * 4);
+      __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, v), r,
+                                            (int)(at < 64 && row < rows ? (unsigned)((tile * T * 2 + ch) * B + 16 * team + row) * 4 : NOWHERE), 0, 0);
+    }
+  };
+
+  In inA, inB;
+  fetch(T - 1, inA);
+  fetch(T - 2, inB);
+  put_side(0, inA);
+  unsigned x;
+  {
+    const float zero[NPT] = {0.f, 0.f};
+    x = form_g(inA, zero);
+    put(0, not_empty(x));
+  }
+  unsigned held = 0;
+  rec.pair_store(p.gfrag, T - 1, (T & 1) != 0, nbt, team, lane, x, 0u);
+  held = x;                            // (read at even steps: the odd one's behind them)
+  fetch(T - 3, inA);
+  team_gather(c, lds, L, team, aux.at);
+  lds_barrier();
+  if (steps == 0 || !team_go(lds, L)) return;
+
+  const __amdgpu_buffer_rsrc_t rinit = team_buffer(p.grad_r_init + (size_t)16 * team * N, p.grad_r_init ? (size_t)(rows < 16 ? rows : 16) * N * 4 : 0);
+  int slot = 0, s = 0;
+  auto round = [&](In& in) {
+    put_side((s + 1) & 1, in);                               // the gates (and r_prev) of the next round, which is this set's step's
+    lds_barrier();                                          // the round's products are complete
+    float carry[NPT];
+    aux.template sum_shares<1>(share, s & 1, carry);
+#pragma unroll
+    for (int i = 0; i < NPT; ++i) carry[i] = ok[i] ? carry[i] : 0.f;
+    const int t = T - 2 - s, tt = t < 0 ? 0 : t, next_slot = slot + 1 == ROWS_SLOTS ? 0 : slot + 1;
+    // (no branches: what a round has nothing to store for is dropped, so that a wait for a load counts what is behind it)
+    x = form_g(in, carry);
+    put(next_slot, not_empty(x));                            // (after the last round: nobody looks)
+    fetch(t - 2, in);
+    put(slot == 0 ? ROWS_SLOTS - 1 : slot - 1, EMPTY);
+    rec.pair_store(p.gfrag, tt, t >= 0 && (t & 1) == 0, nbt, team, lane, x, t + 1 < T ? held : 0u);
+    held = x;
+    __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, carry[0]), rinit, (int)(t < 0 ? aux.row_off : NOWHERE), 0, 0);
+    __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, carry[1]), rinit, (int)(t < 0 && j + 1 < N ? aux.row_off + 4 : NOWHERE), 0, 0);
+    flush(s);
+    slot = next_slot;
+    ++s;
+  };
+  while (s < steps) {
+    round(inB);
+    if (s >= steps) return;
+    round(inA);
+  }
+}
+
+// Sum of the column tiles' dL/dA partials: the sixteen lanes of a row group, the four waves.
+__global__ __launch_bounds__(256) void ring_team_res256_ga_reduce_kernel(const float* __restrict__ part, float* __restrict__ grad_A, int T, int B) {
+  const size_t n = (size_t)T * 2 * B, u = (size_t)blockIdx.x * 256 + threadIdx.x;
+  if (u >= n) return;
+  float v[4];
+#pragma unroll
+  for (int w = 0; w < 4; ++w) {
+    const float* src = part + (size_t)4 * w * n + u;
+    v[w] = (src[0] + src[n]) + (src[2 * n] + src[3 * n]);
+  }
+  const int b = (int)(u % B);
+  const size_t tc = u / B;
+  grad_A[((size_t)b * T + (tc >> 1)) * 2 + (tc & 1)] = ((v[0] + v[1]) + v[2]) + v[3];
+}
+
+// record: with one, or a BPTT; then all 256 neurons have a member (the padding's part of the record is zero)
+RingTeamPlan ring_team_rows_plan(int N, int k, int B, bool record) {
   RingTeamPlan p{};
   if (!ring_res256_applicable(N, k)) return p;
-  p.KC = (N + 31) / 32;
+  p.KC = record ? ROWS_CHUNKS : (N + 31) / 32;
   p.G = (2 * p.KC + ROWS_TILES - 1) / ROWS_TILES;
   p.nteams = (B + 15) / 16;
   p.nt = 1;
@@ -180,6 +478,8 @@ RingTeamPlan ring_team_rows_plan(int N, int k, int B) {
   return p;
 }
 
+size_t ring_team_rows_ga_bytes(int T, int B) { return (size_t)16 * T * 2 * B * sizeof(float); }
+
 hipError_t ring_launch_team_rows(const RingFwdArgs& a, const RingTeamArgs& c, const RingTeamShape& sh, hipStream_t st) {
   const unsigned lds = lds_plan<ROWS_TILES, 1>(c.k, 1, 0, c.KC, 0, false, false).total;
   auto go = [&](auto kern) {
@@ -187,10 +487,25 @@ hipError_t ring_launch_team_rows(const RingFwdArgs& a, const RingTeamArgs& c, co
                            [&](dim3 g, dim3 b, unsigned bytes) { RING_LAUNCH(kern, g, b, bytes, st, a, c); });
   };
   switch (a.act) {
-    case ACT_RELU: return go(ring_team_rows_kernel<ACT_RELU>);
-    case ACT_GELU: return go(ring_team_rows_kernel<ACT_GELU>);
-    case ACT_TANH: return go(ring_team_rows_kernel<ACT_TANH>);
-    case ACT_SILU: return go(ring_team_rows_kernel<ACT_SILU>);
+    case ACT_RELU: return a.dfrag ? go(ring_team_res256_fwd_kernel<ACT_RELU>) : go(ring_team_rows_kernel<ACT_RELU>);
+    case ACT_GELU: return a.dfrag ? go(ring_team_res256_fwd_kernel<ACT_GELU>) : go(ring_team_rows_kernel<ACT_GELU>);
+    case ACT_TANH: return a.dfrag ? go(ring_team_res256_fwd_kernel<ACT_TANH>) : go(ring_team_rows_kernel<ACT_TANH>);
+    case ACT_SILU: return a.dfrag ? go(ring_team_res256_fwd_kernel<ACT_SILU>) : go(ring_team_rows_kernel<ACT_SILU>);
     default: return hipErrorInvalidValue;
   }
+}
+
+hipError_t ring_launch_team_rows_bptt(const RingBpttArgs& a, const RingTeamArgs& c, const RingTeamShape& sh, hipStream_t st) {
+  const unsigned lds = lds_plan<ROWS_TILES, 1>(c.k, 1, 0, c.KC, 0, true, a.grad_A != nullptr).total + (a.grad_A ? ROWS_GA_MORE : 0);
+  auto go = [&](auto kern) {
+    return ring_team_start(reinterpret_cast<const void*>(kern), sh, c.G, lds, st,
+                           [&](dim3 g, dim3 b, unsigned bytes) { RING_LAUNCH(kern, g, b, bytes, st, a, c); });
+  };
+  return a.grad_A ? go(ring_team_res256_bptt_kernel<true>) : go(ring_team_res256_bptt_kernel<false>);
+}
+
+hipError_t ring_launch_team_rows_ga(const float* part, float* grad_A, int T, int B, hipStream_t st) {
+  const size_t n = (size_t)T * 2 * B;
+  hipLaunchKernelGGL(ring_team_res256_ga_reduce_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, part, grad_A, T, B);
+  return hipGetLastError();
 }

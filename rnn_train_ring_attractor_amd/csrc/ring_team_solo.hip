@@ -184,9 +184,9 @@ __global__ __launch_bounds__(512) void ring_team_rebuild_kernel(RingFwdArgs p, R
         f16x4 d;
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-          float aF, aD;
-          act_scaled<ACT>(tot[cc][r][i], asc, aF, aD);
-          d[i] = record_value(aD);
+          ActRecord<ACT> rd;
+          rd.apply(tot[cc][r][i], asc);
+          d[i] = rd.once(asc);
         }
         *reinterpret_cast<f16x4*>(p.dfrag + ((((size_t)t0 + (r & 1)) * p.nbt + tile(r)) * c.cts + 2 * pair + cc) * 256 + (q * 16 + b) * 4) = d;
       }
@@ -253,7 +253,7 @@ __host__ __device__ inline SoloLds solo_lds(int KC, int k, bool ga, bool trig) {
   l.gates = at;
   at += (unsigned)k * 64;
   l.ga = at;
-  at += ga ? SOLO_WAVES * (unsigned)k * 64 : 0;
+  at += ga ? SOLO_WAVES * (unsigned)k * 64 * 2 : 0;       // (weight-resident order: two column tiles' shares)
   l.trig = at;
   at += trig ? (unsigned)KC * 256 : 0;           // (cos, sin) of every neuron's angle
   l.total = at;
@@ -280,16 +280,19 @@ __device__ __forceinline__ bf16x8 solo_weight(const RingTeamArgs& c, int m, int 
 
 // What member `mem` of the team adds up for its column tiles: tot[cc], lane (q, row) with neurons 4q .. 4q + 3 of tile
 // mem * c16 + cc.  GA: also the member's dL/dA shares, from r_prev in rp, into ga[k][16].
+// Weight-resident order (c.rows): the ungated sum starts from `start` (the BPTT's (1 - alpha) G), and a share of dL/dA is a
+// column tile's: ga[cc][k][16].
 template <bool TR, bool GA>
 __device__ __forceinline__ void solo_products(const RingTeamArgs& c, const SoloOperand& o, const float* gates,
-                                              const f32x4 (&rp)[SOLO_C16], float* ga, int mem, int lane, f32x4 (&tot)[SOLO_C16]) {
+                                              const f32x4 (&rp)[SOLO_C16], const f32x4* start, float* ga, int mem, int lane,
+                                              f32x4 (&tot)[SOLO_C16]) {
   const int b = lane & 15;
   for (int cw = 0; cw < c.wk && cw < c.KC; ++cw) {
     f32x4 acc[SOLO_C16];
     float sum = 0.f;
     auto chunks = [&](auto&& use) {              // the wave's K chunks in its order
       for (int i = 0; i < (c.rows ? 8 : c.KC); i += c.wk) {
-        const int kc = c.rows ? rows_chunk(i) : cw + i;
+        const int kc = c.rows && !TR ? rows_chunk(i) : cw + i;
         if (kc < c.KC) use(kc);
       }
     };
@@ -303,14 +306,20 @@ __device__ __forceinline__ void solo_products(const RingTeamArgs& c, const SoloO
       for (int cc = 0; cc < SOLO_C16; ++cc) {
         if (cc >= c.c16) continue;
         f32x4 P = {0.f, 0.f, 0.f, 0.f};
+        if (TR && c.rows && m == 0 && mem * c.c16 + cc < 2 * c.KC) P = start[(mem * c.c16 + cc) * 64];
         chunks([&](int kc) { P = mfma16(solo_weight<TR>(c, m, mem * c.c16 + cc, kc, lane), o.x[kc * 64 + lane], P); });
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
           acc[cc][i] = m == 0 ? fmaf(c.J1, P[i], j0r) : fmaf(g, P[i], acc[cc][i]);
           if (GA) d = fmaf(P[i], rp[cc][i], d);
         }
+        if (GA && m > 0 && c.rows) {
+          d = sum_bits45(d);
+          if (lane < 16) ga[(cc * c.k + m - 1) * 16 + b] = d;
+          d = 0.f;
+        }
       }
-      if (GA && m > 0) {
+      if (GA && m > 0 && !c.rows) {
         d = sum_bits45(d);
         if (lane < 16) ga[(m - 1) * 16 + b] = (cw == 0 ? 0.f : ga[(m - 1) * 16 + b]) + d;
       }
@@ -344,7 +353,8 @@ __device__ __forceinline__ void solo_put4(const SoloOperand& o, int ct, int lane
 }
 
 // A pair of steps of the copy for the weight gradients (hi null: zeros).
-__device__ __forceinline__ void solo_pair(__bf16* base, int t, int nbt, int bt, int cts, int KC, int tid, const bf16x8* lo, const bf16x8* hi) {
+// (split: in the weight-resident kernels' tile order, neuron j in column j % 64 / 4 of tile 4 (j / 64) + j % 4)
+__device__ __forceinline__ void solo_pair(__bf16* base, int t, int nbt, int bt, int cts, int KC, int tid, const bf16x8* lo, const bf16x8* hi, bool split) {
   for (int u = tid; u < 2 * KC * 64; u += 64 * SOLO_WAVES) {
     const int ct = u >> 6, rq = u >> 4 & 3, j = 16 * ct + (u & 15);
     const size_t at = ((size_t)(j >> 5) * 64 + ((j >> 3) & 3) * 16 + 4 * rq) * 8 + (j & 7);
@@ -354,8 +364,17 @@ __device__ __forceinline__ void solo_pair(__bf16* base, int t, int nbt, int bt, 
       o[i] = reinterpret_cast<const __bf16*>(lo)[at + i * 8];
       o[4 + i] = hi ? reinterpret_cast<const __bf16*>(hi)[at + i * 8] : (__bf16)0.f;
     }
-    *reinterpret_cast<bf16x8*>(base + ((((size_t)(t >> 1) * nbt + bt) * cts + ct) * 64 + (u & 63)) * 8) = o;
+    const int slot = split ? (4 * (j >> 6) + (j & 3)) * 64 + rq * 16 + ((j & 63) >> 2) : ct * 64 + (u & 63);
+    *reinterpret_cast<bf16x8*>(base + (((size_t)(t >> 1) * nbt + bt) * cts * 64 + slot) * 8) = o;
   }
+}
+
+// The lane's four values of the derivative record (neurons 16 ct + 4q .., row lane & 15), in either order.
+__device__ __forceinline__ size_t solo_dact_at(const RingTeamArgs& c, int t, int nbt, int bt, int ct, int lane, int i) {
+  const size_t tile = ((size_t)t * nbt + bt) * c.cts * 256;
+  if (!c.rows) return tile + ct * 256 + lane * 4 + i;
+  const int j = 16 * ct + 4 * (lane >> 4) + i, b = lane & 15;
+  return tile + ((j >> 6) * 64 + (b >> 2) * 16 + ((j & 63) >> 2)) * 16 + (j & 3) * 4 + (b & 3);
 }
 
 __device__ __forceinline__ void solo_gates(const RingTeamArgs& c, float* gates, int t, int bt, int tid) {
@@ -395,7 +414,7 @@ __global__ __launch_bounds__(64 * SOLO_WAVES) void ring_team_solo_fwd_kernel(Rin
     for (int mem = w; mem < c.G; mem += SOLO_WAVES) {
       f32x4 x[SOLO_C16];
       const f32x4 none[SOLO_C16] = {};
-      solo_products<false, false>(c, cur, gates, none, nullptr, mem, lane, x);
+      solo_products<false, false>(c, cur, gates, none, nullptr, nullptr, mem, lane, x);
 #pragma unroll
       for (int cc = 0; cc < SOLO_C16; ++cc) {
         const int ct = mem * c.c16 + cc, j = 16 * ct + 4 * q;
@@ -404,20 +423,34 @@ __global__ __launch_bounds__(64 * SOLO_WAVES) void ring_team_solo_fwd_kernel(Rin
         f32x4 rn;
         f16x4 d;
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          float aF, aD;
-          act_scaled<ACT>(x[cc][i], asc, aF, aD);
-          rn[i] = j + i < N ? fmaf(oma, r[i], aF) : 0.f;
-          d[i] = record_value(aD);
+        for (int i = 0; i < 4; i += 2) {
+          float aF[2];
+          const float x2[2] = {x[cc][i], x[cc][i + 1]};
+          ActRecord<ACT> rd[2];
+#pragma unroll
+          for (int h = 0; h < 2; ++h) aF[h] = rd[h].apply(x2[h], asc);
+          const f16x2 both = __builtin_bit_cast(f16x2, ActRecord<ACT>::pair(asc, rd[0], rd[1], !c.rows || (c.rows == 2 && (j & 32) && t + 1 < T)));
+#pragma unroll
+          for (int h = 0; h < 2; ++h) {
+            rn[i + h] = j + i + h < N ? fmaf(oma, r[i + h], aF[h]) : 0.f;
+            d[i + h] = !c.rows || (b < B && j + i + h < N) ? both[h] : (_Float16)0.f;
+          }
         }
         state[ct * 64] = rn;
         solo_put4(next, ct, lane, rn);
         solo_row4_store(p.hist + (size_t)t * B * N, N, B, b, j, rn);
-        if (p.dfrag) *reinterpret_cast<f16x4*>(p.dfrag + (((size_t)t * p.nbt + bt) * c.cts + ct) * 256 + lane * 4) = d;
+        if (p.dfrag) {
+          if (c.rows) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) p.dfrag[solo_dact_at(c, t, p.nbt, bt, ct, lane, i)] = d[i];
+          } else {
+            *reinterpret_cast<f16x4*>(p.dfrag + solo_dact_at(c, t, p.nbt, bt, ct, lane, 0)) = d;
+          }
+        }
       }
     }
     lds_barrier();
-    if (p.rfrag && (t & 1) == 0) solo_pair(p.rfrag, t, p.nbt, bt, c.cts, KC, tid, cur.x, t + 1 < T ? next.x : nullptr);
+    if (p.rfrag && (t & 1) == 0) solo_pair(p.rfrag, t, p.nbt, bt, c.cts, KC, tid, cur.x, t + 1 < T ? next.x : nullptr, c.rows != 0);
   }
 }
 
@@ -435,7 +468,7 @@ __global__ __launch_bounds__(64 * SOLO_WAVES) void ring_team_solo_bptt_kernel(Ri
   };
   f32x4* const state = reinterpret_cast<f32x4*>(lds + L.state) + lane;
   float* const gates = reinterpret_cast<float*>(lds + L.gates);
-  float* const ga = reinterpret_cast<float*>(lds + L.ga) + (size_t)w * k * 16;
+  float* const ga = reinterpret_cast<float*>(lds + L.ga) + (size_t)w * k * 32;
   f32x2* const trig = reinterpret_cast<f32x2*>(lds + L.trig);
   const float oma = 1.f - p.alpha;
   float up = 0.f;
@@ -452,7 +485,13 @@ __global__ __launch_bounds__(64 * SOLO_WAVES) void ring_team_solo_bptt_kernel(Ri
   auto form_g = [&](int t, int ct, const f32x4& carry, const SoloOperand& o) {
     const int j = 16 * ct + 4 * q;
     const f32x4 in = solo_row4((loss ? p.hist : p.grad_out) + (size_t)t * B * N, N, B, b, j);
-    const f16x4 d = *reinterpret_cast<const f16x4*>(p.dfrag + (((size_t)t * p.nbt + bt) * c.cts + ct) * 256 + lane * 4);
+    f16x4 d;
+    if (c.rows) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) d[i] = p.dfrag[solo_dact_at(c, t, p.nbt, bt, ct, lane, i)];
+    } else {
+      d = *reinterpret_cast<const f16x4*>(p.dfrag + solo_dact_at(c, t, p.nbt, bt, ct, lane, 0));
+    }
     float kc = 0.f, ks = 0.f, beta = 0.f;
     if (loss && b < B) {
       const ring_f32x4 cf = p.loss_coef[(size_t)t * B + b];
@@ -480,7 +519,7 @@ __global__ __launch_bounds__(64 * SOLO_WAVES) void ring_team_solo_bptt_kernel(Ri
 
   for (int ct = w; ct < 2 * KC; ct += SOLO_WAVES) form_g(T - 1, ct, f32x4{0.f, 0.f, 0.f, 0.f}, operand(0));
   lds_barrier();
-  if (((T - 1) & 1) == 0) solo_pair(p.gfrag, T - 1, p.nbt, bt, c.cts, KC, tid, operand(0).x, nullptr);
+  if (((T - 1) & 1) == 0) solo_pair(p.gfrag, T - 1, p.nbt, bt, c.cts, KC, tid, operand(0).x, nullptr, c.rows != 0);
   const int steps = (p.grad_r_init || GA) ? T : T - 1;
   for (int s = 0; s < steps; ++s) {
     const SoloOperand cur = operand(s & 1), next = operand((s + 1) & 1);
@@ -492,24 +531,31 @@ __global__ __launch_bounds__(64 * SOLO_WAVES) void ring_team_solo_bptt_kernel(Ri
       if constexpr (GA) {
 #pragma unroll
         for (int cc = 0; cc < SOLO_C16; ++cc)
-          if (cc < c.c16) rp[cc] = solo_row4(t == 0 ? p.r_init : p.hist + (size_t)(t - 1) * B * N, N, B, b, 16 * (mem * c.c16 + cc) + 4 * q);
+          if (cc < c.c16) {
+            rp[cc] = solo_row4(t == 0 ? p.r_init : p.hist + (size_t)(t - 1) * B * N, N, B, b, 16 * (mem * c.c16 + cc) + 4 * q);
+            if (c.rows) {
+#pragma unroll
+              for (int i = 0; i < 4; ++i) rp[cc][i] = (float)(__bf16)rp[cc][i];
+            }
+          }
       }
-      solo_products<true, GA>(c, cur, gates, rp, ga, mem, lane, x);
+      solo_products<true, GA>(c, cur, gates, rp, state, ga, mem, lane, x);
       if constexpr (GA) {
+        const int parts = c.rows ? c.c16 : 1;
         if (lane < 16 && b < B)
-          for (int ch = 0; ch < k; ++ch) c.ga_part[(((size_t)mem * T + t) * k + ch) * B + b] = ga[ch * 16 + lane];
+          for (int u = 0; u < parts * k; ++u) c.ga_part[(((size_t)(mem * parts + u / k) * T + t) * k + u % k) * B + b] = ga[u * 16 + lane];
       }
 #pragma unroll
       for (int cc = 0; cc < SOLO_C16; ++cc) {
         const int ct = mem * c.c16 + cc;
         if (cc >= c.c16 || ct >= 2 * KC) continue;
-        const f32x4 carry = state[ct * 64] + x[cc];
+        const f32x4 carry = c.rows ? x[cc] : state[ct * 64] + x[cc];
         if (t > 0) form_g(t - 1, ct, carry, next);
         else if (p.grad_r_init) solo_row4_store(p.grad_r_init, N, B, b, 16 * ct + 4 * q, carry);
       }
     }
     lds_barrier();
-    if (t > 0 && ((t - 1) & 1) == 0) solo_pair(p.gfrag, t - 1, p.nbt, bt, c.cts, KC, tid, next.x, cur.x);
+    if (t > 0 && ((t - 1) & 1) == 0) solo_pair(p.gfrag, t - 1, p.nbt, bt, c.cts, KC, tid, next.x, cur.x, c.rows != 0);
   }
 }
 

@@ -179,7 +179,7 @@ size_t ringattr_fwd_workspace_bytes(int N, int a_dim, int seq_len, int batch_siz
   const size_t packed = g.wpack_bytes + (ring_cluster_applicable(N, a_dim) ? ring_cluster_workspace_bytes(g.nbt) : 0) +
                         (ring_panel_applicable(g.NC, a_dim) ? align_up(ring_panel_workspace_bytes(g.NC, g.nbt)) : 0);
   // (used instead of the packed weights)
-  const size_t team = ring_team_fwd_bytes(N, a_dim, seq_len, batch_size), rows = ring_team_rows_bytes(N, a_dim, batch_size);
+  const size_t team = ring_team_fwd_bytes(N, a_dim, seq_len, batch_size), rows = ring_team_rows_bytes(N, a_dim, batch_size, true);
   const size_t most = team > rows ? team : rows;
   return packed > most ? packed : most;
 }
@@ -309,9 +309,13 @@ static int fwd_impl(const void* A, const void* Wa, float J0, float J1, const voi
     return RINGATTR_OK;
   }
 
-  // (the loss head's row sums come from the weight-resident forward, whatever the batch)
-  if (!saved && !loss_stats && ring_uses_team_rows(N, a_dim, batch_size) && workspace_bytes >= ring_team_rows_bytes(N, a_dim, batch_size)) {
-    const RingFwdArgs a = fwd_args(A, nullptr, r_init, bump_history, nullptr, g, J0, J1, alpha, activation_type);
+  if (ring_uses_team_rows(N, a_dim, batch_size, saved != nullptr) &&
+      workspace_bytes >= ring_team_rows_bytes(N, a_dim, batch_size, saved != nullptr)) {
+    RingFwdArgs a = fwd_args(A, nullptr, r_init, bump_history, saved, g, J0, J1, alpha, activation_type);
+    a.loss_stats = loss_stats;
+    // (the weight-resident kernels' record, but no transposed weights behind it: the note names none)
+    if (saved) saved_note_put(SavedNote{saved, 2, N, a_dim, seq_len, batch_size, J0, J1, nullptr, nullptr});
+    if (stats_done) *stats_done = loss_stats != nullptr;
     const hipError_t e = ring_run_team_rows(a, (const float*)Wo, (const float*)Wa, workspace, st);
     if (e != hipSuccess) return hip_fail(e, "team forward launch");
     return RINGATTR_OK;
@@ -506,7 +510,10 @@ static int bwd_impl(const char* who, const void* grad_output, const void* loss_w
   if (!team && noted != 0 && (noted == 3) != (family == 3))
     return fail(RINGATTR_ERR_INVALID, "%s: the saved buffer was filled by the other kernel family (its derivative record "
                 "has a different layout); run forward and backward under the same RINGATTR_BLOCK setting", who);
-  if (team) {
+  // small batches of the weight-resident widths: on teams, with their scratch in the split-K partials' place
+  const bool rows = family == 2 && ring_uses_team_rows(N, a_dim, batch_size, true) &&
+                    ring_team_rows_bptt_bytes(N, a_dim, seq_len, batch_size, grad_A != nullptr) <= g.partial_bytes;
+  if (team || rows) {
     // (the team kernels read the fp32 weights)
   } else if (bptt_cluster) {
     e = ring_launch_pack((const float*)Wo, (const float*)Wa, wb, N, a_dim, g.NC, 1,
@@ -551,8 +558,9 @@ static int bwd_impl(const char* who, const void* grad_output, const void* loss_w
   b.B = batch_size;
   b.nbt = g.nbt;
   b.cluster_ws = cluster_ws;
-  e = team ? ring_run_team_bptt(b, (const float*)Wo, (const float*)Wa, ring_res256_applicable(N, a_dim), 4 * g.NC, team_ws, st)
-           : ring_launch_bptt(b, g.NC, st);
+  if (team) e = ring_run_team_bptt(b, (const float*)Wo, (const float*)Wa, ring_res256_applicable(N, a_dim), 4 * g.NC, team_ws, st);
+  else if (rows) e = ring_run_team_rows_bptt(b, (const float*)Wo, (const float*)Wa, partial, st);
+  else e = ring_launch_bptt(b, g.NC, st);
   if (e != hipSuccess) return hip_fail(e, "BPTT launch");
   if (step_family && grad_A) {
     // forward-orientation fragments, packed into the split-K partial area (not yet in use, and never smaller)

@@ -420,3 +420,87 @@ def test_a_wait_that_runs_out_is_reported_once_and_the_other_kernels_take_over(g
                           cwd=ROOT)
     print(proc.stdout[-1500:], proc.stderr[-1500:], flush=True)
     assert proc.returncode == 0 and "give-up path ok" in proc.stdout
+
+
+# one row to all 32 teams, ragged tiles and widths (padding within a chunk, whole chunks of it), single steps, odd and even lengths
+@pytest.mark.parametrize("N,B,T,act", [(256, 1, 7, "gelu"), (256, 128, 100, "gelu"), (256, 512, 12, "tanh"), (256, 40, 2, "silu"), (129, 16, 1, "silu"),
+                                       (131, 9, 3, "gelu"), (200, 257, 33, "gelu"), (250, 300, 6, "tanh"), (222, 64, 17, "relu")])
+def test_small_batches_train_with_the_weight_resident_kernels_bits(N, B, T, act, gpu_device, teams, monkeypatch):
+    """Forward with a record and BPTT over teams against the weight-resident kernels, every output; either family's record
+    through the other one's BPTT; and the single workgroups behind teams that do not gather."""
+    from rnn_train_ring_attractor_amd import rnn_cuda, _lib
+    monkeypatch.delenv("RINGATTR_TEAM", raising=False)
+    print(f"[case] team rows, training N={N} B={B} T={T} {act}", flush=True)
+    p = make_problem(87, B, T, 2, N, action="dense")
+    A, Wa, Wo, r0, G = (_t(p[x], gpu_device) for x in ("A", "Wa", "Wo", "r0", "G"))
+    common = dict(A=A, Wa=Wa, J0=-0.05, J1=0.7, Wo=Wo, r_init=r0, alpha=0.15, activation_type=ACTS[act])
+
+    def fwd(kernel, **env):
+        for k, v in env.items():
+            monkeypatch.setenv(k, v)
+        hist = torch.full((T, B, N), float("nan"), device=gpu_device)
+        saved = torch.empty(rnn_cuda.saved_nbytes(N, 2, T, B), dtype=torch.uint8, device=gpu_device).fill_(0xFF)
+        rnn_cuda.fwd_cuda.fwd(bump_history=hist, saved=saved, **common)
+        torch.cuda.synchronize()
+        for k in env:
+            monkeypatch.delenv(k)
+        assert kernel in _lib.last_kernel_names()["fwd"]
+        return hist, saved
+
+    def bwd(kernel, hist, saved, ga, **env):
+        for k, v in env.items():
+            monkeypatch.setenv(k, v)
+        out = {n: torch.full_like(x, float("nan")) for n, x in (("grad_Wa", Wa), ("grad_Wo", Wo), ("grad_r_init", r0))}
+        if ga:
+            out["grad_A"] = torch.full_like(A, float("nan"))
+        rnn_cuda.bwd_cuda.bwd(grad_output=G, bump_history=hist, saved=saved, accumulate=False, **common, **out)
+        torch.cuda.synchronize()
+        for k in env:
+            monkeypatch.delenv(k)
+        assert kernel in _lib.last_kernel_names()["bptt"]
+        return out
+
+    resident, team = dict(RINGATTR_TEAM="0"), {}
+    hist, record = fwd("ring_fwd_res256", **resident)
+    assert torch.isfinite(hist).all()
+    for ga in (True, False):
+        want = bwd("ring_bptt_res256", hist, record, ga, **resident)
+        for wait_us in (None, "-1", "0"):
+            env = {} if wait_us is None else {"RINGATTR_TEAM_GATHER_US": wait_us}
+            h, s = fwd("ring_team_res256_fwd", **env)
+            assert torch.equal(h, hist), wait_us
+            for got in (bwd("ring_team_res256_bptt", h, s, ga, **env), bwd("ring_bptt_res256", h, s, ga, **resident),
+                        bwd("ring_team_res256_bptt", hist, record, ga, **env)):
+                bad = {x: float((got[x] - want[x]).abs().max() / want[x].abs().max()) for x in want if not torch.equal(got[x], want[x])}
+                assert not bad, (wait_us, ga, bad)
+
+
+# whole and ragged tiles, single steps: the row sums' order and the late columns' record
+@pytest.mark.parametrize("N,B,T,act", [(256, 128, 100, "gelu"), (256, 48, 9, "tanh"), (256, 16, 1, "gelu"), (256, 40, 5, "gelu"), (256, 64, 6, "relu"),
+                                       (200, 100, 6, "tanh"), (131, 32, 4, "silu")])
+def test_fused_loss_head_on_small_batches_of_the_weight_resident_widths(N, B, T, act, gpu_device, teams, monkeypatch):
+    """The loss and every gradient, bit for bit."""
+    from rnn_train_ring_attractor_amd import ring_rnn_loss_func, _lib
+    print(f"[case] team rows, loss N={N} B={B} T={T} {act}", flush=True)
+    p = make_problem(77, B, T, 2, N, action="dense")
+    r0 = _t(p["r0"], gpu_device)
+    angle = torch.rand(B, T, device=gpu_device) * 6.28
+
+    def run(**env):
+        monkeypatch.delenv("RINGATTR_TEAM", raising=False)
+        for k, v in env.items():
+            monkeypatch.setenv(k, v)
+        leaves = [_t(p[x], gpu_device).requires_grad_(True) for x in ("A", "Wa", "Wo")]
+        out = ring_rnn_loss_func(leaves[0], leaves[1], -1.0 / N, 0.6, leaves[2], r0, 0.15, act, angle, 0.2)
+        out[0].backward()
+        torch.cuda.synchronize()
+        for k in env:
+            monkeypatch.delenv(k)
+        return [x.detach() for x in out] + [x.grad for x in leaves]
+
+    want = run(RINGATTR_TEAM="0")
+    assert "ring_bptt_res256" in _lib.last_kernel_names()["bptt"]
+    for env in ({}, {"RINGATTR_TEAM_GATHER_US": "-1"}):
+        got = run(**env)
+        assert "ring_team_res256_bptt" in _lib.last_kernel_names()["bptt"]
+        assert [torch.equal(x, y) for x, y in zip(got, want)] == [True] * len(want), env
