@@ -160,12 +160,10 @@ __global__ __launch_bounds__(512) void ring_fwd_res256_kernel(RingFwdArgs p) {
   load_resident8(reinterpret_cast<const bf16x8*>(p.Wpack), wl, wreg, w, h, lane);
 
   float r[4][2], okf[4][2];
-  // alpha F', or what it is made of (late role of whole tiles), until it is stored.  With the row sums the registers are not
-  // there: the finished fp16 pairs of rows 0, 1 and 2, 3.
+  // alpha F', or what it is made of (late role of whole tiles), until it is stored
   using Record = ActRecord<ACT>;
   float d[4][2];
   Record late[4][2];
-  unsigned dp[2][2];
 #pragma unroll
   for (int e = 0; e < 4; ++e)
 #pragma unroll
@@ -282,8 +280,7 @@ __global__ __launch_bounds__(512) void ring_fwd_res256_kernel(RingFwdArgs p) {
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
           const int e = 2 * (i & 1), cc = i >> 1;
-          if constexpr (STATS) pk[i] = dp[cc][e / 2];
-          else if constexpr (decltype(once)::value) pk[i] = Record::pair_once(asc, late[e][cc], late[e + 1][cc]);
+          if constexpr (decltype(once)::value) pk[i] = Record::pair_once(asc, late[e][cc], late[e + 1][cc]);
           else pk[i] = record_pair(d[e][cc], d[e + 1][cc]);
         }
         *reinterpret_cast<u32x4*>(base + d_lane) = pk;
@@ -369,12 +366,6 @@ __global__ __launch_bounds__(512) void ring_fwd_res256_kernel(RingFwdArgs p) {
           d[e][cc] *= okf[e][cc];                  // (never `once`)
         }
         r[e][cc] = rn;
-        if constexpr (SAVE && STATS) {
-          if (e & 1) {
-            if constexpr (decltype(once)::value) dp[cc][e / 2] = Record::pair_once(asc, late[e - 1][cc], late[e][cc]);
-            else dp[cc][e / 2] = record_pair(d[e - 1][cc], d[e][cc]);
-          }
-        }
       }
   };
   constexpr std::bool_constant<SAVE && FULL && Record::FUSED> late_once{};
