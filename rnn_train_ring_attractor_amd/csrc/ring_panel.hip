@@ -12,12 +12,16 @@
 //   * Per K chunk a workgroup with R row tiles and V virtual columns loads (R + V) KiB for R * V MFMAs: 8 + 17 KiB
 //     against 544 matrix-pipe cycles at B = 256 and 16 channels.  What is left is the rate at which a compute unit takes
 //     in lines that miss its L2; see panel_shape.
-//   * The operand arrives as bf16 MFMA fragments: a small launch before each step converts the state and takes its
-//     row sums (in ring_block.hip's order), 5 us at B = 256.
-// us per step, before (ring_block.hip / ring_bign.hip) -> here, T = 20 with the packing launch:
-//   N = 2048, 16 channels: B = 1: 120 -> 39   B = 256: 102 -> 64 (the step kernel itself 97 -> 57)   B = 1024: 286 -> 189
-//   N = 2048,  2 channels: B = 16: 31 -> 13   B = 256:  35 -> 22                                     B = 1024:  73 -> 47
-//   N = 1100,  2 channels: B = 16: 22 -> 12   B = 200:  29 -> 18     N = 1500, 6 channels, B = 64: 49 -> 16
+//   * The operand arrives as bf16 MFMA fragments: one launch converts the initial state, every step's epilogue the state it
+//     makes.  A row's sum (in ring_block.hip's order) would be a launch between the steps: the epilogue leaves the sums of
+//     four neurons, at the next step each workgroup adds up and announces a row or two, and behind the products takes the
+//     announced sums of all of its rows.  Nobody waits for one: what is not there yet is added up once more.  us per step with
+//     a launch for operand and sums before each step -> here: N = 2048, 16 channels, B = 256: 57.9 -> 55.8; B = 1: 34.1 -> 29.7;
+//     2 channels, B = 1: 11.4 -> 7.5; N = 2047, B = 16: 14.6 -> 8.9; N = 1500, 6 channels, B = 64: 15.0 -> 12.1.
+// us per step, ring_block.hip / ring_bign.hip -> here, T = 20 with the packing launch:
+//   N = 2048, 16 channels: B = 1: 120 -> 35   B = 256: 102 -> 63   B = 1024: 286 -> 181
+//   N = 2048,  2 channels: B = 16: 31 -> 9    B = 256:  35 -> 19   B = 1024:  73 -> 44
+//   N = 1100,  2 channels: B = 16: 22 -> 8.5  B = 200:  29 -> 17   N = 1500, 6 channels, B = 64: 49 -> 13
 // Products, gates and activation are the arithmetic of ring_block.hip in the same order (a product's contraction is
 // never split), so the two families agree bit for bit: tests/test_gpu_panel.py.
 #include "ring_step_common.hpp"
@@ -137,21 +141,59 @@ __device__ __forceinline__ void panel_pass(const PanelPass& p, const unsigned (&
   }
 }
 
+// The sum of a row of a [B][N] state from its fours [N / 4], by 16 lanes: ring_block.hip's order, and ring_panel_operand_kernel's.
+template <int EACH>                                       // loads in flight
+struct PanelRowSum {
+  float v[EACH];
+  __device__ __forceinline__ void load(const float* fours, int N, int at) {       // (past the end: a re-read, not summed)
+    const int last = (N - 1) >> 2;
+#pragma unroll
+    for (int i = 0; i < EACH; ++i) v[i] = fours[at + 16 * i < last ? at + 16 * i : last];
+  }
+  __device__ __forceinline__ void add(float& s, int N, int at) const {
+    const int last = (N - 1) >> 2;
+#pragma unroll
+    for (int i = 0; i < EACH; ++i) s += at + 16 * i <= last ? v[i] : 0.f;
+  }
+};
+__device__ __forceinline__ float panel_row_sum(const float* fours, int N, int sub) {
+  float s = 0.f;
+  for (int at = sub; 4 * at < N; at += 16 * 16) {
+    PanelRowSum<16> some;
+    some.load(fours, N, at);
+    some.add(s, N, at);
+  }
+  return row16_sum_dpp(s);
+}
+
+// What travels between the steps, two of each but the row sums (three: the step before the last one's is emptied).
+struct PanelState {
+  bf16x8* x[2];         // operand fragments [batch tile][K chunk][lane]
+  float* fours[2];      // [row][NPAD / 4]
+  float* rs[3];         // [row]; PANEL_EMPTY: not announced yet
+};
+constexpr unsigned PANEL_EMPTY = 0xFFFFFFFFu;
+
+// Four neurons of a row as bf16, at their place in the operand fragments.
+__device__ __forceinline__ void panel_put(bf16x8* x, int KCH, int b, int j, const f32x4& v) {
+  char* base = reinterpret_cast<char*>(x + (size_t)(b >> 4) * KCH * 64);
+  const bf16x4 pk = {(__bf16)v[0], (__bf16)v[1], (__bf16)v[2], (__bf16)v[3]};
+  *reinterpret_cast<bf16x4*>(base + (size_t)((j >> 5) * 64 + ((j >> 3) & 3) * 16 + (b & 15)) * 16 + (j & 7) * 2) = pk;
+}
+
 }  // namespace
 
-// Operand fragments [batch tile][K chunk][lane][8] and fp32 row sums of one step's rows; four rows per wave.  The sums
-// run in the order of ring_block.hip's stage_tiles.
-__global__ __launch_bounds__(64) void ring_panel_operand_kernel(const float* __restrict__ prev, bf16x8* __restrict__ xfrag,
-                                                                float* __restrict__ rs, int N, int B, int NPAD) {
+// Operand fragments [batch tile][K chunk][lane][8] and fp32 row sums of the initial state's rows; four rows per wave.  The
+// sums run in the order of ring_block.hip's stage_tiles.  (Both fragment buffers: the steps write no padding.)
+__global__ __launch_bounds__(64) void ring_panel_operand_kernel(const float* __restrict__ prev, PanelState ps, int N, int B, int NPAD) {
   const int lane = threadIdx.x, row = 4 * (blockIdx.x & 3) + (lane >> 4), sub = lane & 15, bt = blockIdx.x >> 2;
-  char* base = reinterpret_cast<char*>(xfrag + (size_t)bt * (NPAD >> 5) * 64);
+  const int b = 16 * bt + row;
   float sum = 0.f;
   auto put = [&](int j, f32x4 v) {
     sum += (v[0] + v[1]) + (v[2] + v[3]);
-    const bf16x4 pk = {(__bf16)v[0], (__bf16)v[1], (__bf16)v[2], (__bf16)v[3]};
-    *reinterpret_cast<bf16x4*>(base + (size_t)((j >> 5) * 64 + ((j >> 3) & 3) * 16 + row) * 16 + (j & 7) * 2) = pk;
+    panel_put(ps.x[0], NPAD >> 5, b, j, v);
+    panel_put(ps.x[1], NPAD >> 5, b, j, v);
   };
-  const int b = 16 * bt + row;
   // Sixteen loads in flight: one at a time this launch is all latency, 12.7 against 5 us.  Addresses are clamped into the
   // row; where N is no multiple of four, values that reach past its end are read as the row's last four and moved into
   // place (N = 2047, B = 16, 2 channels: 25 -> 17 us per step).  (NPAD is a multiple of 512; what lies past it is skipped.)
@@ -188,15 +230,18 @@ __global__ __launch_bounds__(64) void ring_panel_operand_kernel(const float* __r
     }
   }
   sum = row16_sum_dpp(sum);
-  if (sub == 0) rs[16 * bt + row] = sum;
+  if (sub == 0) {
+    ps.rs[0][b] = sum;
+    ps.rs[1][b] = __builtin_bit_cast(float, PANEL_EMPTY);
+  }
 }
 
 // One step for R row tiles x C column tiles (16 consecutive neurons each).  Wpack: order 3 of ring_pack_weights_kernel.
 template <int ACT, int R>
-__global__ __launch_bounds__(256) void ring_panel_fwd_kernel(RingFwdArgs p, const bf16x8* __restrict__ xfrag,
-                                                             const float* __restrict__ rs, int NC, int C, int t, int xcd_map) {
+__global__ __launch_bounds__(256) void ring_panel_fwd_kernel(RingFwdArgs p, PanelState state, int NC, int C, int t, int xcd_map) {
   extern __shared__ __attribute__((aligned(16))) char panel_lds[];
   __shared__ int list[BN_GATE_KMAX + 1];
+  __shared__ float row_sums[16 * R];
   const int tid = threadIdx.x, wv = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
   const int N = p.N, B = p.B, T = p.T, k = p.k, KCH = 2 * NC;
   bf16x8* const xs = reinterpret_cast<bf16x8*>(panel_lds);                                  // [2][R][PANEL_S][64]
@@ -205,12 +250,37 @@ __global__ __launch_bounds__(256) void ring_panel_fwd_kernel(RingFwdArgs p, cons
   int rg, cb;
   step_block_coords(xcd_map, rg, cb);
   const int bt0 = rg * R;
+  const bf16x8* const xfrag = state.x[t & 1];
+  // this workgroup's share of the row sums (there are at least as many column blocks as row tiles: a row per 16 lanes at
+  // most), announced to the others of its rows
+  const int sum_row = cb + (int)gridDim.y * (tid >> 4), sum_b = 16 * bt0 + sum_row;
+  const bool sums_row = sum_row < 16 * R && sum_b < B;
+  // (the widest panels, whose steps are long, have its loads in flight over the gates' at the price of a longer program:
+  // N = 2048, 16 channels, B = 256: 57.7 -> 56.2 us per step, but 2 channels, B = 1: 7.6 -> 8.4)
+  constexpr bool EARLY = R == 8;
+  const float* const own_fours = state.fours[t & 1] + (size_t)sum_b * (16 * NC);
+  float own_sum = 0.f;
+  PanelRowSum<EARLY ? 32 : 1> own;                          // (N <= 2048)
+  if (sums_row && t > 0) {
+    if constexpr (EARLY) own.load(own_fours, N, tid & 15);
+    else own_sum = panel_row_sum(own_fours, N, tid & 15);
+  }
 
   for (int idx = tid; idx < R * 16 * k; idx += 256) {
     const int row = idx / k, c = idx - row * k, b = 16 * bt0 + row;
     gl[idx] = b < B ? p.A[((size_t)b * T + t) * k + c] : 0.f;
   }
   for (int i = tid; i < C * R * 64; i += 256) sums[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+  if (sums_row) {
+    if constexpr (EARLY) {
+      own.add(own_sum, N, tid & 15);
+      own_sum = row16_sum_dpp(own_sum);
+    }
+    if ((tid & 15) == 0) {
+      if (t > 0) __hip_atomic_store(state.rs[t % 3] + sum_b, own_sum, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      state.rs[(t + 1) % 3][sum_b] = __builtin_bit_cast(float, PANEL_EMPTY);
+    }
+  }
   lds_barrier();
   // matrices worth multiplying: Wo, and the channels that are not zero in all of the workgroup's rows
   int nact = 1;
@@ -269,17 +339,30 @@ __global__ __launch_bounds__(256) void ring_panel_fwd_kernel(RingFwdArgs p, cons
     }
   }
 
+  // (step and thread as the compiler does not know them from above: what follows from them is not kept over the products)
+  int now = t, me = tid;
+  asm volatile("" : "+s"(now), "+v"(me));
+  for (int row = me >> 4; row < 16 * R; row += 16) {
+    const int b = 16 * bt0 + row, sub = me & 15;
+    if (b >= B) break;
+    float s = __hip_atomic_load(state.rs[now % 3] + b, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (__builtin_bit_cast(unsigned, s) == PANEL_EMPTY)                        // (the same in the row's 16 lanes)
+      s = panel_row_sum(state.fours[now & 1] + (size_t)b * (16 * NC), N, sub);
+    if (sub == 0) row_sums[row] = s;
+  }
+  lds_barrier();
+
   // activation and leak; a thread takes four consecutive neurons of a row
-  const float* prev = (t == 0) ? p.r_init : p.hist + (size_t)(t - 1) * B * N;
-  float* out = p.hist + (size_t)t * B * N;
+  const float* prev = (now == 0) ? p.r_init : p.hist + (size_t)(now - 1) * B * N;
+  float* out = p.hist + (size_t)now * B * N;
   const float oma = 1.f - p.alpha;
   const float* sf = reinterpret_cast<const float*>(sums);
-  for (int idx = tid; idx < R * 16 * 4 * C; idx += 256) {
+  for (int idx = me; idx < R * 16 * 4 * C; idx += 256) {
     const int row = idx / (4 * C), j4 = 4 * (idx % (4 * C)), cc = j4 >> 4, n = j4 & 15;
     const int b = 16 * bt0 + row, j = 16 * C * cb + j4, i = row >> 4;
     if (b >= B || j >= N) continue;
     const f32x4 rp = load4_masked(prev, N, B, b, j);
-    const float js = p.J0 * rs[b];
+    const float js = p.J0 * row_sums[row];
     f32x4 rn;
 #pragma unroll
     for (int x = 0; x < 4; ++x) {
@@ -289,6 +372,12 @@ __global__ __launch_bounds__(256) void ring_panel_fwd_kernel(RingFwdArgs p, cons
       rn[x] = fmaf(p.alpha, F, oma * rp[x]);
     }
     store4_masked(out, N, B, b, j, rn);
+    if (now + 1 < T) {
+#pragma unroll
+      for (int x = 1; x < 4; ++x) rn[x] = j + x < N ? rn[x] : 0.f;
+      panel_put(state.x[(now + 1) & 1], KCH, b, j, rn);
+      state.fours[(now + 1) & 1][(size_t)b * (16 * NC) + (j >> 2)] = (rn[0] + rn[1]) + (rn[2] + rn[3]);
+    }
   }
 }
 
@@ -302,7 +391,8 @@ static size_t panel_lds_bytes(int R, int C, int k) {
 // Row tiles and column tiles of a workgroup.  Per K chunk a workgroup needs the longer of its matrix-pipe time
 // (16 cycles an MFMA, the fullest wave's share) and its loads: a compute unit takes in some 16 bytes per cycle from the
 // memory side of its L2, whatever is in flight (measured: 18 KiB a chunk on 128 compute units and 25 KiB on 256 both run
-// at 15 to 17).  Workgroups beyond one per compute unit queue.  us per step, N = 2048, by (row tiles, column tiles):
+// at 15 to 17).  Workgroups beyond one per compute unit queue.  us per step, N = 2048, by (row tiles, column tiles), with
+// a launch for the operand of 5 us in each:
 //   16 channels, B = 256:  (8,1) 64  (4,1) 71  (4,2) 66  (8,2) 98      B = 1:  (1,1) 39  (4,1) 45  (8,1) 57
 //   16 channels, B = 1024: (8,1) 208 (8,2) 195 (8,4) 189               2 channels, B = 256:  (4,2) 22  (8,1) 27  (8,4) 43
 static void panel_shape(int NC, int nbt, int k, int* R_out, int* C_out) {
@@ -326,7 +416,10 @@ static void panel_shape(int NC, int nbt, int k, int* R_out, int* C_out) {
 
 bool ring_panel_applicable(int NC, int k) { return NC >= 16 && NC % 8 == 0 && k <= BN_GATE_KMAX; }
 
-size_t ring_panel_workspace_bytes(int NC, int nbt) { return (size_t)nbt * 2 * NC * 1024 + (size_t)nbt * 16 * sizeof(float); }
+static size_t panel_operand_bytes(int NC, int nbt) { return (size_t)nbt * 2 * NC * 1024; }
+size_t ring_panel_workspace_bytes(int NC, int nbt) {
+  return 2 * panel_operand_bytes(NC, nbt) + 2 * (size_t)nbt * 16 * 16 * NC * sizeof(float) + 3 * (size_t)nbt * 16 * sizeof(float);
+}
 
 // RINGATTR_PANEL=0: never; a switch that asks for one of the other step-per-launch families is obeyed.
 bool ring_uses_panel(int k, int NC, int nbt) {
@@ -335,7 +428,7 @@ bool ring_uses_panel(int k, int NC, int nbt) {
   if (v && v[0] == '0') return false;
   for (const char* name : {"RINGATTR_WIDE", "RINGATTR_BLOCK", "RINGATTR_BLOCK_SHAPE"})
     if (getenv(name)) return false;
-  return ring_panel_workspace_bytes(NC, nbt) < ((size_t)1 << 30);   // (32-bit offsets; the weights are 0.6 GB at most)
+  return panel_operand_bytes(NC, nbt) < ((size_t)1 << 30);   // (32-bit offsets; the weights are 0.6 GB at most)
 }
 
 template <int ACT, int R>
@@ -344,14 +437,16 @@ static hipError_t panel_run(const RingFwdArgs& a, int NC, int C, hipStream_t st)
   hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&ring_panel_fwd_kernel<ACT, R>),
                                      hipFuncAttributeMaxDynamicSharedMemorySize, (int)dyn);
   if (e != hipSuccess) return e;
-  bf16x8* xfrag = reinterpret_cast<bf16x8*>(a.panel_ws);
-  float* rs = reinterpret_cast<float*>(xfrag + (size_t)a.nbt * 2 * NC * 64);
+  PanelState ps;
+  char* ws = reinterpret_cast<char*>(a.panel_ws);
+  for (int i = 0; i < 2; ++i, ws += panel_operand_bytes(NC, a.nbt)) ps.x[i] = reinterpret_cast<bf16x8*>(ws);
+  for (int i = 0; i < 2; ++i, ws += (size_t)a.nbt * 16 * 16 * NC * sizeof(float)) ps.fours[i] = reinterpret_cast<float*>(ws);
+  for (int i = 0; i < 3; ++i, ws += (size_t)a.nbt * 16 * sizeof(float)) ps.rs[i] = reinterpret_cast<float*>(ws);
   const dim3 grid((a.nbt + R - 1) / R, 4 * NC / C);
   const int xm = step_xcd_map();
+  RING_LAUNCH(ring_panel_operand_kernel, dim3(4 * a.nbt), dim3(64), 0, st, a.r_init, ps, a.N, a.B, 64 * NC);
   for (int t = 0; t < a.T; ++t) {
-    const float* prev = t == 0 ? a.r_init : a.hist + (size_t)(t - 1) * a.B * a.N;
-    RING_LAUNCH(ring_panel_operand_kernel, dim3(4 * a.nbt), dim3(64), 0, st, prev, xfrag, rs, a.N, a.B, 64 * NC);
-    RING_LAUNCH((ring_panel_fwd_kernel<ACT, R>), grid, dim3(256), dyn, st, a, xfrag, rs, NC, C, t, xm);
+    RING_LAUNCH((ring_panel_fwd_kernel<ACT, R>), grid, dim3(256), dyn, st, a, ps, NC, C, t, xm);
     e = hipGetLastError();
     if (e != hipSuccess) return e;
   }

@@ -23,6 +23,8 @@ def _forward(p, act, J0, J1, dev):
     (1, 3, 2, 1025, "relu", None), (17, 3, 1, 1030, "gelu", None), (150, 2, 3, 1536, "tanh", None),
     (40, 2, 16, 2048, "silu", None), (130, 2, 4, 1600, "gelu", "84"), (33, 2, 24, 600, "tanh", None),
     (20, 2, 21, 700, "relu", "22"), (70, 2, 6, 1100, "silu", "42"),
+    # what travels between the steps comes round again: more steps than buffers, the last four neurons not whole
+    (33, 7, 2, 1027, "gelu", "11"), (20, 8, 2, 1025, "tanh", "24"), (150, 7, 3, 1030, "silu", "81"), (1, 9, 16, 2047, "gelu", None),
 ])
 def test_panel_equals_block_kernels_and_oracle(B, T, k, N, act, shape, gpu_device, monkeypatch):
     print(f"[case] panel B={B} T={T} k={k} N={N} {act} shape={shape}", flush=True)
