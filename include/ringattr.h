@@ -157,6 +157,14 @@ RINGATTR_API int ringattr_fwd_loss(const void* A, const void* Wa, float J0, floa
                       const void* target_angle, const void* target_amplitude, float bump_weight, void* loss_out,
                       void* loss_workspace, size_t loss_workspace_bytes, void* stream);
 
+/* The same with the total written to a place of its own as well (one device float, or NULL): what a caller differentiates
+ * need not share memory with what it logs, nor be copied out of it by another launch. */
+RINGATTR_API int ringattr_fwd_loss_total(const void* A, const void* Wa, float J0, float J1, const void* Wo, const void* r_init,
+                      void* bump_history, float alpha, int N, int a_dim, int seq_len, int batch_size,
+                      int activation_type, void* saved, void* workspace, size_t workspace_bytes,
+                      const void* target_angle, const void* target_amplitude, float bump_weight, void* loss_out,
+                      void* loss_total, void* loss_workspace, size_t loss_workspace_bytes, void* stream);
+
 /* ringattr_bwd with the loss head's gradient in place of grad_output: the backward of
  *   total = loss_pair(bump_history),  bump_history = forward(...)
  * in one call.  No counterpart in the reference (its training script lets autograd chain the torch loss ops into

@@ -133,10 +133,10 @@ bool ring_dw_tiled_applicable(int NC);
 int ring_dw_tiled_nz(int NC, int k, long nchunk);
 hipError_t ring_launch_dw_tiled(const RingDwArgs& a, int NC, hipStream_t st);
 
-// Fused decode + loss head over the state history (ring_loss.hip).
+// Fused decode + loss head over the state history (ring_loss.hip).  loss_total: null, or where loss_out[0] goes as well.
 size_t ring_loss_workspace_bytes(int T, int B);
 hipError_t ring_launch_loss_fwd(const float* hist, const float* angle, const float* target_amp, float bump_weight,
-                                float* loss_out, int N, int T, int B, void* workspace, bool have_row_sums,
+                                float* loss_out, float* loss_total, int N, int T, int B, void* workspace, bool have_row_sums,
                                 hipStream_t st);
 // where the forward kernel leaves the per-row sums for ring_launch_loss_fwd(..., have_row_sums = true)
 ring_f32x4* ring_loss_row_sums(void* workspace);

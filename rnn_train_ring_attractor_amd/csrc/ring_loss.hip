@@ -231,7 +231,7 @@ __global__ __launch_bounds__(256) void ring_loss_decode_kernel(f32x4* __restrict
 // are combined by a fixed tree (bitwise repeatable).
 __global__ __launch_bounds__(256) void ring_loss_final_kernel(const float* __restrict__ partial, int nparts,
                                                               const float* __restrict__ sq, int B, float inv_rows,
-                                                              float bump_weight, float* __restrict__ out) {
+                                                              float bump_weight, float* __restrict__ out, float* __restrict__ total) {
   __shared__ double rc[256], ra[256];
   double c = 0.0, a = 0.0;
   for (int i = threadIdx.x; i < nparts; i += 256) c += partial[i];
@@ -251,6 +251,7 @@ __global__ __launch_bounds__(256) void ring_loss_final_kernel(const float* __res
     out[0] = lc + bump_weight * la;
     out[1] = lc;
     out[2] = la;
+    if (total) *total = out[0];
   }
 }
 
@@ -362,7 +363,7 @@ static LossWs carve(void* workspace, int T, int B) {
 // have_row_sums: the workspace's row-sum array (ring_loss_row_sums) is already filled (by the forward kernel); the
 // pass over the history is skipped and `hist` is not read.
 hipError_t ring_launch_loss_fwd(const float* hist, const float* angle, const float* target_amp, float bump_weight,
-                                float* loss_out, int N, int T, int B, void* workspace, bool have_row_sums,
+                                float* loss_out, float* loss_total, int N, int T, int B, void* workspace, bool have_row_sums,
                                 hipStream_t st) {
   if (N > 256 * L_MAXCH) return hipErrorInvalidValue;
   const LossWs w = carve(workspace, T, B);
@@ -376,7 +377,7 @@ hipError_t ring_launch_loss_fwd(const float* hist, const float* angle, const flo
   hipLaunchKernelGGL(ring_loss_decode_kernel, dim3(dgrid), dim3(256), 0, st, w.stats, angle, target_amp, w.sq, w.partial, k,
                      bump_weight, T, B);
   hipLaunchKernelGGL(ring_loss_final_kernel, dim3(1), dim3(256), 0, st, w.partial, dgrid, w.sq, B, 1.f / (float)rows,
-                     bump_weight, loss_out);
+                     bump_weight, loss_out, loss_total);
   return hipGetLastError();
 }
 

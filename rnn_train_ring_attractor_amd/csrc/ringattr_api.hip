@@ -238,6 +238,16 @@ int ringattr_fwd_loss(const void* A, const void* Wa, float J0, float J1, const v
                       void* saved, void* workspace, size_t workspace_bytes, const void* target_angle,
                       const void* target_amplitude, float bump_weight, void* loss_out, void* loss_workspace,
                       size_t loss_workspace_bytes, void* stream) {
+  return ringattr_fwd_loss_total(A, Wa, J0, J1, Wo, r_init, bump_history, alpha, N, a_dim, seq_len, batch_size, activation_type, saved,
+                                 workspace, workspace_bytes, target_angle, target_amplitude, bump_weight, loss_out, nullptr,
+                                 loss_workspace, loss_workspace_bytes, stream);
+}
+
+int ringattr_fwd_loss_total(const void* A, const void* Wa, float J0, float J1, const void* Wo, const void* r_init,
+                            void* bump_history, float alpha, int N, int a_dim, int seq_len, int batch_size, int activation_type,
+                            void* saved, void* workspace, size_t workspace_bytes, const void* target_angle,
+                            const void* target_amplitude, float bump_weight, void* loss_out, void* loss_total,
+                            void* loss_workspace, size_t loss_workspace_bytes, void* stream) {
   const size_t need = ringattr_loss_workspace_bytes(N, seq_len, batch_size);
   if (need == 0) return RINGATTR_ERR_INVALID;
   if (!target_angle || !loss_out) return fail(RINGATTR_ERR_INVALID, "ringattr_fwd_loss: null tensor pointer");
@@ -250,7 +260,7 @@ int ringattr_fwd_loss(const void* A, const void* Wa, float J0, float J1, const v
                           saved, workspace, workspace_bytes, ring_loss_row_sums(loss_workspace), &stats_done, stream);
   if (rc) return rc;
   hipError_t e = ring_launch_loss_fwd((const float*)bump_history, (const float*)target_angle, (const float*)target_amplitude,
-                                      bump_weight, (float*)loss_out, N, seq_len, batch_size, loss_workspace, stats_done,
+                                      bump_weight, (float*)loss_out, (float*)loss_total, N, seq_len, batch_size, loss_workspace, stats_done,
                                       static_cast<hipStream_t>(stream));
   if (e != hipSuccess) return hip_fail(e, "loss head forward launch");
   return RINGATTR_OK;
@@ -616,7 +626,7 @@ int ringattr_loss_fwd(const void* bump_history, const void* target_angle, const 
     return fail(RINGATTR_ERR_WORKSPACE, "ringattr_loss_fwd: workspace of %zu bytes needed, %zu given", need,
                 workspace ? workspace_bytes : (size_t)0);
   hipError_t e = ring_launch_loss_fwd((const float*)bump_history, (const float*)target_angle, (const float*)target_amplitude,
-                                      bump_weight, (float*)loss_out, N, seq_len, batch_size, workspace, false,
+                                      bump_weight, (float*)loss_out, nullptr, N, seq_len, batch_size, workspace, false,
                                       static_cast<hipStream_t>(stream));
   if (e != hipSuccess) return hip_fail(e, "loss head forward launch");
   return RINGATTR_OK;

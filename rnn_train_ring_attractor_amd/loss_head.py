@@ -122,14 +122,15 @@ class RingRnnLossFunc(Function):
                 _lib.check(1)
             lws = torch.empty(nbytes, dtype=torch.uint8, device=dev)
             out = torch.empty(3, dtype=torch.float32, device=dev)
+            total = torch.empty((), dtype=torch.float32, device=dev)     # (the differentiable result does not alias the logging tensor)
         # time loop and loss head in one call: the weight-resident forward kernel forms the loss's row sums itself
         fwd_cuda.fwd(A=A, Wa=Wa_c, J0=J0, J1=J1, Wo=Wo_c, r_init=r0, bump_history=hist, alpha=alpha,
-                     activation_type=act, saved=saved, loss=(angle, amp, float(bump_weight), out, lws))
+                     activation_type=act, saved=saved, loss=(angle, amp, float(bump_weight), out, lws, total))
         ctx.save_for_backward(A, Wa_c, Wo_c, hist, r0, saved, lws, angle, amp)
         ctx.J0, ctx.J1, ctx.alpha, ctx.act, ctx.bump_weight = J0, J1, alpha, act, float(bump_weight)
         ctx.mark_non_differentiable(out, hist)
         ctx.set_materialize_grads(False)         # no [T,B,N] tensor of zeros for the history's unused gradient
-        return out[0].clone(), out, hist
+        return total, out, hist
 
     @staticmethod
     def backward(ctx, grad_total, _grad_parts, _grad_hist):
