@@ -111,10 +111,9 @@ class RingGainNetsFunc(Function):
             ws = torch.empty(nbytes, dtype=torch.uint8, device=signal.device)
             _lib.check(lib.ringattr_gain_nets_bwd(signal.data_ptr(), int(halves), _pointers(params), g.data_ptr(), grad.data_ptr(), k, h,
                                                   T, B, ws.data_ptr(), nbytes, torch.cuda.current_stream(signal.device).cuda_stream))
-        parts = []
-        for row in grad:
-            w1, b1, w2, b2 = row.split((h, h, h, 1))
-            parts += [w1.view(h, 1), b1, w2.view(1, h), b2]
+        parts = list(grad.view(-1).split((h, h, h, 1) * k))
+        for c in range(0, 4 * k, 4):
+            parts[c], parts[c + 2] = parts[c].view(h, 1), parts[c + 2].view(1, h)
         return (None, None, *parts)
 
 
