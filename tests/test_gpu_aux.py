@@ -123,9 +123,10 @@ def test_fused_clip_adam_matches_torch(max_norm, gpu_device):
     assert all(torch.equal(x, y) for x, y in zip(opt2.params, opt3.params))
 
 
-# k a multiple of four and not, a slice that starts off a 16-byte boundary, one sample, more samples than one pass of the grid
+# k a multiple of four and not, a slice that starts off a 16-byte boundary, one sample, more samples than one pass of the grid,
+# the most that a single workgroup takes and one more
 @pytest.mark.parametrize("B,T,k,N,pair,offset", [(1, 1, 3, 17, (0, 2), 0), (5, 7, 16, 33, (0, 1), 0), (40, 9, 6, 130, (2, 5), 3),
-                                                 (700, 513, 4, 20, (1, 3), 1)])
+                                                 (700, 513, 4, 20, (1, 3), 1), (8, 128, 16, 33, (0, 1), 0), (25, 41, 16, 33, (0, 1), 0)])
 def test_compacted_channels_are_the_named_ones_and_the_rest_is_checked(B, T, k, N, pair, offset, gpu_device):
     from rnn_train_ring_attractor_amd.ring_rnn_cuda import _compact
     print(f"[case] compaction B={B} T={T} k={k} N={N} {pair}", flush=True)
