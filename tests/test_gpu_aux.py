@@ -123,6 +123,22 @@ def test_fused_clip_adam_matches_torch(max_norm, gpu_device):
     assert all(torch.equal(x, y) for x, y in zip(opt2.params, opt3.params))
 
 
+# the most partial sums of the norm that every workgroup of the update adds up itself, and one more
+@pytest.mark.parametrize("numel", [1024 * 4096, 1024 * 4096 + 1])
+def test_fused_clip_adam_of_many_parameters(numel, gpu_device):
+    from rnn_train_ring_attractor_amd import FusedClipAdam
+    print(f"[case] clip and Adam, {numel} parameters", flush=True)
+    w = torch.zeros(numel, device=gpu_device, requires_grad=True)
+    w.grad = torch.full((numel,), 0.5, device=gpu_device)
+    opt = FusedClipAdam([w], lr=1e-3, betas=(0.9, 0.999), eps=1e-8, max_norm=1.0)
+    opt.step()
+    torch.cuda.synchronize()
+    norm = 0.5 * numel ** 0.5                # sums of 2^-2: exact in fp32 but for the tree's last roundings
+    assert abs(float(opt.last_grad_norm) - norm) <= 1e-6 * norm
+    g = 0.5 / (norm + 1e-6)
+    assert float((w.grad - g).abs().max()) <= 1e-6 * g and float((w.detach() + 1e-3).abs().max()) <= 1e-3 * (1e-5 + 1e-8 / g)
+
+
 # k a multiple of four and not, a slice that starts off a 16-byte boundary, one sample, more samples than one pass of the grid,
 # the most that a single workgroup takes and one more
 @pytest.mark.parametrize("B,T,k,N,pair,offset", [(1, 1, 3, 17, (0, 2), 0), (5, 7, 16, 33, (0, 1), 0), (40, 9, 6, 130, (2, 5), 3),
