@@ -124,9 +124,9 @@ __device__ __forceinline__ u32x2 quad_rows2(unsigned x, int lane) {
 // Eight consecutive weights of one output neuron `out`, contraction indices k0 .. k0 + 7, from an fp32 [N][N] matrix.
 // Loads and arithmetic are apart so that several fragments' loads can be in flight; addresses are clamped into the
 // matrix and the padding is zeroed afterwards.  ROWS4 (rows that start on 16-byte boundaries): two 16-byte loads, eight
-// fragments at a time; a call of T = 20 steps falls from 181 to 128 us at N = 512, 16 channels, B = 256, from 105 to 70 at
-// N = 1024, two channels, B = 1 (all on their way at once into one XCD: 12.6 MB).  Other rows are slower so than a word at a
-// time (N = 1023, B = 100: 140 against 98 us).
+// fragments on their way; a call of T = 20 steps at N = 512, 16 channels, B = 256 falls from 181 us (a word at a time, four
+// fragments) to 106, at N = 1024, two channels, B = 1 from 105 to 61 (all on their way at once into one XCD: 12.6 MB).
+// Other rows are slower so than a word at a time (N = 1023, B = 100: 140 against 98 us).
 struct WeightLoad { float v[8]; };
 typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));
 typedef float f32x2u __attribute__((ext_vector_type(2), aligned(4)));
@@ -262,28 +262,27 @@ struct TeamCompute {
         }
       }
     }
+    // into registers: each fragment's place is loaded again as soon as it is converted.  In batches that drain before the
+    // next begins, and with conversions left until the fragment's first use, the loads' registers spill (780 bytes a lane in
+    // the kernel of 13 matrices in registers) and the same two calls take 131 and 74 us; so the fragment is opaque here.
+    WeightLoad l[BATCH];
+    auto load = [&](int f) {
+      const int mm = f / (C16 * KPW), cc = f / KPW % C16, kc = w + WK * (f % KPW);
+      const float* W = mm == 0 || mm > c.k ? c.Wo : c.Wa + (size_t)(mm - 1) * c.N * c.N;
+      weight_load<HOW>(l[f % BATCH], W, c.N, 16 * (mem * C16 + cc) + n, 32 * kc + 8 * q);
+    };
 #pragma unroll
-    for (int f0 = 0; f0 < F; f0 += BATCH) {
-      WeightLoad l[BATCH];
+    for (int f = 0; f < BATCH && f < F; ++f) load(f);
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-      for (int i = 0; i < BATCH; ++i) {
-        const int f = f0 + i, mm = f / (C16 * KPW), cc = f / KPW % C16, kc = w + WK * (f % KPW);
-        if (f < F) {
-          const float* W = mm == 0 || mm > c.k ? c.Wo : c.Wa + (size_t)(mm - 1) * c.N * c.N;
-          weight_load<HOW>(l[i], W, c.N, 16 * (mem * C16 + cc) + n, 32 * kc + 8 * q);
-        }
-      }
-      __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-      for (int i = 0; i < BATCH; ++i) {
-        const int f = f0 + i, mm = f / (C16 * KPW), cc = f / KPW % C16, kc = w + WK * (f % KPW);
-        if (f < F) {
-          const bf16x8 v = weight_fragment(l[i], mm <= c.k ? c.N : 0, 16 * (mem * C16 + cc) + n, 32 * kc + 8 * q,
-                                           mm == 0 ? c.scale0 : 1.f, mm == 0 ? c.shift0 : 0.f);
-          if (f < FR) wreg[f < FR ? f : 0] = v;
-          else parked[(f - FR) * 64] = v;
-        }
-      }
+    for (int f = 0; f < F; ++f) {
+      const int mm = f / (C16 * KPW), cc = f / KPW % C16, kc = w + WK * (f % KPW);
+      bf16x8 v = weight_fragment(l[f % BATCH], mm <= c.k ? c.N : 0, 16 * (mem * C16 + cc) + n, 32 * kc + 8 * q,
+                                 mm == 0 ? c.scale0 : 1.f, mm == 0 ? c.shift0 : 0.f);
+      asm volatile("" : "+v"(v));
+      if (f < FR) wreg[f < FR ? f : 0] = v;
+      else parked[(f - FR) * 64] = v;
+      if (f + BATCH < F) load(f + BATCH);
       __builtin_amdgcn_sched_barrier(0);
     }
   }
