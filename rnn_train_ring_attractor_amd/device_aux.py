@@ -45,7 +45,7 @@ def generate_inputs(seed, batch_size, seq_len, num_neurons, action_dim=2, zero_p
 
 
 class FusedClipAdam:
-    """clip_grad_norm_(params, max_norm) + Adam.step() in three launches for all parameter tensors.
+    """clip_grad_norm_(params, max_norm) + Adam.step() in two or three launches for all parameter tensors.
 
     Same update as torch.optim.Adam (no weight decay, no amsgrad) after torch.nn.utils.clip_grad_norm_; state
     (exp_avg, exp_avg_sq, step) is kept per tensor as torch does.  `last_grad_norm` is a device scalar (the norm
