@@ -124,7 +124,7 @@ struct OneLane {
 template <int KCT, int MR, int RW>
 struct OneLds {
   bf16x8 x[2][KCT * 4 * RW];         // operand: [chunk][q][row] x 8 neurons
-  float rs[2][KCT * 4 * RW];         // fp32 sums of the unrounded values, groups of eight neurons
+  float rs[2][KCT * 4 * RW];         // fp32 sums of the unrounded values, groups of eight neurons (zeros without a J0 term)
   float gates[2][(MR - 1) * RW + 1]; // [channel][row], and a word for idle threads
 };
 
@@ -266,6 +266,12 @@ struct OneStream {
   }
 };
 
+// Without a J0 term no step writes row sums: zeros once, because J0 times what LDS was left with need not be zero.
+template <int KCT, int MR, int RW>
+__device__ __forceinline__ void one_no_sums(OneLds<KCT, MR, RW>& L, int tid) {
+  for (int i = tid; i < 2 * KCT * 4 * RW; i += 128 * KCT) (&L.rs[0][0])[i] = 0.f;
+}
+
 __device__ __forceinline__ int one_rows(int first, int B, int RW) { return B - first < 0 ? 0 : (B - first < RW ? B - first : RW); }
 
 }  // namespace
@@ -306,6 +312,7 @@ __global__ __launch_bounds__(128 * KCT, 2) void ring_team_one_fwd_kernel(RingFwd
     before[i] = 0.f;
     d[i] = (_Float16)0.f;
   }
+  if (!sums) one_no_sums(L, tid);
   one_put(L, 0, o, sums, r);
   og.put(L.gates[0], g0);
   const size_t tile_d = (size_t)c.cts * 256, tile_p = (size_t)c.cts * 512;
@@ -403,6 +410,7 @@ __global__ __launch_bounds__(128 * KCT, 2) void ring_team_one_bptt_kernel(RingBp
   };
   In inA, inB;
   og.put(L.gates[0], og.fetch(gate_at));
+  if (!sums) one_no_sums(L, tid);
   bf16x8 wt[MR][KCT];
   one_weights<KCT, MR, true>(c, w, tid & 63, wt);
   fetch(inA);

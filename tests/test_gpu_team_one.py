@@ -61,6 +61,26 @@ def test_teams_of_one_against_the_oracle(B, T, k, N, act, gpu_device):
         assert O.cosine(x, g[name]) >= GRAD_COS and O.max_rel_err(x, g[name]) <= GRAD_TOL, name
 
 
+# 4, 8 and 16 rows per workgroup, whole and cut tiles, both register groups
+@pytest.mark.parametrize("B,k,N", [(64, 2, 120), (2048, 2, 128), (1500, 5, 101), (4096, 2, 120), (40, 2, 50)])
+def test_teams_of_one_without_a_j0_term_after_a_run_of_nan(B, k, N, gpu_device):
+    """J0 = 0: a launch's results do not depend on what an earlier one left in LDS (here operands and row sums of NaN)."""
+    print(f"[case] team of one, J0 = 0, B={B} k={k} N={N}", flush=True)
+    T = 4
+    p = make_problem(500 + N, B, T, k, N, action="dense")
+    left = make_problem(501, 4200, 2, k, N, action="dense")
+    bad = _run({**left, "r0": np.full_like(left["r0"], np.nan)}, "gelu", -1.0 / N, 0.6, gpu_device)
+    assert torch.isnan(bad["hist"]).all() and torch.isnan(bad["grad_r_init"]).all()
+    got = _run(p, "gelu", 0.0, 0.6, gpu_device)
+    ref, _ = O.forward_dense(p["A"], p["Wa"], 0.0, 0.6, p["Wo"], p["r0"], 0.15, "gelu")
+    assert O.max_rel_err(got["hist"].cpu().numpy(), ref) <= TRAJ_TOL
+    g = O.backward_dense(p["G"], p["A"], p["Wa"], 0.0, 0.6, p["Wo"], ref, p["r0"], 0.15, "gelu")
+    for name in ("grad_Wo", "grad_Wa", "grad_r_init", "grad_A"):
+        x = got[name].cpu().numpy()
+        assert np.isfinite(x).all(), name
+        assert O.cosine(x, g[name]) >= GRAD_COS and O.max_rel_err(x, g[name]) <= GRAD_TOL, name
+
+
 @pytest.mark.parametrize("N,k", [(100, 2), (127, 5), (50, 3)])
 def test_rows_of_teams_of_one_do_not_depend_on_the_batch(N, k, gpu_device):
     B, T = 600, 6
