@@ -53,30 +53,39 @@ __device__ __forceinline__ void gates_publish(f32x2* gb, int tid, int B, int bt,
   gb[(j + 16) * 16 + row] = g.b * m;
 }
 
-// The 16 rows of a batch tile in a [B][N] matrix, for the masked kernels: the buffer ends with the batch, so rows past it
-// read zeros and are not written, without a branch per element.  (Of those the BPTT had sixteen a step and the forward
+// The 16 rows of a batch tile in a [B][N] matrix, for the masked kernels: a buffer that ends with the batch, so rows past it
+// read zeros and are not written, without a branch per element.  Nothing goes into a buffer instruction's scalar offset, which
+// is not part of the range check: a store has its row in the vector offset, a load has a buffer from its row on (us, T = 100,
+// N = 200, B = 1000: the loads the other way a pass with the loss and dL/dA 520 -> 556, the stores a forward 145 -> 152; with both
+// in the scalar offset 1 % less).
+// (Of the branches the BPTT had sixteen a step and the forward
 // eight.  us per call, T = 100, gelu: N = 200, B = 1024: BPTT 301 -> 146, forward 159 -> 153; N = 201: 204 -> 181; dL/dA and
 // the loss's gradient, N = 200, B = 4096, relu: 581 -> 342.  The streaming kernels' rows are wider and gain nothing: N = 510,
 // B = 8192, us per step: forward 25.5 -> 27.3, BPTT 24.1 -> 25.1.)
 struct TileRows {
   static constexpr unsigned NOWHERE = 0x80000000u;      // (a column past N)
-  __amdgpu_buffer_rsrc_t r;
-  __device__ __forceinline__ TileRows(const float* slab, int N, int B, int bt) {
-    const int rows = B - 16 * bt < 16 ? B - 16 * bt : 16;
-    r = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(slab + (size_t)16 * bt * N), 0, rows * N * 4, 0x00020000);
+  char* base;
+  int row, bytes;                                       // of one row, of the tile's rows in the batch
+  __device__ __forceinline__ TileRows(const float* slab, int N, int B, int bt)
+      : base(reinterpret_cast<char*>(const_cast<float*>(slab + (size_t)16 * bt * N))), row(N * 4),
+        bytes((B - 16 * bt < 16 ? B - 16 * bt : 16) * N * 4) {}
+  __device__ __forceinline__ __amdgpu_buffer_rsrc_t from(int e) const {
+    const int left = bytes - e * row;
+    return __builtin_amdgcn_make_buffer_rsrc(base + e * row, 0, left > 0 ? left : 0, 0x00020000);
   }
-  __device__ __forceinline__ f32x4 load4(unsigned off, unsigned row) const {
-    return __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(r, (int)off, (int)row, 0));
+  // off: of a lane's first row and column in the tile; e: how many rows further on
+  __device__ __forceinline__ f32x4 load4(unsigned off, int e) const {
+    return __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(from(e), (int)off, 0, 0));
   }
-  __device__ __forceinline__ float load1(unsigned off, unsigned row) const {
-    return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, (int)off, (int)row, 0));
+  __device__ __forceinline__ float load1(unsigned off, int e) const {
+    return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(from(e), (int)off, 0, 0));
   }
-  __device__ __forceinline__ void store2(f32x2 v, unsigned off, unsigned row) const {
+  __device__ __forceinline__ void store2(f32x2 v, unsigned off, int e) const {
     typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
-    __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2, v), r, (int)off, (int)row, 0);
+    __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2, v), from(0), (int)(off + (unsigned)(e * row)), 0, 0);
   }
-  __device__ __forceinline__ void store1(float v, unsigned off, unsigned row) const {
-    __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, v), r, (int)off, (int)row, 0);
+  __device__ __forceinline__ void store1(float v, unsigned off, int e) const {
+    __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, v), from(0), (int)(off + (unsigned)(e * row)), 0, 0);
   }
 };
 
@@ -293,12 +302,12 @@ __global__ __launch_bounds__(512) void ring_fwd_res256_kernel(RingFwdArgs p) {
         *reinterpret_cast<f32x2*>(base + hist_lane + e * 1024) = f32x2{r[e][0], r[e][1]};
       } else {
         const TileRows tile(p.hist + (size_t)t * B * N, N, B, bt);
-        const unsigned at = (unsigned)(4 * q * N + i0) * 4u, row = (unsigned)(e * N) * 4u;
+        const unsigned at = (unsigned)(4 * q * N + i0) * 4u;
         if ((N & 1) == 0) {
-          tile.store2(f32x2{r[e][0], r[e][1]}, i0 < N ? at : TileRows::NOWHERE, row);
+          tile.store2(f32x2{r[e][0], r[e][1]}, i0 < N ? at : TileRows::NOWHERE, e);
         } else {
-          tile.store1(r[e][0], i0 < N ? at : TileRows::NOWHERE, row);
-          tile.store1(r[e][1], i0 + 1 < N ? at + 4u : TileRows::NOWHERE, row);
+          tile.store1(r[e][0], i0 < N ? at : TileRows::NOWHERE, e);
+          tile.store1(r[e][1], i0 + 1 < N ? at + 4u : TileRows::NOWHERE, e);
         }
       }
     } else if (slot < 6) {
@@ -570,17 +579,17 @@ __device__ __forceinline__ void bptt_stage_load(const RingBpttArgs& p, int t, in
     (void)i0;
   } else {
     const TileRows tile(rows + (size_t)t * p.B * p.N, p.N, p.B, bt);
-    const unsigned at = (unsigned)(4 * (lane >> 4) * p.N + i0) * 4u, row = (unsigned)p.N * 4u;
+    const unsigned at = (unsigned)(4 * (lane >> 4) * p.N + i0) * 4u;
     if ((p.N & 3) == 0) {
       const unsigned off = i0 < p.N ? at : TileRows::NOWHERE;
 #pragma unroll
-      for (int e = 0; e < 4; ++e) s.G[e] = tile.load4(off, e * row);
+      for (int e = 0; e < 4; ++e) s.G[e] = tile.load4(off, e);
     } else {
 #pragma unroll
       for (int c = 0; c < R_NC; ++c) {
         const unsigned off = i0 + c < p.N ? at + 4u * c : TileRows::NOWHERE;
 #pragma unroll
-        for (int e = 0; e < 4; ++e) s.G[e][c] = tile.load1(off, e * row);
+        for (int e = 0; e < 4; ++e) s.G[e][c] = tile.load1(off, e);
       }
     }
     s.D[0] = *reinterpret_cast<const f32x4*>(drec);

@@ -469,6 +469,43 @@ def test_block_kernel_shapes_and_workgroup_orders_agree_bitwise(B, T, k, N, act,
     assert O.max_rel_err(outs[0][0], ref_hist) <= TRAJ_TOL
 
 
+@pytest.mark.parametrize("N", [200, 201, 256])
+@pytest.mark.parametrize("B", [17, 34, 3, 21])
+def test_masked_resident_kernels_stay_inside_their_tensors(B, N, gpu_device, monkeypatch):
+    """Last batch tiles of 1, 2, 3 and 5 rows on the weight-resident kernels: nothing is written behind the history, and
+    what lies behind it and behind grad_output (here NaN) goes into nothing."""
+    from rnn_train_ring_attractor_amd import _lib, rnn_cuda
+    monkeypatch.setenv("RINGATTR_TEAM", "0")
+    T, k = 5, 2
+    print(f"[case] masked resident kernels, last tile B={B} N={N}", flush=True)
+    p = make_problem(93, B, T, k, N, action="dense")
+    A, Wa, Wo, r0 = (_t(p[x], gpu_device) for x in ("A", "Wa", "Wo", "r0"))
+
+    def inside(guard):
+        room = torch.full((T * B * N + 2 * guard,), float("nan"), device=gpu_device)
+        return room, room[guard:guard + T * B * N].view(T, B, N)
+
+    outs = []
+    for guard in (0, 16 * N * 4):
+        (room, hist), (_, G) = inside(guard), inside(guard)
+        G.copy_(_t(p["G"], gpu_device))
+        sv = torch.empty(rnn_cuda.saved_nbytes(N, k, T, B), dtype=torch.uint8, device=gpu_device)
+        common = dict(A=A, Wa=Wa, J0=-0.1, J1=0.3, Wo=Wo, r_init=r0, bump_history=hist, alpha=0.15, activation_type=1, saved=sv)
+        rnn_cuda.fwd_cuda.fwd(**common)
+        grads = {"grad_Wa": torch.zeros_like(Wa), "grad_Wo": torch.zeros_like(Wo), "grad_r_init": torch.zeros_like(r0),
+                 "grad_A": torch.zeros_like(A)}
+        rnn_cuda.bwd_cuda.bwd(grad_output=G, accumulate=False, **common, **grads)
+        torch.cuda.synchronize()
+        names = _lib.last_kernel_names()
+        assert "ring_fwd_res256" in names["fwd"] and "ring_bptt_res256" in names["bptt"], names
+        assert torch.isnan(room[:guard]).all() and torch.isnan(room[guard + T * B * N:]).all()
+        outs.append([hist.clone(), *grads.values()])
+    for x, y in zip(*outs):
+        assert torch.isfinite(x).all() and torch.equal(x, y)
+    ref, _ = O.forward_dense(p["A"], p["Wa"], -0.1, 0.3, p["Wo"], p["r0"], 0.15, "gelu")
+    assert O.max_rel_err(outs[0][0].cpu().numpy(), ref) <= TRAJ_TOL
+
+
 @pytest.mark.parametrize("driven", [(3, 9), (5,), ()], ids=["two", "one", "none"])
 def test_silent_action_channels_are_compacted(driven, gpu_device, monkeypatch):
     """With a_dim > 2 and the caller's statement that at most two named channels are driven, the Python operator runs
