@@ -229,6 +229,11 @@ RINGATTR_API int ringattr_generate_inputs(unsigned long long seed, int N, int a_
  * [B,T,a_dim].  grad_params comes packed, [a_dim, 3 hidden + 1]; the workspace is ringattr_gain_workspace_bytes large. */
 RINGATTR_API int ringattr_gain_nets_fwd(const void* signal, int halves, const void* const* nets, void* action_signal, int a_dim,
                       int hidden, int seq_len, int batch_size, void* stream);
+/* The same leaving in kept (or NULL) what a backward needs, should the parameters or the velocity be written to before it:
+ * [a_dim, 3 hidden + 1] as the packed parameters are, behind them, for halves, the velocity [B,T].  ringattr_gain_nets_bwd then
+ * gets pointers into it. */
+RINGATTR_API int ringattr_gain_nets_fwd_kept(const void* signal, int halves, const void* const* nets, void* action_signal, void* kept,
+                      int a_dim, int hidden, int seq_len, int batch_size, void* stream);
 RINGATTR_API int ringattr_gain_nets_bwd(const void* signal, int halves, const void* const* nets, const void* grad_action_signal,
                       void* grad_params, int a_dim, int hidden, int seq_len, int batch_size, void* workspace,
                       size_t workspace_bytes, void* stream);

@@ -59,6 +59,8 @@ PROTOTYPES = {
                                          ctypes.POINTER(c_float), c_int, c_float, c_int, c_int, c_float,
                                          c_void_p, c_void_p, c_void_p, c_void_p, c_void_p]),
     "ringattr_gain_nets_fwd": (c_int, [c_void_p, c_int, ctypes.POINTER(c_void_p), c_void_p, c_int, c_int, c_int, c_int, c_void_p]),
+    "ringattr_gain_nets_fwd_kept": (c_int, [c_void_p, c_int, ctypes.POINTER(c_void_p), c_void_p, c_void_p, c_int, c_int, c_int, c_int,
+                                            c_void_p]),
     "ringattr_gain_nets_bwd": (c_int, [c_void_p, c_int, ctypes.POINTER(c_void_p), c_void_p, c_void_p, c_int, c_int, c_int, c_int,
                                        c_void_p, c_size_t, c_void_p]),
     "ringattr_action_signal": (c_int, [c_void_p, c_void_p, c_int, c_int, c_int, c_void_p]),

@@ -13,6 +13,7 @@
 // Parameters are packed per channel as [w1[0..h) | b1[0..h) | w2[0..h) | b2]; gradients use the same packing.  They may
 // also be given as the networks' own tensors, and the signal as the angular velocity whose two halves (relu(-av), relu(av))
 // are the channels: at N = 120, B = 128, T = 120 packing, splitting and their way back were sixteen of a training pass's launches.
+// The forward leaves a copy of both for the backward, which may come after they have been written to.
 #include "ring_common.hpp"
 #include "ring_kernels.hpp"
 
@@ -61,10 +62,18 @@ __global__ __launch_bounds__(GAIN_THREADS) void ring_gain_fwd_kernel(const float
     prm[i] = v;
   }
   __syncthreads();
+  const int per = 3 * h + 1;
+  float* const kept_signal = params.kept && params.halves ? params.kept + (size_t)k * per : nullptr;
+  if (params.kept && blockIdx.x == 0)
+    for (int i = threadIdx.x; i < k * per; i += GAIN_THREADS) {
+      const int c = i / per, o = i % per;
+      params.kept[i] = prm[c * PS + (o == 3 * h ? 3 * H : o / h * H + o % h)];
+    }
   for (long idx = (long)blockIdx.x * GAIN_THREADS + threadIdx.x; idx < total; idx += (long)gridDim.x * GAIN_THREADS) {
     const int c = (int)(idx % k);
     const float* pc = prm + c * PS;
     const float xv = gain_input(params, x, idx / k, k, c), m = fabsf(xv);
+    if (kept_signal && c == 0) kept_signal[idx / k] = x[idx / k];
     float z = pc[3 * H];
 #pragma unroll
     for (int j = 0; j < H; ++j) {

@@ -155,6 +155,7 @@ struct RingGainParams {
   const float* packed;                          // [k][3h+1], or null:
   const float* part[4 * RING_GAIN_NETS];        // w1 [h], b1 [h], w2 [h], b2 [1] of every channel
   int halves;                                   // non-zero: the signal is an angular velocity, channels relu(-av) and relu(av)
+  float* kept;                                  // forward: null, or where the packed parameters go, behind them the signal if halves
 };
 hipError_t ring_launch_gain_fwd(const float* x, const RingGainParams& params, float* out, int k, int h, long samples, hipStream_t st);
 hipError_t ring_launch_gain_bwd(const float* x, const RingGainParams& params, const float* grad_A, float* grad_params, float* grad_x,

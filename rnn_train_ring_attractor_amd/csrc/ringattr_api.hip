@@ -715,10 +715,16 @@ static bool gain_nets(const char* who, const void* const* nets, int halves, int 
 
 int ringattr_gain_nets_fwd(const void* signal, int halves, const void* const* nets, void* action_signal, int a_dim, int hidden,
                            int seq_len, int batch_size, void* stream) {
+  return ringattr_gain_nets_fwd_kept(signal, halves, nets, action_signal, nullptr, a_dim, hidden, seq_len, batch_size, stream);
+}
+
+int ringattr_gain_nets_fwd_kept(const void* signal, int halves, const void* const* nets, void* action_signal, void* kept, int a_dim,
+                                int hidden, int seq_len, int batch_size, void* stream) {
   if (ringattr_gain_workspace_bytes(a_dim, hidden, seq_len, batch_size) == 0) return RINGATTR_ERR_INVALID;
   if (!signal || !action_signal) return fail(RINGATTR_ERR_INVALID, "ringattr_gain_nets_fwd: null tensor pointer");
   RingGainParams prm;
   if (!gain_nets("ringattr_gain_nets_fwd", nets, halves, a_dim, prm)) return RINGATTR_ERR_INVALID;
+  prm.kept = (float*)kept;
   hipError_t e = ring_launch_gain_fwd((const float*)signal, prm, (float*)action_signal, a_dim, hidden, (long)seq_len * batch_size,
                                       static_cast<hipStream_t>(stream));
   if (e != hipSuccess) return hip_fail(e, "gain network forward launch");

@@ -83,42 +83,51 @@ def ring_gain_func(base_signal, params):
 
 class RingGainNetsFunc(Function):
     """The same operator with the modules' own parameter tensors (four per channel) as inputs, for a signal that needs no
-    gradient; halves: the signal is an angular velocity [B,T] and the channels are relu(-av) and relu(av)."""
+    gradient; halves: the signal is an angular velocity [B,T] and the channels are relu(-av) and relu(av).  The forward kernel
+    leaves a copy of the parameters, and of an angular velocity, for the backward: either may be written to in between, as
+    where `pack_gain_nets` and the two halves make new tensors."""
 
     @staticmethod
     def forward(ctx, signal, halves, *params):
         B, T = signal.shape[:2]
         k, h = len(params) // 4, params[0].numel()
-        ctx.save_for_backward(signal, *params)
         ctx.dims = (B, T, k, h, halves)
         out = torch.empty(B, T, k, dtype=signal.dtype, device=signal.device)
+        kept = None
+        if any(ctx.needs_input_grad):
+            kept = torch.empty(k * (3 * h + 1) + (B * T if halves else 0), dtype=signal.dtype, device=signal.device)
+            ctx.save_for_backward(kept, None if halves else signal)
         with torch.cuda.device(signal.device):
-            _lib.check(_lib.load().ringattr_gain_nets_fwd(signal.data_ptr(), int(halves), _pointers(params), out.data_ptr(), k, h, T, B,
-                                                          torch.cuda.current_stream(signal.device).cuda_stream))
+            _lib.check(_lib.load().ringattr_gain_nets_fwd_kept(signal.data_ptr(), int(halves), _pointers([p.data_ptr() for p in params]),
+                                                               out.data_ptr(), kept.data_ptr() if kept is not None else None, k, h, T, B,
+                                                               torch.cuda.current_stream(signal.device).cuda_stream))
         return out
 
     @staticmethod
     def backward(ctx, grad_out):
-        signal, *params = ctx.saved_tensors
+        kept, signal = ctx.saved_tensors
         B, T, k, h, halves = ctx.dims
         lib = _lib.load()
         g = grad_out.contiguous()
-        grad = torch.empty(k, 3 * h + 1, dtype=signal.dtype, device=signal.device)
-        with torch.cuda.device(signal.device):
+        grad = torch.empty(k, 3 * h + 1, dtype=kept.dtype, device=kept.device)
+        at = kept.data_ptr()
+        nets = _pointers([at + 4 * (c * (3 * h + 1) + part * h) for c in range(k) for part in range(4)])
+        x = at + 4 * k * (3 * h + 1) if halves else signal.data_ptr()
+        with torch.cuda.device(kept.device):
             nbytes = lib.ringattr_gain_workspace_bytes(k, h, T, B)
             if nbytes == 0:
                 _lib.check(1)
-            ws = torch.empty(nbytes, dtype=torch.uint8, device=signal.device)
-            _lib.check(lib.ringattr_gain_nets_bwd(signal.data_ptr(), int(halves), _pointers(params), g.data_ptr(), grad.data_ptr(), k, h,
-                                                  T, B, ws.data_ptr(), nbytes, torch.cuda.current_stream(signal.device).cuda_stream))
+            ws = torch.empty(nbytes, dtype=torch.uint8, device=kept.device)
+            _lib.check(lib.ringattr_gain_nets_bwd(x, int(halves), nets, g.data_ptr(), grad.data_ptr(), k, h, T, B, ws.data_ptr(), nbytes,
+                                                  torch.cuda.current_stream(kept.device).cuda_stream))
         parts = list(grad.view(-1).split((h, h, h, 1) * k))
         for c in range(0, 4 * k, 4):
             parts[c], parts[c + 2] = parts[c].view(h, 1), parts[c + 2].view(1, h)
         return (None, None, *parts)
 
 
-def _pointers(tensors):
-    return (ctypes.c_void_p * len(tensors))(*[t.data_ptr() for t in tensors])
+def _pointers(addresses):
+    return (ctypes.c_void_p * len(addresses))(*addresses)
 
 
 def _net_parameters(nets, signal):

@@ -90,3 +90,38 @@ def test_networks_read_in_place_equal_the_packed_operator(B, T, h, k, gpu_device
         base = torch.stack([torch.relu(-av), torch.relu(av)], dim=2)
         for a, b in zip(grads(gain.ring_gain_halves(av, nets), g), grads(gain.ring_gain_func(base, gain.pack_gain_nets(nets)), g)):
             assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("write", ["in_place", "data", "adam"])
+def test_networks_and_velocity_may_be_written_to_before_the_backward(write, gpu_device):
+    """Gradients are those of the values the forward saw, as with the packed operator, which works on new tensors."""
+    from rnn_train_ring_attractor_amd import FusedClipAdam, gain
+    B, T, h = 33, 21, 5
+    print(f"[case] gain networks written to before the backward: {write}", flush=True)
+    g = torch.randn(B, T, 2, device=gpu_device)
+    av0 = torch.randn(B, T, device=gpu_device)
+    grads = []
+    for fused in (True, False):
+        torch.manual_seed(4)
+        nets = [torch.nn.Sequential(torch.nn.Linear(1, h), torch.nn.GELU(), torch.nn.Linear(h, 1), torch.nn.Softplus()).to(gpu_device)
+                for _ in range(2)]
+        params = [p for net in nets for p in net.parameters()]
+        av = av0.clone()
+        base = lambda: torch.stack([torch.relu(-av), torch.relu(av)], dim=2)
+        x = base()
+        outs = [gain.ring_gain_halves(av, nets), gain.ring_gain_nets(x, nets)] if fused else \
+               [gain.ring_gain_func(base(), gain.pack_gain_nets(nets)), gain.ring_gain_func(x, gain.pack_gain_nets(nets))]
+        if write == "adam":
+            for p in params:
+                p.grad = torch.ones_like(p)
+            FusedClipAdam(params, lr=0.5, max_norm=0.0).step()
+        with torch.no_grad():
+            for p in params:
+                if write == "in_place":
+                    p.add_(1.0)
+                elif write == "data":
+                    p.data.mul_(-2.0)
+            (av if write == "in_place" else av.data).fill_(0.3)
+        grads.append([t for out in outs for t in torch.autograd.grad(out, params, g)])
+    for a, b in zip(*grads):
+        assert torch.equal(a, b)
