@@ -39,8 +39,8 @@ def generate_inputs(seed, batch_size, seq_len, num_neurons, action_dim=2, zero_p
             0 if zero_padding else 1, kind, float(bump_param), av.data_ptr(), angle.data_ptr(), action.data_ptr(),
             r0.data_ptr(), torch.cuda.current_stream(dev).cuda_stream))
     if zero_padding and k > 2:
-        from .ring_rnn_cuda import state_driven_channels
-        state_driven_channels(action, (0, 1))      # by construction channels 2.. are identically zero
+        from .ring_rnn_cuda import DRIVEN_ATTR
+        setattr(action, DRIVEN_ATTR, (0, 1))      # by construction channels 2.. are identically zero
     return av, angle, action, r0
 
 

@@ -77,49 +77,36 @@ def _split_wo(action_signal, Wa, J1, Wo):
 
 
 DRIVEN_ATTR = "_ring_driven_channels"     # set on zero-padded action signals by the host helper that builds them
-DRIVEN_VERSION_ATTR = "_ring_driven_version"   # the tensor's version counter at that time
-
-
-def state_driven_channels(action_signal, channels):
-    """Leaves on a tensor the statement that every channel outside `channels` is identically zero."""
-    setattr(action_signal, DRIVEN_ATTR, channels)
-    if not action_signal.is_inference():
-        setattr(action_signal, DRIVEN_VERSION_ATTR, action_signal._version)
 
 
 def _driven_pair(action_signal, Wa, driven_channels=None):
     """The training script pads the two driven action channels with zeros up to a_dim = 16
     (train_general_ring_no_gain.py:52-66 of the reference).  A channel that is zero for every sample and step
     contributes nothing forward and has an exactly zero weight gradient, so when the caller states which (at most
-    two) channels are driven, the operator runs on those two (`_compact`); silent channels get exactly zero gradients.
-    Returns their indices, or None for the operator on all channels.
+    two) channels are driven and N fits the weight-resident kernels (128 < N <= 256), the operator runs on those two
+    (`_compact`); silent channels get exactly zero gradients.  Returns their indices, or None for the operator on all channels.
 
     Nothing here reads the device back: which channels are driven comes from the caller (`driven_channels=`, or the
     attribute the host helper leaves on the tensors it pads), so the call stays asynchronous and capturable.  The
     statement is checked on the device: if a channel declared silent is not, the compacted action signal is
     poisoned with NaN, which the kernels carry into every output instead of returning a plausible wrong result.
-    A statement in the call is acted on where the ring fits the weight-resident kernels (128 < N <= 256).  One that the
-    tensor carries is acted on at every width, as long as nothing has written to the tensor since it was made (nor can,
-    unseen, as in a graph that is replayed): fewer
-    matrices cost less everywhere (us per pass with 16 channels and with the two: N = 800, B = 100, T = 120, forward and
-    backward 8116 and 700; N = 512, B = 512, T = 120 2146 and 615; forward alone N = 120, B = 64, T = 100 178 and 94,
-    N = 2048, B = 64, T = 20 385 and 298).
+    At other widths fewer matrices cost less too (us per pass with 16 channels and with the two: N = 800, B = 100, T = 120,
+    forward and backward 8116 and 700; N = 512, B = 512, T = 120 2146 and 615), but a padded tensor that has been written to
+    since must give its own results there, and its version counter does not see every write (`.data`, DLPack, a kernel
+    that has its address).
     Without a statement the operator runs on all channels (the general kernels skip all-zero channels step by step).
     RINGATTR_COMPACT_CHANNELS=0 switches the compaction off."""
     import os
     if os.environ.get("RINGATTR_COMPACT_CHANNELS", "1") == "0":
         return None
-    untouched = False
     if driven_channels is None:
         driven_channels = getattr(action_signal, DRIVEN_ATTR, None)
-        if driven_channels is None:
-            return None
-        untouched = not action_signal.is_inference() and getattr(action_signal, DRIVEN_VERSION_ATTR, None) == action_signal._version \
-            and not (action_signal.is_cuda and torch.cuda.is_current_stream_capturing())    # (a graph's input may be written to later)
+    if driven_channels is None:
+        return None
     if action_signal.dim() != 3 or Wa.dim() != 3 or not action_signal.is_cuda:
         return None
     k, N = action_signal.shape[2], Wa.shape[1]
-    if k <= 2 or not (untouched or 128 < N <= 256) or Wa.shape[0] != k:
+    if k <= 2 or not (128 < N <= 256) or Wa.shape[0] != k:
         return None
     if action_signal.requires_grad:        # dL/dA of a silent channel is not zero: keep every channel
         return None
@@ -128,7 +115,7 @@ def _driven_pair(action_signal, Wa, driven_channels=None):
         raise ValueError(f"driven_channels must name at most two channels in [0, {k}), got {list(driven_channels)}")
     # (what the operator refuses, it refuses in the call on all channels)
     if action_signal.dtype != torch.float32 or Wa.dtype != torch.float32 or Wa.device != action_signal.device \
-            or Wa.shape[2] != N or action_signal.numel() == 0 or not 0 < N <= 2048:
+            or Wa.shape[2] != N or action_signal.numel() == 0:
         return None
     for c in range(k):                     # fewer than two driven: fill up with silent ones (their gates are zero)
         if len(driven) == 2:

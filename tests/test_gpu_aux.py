@@ -160,8 +160,9 @@ def test_compacted_channels_are_the_named_ones_and_the_rest_is_checked(B, T, k, 
 
 
 @pytest.mark.parametrize("N,k", [(60, 16), (300, 5), (600, 6)])
-def test_a_padded_signal_runs_on_its_driven_channels_at_every_width(N, k, gpu_device):
-    """The helper's statement is acted on outside the weight-resident widths too, unless the tensor has been written to."""
+def test_a_padded_signal_that_was_written_to_gives_its_own_results(N, k, gpu_device):
+    """Outside the weight-resident widths the helper's statement decides nothing: a silent channel that has been written to
+    counts, also where the tensor's version counter has not seen the write."""
     from rnn_train_ring_attractor_amd import host, ring_rnn_cuda_func
     from rnn_train_ring_attractor_amd.ring_rnn_cuda import _driven_pair
     B, T = 20, 6
@@ -175,14 +176,15 @@ def test_a_padded_signal_runs_on_its_driven_channels_at_every_width(N, k, gpu_de
         h = ring_rnn_cuda_func(signal, Wa, -0.05, 0.5, Wo, r0, 0.15, "tanh")
         h.backward(G)
         outs.append((h.detach(), Wa.grad, Wo.grad))
-    assert _driven_pair(A, Wa) == (0, 1) and _driven_pair(A.clone(), Wa) is None
+    assert _driven_pair(A, Wa) is None and _driven_pair(A.clone(), Wa) is None
     assert torch.count_nonzero(outs[0][1][2:]) == 0
-    for x, y in zip(*outs):                             # two kernel families: other row-sum roundings
-        assert float((x - y).abs().max()) <= 5e-3 * float(y.abs().max())
-    A[0, 0, 2] = 0.1
-    assert _driven_pair(A, Wa) is None
-    want = ring_rnn_cuda_func(A.clone(), Wa, -0.05, 0.5, Wo, r0, 0.15, "tanh")
-    assert torch.equal(ring_rnn_cuda_func(A, Wa, -0.05, 0.5, Wo, r0, 0.15, "tanh"), want)
+    for x, y in zip(*outs):
+        assert torch.equal(x, y)
+    A.data[0, 0, 2] = 0.1
+    for _ in range(2):
+        want = ring_rnn_cuda_func(A.clone(), Wa, -0.05, 0.5, Wo, r0, 0.15, "tanh")
+        assert torch.isfinite(want).all() and torch.equal(ring_rnn_cuda_func(A, Wa, -0.05, 0.5, Wo, r0, 0.15, "tanh"), want)
+        A[0, 0, 2] = 0.2
 
 
 @pytest.mark.parametrize("B,T,k", [(1, 1, 2), (5, 7, 3), (33, 20, 16), (700, 513, 5)])
