@@ -162,6 +162,14 @@ def plain_gpu_tensor(t) -> bool:
         return False
     if (t.requires_grad and torch.is_grad_enabled()) or torch.compiler.is_compiling() or torch.jit.is_tracing():
         return False
-    if torch._C._functorch.maybe_current_level() is not None or torch.autograd.forward_ad._current_level >= 0:
-        return False
-    return torch._C._len_torch_dispatch_stack() == 0 and torch._C._len_torch_function_stack() == 0 and not t.is_neg() and t.numel() > 0
+    return not _watched() and not t.is_neg() and t.numel() > 0
+
+
+def _watched() -> bool:
+    """functorch, forward mode, a dispatch or function mode.  These are torch's private names: where a version has them no
+    longer, the helpers keep to the tensor operations."""
+    try:
+        return (torch._C._functorch.maybe_current_level() is not None or torch.autograd.forward_ad._current_level >= 0
+                or torch._C._len_torch_dispatch_stack() != 0 or torch._C._len_torch_function_stack() != 0)
+    except AttributeError:
+        return True

@@ -220,3 +220,17 @@ def test_helpers_keep_to_tensor_operations_where_something_watches_them(gpu_devi
     assert float(tangent.abs().max()) > 0
     traced = torch.jit.trace(lambda a: host.av_to_action_signal(a), av[0])
     assert torch.equal(traced(av[1]), host.av_to_action_signal(av[1]))
+
+
+@pytest.mark.parametrize("owner,name", [("torch._C._functorch", "maybe_current_level"), ("torch.autograd.forward_ad", "_current_level"),
+                                        ("torch._C", "_len_torch_dispatch_stack"), ("torch._C", "_len_torch_function_stack")])
+def test_helpers_keep_to_tensor_operations_where_torch_lacks_a_private_name(owner, name, gpu_device, monkeypatch):
+    import operator
+    from rnn_train_ring_attractor_amd import _lib, host
+    av, angle = torch.randn(4, 5, device=gpu_device), torch.rand(4, device=gpu_device)
+    want = host.av_to_action_signal(av), host.av_to_action_signal_ND(av, 5), host.create_initial_bump(angle, 32, device=gpu_device)
+    assert _lib.plain_gpu_tensor(av)
+    monkeypatch.delattr(operator.attrgetter(owner.partition(".")[2])(torch), name)
+    assert not _lib.plain_gpu_tensor(av)
+    got = host.av_to_action_signal(av), host.av_to_action_signal_ND(av, 5), host.create_initial_bump(angle, 32, device=gpu_device)
+    assert all(torch.equal(a, b) for a, b in zip(got, want))
