@@ -179,9 +179,12 @@ size_t ringattr_fwd_workspace_bytes(int N, int a_dim, int seq_len, int batch_siz
   const size_t packed = g.wpack_bytes + (ring_cluster_applicable(N, a_dim) ? ring_cluster_workspace_bytes(g.nbt) : 0) +
                         (ring_panel_applicable(g.NC, a_dim) ? align_up(ring_panel_workspace_bytes(g.NC, g.nbt)) : 0);
   // (used instead of the packed weights)
-  const size_t team = ring_team_fwd_bytes(N, a_dim, seq_len, batch_size), rows = ring_team_rows_bytes(N, a_dim, batch_size, true);
-  const size_t most = team > rows ? team : rows;
-  return packed > most ? packed : most;
+  // (with a record and without one: narrower rings have teams for more rows without one)
+  size_t most = packed;
+  for (const size_t other : {ring_team_fwd_bytes(N, a_dim, seq_len, batch_size), ring_team_rows_bytes(N, a_dim, batch_size, true),
+                             ring_team_rows_bytes(N, a_dim, batch_size, false)})
+    most = other > most ? other : most;
+  return most;
 }
 
 // A backward's workspace.  Most families: packed weights, operand copy of g, split-K partials, the small areas, and

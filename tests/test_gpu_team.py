@@ -144,6 +144,22 @@ def test_small_batches_without_a_record_have_the_weight_resident_forwards_bits(N
             assert torch.equal(got, want), wait_us
 
 
+# rings with teams for more than 512 rows as long as no record is wanted: the most of each number of members, and one more
+@pytest.mark.parametrize("N,B,kernel", [(129, 513, "ring_team_rows"), (160, 768, "ring_team_rows"), (160, 769, "ring_fwd_res256"),
+                                        (192, 640, "ring_team_rows"), (192, 641, "ring_fwd_res256"), (193, 513, "ring_fwd_res256")])
+def test_forwards_without_a_record_take_teams_as_far_as_they_go(N, B, kernel, gpu_device, monkeypatch):
+    from rnn_train_ring_attractor_amd import ring_rnn_cuda_func, _lib
+    monkeypatch.delenv("RINGATTR_TEAM", raising=False)
+    print(f"[case] team rows as far as they go N={N} B={B}", flush=True)
+    p = make_problem(86, B, 3, 2, N, action="dense")
+    args = [_t(p["A"], gpu_device), _t(p["Wa"], gpu_device), -0.05, 0.7, _t(p["Wo"], gpu_device), _t(p["r0"], gpu_device), 0.15, "gelu"]
+    with torch.no_grad():
+        got = ring_rnn_cuda_func(*args)
+        assert kernel in _lib.last_kernel_names()["fwd"]
+        monkeypatch.setenv("RINGATTR_TEAM", "0")
+        assert torch.equal(got, ring_rnn_cuda_func(*args))
+
+
 # the kernels of 128 < N <= 256 with two channels, whole and ragged widths; teams with members of different width per batch
 @pytest.mark.parametrize("N,k,B,kernel", [(256, 2, 4096, "res256"), (200, 2, 1500, "res256"), (120, 2, 4096, "team"),
                                           (360, 2, 2048, "team"), (333, 3, 1000, "team"), (700, 2, 1024, "team")])
