@@ -166,7 +166,8 @@ __device__ __forceinline__ float panel_row_sum(const float* fours, int N, int su
   return row16_sum_dpp(s);
 }
 
-// What travels between the steps, two of each but the row sums (three: the step before the last one's is emptied).
+// What travels between the steps, two of each but the row sums (three: the step before the last one's is emptied).  Only the
+// first operand and row sums where they come from a launch of their own.
 struct PanelState {
   bf16x8* x[2];         // operand fragments [batch tile][K chunk][lane]
   float* fours[2];      // [row][NPAD / 4]
@@ -184,7 +185,8 @@ __device__ __forceinline__ void panel_put(bf16x8* x, int KCH, int b, int j, cons
 }  // namespace
 
 // Operand fragments [batch tile][K chunk][lane][8] and fp32 row sums of the initial state's rows; four rows per wave.  The
-// sums run in the order of ring_block.hip's stage_tiles.  (Both fragment buffers: the steps write no padding.)
+// sums run in the order of ring_block.hip's stage_tiles.  (Both fragment buffers, if there are two: the steps write no
+// padding.)
 __global__ __launch_bounds__(64) void ring_panel_operand_kernel(const float* __restrict__ prev, PanelState ps, int N, int B, int NPAD) {
   const int lane = threadIdx.x, row = 4 * (blockIdx.x & 3) + (lane >> 4), sub = lane & 15, bt = blockIdx.x >> 2;
   const int b = 16 * bt + row;
@@ -192,7 +194,7 @@ __global__ __launch_bounds__(64) void ring_panel_operand_kernel(const float* __r
   auto put = [&](int j, f32x4 v) {
     sum += (v[0] + v[1]) + (v[2] + v[3]);
     panel_put(ps.x[0], NPAD >> 5, b, j, v);
-    panel_put(ps.x[1], NPAD >> 5, b, j, v);
+    if (ps.x[1]) panel_put(ps.x[1], NPAD >> 5, b, j, v);
   };
   // Sixteen loads in flight: one at a time this launch is all latency, 12.7 against 5 us.  Addresses are clamped into the
   // row; where N is no multiple of four, values that reach past its end are read as the row's last four and moved into
@@ -232,12 +234,13 @@ __global__ __launch_bounds__(64) void ring_panel_operand_kernel(const float* __r
   sum = row16_sum_dpp(sum);
   if (sub == 0) {
     ps.rs[0][b] = sum;
-    ps.rs[1][b] = __builtin_bit_cast(float, PANEL_EMPTY);
+    if (ps.rs[1]) ps.rs[1][b] = __builtin_bit_cast(float, PANEL_EMPTY);
   }
 }
 
 // One step for R row tiles x C column tiles (16 consecutive neurons each).  Wpack: order 3 of ring_pack_weights_kernel.
-template <int ACT, int R>
+// CARRY: with the next step's operand and the sums of its fours.
+template <int ACT, int R, bool CARRY>
 __global__ __launch_bounds__(256) void ring_panel_fwd_kernel(RingFwdArgs p, PanelState state, int NC, int C, int t, int xcd_map) {
   extern __shared__ __attribute__((aligned(16))) char panel_lds[];
   __shared__ int list[BN_GATE_KMAX + 1];
@@ -250,15 +253,15 @@ __global__ __launch_bounds__(256) void ring_panel_fwd_kernel(RingFwdArgs p, Pane
   int rg, cb;
   step_block_coords(xcd_map, rg, cb);
   const int bt0 = rg * R;
-  const bf16x8* const xfrag = state.x[t & 1];
+  const bf16x8* const xfrag = state.x[CARRY ? t & 1 : 0];
   // this workgroup's share of the row sums (there are at least as many column blocks as row tiles: a row per 16 lanes at
   // most), announced to the others of its rows
   const int sum_row = cb + (int)gridDim.y * (tid >> 4), sum_b = 16 * bt0 + sum_row;
-  const bool sums_row = sum_row < 16 * R && sum_b < B;
+  const bool sums_row = CARRY && sum_row < 16 * R && sum_b < B;
   // (the widest panels, whose steps are long, have its loads in flight over the gates' at the price of a longer program:
   // N = 2048, 16 channels, B = 256: 57.7 -> 56.2 us per step, but 2 channels, B = 1: 7.6 -> 8.4)
   constexpr bool EARLY = R == 8;
-  const float* const own_fours = state.fours[t & 1] + (size_t)sum_b * (16 * NC);
+  const float* const own_fours = CARRY ? state.fours[t & 1] + (size_t)sum_b * (16 * NC) : nullptr;
   float own_sum = 0.f;
   PanelRowSum<EARLY ? 32 : 1> own;                          // (N <= 2048)
   if (sums_row && t > 0) {
@@ -341,16 +344,18 @@ __global__ __launch_bounds__(256) void ring_panel_fwd_kernel(RingFwdArgs p, Pane
 
   // (step and thread as the compiler does not know them from above: what follows from them is not kept over the products)
   int now = t, me = tid;
-  asm volatile("" : "+s"(now), "+v"(me));
-  for (int row = me >> 4; row < 16 * R; row += 16) {
-    const int b = 16 * bt0 + row, sub = me & 15;
-    if (b >= B) break;
-    float s = __hip_atomic_load(state.rs[now % 3] + b, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    if (__builtin_bit_cast(unsigned, s) == PANEL_EMPTY)                        // (the same in the row's 16 lanes)
-      s = panel_row_sum(state.fours[now & 1] + (size_t)b * (16 * NC), N, sub);
-    if (sub == 0) row_sums[row] = s;
+  if constexpr (CARRY) {
+    asm volatile("" : "+s"(now), "+v"(me));
+    for (int row = me >> 4; row < 16 * R; row += 16) {
+      const int b = 16 * bt0 + row, sub = me & 15;
+      if (b >= B) break;
+      float s = __hip_atomic_load(state.rs[now % 3] + b, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      if (__builtin_bit_cast(unsigned, s) == PANEL_EMPTY)                      // (the same in the row's 16 lanes)
+        s = panel_row_sum(state.fours[now & 1] + (size_t)b * (16 * NC), N, sub);
+      if (sub == 0) row_sums[row] = s;
+    }
+    lds_barrier();
   }
-  lds_barrier();
 
   // activation and leak; a thread takes four consecutive neurons of a row
   const float* prev = (now == 0) ? p.r_init : p.hist + (size_t)(now - 1) * B * N;
@@ -362,7 +367,7 @@ __global__ __launch_bounds__(256) void ring_panel_fwd_kernel(RingFwdArgs p, Pane
     const int b = 16 * bt0 + row, j = 16 * C * cb + j4, i = row >> 4;
     if (b >= B || j >= N) continue;
     const f32x4 rp = load4_masked(prev, N, B, b, j);
-    const float js = p.J0 * row_sums[row];
+    const float js = p.J0 * (CARRY ? row_sums[row] : state.rs[0][b]);
     f32x4 rn;
 #pragma unroll
     for (int x = 0; x < 4; ++x) {
@@ -372,7 +377,7 @@ __global__ __launch_bounds__(256) void ring_panel_fwd_kernel(RingFwdArgs p, Pane
       rn[x] = fmaf(p.alpha, F, oma * rp[x]);
     }
     store4_masked(out, N, B, b, j, rn);
-    if (now + 1 < T) {
+    if (CARRY && now + 1 < T) {
 #pragma unroll
       for (int x = 1; x < 4; ++x) rn[x] = j + x < N ? rn[x] : 0.f;
       panel_put(state.x[(now + 1) & 1], KCH, b, j, rn);
@@ -431,26 +436,39 @@ bool ring_uses_panel(int k, int NC, int nbt) {
   return panel_operand_bytes(NC, nbt) < ((size_t)1 << 30);   // (32-bit offsets; the weights are 0.6 GB at most)
 }
 
-template <int ACT, int R>
-static hipError_t panel_run(const RingFwdArgs& a, int NC, int C, hipStream_t st) {
+template <int ACT, int R, bool CARRY>
+static hipError_t panel_steps(const RingFwdArgs& a, int NC, int C, hipStream_t st) {
   const size_t dyn = panel_lds_bytes(R, C, a.k);
-  hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&ring_panel_fwd_kernel<ACT, R>),
+  hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&ring_panel_fwd_kernel<ACT, R, CARRY>),
                                      hipFuncAttributeMaxDynamicSharedMemorySize, (int)dyn);
   if (e != hipSuccess) return e;
-  PanelState ps;
+  PanelState ps = {};
   char* ws = reinterpret_cast<char*>(a.panel_ws);
   for (int i = 0; i < 2; ++i, ws += panel_operand_bytes(NC, a.nbt)) ps.x[i] = reinterpret_cast<bf16x8*>(ws);
   for (int i = 0; i < 2; ++i, ws += (size_t)a.nbt * 16 * 16 * NC * sizeof(float)) ps.fours[i] = reinterpret_cast<float*>(ws);
   for (int i = 0; i < 3; ++i, ws += (size_t)a.nbt * 16 * sizeof(float)) ps.rs[i] = reinterpret_cast<float*>(ws);
+  if (!CARRY) ps.x[1] = nullptr, ps.rs[1] = nullptr;
   const dim3 grid((a.nbt + R - 1) / R, 4 * NC / C);
   const int xm = step_xcd_map();
-  RING_LAUNCH(ring_panel_operand_kernel, dim3(4 * a.nbt), dim3(64), 0, st, a.r_init, ps, a.N, a.B, 64 * NC);
   for (int t = 0; t < a.T; ++t) {
-    RING_LAUNCH((ring_panel_fwd_kernel<ACT, R>), grid, dim3(256), dyn, st, a, ps, NC, C, t, xm);
+    if (t == 0 || !CARRY)
+      RING_LAUNCH(ring_panel_operand_kernel, dim3(4 * a.nbt), dim3(64), 0, st, t == 0 ? a.r_init : a.hist + (size_t)(t - 1) * a.B * a.N, ps,
+                  a.N, a.B, 64 * NC);
+    RING_LAUNCH((ring_panel_fwd_kernel<ACT, R, CARRY>), grid, dim3(256), dyn, st, a, ps, NC, C, t, xm);
     e = hipGetLastError();
     if (e != hipSuccess) return e;
   }
   return hipSuccess;
+}
+
+// Where workgroups queue, a step's first ones find no announced sums (who would announce them has not begun) and add up all of
+// their rows: with more than one a compute unit, operand and sums are a launch's.  us per step, carried and with the launch,
+// N = 1100, 16 channels: B = 1000 146 and 133, B = 3000 444 and 385; N = 2048, one channel, B = 3000 126 and 110; with one a
+// compute unit, N = 2048, B = 1000: one channel 39 and 41, 16 channels 191 and 193.
+template <int ACT, int R>
+static hipError_t panel_run(const RingFwdArgs& a, int NC, int C, hipStream_t st) {
+  const bool queue = (long)((a.nbt + R - 1) / R) * (4 * NC / C) > 256;
+  return queue ? panel_steps<ACT, R, false>(a, NC, C, st) : panel_steps<ACT, R, true>(a, NC, C, st);
 }
 
 template <int ACT>
