@@ -223,7 +223,16 @@ __global__ __launch_bounds__(256) void ring_dw_direct_kernel(RingDwArgs p, int m
   }
 }
 
-bool ring_dw_tiled_applicable(int NC) { return NC == 2 || NC == 4 || NC == 8 || NC == 16 || NC == 24 || NC == 32; }
+// N <= 128: a launch per three matrices, of a few workgroups where there is little to contract, against one launch for all
+// matrices of the kernel with a wave per 32 x 128 block (us of a training pass there and here, N = 120, T = 20, B = 1, 10 chunks:
+// a_dim 3 59.5 and 62.6, 7 89 and 100, 16 135 and 168; 40 chunks: a_dim 7 101.5 and 104.6, 16 154 and 174; 60 chunks: a_dim 7 392
+// and 379; 240 chunks: a_dim 12 566 and 573, 480 345 and 338; N = 96, a_dim 24, 480 chunks 1539 and 1560, 960 3023 and 3010).  Up
+// to two channels there is one launch here too.
+bool ring_dw_tiled_applicable(int NC, int k, long nchunk) {
+  const int launches = (k + 3) / 3;
+  if (NC == 2) return launches == 1 || nchunk > (launches <= 4 ? 48 : launches <= 6 ? 256 : 512);
+  return NC == 4 || NC == 8 || NC == 16 || NC == 24 || NC == 32;
+}
 
 // K splits: one workgroup per CU, a multiple of 8 when possible (XCD grouping).  One launch per
 // group of three matrices, so the grid of a launch does not depend on a_dim.

@@ -1418,16 +1418,17 @@ hipError_t ring_launch_bptt(const RingBpttArgs& a, int NCv, hipStream_t st) {
 
 hipError_t ring_launch_dw(const RingDwArgs& a, int NCv, hipStream_t st) {
   const int NT = 4 * NCv;
-  const long waves = (long)(NT / 2) * (NT / 4) * ((a.k + 3) / 3) * a.nz;
+  const long waves = (long)(NT / 2) * ((a.k + 3) / 3) * a.nz;
   const int blocks = (int)((waves + 3) / 4);
   hipError_t e;
   {
   ProfScope prof(4, st);
-  if (ring_dw_tiled_applicable(NCv)) {
+  if (ring_dw_tiled_applicable(NCv, a.k, (long)a.nbt * ((a.T + 1) / 2))) {
     e = ring_launch_dw_tiled(a, NCv, st);   // every group's launch status, first failure wins
   } else {
-    if (NCv != 1) return hipErrorInvalidValue;
-    RING_LAUNCH((ring_dw_kernel<1, 4>), dim3(blocks), dim3(256), 0, st, a);
+    if (NCv == 1) RING_LAUNCH((ring_dw_kernel<1, 4>), dim3(blocks), dim3(256), 0, st, a);
+    else if (NCv == 2) RING_LAUNCH((ring_dw_kernel<2, 8>), dim3(blocks), dim3(256), 0, st, a);
+    else return hipErrorInvalidValue;
     e = hipGetLastError();
   }
   }

@@ -129,7 +129,7 @@ size_t ring_panel_workspace_bytes(int NC, int nbt);
 hipError_t ring_launch_panel_fwd(const RingFwdArgs& a, int NC, hipStream_t st);
 
 // LDS-tiled weight-gradient contraction for NC in {4, 8, 16, 24, 32} (ring_dw.hip).
-bool ring_dw_tiled_applicable(int NC);
+bool ring_dw_tiled_applicable(int NC, int k, long nchunk);      // nchunk: batch tiles times pairs of steps
 int ring_dw_tiled_nz(int NC, int k, long nchunk);
 hipError_t ring_launch_dw_tiled(const RingDwArgs& a, int NC, hipStream_t st);
 
@@ -218,7 +218,6 @@ int ring_last_kernel_name(int id, char* buf, size_t n);
     hipLaunchKernelGGL(kern, grid, block, lds, st, __VA_ARGS__);           \
   } while (0)
 
-bool ring_dw_tiled_applicable(int NC);
 int ring_dw_tiled_segments(int nbt, int T, int nz);   // launches per matrix group of the tiled weight-gradient kernel
 
 // Optional event bracketing of launches (benchmark support).

@@ -69,14 +69,14 @@ int make_geo(int N, int k, int T, int B, Geo& g) {
   g.side_bytes = align_up((size_t)T * g.nbt * 16 * g.NPAD * 2);
   g.pair_bytes = align_up((size_t)((T + 1) / 2) * 2 * g.nbt * 16 * g.NPAD * 2);
   const int NT = 4 * nc;
-  const long per_z = (long)(NT / 2) * (NT / 4) * ((k + 3) / 3);  // wave work items per K split (of the kernel for N <= 64)
+  const long per_z = (long)(NT / 2) * ((k + 3) / 3);  // wave work items per K split (of the kernel for N <= 128)
   const long nchunk = (long)g.nbt * ((T + 1) / 2);
   if (nchunk > 0x7fffffffL) return fail(RINGATTR_ERR_INVALID, "batch_size * seq_len is too large");
   long nz = (2048 + per_z - 1) / per_z;
   if (nz > 128) nz = 128;
   if (nz > nchunk) nz = nchunk;
   if (nz < 1) nz = 1;
-  g.nz = ring_dw_tiled_applicable(nc) ? ring_dw_tiled_nz(nc, k, nchunk) : (int)nz;
+  g.nz = ring_dw_tiled_applicable(nc, k, nchunk) ? ring_dw_tiled_nz(nc, k, nchunk) : (int)nz;
   g.partial_bytes = align_up((size_t)g.nz * (1 + k) * g.NPAD * g.NPAD * 4);
   g.carry_bytes = nc >= 4 ? align_up(ring_wide_carry_bytes(nc, g.nbt)) : 0;   // (small; sized whichever family runs)
   g.trig_bytes = nc >= 4 ? align_up((size_t)g.NPAD * 2 * sizeof(float)) : 0;
@@ -916,7 +916,7 @@ int ringattr_profile_enable(int on) {
 int ringattr_dw_segments(int N, int a_dim, int seq_len, int batch_size) {
   Geo g;
   if (make_geo(N, a_dim, seq_len, batch_size, g) != RINGATTR_OK) return -1;
-  return ring_dw_tiled_applicable(g.NC) ? ring_dw_tiled_segments(g.nbt, seq_len, g.nz) : 1;
+  return ring_dw_tiled_applicable(g.NC, g.k, (long)g.nbt * ((g.T + 1) / 2)) ? ring_dw_tiled_segments(g.nbt, seq_len, g.nz) : 1;
 }
 
 int ringattr_last_kernel_name(int kernel, char* buf, size_t buf_bytes) {

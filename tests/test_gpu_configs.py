@@ -952,3 +952,22 @@ def test_weight_gradient_time_segments_add_up(B, T, k, N, act, gpu_device, monke
     ref, _ = O.forward_dense(p["A"], p["Wa"], J0, J1, p["Wo"], p["r0"], 0.15, act)
     g = O.backward_dense(p["G"], p["A"], p["Wa"], J0, J1, p["Wo"], ref, p["r0"], 0.15, act)
     assert O.max_rel_err(cut[1], g["grad_Wo"]) <= GRAD_TOL and O.max_rel_err(cut[0], g["grad_Wa"]) <= GRAD_TOL
+
+
+# N <= 128: the last shapes of one contraction kernel and the first of the other, few and many launches; always one launch
+@pytest.mark.parametrize("B,T,k,N,kernel", [(64, 24, 7, 100, "ring_dw_kernel"), (64, 25, 7, 100, "ring_dw_direct_kernel"),
+                                            (16, 1, 3, 65, "ring_dw_kernel"), (512, 16, 13, 128, "ring_dw_kernel"),
+                                            (512, 17, 13, 128, "ring_dw_direct_kernel"), (16, 1, 2, 120, "ring_dw_direct_kernel")])
+def test_weight_gradient_kernels_of_narrow_rings_on_either_side_of_their_line(B, T, k, N, kernel, gpu_device):
+    from rnn_train_ring_attractor_amd import ring_rnn_cuda_func, _lib
+    print(f"[case] weight gradients of a narrow ring B={B} T={T} k={k} N={N}", flush=True)
+    p = make_problem(94, B, T, k, N, action="dense")
+    Wa, Wo = _t(p["Wa"], gpu_device).requires_grad_(True), _t(p["Wo"], gpu_device).requires_grad_(True)
+    h = ring_rnn_cuda_func(_t(p["A"], gpu_device), Wa, -0.05, 0.4, Wo, _t(p["r0"], gpu_device), 0.15, "tanh")
+    h.backward(_t(p["G"], gpu_device))
+    assert _lib.last_kernel_names()["dw"].startswith(kernel + "<")
+    ref, _ = O.forward_dense(p["A"], p["Wa"], -0.05, 0.4, p["Wo"], p["r0"], 0.15, "tanh")
+    g = O.backward_dense(p["G"], p["A"], p["Wa"], -0.05, 0.4, p["Wo"], ref, p["r0"], 0.15, "tanh")
+    for got, name in ((Wa.grad, "grad_Wa"), (Wo.grad, "grad_Wo")):
+        x = got.cpu().numpy()
+        assert O.cosine(x, g[name]) >= GRAD_COS and O.max_rel_err(x, g[name]) <= GRAD_TOL, name
