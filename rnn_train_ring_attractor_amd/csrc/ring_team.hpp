@@ -134,19 +134,19 @@ enum : int { WEIGHT_ROWS, WEIGHT_ROWS4, WEIGHT_COLUMNS };      // COLUMNS: the t
 
 template <int HOW>
 __device__ __forceinline__ void weight_load(WeightLoad& l, const float* __restrict__ W, int N, int out, int k0) {
-  const unsigned o = out < N ? out : N - 1;          // (offsets in 32 bits: one register an address, not two)
+  const unsigned o = out < N ? out : N - 1;
   if constexpr (HOW == WEIGHT_COLUMNS) {
 #pragma unroll
-    for (int x = 0; x < 8; ++x) l.v[x] = W[(unsigned)(k0 + x < N ? k0 + x : N - 1) * (unsigned)N + o];
+    for (int x = 0; x < 8; ++x) l.v[x] = W[(size_t)(k0 + x < N ? k0 + x : N - 1) * N + o];
   } else if constexpr (HOW == WEIGHT_ROWS4) {      // (N is a multiple of four: a group of four is in the row or past it)
-    const unsigned at = o * (unsigned)N;
+    const unsigned at = o * (unsigned)N;             // (32 bits here: one register an address, not two)
     const f32x4 lo = *reinterpret_cast<const f32x4*>(W + (at + (unsigned)(k0 < N ? k0 : 0))),
                 hi = *reinterpret_cast<const f32x4*>(W + (at + (unsigned)(k0 + 4 < N ? k0 + 4 : 0)));
 #pragma unroll
     for (int x = 0; x < 4; ++x) { l.v[x] = lo[x]; l.v[4 + x] = hi[x]; }
   } else {
 #pragma unroll
-    for (int x = 0; x < 8; ++x) l.v[x] = W[o * (unsigned)N + (unsigned)(k0 + x < N ? k0 + x : N - 1)];
+    for (int x = 0; x < 8; ++x) l.v[x] = W[(size_t)o * N + (k0 + x < N ? k0 + x : N - 1)];
   }
 }
 __device__ __forceinline__ bf16x8 weight_fragment(const WeightLoad& l, int N, int out, int k0, float scale, float shift) {
@@ -239,51 +239,88 @@ struct TeamCompute {
   // offsets).  Only the last one can lie past the contraction: its lanes then point past the buffer and read zero.
   unsigned x_lane, rs_lane, x_last, rs_last;
 
+  // The order of the loads, by what was measured.  Rolling: a fragment's place is loaded again as soon as it is converted.
+  // Otherwise batches drain before the next begins.  Rows on 16-byte boundaries roll (in batches the loads' registers spill,
+  // 780 bytes a lane in the kernel of 13 matrices in registers, and two calls, N = 512 with 16 channels and N = 1024 with two,
+  // take 131 and 74 us, not 106 and 61).  A word at a time, batches of four spill less: us a call, T = 20, rolling and in
+  // batches: N = 129, 3 channels, B = 64 33 and 29; N = 513, 3 channels, B = 1 78 and 65; N = 1023, 2 channels, B = 1 94 and 72;
+  // training N = 1023, B = 64 227 and 188.  Only with 24 fragments in registers and matrices in LDS do batches leave spills in the
+  // loop over the steps, also for rows on 16-byte boundaries (N = 800, 3 channels, B = 300 106 and 134).
   template <int HOW>
   __device__ __forceinline__ void load_matrices(const RingTeamArgs& c, bf16x8* wl, int mem, int w, int lane) {
-    const int q = lane >> 4, n = lane & 15;
+    constexpr bool ROLL = HOW == WEIGHT_ROWS4 || (EX && F >= 24);
     constexpr int BATCH = HOW == WEIGHT_ROWS4 ? 8 : 4;      // fragments on their way at a time
+    const int q = lane >> 4, n = lane & 15;
+    auto matrix = [&](int mm) { return mm == 0 || mm > c.k ? c.Wo : c.Wa + (size_t)(mm - 1) * c.N * c.N; };
     // into LDS: the matrices past the registers', this wave's own chunks
     if constexpr (EX) {
-      const int total = (c.k + 1 - MR) * C16 * KPW;
-      for (int f0 = 0; f0 < total; f0 += BATCH) {
-        WeightLoad l[BATCH];
+      auto load = [&](WeightLoad& l, int mm, int cc, int kc) { weight_load<HOW>(l, matrix(mm), c.N, 16 * (mem * C16 + cc) + n, 32 * kc + 8 * q); };
+      auto put = [&](const WeightLoad& l, int mm, int cc, int kc) {
+        wl[((size_t)((mm - MR) * C16 + cc) * c.KC + kc) * 64 + lane] = weight_fragment(l, c.N, 16 * (mem * C16 + cc) + n, 32 * kc + 8 * q, 1.f, 0.f);
+      };
+      if constexpr (ROLL) {
+        const int total = (c.k + 1 - MR) * C16 * KPW;
+        for (int f0 = 0; f0 < total; f0 += BATCH) {
+          WeightLoad l[BATCH];
 #pragma unroll
-        for (int i = 0; i < BATCH; ++i) {
-          const int f = f0 + i < total ? f0 + i : total - 1, mm = MR + f / (C16 * KPW), cc = f / KPW % C16, kc = w + WK * (f % KPW);
-          weight_load<HOW>(l[i], c.Wa + (size_t)(mm - 1) * c.N * c.N, c.N, 16 * (mem * C16 + cc) + n, 32 * kc + 8 * q);
-        }
-        __builtin_amdgcn_sched_barrier(0);
+          for (int i = 0; i < BATCH; ++i) {
+            const int f = f0 + i < total ? f0 + i : total - 1;
+            load(l[i], MR + f / (C16 * KPW), f / KPW % C16, w + WK * (f % KPW));
+          }
+          __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int i = 0; i < BATCH; ++i) {
-          const int f = f0 + i, mm = MR + f / (C16 * KPW), cc = f / KPW % C16, kc = w + WK * (f % KPW);
-          if (f < total && kc < c.KC)
-            wl[((size_t)((mm - MR) * C16 + cc) * c.KC + kc) * 64 + lane] = weight_fragment(l[i], c.N, 16 * (mem * C16 + cc) + n, 32 * kc + 8 * q, 1.f, 0.f);
+          for (int i = 0; i < BATCH; ++i) {
+            const int f = f0 + i, kc = w + WK * (f % KPW);
+            if (f < total && kc < c.KC) put(l[i], MR + f / (C16 * KPW), f / KPW % C16, kc);
+          }
         }
+      } else {
+        for (int mm = MR; mm <= c.k; ++mm)
+          for (int kc = w; kc < c.KC; kc += WK) {
+            WeightLoad l[C16];
+#pragma unroll
+            for (int cc = 0; cc < C16; ++cc) load(l[cc], mm, cc, kc);
+#pragma unroll
+            for (int cc = 0; cc < C16; ++cc) put(l[cc], mm, cc, kc);
+          }
       }
     }
-    // into registers: each fragment's place is loaded again as soon as it is converted.  In batches that drain before the
-    // next begins, and with conversions left until the fragment's first use, the loads' registers spill (780 bytes a lane in
-    // the kernel of 13 matrices in registers) and the same two calls take 131 and 74 us; so the fragment is opaque here.
-    WeightLoad l[BATCH];
-    auto load = [&](int f) {
-      const int mm = f / (C16 * KPW), cc = f / KPW % C16, kc = w + WK * (f % KPW);
-      const float* W = mm == 0 || mm > c.k ? c.Wo : c.Wa + (size_t)(mm - 1) * c.N * c.N;
-      weight_load<HOW>(l[f % BATCH], W, c.N, 16 * (mem * C16 + cc) + n, 32 * kc + 8 * q);
+    // into registers
+    auto load = [&](WeightLoad& l, int f) {
+      weight_load<HOW>(l, matrix(f / (C16 * KPW)), c.N, 16 * (mem * C16 + f / KPW % C16) + n, 32 * (w + WK * (f % KPW)) + 8 * q);
     };
-#pragma unroll
-    for (int f = 0; f < BATCH && f < F; ++f) load(f);
-    __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-    for (int f = 0; f < F; ++f) {
-      const int mm = f / (C16 * KPW), cc = f / KPW % C16, kc = w + WK * (f % KPW);
-      bf16x8 v = weight_fragment(l[f % BATCH], mm <= c.k ? c.N : 0, 16 * (mem * C16 + cc) + n, 32 * kc + 8 * q,
+    auto keep = [&](const WeightLoad& l, int f) {
+      const int mm = f / (C16 * KPW);
+      bf16x8 v = weight_fragment(l, mm <= c.k ? c.N : 0, 16 * (mem * C16 + f / KPW % C16) + n, 32 * (w + WK * (f % KPW)) + 8 * q,
                                  mm == 0 ? c.scale0 : 1.f, mm == 0 ? c.shift0 : 0.f);
-      asm volatile("" : "+v"(v));
+      asm volatile("" : "+v"(v));          // (converted here, not at its first use: twice the registers until then)
       if (f < FR) wreg[f < FR ? f : 0] = v;
       else parked[(f - FR) * 64] = v;
-      if (f + BATCH < F) load(f + BATCH);
+    };
+    if constexpr (ROLL) {
+      WeightLoad l[BATCH];
+#pragma unroll
+      for (int f = 0; f < BATCH && f < F; ++f) load(l[f], f);
       __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int f = 0; f < F; ++f) {
+        keep(l[f % BATCH], f);
+        if (f + BATCH < F) load(l[f % BATCH], f + BATCH);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    } else {
+#pragma unroll
+      for (int f0 = 0; f0 < F; f0 += BATCH) {
+        WeightLoad l[BATCH];
+#pragma unroll
+        for (int i = 0; i < BATCH; ++i)
+          if (f0 + i < F) load(l[i], f0 + i);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int i = 0; i < BATCH; ++i)
+          if (f0 + i < F) keep(l[i], f0 + i);
+        __builtin_amdgcn_sched_barrier(0);
+      }
     }
   }
   template <bool TR>
