@@ -126,7 +126,7 @@ __device__ __forceinline__ u32x2 quad_rows2(unsigned x, int lane) {
 // matrix and the padding is zeroed afterwards.  ROWS4 (rows that start on 16-byte boundaries): two 16-byte loads, eight
 // fragments on their way; a call of T = 20 steps at N = 512, 16 channels, B = 256 falls from 181 us (a word at a time, four
 // fragments) to 106, at N = 1024, two channels, B = 1 from 105 to 61 (all on their way at once into one XCD: 12.6 MB).
-// Other rows are slower so than a word at a time (N = 1023, B = 100: 140 against 98 us).
+// Other rows are slower so than a word at a time in a team (N = 1023, B = 100: 140 against 98 us).
 struct WeightLoad { float v[8]; };
 typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));
 typedef float f32x2u __attribute__((ext_vector_type(2), aligned(4)));

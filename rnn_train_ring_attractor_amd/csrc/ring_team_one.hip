@@ -157,20 +157,38 @@ __device__ __forceinline__ void one_put(OneLds<KCT, MR, RW>& L, int buf, const O
   }
 }
 
-// The wave's weight fragments: output neurons of its column tile, all chunks.
+// The wave's weight fragments: output neurons of its column tile, all chunks; matrices past a_dim are zero.
+// The workgroup takes in the whole ring, which a short call feels.  Rows off 16-byte boundaries come in 16-byte loads too,
+// where a chunk is whole, and nothing is loaded for matrices that are not there.  us a call, T = 20, three channels, teams of
+// eight workgroups, here a word at a time with seven matrices, now: N = 101, B = 64: 27 39 22, B = 20000: 164 232 151; N = 65,
+// B = 1: 26.6 29.4 21.2; five channels, N = 127, B = 64: 33 44 30.
 template <int KCT, int MR, bool TR>
 __device__ __forceinline__ void one_weights(const RingTeamArgs& c, int w, int lane, bf16x8 (&wt)[MR][KCT]) {
   const int q = lane >> 4, out = 16 * w + (lane & 15);
   auto load = [&](auto how) {
     constexpr int HOW = decltype(how)::value, F = MR * KCT, BATCH = 4;
+    auto fetch = [&](WeightLoad& l, int m, int kc) {
+      const float* W = m == 0 || m > c.k ? c.Wo : c.Wa + (size_t)(m - 1) * c.N * c.N;
+      if (HOW == WEIGHT_ROWS && 32 * kc + 32 <= c.N) {
+        const float* src = W + (size_t)(out < c.N ? out : c.N - 1) * c.N + (32 * kc + 8 * q);
+        const f32x4 lo = *reinterpret_cast<const f32x4u*>(src), hi = *reinterpret_cast<const f32x4u*>(src + 4);
+#pragma unroll
+        for (int x = 0; x < 4; ++x) { l.v[x] = lo[x]; l.v[4 + x] = hi[x]; }
+      } else {
+        weight_load<HOW>(l, W, c.N, out, 32 * kc + 8 * q);
+      }
+    };
 #pragma unroll
     for (int f0 = 0; f0 < F; f0 += BATCH) {
+      if (f0 / KCT > c.k) {
+#pragma unroll
+        for (int f = f0; f < f0 + BATCH && f < F; ++f) wt[f / KCT][f % KCT] = bf16x8{};
+        continue;
+      }
       WeightLoad l[BATCH];
 #pragma unroll
-      for (int i = 0; i < BATCH; ++i) {
-        const int m = (f0 + i) / KCT, kc = (f0 + i) % KCT;
-        if (f0 + i < F) weight_load<HOW>(l[i], m == 0 || m > c.k ? c.Wo : c.Wa + (size_t)(m - 1) * c.N * c.N, c.N, out, 32 * kc + 8 * q);
-      }
+      for (int i = 0; i < BATCH; ++i)
+        if (f0 + i < F) fetch(l[i], (f0 + i) / KCT, (f0 + i) % KCT);
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
       for (int i = 0; i < BATCH; ++i) {
