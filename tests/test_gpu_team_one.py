@@ -15,9 +15,12 @@ TRAJ_TOL = 1e-2      # bf16 operands against fp64, as in the parity tests of the
 GRAD_COS, GRAD_TOL = 0.999, 2e-2
 
 # B, T, k, N, act: two and four chunks, whole and cut; widths 0 to 3 modulo 4; single steps, odd and even lengths; one to six
-# channels (both register groups); ragged tiles, one row, more tiles than compute units
+# channels (both register groups); ragged tiles, one row, more tiles than compute units; 4 rows per workgroup up to 1024, 8 up
+# to 2048, then 16, each with both register groups and with odd widths
 CASES = [(1, 1, 1, 17, "tanh"), (16, 2, 2, 32, "gelu"), (33, 3, 2, 64, "silu"), (20, 7, 3, 65, "gelu"), (15, 4, 4, 99, "tanh"),
-         (64, 9, 2, 120, "tanh"), (50, 6, 6, 126, "gelu"), (40, 5, 5, 127, "silu"), (17, 8, 2, 128, "gelu"), (4200, 3, 2, 101, "gelu")]
+         (64, 9, 2, 120, "tanh"), (50, 6, 6, 126, "gelu"), (40, 5, 5, 127, "silu"), (17, 8, 2, 128, "gelu"), (4200, 3, 2, 101, "gelu"),
+         (1500, 5, 2, 101, "gelu"), (1100, 4, 5, 120, "silu"), (1500, 5, 5, 101, "tanh"), (2047, 4, 2, 120, "tanh"), (1030, 3, 3, 50, "gelu"),
+         (2101, 5, 5, 127, "silu")]
 
 
 def _t(x, dev):
@@ -83,11 +86,11 @@ def test_teams_of_one_without_a_j0_term_after_a_run_of_nan(B, k, N, gpu_device):
 
 @pytest.mark.parametrize("N,k", [(100, 2), (127, 5), (50, 3)])
 def test_rows_of_teams_of_one_do_not_depend_on_the_batch(N, k, gpu_device):
-    B, T = 600, 6
+    B, T = 2300, 6                       # (16 rows per workgroup; the parts have 4 and 8)
     print(f"[case] team of one, rows N={N} k={k}", flush=True)
     p = make_problem(31, B, T, k, N, action="dense")
     whole = _run(p, "gelu", -1.0 / N, 0.6, gpu_device)
-    for lo, n in ((0, 1), (5, 16), (37, 100), (16, 512)):
+    for lo, n in ((0, 1), (5, 16), (37, 100), (16, 512), (1276, 1024), (3, 1025), (250, 2048)):
         part = _run({**p, "A": p["A"][lo:lo + n], "r0": p["r0"][lo:lo + n], "G": p["G"][:, lo:lo + n]}, "gelu", -1.0 / N, 0.6, gpu_device)
         assert torch.equal(part["hist"], whole["hist"][:, lo:lo + n])
         assert torch.equal(part["grad_r_init"], whole["grad_r_init"][lo:lo + n]) and torch.equal(part["grad_A"], whole["grad_A"][lo:lo + n])
