@@ -224,13 +224,17 @@ __global__ __launch_bounds__(256) void ring_dw_direct_kernel(RingDwArgs p, int m
 }
 
 // N <= 128: a launch per three matrices, of a few workgroups where there is little to contract, against one launch for all
-// matrices of the kernel with a wave per 32 x 128 block (us of a training pass there and here, N = 120, T = 20, B = 1, 10 chunks:
-// a_dim 3 59.5 and 62.6, 7 89 and 100, 16 135 and 168; 40 chunks: a_dim 7 101.5 and 104.6, 16 154 and 174; 60 chunks: a_dim 7 392
-// and 379; 240 chunks: a_dim 12 566 and 573, 480 345 and 338; N = 96, a_dim 24, 480 chunks 1539 and 1560, 960 3023 and 3010).  Up
-// to two channels there is one launch here too.
+// matrices of the kernel with a wave per 32 x 128 block.  A training pass on this kernel, as a share of its time on that one,
+// N = 65 to 128, by launches and chunks of the contraction (16 rows x two steps):
+//   two launches    10: 1.07-1.10   50: 1.03-1.07   64: 0.90-0.98   128: 0.84-0.95   440: 0.95-0.99
+//   three           10: 1.14-1.18   50: 1.11-1.14   64: 1.02-1.09   88: 0.99-1.03   128: 0.94-0.98   440: 0.90-0.94
+//   four            10: 1.19-1.20   64: 1.15-1.20   88: 1.04-1.08   128: 0.96-1.00   440: 0.96-0.98
+//   five and six    10: 1.22-1.26   64: 1.18-1.31   128: 1.05-1.12   190: 1.05-1.08   440: 0.96-0.98
+//   nine            480: 0.99   960: 1.00
+// Up to two channels there is one launch here too.
 bool ring_dw_tiled_applicable(int NC, int k, long nchunk) {
   const int launches = (k + 3) / 3;
-  if (NC == 2) return launches == 1 || nchunk > (launches <= 4 ? 48 : launches <= 6 ? 256 : 512);
+  if (NC == 2) return launches == 1 || nchunk > (launches == 2 ? 56 : launches == 3 ? 96 : launches == 4 ? 112 : launches <= 6 ? 256 : 512);
   return NC == 4 || NC == 8 || NC == 16 || NC == 24 || NC == 32;
 }
 

@@ -955,7 +955,9 @@ def test_weight_gradient_time_segments_add_up(B, T, k, N, act, gpu_device, monke
 
 
 # N <= 128: the last shapes of one contraction kernel and the first of the other, few and many launches; always one launch
-@pytest.mark.parametrize("B,T,k,N,kernel", [(64, 24, 7, 100, "ring_dw_kernel"), (64, 25, 7, 100, "ring_dw_direct_kernel"),
+@pytest.mark.parametrize("B,T,k,N,kernel", [(64, 48, 7, 100, "ring_dw_kernel"), (64, 49, 7, 100, "ring_dw_direct_kernel"),
+                                            (64, 28, 3, 65, "ring_dw_kernel"), (64, 29, 5, 100, "ring_dw_direct_kernel"),
+                                            (64, 56, 11, 120, "ring_dw_kernel"), (64, 57, 9, 128, "ring_dw_direct_kernel"),
                                             (16, 1, 3, 65, "ring_dw_kernel"), (512, 16, 13, 128, "ring_dw_kernel"),
                                             (512, 17, 13, 128, "ring_dw_direct_kernel"), (16, 1, 2, 120, "ring_dw_direct_kernel")])
 def test_weight_gradient_kernels_of_narrow_rings_on_either_side_of_their_line(B, T, k, N, kernel, gpu_device):
