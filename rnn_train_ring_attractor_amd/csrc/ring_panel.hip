@@ -464,11 +464,12 @@ static hipError_t panel_steps(const RingFwdArgs& a, int NC, int C, hipStream_t s
 // Where workgroups queue, a step's first ones find no announced sums (who would announce them has not begun) and add up all of
 // their rows: with more than one a compute unit, operand and sums are a launch's.  us per step, carried and with the launch,
 // N = 1100, 16 channels: B = 1000 146 and 133, B = 3000 444 and 385; N = 2048, one channel, B = 3000 126 and 110; with one a
-// compute unit, N = 2048, B = 1000: one channel 39 and 41, 16 channels 191 and 193.
+// compute unit, N = 2048, B = 1000: one channel 39 and 41, 16 channels 191 and 193.  A single step has nothing to carry either
+// (us a call: N = 1024, 5 channels, B = 512 36.2 and 33.2).
 template <int ACT, int R>
 static hipError_t panel_run(const RingFwdArgs& a, int NC, int C, hipStream_t st) {
   const bool queue = (long)((a.nbt + R - 1) / R) * (4 * NC / C) > 256;
-  return queue ? panel_steps<ACT, R, false>(a, NC, C, st) : panel_steps<ACT, R, true>(a, NC, C, st);
+  return queue || a.T == 1 ? panel_steps<ACT, R, false>(a, NC, C, st) : panel_steps<ACT, R, true>(a, NC, C, st);
 }
 
 template <int ACT>

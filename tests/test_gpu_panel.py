@@ -27,6 +27,8 @@ def _forward(p, act, J0, J1, dev):
     (33, 7, 2, 1027, "gelu", "11"), (20, 8, 2, 1025, "tanh", "24"), (150, 7, 3, 1030, "silu", "81"), (1, 9, 16, 2047, "gelu", None),
     # the most workgroups that do not queue (256), and more
     (32, 5, 2, 2047, "gelu", "11"), (33, 5, 2, 2047, "gelu", "11"), (1000, 4, 16, 1100, "tanh", None),
+    # a single step, and two
+    (20, 1, 2, 2047, "gelu", None), (130, 1, 7, 768, "silu", None), (130, 2, 7, 768, "silu", None),
 ])
 def test_panel_equals_block_kernels_and_oracle(B, T, k, N, act, shape, gpu_device, monkeypatch):
     print(f"[case] panel B={B} T={T} k={k} N={N} {act} shape={shape}", flush=True)
