@@ -160,20 +160,46 @@ __device__ __forceinline__ void one_put(OneLds<KCT, MR, RW>& L, int buf, const O
 // The wave's weight fragments: output neurons of its column tile, all chunks; matrices past a_dim are zero.
 // The workgroup takes in the whole ring, which a short call feels.  Rows off 16-byte boundaries come in 16-byte loads too,
 // where a chunk is whole, and nothing is loaded for matrices that are not there.  us a call, T = 20, three channels, teams of
-// eight workgroups, here a word at a time with seven matrices, now: N = 101, B = 64: 27 39 22, B = 20000: 164 232 151; N = 65,
+// eight workgroups, here a word at a time with seven matrices, so: N = 101, B = 64: 27 39 22, B = 20000: 164 232 151; N = 65,
 // B = 1: 26.6 29.4 21.2; five channels, N = 127, B = 64: 33 44 30.
+// What is left is instruction issue, so few are spent on a value: a chunk's mask is made once for all matrices and put on pairs,
+// addresses are 32-bit offsets, and rows of the transposed matrix that are not there are past a buffer's end.  us of a training
+// pass, teams of eight, a mask and an address a value, so: N = 65, B = 1, T = 1, six channels 37.2 43.7 37.9; N = 128, B = 64, T = 3,
+// six 40.4 43.1 39.5; N = 101, B = 300, T = 8, six 81.7 80.2 75.3; forward, N = 65, B = 300, T = 8, four 16.6 17.3 16.0.  The
+// forward of one to three steps stays up to 1.3 us behind the teams (N = 101, four channels: 9.3 and 10.5), 4.7 where rows are
+// off their boundaries and all seven matrices there (N = 127, six: 13.2 and 17.9; a row of 128 bytes touches two lines twice).
 template <int KCT, int MR, bool TR>
 __device__ __forceinline__ void one_weights(const RingTeamArgs& c, int w, int lane, bf16x8 (&wt)[MR][KCT]) {
   const int q = lane >> 4, out = 16 * w + (lane & 15);
+  const unsigned o = out < c.N ? out : c.N - 1;
+  u32x4 keep[KCT];                     // what of a fragment is in the matrix
+#pragma unroll
+  for (int kc = 0; kc < KCT; ++kc)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int left = out < c.N ? c.N - (32 * kc + 8 * q + 2 * i) : 0;
+      keep[kc][i] = left > 1 ? 0xFFFFFFFFu : (left > 0 ? 0xFFFFu : 0u);
+    }
   auto load = [&](auto how) {
     constexpr int HOW = decltype(how)::value, F = MR * KCT, BATCH = 4;
+    const unsigned row = (unsigned)c.N * 4u, at = HOW == WEIGHT_COLUMNS ? 8 * q * row + 4u * o : o * row + 32u * q;      // bytes
     auto fetch = [&](WeightLoad& l, int m, int kc) {
       const float* W = m == 0 || m > c.k ? c.Wo : c.Wa + (size_t)(m - 1) * c.N * c.N;
-      if (HOW == WEIGHT_ROWS && 32 * kc + 32 <= c.N) {
-        const float* src = W + (size_t)(out < c.N ? out : c.N - 1) * c.N + (32 * kc + 8 * q);
-        const f32x4 lo = *reinterpret_cast<const f32x4u*>(src), hi = *reinterpret_cast<const f32x4u*>(src + 4);
+      if constexpr (HOW == WEIGHT_COLUMNS) {           // (rows past the matrix are past the buffer: zeros)
+        const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(W), 0, (int)(c.N * row), 0x00020000);
+#pragma unroll
+        for (int x = 0; x < 8; ++x)
+          l.v[x] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, (int)(at + (32 * kc + x) * row), 0, 0));
+      } else if (HOW == WEIGHT_ROWS && 32 * kc + 32 <= c.N) {
+        const char* src = reinterpret_cast<const char*>(W + 32 * kc) + at;
+        const f32x4 lo = *reinterpret_cast<const f32x4u*>(src), hi = *reinterpret_cast<const f32x4u*>(src + 16);
 #pragma unroll
         for (int x = 0; x < 4; ++x) { l.v[x] = lo[x]; l.v[4 + x] = hi[x]; }
+      } else if (HOW == WEIGHT_ROWS) {
+        const unsigned last = c.N - 1, k0 = 32 * kc + 8 * q;
+        const char* src = reinterpret_cast<const char*>(W);
+#pragma unroll
+        for (int x = 0; x < 8; ++x) l.v[x] = *reinterpret_cast<const float*>(src + (o * row + 4u * (k0 + x < last ? k0 + x : last)));
       } else {
         weight_load<HOW>(l, W, c.N, out, 32 * kc + 8 * q);
       }
@@ -194,9 +220,14 @@ __device__ __forceinline__ void one_weights(const RingTeamArgs& c, int w, int la
       for (int i = 0; i < BATCH; ++i) {
         const int m = (f0 + i) / KCT, kc = (f0 + i) % KCT;
         if (f0 + i < F) {
-          bf16x8 f = weight_fragment(l[i], m <= c.k ? c.N : 0, out, 32 * kc + 8 * q, 1.f, 0.f);
+          u32x4 f;
+#pragma unroll
+          for (int x = 0; x < 4; ++x) {
+            f[x] = pack_bf16(l[i].v[2 * x], l[i].v[2 * x + 1]) & keep[kc][x];
+            if (f0 % KCT != 0 || BATCH > KCT) f[x] = m <= c.k ? f[x] : 0u;      // (otherwise the batch is one matrix)
+          }
           asm volatile("" : "+v"(f));              // (here, not at its first use: twice the registers until then)
-          wt[m][kc] = f;
+          wt[m][kc] = __builtin_bit_cast(bf16x8, f);
         }
       }
       __builtin_amdgcn_sched_barrier(0);
