@@ -254,7 +254,9 @@ struct TeamCompute {
     auto matrix = [&](int mm) { return mm == 0 || mm > c.k ? c.Wo : c.Wa + (size_t)(mm - 1) * c.N * c.N; };
     // into LDS: the matrices past the registers', this wave's own chunks
     if constexpr (EX) {
-      auto load = [&](WeightLoad& l, int mm, int cc, int kc) { weight_load<HOW>(l, matrix(mm), c.N, 16 * (mem * C16 + cc) + n, 32 * kc + 8 * q); };
+      auto load = [&](WeightLoad& l, int mm, int cc, int kc) {
+        weight_load<HOW>(l, c.Wa + (size_t)(mm - 1) * c.N * c.N, c.N, 16 * (mem * C16 + cc) + n, 32 * kc + 8 * q);
+      };
       auto put = [&](const WeightLoad& l, int mm, int cc, int kc) {
         wl[((size_t)((mm - MR) * C16 + cc) * c.KC + kc) * 64 + lane] = weight_fragment(l, c.N, 16 * (mem * C16 + cc) + n, 32 * kc + 8 * q, 1.f, 0.f);
       };
