@@ -215,8 +215,10 @@ hipError_t ring_launch_bump(const float* angle, size_t stride, float* out, int N
 // not zero.  The first `signal` workgroups go through the samples, a thread each, the others copy the matrices.
 // Bound by launches at the sizes of a training step: with the launch behind it 6 us where a chain of thirteen tensor
 // operations took 33 (k = 16, B = 1, T = 100, N = 256).
-// A signal of up to COMPACT_ALONE samples is one workgroup's and needs no launch behind it (the evaluation of
-// one trial, 100 samples: 97.2 -> 96.1 us a call)
+// A short signal is one workgroup's and needs no launch behind it (the evaluation of one trial, 100 samples: 97.2 -> 96.1 us a
+// call): up to COMPACT_ALONE samples, and no more than 32 loads a thread one after the other (16 of 16 bytes).  us by channels and
+// samples, one workgroup's, against 6.3 to 6.5 with the launch behind it (64 channels: 8.5): 3: 1024 3.8; 15: 400 5.4, 700 7.3,
+// 1024 9.2; 16: 400 4.0, 700 5.2, 1024 6.5; 64: 100 6.2, 400 11.4, 1024 22.
 constexpr int COMPACT_BLOCK = 256, COMPACT_SIGNAL_MAX = RING_COMPACT_FLAGS, COMPACT_COPY = 512, COMPACT_ALONE = 1024;
 __global__ __launch_bounds__(COMPACT_BLOCK) void ring_compact_kernel(const float* __restrict__ A, const float* __restrict__ Wa,
                                                                      f32x2* __restrict__ out, float* __restrict__ Wout, int* violated,
@@ -274,7 +276,9 @@ hipError_t ring_launch_compact(const float* A, const float* Wa, float* out, floa
                                int c0, int c1, hipStream_t st) {
   const size_t nn = (size_t)N * N;
   const size_t blocks = (samples + COMPACT_BLOCK - 1) / COMPACT_BLOCK, copies = (nn + COMPACT_BLOCK - 1) / COMPACT_BLOCK;
-  const int signal = samples <= COMPACT_ALONE ? 1 : (int)(blocks < COMPACT_SIGNAL_MAX ? blocks : COMPACT_SIGNAL_MAX);
+  const size_t loads = (k & 3) == 0 && (reinterpret_cast<uintptr_t>(A) & 15) == 0 ? k / 2 : k;      // (one of 16 bytes counts twice)
+  const bool alone = samples <= COMPACT_ALONE && blocks * loads <= 32;
+  const int signal = alone ? 1 : (int)(blocks < COMPACT_SIGNAL_MAX ? blocks : COMPACT_SIGNAL_MAX);
   const int copy = (int)(copies < COMPACT_COPY ? copies : COMPACT_COPY);
   hipLaunchKernelGGL(ring_compact_kernel, dim3(signal + copy), dim3(COMPACT_BLOCK), 0, st, A, Wa, reinterpret_cast<f32x2*>(out), Wout,
                      violated, samples, nn, k, c0, c1, signal);

@@ -140,9 +140,11 @@ def test_fused_clip_adam_of_many_parameters(numel, gpu_device):
 
 
 # k a multiple of four and not, a slice that starts off a 16-byte boundary, one sample, more samples than one pass of the grid,
-# the most that a single workgroup takes and one more
+# the most that a single workgroup takes and one more, also with more channels
 @pytest.mark.parametrize("B,T,k,N,pair,offset", [(1, 1, 3, 17, (0, 2), 0), (5, 7, 16, 33, (0, 1), 0), (40, 9, 6, 130, (2, 5), 3),
-                                                 (700, 513, 4, 20, (1, 3), 1), (8, 128, 16, 33, (0, 1), 0), (25, 41, 16, 33, (0, 1), 0)])
+                                                 (700, 513, 4, 20, (1, 3), 1), (8, 128, 16, 33, (0, 1), 0), (25, 41, 16, 33, (0, 1), 0),
+                                                 (2, 256, 15, 20, (0, 1), 0), (19, 27, 15, 20, (0, 1), 0), (1, 256, 64, 20, (0, 1), 0),
+                                                 (1, 257, 64, 20, (3, 60), 0), (1, 257, 16, 20, (0, 1), 2), (3, 171, 16, 20, (0, 1), 2)])
 def test_compacted_channels_are_the_named_ones_and_the_rest_is_checked(B, T, k, N, pair, offset, gpu_device):
     from rnn_train_ring_attractor_amd.ring_rnn_cuda import _compact
     print(f"[case] compaction B={B} T={T} k={k} N={N} {pair}", flush=True)
