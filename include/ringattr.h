@@ -253,7 +253,7 @@ RINGATTR_API int ringattr_compact_channels(const void* A, const void* Wa, void* 
                       int seq_len, int batch_size, int c0, int c1, void* workspace, size_t workspace_bytes, void* stream);
 
 /* Optimizer tail of a training step: torch.nn.utils.clip_grad_norm_(parameters, max_norm) followed by
- * torch.optim.Adam.step() (root train_general_ring_no_gain.py:333-336), for up to 16 fp32 tensors in three launches.
+ * torch.optim.Adam.step() (root train_general_ring_no_gain.py:333-336), for up to 16 fp32 tensors in two or three launches.
  * The gradient norm is summed in a fixed order (repeatable).  params / grads / exp_avg / exp_avg_sq are HOST arrays of
  * n_tensors device pointers, numel a host array; grads are scaled in place by min(1, max_norm / (norm + 1e-6))
  * (max_norm <= 0: no clipping), then m, v and the parameters are updated in place; `step` counts from 1.

@@ -13,8 +13,9 @@
 // is this file's own counter-based generator (same distributions as the reference, not the same bits as torch's).
 //
 // Optimizer tail (root train_general_ring_no_gain.py:333-336: clip_grad_norm_(parameters, max_norm) then Adam.step()):
-// the squared gradient norm over all tensors in a fixed order (two launches), then one launch that scales the
-// gradients by min(1, max_norm / (norm + 1e-6)) and applies the Adam update to every tensor.
+// the squared gradient norm over all tensors in a fixed order, then one launch that scales the gradients by
+// min(1, max_norm / (norm + 1e-6)) and applies the Adam update to every tensor.  The norm takes two launches, one where that
+// last launch adds up the partial sums itself.
 //
 // Compaction of a zero-padded action signal (root train_general_ring_no_gain.py:52-66): the two driven channels and
 // their matrices side by side, and the check that the others are zero.
@@ -424,7 +425,7 @@ hipError_t ring_launch_clip_adam(const RingOptArgs& a, float* workspace, hipStre
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
   // A launch for the norm alone pays where there are many partial sums, or a step counter that one thread advances.
-  // (N = 256, 16 channels, 272 of them: three launches 17.3 us, two 14.0)
+  // (us a step by partial sums, three launches and two: 17 15.6 and 13.3, 272 17.0 and 13.9, 500 16.0 and 14.0, 1020 27.4 and 26.7)
   if (total <= OPT_OWN_NORM && !a.step_counter) {
     hipLaunchKernelGGL((ring_clip_adam_kernel<true>), dim3(total), dim3(OPT_BLOCK), 0, st, a, norm, workspace, total);
     return hipGetLastError();

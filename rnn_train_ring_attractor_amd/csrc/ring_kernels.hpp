@@ -128,7 +128,8 @@ bool ring_uses_panel(int k, int NC, int nbt);
 size_t ring_panel_workspace_bytes(int NC, int nbt);
 hipError_t ring_launch_panel_fwd(const RingFwdArgs& a, int NC, hipStream_t st);
 
-// LDS-tiled weight-gradient contraction for NC in {4, 8, 16, 24, 32} (ring_dw.hip).
+// LDS-tiled weight-gradient contraction for NC in {2, 4, 8, 16, 24, 32} (ring_dw.hip); NC = 2 not for short contractions with many
+// channels.
 bool ring_dw_tiled_applicable(int NC, int k, long nchunk);      // nchunk: batch tiles times pairs of steps
 int ring_dw_tiled_nz(int NC, int k, long nchunk);
 hipError_t ring_launch_dw_tiled(const RingDwArgs& a, int NC, hipStream_t st);

@@ -161,14 +161,14 @@ __device__ __forceinline__ void write_half(bf16x8* half, const float (&v)[4][2],
   }
 }
 
+struct NoStores {};
+
 }  // namespace
 
 // STATS: also leave the loss head's three sums of every history row (sum_i r_i cos(phi_i), sum_i r_i sin(phi_i),
 // sum_i |r_i|, phi_i = 2 pi i / N) in p.loss_stats[t * B + b], so that the loss needs no pass of its own over the
 // history.  Each wave reduces its 32 neurons' share over the row group's 16 lanes right after the activation, the
 // eight shares meet in LDS (buffer by step parity) and wave 0 adds them in wave order behind the next barrier.
-struct NoStores {};
-
 template <int ACT, bool SAVE, bool FULL, bool STATS>
 __global__ __launch_bounds__(512) void ring_fwd_res256_kernel(RingFwdArgs p) {
   extern __shared__ __attribute__((aligned(16))) char smem[];

@@ -112,12 +112,16 @@ static bool forced() {
   return v && v[0] == '1';
 }
 
+// Whether a workgroup per 4 to 16 rows does it; RINGATTR_TEAM=1 asks for the exchange through L2.
+bool ring_uses_team_one(int N, int k) { return ring_team_one_applicable(N, k) && !forced(); }
+
 // Where teams run (us per time step, measured with T = 60, gelu; forward for inference / forward + backward):
-//   N = 120, a_dim 2:  B = 64: 2.5 -> 0.9 / 5.8 -> 2.3    B = 4096: 2.7 -> 1.9 / 9.6 -> 8.0
 //   N = 360, a_dim 2:  B = 64: 8.2 -> 1.5 / 30.6 -> 3.4   B = 1024: 12.9 -> 3.3 / 31.9 -> 7.8   B = 4096: 15.6 -> 8.0 / 37 -> 23
 //   N = 512, a_dim 2:  B = 64: 8.9 -> 1.6 / 29.1 -> 3.7   B = 2048: 14.3 -> 5.5 / 32.4 -> 14.8
 //   N = 1024, a_dim 2: B = 64: 17.8 -> 3.3 / 43 -> 6.9    B = 2048: 40 -> 19 / 104 -> 50
 // against the streaming and step-per-launch kernels.  The exceptions:
+//   * up to 128 neurons and six channels a workgroup holds the whole ring (ring_team_one.hip); more channels run on teams
+//     (N = 120, a_dim 2, B = 64, while it ran on teams of eight: 2.5 -> 0.9 / 5.8 -> 2.3);
 //   * 128 < N <= 256 with two channels belongs to the weight-resident kernels, which are far ahead on large batches (N = 200,
 //     B = 4096, forward and backward: 7.4 against 10.5).  A slice of a batch has to reproduce its rows bit for bit and the two
 //     families sum in a different order, so batches of up to 512 rows run on teams that sum in the weight-resident order
@@ -128,9 +132,6 @@ static bool forced() {
 //     46 against 37, B = 6016: 49 against 54).  Rows reproduce between batches on the same side of this line: members of
 //     any width sum a row alike.
 // The rule does not ask whether a record is wanted: a history is the same with and without one.
-// Whether a workgroup per batch tile does it; RINGATTR_TEAM=1 asks for the exchange through L2.
-bool ring_uses_team_one(int N, int k) { return ring_team_one_applicable(N, k) && !forced(); }
-
 static bool team_shape(int N, int k, int T, int B) {
   if (ring_uses_team_one(N, k)) return true;
   if (ring_res256_applicable(N, k) && !forced()) return false;

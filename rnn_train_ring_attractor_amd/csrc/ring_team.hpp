@@ -519,7 +519,7 @@ __device__ __forceinline__ void team_compute_loop(const RingTeamArgs& c, const L
     int spins = 0;
     // Wide rings: the operand is nearly always there when several tiles share a team, and with the polling loop out of the
     // way the path straight on is shorter: N = 700, B = 500 11.55 -> 11.1 us per step forward and backward, N = 1024,
-    // B = 2048 51.2 -> 50.3.  Up to N = 512 it gains nothing (and N = 120, B = 64 loses 2 %).
+    // B = 2048 51.2 -> 50.3.  Up to N = 512 it gains nothing (and N = 120, B = 64 in teams of eight loses 2 %).
     if constexpr (KPW >= 3) {
       if (__builtin_expect(!dead && !op.ready(), 0)) {
         const unsigned at = (unsigned)slot * slot_bytes + (unsigned)(team + c.nteams * j) * tile_bytes;

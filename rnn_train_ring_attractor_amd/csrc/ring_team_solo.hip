@@ -232,7 +232,7 @@ hipError_t ring_launch_team_rebuild(const RingFwdArgs& a, const RingTeamArgs& c,
 // Forward and BPTT of the teams that did not gather, a workgroup per batch tile that goes through the team's members one
 // after the other.  The weights are read in fp32 from memory every step: tens of times slower than a team, and hardly
 // ever needed.  Workgroups of gathered teams leave at once: the launch and the wait for the members cost a call 3 to 4 us
-// (N = 256, B = 1, T = 100: 127 -> 130; N = 120, B = 64, T = 120, forward and backward: 238 -> 242).
+// (N = 256, B = 1, T = 100: 127 -> 130; N = 120, B = 64, T = 120 in teams of eight, forward and backward: 238 -> 242).
 // ------------------------------------------------------------------------------------------------
 namespace {
 
