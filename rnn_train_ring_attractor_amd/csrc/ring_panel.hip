@@ -18,6 +18,14 @@
 //     announced sums of all of its rows.  Nobody waits for one: what is not there yet is added up once more.  us per step with
 //     a launch for operand and sums before each step -> here: N = 2048, 16 channels, B = 256: 57.9 -> 55.8; B = 1: 34.1 -> 29.7;
 //     2 channels, B = 1: 11.4 -> 7.5; N = 2047, B = 16: 14.6 -> 8.9; N = 1500, 6 channels, B = 64: 15.0 -> 12.1.
+//   * Around the products everything that waits for memory or LDS waits once, not once per row: the gates are loaded together, the
+//     list of driven channels comes from sixteen channels at a time, a row tile's sum goes from wave to wave behind the tile
+//     before it (and stays in registers where a workgroup has one column tile), the previous state is on its way meanwhile, the
+//     announced row sums are asked for together.  At N = 2048, 16 channels, B = 256 these were 57 of the 130 thousand cycles of
+//     a step, the products 72 (now some 30 and 60; the weights alone take 22 us to read, 6.6 TB/s).  us per step, T = 20 with
+//     the packing launch: N = 2048, 16 channels, B = 256 66.2 -> 52.6, B = 1 35.2 -> 33.2; 12 channels, B = 1024 144 -> 111;
+//     2 channels, B = 1024 48.8 -> 42.0; N = 1100, 16 channels, B = 1024 133 -> 94; N = 700, 6 channels, B = 1024 36.7 -> 28.7;
+//     N = 1500, 6 channels, B = 64 14.4 -> 12.8.
 // us per step, ring_block.hip / ring_bign.hip -> here, T = 20 with the packing launch:
 //   N = 2048, 16 channels: B = 1: 120 -> 35   B = 256: 102 -> 63   B = 1024: 286 -> 181
 //   N = 2048,  2 channels: B = 16: 31 -> 9    B = 256:  35 -> 19   B = 1024:  73 -> 44
@@ -38,9 +46,16 @@ struct PanelPass {
   __amdgpu_buffer_rsrc_t x, w;        // operand fragments, packed weights
   unsigned wat[PANEL_NV];             // byte offset of the wave's virtual columns, chunk 0
   int mat[PANEL_NV], col[PANEL_NV];   // their matrix and column tile
-  const float* gl;       // gates [16 R][k]
-  float J1;
-  int KCH, k, nv, wv;
+  const float* gl;       // gates [1 + k][16 R + 4], those of matrix 0 all J1
+  int KCH, C, nv, wv;
+};
+
+// The previous state of the outputs a thread will form (four neurons of a row each): on its way while the products are summed,
+// then in LDS (where the operand was), in the thread's own places.
+template <int R>
+struct PanelPrev {
+  const float* prev;     // null: not behind this pass
+  int N, B, C, first_row, first_col, tid;
 };
 
 // A fragment per lane from a scalar byte offset.  (Buffer loads: every address but the lane's own 16 bytes is scalar, which
@@ -50,9 +65,10 @@ __device__ __forceinline__ bf16x8 panel_load(__amdgpu_buffer_rsrc_t r, unsigned 
 }
 
 // The products X_i @ W_v of a wave's NV virtual columns with all row tiles, then gates and the sum over the matrices in
-// their order, one wave after the other, into sums [C][R][64].
+// their order into sums [C][R][64]: a row tile goes from wave to wave, the next one a barrier behind it.  (All of a wave's tiles
+// before the next wave's took 28 of 136 thousand cycles at N = 2048, 16 channels, B = 256.)
 template <int R, int NV>
-__device__ __forceinline__ void panel_pass(const PanelPass& p, const unsigned (&xrow)[R], bf16x8* xs, f32x4* sums, int lane) {
+__device__ __forceinline__ void panel_pass(const PanelPass& p, const unsigned (&xrow)[R], bf16x8* xs, f32x4* sums, int lane, const PanelPrev<R>& was) {
   const int KCH = p.KCH, nst = KCH / PANEL_S, wv = p.wv;
   auto stage = [&](int buf, int i, int d) { return xs + ((buf * R + i) * PANEL_S + d) * 64 + lane; };
   f32x4 acc[NV][R];
@@ -118,26 +134,46 @@ __device__ __forceinline__ void panel_pass(const PanelPass& p, const unsigned (&
         __builtin_amdgcn_sched_barrier(0);
       }
     }
+  f32x4 prev[R];                         // (R C / 4 of them are used)
+  if (was.prev) {
+#pragma unroll
+    for (int n = 0; n < R; ++n) {
+      const int idx = was.tid + 256 * n, row = idx / (4 * was.C), j4 = 4 * (idx % (4 * was.C));
+      if (idx < R * 16 * 4 * was.C) prev[n] = load4_masked(was.prev, was.N, was.B, was.first_row + row, was.first_col + j4);
+    }
+  }
 #pragma unroll 1
-  for (int r = 0; r < 4; ++r) {
-    if (wv == r && p.nv > 0) {
+  for (int r = 0; r < wv; ++r) lds_barrier();
+#pragma unroll
+  for (int i = 0; i < R; ++i) {
+    if (p.nv > 0) {
+      f32x4 g[NV];
+#pragma unroll
+      for (int v = 0; v < NV; ++v) g[v] = *reinterpret_cast<const f32x4*>(p.gl + p.mat[v] * (16 * R + 4) + 16 * i + 4 * (lane >> 4));
+      f32x4* dst = sums + (p.col[0] * R + i) * 64 + lane;
+      f32x4 s = *dst;
 #pragma unroll
       for (int v = 0; v < NV; ++v) {
-        const int m = p.mat[v];
-#pragma unroll
-        for (int i = 0; i < R; ++i) {
-          f32x4* dst = sums + (p.col[v] * R + i) * 64 + lane;
-          f32x4 s = *dst;
-#pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            const float g = p.gl[(16 * i + 4 * (lane >> 4) + e) * p.k + (m > 0 ? m - 1 : 0)];
-            s[e] = fmaf(m > 0 ? g : p.J1, acc[v][i][e], s[e]);
-          }
+        if (v > 0 && p.C > 1) {                           // (with one column tile the sum stays in registers)
           *dst = s;
+          dst = sums + (p.col[v] * R + i) * 64 + lane;
+          s = *dst;
         }
+#pragma unroll
+        for (int e = 0; e < 4; ++e) s[e] = fmaf(g[v][e], acc[v][i][e], s[e]);
       }
+      *dst = s;
     }
     lds_barrier();
+  }
+#pragma unroll 1
+  for (int r = wv; r < 3; ++r) lds_barrier();
+  if (was.prev) {
+#pragma unroll
+    for (int n = 0; n < R; ++n) {
+      const int idx = was.tid + 256 * n;
+      if (idx < R * 16 * 4 * was.C) reinterpret_cast<f32x4*>(xs)[idx] = prev[n];
+    }
   }
 }
 
@@ -249,7 +285,8 @@ __global__ __launch_bounds__(256) void ring_panel_fwd_kernel(RingFwdArgs p, Pane
   const int N = p.N, B = p.B, T = p.T, k = p.k, KCH = 2 * NC;
   bf16x8* const xs = reinterpret_cast<bf16x8*>(panel_lds);                                  // [2][R][PANEL_S][64]
   f32x4* const sums = reinterpret_cast<f32x4*>(xs + (size_t)2 * R * PANEL_S * 64);          // [C][R][64]
-  float* const gl = reinterpret_cast<float*>(sums + (size_t)C * R * 64);                    // [16 R][k]
+  float* const gl = reinterpret_cast<float*>(sums + (size_t)C * R * 64);                    // [1 + k][16 R + 4]
+  constexpr int GS = 16 * R + 4;
   int rg, cb;
   step_block_coords(xcd_map, rg, cb);
   const int bt0 = rg * R;
@@ -269,10 +306,21 @@ __global__ __launch_bounds__(256) void ring_panel_fwd_kernel(RingFwdArgs p, Pane
     else own_sum = panel_row_sum(own_fours, N, tid & 15);
   }
 
-  for (int idx = tid; idx < R * 16 * k; idx += 256) {
-    const int row = idx / k, c = idx - row * k, b = 16 * bt0 + row;
-    gl[idx] = b < B ? p.A[((size_t)b * T + t) * k + c] : 0.f;
+  // (R loads on their way at a time: memory is busy with other workgroups' weights, and a load takes long)
+  for (int idx0 = tid; idx0 < R * 16 * k; idx0 += 256 * R) {
+    float g[R];
+#pragma unroll
+    for (int n = 0; n < R; ++n) {
+      const int idx = idx0 + 256 * n, row = idx / k, c = idx - row * k, b = 16 * bt0 + row;
+      g[n] = p.A[((size_t)(idx < R * 16 * k && b < B ? b : 0) * T + t) * k + c];
+    }
+#pragma unroll
+    for (int n = 0; n < R; ++n) {
+      const int idx = idx0 + 256 * n, row = idx / k, c = idx - row * k;
+      if (idx < R * 16 * k) gl[(1 + c) * GS + row] = 16 * bt0 + row < B ? g[n] : 0.f;
+    }
   }
+  for (int i = tid; i < 16 * R; i += 256) gl[i] = p.J1;
   for (int i = tid; i < C * R * 64; i += 256) sums[i] = f32x4{0.f, 0.f, 0.f, 0.f};
   if (sums_row) {
     if constexpr (EARLY) {
@@ -286,25 +334,22 @@ __global__ __launch_bounds__(256) void ring_panel_fwd_kernel(RingFwdArgs p, Pane
   }
   lds_barrier();
   // matrices worth multiplying: Wo, and the channels that are not zero in all of the workgroup's rows
+  // (four lanes a channel, sixteen channels at once)
   int nact = 1;
-  {
-    unsigned long long m = 0;
-    for (int c0 = 0; c0 < k; c0 += 4) {
-      const int c = c0 + (lane >> 4);
-      bool nz = false;
+  if (tid == 0) list[0] = 0;
+  for (int c0 = 0; c0 < k; c0 += 16) {
+    const int c = c0 + (lane >> 2);
+    bool nz = false;
 #pragma unroll
-      for (int i = 0; i < R; ++i) nz |= c < k && gl[(16 * i + (lane & 15)) * k + (c < k ? c : 0)] != 0.f;
-      const unsigned long long bal = __ballot(nz);
-#pragma unroll
-      for (int j = 0; j < 4; ++j)
-        if ((bal >> (16 * j)) & 0xffffull) m |= 1ull << (c0 + j);
+    for (int i = 0; i < R; ++i) {
+      const f32x4 v = *reinterpret_cast<const f32x4*>(gl + (1 + (c < k ? c : 0)) * GS + 16 * i + 4 * (lane & 3));
+      nz |= v[0] != 0.f || v[1] != 0.f || v[2] != 0.f || v[3] != 0.f;
     }
-    if (tid == 0) list[0] = 0;
-    for (int c = 0; c < k; ++c)
-      if ((m >> c) & 1ull) {
-        if (tid == 0) list[nact] = c + 1;
-        ++nact;
-      }
+    unsigned long long any = __ballot(nz && c < k);
+    any |= any >> 1;
+    any = (any | any >> 2) & 0x1111111111111111ull;        // a bit per channel, that of its first lane
+    if (wv == 0 && (any >> lane) & 1) list[nact + __popcll(any & ((1ull << lane) - 1))] = c + 1;
+    nact += __popcll(any);
   }
   nact = __builtin_amdgcn_readfirstlane(nact);
   lds_barrier();
@@ -316,29 +361,35 @@ __global__ __launch_bounds__(256) void ring_panel_fwd_kernel(RingFwdArgs p, Pane
   ps.x = __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16x8*>(xfrag), 0, (int)((unsigned)p.nbt * (unsigned)KCH * 1024u), 0x00020000);
   ps.w = __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p.Wpack), 0, (int)((unsigned)(k + 1) * 4u * NC * KCH * 1024u), 0x00020000);
   ps.gl = gl;
-  ps.J1 = p.J1;
+  ps.C = C;
   ps.KCH = KCH;
-  ps.k = k;
   ps.wv = wv;
-  const int per_pass = (4 * PANEL_NV) / C;                // matrices per pass over the contraction
+  const int cs = C == 4 ? 2 : C - 1;                      // C is 1, 2 or 4
+  const int per_pass = (4 * PANEL_NV) >> cs;              // matrices per pass over the contraction
+  const float* const prev = t == 0 ? p.r_init : p.hist + (size_t)(t - 1) * B * N;
+  PanelPrev<R> was{nullptr, N, B, C, 16 * bt0, 16 * C * cb, tid};
   for (int m0 = 0; m0 < nact; m0 += per_pass) {
-    const int nm = nact - m0 < per_pass ? nact - m0 : per_pass, V = nm * C;
+    const int nm = nact - m0 < per_pass ? nact - m0 : per_pass, V = nm << cs;
     const int v0 = wv * V / 4;
     ps.nv = (wv + 1) * V / 4 - v0;                        // this wave's run; matrices ascending
+    int mats[PANEL_NV];
+#pragma unroll
+    for (int v = 0; v < PANEL_NV; ++v) mats[v] = list[m0 + ((v < ps.nv ? v0 + v : (ps.nv > 0 ? v0 : 0)) >> cs)];
 #pragma unroll
     for (int v = 0; v < PANEL_NV; ++v) {
       const int u = v < ps.nv ? v0 + v : (ps.nv > 0 ? v0 : 0);
-      ps.mat[v] = __builtin_amdgcn_readfirstlane(list[m0 + u / C]);
-      ps.col[v] = u % C;
+      ps.mat[v] = __builtin_amdgcn_readfirstlane(mats[v]);
+      ps.col[v] = u & (C - 1);
       ps.wat[v] = ((unsigned)ps.mat[v] * 4u * NC + (unsigned)(cb * C + ps.col[v])) * (unsigned)KCH * 1024u;
     }
+    was.prev = m0 + per_pass >= nact ? prev : nullptr;
     // (every variant passes the same number of barriers; a wave without a column of its own helps with the staging)
     switch (ps.nv) {
-      case 5: panel_pass<R, 5>(ps, xrow, xs, sums, lane); break;
-      case 4: panel_pass<R, 4>(ps, xrow, xs, sums, lane); break;
-      case 3: panel_pass<R, 3>(ps, xrow, xs, sums, lane); break;
-      case 2: panel_pass<R, 2>(ps, xrow, xs, sums, lane); break;
-      default: panel_pass<R, 1>(ps, xrow, xs, sums, lane); break;
+      case 5: panel_pass<R, 5>(ps, xrow, xs, sums, lane, was); break;
+      case 4: panel_pass<R, 4>(ps, xrow, xs, sums, lane, was); break;
+      case 3: panel_pass<R, 3>(ps, xrow, xs, sums, lane, was); break;
+      case 2: panel_pass<R, 2>(ps, xrow, xs, sums, lane, was); break;
+      default: panel_pass<R, 1>(ps, xrow, xs, sums, lane, was); break;
     }
   }
 
@@ -346,10 +397,17 @@ __global__ __launch_bounds__(256) void ring_panel_fwd_kernel(RingFwdArgs p, Pane
   int now = t, me = tid;
   if constexpr (CARRY) {
     asm volatile("" : "+s"(now), "+v"(me));
-    for (int row = me >> 4; row < 16 * R; row += 16) {
-      const int b = 16 * bt0 + row, sub = me & 15;
+    float rs[R];
+#pragma unroll
+    for (int n = 0; n < R; ++n) {
+      const int b = 16 * bt0 + (me >> 4) + 16 * n;
+      rs[n] = __hip_atomic_load(state.rs[now % 3] + (b < B ? b : 0), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+#pragma unroll
+    for (int n = 0; n < R; ++n) {
+      const int row = (me >> 4) + 16 * n, b = 16 * bt0 + row, sub = me & 15;
       if (b >= B) break;
-      float s = __hip_atomic_load(state.rs[now % 3] + b, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      float s = rs[n];
       if (__builtin_bit_cast(unsigned, s) == PANEL_EMPTY)                      // (the same in the row's 16 lanes)
         s = panel_row_sum(state.fours[now & 1] + (size_t)b * (16 * NC), N, sub);
       if (sub == 0) row_sums[row] = s;
@@ -358,20 +416,22 @@ __global__ __launch_bounds__(256) void ring_panel_fwd_kernel(RingFwdArgs p, Pane
   }
 
   // activation and leak; a thread takes four consecutive neurons of a row
-  const float* prev = (now == 0) ? p.r_init : p.hist + (size_t)(now - 1) * B * N;
   float* out = p.hist + (size_t)now * B * N;
   const float oma = 1.f - p.alpha;
   const float* sf = reinterpret_cast<const float*>(sums);
-  for (int idx = me; idx < R * 16 * 4 * C; idx += 256) {
-    const int row = idx / (4 * C), j4 = 4 * (idx % (4 * C)), cc = j4 >> 4, n = j4 & 15;
+#pragma unroll
+  for (int n = 0; n < R; ++n) {
+    const int idx = me + 256 * n;
+    if (idx >= R * 16 * 4 * C) break;
+    const int row = idx / (4 * C), j4 = 4 * (idx % (4 * C)), cc = j4 >> 4, nn = j4 & 15;
     const int b = 16 * bt0 + row, j = 16 * C * cb + j4, i = row >> 4;
     if (b >= B || j >= N) continue;
-    const f32x4 rp = load4_masked(prev, N, B, b, j);
+    const f32x4 rp = reinterpret_cast<const f32x4*>(xs)[idx];
     const float js = p.J0 * (CARRY ? row_sums[row] : state.rs[0][b]);
     f32x4 rn;
 #pragma unroll
     for (int x = 0; x < 4; ++x) {
-      const float s = sf[((size_t)(cc * R + i) * 64 + ((row & 15) >> 2) * 16 + n + x) * 4 + (row & 3)];
+      const float s = sf[((size_t)(cc * R + i) * 64 + ((row & 15) >> 2) * 16 + nn + x) * 4 + (row & 3)];
       float F, D;
       act_fast<ACT>(s + js, F, D);
       rn[x] = fmaf(p.alpha, F, oma * rp[x]);
@@ -390,7 +450,7 @@ __global__ __launch_bounds__(256) void ring_panel_fwd_kernel(RingFwdArgs p, Pane
 // Launchers
 // ------------------------------------------------------------------------------------------------
 static size_t panel_lds_bytes(int R, int C, int k) {
-  return (size_t)2 * R * PANEL_S * 1024 + (size_t)C * R * 1024 + (size_t)R * 16 * k * sizeof(float);
+  return (size_t)2 * R * PANEL_S * 1024 + (size_t)C * R * 1024 + (size_t)(R * 16 + 4) * (k + 1) * sizeof(float);
 }
 
 // Row tiles and column tiles of a workgroup.  Per K chunk a workgroup needs the longer of its matrix-pipe time
