@@ -1361,6 +1361,10 @@ hipError_t ring_run_team_fwd(const RingFwdArgs& a, const float* Wo, const float*
   ProfScope prof(1, st);
   return ring_team_fwd(a, Wo, Wa, folded, cts, ws, st);
 }
+hipError_t ring_run_chip_fwd(const RingFwdArgs& a, const float* Wo, const float* Wa, void* ws, hipStream_t st) {
+  ProfScope prof(1, st);
+  return ring_chip_fwd(a, Wo, Wa, ws, st);
+}
 hipError_t ring_run_team_rows(const RingFwdArgs& a, const float* Wo, const float* Wa, void* ws, hipStream_t st) {
   ProfScope prof(1, st);
   return ring_team_rows(a, Wo, Wa, ws, st);

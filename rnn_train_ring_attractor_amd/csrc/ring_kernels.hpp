@@ -126,7 +126,14 @@ bool ring_uses_step_kernels(int N, int k, int NC, int nbt);
 bool ring_panel_applicable(int NC, int k);
 bool ring_uses_panel(int k, int NC, int nbt);
 size_t ring_panel_workspace_bytes(int NC, int nbt);
+float ring_panel_step_cycles(int NC, int nbt, int k);
 hipError_t ring_launch_panel_fwd(const RingFwdArgs& a, int NC, hipStream_t st);
+
+// Forward without a saved record on all compute units at once, the weights on chip, wide rings (ring_chip.hip).
+bool ring_uses_chip(int N, int k, int T, int B);
+size_t ring_chip_bytes(int N, int k, int T, int B);       // scratch of one launch (0 where no call of this shape comes here)
+hipError_t ring_chip_fwd(const RingFwdArgs& a, const float* Wo, const float* Wa, void* ws, hipStream_t st);
+hipError_t ring_run_chip_fwd(const RingFwdArgs& a, const float* Wo, const float* Wa, void* ws, hipStream_t st);
 
 // LDS-tiled weight-gradient contraction for NC in {2, 4, 8, 16, 24, 32} (ring_dw.hip); NC = 2 not for short contractions with many
 // channels.
@@ -272,6 +279,9 @@ struct RingTeamPlan {
   float step_cycles;     // what the cost model expects of one time step
 };
 RingTeamPlan ring_team_plan(int N, int k, int T, int B, bool bptt, bool ga);
+bool ring_teams_allowed();                                // the device has the compute units, no switch and no earlier failure forbids it
+void ring_team_limits(int* spin_max, int* gather_ticks);
+hipError_t ring_team_fill(void* ws, size_t xchg_bytes, size_t gather_bytes, hipStream_t st);   // exchange area empty, the words behind it zero
 bool ring_uses_team(int N, int k, int T, int B);
 size_t ring_team_fwd_bytes(int N, int k, int T, int B);   // scratch of one launch (0 where teams do not apply)
 size_t ring_team_bptt_bytes(int N, int k, int T, int B, bool ga);

@@ -460,8 +460,8 @@ static size_t panel_lds_bytes(int R, int C, int k) {
 // a launch for the operand of 5 us in each:
 //   16 channels, B = 256:  (8,1) 64  (4,1) 71  (4,2) 66  (8,2) 98      B = 1:  (1,1) 39  (4,1) 45  (8,1) 57
 //   16 channels, B = 1024: (8,1) 208 (8,2) 195 (8,4) 189               2 channels, B = 256:  (4,2) 22  (8,1) 27  (8,4) 43
-static void panel_shape(int NC, int nbt, int k, int* R_out, int* C_out) {
-  float best = 0.f;
+static float panel_shape(int NC, int nbt, int k, int* R_out, int* C_out) {
+  float best = 0.f, step = 0.f;
   for (int R = 1; R <= 8; R *= 2)
     for (int C = 1; C <= 4; C *= 2) {
       const int V = (k + 1) * C;
@@ -475,8 +475,17 @@ static void panel_shape(int NC, int nbt, int k, int* R_out, int* C_out) {
         best = cost;
         *R_out = R;
         *C_out = C;
+        step = 0.72f * 2.f * NC * cost + (float)(rounds * passes * (R - 4)) * 2500.f + 14300.f;
       }
     }
+  return step;
+}
+
+// Cycles of a step at 2.4 GHz, launch included, as fitted to 165 measured shapes (N = 640 to 2048, 2 to 16 channels, B = 4 to 1024:
+// mean deviation 8 %, largest 27 %).
+float ring_panel_step_cycles(int NC, int nbt, int k) {
+  int R, C;
+  return panel_shape(NC, nbt, k, &R, &C);
 }
 
 bool ring_panel_applicable(int NC, int k) { return NC >= 16 && NC % 8 == 0 && k <= BN_GATE_KMAX; }

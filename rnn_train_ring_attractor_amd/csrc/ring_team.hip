@@ -140,7 +140,7 @@ static bool team_shape(int N, int k, int T, int B) {
   return forced() || N > 512 || f.nt <= 8;
 }
 
-static bool teams_allowed() {
+bool ring_teams_allowed() {
   const char* v = getenv("RINGATTR_TEAM");
   if ((v && v[0] == '0') || ring_cluster_error()) return false;
   // a switch that asks for one of the other families by name is obeyed
@@ -150,11 +150,11 @@ static bool teams_allowed() {
   return device_cus() == XCDS * CUS_PER_XCD;
 }
 
-bool ring_uses_team(int N, int k, int T, int B) { return teams_allowed() && team_shape(N, k, T, B); }
+bool ring_uses_team(int N, int k, int T, int B) { return ring_teams_allowed() && team_shape(N, k, T, B); }
 
 // Same bits and record as the weight-resident kernels, so the batch may decide: wherever every batch tile gets a team.
 bool ring_uses_team_rows(int N, int k, int B, bool record) {
-  return !forced() && teams_allowed() && ring_uses_resident(N, k) && ring_team_rows_plan(N, k, B, record).ok;
+  return !forced() && ring_teams_allowed() && ring_uses_resident(N, k) && ring_team_rows_plan(N, k, B, record).ok;
 }
 size_t ring_team_rows_bytes(int N, int k, int B, bool record) {
   const RingTeamPlan p = ring_team_rows_plan(N, k, B, record);
@@ -172,6 +172,27 @@ static size_t plan_bytes(int N, int k, int T, int B, bool bptt, bool ga) {
 }
 size_t ring_team_fwd_bytes(int N, int k, int T, int B) { return plan_bytes(N, k, T, B, false, false); }
 size_t ring_team_bptt_bytes(int N, int k, int T, int B, bool ga) { return plan_bytes(N, k, T, B, true, ga); }
+
+// How long a wait inside the time loop polls, and how long members wait for each other before it (RingTeamArgs).
+void ring_team_limits(int* spin_max, int* gather_ticks) {
+  *spin_max = 16000000;   // some seconds of polling
+  if (const char* v = getenv("RINGATTR_CLUSTER_SPIN")) {
+    const long s = atol(v);
+    if (s >= -1 && s <= 100000000L) *spin_max = (int)s;
+  }
+  // A team whose compute units are busy waits about as long as the way round it takes (some 50 ms at N = 1024, T = 120).
+  *gather_ticks = 5000000;
+  if (const char* v = getenv("RINGATTR_TEAM_GATHER_US")) {
+    const long us = atol(v);
+    if (us >= -1 && us <= 10000000L) *gather_ticks = us < 0 ? -1 : (int)us * 100;
+  }
+}
+
+hipError_t ring_team_fill(void* ws, size_t xchg_bytes, size_t gather_bytes, hipStream_t st) {
+  const unsigned nx = (unsigned)(xchg_bytes / 16), n = (unsigned)((xchg_bytes + gather_bytes) / 16);
+  hipLaunchKernelGGL(ring_team_fill_kernel, dim3(std::min(1024u, (n + 255) / 256)), dim3(256), 0, st, reinterpret_cast<u32x4*>(ws), nx, n);
+  return hipGetLastError();
+}
 
 static hipError_t team_args(const RingTeamPlan& p, const float* Wo, const float* Wa, const float* A, float J0, float J1,
                             bool folded, int N, int k, int T, int B, int cts, void* ws, RingTeamArgs& c,
@@ -200,24 +221,12 @@ static hipError_t team_args(const RingTeamPlan& p, const float* Wo, const float*
   c.nt = p.nt;
   c.slots = p.slots;
   c.cts = cts;
-  c.spin_max = 16000000;   // some seconds of polling
-  if (const char* v = getenv("RINGATTR_CLUSTER_SPIN")) {
-    const long s = atol(v);
-    if (s >= -1 && s <= 100000000L) c.spin_max = (int)s;
-  }
-  // A team whose compute units are busy waits about as long as the way round it takes (some 50 ms at N = 1024, T = 120).
-  c.gather_ticks = 5000000;
-  if (const char* v = getenv("RINGATTR_TEAM_GATHER_US")) {
-    const long us = atol(v);
-    if (us >= -1 && us <= 10000000L) c.gather_ticks = us < 0 ? -1 : (int)us * 100;
-  }
+  ring_team_limits(&c.spin_max, &c.gather_ticks);
   c.c16 = p.shape.c16;
   c.mr = p.shape.mr;
   c.wk = p.shape.wk;
   c.rows = 0;
-  const unsigned nx = (unsigned)(p.xchg_bytes / 16), n = (unsigned)((p.xchg_bytes + p.gather_bytes) / 16);
-  hipLaunchKernelGGL(ring_team_fill_kernel, dim3(std::min(1024u, (n + 255) / 256)), dim3(256), 0, st, reinterpret_cast<u32x4*>(ws), nx, n);
-  return hipGetLastError();
+  return ring_team_fill(ws, p.xchg_bytes, p.gather_bytes, st);
 }
 
 // (the fields that a workgroup on its own needs)

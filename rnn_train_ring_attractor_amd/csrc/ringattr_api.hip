@@ -182,7 +182,7 @@ size_t ringattr_fwd_workspace_bytes(int N, int a_dim, int seq_len, int batch_siz
   // (with a record and without one: narrower rings have teams for more rows without one)
   size_t most = packed;
   for (const size_t other : {ring_team_fwd_bytes(N, a_dim, seq_len, batch_size), ring_team_rows_bytes(N, a_dim, batch_size, true),
-                             ring_team_rows_bytes(N, a_dim, batch_size, false)})
+                             ring_team_rows_bytes(N, a_dim, batch_size, false), ring_chip_bytes(N, a_dim, seq_len, batch_size)})
     most = other > most ? other : most;
   return most;
 }
@@ -331,6 +331,14 @@ static int fwd_impl(const void* A, const void* Wa, float J0, float J1, const voi
     if (stats_done) *stats_done = loss_stats != nullptr;
     const hipError_t e = ring_run_team_rows(a, (const float*)Wo, (const float*)Wa, workspace, st);
     if (e != hipSuccess) return hip_fail(e, "team forward launch");
+    return RINGATTR_OK;
+  }
+
+  if (!saved && ring_uses_chip(N, a_dim, seq_len, batch_size) && workspace_bytes >= ring_chip_bytes(N, a_dim, seq_len, batch_size)) {
+    RingFwdArgs a = fwd_args(A, nullptr, r_init, bump_history, nullptr, g, J0, J1, alpha, activation_type);
+    if (stats_done) *stats_done = false;
+    const hipError_t e = ring_run_chip_fwd(a, (const float*)Wo, (const float*)Wa, workspace, st);
+    if (e != hipSuccess) return hip_fail(e, "chip forward launch");
     return RINGATTR_OK;
   }
 

@@ -1,0 +1,127 @@
+"""GPU tests of the chip kernels (forward without a record of wide rings, the weights on chip across all compute units):
+the fp64 oracle, the same bits whatever the members' width, from single workgroups where a row group does not gather, in any
+batch and in replayed graphs, and the rule that takes calls there."""
+import numpy as np
+import pytest
+import torch
+
+from oracle import ring_oracle as O
+from tests.ring_cases import make_problem
+
+pytestmark = pytest.mark.gpu
+
+SWITCHES = ("RINGATTR_CHIP", "RINGATTR_TEAM", "RINGATTR_TEAM_GATHER_US", "RINGATTR_PANEL", "RINGATTR_PANEL_SHAPE", "RINGATTR_BLOCK", "RINGATTR_WIDE",
+            "RINGATTR_BLOCK_SHAPE", "RINGATTR_STREAMING", "RINGATTR_CLUSTER")
+
+
+@pytest.fixture(autouse=True)
+def no_switches(monkeypatch):
+    for name in SWITCHES:
+        monkeypatch.delenv(name, raising=False)
+
+
+def _tensors(p, dev):
+    return [torch.as_tensor(p[x], dtype=torch.float32, device=dev) for x in ("A", "Wa", "Wo", "r0")]
+
+
+def _forward(t, act, J0, J1):
+    from rnn_train_ring_attractor_amd import _lib, ring_rnn_cuda_func
+    A, Wa, Wo, r0 = t
+    with torch.no_grad():
+        h = ring_rnn_cuda_func(A, Wa, J0, J1, Wo, r0, 0.15, act)
+    return h, _lib.last_kernel_names()["fwd"]
+
+
+# rows: one, a whole tile, ragged, one to many tiles per row group, more groups than tiles; neurons: the fewest, K chunks that
+# are not whole, one past a wave's share of them (769, 1025, 1537), no multiple of four, the most; channels: one, an even and
+# an odd number of matrices, more than fit the registers, sixteen, a silent one; more steps than slots
+@pytest.mark.parametrize("B,T,k,N,act", [
+    (1, 3, 7, 513, "relu"), (9, 3, 1, 1200, "tanh"), (16, 12, 5, 640, "gelu"), (100, 6, 16, 700, "silu"), (33, 9, 6, 769, "tanh"), (7, 2, 12, 1023, "gelu"),
+    (40, 10, 16, 1024, "tanh"), (300, 5, 3, 1025, "gelu"), (50, 4, 2, 1300, "silu"), (20, 9, 16, 1536, "gelu"), (130, 3, 7, 1537, "relu"),
+    (17, 1, 2, 2047, "tanh"), (64, 9, 13, 2048, "silu"), (1, 20, 3, 2048, "gelu"),
+])
+def test_chip_kernels_against_the_oracle(B, T, k, N, act, gpu_device, monkeypatch):
+    print(f"[case] chip B={B} T={T} k={k} N={N} {act}", flush=True)
+    J0, J1 = -1.0 / N, 0.5
+    p = make_problem(11, B, T, k, N, bump="vm", action="dense")
+    if k > 2:
+        p["A"][:, :, 1] = 0.0
+    t = _tensors(p, gpu_device)
+    ref, _ = O.forward_dense(p["A"], p["Wa"], J0, J1, p["Wo"], p["r0"], 0.15, act)
+    ran = {}
+    for width in ("1", "8", "16", "32"):                 # (1: the rule's own choice)
+        monkeypatch.setenv("RINGATTR_CHIP", width)
+        h, name = _forward(t, act, J0, J1)
+        if "chip" in name:
+            ran[width] = h
+    assert "1" in ran and len(ran) >= 2                  # not every width has room for every number of channels
+    got = ran["1"]
+    assert O.max_rel_err(got.cpu().numpy(), ref) <= 1e-2 # one bf16 rounding per operand, as everywhere
+    assert all(torch.equal(got, h) for h in ran.values())
+    monkeypatch.setenv("RINGATTR_TEAM_GATHER_US", "-1")  # no group gathers: a workgroup per tile
+    for width in ran:
+        monkeypatch.setenv("RINGATTR_CHIP", width)
+        h, _ = _forward(t, act, J0, J1)
+        assert torch.equal(got, h)
+    monkeypatch.delenv("RINGATTR_TEAM_GATHER_US")
+    monkeypatch.setenv("RINGATTR_CHIP", "1")
+    rows = slice(B // 2, B)                              # the same rows in another batch
+    h, name = _forward([t[0][rows].clone(), t[1], t[2], t[3][rows].clone()], act, J0, J1)
+    assert "chip" in name and torch.equal(h, got[:, rows])
+
+
+def test_infinite_states_and_absent_matrices(gpu_device, monkeypatch):
+    """Column tiles hold an even number of matrices; the one that is not there takes nothing from an infinite state."""
+    monkeypatch.setenv("RINGATTR_CHIP", "8")
+    B, T, k, N = 5, 4, 2, 1100
+    p = make_problem(12, B, T, k, N, bump="vm", action="dense")
+    p["Wo"], p["Wa"] = np.abs(p["Wo"]), np.abs(p["Wa"])
+    p["A"] = np.abs(p["A"]) + 0.1
+    p["r0"][2] = np.inf
+    h, name = _forward(_tensors(p, gpu_device), "relu", 0.0, 1.0)
+    assert "chip" in name
+    assert torch.isinf(h[:, 2]).all() and torch.isfinite(h[:, [0, 1, 3, 4]]).all()
+
+
+def test_slots_come_round_many_times(gpu_device, monkeypatch):
+    """Hundreds of rounds through the exchange slots with one, two and many tiles per group: the same bits as without any."""
+    for B, k, N, width in ((16, 3, 1100, "8"), (32, 3, 1100, "16"), (64, 3, 1100, "16"), (100, 16, 1024, "8"), (256, 2, 2048, "32")):
+        print(f"[case] chip rounds B={B} k={k} N={N} width {width}", flush=True)
+        t = _tensors(make_problem(13, B, 150, k, N, bump="vm", action="dense"), gpu_device)
+        monkeypatch.setenv("RINGATTR_CHIP", width)
+        h, name = _forward(t, "tanh", -1.0 / N, 0.9)
+        assert "chip" in name
+        monkeypatch.setenv("RINGATTR_CHIP", "8")         # the same rows a few at a time: other numbers of tiles and slots
+        part, name = _forward([t[0][:9].clone(), t[1], t[2], t[3][:9].clone()], "tanh", -1.0 / N, 0.9)
+        assert "chip" in name and torch.equal(part, h[:, :9])
+
+
+def test_replayed_graph(gpu_device):
+    B, T, k, N = 20, 12, 6, 1024
+    t = _tensors(make_problem(14, B, T, k, N, bump="vm", action="dense"), gpu_device)
+    want, name = _forward(t, "gelu", -1.0 / N, 0.9)
+    assert "chip" in name
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        _forward(t, "gelu", -1.0 / N, 0.9)
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=side):
+            out, _ = _forward(t, "gelu", -1.0 / N, 0.9)
+    torch.cuda.current_stream().wait_stream(side)
+    scale = 1.0
+    for _ in range(3):
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, want)
+        scale *= 0.5
+        t[3].mul_(scale)
+        want, _ = _forward(t, "gelu", -1.0 / N, 0.9)
+
+
+def test_rule(gpu_device):
+    """Few steps, narrow rings and batches that fill the chip stay where they were."""
+    for B, T, k, N, chip in ((1, 12, 6, 1024, True), (1, 9, 6, 1024, False), (1, 12, 2, 1024, False), (64, 12, 2, 1100, True), (1, 12, 17, 1100, False),
+                             (256, 12, 16, 2048, False), (1, 12, 6, 512, False)):
+        _, name = _forward(_tensors(make_problem(15, B, T, k, N, bump="vm", action="dense"), gpu_device), "relu", 0.0, 0.5)
+        assert ("chip" in name) == chip, (B, T, k, N, name)
