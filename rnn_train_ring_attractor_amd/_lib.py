@@ -154,6 +154,31 @@ def profile_read():
     return {KERNEL_NAMES[i]: (ms[i], cnt[i]) for i in range(n)}
 
 
+class _Here:
+    def __enter__(self):
+        return None
+
+    def __exit__(self, *exc):
+        return False
+
+
+_HERE = _Here()
+
+
+def on_device(device):
+    """`torch.cuda.device(device)` for a tensor's device; nothing to enter and leave where it is the current one."""
+    return _HERE if torch.cuda.current_device() == device.index else torch.cuda.device(device)
+
+
+def stream_handle(device) -> int:
+    """The current stream of a tensor's device, as the library takes it.  (Without the Stream object around it, where torch
+    still has that private name.)"""
+    try:
+        return torch._C._cuda_getCurrentRawStream(device.index)
+    except AttributeError:
+        return torch.cuda.current_stream(device).cuda_stream
+
+
 def plain_gpu_tensor(t) -> bool:
     """Whether a helper may hand t's memory to a kernel in place of a chain of torch operations: an fp32 GPU tensor that no
     derivative is wanted of, and nothing that watches or transforms the operations (autograd, forward mode, functorch,

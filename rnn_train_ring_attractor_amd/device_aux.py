@@ -96,8 +96,8 @@ class FusedClipAdam:
         n = len(self.params)
         ptrs = lambda ts: (ctypes.c_void_p * n)(*[t.data_ptr() for t in ts])
         dev = self.params[0].device
-        with torch.cuda.device(dev), torch.no_grad():
-            lib, stream = _lib.load(), torch.cuda.current_stream(dev).cuda_stream
+        with _lib.on_device(dev):
+            lib, stream = _lib.load(), _lib.stream_handle(dev)
             common = (n, ptrs(self.params), ptrs(grads), ptrs(self.exp_avg), ptrs(self.exp_avg_sq), self._numel, self.lr,
                       self.betas[0], self.betas[1], self.eps, self.max_norm)
             if self.step_counter is not None:

@@ -50,9 +50,9 @@ class RingGainFunc(Function):
         _check("params", prm, (k, 3 * h + 1))
         lib = _lib.load()
         out = torch.empty_like(x)
-        with torch.cuda.device(x.device):
+        with _lib.on_device(x.device):
             _lib.check(lib.ringattr_gain_fwd(x.data_ptr(), prm.data_ptr(), out.data_ptr(), k, h, T, B,
-                                             torch.cuda.current_stream(x.device).cuda_stream))
+                                             _lib.stream_handle(x.device)))
         ctx.save_for_backward(x, prm)
         ctx.dims = (B, T, k, h)
         return out
@@ -65,14 +65,14 @@ class RingGainFunc(Function):
         g = grad_out.contiguous()
         grad_prm = torch.empty_like(prm)
         grad_x = torch.empty_like(x) if ctx.needs_input_grad[0] else None
-        with torch.cuda.device(x.device):
+        with _lib.on_device(x.device):
             nbytes = lib.ringattr_gain_workspace_bytes(k, h, T, B)
             if nbytes == 0:
                 _lib.check(1)
             ws = torch.empty(nbytes, dtype=torch.uint8, device=x.device)
             _lib.check(lib.ringattr_gain_bwd(x.data_ptr(), prm.data_ptr(), g.data_ptr(), grad_prm.data_ptr(),
                                              grad_x.data_ptr() if grad_x is not None else None, k, h, T, B,
-                                             ws.data_ptr(), nbytes, torch.cuda.current_stream(x.device).cuda_stream))
+                                             ws.data_ptr(), nbytes, _lib.stream_handle(x.device)))
         return grad_x, grad_prm
 
 
@@ -97,10 +97,10 @@ class RingGainNetsFunc(Function):
         if any(ctx.needs_input_grad):
             kept = torch.empty(k * (3 * h + 1) + (B * T if halves else 0), dtype=signal.dtype, device=signal.device)
             ctx.save_for_backward(kept, None if halves else signal)
-        with torch.cuda.device(signal.device):
+        with _lib.on_device(signal.device):
             _lib.check(_lib.load().ringattr_gain_nets_fwd_kept(signal.data_ptr(), int(halves), _pointers([p.data_ptr() for p in params]),
                                                                out.data_ptr(), kept.data_ptr() if kept is not None else None, k, h, T, B,
-                                                               torch.cuda.current_stream(signal.device).cuda_stream))
+                                                               _lib.stream_handle(signal.device)))
         return out
 
     @staticmethod
@@ -113,13 +113,13 @@ class RingGainNetsFunc(Function):
         at = kept.data_ptr()
         nets = _pointers([at + 4 * (c * (3 * h + 1) + part * h) for c in range(k) for part in range(4)])
         x = at + 4 * k * (3 * h + 1) if halves else signal.data_ptr()
-        with torch.cuda.device(kept.device):
+        with _lib.on_device(kept.device):
             nbytes = lib.ringattr_gain_workspace_bytes(k, h, T, B)
             if nbytes == 0:
                 _lib.check(1)
             ws = torch.empty(nbytes, dtype=torch.uint8, device=kept.device)
             _lib.check(lib.ringattr_gain_nets_bwd(x, int(halves), nets, g.data_ptr(), grad.data_ptr(), k, h, T, B, ws.data_ptr(), nbytes,
-                                                  torch.cuda.current_stream(kept.device).cuda_stream))
+                                                  _lib.stream_handle(kept.device)))
         parts = list(grad.view(-1).split((h, h, h, 1) * k))
         for c in range(0, 4 * k, 4):
             parts[c], parts[c + 2] = parts[c].view(h, 1), parts[c + 2].view(1, h)
@@ -134,12 +134,12 @@ def _net_parameters(nets, signal):
     """The parameter tensors as RingGainNetsFunc takes them, or None if these networks or this signal are not its case."""
     if not 1 <= len(nets) <= 16 or signal.dtype != torch.float32 or signal.requires_grad or signal.numel() == 0:
         return None
-    h = nets[0][0].weight.shape[0]
+    h, device = nets[0][0].weight.shape[0], signal.device
     params = []
     for net in nets:
-        shaped = ((net[0].weight, (h, 1)), (net[0].bias, (h,)), (net[2].weight, (1, h)), (net[2].bias, (1,)))
-        for t, shape in shaped:
-            if t is None or tuple(t.shape) != shape or t.dtype != torch.float32 or t.device != signal.device or not t.is_contiguous():
+        lin1, lin2 = net[0], net[2]
+        for t, shape in ((lin1.weight, (h, 1)), (lin1.bias, (h,)), (lin2.weight, (1, h)), (lin2.bias, (1,))):
+            if t is None or t.shape != shape or t.dtype != torch.float32 or t.device != device or not t.is_contiguous():
                 return None
             params.append(t)
     return params if 1 <= h <= 32 else None

@@ -13,7 +13,7 @@ import math
 import torch
 import torch.nn as nn
 
-from ._lib import check, load, plain_gpu_tensor
+from ._lib import check, load, on_device, plain_gpu_tensor, stream_handle
 
 
 def non_linear(x, activation_name):
@@ -28,10 +28,10 @@ def create_initial_bump(initial_angles, num_neurons, bump_width_factor=10, devic
     ang = initial_angles.to(device)
     if type(num_neurons) is int and num_neurons > 0 and type(bump_width_factor) in (int, float) and ang.dim() == 1 and plain_gpu_tensor(ang):
         sigma = num_neurons / bump_width_factor
-        with torch.cuda.device(ang.device):
+        with on_device(ang.device):
             bump = torch.empty(ang.shape[0], num_neurons, dtype=torch.float32, device=ang.device)
             check(load().ringattr_bump(ang.data_ptr(), ang.stride(0), bump.data_ptr(), num_neurons, ang.shape[0],
-                                       2 * sigma * sigma, torch.cuda.current_stream(ang.device).cuda_stream))
+                                       2 * sigma * sigma, stream_handle(ang.device)))
         return bump / bump.norm(dim=1, keepdim=True)
     centre = (ang * num_neurons / (2 * math.pi)).unsqueeze(1)
     idx = torch.arange(num_neurons, device=device).unsqueeze(0)
@@ -83,10 +83,10 @@ def _action_signal(av_signal, action_dim):
     if action_dim < 2 or av_signal.dim() != 2 or not av_signal.is_contiguous() or not plain_gpu_tensor(av_signal):
         return None
     B, T = av_signal.shape
-    with torch.cuda.device(av_signal.device):
+    with on_device(av_signal.device):
         out = torch.empty(B, T, action_dim, dtype=torch.float32, device=av_signal.device)
         check(load().ringattr_action_signal(av_signal.data_ptr(), out.data_ptr(), action_dim, T, B,
-                                            torch.cuda.current_stream(av_signal.device).cuda_stream))
+                                            stream_handle(av_signal.device)))
     return out
 
 

@@ -20,6 +20,7 @@ import torch
 from torch.autograd import Function
 
 from . import _lib
+from .ring_rnn_cuda import _activation_id, _compact, _driven_pair, _grad_buffers, _grad_gather
 from .rnn_cuda import fwd_cuda, bwd_cuda, saved_nbytes
 
 
@@ -50,7 +51,7 @@ class RingLossPair(Function):
             amp = target_amplitude.reshape(-1).contiguous()
             _check("target_amplitude", amp, (B,), dev)
         lib = _lib.load()
-        with torch.cuda.device(dev):
+        with _lib.on_device(dev):
             nbytes = lib.ringattr_loss_workspace_bytes(N, T, B)
             if nbytes == 0:
                 _lib.check(1)
@@ -58,7 +59,7 @@ class RingLossPair(Function):
             out = torch.empty(3, dtype=torch.float32, device=dev)
             _lib.check(lib.ringattr_loss_fwd(hist.data_ptr(), angle.data_ptr(), amp.data_ptr() if amp is not None else None,
                                              float(bump_weight), out.data_ptr(), N, T, B, ws.data_ptr(), nbytes,
-                                             torch.cuda.current_stream(dev).cuda_stream))
+                                             _lib.stream_handle(dev)))
         ctx.save_for_backward(hist, angle, ws, amp if amp is not None else torch.empty(0, device=dev))
         ctx.has_amp, ctx.bump_weight = amp is not None, float(bump_weight)
         ctx.mark_non_differentiable(out)          # the parts are returned for logging; total carries the gradient
@@ -73,10 +74,10 @@ class RingLossPair(Function):
         grad = torch.empty_like(hist)
         up = grad_total.to(torch.float32).reshape(1).contiguous()
         lib = _lib.load()
-        with torch.cuda.device(dev):
+        with _lib.on_device(dev):
             _lib.check(lib.ringattr_loss_bwd(hist.data_ptr(), angle.data_ptr(), amp.data_ptr() if ctx.has_amp else None,
                                              ctx.bump_weight, up.data_ptr(), grad.data_ptr(), N, T, B, ws.data_ptr(),
-                                             ws.numel(), torch.cuda.current_stream(dev).cuda_stream))
+                                             ws.numel(), _lib.stream_handle(dev)))
         return grad, None, None, None
 
 
@@ -94,7 +95,6 @@ class RingRnnLossFunc(Function):
     @staticmethod
     def forward(ctx, action_signal, Wa, J0, J1, Wo, r_init, alpha, activation_name, target_angle, bump_weight,
                 target_amplitude, grad_mode=None, pair=None):
-        from .ring_rnn_cuda import _activation_id, _compact
         act = _activation_id(activation_name)
         B, T, k = action_signal.shape
         N = Wa.shape[1]
@@ -116,7 +116,7 @@ class RingRnnLossFunc(Function):
         ctx.extra_inputs = 0 if grad_mode is None else 2
         saved = torch.empty(saved_nbytes(N, k, T, B), dtype=torch.uint8, device=dev) if needs_grad else None
         lib = _lib.load()
-        with torch.cuda.device(dev):
+        with _lib.on_device(dev):
             nbytes = lib.ringattr_loss_workspace_bytes(N, T, B)
             if nbytes == 0:
                 _lib.check(1)
@@ -135,7 +135,6 @@ class RingRnnLossFunc(Function):
     @staticmethod
     def backward(ctx, grad_total, _grad_parts, _grad_hist):
         A, Wa, Wo, hist, r0, saved, lws, angle, amp = ctx.saved_tensors
-        from .ring_rnn_cuda import _grad_buffers, _grad_gather
         grad_Wa, part = _grad_buffers(Wa, ctx.Wa_shape, ctx.pair)         # written, not accumulated into
         grad_Wo = torch.empty_like(Wo)
         grad_A = torch.empty_like(A) if ctx.needs_input_grad[0] else None
@@ -149,10 +148,10 @@ class RingRnnLossFunc(Function):
             # the step-per-launch kernels (wide rings) read grad_output: the loss head writes it, the backward reads it
             grad_hist = torch.empty_like(hist)
             dev = hist.device
-            with torch.cuda.device(dev):
+            with _lib.on_device(dev):
                 _lib.check(lib.ringattr_loss_bwd(hist.data_ptr(), angle.data_ptr(), amp.data_ptr() if amp is not None else None,
                                                  ctx.bump_weight, up.data_ptr(), grad_hist.data_ptr(), N, T, B,
-                                                 lws.data_ptr(), lws.numel(), torch.cuda.current_stream(dev).cuda_stream))
+                                                 lws.data_ptr(), lws.numel(), _lib.stream_handle(dev)))
             bwd_cuda.bwd(grad_output=grad_hist, A=A, Wa=Wa, J0=ctx.J0, J1=ctx.J1, Wo=Wo, bump_history=hist, r_init=r0,
                          grad_Wa=part, grad_Wo=grad_Wo, alpha=ctx.alpha, activation_type=ctx.act, saved=saved,
                          grad_A=grad_A, grad_r_init=grad_r0, accumulate=False)
@@ -169,7 +168,6 @@ def ring_rnn_loss_func(action_signal, Wa, J0, J1, Wo, r_init, alpha, activation,
 
     Returns (total, cos_loss, amp_loss, bump_history); only `total` is differentiable (w.r.t. Wa, Wo and, when they
     require it, action_signal and r_init); bump_history [T,B,N] is returned detached for decoding and logging."""
-    from .ring_rnn_cuda import _driven_pair
     pair = _driven_pair(action_signal, Wa, driven_channels)
     total, parts, hist = RingRnnLossFunc.apply(action_signal, Wa, J0, J1, Wo, r_init, alpha, activation, target_angle,
                                                bump_weight, target_amplitude, torch.is_grad_enabled(), pair)

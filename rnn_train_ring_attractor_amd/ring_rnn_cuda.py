@@ -5,6 +5,8 @@ Same public names, argument order and semantics as the reference's cpp/ring_rnn_
 bump_history [T,B,N] and is differentiable w.r.t. Wa and Wo.  A star-import also hands out `torch`,
 which the reference training script relies on (train_general_ring_no_gain.py:19, 40).
 """
+from os import environ as _environ
+
 import torch
 from torch.autograd import Function
 
@@ -96,8 +98,7 @@ def _driven_pair(action_signal, Wa, driven_channels=None):
     that has its address).
     Without a statement the operator runs on all channels (the general kernels skip all-zero channels step by step).
     RINGATTR_COMPACT_CHANNELS=0 switches the compaction off."""
-    import os
-    if os.environ.get("RINGATTR_COMPACT_CHANNELS", "1") == "0":
+    if _environ.get("RINGATTR_COMPACT_CHANNELS", "1") == "0":
         return None
     if driven_channels is None:
         driven_channels = getattr(action_signal, DRIVEN_ATTR, None)
@@ -131,14 +132,14 @@ def _compact(action_signal, Wa, pair):
     N = Wa.shape[1]
     dev = action_signal.device
     lib = _lib.load()
-    with torch.cuda.device(dev):
+    with _lib.on_device(dev):
         a2 = torch.empty(B, T, 2, dtype=torch.float32, device=dev)
         Wa2 = torch.empty(2, N, N, dtype=torch.float32, device=dev)
         nbytes = lib.ringattr_compact_workspace_bytes()
         ws = torch.empty(nbytes, dtype=torch.uint8, device=dev)
         _lib.check(lib.ringattr_compact_channels(action_signal.data_ptr(), Wa.data_ptr(), a2.data_ptr(), Wa2.data_ptr(), N, k, T, B,
                                                  pair[0], pair[1], ws.data_ptr(), nbytes,
-                                                 torch.cuda.current_stream(dev).cuda_stream))
+                                                 _lib.stream_handle(dev)))
     return a2, Wa2
 
 

@@ -41,7 +41,7 @@ def _f32_cuda(specs):
         _contig(name, t)
         if t.dtype != torch.float32:
             raise TypeError(f"{name} must be float32, got {t.dtype}")
-        if tuple(t.shape) != tuple(shape):
+        if t.shape != shape:
             raise ValueError(f"{name} must have shape {tuple(shape)}, got {tuple(t.shape)}")
     device = specs[0][1].device
     for name, t, _ in specs:
@@ -80,7 +80,7 @@ def _act(activation_type) -> int:
 
 def _stream_ptr(stream, device):
     if stream is None:
-        stream = torch.cuda.current_stream(device)
+        return _lib.stream_handle(device)
     return stream.cuda_stream if hasattr(stream, "cuda_stream") else int(stream)
 
 
@@ -128,7 +128,7 @@ class _Fwd:
             need = lib.ringattr_saved_bytes(N, k, T, B)
             if saved.dtype != torch.uint8 or saved.numel() < need or saved.device != dev:
                 raise ValueError(f"saved must be a uint8 tensor of at least {need} bytes on {dev}")
-        with torch.cuda.device(dev):
+        with _lib.on_device(dev):
             ws_bytes = lib.ringattr_fwd_workspace_bytes(N, k, T, B)
             if ws_bytes == 0:
                 _lib.check(1)
@@ -203,7 +203,7 @@ class _Bwd:
                 _lib.check(1)
             if loss_workspace.dtype != torch.uint8 or loss_workspace.numel() < need or loss_workspace.device != dev:
                 raise ValueError(f"loss_workspace must be a uint8 tensor of at least {need} bytes on {dev}")
-            with torch.cuda.device(dev):
+            with _lib.on_device(dev):
                 ws_bytes = lib.ringattr_bwd_workspace_bytes_for(N, k, T, B, int(saved is not None), int(grad_A is not None))
                 if ws_bytes == 0:
                     _lib.check(1)
@@ -214,7 +214,7 @@ class _Bwd:
                                            _stream_ptr(stream, dev))
             _lib.check(rc)
             return None
-        with torch.cuda.device(dev):
+        with _lib.on_device(dev):
             ws_bytes = lib.ringattr_bwd_workspace_bytes_for(N, k, T, B, int(saved is not None), int(grad_A is not None))
             if ws_bytes == 0:
                 _lib.check(1)

@@ -236,3 +236,15 @@ def test_helpers_keep_to_tensor_operations_where_torch_lacks_a_private_name(owne
     assert not _lib.plain_gpu_tensor(av)
     got = host.av_to_action_signal(av), host.av_to_action_signal_ND(av, 5), host.create_initial_bump(angle, 32, device=gpu_device)
     assert all(torch.equal(a, b) for a, b in zip(got, want))
+
+
+def test_stream_handle_is_the_current_streams(gpu_device, monkeypatch):
+    from rnn_train_ring_attractor_amd import _lib
+    side = torch.cuda.Stream()
+    device = torch.zeros(1, device=gpu_device).device
+    for missing in (False, True):                      # (torch's private name may be missing)
+        if missing:
+            monkeypatch.delattr(torch._C, "_cuda_getCurrentRawStream")
+        assert _lib.stream_handle(device) == torch.cuda.current_stream(device).cuda_stream
+        with torch.cuda.stream(side), _lib.on_device(device):
+            assert _lib.stream_handle(device) == side.cuda_stream and torch.cuda.current_device() == device.index
