@@ -230,6 +230,12 @@ __device__ __forceinline__ float row16_sum(float v) {
   return v;
 }
 
+// A lane's value from within its row of 16 lanes.
+template <int CTRL>
+__device__ __forceinline__ float dpp_row(float v) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xF, 0xF, false));
+}
+
 // The same sum with data-parallel-primitive adds (no LDS traffic): butterfly inside each row of 16 lanes.
 __device__ __forceinline__ float row16_sum_dpp(float v) {
 #define RING_DPP_ADD(CTRL) \

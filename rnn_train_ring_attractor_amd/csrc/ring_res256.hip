@@ -133,7 +133,7 @@ __device__ __forceinline__ void load_resident(const bf16x8* Wp, bf16x8* wl, bf16
 namespace {
 
 constexpr int R8_HALF_SLOTS = 4 * 4 * XG;   // 16-byte slots of one operand half (4 K chunks)
-constexpr size_t R8_STAT_FLOATS = 2 * 8 * 3 * 16;   // loss-head row sums per wave: [step parity][wave][C, S, |r|][row]
+constexpr size_t R8_STAT_FLOATS = 2 * 8 * 4 * 16;   // loss-head row sums per wave: [step parity][wave][C, S, |r|, spare][row]
 constexpr size_t R8_LDS_BYTES = (size_t)(R_WLDS_SLOTS + 3 * R8_HALF_SLOTS) * 16 + 2 * R_GCH * 16 * 8 + R8_STAT_FLOATS * 4;
 
 __device__ __forceinline__ void load_resident8(const bf16x8* Wp, bf16x8* wl, bf16x8 (&wreg)[2][2][R_KCH], int w, int h,
@@ -167,8 +167,11 @@ struct NoStores {};
 
 // STATS: also leave the loss head's three sums of every history row (sum_i r_i cos(phi_i), sum_i r_i sin(phi_i),
 // sum_i |r_i|, phi_i = 2 pi i / N) in p.loss_stats[t * B + b], so that the loss needs no pass of its own over the
-// history.  Each wave reduces its 32 neurons' share over the row group's 16 lanes right after the activation, the
-// eight shares meet in LDS (buffer by step parity) and wave 0 adds them in wave order behind the next barrier.
+// history.  Each wave reduces its 32 neurons' share over the row group's 16 lanes, a sum at a time between the matrix
+// instructions of the following contraction, the eight shares meet in LDS (buffer by step parity) and wave 0 adds them in wave
+// order a step later.  (Reduced right after the activation, in front of the barrier that the other role waits at, the sums were
+// on the step's serial chain: forward of T = 100, gelu, N = 256, B = 1024 211 -> 169 us, without the sums 144; N = 200 209 -> 176.
+// At B = 4096 the history's stores bound the step and nothing changes.)
 template <int ACT, bool SAVE, bool FULL, bool STATS>
 __global__ __launch_bounds__(512) void ring_fwd_res256_kernel(RingFwdArgs p) {
   extern __shared__ __attribute__((aligned(16))) char smem[];
@@ -195,7 +198,8 @@ __global__ __launch_bounds__(512) void ring_fwd_res256_kernel(RingFwdArgs p) {
   bf16x8* wl = wlds + (size_t)(w8 * 2 * R_KCH) * 64 + lane;
   load_resident8(reinterpret_cast<const bf16x8*>(p.Wpack), wl, wreg, w, h, lane);
 
-  float r[4][2], okf[4][2];
+  float r[4][2];
+  bool ok[4][2];
   // alpha F', or what it is made of (late role of whole tiles), until it is stored
   using Record = ActRecord<ACT>;
   float d[4][2];
@@ -204,9 +208,8 @@ __global__ __launch_bounds__(512) void ring_fwd_res256_kernel(RingFwdArgs p) {
   for (int e = 0; e < 4; ++e)
 #pragma unroll
     for (int cc = 0; cc < 2; ++cc) {
-      const bool ok = (b0 + e < B) && (i0 + cc < N);
-      okf[e][cc] = ok ? 1.f : 0.f;
-      r[e][cc] = ok ? p.r_init[(size_t)(b0 + e) * N + i0 + cc] : 0.f;
+      ok[e][cc] = (b0 + e < B) && (i0 + cc < N);
+      r[e][cc] = ok[e][cc] ? p.r_init[(size_t)(b0 + e) * N + i0 + cc] : 0.f;
     }
   auto save_r = [&](int t) {   // bf16 copy of r_t (operand of step t) for the weight-gradient GEMM
 #pragma unroll
@@ -220,33 +223,34 @@ __global__ __launch_bounds__(512) void ring_fwd_res256_kernel(RingFwdArgs p) {
 #pragma unroll
     for (int cc = 0; cc < 2; ++cc) sincosf(6.283185307179586f * (float)(i0 + cc) / (float)N, &ssn[cc], &scs[cc]);
   }
-  // r[][] holds this wave's part of history row `row_t` (masked entries are zero): its share of the three sums
-  auto stat_share = [&](int row_t) {
-    float* dst = statp + (size_t)(((row_t & 1) * 8 + w8) * 3) * 16 + 4 * q;
+  // r[][] holds this wave's part of a history row (masked entries are zero): its share of one of the three sums.  Lane n ends up
+  // with the sum of row n >> 2 of the row group: the quads add up, then two rows' sums cross over to one half of the lanes each.
+  float share = 0.f;
+  auto stat_sum = [&](int kind) {
+    float v[4];
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
-      float c = fmaf(r[e][1], scs[1], r[e][0] * scs[0]);
-      float sn = fmaf(r[e][1], ssn[1], r[e][0] * ssn[0]);
-      float ab = fabsf(r[e][0]) + fabsf(r[e][1]);
-      c = row16_sum_dpp(c);
-      sn = row16_sum_dpp(sn);
-      ab = row16_sum_dpp(ab);
-      if (n == 0) {
-        dst[e] = c;
-        dst[16 + e] = sn;
-        dst[32 + e] = ab;
-      }
+      v[e] = kind == 2 ? fabsf(r[e][0]) + fabsf(r[e][1])
+                       : fmaf(r[e][1], kind == 0 ? scs[1] : ssn[1], r[e][0] * (kind == 0 ? scs[0] : ssn[0]));
+      v[e] += dpp_row<0xB1>(v[e]);         // quad_perm [1,0,3,2]
+      v[e] += dpp_row<0x4E>(v[e]);         // quad_perm [2,3,0,1]
     }
+    const bool odd = n & 4, high = n & 8;
+    const float lo = (odd ? v[1] : v[0]) + dpp_row<0x141>(odd ? v[0] : v[1]);     // row_half_mirror: the other quad of eight lanes
+    const float hi = (odd ? v[3] : v[2]) + dpp_row<0x141>(odd ? v[2] : v[3]);
+    const float sum = (high ? hi : lo) + dpp_row<0x128>(high ? lo : hi);          // row_ror:8: the other eight
+    share = kind == 0 || (n & 3) == kind ? sum : share;
   };
+  auto stat_put = [&](int row_t) { statp[(((row_t & 1) * 8 + w8) * 4 + (n & 3)) * 16 + 4 * q + (n >> 2)] = share; };
   // the eight shares of row `row_t` are complete behind a barrier: wave 0 adds them in wave order and stores the row sums
   auto stat_flush = [&](int row_t) {
-    if (w8 == 0) {
+    if (wu == 0 && hu == 0) {
       const int kind = lane >> 4, row = lane & 15, b = 16 * bt + row;
       float v = 0.f;
       if (kind < 3) {
-        const float* src = statp + (size_t)((row_t & 1) * 8 * 3 + kind) * 16 + row;
+        const float* src = statp + (size_t)((row_t & 1) * 8 * 4 + kind) * 16 + row;
 #pragma unroll
-        for (int wv = 0; wv < 8; ++wv) v += src[wv * 3 * 16];
+        for (int wv = 0; wv < 8; ++wv) v += src[wv * 4 * 16];
       }
       if (b < B) reinterpret_cast<float*>(p.loss_stats + (size_t)row_t * B + b)[kind] = v;
     }
@@ -294,6 +298,11 @@ __global__ __launch_bounds__(512) void ring_fwd_res256_kernel(RingFwdArgs p) {
   const unsigned r_lane = (unsigned)((ct0 * 64 + lc) * 16);                                // + tile cc * 1 KiB
   auto emit_store = [&](int t, int slot, auto once) {
     __builtin_amdgcn_sched_barrier(0);
+    if constexpr (STATS) {
+      if (slot < 3) stat_sum(slot);
+      if (slot == 3) stat_put(t);
+      if (slot == 5 && t > 0) stat_flush(t - 1);         // (step t's contraction: the shares came in before its first barrier)
+    }
     if (slot < 4) {
       if (p.hist == nullptr) return;   // recompute of the saved record only: the history already exists
       const int e = slot;
@@ -403,8 +412,10 @@ __global__ __launch_bounds__(512) void ring_fwd_res256_kernel(RingFwdArgs p) {
         else act_scaled<ACT>(x[e][cc], asc, aF, d[e][cc]);
         float rn = fmaf(oma, r[e][cc], aF);
         if constexpr (!FULL) {
-          rn *= okf[e][cc];
-          d[e][cc] *= okf[e][cc];                  // (never `once`)
+          // (lanes' masks in scalar registers: eight factors of 0 or 1 spilled up to 23 registers here, 20 in the BPTT with the loss
+          // and dL/dA: N = 201, B = 1748 3.54 -> 3.37 us per step)
+          rn = ok[e][cc] ? rn : 0.f;
+          d[e][cc] = ok[e][cc] ? d[e][cc] : 0.f;   // (never `once`)
         }
         r[e][cc] = rn;
       }
@@ -419,14 +430,10 @@ __global__ __launch_bounds__(512) void ring_fwd_res256_kernel(RingFwdArgs p) {
       if (l == 0 && (ci + 1) * R_GCH < T) gates_fetch(p.A, T, B, bt, ci + 1, +1, tid, gs);
       contract_half(0, xE + (t & 1) * R8_HALF_SLOTS, t - 1, emit);
       lds_barrier();   // B_t
-      if constexpr (STATS) {
-        if (t > 0) stat_flush(t - 1);            // both roles' shares of row t-1 are in
-      }
       contract_half(1, xL, t - 1, emit);
       float x[4][2];
       preactivation(t, x);
       activate(x, std::false_type{});
-      if constexpr (STATS) stat_share(t);
       if (t + 1 < T) write_half(xE + ((t + 1) & 1) * R8_HALF_SLOTS, r, w, q, n);
       // the next chunk's gates are first read after barrier B of its first step
       if (l == R_GCH - 1 && t + 1 < T) gates_publish(gbuf + ((ci + 1) & 1) * R_GCH * 16, tid, B, bt, gs);
@@ -444,7 +451,6 @@ __global__ __launch_bounds__(512) void ring_fwd_res256_kernel(RingFwdArgs p) {
     lds_barrier();   // A_1
     for (int t = 1; t < T; ++t) {
       activate(x, late_once);   // step t-1 -> r^L_t
-      if constexpr (STATS) stat_share(t - 1);
       write_half(xL, r, w, q, n);
       lds_barrier();   // B_t
       contract_half(0, xE + (t & 1) * R8_HALF_SLOTS, t - 1, late_once);
@@ -453,15 +459,14 @@ __global__ __launch_bounds__(512) void ring_fwd_res256_kernel(RingFwdArgs p) {
       lds_barrier();   // A_{t+1}
     }
     activate(x, std::false_type{});
-    if constexpr (STATS) stat_share(T - 1);
-  }
-  if constexpr (STATS) {
-    lds_barrier();                                 // the late role's share of the last row
-    stat_flush(T - 1);
   }
   // stores of the last step (its state is not an operand of any further step)
 #pragma unroll
   for (int slot = 0; slot < 6; ++slot) emit_store(T - 1, slot, std::false_type{});
+  if constexpr (STATS) {
+    lds_barrier();                                 // the shares of the last row
+    stat_flush(T - 1);
+  }
 }
 
 // ------------------------------------------------------------------------------------------------
@@ -676,13 +681,13 @@ __global__ __launch_bounds__(256) void ring_bptt_res256_kernel(RingBpttArgs p) {
   load_resident(reinterpret_cast<const bf16x8*>(p.Wpack), wl, wreg, w, lane);
 
   float carry[4][R_NC];
-  float okf[4][R_NC];
+  bool ok[4][R_NC];
 #pragma unroll
   for (int e = 0; e < 4; ++e)
 #pragma unroll
     for (int c = 0; c < R_NC; ++c) {
       carry[e][c] = 0.f;
-      okf[e][c] = ((b0 + e < B) && (i0 + c < N)) ? 1.f : 0.f;
+      ok[e][c] = (b0 + e < B) && (i0 + c < N);
     }
 
   float cs[R_NC], sn[R_NC], up = 0.f;
@@ -816,7 +821,7 @@ __global__ __launch_bounds__(256) void ring_bptt_res256_kernel(RingBpttArgs p) {
         for (int e = 0; e < 4; ++e) {
           float x = fmaf(gate[e][0], P1[e], P0[e]);
           x = fmaf(gate[e][1], P2[e], x);
-          if constexpr (!FULL) x *= okf[e][c];
+          if constexpr (!FULL) x = ok[e][c] ? x : 0.f;
           carry[e][c] = x;
         }
         if constexpr (GA) {

@@ -213,3 +213,20 @@ def test_loss_gradient_inside_the_step_per_launch_backward(B, T, k, N, act, fami
     for name, a, b in zip(("grad_Wo", "grad_Wa", "grad_r_init", "grad_A"), res[True][1:], res[False][1:]):
         assert np.isfinite(a).all() and np.abs(b).max() > 0, name
         assert O.max_rel_err(a, b) <= 2e-3 and O.cosine(a, b) >= 0.99999, name
+
+
+@pytest.mark.parametrize("N,B,T,act", [(256, 528, 1, "gelu"), (256, 528, 2, "relu"), (256, 528, 5, "tanh"), (129, 513, 3, "silu"),
+                                       (200, 530, 34, "gelu")])
+def test_row_sums_of_the_weight_resident_forward(N, B, T, act, gpu_device):
+    """Batches past the teams: the forward forms the loss's sums a step behind the state.  Its losses against the loss head's own pass
+    over the same history: both add 256 fp32 terms per sum, in another order, 256 * 2^-24 = 1.5e-5 at most."""
+    from rnn_train_ring_attractor_amd import ring_loss_pair, ring_rnn_loss_func
+    from tests.ring_cases import make_problem
+    print(f"[case] row sums N={N} B={B} T={T}", flush=True)
+    p = make_problem(N + T, B, T, 2, N, weights="perfect")
+    t = lambda x: torch.tensor(x, device=gpu_device)
+    for record in (False, True):
+        Wo = t(p["Wo"]).requires_grad_(record)
+        total, lc, la, hist = ring_rnn_loss_func(t(p["A"]), t(p["Wa"]), -1.0 / N, 2.0 / N, Wo, t(p["r0"]), 0.15, act, t(p["angle"]), 0.2)
+        for got, want in zip((total, lc, la), ring_loss_pair(hist.detach(), t(p["angle"]), 0.2)):
+            assert abs(float(got.detach()) - float(want)) <= 2e-5 * max(1.0, abs(float(want)))
