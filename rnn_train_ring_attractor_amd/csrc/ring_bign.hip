@@ -111,7 +111,8 @@ __global__ __launch_bounds__(256) void ring_wide_fwd_kernel(RingFwdArgs p, int N
   const bool staged = p.k <= BN_GATE_KMAX;
   const float* prev = (t == 0) ? p.r_init : p.hist + (size_t)(t - 1) * B * N;
 
-  stage_rows(xb, rs, NPAD, tid, [&](int row, int j) { return load4_masked(prev, N, B, 16 * bt + row, j); });
+  const __amdgpu_buffer_rsrc_t prev_rows = rows_buffer(prev, (size_t)16 * bt, (size_t)B, 16, (size_t)N * 4);
+  with_whole(N, [&](auto whole) { stage_rows<1>(xb, 0, rs, NPAD, tid, StateRows<decltype(whole)::value>{prev_rows, N}); });
   if (staged) stage_gates(gl, p.A, p.k, T, B, t, bt, tid);
   lds_barrier();
 
@@ -184,38 +185,28 @@ __global__ __launch_bounds__(256) void ring_wide_bptt_kernel(RingBpttArgs p, int
   step_block_coords(xcd_map, bt, cb);
   const int N = p.N, B = p.B, T = p.T, NPAD = 64 * NC;
   const bool staged = p.k <= BN_GATE_KMAX;
-  const size_t rows_pad = (size_t)16 * p.nbt;
-  const float* gout = LOSS ? nullptr : p.grad_out + (size_t)t * B * N;
-  const _Float16* drow = p.dfrag + (size_t)t * rows_pad * NPAD;
-  // LOSS: grad_output is not read; it is formed from the state history and the loss head's row coefficients
   const float up = LOSS ? (p.loss_upstream ? p.loss_upstream[0] : 1.f) * p.loss_inv_rows : 0.f;
-
-  // g of (row, j..j+3): carry rows live in a padded [16*nbt][NPAD] buffer
-  auto g4 = [&](int row, int j, f32x4& G) {
-    const int b = 16 * bt + row;
-    if constexpr (LOSS) G = loss_grad4(p, t, b, j, up);
-    else G = load4_masked(gout, N, B, b, j);
-    if (carry_in) {
-      const f32x4 cin = *reinterpret_cast<const f32x4*>(carry_in + ((size_t)16 * bt + row) * NPAD + j);
-      G += cin;
-    }
-    const f16x4 d = *reinterpret_cast<const f16x4*>(drow + ((size_t)16 * bt + row) * NPAD + j);
-    // products rounded on their own (never contracted into the row sum that follows), so that both step-per-launch
-    // families form bit-identical g and row sums whatever the compiler does with the surrounding code
-    f32x4 g;
-    {
-#pragma clang fp contract(off)
-      g = f32x4{(float)d[0] * G[0], (float)d[1] * G[1], (float)d[2] * G[2], (float)d[3] * G[3]};
-    }
-    return g;
-  };
-  stage_rows(xb, rs, NPAD, tid, [&](int row, int j) { f32x4 G; return g4(row, j, G); });
-  if (staged) stage_gates(gl, p.A, p.k, T, B, t, bt, tid);
-  lds_barrier();
 
   const int tg0 = 16 * cb + 4 * wv;
   const int wg = tg0 / NC, c0 = tg0 % NC;
   const int j0 = 16 * NC * wg + NC * n + c0;
+  // the lane's own rows and neurons (on their way while the rows are staged)
+  GradRaw<LOSS> own[4];
+  GradCoef own_coef[4];
+  GradTrig own_trig;
+  with_whole(N, [&](auto whole) {
+    const GradRows<LOSS, decltype(whole)::value> src(p, t, 16 * bt, 16, NPAD, carry_in, up);
+    own_trig = src.load_trig(j0);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      own[e] = src.load_row(4 * q + e, j0);
+      own_coef[e] = src.row(4 * q + e);
+    }
+    stage_rows<1>(xb, 0, rs, NPAD, tid, src);
+  });
+  if (staged) stage_gates(gl, p.A, p.k, T, B, t, bt, tid);
+  lds_barrier();
+
   const int b0 = 16 * bt + 4 * q;
   const float oma = 1.f - p.alpha;
   f32x4 acc[4];
@@ -223,7 +214,7 @@ __global__ __launch_bounds__(256) void ring_wide_bptt_kernel(RingBpttArgs p, int
 #pragma unroll
   for (int e = 0; e < 4; ++e) {
     f32x4 G;
-    const f32x4 g = g4(4 * q + e, j0, G);
+    const f32x4 g = GradRows<LOSS, true>::form(own[e], own_trig, own_coef[e], j0, N, carry_in != nullptr, G);
     const float js = p.J0 * rs[4 * q + e];
 #pragma unroll
     for (int cl = 0; cl < 4; ++cl) {

@@ -22,47 +22,55 @@
 
 namespace {
 
-// Stage RT batch tiles' operand rows (bf16, tile i at xb + i * slots) and their fp32 row sums (rs[16*i + row]).
-template <int RT, typename F>
-__device__ __forceinline__ void stage_tiles(bf16x8* xb, int slots, float* rs, int NPAD, int tid, F&& value4) {
-  const int row = tid >> 4, sub = tid & 15;
-#pragma unroll 1
-  for (int i = 0; i < RT; ++i) {
-    float sum = 0.f;
-    char* base = reinterpret_cast<char*>(xb + (size_t)i * slots);
-    for (int j = 4 * sub; j < NPAD; j += 64) {
-      const f32x4 v = value4(16 * i + row, j);
-      sum += (v[0] + v[1]) + (v[2] + v[3]);
-      const bf16x4 pk = {(__bf16)v[0], (__bf16)v[1], (__bf16)v[2], (__bf16)v[3]};
-      *reinterpret_cast<bf16x4*>(base + (size_t)op_slot(j, row) * 16 + (j & 7) * 2) = pk;
-    }
-    sum = row16_sum_dpp(sum);
-    if (sub == 0) rs[16 * i + row] = sum;
-  }
-}
-
-// gates of the workgroup's RT*16 rows at step t, row-major with stride k (dynamic LDS behind the operand tiles)
+// Gates of the workgroup's RT*16 rows at step t, row-major with stride k (dynamic LDS behind the operand tiles): the first two of
+// a thread are asked for before the operand's rows.
 template <int RT>
-__device__ __forceinline__ void stage_gates_rt(float* gl, const float* __restrict__ A, int k, int T, int B, int t, int bt0,
-                                               int tid) {
-  for (int idx = tid; idx < RT * 16 * k; idx += 256) {
-    const int row = idx / k, c = idx - row * k, b = 16 * bt0 + row;
-    gl[idx] = b < B ? A[((size_t)b * T + t) * k + c] : 0.f;
+struct GateRows {
+  float v[2];
+  __device__ __forceinline__ static bool inside(int idx, int k, int B, int bt0) { return idx < RT * 16 * k && 16 * bt0 + idx / k < B; }
+  __device__ __forceinline__ void fetch(const float* __restrict__ A, int k, int T, int B, int t, int bt0, int tid) {
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const int idx = tid + 256 * i, row = idx / k, c = idx - row * k;
+      v[i] = A[inside(idx, k, B, bt0) ? ((size_t)(16 * bt0 + row) * T + t) * k + c : 0];
+    }
   }
-}
+  __device__ __forceinline__ void put(float* gl, const float* __restrict__ A, int k, int T, int B, int t, int bt0, int tid) const {
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const int idx = tid + 256 * i;
+      if (idx < RT * 16 * k) gl[idx] = inside(idx, k, B, bt0) ? v[i] : 0.f;
+    }
+    for (int idx = tid + 512; idx < RT * 16 * k; idx += 256) {
+      const int row = idx / k, c = idx - row * k, b = 16 * bt0 + row;
+      gl[idx] = b < B ? A[((size_t)b * T + t) * k + c] : 0.f;
+    }
+  }
+};
 
-// bit c set <=> channel c has a non-zero gate in some of the workgroup's RT*16 rows
+// bit c set <=> channel c has a non-zero gate in some of the workgroup's RT*16 rows; sixteen channels at a time
 template <int RT>
 __device__ __forceinline__ unsigned long long active_channels_rt(const float* gl, int k, int lane) {
   unsigned long long m = 0;
-  for (int c0 = 0; c0 < k; c0 += 4) {
-    const int c = c0 + (lane >> 4);
-    bool nz = false;
-    for (int i = 0; i < RT; ++i) nz |= c < k && gl[(16 * i + (lane & 15)) * k + c] != 0.f;
-    const unsigned long long bal = __ballot(nz);
+  for (int c0 = 0; c0 < k; c0 += 16) {
+    float v[4][RT];
 #pragma unroll
-    for (int j = 0; j < 4; ++j)
-      if ((bal >> (16 * j)) & 0xffffull) m |= 1ull << (c0 + j);
+    for (int g = 0; g < 4; ++g)
+#pragma unroll
+      for (int i = 0; i < RT; ++i) {
+        const int c = c0 + 4 * g + (lane >> 4);
+        v[g][i] = gl[(16 * i + (lane & 15)) * k + (c < k ? c : 0)];
+      }
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      bool nz = false;
+#pragma unroll
+      for (int i = 0; i < RT; ++i) nz |= v[g][i] != 0.f;
+      const unsigned long long bal = __ballot(nz && c0 + 4 * g + (lane >> 4) < k);
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        if ((bal >> (16 * j)) & 0xffffull) m |= 1ull << (c0 + 4 * g + j);
+    }
   }
   const unsigned lo = __builtin_amdgcn_readfirstlane((unsigned)m), hi = __builtin_amdgcn_readfirstlane((unsigned)(m >> 32));
   return ((unsigned long long)hi << 32) | lo;
@@ -178,13 +186,21 @@ __global__ __launch_bounds__(256) void ring_block_fwd_kernel(RingFwdArgs p, int 
   float* gl = reinterpret_cast<float*>(xb + (size_t)RT * slots);
   const float* prev = (t == 0) ? p.r_init : p.hist + (size_t)(t - 1) * B * N;
 
-  stage_tiles<RT>(xb, slots, rs, NPAD, tid, [&](int row, int j) { return load4_masked(prev, N, B, 16 * bt0 + row, j); });
-  if (staged) stage_gates_rt<RT>(gl, p.A, p.k, T, B, t, bt0, tid);
-  lds_barrier();
-
   const int tg0 = 4 * TPW * cb + TPW * wv;                // this wave's first column tile
   const int wg = tg0 / NC, c0 = tg0 % NC;                 // common tile order: tile = wg * NC + c
   const int j0 = 16 * NC * wg + NC * n + c0;              // the lane's TPW consecutive neurons
+  GateRows<RT> gates;
+  if (staged) gates.fetch(p.A, p.k, T, B, t, bt0, tid);
+  const __amdgpu_buffer_rsrc_t prev_rows = rows_buffer(prev, (size_t)16 * bt0, (size_t)B, 16 * RT, (size_t)N * 4);
+  f32x4 own[RT][4];                                       // r_prev of the lane's rows and neurons
+#pragma unroll
+  for (int i = 0; i < RT; ++i)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) own[i][e] = row_columns<TPW, false>(prev_rows, 16 * i + 4 * q + e, N, j0);
+  with_whole(N, [&](auto whole) { stage_rows<RT>(xb, slots, rs, NPAD, tid, StateRows<decltype(whole)::value>{prev_rows, N}); });
+  if (staged) gates.put(gl, p.A, p.k, T, B, t, bt0, tid);
+  lds_barrier();
+
   const int b0 = 16 * bt0 + 4 * q;
   f32x4 acc[RT][TPW];
 #pragma unroll
@@ -202,7 +218,7 @@ __global__ __launch_bounds__(256) void ring_block_fwd_kernel(RingFwdArgs p, int 
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
       const int b = b0 + 16 * i + e;
-      const f32x4 rp = loadv_masked<TPW>(prev, N, B, b, j0);
+      const f32x4 rp = own[i][e];
       const float js = p.J0 * rs[16 * i + 4 * q + e];
       f32x4 rn = {0.f, 0.f, 0.f, 0.f}, dd = rn;
 #pragma unroll
@@ -255,39 +271,33 @@ __global__ __launch_bounds__(256) void ring_block_bptt_kernel(RingBpttArgs p, in
   const int N = p.N, B = p.B, T = p.T, NPAD = 64 * NC, slots = 2 * NC * 4 * XG;
   const bool staged = p.k <= BN_GATE_KMAX;
   float* gl = reinterpret_cast<float*>(xb + (size_t)RT * slots);
-  const size_t rows_pad = (size_t)16 * p.nbt;
-  const float* gout = LOSS ? nullptr : p.grad_out + (size_t)t * B * N;
-  const _Float16* drow = p.dfrag + (size_t)t * rows_pad * NPAD;
-  // LOSS: grad_output is not read; it is formed from the state history and the loss head's row coefficients
   const float up = LOSS ? (p.loss_upstream ? p.loss_upstream[0] : 1.f) * p.loss_inv_rows : 0.f;
-
-  // g of (row within the block, j..j+V-1); carry rows live in a padded [16*nbt][NPAD] buffer.  Rows of batch tiles
-  // past the last one (a partial last block) read as zero.
-  auto g4 = [&](int row, int j, f32x4& G) {
-    const size_t prow = (size_t)16 * bt0 + row;
-    G = f32x4{0.f, 0.f, 0.f, 0.f};
-    if (prow >= rows_pad) return G;
-    if constexpr (LOSS) G = loss_grad4(p, t, (int)prow, j, up);
-    else G = load4_masked(gout, N, B, (int)prow, j);
-    if (carry_in) G += *reinterpret_cast<const f32x4*>(carry_in + prow * NPAD + j);
-    const f16x4 d = *reinterpret_cast<const f16x4*>(drow + prow * NPAD + j);
-    // products rounded on their own (never contracted into the row sum that follows), so that both step-per-launch
-    // families form bit-identical g and row sums whatever the compiler does with the surrounding code
-    f32x4 g;
-    {
-#pragma clang fp contract(off)
-      g = f32x4{(float)d[0] * G[0], (float)d[1] * G[1], (float)d[2] * G[2], (float)d[3] * G[3]};
-    }
-    return g;
-  };
-  stage_tiles<RT>(xb, slots, rs, NPAD, tid, [&](int row, int j) { f32x4 G; return g4(row, j, G); });
-  if (staged) stage_gates_rt<RT>(gl, p.A, p.k, T, B, t, bt0, tid);
-  lds_barrier();
 
   const int tg0 = 4 * TPW * cb + TPW * wv;
   const int wg = tg0 / NC, c0 = tg0 % NC;
   const int j0 = 16 * NC * wg + NC * n + c0;
   const int j4 = j0 & ~3, jo = j0 & 3;                    // the 16-byte group holding the lane's TPW neurons
+  GateRows<RT> gates;
+  if (staged) gates.fetch(p.A, p.k, T, B, t, bt0, tid);
+  // the lane's own rows and neurons (on their way while the rows are staged)
+  GradRaw<LOSS> own[RT][4];
+  GradCoef own_coef[RT][4];
+  GradTrig own_trig;
+  with_whole(N, [&](auto whole) {
+    const GradRows<LOSS, decltype(whole)::value> src(p, t, 16 * bt0, 16 * RT, NPAD, carry_in, up);
+    own_trig = src.load_trig(j4);
+#pragma unroll
+    for (int i = 0; i < RT; ++i)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        own[i][e] = src.load_row(16 * i + 4 * q + e, j4);
+        own_coef[i][e] = src.row(16 * i + 4 * q + e);
+      }
+    stage_rows<RT>(xb, slots, rs, NPAD, tid, src);
+  });
+  if (staged) gates.put(gl, p.A, p.k, T, B, t, bt0, tid);
+  lds_barrier();
+
   const int b0 = 16 * bt0 + 4 * q;
   const float oma = 1.f - p.alpha;
   f32x4 acc[RT][TPW];
@@ -297,7 +307,7 @@ __global__ __launch_bounds__(256) void ring_block_bptt_kernel(RingBpttArgs p, in
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
       f32x4 G;
-      const f32x4 g = g4(16 * i + 4 * q + e, j4, G);
+      const f32x4 g = GradRows<LOSS, true>::form(own[i][e], own_trig, own_coef[i][e], j4, N, carry_in != nullptr, G);
       const float js = p.J0 * rs[16 * i + 4 * q + e];
 #pragma unroll
       for (int cl = 0; cl < TPW; ++cl) {
@@ -351,7 +361,8 @@ __global__ __launch_bounds__(256) void ring_block_grad_A_kernel(RingBpttArgs p, 
   const int bt = blockIdx.x, t = blockIdx.y;
   const int N = p.N, B = p.B, T = p.T, k = p.k, NPAD = 64 * NC, slots = 2 * NC * 4 * XG, KCH = 2 * NC;
   const float* prev = (t == 0) ? p.r_init : p.hist + (size_t)(t - 1) * B * N;
-  stage_tiles<1>(xb, slots, rs, NPAD, tid, [&](int row, int j) { return load4_masked(prev, N, B, 16 * bt + row, j); });
+  const __amdgpu_buffer_rsrc_t prev_rows = rows_buffer(prev, (size_t)16 * bt, (size_t)B, 16, (size_t)N * 4);
+  with_whole(N, [&](auto whole) { stage_rows<1>(xb, slots, rs, NPAD, tid, StateRows<decltype(whole)::value>{prev_rows, N}); });
   lds_barrier();
 
   for (int m0 = 1; m0 <= k; m0 += 3) {

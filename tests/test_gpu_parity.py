@@ -452,3 +452,24 @@ def test_operator_switches_recompute_and_precise_wo(B, T, k, N, act, gpu_device)
     for got, key in zip(pre[1:], ("grad_Wa", "grad_Wo", "grad_A", "grad_r_init")):
         assert O.cosine(got, ref[key]) >= GRAD_COS, key
         assert O.max_rel_err(got, ref[key]) <= GRAD_TOL, key
+
+
+@pytest.mark.parametrize("B,T,k,N,act,shape", [(33, 3, 6, 701, "gelu", "21"), (49, 2, 20, 1025, "tanh", "22"), (17, 3, 6, 1500, "silu", "12"),
+                                               (33, 2, 4, 1023, "gelu", None)])
+def test_ragged_rows_of_the_step_per_launch_kernels(B, T, k, N, act, shape, gpu_device, monkeypatch):
+    """Widths that are no multiple of four or of a wave's columns, a last batch tile of one row, an odd number of tiles for workgroups of
+    two (`shape`: row tiles, column tiles; None: the one-tile kernels), gates past what a thread fetches ahead."""
+    print(f"[case] step kernels B={B} T={T} k={k} N={N} {act} {shape}", flush=True)
+    monkeypatch.setenv("RINGATTR_TEAM", "0")
+    monkeypatch.setenv("RINGATTR_WIDE", "0" if shape else "1")
+    if shape:
+        monkeypatch.setenv("RINGATTR_BLOCK_SHAPE", shape)
+    p = _problem(300 + N, B, T, k, N, "dense")
+    hist, Wa, Wo = _run_op(p, -0.05, 0.4, act, gpu_device)
+    hist.backward(_dev(p["G"], gpu_device))
+    torch.cuda.synchronize()
+    ref, _ = O.forward_dense(p["A"], p["Wa"], -0.05, 0.4, p["Wo"], p["r0"], 0.15, act)
+    g = O.backward_dense(p["G"], p["A"], p["Wa"], -0.05, 0.4, p["Wo"], ref, p["r0"], 0.15, act)
+    assert O.max_rel_err(hist.detach().cpu().numpy(), ref) <= 1e-2        # (bf16 operands, as everywhere in this file)
+    for got, want in ((Wo.grad, g["grad_Wo"]), (Wa.grad, g["grad_Wa"])):
+        assert O.cosine(got.cpu().numpy(), want) >= GRAD_COS and O.max_rel_err(got.cpu().numpy(), want) <= GRAD_TOL
