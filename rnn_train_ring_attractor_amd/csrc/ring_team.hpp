@@ -362,11 +362,12 @@ struct TeamOperand {
   }
 };
 
-// One item's products: acc[c] = J1 * P_0 + J0 * rowsum + sum_m gate_m P_m over this wave's K chunks.
+// One item's products: acc[c] = J1 * P_0 + J0 * rowsum + sum_m gate_m P_m over this wave's K chunks: the matrices in registers
+// and those in LDS up to channel `last`.
 template <int KPW, int C16, int MR, int WK, bool EX, bool GA>
 __device__ __forceinline__ void team_products(const TeamCompute<KPW, C16, MR, WK, EX, GA>& tc, const TeamOperand<KPW>& op,
                                               const RingTeamArgs& c, const bf16x8* wl, const float (&gate)[MR], const float* gates,
-                                              const f32x4* rows, float* ga, int w, int lane, f32x4 (&acc)[C16]) {
+                                              const f32x4* rows, float* ga, int w, int lane, int last, f32x4 (&acc)[C16]) {
   const int b = lane & 15;
   bf16x8 x[KPW];
 #pragma unroll
@@ -418,8 +419,11 @@ __device__ __forceinline__ void team_products(const TeamCompute<KPW, C16, MR, WK
     if (GA && m <= c.k) row_put(d, m);
   }
   if constexpr (EX) {
-    for (int m = MR; m <= c.k; ++m) {
-      const float gm = gates[(m - 1) * 16 + b];
+    // (gates are read a matrix ahead: forward N = 512, 16 channels, B = 256, T = 20 95.5 -> 93.2 us, N = 168, B = 223, T = 76 158.7 -> 152.3)
+    float gn = gates[(MR - 1) * 16 + b];
+    for (int m = MR; m <= last; ++m) {
+      const float gm = gn;
+      gn = gates[(m < c.k ? m : c.k - 1) * 16 + b];
       // a channel that is zero for all 16 rows contributes nothing (zero-padded action signals); dL/dA needs every product
       if (!GA && __ballot(gm != 0.f) == 0) continue;
       float d = 0.f;
@@ -492,6 +496,7 @@ __device__ __forceinline__ void team_compute_loop(const RingTeamArgs& c, const L
                                                   __amdgpu_buffer_rsrc_t rsrc, int mem, int team, int my_nt, int steps, int w,
                                                   int lane) {
   using AM = AuxMap<C16>;
+  constexpr bool PADS = EX && MR == 3 && !GA;             // (dL/dA needs every product)
   TeamCompute<KPW, C16, MR, WK, EX, GA> tc;
   bf16x8* const wl = reinterpret_cast<bf16x8*>(lds + L.weights);
   tc.template load_weights<TR>(c, wl, reinterpret_cast<bf16x8*>(lds + L.parked), mem, w, lane);
@@ -516,6 +521,18 @@ __device__ __forceinline__ void team_compute_loop(const RingTeamArgs& c, const L
     float gate[MR];                  // (in LDS since the last barrier; read while the operand is on its way)
 #pragma unroll
     for (int m = 1; m < MR; ++m) gate[m] = m <= c.k ? gates[(it & 1) * c.k * 16 + (m - 1) * 16 + b] : 0.f;
+    // Zero-padded action signals: are all channels whose matrices are in LDS silent in the item's rows?  Their gates (up to 14
+    // channels of 16 rows) lie one after the other: four a lane, looked at once the operand is there.  Asked matrix by matrix, one
+    // read of a gate behind the other, silent channels took a quarter of an item: training N = 112, B = 200, T = 100, 16 channels,
+    // two driven 455 -> 325 us a pass.  With nine or thirteen matrices in registers few are left to ask for, and it costs the
+    // others: 16 channels, all driven, N = 512, B = 256, T = 20 93.2 us a call, 96.1 with it (two driven: N = 300, B = 500, T = 100,
+    // training 1612 and 1479).  A second copy of the products without the silent matrices in registers: 1253, but 8 % more where all
+    // are driven.
+    u32x4 tail = {1u, 1u, 1u, 1u};
+    if (PADS && c.k > MR) {
+      const int first = (MR - 1) * 16 + 4 * lane;
+      tail = *reinterpret_cast<const u32x4*>(gates + (it & 1) * c.k * 16 + (first < c.k * 16 ? first : (MR - 1) * 16));
+    }
     int spins = 0;
     // Wide rings: the operand is nearly always there when several tiles share a team, and with the polling loop out of the
     // way the path straight on is shorter: N = 700, B = 500 11.55 -> 11.1 us per step forward and backward, N = 1024,
@@ -545,8 +562,9 @@ __device__ __forceinline__ void team_compute_loop(const RingTeamArgs& c, const L
     const int jn = wrap ? 0 : j + 1, sn = !wrap ? slot : (slot + 1 == c.slots ? 0 : slot + 1);
     nx.template issue<WK>(rsrc, tc, (unsigned)sn * slot_bytes + (unsigned)(team + c.nteams * jn) * tile_bytes);
     f32x4 acc[C16];
+    const bool padding = PADS && __ballot(((tail[0] | tail[1] | tail[2] | tail[3]) & 0x7FFFFFFFu) != 0) == 0;
     team_products<KPW, C16, MR, WK, EX, GA>(tc, op, c, wl, gate, gates + (it & 1) * c.k * 16, rows + (it & 1) * C16 * 64,
-                                            ga + (size_t)((it & 1) * WK + w) * c.k * 16, w, lane, acc);
+                                            ga + (size_t)((it & 1) * WK + w) * c.k * 16, w, lane, padding ? 0 : c.k, acc);
     float* dst = share + (it & 1) * (WK * C16 * AM::SHARE);
 #pragma unroll
     for (int cc = 0; cc < C16; ++cc) *reinterpret_cast<f32x4*>(dst + cc * AM::SHARE) = acc[cc];

@@ -520,3 +520,31 @@ def test_fused_loss_head_on_small_batches_of_the_weight_resident_widths(N, B, T,
         got = run(**env)
         assert "ring_team_res256_bptt" in _lib.last_kernel_names()["bptt"]
         assert [torch.equal(x, y) for x, y in zip(got, want)] == [True] * len(want), env
+
+
+@pytest.mark.parametrize("N,B,k", [(112, 40, 16), (144, 33, 12), (300, 200, 16), (385, 20, 7)])
+def test_channels_that_are_silent_in_some_items(N, B, k, gpu_device):
+    """Matrices in LDS are passed by where their channels are silent in an item's 16 rows: none driven, only the last, only in some
+    rows, gates of minus zero; against the oracle (bf16 operands: the bounds of the parity tests)."""
+    from oracle import ring_oracle as O
+    from tests.ring_cases import make_problem
+    from rnn_train_ring_attractor_amd import ring_rnn_cuda_func
+    T = 6
+    print(f"[case] silent channels N={N} B={B} k={k}", flush=True)
+    p = make_problem(500 + N, B, T, k, N, action="dense")
+    A = p["A"]
+    A[:, 0, 2:] = 0.0
+    A[:16, 1, :-1] = 0.0
+    A[16:, 2, 3:] = -0.0
+    A[1:, 3, -1] = 0.0
+    A[:, 4, :] = 0.0
+    t = lambda x: torch.tensor(x, device=gpu_device)
+    Wa, Wo = t(p["Wa"]).requires_grad_(True), t(p["Wo"]).requires_grad_(True)
+    hist = ring_rnn_cuda_func(t(A), Wa, -0.05, 0.4, Wo, t(p["r0"]), 0.15, "gelu")
+    hist.backward(t(p["G"]))
+    torch.cuda.synchronize()
+    ref, _ = O.forward_dense(A, p["Wa"], -0.05, 0.4, p["Wo"], p["r0"], 0.15, "gelu")
+    g = O.backward_dense(p["G"], A, p["Wa"], -0.05, 0.4, p["Wo"], ref, p["r0"], 0.15, "gelu")
+    assert O.max_rel_err(hist.detach().cpu().numpy(), ref) <= 1e-2
+    for got, want in ((Wo.grad, g["grad_Wo"]), (Wa.grad, g["grad_Wa"])):
+        assert O.cosine(got.cpu().numpy(), want) >= 0.999 and O.max_rel_err(got.cpu().numpy(), want) <= 2e-2
