@@ -433,11 +433,15 @@ static size_t block_lds_bytes(int NC, int RT, int k) {
 //    tiles per workgroup (every fetched fragment feeds two MFMAs) and one tile per wave while all workgroups are
 //    resident at once (twice the streams in flight), two tiles per wave beyond that;
 //  * few matrices: staging the operand rows is what a workgroup waits for, so one row tile and two tiles per wave
-//    (fewest workgroups re-staging the same rows) until the grid covers the device also with two row tiles.
+//    (fewest workgroups re-staging the same rows) until the grid covers the device also with two row tiles.  One step at a time
+//    takes the shape of many matrices while all its workgroups are resident (training, us per step, 3 channels: N = 1000, B = 300
+//    50.9 -> 47.8, N = 1500, B = 100 79 -> 60, N = 2048, B = 240 94 -> 85; 264 workgroups of 104 KB, N = 1500, B = 330, would take
+//    113 instead of 94); not the rebuild, all steps at once, nor the BPTT with the loss (objective N = 900, 5 channels, B = 300
+//    58.7 -> 59.3).
 // RINGATTR_BLOCK_SHAPE=<rt><tpw> (e.g. 21) forces a shape (cross-checks).
 bool ring_block_many_matrices(int k) { return 1 + k > 6; }
 
-void ring_block_geometry(int NC, int nbt, int k, int* rt_out, int* tpw_out) {
+static void block_geometry(int NC, int nbt, int k, bool pairs, int* rt_out, int* tpw_out) {
   int dev = 0, cus = 0;
   if (hipGetDevice(&dev) != hipSuccess ||
       hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0) cus = 256;
@@ -450,6 +454,10 @@ void ring_block_geometry(int NC, int nbt, int k, int* rt_out, int* tpw_out) {
   } else {
     tpw = 2;
     rt = (block_lds_bytes(NC, 2, k) <= lds_cap && (long)((nbt + 1) / 2) * (NC / 2) >= cus) ? 2 : 1;
+    if (pairs && nbt >= 2 && (long)((nbt + 1) / 2) * NC <= (long)cus * (long)(lds_cap / block_lds_bytes(NC, 2, k))) {
+      rt = 2;
+      tpw = 1;
+    }
   }
   if (const char* v = getenv("RINGATTR_BLOCK_SHAPE")) {
     if ((v[0] == '1' || v[0] == '2') && (v[1] == '1' || v[1] == '2') && v[2] == 0) {
@@ -497,7 +505,7 @@ static hipError_t block_fwd_act(const RingFwdArgs& a, int NC, bool rebuild, int 
 hipError_t ring_launch_block_fwd(const RingFwdArgs& a, int NC, bool rebuild, hipStream_t st) {
   if (NC % 2 != 0) return hipErrorInvalidValue;
   int rt, tpw;
-  ring_block_geometry(NC, a.nbt, a.k, &rt, &tpw);
+  block_geometry(NC, a.nbt, a.k, !rebuild, &rt, &tpw);
   switch (a.act) {
     case ACT_RELU: return block_fwd_act<ACT_RELU>(a, NC, rebuild, rt, tpw, st);
     case ACT_GELU: return block_fwd_act<ACT_GELU>(a, NC, rebuild, rt, tpw, st);
@@ -529,7 +537,7 @@ static hipError_t block_bptt_shape(const RingBpttArgs& a, int NC, float* carry, 
 hipError_t ring_launch_block_bptt(const RingBpttArgs& a, int NC, float* carry, hipStream_t st) {
   if (NC % 2 != 0) return hipErrorInvalidValue;
   int rt, tpw;
-  ring_block_geometry(NC, a.nbt, a.k, &rt, &tpw);
+  block_geometry(NC, a.nbt, a.k, a.loss_coef == nullptr, &rt, &tpw);
   if (a.loss_coef) {
     if (!a.loss_trig || !a.hist) return hipErrorInvalidValue;
     if (rt == 2) return tpw == 2 ? block_bptt_shape<2, 2, true>(a, NC, carry, st) : block_bptt_shape<2, 1, true>(a, NC, carry, st);
