@@ -15,7 +15,7 @@ PKG_DIR = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(PKG_DIR, "csrc")
 INCLUDE = os.path.join(os.path.dirname(PKG_DIR), "include")
 LIB_PATH = os.path.join(PKG_DIR, "libringattr.so")
-SOURCES = ["ring_kernels.hip", "ring_res256.hip", "ring_cluster.hip", "ring_team.hip", "ring_team_fwd.hip",
+SOURCES = ["ring_kernels.hip", "ring_res256.hip", "ring_cluster.hip", "ring_team.hip", "ring_team_fwd.hip", "ring_team_fwd_lds1.hip", "ring_team_fwd_lds4.hip",
            "ring_team_bptt.hip", "ring_team_bptt_ga.hip", "ring_team_solo.hip", "ring_team_rows.hip", "ring_team_one.hip", "ring_dw.hip", "ring_loss.hip", "ring_gain.hip", "ring_bign.hip", "ring_block.hip", "ring_panel.hip", "ring_chip.hip", "ring_aux.hip", "ringattr_api.hip"]
 ARCH = os.environ.get("RINGATTR_ARCH", "gfx950")
 

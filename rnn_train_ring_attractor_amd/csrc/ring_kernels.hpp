@@ -309,6 +309,8 @@ hipError_t ring_launch_team_one_bptt(const RingBpttArgs& a, const RingTeamArgs& 
 hipError_t ring_team_rebuild(const RingFwdArgs& a, bool folded, int cts, hipStream_t st);
 hipError_t ring_launch_team_rebuild(const RingFwdArgs& a, const RingTeamArgs& c, int wk, hipStream_t st);
 hipError_t ring_launch_team_fwd(const RingFwdArgs& a, const RingTeamArgs& c, const RingTeamShape& sh, hipStream_t st);
+hipError_t ring_launch_team_fwd_lds1(const RingFwdArgs& a, const RingTeamArgs& c, const RingTeamShape& sh, hipStream_t st);
+hipError_t ring_launch_team_fwd_lds4(const RingFwdArgs& a, const RingTeamArgs& c, const RingTeamShape& sh, hipStream_t st);
 hipError_t ring_launch_team_bptt(const RingBpttArgs& a, const RingTeamArgs& c, const RingTeamShape& sh, hipStream_t st);
 hipError_t ring_launch_team_bptt_ga(const RingBpttArgs& a, const RingTeamArgs& c, const RingTeamShape& sh, hipStream_t st);
 // the teams that did not gather, a workgroup per batch tile (ring_team_solo.hip)

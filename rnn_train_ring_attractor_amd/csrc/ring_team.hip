@@ -47,7 +47,7 @@ size_t shape_lds(const RingTeamShape& s, int k, int nt, int KC, bool bptt, bool 
 }
 
 const RingTeamShape kShapes[] = {
-#define RING_TEAM_ROW(KPW, C16, MR, WK, EX) {KPW, C16, MR, WK, EX, 0},      // (lds_mats here: whether there may be any)
+#define RING_TEAM_ROW(KPW, C16, MR, WK, FEW, MORE) {KPW, C16, MR, WK, MORE ? TEAM_MORE : FEW, 0},      // (lds_mats here: how many there may be)
     RING_TEAM_SHAPES(RING_TEAM_ROW)
 #undef RING_TEAM_ROW
 };
@@ -76,7 +76,7 @@ RingTeamPlan ring_team_plan(int N, int k, int T, int B, bool bptt, bool ga) {
     if (s.wk == 4 ? KC > 4 : KC <= 4) continue;
     if (s.kpw != (KC + s.wk - 1) / s.wk) continue;
     s.lds_mats = std::max(0, k + 1 - s.mr);
-    if (s.lds_mats > 0 && !s0.lds_mats) continue;
+    if (s.lds_mats > s0.lds_mats) continue;
     const int G = (2 * KC + s.c16 - 1) / s.c16;
     if (G > CUS_PER_XCD) continue;
     const int nteams = std::min(nbt, XCDS * (CUS_PER_XCD / G)), nt = (nbt + nteams - 1) / nteams;

@@ -228,9 +228,11 @@ __host__ __device__ inline LdsPlan lds_plan(int k, int nt, int lds_mats, int KC,
 }
 
 // ------------------------------------------------------------------------------------------------
-// Compute role, shared by forward and BPTT.
+// Compute role, shared by forward and BPTT.  EX: matrices in LDS, none, exactly that many, or TEAM_MORE: any number.
 // ------------------------------------------------------------------------------------------------
-template <int KPW, int C16, int MR, int WK, bool EX, bool GA>
+constexpr int TEAM_MORE = 100;
+
+template <int KPW, int C16, int MR, int WK, int EX, bool GA>
 struct TeamCompute {
   static constexpr int F = MR * C16 * KPW, FR = F - parked_fragments<KPW, C16, MR, GA>();
   bf16x8 wreg[FR];                 // fragment (matrix, column tile, chunk) in that order
@@ -363,8 +365,8 @@ struct TeamOperand {
 };
 
 // One item's products: acc[c] = J1 * P_0 + J0 * rowsum + sum_m gate_m P_m over this wave's K chunks: the matrices in registers
-// and those in LDS up to channel `last`.
-template <int KPW, int C16, int MR, int WK, bool EX, bool GA>
+// and those in LDS (any number of them: up to channel `last`).
+template <int KPW, int C16, int MR, int WK, int EX, bool GA>
 __device__ __forceinline__ void team_products(const TeamCompute<KPW, C16, MR, WK, EX, GA>& tc, const TeamOperand<KPW>& op,
                                               const RingTeamArgs& c, const bf16x8* wl, const float (&gate)[MR], const float* gates,
                                               const f32x4* rows, float* ga, int w, int lane, int last, f32x4 (&acc)[C16]) {
@@ -418,28 +420,37 @@ __device__ __forceinline__ void team_products(const TeamCompute<KPW, C16, MR, WK
     }
     if (GA && m <= c.k) row_put(d, m);
   }
-  if constexpr (EX) {
+  auto lds_matrix = [&](int m, float gm) {
+    // a channel that is zero for all 16 rows contributes nothing (zero-padded action signals); dL/dA needs every product
+    if (!GA && __ballot(gm != 0.f) == 0) return;
+    float d = 0.f;
+#pragma unroll
+    for (int cc = 0; cc < C16; ++cc) {
+      f32x4 P = zero;
+      const bf16x8* src = wl + ((size_t)((m - MR) * C16 + cc) * c.KC + w) * 64 + lane;
+#pragma unroll
+      for (int kk = 0; kk < KPW; ++kk)
+        if (kk + 1 < KPW || w + WK * kk < c.KC) P = mfma16(src[(size_t)WK * kk * 64], x[kk], P);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) acc[cc][i] = fmaf(gm, P[i], acc[cc][i]);
+      row_dot(d, P, cc);
+    }
+    row_put(d, m);
+  };
+  if constexpr (EX == TEAM_MORE) {
     // (gates are read a matrix ahead: forward N = 512, 16 channels, B = 256, T = 20 95.5 -> 93.2 us, N = 168, B = 223, T = 76 158.7 -> 152.3)
     float gn = gates[(MR - 1) * 16 + b];
     for (int m = MR; m <= last; ++m) {
       const float gm = gn;
       gn = gates[(m < c.k ? m : c.k - 1) * 16 + b];
-      // a channel that is zero for all 16 rows contributes nothing (zero-padded action signals); dL/dA needs every product
-      if (!GA && __ballot(gm != 0.f) == 0) continue;
-      float d = 0.f;
-#pragma unroll
-      for (int cc = 0; cc < C16; ++cc) {
-        f32x4 P = zero;
-        const bf16x8* src = wl + ((size_t)((m - MR) * C16 + cc) * c.KC + w) * 64 + lane;
-#pragma unroll
-        for (int kk = 0; kk < KPW; ++kk)
-          if (kk + 1 < KPW || w + WK * kk < c.KC) P = mfma16(src[(size_t)WK * kk * 64], x[kk], P);
-#pragma unroll
-        for (int i = 0; i < 4; ++i) acc[cc][i] = fmaf(gm, P[i], acc[cc][i]);
-        row_dot(d, P, cc);
-      }
-      row_put(d, m);
+      lds_matrix(m, gm);
     }
+  } else if constexpr (EX > 0) {
+    float g[EX];
+#pragma unroll
+    for (int i = 0; i < EX; ++i) g[i] = gates[(MR - 1 + i) * 16 + b];
+#pragma unroll
+    for (int i = 0; i < EX; ++i) lds_matrix(MR + i, g[i]);
   }
 }
 
@@ -491,12 +502,12 @@ __device__ __forceinline__ bool team_go(const char* lds, const LdsPlan& L) {
 
 // The compute waves' loop: `steps` rounds over the team's my_nt tiles, operand number s of round s.
 // (TR: with the transposed matrices)
-template <bool TR, int KPW, int C16, int MR, int WK, bool EX, bool GA>
+template <bool TR, int KPW, int C16, int MR, int WK, int EX, bool GA>
 __device__ __forceinline__ void team_compute_loop(const RingTeamArgs& c, const LdsPlan& L, char* lds,
                                                   __amdgpu_buffer_rsrc_t rsrc, int mem, int team, int my_nt, int steps, int w,
                                                   int lane) {
   using AM = AuxMap<C16>;
-  constexpr bool PADS = EX && MR == 3 && !GA;             // (dL/dA needs every product)
+  constexpr bool PADS = EX == TEAM_MORE && MR == 3 && !GA;             // (dL/dA needs every product)
   TeamCompute<KPW, C16, MR, WK, EX, GA> tc;
   bf16x8* const wl = reinterpret_cast<bf16x8*>(lds + L.weights);
   tc.template load_weights<TR>(c, wl, reinterpret_cast<bf16x8*>(lds + L.parked), mem, w, lane);
@@ -785,16 +796,23 @@ __device__ __forceinline__ bool team_coords(const RingTeamArgs& c, int& team, in
 
 }  // namespace
 
-// Shapes that are built: K chunks per compute wave, column tiles per member, matrices in registers, compute waves, and
-// whether also with further matrices in LDS.  (kpw * wk chunks cover the contraction; c16 * kpw * mr weight fragments of
+// Shapes that are built: K chunks per compute wave, column tiles per member, matrices in registers, compute waves, up to how many
+// further matrices in LDS there is a kernel for exactly that number, and whether there is one for any number (not where LDS or a cheaper
+// shape leaves no call for it).  (kpw * wk chunks cover the contraction; c16 * kpw * mr weight fragments of
 // four registers per wave.  Past N = 512 one column tile per member would make teams of more than an XCD's 32 compute
 // units; four at 256 < N <= 512 leave LDS room for a further matrix only up to N = 288, where two are as fast: N = 257,
 // a_dim 3, B = 1395, T = 60 forward 235 us with four, 233 with two.)
-#define RING_TEAM_SHAPES(X)                                                                              \
-  X(1, 1, 3, 4, true) X(1, 2, 3, 4, true) X(1, 4, 3, 4, true)                                            \
-  X(1, 1, 3, 8, true) X(1, 2, 3, 8, true) X(1, 4, 3, 8, true) X(1, 1, 9, 8, true) X(1, 2, 13, 8, true)   \
-  X(2, 1, 3, 8, true) X(2, 2, 3, 8, true) X(2, 4, 3, 8, false) X(2, 1, 9, 8, true) X(2, 1, 13, 8, true)  \
-  X(3, 2, 3, 8, true) X(4, 2, 3, 8, true)
+// One to four matrices in LDS with three in registers, or one with nine, are multiplied without a loop, their gates read together and
+// no look at whether all of them are silent; us a call of T = 40 with the loop of any number -> without: forward N = 653, 3 channels,
+// B = 973 393 -> 358, N = 700, 4 channels, B = 500 239 -> 215, N = 144, 5 channels, B = 900 114 -> 95, N = 300, 9 channels, B = 800
+// 291 -> 285; training N = 300, 6 channels, B = 800 500 -> 462; with two of six driven forward 107 -> 109.  One with thirteen: N = 500,
+// 13 channels, B = 300 179 -> 184.  One kernel for up to four, each behind a test of the number of channels: N = 653 372, N = 700 222,
+// N = 144 101, two of six driven 117.
+#define RING_TEAM_SHAPES(X)                                                                                                  \
+  X(1, 1, 3, 4, 0, true) X(1, 2, 3, 4, 0, true) X(1, 4, 3, 4, 0, true)                                                       \
+  X(1, 1, 3, 8, 3, false) X(1, 2, 3, 8, 4, true) X(1, 4, 3, 8, 3, false) X(1, 1, 9, 8, 1, true) X(1, 2, 13, 8, 0, true)      \
+  X(2, 1, 3, 8, 3, false) X(2, 2, 3, 8, 4, true) X(2, 4, 3, 8, 0, false) X(2, 1, 9, 8, 1, true) X(2, 1, 13, 8, 0, true)      \
+  X(3, 2, 3, 8, 2, false) X(4, 2, 3, 8, 1, false)
 
 // Launches one team kernel.
 template <typename F>

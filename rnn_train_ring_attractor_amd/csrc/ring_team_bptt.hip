@@ -9,10 +9,14 @@ hipError_t ring_launch_team_bptt(const RingBpttArgs& a, const RingTeamArgs& c, c
                          [&](dim3 g, dim3 b, unsigned lds) {                                                          \
                            RING_LAUNCH((ring_team_bptt_kernel<KPW, C16, MR, WK, EX, GA>), g, b, lds, st, a, c);       \
                          })
-#define RING_TEAM_CASE(KPW, C16, MR, WK, EX)                                                                          \
+#define RING_TEAM_CASE(KPW, C16, MR, WK, FEW, MORE)                                                                   \
   if (sh.kpw == KPW && sh.c16 == C16 && sh.mr == MR && sh.wk == WK) {                                                 \
-    if (sh.lds_mats == 0) RING_TEAM_RUN(KPW, C16, MR, WK, false);                                                     \
-    if constexpr (EX) RING_TEAM_RUN(KPW, C16, MR, WK, true);                                                          \
+    if (sh.lds_mats == 0) RING_TEAM_RUN(KPW, C16, MR, WK, 0);                                                         \
+    if constexpr (FEW >= 1) if (sh.lds_mats == 1) RING_TEAM_RUN(KPW, C16, MR, WK, 1);                                 \
+    if constexpr (FEW >= 2) if (sh.lds_mats == 2) RING_TEAM_RUN(KPW, C16, MR, WK, 2);                                 \
+    if constexpr (FEW >= 3) if (sh.lds_mats == 3) RING_TEAM_RUN(KPW, C16, MR, WK, 3);                                 \
+    if constexpr (FEW >= 4) if (sh.lds_mats == 4) RING_TEAM_RUN(KPW, C16, MR, WK, 4);                                 \
+    if constexpr (MORE) RING_TEAM_RUN(KPW, C16, MR, WK, TEAM_MORE);                                                   \
   }
   RING_TEAM_SHAPES(RING_TEAM_CASE)
 #undef RING_TEAM_CASE

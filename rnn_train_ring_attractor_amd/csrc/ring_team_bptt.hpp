@@ -6,7 +6,7 @@
 // BPTT, reverse time.  Operand number s is g of step T - 1 - s; the products of round s give the carry into step
 // T - 2 - s (the last round, which only grad_r_init needs, is left out when that is not asked for).
 // ------------------------------------------------------------------------------------------------
-template <int KPW, int C16, int MR, int WK, bool EX, bool GA>
+template <int KPW, int C16, int MR, int WK, int EX, bool GA>
 __global__ __launch_bounds__(64 * (WK + AUX)) void ring_team_bptt_kernel(RingBpttArgs p, RingTeamArgs c) {
   extern __shared__ __attribute__((aligned(16))) char lds[];
   int team, mem;

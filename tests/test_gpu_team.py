@@ -548,3 +548,29 @@ def test_channels_that_are_silent_in_some_items(N, B, k, gpu_device):
     assert O.max_rel_err(hist.detach().cpu().numpy(), ref) <= 1e-2
     for got, want in ((Wo.grad, g["grad_Wo"]), (Wa.grad, g["grad_Wa"])):
         assert O.cosine(got.cpu().numpy(), want) >= 0.999 and O.max_rel_err(got.cpu().numpy(), want) <= 2e-2
+
+
+# a case for every kernel that is built for an exact number of matrices in LDS (K chunks 1 to 4 a wave, one to four column tiles a
+# member, three or nine matrices in registers)
+@pytest.mark.parametrize("B,k,N", [
+    (9, 3, 144), (9, 4, 144), (9, 5, 144), (9, 9, 144), (521, 3, 200), (777, 4, 200), (777, 5, 200), (777, 6, 200), (1545, 3, 200), (1545, 4, 200),
+    (2313, 5, 144), (9, 3, 260), (9, 4, 260), (9, 5, 260), (9, 9, 260), (393, 3, 260), (393, 4, 260), (265, 5, 290), (265, 6, 260), (9, 3, 520),
+    (9, 4, 520), (9, 3, 800)])
+def test_few_matrices_in_lds(B, k, N, gpu_device, teams, monkeypatch):
+    """Their channels all driven, one of them silent, all of them silent, gates of minus zero: the bits of the single workgroups, and the
+    oracle for the first rows."""
+    print(f"[case] few matrices in LDS B={B} k={k} N={N}", flush=True)
+    T = 5
+    p = make_problem(700 + N + k, B, T, k, N, action="dense")
+    A = p["A"]
+    A[:, 1, 2:] = 0.0
+    A[:16, 2, -1] = -0.0
+    A[:, 3, -2:-1] = 0.0
+    for ga in (True, False):
+        want = _run(p, "gelu", -1.0 / N, 0.6, gpu_device, ga=ga)
+        monkeypatch.setenv("RINGATTR_TEAM_GATHER_US", "-1")
+        got = _run(p, "gelu", -1.0 / N, 0.6, gpu_device, ga=ga)
+        monkeypatch.delenv("RINGATTR_TEAM_GATHER_US")
+        assert all(torch.equal(got[x], want[x]) for x in want), [x for x in want if not torch.equal(got[x], want[x])]
+    ref, _ = O.forward_dense(A[:9], p["Wa"], -1.0 / N, 0.6, p["Wo"], p["r0"][:9], 0.15, "gelu")
+    assert O.max_rel_err(want["hist"][:, :9].cpu().numpy(), ref) <= TRAJ_TOL
