@@ -279,21 +279,27 @@ __global__ __launch_bounds__(256) void ring_block_bptt_kernel(RingBpttArgs p, in
   const int j4 = j0 & ~3, jo = j0 & 3;                    // the 16-byte group holding the lane's TPW neurons
   GateRows<RT> gates;
   if (staged) gates.fetch(p.A, p.k, T, B, t, bt0, tid);
-  // the lane's own rows and neurons (on their way while the rows are staged)
+  // The lane's own rows and neurons (on their way while the rows are staged).  What the loss adds to two row tiles is asked for behind
+  // the staging: held across it, it took 245 + 24 registers and with them one of the two waves per SIMD that the geometry counts
+  // on (objective, us a call of T = 20: N = 576, 12 channels, B = 600 3409 -> 2699, N = 761, 8 channels, B = 1000 3240 -> 2751; with
+  // few workgroups, N = 1000, 16 channels, B = 64, 1150 -> 1157, and 1169 with the coefficients left in LDS by the staging).
+  constexpr bool LATE = LOSS && RT > 1;
   GradRaw<LOSS> own[RT][4];
   GradCoef own_coef[RT][4];
   GradTrig own_trig;
   with_whole(N, [&](auto whole) {
     const GradRows<LOSS, decltype(whole)::value> src(p, t, 16 * bt0, 16 * RT, NPAD, carry_in, up);
+#pragma unroll
+    for (int i = 0; i < RT; ++i)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) own[i][e] = src.load_row(16 * i + 4 * q + e, j4);
+    if constexpr (LATE) stage_rows<RT>(xb, slots, rs, NPAD, tid, src);
     own_trig = src.load_trig(j4);
 #pragma unroll
     for (int i = 0; i < RT; ++i)
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        own[i][e] = src.load_row(16 * i + 4 * q + e, j4);
-        own_coef[i][e] = src.row(16 * i + 4 * q + e);
-      }
-    stage_rows<RT>(xb, slots, rs, NPAD, tid, src);
+      for (int e = 0; e < 4; ++e) own_coef[i][e] = src.row(16 * i + 4 * q + e);
+    if constexpr (!LATE) stage_rows<RT>(xb, slots, rs, NPAD, tid, src);
   });
   if (staged) gates.put(gl, p.A, p.k, T, B, t, bt0, tid);
   lds_barrier();

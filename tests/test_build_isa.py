@@ -126,6 +126,19 @@ def test_hot_kernels_use_no_scratch(res256_asm):
     assert seen >= 12
 
 
+def test_block_kernels_keep_two_waves_per_simd(tmp_path):
+    """block_geometry counts workgroups of four waves as resident by their LDS alone, two per compute unit at 512 < N <= 1024: their
+    registers must not allow fewer."""
+    proc = subprocess.run([HIPCC, "--offload-arch=gfx950", "-O3", "-std=c++17", "-c", "--cuda-device-only", f"-I{ROOT}/include", f"-I{CSRC}",
+                           "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops", *PER_SOURCE_FLAGS.get("ring_block.hip", []),
+                           "-Rpass-analysis=kernel-resource-usage", os.path.join(CSRC, "ring_block.hip"), "-o", str(tmp_path / "block.o")],
+                          capture_output=True, text=True)
+    assert proc.returncode == 0, proc.stderr[-2000:]
+    kernels = re.findall(r"Function Name: (_Z2[12]ring_block_(?:fwd|bptt)_kernel\S+).*?Occupancy \[waves/SIMD\]: (\d+)", proc.stderr, re.S)
+    assert len(kernels) >= 40
+    assert all(int(waves) >= 2 for _, waves in kernels), [k for k in kernels if int(k[1]) < 2]
+
+
 # ------------------------------------------------------------------------------------------------
 # The N = 512 cluster forward issues its flag, gate, previous-state and operand loads with inline assembly as
 # well and waits for them with counted s_waitcnt.  Same proof on its emitted code: between such a load and the first
