@@ -165,13 +165,25 @@ struct NoStores {};
 
 }  // namespace
 
+namespace {
+
+// What keeps a ragged ring's or batch's surplus at zero: a lane mask in scalar registers, or a factor of 0 or 1.  Masks where factors
+// would spill, factors where masks spill scalars without need or, with relu, cost more than the vector registers they spare.
+template <bool LANES> using RingKeep = std::conditional_t<LANES, bool, float>;
+__device__ __forceinline__ float kept(bool keep, float v) { return keep ? v : 0.f; }
+__device__ __forceinline__ float kept(float keep, float v) { return v * keep; }
+
+}  // namespace
+
 // STATS: also leave the loss head's three sums of every history row (sum_i r_i cos(phi_i), sum_i r_i sin(phi_i),
 // sum_i |r_i|, phi_i = 2 pi i / N) in p.loss_stats[t * B + b], so that the loss needs no pass of its own over the
 // history.  Each wave reduces its 32 neurons' share over the row group's 16 lanes, a sum at a time between the matrix
 // instructions of the following contraction, the eight shares meet in LDS (buffer by step parity) and wave 0 adds them in wave
 // order a step later.  (Reduced right after the activation, in front of the barrier that the other role waits at, the sums were
 // on the step's serial chain: forward of T = 100, gelu, N = 256, B = 1024 211 -> 169 us, without the sums 144; N = 200 209 -> 176.
-// At B = 4096 the history's stores bound the step and nothing changes.)
+// At B = 4096 the history's stores bound the step and nothing changes.  Not with relu, whose activation leaves the vector unit time
+// enough: there they follow it, a sum over both rows' lanes each as above; objective, N = 256, B = 1180 457 -> 421 us a call, B = 2048
+// 439 -> 414.)
 template <int ACT, bool SAVE, bool FULL, bool STATS>
 __global__ __launch_bounds__(512) void ring_fwd_res256_kernel(RingFwdArgs p) {
   extern __shared__ __attribute__((aligned(16))) char smem[];
@@ -199,7 +211,7 @@ __global__ __launch_bounds__(512) void ring_fwd_res256_kernel(RingFwdArgs p) {
   load_resident8(reinterpret_cast<const bf16x8*>(p.Wpack), wl, wreg, w, h, lane);
 
   float r[4][2];
-  bool ok[4][2];
+  RingKeep<ACT != ACT_RELU> ok[4][2];     // (training, factors and masks: gelu, N = 200, B = 1024 358 and 353 us a call; relu, N = 256, B = 968 347 and 349)
   // alpha F', or what it is made of (late role of whole tiles), until it is stored
   using Record = ActRecord<ACT>;
   float d[4][2];
@@ -208,8 +220,9 @@ __global__ __launch_bounds__(512) void ring_fwd_res256_kernel(RingFwdArgs p) {
   for (int e = 0; e < 4; ++e)
 #pragma unroll
     for (int cc = 0; cc < 2; ++cc) {
-      ok[e][cc] = (b0 + e < B) && (i0 + cc < N);
-      r[e][cc] = ok[e][cc] ? p.r_init[(size_t)(b0 + e) * N + i0 + cc] : 0.f;
+      const bool inside = (b0 + e < B) && (i0 + cc < N);
+      ok[e][cc] = inside;
+      r[e][cc] = inside ? p.r_init[(size_t)(b0 + e) * N + i0 + cc] : 0.f;
     }
   auto save_r = [&](int t) {   // bf16 copy of r_t (operand of step t) for the weight-gradient GEMM
 #pragma unroll
@@ -241,7 +254,15 @@ __global__ __launch_bounds__(512) void ring_fwd_res256_kernel(RingFwdArgs p) {
     const float sum = (high ? hi : lo) + dpp_row<0x128>(high ? lo : hi);          // row_ror:8: the other eight
     share = kind == 0 || (n & 3) == kind ? sum : share;
   };
+  constexpr bool BEHIND = ACT != ACT_RELU;
   auto stat_put = [&](int row_t) { statp[(((row_t & 1) * 8 + w8) * 4 + (n & 3)) * 16 + 4 * q + (n >> 2)] = share; };
+  auto stat_now = [&](int row_t) {
+    if constexpr (STATS && !BEHIND) {
+#pragma unroll
+      for (int kind = 0; kind < 3; ++kind) stat_sum(kind);
+      stat_put(row_t);
+    }
+  };
   // the eight shares of row `row_t` are complete behind a barrier: wave 0 adds them in wave order and stores the row sums
   auto stat_flush = [&](int row_t) {
     if (wu == 0 && hu == 0) {
@@ -299,9 +320,11 @@ __global__ __launch_bounds__(512) void ring_fwd_res256_kernel(RingFwdArgs p) {
   auto emit_store = [&](int t, int slot, auto once) {
     __builtin_amdgcn_sched_barrier(0);
     if constexpr (STATS) {
-      if (slot < 3) stat_sum(slot);
-      if (slot == 3) stat_put(t);
-      if (slot == 5 && t > 0) stat_flush(t - 1);         // (step t's contraction: the shares came in before its first barrier)
+      // (row t goes out in step t + 1's contraction.  Behind: row t - 1's shares came in before that step's barrier A; else row t's
+      // before its barrier B, which slots 4 and up follow, but for the last row, flushed at the end)
+      if (BEHIND && slot < 3) stat_sum(slot);
+      if (BEHIND && slot == 3) stat_put(t);
+      if (slot == 5 && (BEHIND ? t > 0 : t + 1 < T)) stat_flush(BEHIND ? t - 1 : t);
     }
     if (slot < 4) {
       if (p.hist == nullptr) return;   // recompute of the saved record only: the history already exists
@@ -412,10 +435,9 @@ __global__ __launch_bounds__(512) void ring_fwd_res256_kernel(RingFwdArgs p) {
         else act_scaled<ACT>(x[e][cc], asc, aF, d[e][cc]);
         float rn = fmaf(oma, r[e][cc], aF);
         if constexpr (!FULL) {
-          // (lanes' masks in scalar registers: eight factors of 0 or 1 spilled up to 23 registers here, 20 in the BPTT with the loss
-          // and dL/dA: N = 201, B = 1748 3.54 -> 3.37 us per step)
-          rn = ok[e][cc] ? rn : 0.f;
-          d[e][cc] = ok[e][cc] ? d[e][cc] : 0.f;   // (never `once`)
+          // (eight factors of 0 or 1 spilled up to 23 registers here, with the sums and gelu)
+          rn = kept(ok[e][cc], rn);
+          d[e][cc] = kept(ok[e][cc], d[e][cc]);    // (never `once`)
         }
         r[e][cc] = rn;
       }
@@ -434,6 +456,7 @@ __global__ __launch_bounds__(512) void ring_fwd_res256_kernel(RingFwdArgs p) {
       float x[4][2];
       preactivation(t, x);
       activate(x, std::false_type{});
+      stat_now(t);
       if (t + 1 < T) write_half(xE + ((t + 1) & 1) * R8_HALF_SLOTS, r, w, q, n);
       // the next chunk's gates are first read after barrier B of its first step
       if (l == R_GCH - 1 && t + 1 < T) gates_publish(gbuf + ((ci + 1) & 1) * R_GCH * 16, tid, B, bt, gs);
@@ -451,6 +474,7 @@ __global__ __launch_bounds__(512) void ring_fwd_res256_kernel(RingFwdArgs p) {
     lds_barrier();   // A_1
     for (int t = 1; t < T; ++t) {
       activate(x, late_once);   // step t-1 -> r^L_t
+      stat_now(t - 1);
       write_half(xL, r, w, q, n);
       lds_barrier();   // B_t
       contract_half(0, xE + (t & 1) * R8_HALF_SLOTS, t - 1, late_once);
@@ -459,6 +483,7 @@ __global__ __launch_bounds__(512) void ring_fwd_res256_kernel(RingFwdArgs p) {
       lds_barrier();   // A_{t+1}
     }
     activate(x, std::false_type{});
+    stat_now(T - 1);
   }
   // stores of the last step (its state is not an operand of any further step)
 #pragma unroll
@@ -681,7 +706,10 @@ __global__ __launch_bounds__(256) void ring_bptt_res256_kernel(RingBpttArgs p) {
   load_resident(reinterpret_cast<const bf16x8*>(p.Wpack), wl, wreg, w, lane);
 
   float carry[4][R_NC];
-  bool ok[4][R_NC];
+  // (masks: with the loss and dL/dA factors spilled 20 registers, N = 201, B = 1748 3.54 -> 3.37 us per step; with dL/dA alone N = 256,
+  // B = 1000, T = 100 420 -> 404 us a call; with neither N = 200, B = 1024 175 -> 173.  With the loss alone factors fit, masks spill seven
+  // scalars: N = 250, B = 2000 241 against 245)
+  RingKeep<!LOSS || GA> ok[4][R_NC];
 #pragma unroll
   for (int e = 0; e < 4; ++e)
 #pragma unroll
@@ -821,7 +849,7 @@ __global__ __launch_bounds__(256) void ring_bptt_res256_kernel(RingBpttArgs p) {
         for (int e = 0; e < 4; ++e) {
           float x = fmaf(gate[e][0], P1[e], P0[e]);
           x = fmaf(gate[e][1], P2[e], x);
-          if constexpr (!FULL) x = ok[e][c] ? x : 0.f;
+          if constexpr (!FULL) x = kept(ok[e][c], x);
           carry[e][c] = x;
         }
         if constexpr (GA) {

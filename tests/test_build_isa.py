@@ -126,6 +126,13 @@ def test_hot_kernels_use_no_scratch(res256_asm):
     assert seen >= 12
 
 
+def test_masked_bptt_with_the_loss_spills_nothing(res256_asm):
+    """Sixteen lane masks are 32 scalar registers; where sixteen factors fit the vector registers they are the cheaper form."""
+    _, remarks = res256_asm
+    m = re.search(r"Function Name: _Z23ring_bptt_res256_kernelILb0ELb1ELb0ELi2ELb0EE.*?SGPRs Spill: (\d+).*?VGPRs Spill: (\d+)", remarks, re.S)
+    assert m and m.groups() == ("0", "0")
+
+
 def test_block_kernels_keep_two_waves_per_simd(tmp_path):
     """block_geometry counts workgroups of four waves as resident by their LDS alone, two per compute unit at 512 < N <= 1024: their
     registers must not allow fewer."""

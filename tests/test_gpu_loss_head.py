@@ -230,3 +230,18 @@ def test_row_sums_of_the_weight_resident_forward(N, B, T, act, gpu_device):
         total, lc, la, hist = ring_rnn_loss_func(t(p["A"]), t(p["Wa"]), -1.0 / N, 2.0 / N, Wo, t(p["r0"]), 0.15, act, t(p["angle"]), 0.2)
         for got, want in zip((total, lc, la), ring_loss_pair(hist.detach(), t(p["angle"]), 0.2)):
             assert abs(float(got.detach()) - float(want)) <= 2e-5 * max(1.0, abs(float(want)))
+
+
+@pytest.mark.parametrize("N,B,T", [(256, 528, 1), (256, 528, 3), (256, 1024, 34), (129, 513, 2), (200, 530, 35)])
+def test_row_sums_right_after_the_activation(N, B, T, gpu_device):
+    """relu forms them there, not a step behind: every row's, odd and even, first and last, with the bound of the test above."""
+    from rnn_train_ring_attractor_amd import ring_loss_pair, ring_rnn_loss_func
+    from tests.ring_cases import make_problem
+    print(f"[case] relu row sums N={N} B={B} T={T}", flush=True)
+    p = make_problem(N + T, B, T, 2, N, weights="perfect")
+    t = lambda x: torch.tensor(x, device=gpu_device)
+    for record in (False, True):
+        Wo = t(p["Wo"]).requires_grad_(record)
+        total, lc, la, hist = ring_rnn_loss_func(t(p["A"]), t(p["Wa"]), -1.0 / N, 2.0 / N, Wo, t(p["r0"]), 0.15, "relu", t(p["angle"]), 0.2)
+        for got, want in zip((total, lc, la), ring_loss_pair(hist.detach(), t(p["angle"]), 0.2)):
+            assert abs(float(got.detach()) - float(want)) <= 2e-5 * max(1.0, abs(float(want)))
