@@ -33,7 +33,8 @@
 // and 6, 6 with three (two) and 6, 3 from four (three) up and 4.
 //
 // Residence: as in ring_team.hpp a row group counts itself before the time loop and gives up as a whole if it is not complete in
-// time; ring_chip_solo_kernel behind this launch does the tiles of groups that gave up, a workgroup each, with the same bits.
+// time; ring_chip_rest_kernel behind this launch does the tiles of groups that gave up, with the same bits, on what compute units
+// there are.
 #include "ring_team.hpp"
 
 #include <stdlib.h>
@@ -51,7 +52,9 @@ struct RingChipArgs {
   const float *A, *Wo, *Wa, *r_init;
   float* hist;
   void* xchg;                    // [slots][batch tiles][K chunks][1280 bytes], all 0xFF at launch
-  unsigned long long* gather;    // a word per row group, 0 at launch: members that are resident; top bit: given up
+  // A word per row group, 0 at launch: members that are resident; top bit: given up.  Behind them ring_chip_rest_kernel's, 0 at launch:
+  // units drawn, and per tile block those that are done.
+  unsigned long long* gather;
   int* host_err;
   unsigned xchg_bytes;
   float J0, J1, alpha;
@@ -468,71 +471,149 @@ __global__ __launch_bounds__(64 * W) void ring_chip_fwd_kernel(RingChipArgs c) {
   }
 }
 
-// The tiles of row groups that gave up: a workgroup of eight waves per tile, every sum in the order of the kernel above.  The state's
-// fragments and row sums of one step are in LDS; weights come from memory for every step.  (What it costs does not matter
-// much: it runs where other work holds compute units for longer than the gathering waits.)
-__global__ __launch_bounds__(512) void ring_chip_solo_kernel(RingChipArgs c) {
-  extern __shared__ __attribute__((aligned(16))) char lds[];
-  const int bt = blockIdx.x;
-  if (!(__hip_atomic_load(c.gather + (size_t)(bt % c.nrg) * RING_TEAM_WORD, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) & CHIP_GAVE_UP)) return;
+// Eight consecutive neurons of a row of N; past the end: zero.
+template <bool WHOLE>
+__device__ __forceinline__ void row_eight(const float* row, int N, int j, f32x4& lo, f32x4& hi) {
+  if constexpr (WHOLE) {                  // (N is a multiple of four)
+    const f32x4 zero = {0.f, 0.f, 0.f, 0.f}, a = *reinterpret_cast<const f32x4*>(row + (j < N ? j : 0)), b = *reinterpret_cast<const f32x4*>(row + (j + 4 < N ? j + 4 : 0));
+    lo = j < N ? a : zero;
+    hi = j + 4 < N ? b : zero;
+  } else {
+    lo = row_quad(row, N, j);
+    hi = row_quad(row, N, j + 4);
+  }
+}
+
+// The tiles of row groups that gave up, on as many workgroups as there are compute units free, with every sum in the order of the
+// kernel above.  A unit of work is a step of RT tiles and 16 neurons; workgroups draw units in the order of their steps and wait
+// for the step before of the same tiles.  Whoever is waited for has drawn earlier and is running, so this ends with any number of
+// workgroups resident, one included.  Weights come from memory for every unit (fp32, read while the wait lasts), the state from the
+// history.  A unit's wave w contracts its chunks w, w + 8, ... of all matrices; the eight shares meet in LDS.
+template <int KPW, int RT>
+__global__ __launch_bounds__(64 * W) void ring_chip_rest_kernel(RingChipArgs c) {
+  __shared__ f32x4 share[W][RT][64];
+  __shared__ unsigned long long drawn;
   const int tid = threadIdx.x, w = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, q = lane >> 4, b = lane & 15;
-  const int N = c.N, B = c.B, T = c.T, k = c.k, KC = c.KC;
-  bf16x8* const xs = reinterpret_cast<bf16x8*>(lds);                          // [KC][64]
-  float* const rs = reinterpret_cast<float*>(lds + (size_t)KC * 1024);       // [KC][16 rows][4]
-  float* const gl = rs + (size_t)KC * 64;                                     // [k + 1][16]
+  const unsigned long long word = __hip_atomic_load(c.gather + (size_t)(lane < c.nrg ? lane : 0) * RING_TEAM_WORD, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  const unsigned groups = (unsigned)__ballot(lane < c.nrg && (word & CHIP_GAVE_UP));
+  if (groups == 0) return;
+  const int N = c.N, B = c.B, T = c.T, k = c.k;
+  const int blocks = (c.nt + RT - 1) / RT, ncg = (N + 15) / 16;                 // tile blocks of a group, column groups
+  const unsigned long long per_step = (unsigned long long)__popc(groups) * blocks * ncg, total = per_step * T;
+  unsigned long long* const rest = c.gather + (size_t)c.nrg * RING_TEAM_WORD;
   const float oma = 1.f - c.alpha;
-  for (int t = 0; t < T; ++t) {
-    const float* prev = t == 0 ? c.r_init : c.hist + (size_t)(t - 1) * B * N;
-    __syncthreads();                                                          // (the step before: its stores have landed, its reads are done)
-    for (int kc = w; kc < KC; kc += 8) {
-      const int row = 16 * bt + b, j = 32 * kc + 8 * q;
-      const float* src = prev + (size_t)(row < B ? row : B - 1) * N;
-      f32x4 lo = row_quad(src, N, j), hi = row_quad(src, N, j + 4);
-      if (row >= B) lo = hi = f32x4{0.f, 0.f, 0.f, 0.f};
-      const u32x4 v = {not_empty(pack_bf16(lo[0], lo[1])), not_empty(pack_bf16(lo[2], lo[3])), not_empty(pack_bf16(hi[0], hi[1])),
-                       not_empty(pack_bf16(hi[2], hi[3]))};
-      xs[kc * 64 + lane] = __builtin_bit_cast(bf16x8, v);
-      rs[kc * 64 + b * 4 + q] = __builtin_bit_cast(float, not_empty(__builtin_bit_cast(unsigned, sum4(lo) + sum4(hi))));
-    }
-    for (int u = tid; u < 16 * (k + 1); u += 512) {
-      const int m = u >> 4, row = 16 * bt + (u & 15);
-      gl[u] = m == 0 ? c.J1 : c.A[((size_t)(row < B ? row : B - 1) * T + t) * k + m - 1];
-    }
-    __syncthreads();
-    for (int cg = w; 16 * cg < N; cg += 8) {
-      f32x4 total = {0.f, 0.f, 0.f, 0.f};
-      for (int part = 0; part < W; ++part) {
-        float rsum = 0.f;
-        for (int kc = part; kc < KC; kc += W) rsum += rs[kc * 64 + b * 4 + q];
-        const float j0r = c.J0 * sum_bits45(rsum);
-        f32x4 s[2] = {{j0r, j0r, j0r, j0r}, {0.f, 0.f, 0.f, 0.f}};
-        for (int m = 0; m <= k; ++m) {
-          const float* W_ = m == 0 ? c.Wo : c.Wa + (size_t)(m - 1) * N * N;
-          f32x4 P = {0.f, 0.f, 0.f, 0.f};
-          for (int kc = part; kc < KC; kc += W) {
-            WeightLoad l;
-            weight_load<WEIGHT_ROWS>(l, W_, N, 16 * cg + b, 32 * kc + 8 * q);
-            P = mfma16(weight_fragment(l, N, 16 * cg + b, 32 * kc + 8 * q, 1.f, 0.f), xs[kc * 64 + lane], P);
-          }
-          const float gm = gl[m * 16 + b];
-          f32x4 v = m & 1 ? s[1] : s[0];
+  bool dead = c.spin_max < 0;
+  if (dead && tid == 0) *c.host_err = RING_CLUSTER_ERR_WAIT;
+  auto units = [&](auto whole) {
+    constexpr bool WHOLE = decltype(whole)::value;
+    for (;;) {
+      if (tid == 0) drawn = __hip_atomic_fetch_add(rest, 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      __syncthreads();
+      const unsigned long long u = (unsigned long long)(unsigned)__builtin_amdgcn_readfirstlane((int)(drawn >> 32)) << 32 |
+                                   (unsigned)__builtin_amdgcn_readfirstlane((int)drawn);
+      if (u >= total) return;
+      const int t = (int)(u / per_step), in_step = (int)(u % per_step), block = in_step / ncg, cg = in_step % ncg;
+      unsigned left = groups;
+      for (int i = block / blocks; i > 0; --i) left &= left - 1;
+      const int rg = __ffs(left) - 1, first = block % blocks * RT;
+      auto tile = [&](int i) { return rg + c.nrg * (first + i); };
+      unsigned long long* const done = rest + (size_t)(1 + block) * RING_TEAM_WORD;
+
+      WeightLoad l[KPW];
+      auto chunk = [&](int kk) {
+        int k0 = 32 * (w + W * kk) + 8 * q;
+        asm volatile("" : "+v"(k0));         // (or addresses and masks are kept from one matrix to the next: registers)
+        return k0;
+      };
+      auto load = [&](int m) {
+        const float* W_ = m == 0 ? c.Wo : c.Wa + (size_t)(m - 1) * N * N;
 #pragma unroll
-          for (int e = 0; e < 4; ++e) v[e] = fmaf(gm, P[e], v[e]);
-          if (m & 1) s[1] = v;
-          else s[0] = v;
+        for (int kk = 0; kk < KPW; ++kk) weight_load<WHOLE ? WEIGHT_ROWS4 : WEIGHT_ROWS>(l[kk], W_, N, 16 * cg + b, chunk(kk));
+      };
+      load(0);
+      if (t > 0) {
+        if (tid == 0 && !dead) {
+          const unsigned long long want = (unsigned long long)t * ncg;
+          for (int spins = 0; __hip_atomic_load(done, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < want; ++spins) {
+            if (spins > c.spin_max) {
+              dead = true;
+              *c.host_err = RING_CLUSTER_ERR_WAIT;
+              break;
+            }
+            __builtin_amdgcn_s_sleep(8);
+          }
         }
-        const f32x4 v = s[0] + s[1];
-        total = part == 0 ? v : total + v;
+        __syncthreads();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
       }
-      const int row = 16 * bt + b, j0 = 16 * cg + 4 * q;
-      if (row < B) {
-        const f32x4 r = row_quad(prev + (size_t)row * N, N, j0), aF = {chip_act(c.act, total[0]), chip_act(c.act, total[1]), chip_act(c.act, total[2]), chip_act(c.act, total[3])};
+      const float* const prev = t == 0 ? c.r_init : c.hist + (size_t)(t - 1) * B * N;
+      bf16x8 x[RT][KPW];
+      f32x4 sum[RT][2];                     // the even and the odd matrices
+      const float* gates[RT];
+#pragma unroll
+      for (int i = 0; i < RT; ++i) {
+        const int row = 16 * tile(i) + b;
+        const size_t at = row < B ? row : B - 1;
+        gates[i] = c.A + (at * T + t) * k;
+        float rsum = 0.f;
+#pragma unroll
+        for (int kk = 0; kk < KPW; ++kk) {
+          f32x4 lo, hi;
+          row_eight<WHOLE>(prev + at * N, N, chunk(kk), lo, hi);
+          if (row >= B) lo = hi = f32x4{0.f, 0.f, 0.f, 0.f};
+          x[i][kk] = __builtin_bit_cast(bf16x8, u32x4{not_empty(pack_bf16(lo[0], lo[1])), not_empty(pack_bf16(lo[2], lo[3])),
+                                                      not_empty(pack_bf16(hi[0], hi[1])), not_empty(pack_bf16(hi[2], hi[3]))});
+          rsum += __builtin_bit_cast(float, not_empty(__builtin_bit_cast(unsigned, sum4(lo) + sum4(hi))));
+        }
+        const float j0r = c.J0 * sum_bits45(rsum);
+        sum[i][0] = f32x4{j0r, j0r, j0r, j0r};
+        sum[i][1] = f32x4{0.f, 0.f, 0.f, 0.f};
+      }
+      auto matrix = [&](int m, int odd) {
+        bf16x8 f[KPW];
+#pragma unroll
+        for (int kk = 0; kk < KPW; ++kk) f[kk] = weight_fragment(l[kk], N, 16 * cg + b, chunk(kk), 1.f, 0.f);
+        float g[RT];
+#pragma unroll
+        for (int i = 0; i < RT; ++i) g[i] = m == 0 ? c.J1 : gates[i][m > 0 ? m - 1 : 0];
+        if (m < k) load(m + 1);
+#pragma unroll
+        for (int i = 0; i < RT; ++i) {
+          f32x4 P = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+          for (int kk = 0; kk < KPW; ++kk) P = mfma16(f[kk], x[i][kk], P);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) sum[i][odd][e] = fmaf(g[i], P[e], sum[i][odd][e]);
+        }
+      };
+#pragma unroll 1
+      for (int m = 0; m <= k; m += 2) {
+        matrix(m, 0);
+        if (m < k) matrix(m + 1, 1);
+      }
+#pragma unroll
+      for (int i = 0; i < RT; ++i) share[w][i][lane] = sum[i][0] + sum[i][1];
+      __syncthreads();
+      if (w < RT && 16 * tile(w) + b < B) {
+        f32x4 v = share[0][w][lane];
+        for (int i = 1; i < W; ++i) v += share[i][w][lane];
+        const size_t row = 16 * tile(w) + b;
+        const int j = 16 * cg + 4 * q;
+        const f32x4 r = row_quad(prev + row * N, N, j);
 #pragma unroll
         for (int e = 0; e < 4; ++e)
-          if (j0 + e < N) c.hist[((size_t)t * B + row) * N + j0 + e] = fmaf(c.alpha, aF[e], oma * r[e]);
+          if (j + e < N)
+            __hip_atomic_store(c.hist + ((size_t)t * B + row) * N + j + e, fmaf(c.alpha, chip_act(c.act, v[e]), oma * r[e]), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       }
+      // The stores above go through to where all XCDs see them; here they have arrived.  (Plain stores and a fence, which writes the
+      // whole L2 back for every unit: N = 776, 6 channels, B = 656 208 against 71 us per step.)
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      __syncthreads();
+      if (tid == 0) __hip_atomic_fetch_add(done, 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
-  }
+  };
+  if ((N & 3) == 0) units(std::true_type{});
+  else units(std::false_type{});
 }
 
 // ------------------------------------------------------------------------------------------------
@@ -561,7 +642,13 @@ struct ChipPlan {
   int depth, KC, G, nrg, nt, slots;
   size_t xchg_bytes, gather_bytes;
   float cycles;          // what the model expects of a step
+  int rest_tiles() const { return row.kpw > 4 ? 2 : 4; }       // of a tile block of ring_chip_rest_kernel
 };
+
+// How long a row group gathers: about what the way round it costs.  us a call, here / all groups given up / panel kernels: N = 2048, 12
+// channels, B = 1, T = 60 311 / 3615 / 1429; N = 1100, 2 channels, B = 256, T = 60 487 / 3343 / 887; N = 776, 6 channels, B = 656, T = 20
+// 342 / 1429 / 575.  (A workgroup per tile on its own took 1.37 s, 69 ms and 38 ms, and the gathering 50 ms before that.)
+constexpr int CHIP_GATHER_US = 5000;
 
 ChipPlan chip_plan(int N, int k, int T, int B) {
   ChipPlan best{};
@@ -595,7 +682,8 @@ ChipPlan chip_plan(int N, int k, int T, int B) {
     const float one = 5000.f + 45.f * kc + 25.f * (float)G + 38.f * F - (B < 16 ? 1500.f : 0.f);
     const float cycles = nt == 1 ? one : std::max(1.6f * one, (float)nt * item);
     if (!best.ok || cycles < best.cycles) {
-      best = ChipPlan{true, r, depth, KC, G, nrg, nt, slots, (xbytes + 255) & ~(size_t)255, (size_t)nrg * RING_TEAM_WORD * sizeof(unsigned long long), cycles};
+      best = ChipPlan{true, r, depth, KC, G, nrg, nt, slots, (xbytes + 255) & ~(size_t)255, 0, cycles};
+      best.gather_bytes = (size_t)(nrg + 1 + nrg * ((nt + best.rest_tiles() - 1) / best.rest_tiles())) * RING_TEAM_WORD * sizeof(unsigned long long);
     }
   }
   return best;
@@ -684,6 +772,7 @@ hipError_t ring_chip_fwd(const RingFwdArgs& a, const float* Wo, const float* Wa,
   c.slots = p.slots;
   c.act = a.act;
   ring_team_limits(&c.spin_max, &c.gather_ticks);
+  if (!getenv("RINGATTR_TEAM_GATHER_US")) c.gather_ticks = CHIP_GATHER_US * 100;
   e = ring_team_fill(ws, p.xchg_bytes, p.gather_bytes, st);
   if (e != hipSuccess) return e;
   e = hipErrorInvalidValue;
@@ -692,9 +781,14 @@ hipError_t ring_chip_fwd(const RingFwdArgs& a, const float* Wo, const float* Wa,
   RING_CHIP_SHAPES(RING_CHIP_CASE)
 #undef RING_CHIP_CASE
   if (e != hipSuccess) return e;
-  const size_t solo = (size_t)p.KC * (1024 + 256) + (size_t)(a.k + 1) * 64;
-  e = hipFuncSetAttribute(reinterpret_cast<const void*>(&ring_chip_solo_kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)solo);
-  if (e != hipSuccess) return e;
-  hipLaunchKernelGGL(ring_chip_solo_kernel, dim3(a.nbt), dim3(512), solo, st, c);
+  const int units = p.nrg * ((p.nt + p.rest_tiles() - 1) / p.rest_tiles()) * ((a.N + 15) / 16);
+  const dim3 grid((unsigned)std::min(units, 256)), block(64 * W);
+  switch (p.row.kpw) {
+    case 3: hipLaunchKernelGGL((ring_chip_rest_kernel<3, 4>), grid, block, 0, st, c); break;
+    case 4: hipLaunchKernelGGL((ring_chip_rest_kernel<4, 4>), grid, block, 0, st, c); break;
+    case 6: hipLaunchKernelGGL((ring_chip_rest_kernel<6, 2>), grid, block, 0, st, c); break;
+    case 8: hipLaunchKernelGGL((ring_chip_rest_kernel<8, 2>), grid, block, 0, st, c); break;
+    default: return hipErrorInvalidValue;
+  }
   return hipGetLastError();
 }

@@ -125,3 +125,84 @@ def test_rule(gpu_device):
                              (256, 12, 16, 2048, False), (1, 12, 6, 512, False)):
         _, name = _forward(_tensors(make_problem(15, B, T, k, N, bump="vm", action="dense"), gpu_device), "relu", 0.0, 0.5)
         assert ("chip" in name) == chip, (B, T, k, N, name)
+
+
+def test_row_groups_that_do_not_gather_cost_little(gpu_device, monkeypatch):
+    """Compute units held by another stream, graph or process: the tiles are done on those there are, in a small multiple of the panel
+    kernels' time (a workgroup per tile took nearly a thousand times as long)."""
+    B, T, k, N = 1, 12, 12, 2048
+    t = _tensors(make_problem(16, B, T, k, N, bump="vm", action="dense"), gpu_device)
+
+    def ms(want, **switches):
+        for name, value in switches.items():
+            monkeypatch.setenv(name, value)
+        times = []
+        for _ in range(3):
+            start, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            start.record()
+            h, kernel = _forward(t, "gelu", -1.0 / N, 0.5)
+            end.record()
+            torch.cuda.synchronize()
+            times.append(start.elapsed_time(end))
+            assert want in kernel
+        for name in switches:
+            monkeypatch.delenv(name)
+        return min(times), h
+
+    _, whole = ms("chip")
+    rest, h = ms("chip", RINGATTR_TEAM_GATHER_US="-1")
+    panel, _ = ms("panel", RINGATTR_CHIP="0")
+    print(f"[case] chip, no group gathered: {rest:.2f} ms, panels {panel:.2f} ms", flush=True)
+    assert torch.equal(h, whole) and rest < 20 * panel
+
+
+# all row groups, and those that are not complete at once; one and several row groups, tile blocks that are not full
+@pytest.mark.parametrize("B,T,k,N", [(1, 12, 6, 1024), (100, 10, 16, 700), (378, 10, 3, 1021), (130, 11, 2, 1537), (250, 10, 5, 640)])
+def test_groups_that_are_not_complete_in_time(B, T, k, N, gpu_device, monkeypatch):
+    print(f"[case] chip groups give up B={B} T={T} k={k} N={N}", flush=True)
+    monkeypatch.setenv("RINGATTR_CHIP", "1")
+    monkeypatch.setenv("RINGATTR_TEAM_GATHER_US", "1000000")
+    t = _tensors(make_problem(17, B, T, k, N, bump="vm", action="dense"), gpu_device)
+    want, name = _forward(t, "silu", -1.0 / N, 0.8)
+    assert "chip" in name
+    for wait_us in ("-1", "0", "2", "10"):
+        monkeypatch.setenv("RINGATTR_TEAM_GATHER_US", wait_us)
+        for _ in range(2):
+            h, _ = _forward(t, "silu", -1.0 / N, 0.8)
+            assert torch.equal(h, want), wait_us
+
+
+@pytest.mark.parametrize("B,T,k,N", [(40, 12, 6, 1024), (20, 10, 2, 2000)])
+def test_two_streams_and_two_graphs(B, T, k, N, gpu_device, monkeypatch):
+    """Launches that each want every compute unit: eager ones are ordered by the library, replayed graphs are not."""
+    monkeypatch.setenv("RINGATTR_CHIP", "1")
+    t = _tensors(make_problem(18, B, T, k, N, bump="vm", action="dense"), gpu_device)
+    want, name = _forward(t, "tanh", -1.0 / N, 0.9)
+    assert "chip" in name
+    print("[case] chip on two streams", flush=True)
+    streams = [torch.cuda.Stream() for _ in range(2)]
+    torch.cuda.synchronize()
+    got = []
+    for _ in range(3):
+        for s in streams:
+            with torch.cuda.stream(s):
+                got.append(_forward(t, "tanh", -1.0 / N, 0.9)[0])
+    torch.cuda.synchronize()
+    assert all(torch.equal(h, want) for h in got)
+    graphs, outs = [], []
+    for s in streams:
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=s):
+            outs.append(_forward(t, "tanh", -1.0 / N, 0.9)[0])
+        graphs.append(graph)
+    for _ in range(4):
+        for o in outs:
+            o.fill_(float("nan"))
+        torch.cuda.synchronize()
+        print("[case] chip graphs on two streams", flush=True)
+        for s, graph in zip(streams, graphs):
+            with torch.cuda.stream(s):
+                graph.replay()
+        torch.cuda.synchronize()
+        assert all(torch.equal(o, want) for o in outs)
+    _forward(t, "tanh", -1.0 / N, 0.9)          # (a wait that had run out would be reported by this call)
