@@ -650,6 +650,10 @@ struct ChipPlan {
 // 342 / 1429 / 575.  (A workgroup per tile on its own took 1.37 s, 69 ms and 38 ms, and the gathering 50 ms before that.)
 constexpr int CHIP_GATHER_US = 5000;
 
+// The kernel goes from a tile's gates to those of the group's next one in 32 bits.
+constexpr bool chip_gates_in_reach(int nrg, int T, int k) { return (size_t)nrg * 16 * T * k * 4 <= 0xFFFFFFFFu; }
+static_assert(chip_gates_in_reach(8, (1 << 23) - 1, 1) && !chip_gates_in_reach(8, 1 << 23, 1) && !chip_gates_in_reach(8, 1 << 20, 8), "");
+
 ChipPlan chip_plan(int N, int k, int T, int B) {
   ChipPlan best{};
   if (N <= 512 || N > 2048 || k < 1 || k > 16 || B < 1 || T < 1 || (size_t)16 * T * k * 4 >= ((size_t)1 << 30)) return best;
@@ -666,6 +670,7 @@ ChipPlan chip_plan(int N, int k, int T, int B) {
     int nrg = 8;
     while (nrg > 1 && (G > 32 * (8 / nrg) || nrg > nbt)) nrg /= 2;
     if (G > 32 * (8 / nrg)) continue;
+    if (!chip_gates_in_reach(nrg, T, k)) continue;
     const int nt = (nbt + nrg - 1) / nrg, slots = nt == 1 ? 8 : (nt < 4 ? 6 : 4);
     const size_t xbytes = (size_t)slots * nbt * KC * CHUNK_BYTES;
     if (xbytes >= ((size_t)1 << 30)) continue;           // (offsets past the buffer say 'nowhere')
