@@ -708,22 +708,24 @@ ChipPlan chip_plan(int N, int k, int T, int B) {
 // with the panels where two driven channels would be clearly faster there.
 // Short sequences stay with the panels, whose bits are those of the kernels that write a record: fewer than ten steps gain
 // little (loading the weights takes as long as four of them).
-bool ring_uses_chip(int N, int k, int T, int B) {
+static bool chip_rule(const ChipPlan& p, int N, int k, int T, int B) {
   const char* v = getenv("RINGATTR_CHIP");
-  if (v && v[0] == '0') return false;
-  for (const char* name : {"RINGATTR_PANEL", "RINGATTR_PANEL_SHAPE", "RINGATTR_WIDE", "RINGATTR_BLOCK", "RINGATTR_BLOCK_SHAPE"})
-    if (getenv(name)) return false;
-  if (!ring_teams_allowed()) return false;
-  const ChipPlan p = chip_plan(N, k, T, B);
-  if (!p.ok || v) return p.ok;
+  if (!p.ok || (v && v[0] == '0') || ring_team_fwd_bytes(N, k, T, B)) return false;       // (teams come first)
+  if (v) return true;
   const int NC = (N + 511) / 512 * 8;
   auto panel = [&](int channels) { return ring_panel_step_cycles(NC < 16 ? 16 : NC, (B + 15) / 16, channels); };
   return T >= 10 && p.cycles < 0.95f * panel(k) && p.cycles < 1.1f * panel(k < 2 ? k : 2);
 }
 
+bool ring_uses_chip(int N, int k, int T, int B) {
+  for (const char* name : {"RINGATTR_PANEL", "RINGATTR_PANEL_SHAPE", "RINGATTR_WIDE", "RINGATTR_BLOCK", "RINGATTR_BLOCK_SHAPE"})
+    if (getenv(name)) return false;
+  return ring_teams_allowed() && chip_rule(chip_plan(N, k, T, B), N, k, T, B);
+}
+
 size_t ring_chip_bytes(int N, int k, int T, int B) {
   const ChipPlan p = chip_plan(N, k, T, B);
-  return p.ok ? p.xchg_bytes + p.gather_bytes : 0;
+  return chip_rule(p, N, k, T, B) ? p.xchg_bytes + p.gather_bytes : 0;
 }
 
 template <int NPW, int KPW, int CT, int DEPTH>

@@ -131,7 +131,7 @@ hipError_t ring_launch_panel_fwd(const RingFwdArgs& a, int NC, hipStream_t st);
 
 // Forward without a saved record on all compute units at once, the weights on chip, wide rings (ring_chip.hip).
 bool ring_uses_chip(int N, int k, int T, int B);
-size_t ring_chip_bytes(int N, int k, int T, int B);       // scratch of one launch (0 where no call of this shape comes here)
+size_t ring_chip_bytes(int N, int k, int T, int B);       // scratch of one launch (0 where the rule takes no call of this shape)
 hipError_t ring_chip_fwd(const RingFwdArgs& a, const float* Wo, const float* Wa, void* ws, hipStream_t st);
 hipError_t ring_run_chip_fwd(const RingFwdArgs& a, const float* Wo, const float* Wa, void* ws, hipStream_t st);
 

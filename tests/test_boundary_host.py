@@ -66,6 +66,18 @@ def test_backward_workspace_holds_no_team_scratch_that_is_not_used():
         assert lib.ringattr_bwd_workspace_bytes(N, k, T, B, saved) == max(without, with_a)
 
 
+def test_forward_workspace_holds_no_chip_scratch_that_is_not_used(monkeypatch):
+    """The chip kernels' exchange area is asked for only where their rule sends a call of this shape: not where the panel kernels are
+    faster, not for fewer than ten steps, not with the switch off (bytes: packed weights and the panel kernels' area)."""
+    monkeypatch.delenv("RINGATTR_CHIP", raising=False)
+    lib = _lib.load()
+    for (N, k, B, T), size in {(1012, 2, 7746, 60): 54062080, (1013, 1, 7660, 5): 51374080, (981, 3, 6187, 9): 46506752}.items():
+        assert lib.ringattr_fwd_workspace_bytes(N, k, T, B) == size, (N, k, B, T)
+    assert lib.ringattr_fwd_workspace_bytes(981, 3, 60, 6187) == 61453568            # here they run
+    monkeypatch.setenv("RINGATTR_CHIP", "0")
+    assert lib.ringattr_fwd_workspace_bytes(981, 3, 60, 6187) == 46506752
+
+
 def test_c_abi_rejects_bad_arguments_with_codes_not_exit():
     lib = _lib.load()
     buf = (ctypes.c_char * 4096)()
