@@ -83,17 +83,87 @@ def test_infinite_states_and_absent_matrices(gpu_device, monkeypatch):
     assert torch.isinf(h[:, 2]).all() and torch.isfinite(h[:, [0, 1, 3, 4]]).all()
 
 
-def test_slots_come_round_many_times(gpu_device, monkeypatch):
-    """Hundreds of rounds through the exchange slots with one, two and many tiles per group: the same bits as without any."""
-    for B, k, N, width in ((16, 3, 1100, "8"), (32, 3, 1100, "16"), (64, 3, 1100, "16"), (100, 16, 1024, "8"), (256, 2, 2048, "32")):
-        print(f"[case] chip rounds B={B} k={k} N={N} width {width}", flush=True)
-        t = _tensors(make_problem(13, B, 150, k, N, bump="vm", action="dense"), gpu_device)
-        monkeypatch.setenv("RINGATTR_CHIP", width)
-        h, name = _forward(t, "tanh", -1.0 / N, 0.9)
-        assert "chip" in name
-        monkeypatch.setenv("RINGATTR_CHIP", "8")         # the same rows a few at a time: other numbers of tiles and slots
+# one, two, three and more tiles per row group (8, 6, 6 and 4 slots), operands one to three items ahead, one to eight row groups, the
+# last of them a tile short
+@pytest.mark.parametrize("B,k,N,width", [
+    (16, 3, 1100, "8"), (32, 3, 1100, "16"), (64, 3, 1100, "16"), (41, 8, 1100, "8"), (41, 16, 1100, "8"), (73, 7, 600, "8"), (100, 16, 1024, "8"),
+    (300, 3, 1021, "32"), (400, 4, 900, "16"), (150, 2, 2048, "32"), (256, 2, 2048, "32")])
+def test_slots_come_round_many_times(B, k, N, width, gpu_device, monkeypatch):
+    """150 steps, 19 to 37 rounds through the exchange slots: every row has the bits that the way without slots gives it."""
+    print(f"[case] chip rounds B={B} k={k} N={N} width {width}", flush=True)
+    t = _tensors(make_problem(13, B, 150, k, N, bump="vm", action="dense"), gpu_device)
+    monkeypatch.setenv("RINGATTR_CHIP", width)
+    h, name = _forward(t, "tanh", -1.0 / N, 0.9)
+    assert "chip" in name
+    monkeypatch.setenv("RINGATTR_TEAM_GATHER_US", "-1")
+    without, _ = _forward(t, "tanh", -1.0 / N, 0.9)
+    assert torch.equal(without, h)
+    monkeypatch.delenv("RINGATTR_TEAM_GATHER_US")
+    if N > 1024 or k > 3:                                # the same rows a few at a time: other numbers of tiles and slots
+        monkeypatch.setenv("RINGATTR_CHIP", "8")         # (nine rows of N <= 1024 and three channels are the teams')
         part, name = _forward([t[0][:9].clone(), t[1], t[2], t[3][:9].clone()], "tanh", -1.0 / N, 0.9)
         assert "chip" in name and torch.equal(part, h[:, :9])
+
+
+# Every kernel that is built, but for those of FEW_CHANNELS: neurons per workgroup, K chunks and column tiles of a wave, the fewest and the
+# most channels that take that many column tiles, and how many items ahead an operand can be asked for at most (with that many tiles
+# per row group or more).
+KERNELS = [
+    (8, 3, 4, 5, 7, 3), (8, 3, 7, 8, 13, 3), (8, 3, 9, 14, 16, 3), (8, 4, 4, 4, 7, 3), (8, 4, 7, 8, 13, 3), (8, 4, 9, 14, 16, 3),
+    (8, 6, 2, 1, 3, 3), (8, 6, 4, 4, 7, 3), (8, 6, 7, 8, 13, 2), (8, 6, 9, 14, 16, 1), (8, 8, 2, 1, 3, 3), (8, 8, 4, 4, 7, 2), (8, 8, 7, 8, 13, 1),
+    (16, 3, 7, 5, 6, 3), (16, 4, 7, 4, 6, 3), (16, 6, 3, 1, 2, 3), (16, 6, 4, 3, 3, 3), (16, 6, 7, 4, 6, 2), (16, 8, 3, 1, 2, 2), (16, 8, 4, 3, 3, 2),
+    (16, 8, 7, 4, 6, 1), (32, 6, 6, 1, 2, 2), (32, 6, 8, 3, 3, 2), (32, 8, 6, 1, 2, 1),
+]
+# Up to three channels at N <= 1024 come here with many rows only (the teams take the others): workgroup, chunks, tiles, N, channels, rows
+FEW_CHANNELS = [
+    (8, 3, 2, 765, 3, 2317), (8, 4, 2, 1001, 3, 265), (8, 4, 2, 1024, 3, 400), (16, 3, 4, 517, 3, 2957), (16, 4, 3, 779, 1, 3117), (16, 4, 4, 1021, 3, 265),
+    (32, 3, 6, 513, 1, 4557), (32, 3, 6, 768, 2, 4557), (32, 3, 8, 516, 3, 2957), (32, 4, 6, 778, 1, 3117), (32, 4, 8, 1021, 3, 378), (32, 4, 8, 1024, 3, 265)]
+WIDTHS = {3: (517, 764), 4: (771, 1024), 6: (1031, 1536), 8: (1541, 2048)}           # N by K chunks of a wave: odd, a multiple of four
+
+
+@pytest.mark.parametrize("npw,kpw,ct,fewest,most,depth", KERNELS)
+def test_every_kernel(npw, kpw, ct, fewest, most, depth, gpu_device, monkeypatch):
+    """One to four tiles per row group, the last group's one short: the oracle for rows of the first, a middle and the last tile, every
+    row the bits of the way without slots and of every other batch."""
+    T = 12
+    for N, k in zip(WIDTHS[kpw], (fewest, most)):
+        groups = 8
+        while 32 * ((N + 31) // 32) // npw > 256 // groups:
+            groups //= 2
+        batches = [16 * groups - 7] + [16 * (groups * (nt - 1) + max(1, groups - 1)) - 7 for nt in (2, 3, 4)]
+        batches = batches[:2] if (npw, kpw, ct) == (16, 8, 7) else batches           # (LDS holds two tiles' states beside its weights)
+        print(f"[case] chip <{npw}, {kpw}, {ct}> N={N} k={k} B={batches}", flush=True)
+        J0, J1, B = -1.0 / N, 0.6, batches[-1]
+        p = make_problem(19 + ct, B, T, k, N, bump="vm", action="dense")
+        t = _tensors(p, gpu_device)
+        monkeypatch.setenv("RINGATTR_CHIP", str(npw))
+        monkeypatch.setenv("RINGATTR_TEAM_GATHER_US", "-1")
+        want, _ = _forward(t, "gelu", J0, J1)
+        monkeypatch.delenv("RINGATTR_TEAM_GATHER_US")
+        for nt, rows in enumerate(batches, 1):
+            h, name = _forward([t[0][:rows].clone(), t[1], t[2], t[3][:rows].clone()], "gelu", J0, J1)
+            assert f"<{npw},{kpw},{ct},{min(nt, depth)}>" in name, (N, k, rows, name)
+            assert torch.equal(h, want[:, :rows]), (N, k, rows)
+        some = [0, 15, B // 2, B - 1]
+        ref, _ = O.forward_dense(p["A"][some], p["Wa"], J0, J1, p["Wo"], p["r0"][some], 0.15, "gelu")
+        assert O.max_rel_err(want[:, some].cpu().numpy(), ref) <= 1e-2               # one bf16 rounding per operand, as everywhere
+
+
+@pytest.mark.parametrize("npw,kpw,ct,N,k,B", FEW_CHANNELS)
+def test_every_kernel_of_few_channels(npw, kpw, ct, N, k, B, gpu_device, monkeypatch):
+    print(f"[case] chip <{npw}, {kpw}, {ct}> N={N} k={k} B={B}", flush=True)
+    J0, J1 = -1.0 / N, 0.6
+    p = make_problem(23, B, 12, k, N, bump="vm", action="dense")
+    t = _tensors(p, gpu_device)
+    monkeypatch.setenv("RINGATTR_CHIP", str(npw))
+    h, name = _forward(t, "silu", J0, J1)
+    assert f"<{npw},{kpw},{ct},3>" in name, name
+    monkeypatch.setenv("RINGATTR_TEAM_GATHER_US", "-1")
+    without, _ = _forward(t, "silu", J0, J1)
+    assert torch.equal(h, without)
+    some = [0, 15, B // 2, B - 1]
+    ref, _ = O.forward_dense(p["A"][some], p["Wa"], J0, J1, p["Wo"], p["r0"][some], 0.15, "silu")
+    assert O.max_rel_err(h[:, some].cpu().numpy(), ref) <= 1e-2                      # one bf16 rounding per operand, as everywhere
 
 
 def test_replayed_graph(gpu_device):
@@ -119,12 +189,15 @@ def test_replayed_graph(gpu_device):
         want, _ = _forward(t, "gelu", -1.0 / N, 0.9)
 
 
-def test_rule(gpu_device):
-    """Few steps, narrow rings and batches that fill the chip stay where they were."""
-    for B, T, k, N, chip in ((1, 12, 6, 1024, True), (1, 9, 6, 1024, False), (1, 12, 2, 1024, False), (64, 12, 2, 1100, True), (1, 12, 17, 1100, False),
-                             (256, 12, 16, 2048, False), (1, 12, 6, 512, False)):
-        _, name = _forward(_tensors(make_problem(15, B, T, k, N, bump="vm", action="dense"), gpu_device), "relu", 0.0, 0.5)
-        assert ("chip" in name) == chip, (B, T, k, N, name)
+# Where the default takes a call: few steps, two channels that the teams take, narrow rings, more channels than are built, more weights than fit
+# (17 matrices past N = 1536), batches that take longer than on the panels, and those that would if only two channels were driven
+@pytest.mark.parametrize("B,T,k,N,chip", [
+    (1, 12, 6, 1024, True), (64, 12, 2, 1100, True), (256, 12, 6, 1024, True), (1, 12, 13, 2048, True),
+    (1, 9, 6, 1024, False), (1, 12, 2, 1024, False), (1, 12, 6, 512, False), (1, 12, 17, 1100, False), (256, 12, 16, 2048, False), (1, 12, 14, 2048, False),
+    (1024, 10, 2, 2048, False), (1024, 10, 16, 1024, False), (64, 12, 16, 1500, False), (256, 12, 16, 1024, False), (1024, 10, 6, 640, False)])
+def test_rule(B, T, k, N, chip, gpu_device):
+    _, name = _forward(_tensors(make_problem(15, B, T, k, N, bump="vm", action="dense"), gpu_device), "relu", 0.0, 0.5)
+    assert ("chip" in name) == chip, name
 
 
 def test_row_groups_that_do_not_gather_cost_little(gpu_device, monkeypatch):
