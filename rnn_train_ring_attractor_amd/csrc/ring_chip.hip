@@ -74,6 +74,9 @@ struct ChipShape {
   static constexpr int FULL = NPW == 8 ? (CT == 2 ? 1 : CT == 4 ? 2 : CT == 7 ? 4 : 7) : NPW == 16 ? (CT == 3 ? 2 : CT == 4 ? 4 : 5) : (CT == 6 ? 4 : 8);
   static constexpr int SHARE = NPW / 4 * CHIP_QS;               // floats of one wave's share
   static constexpr int MATS = NPW == 8 ? 2 * CT : (NPW == 16 ? CT : CT / 2);      // matrices that there is room for
+  static constexpr int LEAST = NPW == 8 ? 2 * FULL : (NPW == 16 ? FULL : FULL / 2);      // and that fill the tiles without a gap
+  // Up to three channels at N <= 1024 the teams take every call with fewer than three tiles per row group of any width.
+  static constexpr bool BUILT = DEPTH == 1 ? KPW > 4 || MATS > 4 : DEPTH == 2 ? P * W <= 144 && (KPW > 4 || MATS > 4) : P == 0;
   static constexpr int before(int f) { return f * P / F; }                        // parked ones among the first f
   static constexpr bool is_parked(int f) { return before(f + 1) > before(f); }
 };
@@ -621,17 +624,20 @@ __global__ __launch_bounds__(64 * W) void ring_chip_rest_kernel(RingChipArgs c) 
 // ------------------------------------------------------------------------------------------------
 // Shapes that are built: neurons per member, K chunks of a wave, column tiles.
 #define RING_CHIP_COLUMNS(X, KPW) \
-  X(8, KPW, 2) X(8, KPW, 4) X(8, KPW, 7) X(16, KPW, 3) X(16, KPW, 4) X(16, KPW, 7) X(32, KPW, 6)
+  X(8, KPW, 2) X(8, KPW, 4) X(8, KPW, 7) X(16, KPW, 4) X(16, KPW, 7) X(32, KPW, 6)
+// (16, 3, 3: the teams take every call of one or two channels that it has LDS for)
 #define RING_CHIP_SHAPES(X)                                                                                          \
-  RING_CHIP_COLUMNS(X, 3) X(8, 3, 9) X(32, 3, 8) RING_CHIP_COLUMNS(X, 4) X(8, 4, 9) X(32, 4, 8)                      \
-  RING_CHIP_COLUMNS(X, 6) X(8, 6, 9) X(32, 6, 8) RING_CHIP_COLUMNS(X, 8)
+  RING_CHIP_COLUMNS(X, 3) X(8, 3, 9) X(32, 3, 8) RING_CHIP_COLUMNS(X, 4) X(8, 4, 9) X(16, 4, 3) X(32, 4, 8)          \
+  RING_CHIP_COLUMNS(X, 6) X(8, 6, 9) X(16, 6, 3) X(32, 6, 8) RING_CHIP_COLUMNS(X, 8) X(16, 8, 3)
 
 namespace {
 
-struct ChipRow { int npw, kpw, ct, mats, parked[3]; };      // parked: by depth - 1
+struct ChipRow { int npw, kpw, ct, least, mats, parked[3]; bool built[3]; };      // parked, built: by depth - 1
 const ChipRow kChipRows[] = {
-#define RING_CHIP_ROW(NPW, KPW, CT) \
-  {NPW, KPW, CT, ChipShape<NPW, KPW, CT, 1>::MATS, {ChipShape<NPW, KPW, CT, 1>::P, ChipShape<NPW, KPW, CT, 2>::P, ChipShape<NPW, KPW, CT, 3>::P}},
+#define RING_CHIP_ROW(NPW, KPW, CT)                                                                                                        \
+  {NPW, KPW, CT, ChipShape<NPW, KPW, CT, 1>::LEAST, ChipShape<NPW, KPW, CT, 1>::MATS,                                                      \
+   {ChipShape<NPW, KPW, CT, 1>::P, ChipShape<NPW, KPW, CT, 2>::P, ChipShape<NPW, KPW, CT, 3>::P},                                          \
+   {ChipShape<NPW, KPW, CT, 1>::BUILT, ChipShape<NPW, KPW, CT, 2>::BUILT, ChipShape<NPW, KPW, CT, 3>::BUILT}},
     RING_CHIP_SHAPES(RING_CHIP_ROW)
 #undef RING_CHIP_ROW
 };
@@ -664,7 +670,7 @@ ChipPlan chip_plan(int N, int k, int T, int B) {
   const char* force = getenv("RINGATTR_CHIP");           // 8, 16 or 32: neurons per member (cross-checks)
   const int npw = force ? atoi(force) : 0;
   for (const ChipRow& r : kChipRows) {
-    if (r.kpw != kpw || r.mats < k + 1) continue;
+    if (r.kpw != kpw || r.least > k + 1 || r.mats < k + 1) continue;
     if (npw > 1 && r.npw != npw) continue;
     const int G = 32 * KC / r.npw;                       // (whole K chunks: the padding is published too)
     int nrg = 8;
@@ -677,7 +683,7 @@ ChipPlan chip_plan(int N, int k, int T, int B) {
     // the deepest prefetch that the tiles can use and LDS has room for
     int depth = nt >= 3 ? 3 : (nt == 2 ? 2 : 1);
     while (depth > 1 && (depth == 3 ? r.parked[2] > 0 : chip_lds(r.npw, r.mats, r.parked[1], nt).total > CHIP_LDS)) --depth;
-    if (chip_lds(r.npw, r.mats, r.parked[depth - 1], nt).total > CHIP_LDS) continue;
+    if (!r.built[depth - 1] || chip_lds(r.npw, r.mats, r.parked[depth - 1], nt).total > CHIP_LDS) continue;
     // Cycles of a step at 2.4 GHz, fitted to 180 measured shapes (N = 640 to 2048, 2 to 16 channels, B = 1 to 1024).  Many tiles per
     // group: what an item takes.  One: products, hand-over (the more members, the slower) and epilogue one after the other;
     // a few: the items of a tile wait for its hand-over.
@@ -743,11 +749,13 @@ static hipError_t chip_start(const RingChipArgs& c, const ChipPlan& p, hipStream
 
 template <int NPW, int KPW, int CT>
 static hipError_t chip_shape(const RingChipArgs& c, const ChipPlan& p, hipStream_t st) {
-  if constexpr (ChipShape<NPW, KPW, CT, 3>::P == 0)
+  if constexpr (ChipShape<NPW, KPW, CT, 3>::BUILT)
     if (p.depth == 3) return chip_start<NPW, KPW, CT, 3>(c, p, st);
-  if constexpr (ChipShape<NPW, KPW, CT, 2>::P * W <= 144)
+  if constexpr (ChipShape<NPW, KPW, CT, 2>::BUILT)
     if (p.depth == 2) return chip_start<NPW, KPW, CT, 2>(c, p, st);
-  return p.depth == 1 ? chip_start<NPW, KPW, CT, 1>(c, p, st) : hipErrorInvalidValue;
+  if constexpr (ChipShape<NPW, KPW, CT, 1>::BUILT)
+    if (p.depth == 1) return chip_start<NPW, KPW, CT, 1>(c, p, st);
+  return hipErrorInvalidValue;
 }
 
 hipError_t ring_chip_fwd(const RingFwdArgs& a, const float* Wo, const float* Wa, void* ws, hipStream_t st) {
