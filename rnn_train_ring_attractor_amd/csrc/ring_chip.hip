@@ -2,10 +2,11 @@
 // of ALL compute units for the whole sequence, the state handed over between the XCDs once per step.
 //
 // What bounds the step-per-launch kernels here (ring_panel.hip) is that every step pulls all (1 + a_dim) N^2 weights from
-// beyond L2 again and waits for a launch: at N = 2048 with 16 channels 143 MB a step.  The chip holds 128 MB of registers and
-// 40 MB of LDS, so all of it fits on chip.  A member (a workgroup) keeps all matrices of NPW = 8, 16 or 32 neurons; G = N / NPW
-// members make a row group, which takes every nrg-th batch tile of 16 rows through the sequence.  Fewer neurons per member spread
-// the weights over more compute units, more let several row groups work side by side, each reading the state of its own rows only.
+// beyond L2 again and waits for a launch: at N = 2048 with 12 channels 109 MB a step.  The chip holds 128 MB of registers and
+// 40 MB of LDS.  Beside what a step works with there is room for 16 channels up to N = 1536 and for 13 up to N = 2048 (117 MB).  A
+// member (a workgroup) keeps all matrices of NPW = 8, 16 or 32 neurons; G = N / NPW members make a row group, which takes every
+// nrg-th batch tile of 16 rows through the sequence.  Fewer neurons per member spread the weights over more compute units, more let
+// several row groups work side by side, each reading the state of its own rows only.
 //
 //   * Eight waves split the contraction as in ring_team.hpp (wave w owns K chunks w, w + 8, ...); a wave loads just its chunks of the
 //     state, multiplies them with its resident fragments (weights are the A operand: a lane ends up with four neurons of one batch
@@ -702,16 +703,17 @@ ChipPlan chip_plan(int N, int k, int T, int B) {
 
 }  // namespace
 
-// Where it runs: wherever the model above expects it to be faster than the step-per-launch kernels.  us per step (T = 60, panel
-// kernels / here):
-//   N = 640,   6 channels: B = 1: 7.4 / 3.1    B = 64: 8.1 / 4.4    B = 1024: 28 / 20
-//   N = 1024, 16 channels: B = 1: 12.5 / 3.8   B = 32: 12.7 / 5.5   B = 256: 19 / 14     B = 1024: 49 / 50
+// Where it runs: where the model above expects it to be faster than the step-per-launch kernels, with all channels driven and, within a
+// tenth, with two of them.  us per step (T = 60, all channels driven, panel kernels / here; *: stays with the panels as slower,
+// +: because of what two driven channels would cost):
+//   N = 640,   6 channels: B = 1: 7.4 / 3.1    B = 64: 8.1 / 4.4    B = 1024: 28 / 20 +
+//   N = 1024, 16 channels: B = 1: 12.5 / 3.8   B = 32: 12.7 / 5.5   B = 256: 19 / 14 +   B = 1024: 49 / 50 *
 //   N = 1100,  2 channels: B = 1: 7.2 / 3.2    B = 64: 9.1 / 5.0    B = 1024: 33 / 28
-//   N = 1500, 16 channels: B = 1: 18 / 4.7     B = 64: 20 / 11.5    B = 256: 33 / 42
-//   N = 2048,  2 channels: B = 1: 8.0 / 3.9    B = 64: 10.2 / 6.4   B = 1024: 38 / 44;   12 channels, B = 1: 24 / 5.2
+//   N = 1500, 16 channels: B = 1: 18 / 4.7     B = 64: 20 / 11.5 +  B = 256: 33 / 42 *
+//   N = 2048,  2 channels: B = 1: 8.0 / 3.9    B = 64: 10.2 / 6.4   B = 1024: 38 / 44 *;   12 channels, B = 1: 24 / 5.2
 // Channels that are silent in all rows of a workgroup (zero-padded action signals) cost the panels nothing; here passing them by
-// costs the others more than it saves (N = 1024, B = 1024: 16 channels 49.6 -> 53.6, two of 16 driven 44, panels 22): a call stays
-// with the panels where two driven channels would be clearly faster there.
+// costs the others more than it saves (N = 1024, B = 1024: 16 channels 49.6 -> 53.6, two of 16 driven 44, panels 22).  What channels
+// carry is not known when the kernels are chosen, so the rule protects padded calls, at the price of dense ones as marked.
 // Short sequences stay with the panels, whose bits are those of the kernels that write a record: fewer than ten steps gain
 // little (loading the weights takes as long as four of them).
 static bool chip_rule(const ChipPlan& p, int N, int k, int T, int B) {

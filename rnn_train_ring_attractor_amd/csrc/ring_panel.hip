@@ -221,7 +221,7 @@ __device__ __forceinline__ void panel_put(bf16x8* x, int KCH, int b, int j, cons
 }  // namespace
 
 // Operand fragments [batch tile][K chunk][lane][8] and fp32 row sums of the initial state's rows; four rows per wave.  The
-// sums run in the order of ring_block.hip's stage_tiles.  (Both fragment buffers, if there are two: the steps write no
+// sums run in the order of stage_rows (ring_step_common.hpp).  (Both fragment buffers, if there are two: the steps write no
 // padding.)
 __global__ __launch_bounds__(64) void ring_panel_operand_kernel(const float* __restrict__ prev, PanelState ps, int N, int B, int NPAD) {
   const int lane = threadIdx.x, row = 4 * (blockIdx.x & 3) + (lane >> 4), sub = lane & 15, bt = blockIdx.x >> 2;
