@@ -18,9 +18,10 @@
 //     item in turn, whose stores held up its next operand (one in-order counter): N = 1100, 2 channels, B = 1 3.9 against 3.2 us
 //     per step, N = 700, 6 channels, B = 1 3.4 against 3.0.  All waves issue the same operations, so the compiler waits for
 //     an operand's loads and not for the stores behind them.
-// What bounds an item (step, tile of 16 rows) with many tiles per group is instructions: some 3.3 to 4.4 thousand cycles, of which
-// products 0.4 to 1.3 and taking in the state (35 bytes per cycle and compute unit, 256 of them reading the same) 0.8 to 2; with
-// one tile the hand-over between the XCDs, 1.9 us of 3 to 6.
+// What bounds an item (step, tile of 16 rows) with several tiles per group is instructions.  Cycles of a wave's item at N = 1024, 6
+// channels, B = 256 (N = 640 to 1100, B = 512 and 1024: 2900 to 3800): 3250, of them products with the gates 1500, epilogue 890, barrier 550,
+// waiting for the state 300; a compute unit takes in 13 bytes a cycle.  With one tile it is the hand-over: 6600 to 8400 of 9200 to
+// 11300 cycles (N = 640 to 2048) are the epilogue, which publishes and then waits to poll, and the wait for the state.
 //
 // Exchange: the protocol of ring_team.hpp (the data is its own flag, slots refilled with a pattern no state can be), but with
 // stores that go through to where all XCDs see them.  Measured for 256 members and one tile: 1.9 us from step to step, 2.6 with
