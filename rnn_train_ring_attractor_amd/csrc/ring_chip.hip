@@ -64,8 +64,8 @@ struct RingChipArgs {
 };
 
 // Fragments of a wave: F, of which FR in registers and the rest in LDS, spread evenly over a column tile's products.
-// DEPTH: operands on their way or in use.  1: the next item's is asked for behind this one's products (one tile per group: it cannot
-// be there earlier); 2 and 3: before them, one item or two ahead.
+// DEPTH: operands on their way or in use.  1: the next item's is asked for behind this one's epilogue (one tile per group or two: it
+// cannot be there earlier); 2 and 3: before its products, one item or two ahead (see chip_plan).
 template <int NPW, int KPW, int CT, int DEPTH>
 struct ChipShape {
   static constexpr int F = CT * KPW;
@@ -77,8 +77,10 @@ struct ChipShape {
   static constexpr int SHARE = NPW / 4 * CHIP_QS;               // floats of one wave's share
   static constexpr int MATS = NPW == 8 ? 2 * CT : (NPW == 16 ? CT : CT / 2);      // matrices that there is room for
   static constexpr int LEAST = NPW == 8 ? 2 * FULL : (NPW == 16 ? FULL : FULL / 2);      // and that fill the tiles without a gap
-  // Up to three channels at N <= 1024 the teams take every call with fewer than three tiles per row group of any width.
-  static constexpr bool BUILT = DEPTH == 1 ? KPW > 4 || MATS > 4 : DEPTH == 2 ? P * W <= 144 && (KPW > 4 || MATS > 4) : P == 0;
+  // Up to three channels at N <= 1024 the teams take every call with few tiles per row group: fewer than three with 32 neurons a member
+  // and three channels, fewer than five else.
+  static constexpr int TEAMS_UP_TO = KPW > 4 || MATS > 4 ? 0 : (NPW == 32 && KPW == 4 && CT == 8 ? 2 : 4);
+  static constexpr bool BUILT = DEPTH == 1 ? TEAMS_UP_TO < 2 : DEPTH == 2 ? P * W <= 144 && TEAMS_UP_TO < 4 : P == 0;
   static constexpr int before(int f) { return f * P / F; }                        // parked ones among the first f
   static constexpr bool is_parked(int f) { return before(f + 1) > before(f); }
 };
@@ -682,8 +684,13 @@ ChipPlan chip_plan(int N, int k, int T, int B) {
     const int nt = (nbt + nrg - 1) / nrg, slots = nt == 1 ? 8 : (nt < 4 ? 6 : 4);
     const size_t xbytes = (size_t)slots * nbt * KC * CHUNK_BYTES;
     if (xbytes >= ((size_t)1 << 30)) continue;           // (offsets past the buffer say 'nowhere')
-    // the deepest prefetch that the tiles can use and LDS has room for
-    int depth = nt >= 3 ? 3 : (nt == 2 ? 2 : 1);
+    // The deepest prefetch that registers and LDS have room for and the tiles can use: an operand is the state that the group made
+    // its tiles' number of items ago, and asked for as soon as the item behind that, it is not there.  What is asked again then
+    // holds up the stores it waits for (us a call of T = 40, three, two and one item ahead): one tile per group behind, N = 1021, 3
+    // channels, B = 377 539, 261, 279, N = 896, 16 channels, B = 89 404, 239, 266, N = 768, 6 channels, B = 121 two and one 225, 150;
+    // two behind, N = 896, B = 121 280, 294, 347.  A group that is a tile short decides for all from four tiles on: B = 107 368, 303.
+    const int fewest = nbt / nrg;
+    int depth = fewest >= 4 ? 3 : (nt >= 3 ? 2 : 1);
     while (depth > 1 && (depth == 3 ? r.parked[2] > 0 : chip_lds(r.npw, r.mats, r.parked[1], nt).total > CHIP_LDS)) --depth;
     if (!r.built[depth - 1] || chip_lds(r.npw, r.mats, r.parked[depth - 1], nt).total > CHIP_LDS) continue;
     // Cycles of a step at 2.4 GHz, fitted to 180 measured shapes (N = 640 to 2048, 2 to 16 channels, B = 1 to 1024).  Many tiles per
@@ -691,7 +698,7 @@ ChipPlan chip_plan(int N, int k, int T, int B) {
     // a few: the items of a tile wait for its hand-over.
     const int parked = r.parked[depth - 1];
     const float F = (float)(r.ct * r.kpw), kc = (float)KC;
-    const float item = 2000.f + 30.f * kc + 25.f * F + (depth == 1 ? 1100.f : 0.f) + 40.f * (float)parked;
+    const float item = 2000.f + 30.f * kc + 25.f * F + (depth == 1 && nt > 2 ? 1100.f : 0.f) + 40.f * (float)parked;
     const float one = 5000.f + 45.f * kc + 25.f * (float)G + 38.f * F - (B < 16 ? 1500.f : 0.f);
     const float cycles = nt == 1 ? one : std::max(1.6f * one, (float)nt * item);
     if (!best.ok || cycles < best.cycles) {
@@ -714,7 +721,9 @@ ChipPlan chip_plan(int N, int k, int T, int B) {
 //   N = 2048,  2 channels: B = 1: 8.0 / 3.9    B = 64: 10.2 / 6.4   B = 1024: 38 / 44 *;   12 channels, B = 1: 24 / 5.2
 // Channels that are silent in all rows of a workgroup (zero-padded action signals) cost the panels nothing; here passing them by
 // costs the others more than it saves (N = 1024, B = 1024: 16 channels 49.6 -> 53.6, two of 16 driven 44, panels 22).  What channels
-// carry is not known when the kernels are chosen, so the rule protects padded calls, at the price of dense ones as marked.
+// carry is not known when the kernels are chosen, so the rule protects padded calls, at the price of dense ones as marked.  Of 760
+// random calls that it takes (all channels driven or two; T = 60) 15 are slower than on the panels, by 18 % at most (N = 1848, 4
+// channels, two driven, B = 124); the mean is 1.74 times as fast.
 // Short sequences stay with the panels, whose bits are those of the kernels that write a record: fewer than ten steps gain
 // little (loading the weights takes as long as four of them).
 static bool chip_rule(const ChipPlan& p, int N, int k, int T, int B) {

@@ -87,7 +87,7 @@ def test_infinite_states_and_absent_matrices(gpu_device, monkeypatch):
 # last of them a tile short
 @pytest.mark.parametrize("B,k,N,width", [
     (16, 3, 1100, "8"), (32, 3, 1100, "16"), (64, 3, 1100, "16"), (41, 8, 1100, "8"), (41, 16, 1100, "8"), (73, 7, 600, "8"), (100, 16, 1024, "8"),
-    (300, 3, 1021, "32"), (400, 4, 900, "16"), (150, 2, 2048, "32"), (256, 2, 2048, "32")])
+    (120, 10, 900, "8"), (300, 3, 1021, "32"), (400, 4, 900, "16"), (150, 2, 2048, "32"), (256, 2, 2048, "32")])
 def test_slots_come_round_many_times(B, k, N, width, gpu_device, monkeypatch):
     """150 steps, 19 to 37 rounds through the exchange slots: every row has the bits that the way without slots gives it."""
     print(f"[case] chip rounds B={B} k={k} N={N} width {width}", flush=True)
@@ -106,31 +106,32 @@ def test_slots_come_round_many_times(B, k, N, width, gpu_device, monkeypatch):
 
 
 # Every kernel that is built, but for those of FEW_CHANNELS: neurons per workgroup, K chunks and column tiles of a wave, the fewest and the
-# most channels that take that many column tiles, and how many items ahead an operand can be asked for at most (with that many tiles
-# per row group or more).
+# most channels that take that many column tiles, and how many operands can be on their way at most.
 KERNELS = [
     (8, 3, 4, 5, 7, 3), (8, 3, 7, 8, 13, 3), (8, 3, 9, 14, 16, 3), (8, 4, 4, 4, 7, 3), (8, 4, 7, 8, 13, 3), (8, 4, 9, 14, 16, 3),
     (8, 6, 2, 1, 3, 3), (8, 6, 4, 4, 7, 3), (8, 6, 7, 8, 13, 2), (8, 6, 9, 14, 16, 1), (8, 8, 2, 1, 3, 3), (8, 8, 4, 4, 7, 2), (8, 8, 7, 8, 13, 1),
     (16, 3, 7, 5, 6, 3), (16, 4, 7, 4, 6, 3), (16, 6, 3, 1, 2, 3), (16, 6, 4, 3, 3, 3), (16, 6, 7, 4, 6, 2), (16, 8, 3, 1, 2, 2), (16, 8, 4, 3, 3, 2),
     (16, 8, 7, 4, 6, 1), (32, 6, 6, 1, 2, 2), (32, 6, 8, 3, 3, 2), (32, 8, 6, 1, 2, 1),
 ]
-# Up to three channels at N <= 1024 come here with many rows only (the teams take the others): workgroup, chunks, tiles, N, channels, rows
+# Up to three channels at N <= 1024 come here with many rows only (the teams take the others): workgroup, chunks, tiles, operands on
+# their way, N, channels, rows
 FEW_CHANNELS = [
-    (8, 3, 2, 765, 3, 2317), (8, 4, 2, 1001, 3, 265), (8, 4, 2, 1024, 3, 400), (16, 3, 4, 517, 3, 2957), (16, 4, 3, 779, 1, 3117), (16, 4, 4, 1021, 3, 265),
-    (32, 3, 6, 513, 1, 4557), (32, 3, 6, 768, 2, 4557), (32, 3, 8, 516, 3, 2957), (32, 4, 6, 778, 1, 3117), (32, 4, 8, 1021, 3, 378), (32, 4, 8, 1024, 3, 265)]
+    (8, 3, 2, 3, 765, 3, 2317), (8, 4, 2, 3, 1001, 3, 265), (8, 4, 2, 3, 1024, 3, 400), (16, 3, 4, 3, 517, 3, 2957), (16, 4, 3, 3, 779, 1, 3117),
+    (16, 4, 4, 3, 1021, 3, 265), (32, 3, 6, 3, 513, 1, 4557), (32, 3, 6, 3, 768, 2, 4557), (32, 3, 8, 3, 516, 3, 2957), (32, 4, 6, 3, 778, 1, 3117),
+    (32, 4, 8, 2, 1021, 3, 378), (32, 4, 8, 2, 1024, 3, 265), (32, 4, 8, 3, 1021, 3, 633)]
 WIDTHS = {3: (517, 764), 4: (771, 1024), 6: (1031, 1536), 8: (1541, 2048)}           # N by K chunks of a wave: odd, a multiple of four
 
 
 @pytest.mark.parametrize("npw,kpw,ct,fewest,most,depth", KERNELS)
 def test_every_kernel(npw, kpw, ct, fewest, most, depth, gpu_device, monkeypatch):
-    """One to four tiles per row group, the last group's one short: the oracle for rows of the first, a middle and the last tile, every
-    row the bits of the way without slots and of every other batch."""
+    """One to five tiles per row group, the last group's one short: the oracle for rows of the first, a middle and the last tile, every
+    row the bits of the way without slots and of every other batch.  An operand is asked for one item ahead of its group's tiles at most."""
     T = 12
     for N, k in zip(WIDTHS[kpw], (fewest, most)):
         groups = 8
         while 32 * ((N + 31) // 32) // npw > 256 // groups:
             groups //= 2
-        batches = [16 * groups - 7] + [16 * (groups * (nt - 1) + max(1, groups - 1)) - 7 for nt in (2, 3, 4)]
+        batches = [16 * groups - 7] + [16 * (groups * (nt - 1) + max(1, groups - 1)) - 7 for nt in (2, 3, 4, 5)]
         batches = batches[:2] if (npw, kpw, ct) == (16, 8, 7) else batches           # (LDS holds two tiles' states beside its weights)
         print(f"[case] chip <{npw}, {kpw}, {ct}> N={N} k={k} B={batches}", flush=True)
         J0, J1, B = -1.0 / N, 0.6, batches[-1]
@@ -142,22 +143,23 @@ def test_every_kernel(npw, kpw, ct, fewest, most, depth, gpu_device, monkeypatch
         monkeypatch.delenv("RINGATTR_TEAM_GATHER_US")
         for nt, rows in enumerate(batches, 1):
             h, name = _forward([t[0][:rows].clone(), t[1], t[2], t[3][:rows].clone()], "gelu", J0, J1)
-            assert f"<{npw},{kpw},{ct},{min(nt, depth)}>" in name, (N, k, rows, name)
+            ahead = 1 if nt <= 2 else 3 if (rows + 15) // 16 // groups >= 4 else 2
+            assert f"<{npw},{kpw},{ct},{min(ahead, depth)}>" in name, (N, k, rows, name)
             assert torch.equal(h, want[:, :rows]), (N, k, rows)
         some = [0, 15, B // 2, B - 1]
         ref, _ = O.forward_dense(p["A"][some], p["Wa"], J0, J1, p["Wo"], p["r0"][some], 0.15, "gelu")
         assert O.max_rel_err(want[:, some].cpu().numpy(), ref) <= 1e-2               # one bf16 rounding per operand, as everywhere
 
 
-@pytest.mark.parametrize("npw,kpw,ct,N,k,B", FEW_CHANNELS)
-def test_every_kernel_of_few_channels(npw, kpw, ct, N, k, B, gpu_device, monkeypatch):
-    print(f"[case] chip <{npw}, {kpw}, {ct}> N={N} k={k} B={B}", flush=True)
+@pytest.mark.parametrize("npw,kpw,ct,depth,N,k,B", FEW_CHANNELS)
+def test_every_kernel_of_few_channels(npw, kpw, ct, depth, N, k, B, gpu_device, monkeypatch):
+    print(f"[case] chip <{npw}, {kpw}, {ct}, {depth}> N={N} k={k} B={B}", flush=True)
     J0, J1 = -1.0 / N, 0.6
     p = make_problem(23, B, 12, k, N, bump="vm", action="dense")
     t = _tensors(p, gpu_device)
     monkeypatch.setenv("RINGATTR_CHIP", str(npw))
     h, name = _forward(t, "silu", J0, J1)
-    assert f"<{npw},{kpw},{ct},3>" in name, name
+    assert f"<{npw},{kpw},{ct},{depth}>" in name, name
     monkeypatch.setenv("RINGATTR_TEAM_GATHER_US", "-1")
     without, _ = _forward(t, "silu", J0, J1)
     assert torch.equal(h, without)
@@ -198,6 +200,32 @@ def test_replayed_graph(gpu_device):
 def test_rule(B, T, k, N, chip, gpu_device):
     _, name = _forward(_tensors(make_problem(15, B, T, k, N, bump="vm", action="dense"), gpu_device), "relu", 0.0, 0.5)
     assert ("chip" in name) == chip, name
+
+
+# two of the channels driven; three tiles in every row group, and four in all but one
+@pytest.mark.parametrize("B,k,N", [(89, 16, 896), (107, 8, 891), (75, 14, 920)])
+def test_few_tiles_per_group_take_no_longer_than_the_panels(B, k, N, gpu_device, monkeypatch):
+    """An operand that was asked for before it could be there held up what it waited for (896: 404 us, the panels 331; now 239)."""
+    T = 40
+    p = make_problem(20, B, T, k, N, bump="vm", action="dense")
+    p["A"][:, :, 2:] = 0.0
+    t = _tensors(p, gpu_device)
+    least = {}
+    for switch, want in (("", "chip"), ("0", "panel"), ("", "chip"), ("0", "panel")):
+        if switch:
+            monkeypatch.setenv("RINGATTR_CHIP", switch)
+        else:
+            monkeypatch.delenv("RINGATTR_CHIP", raising=False)
+        for _ in range(6):
+            start, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            start.record()
+            _, name = _forward(t, "tanh", -1.0 / N, 0.5)
+            end.record()
+            torch.cuda.synchronize()
+            assert want in name
+            least[want] = min(least.get(want, 1e9), start.elapsed_time(end))
+    print(f"[case] B={B} k={k} N={N}: chip {least['chip']:.3f} ms, panels {least['panel']:.3f}", flush=True)
+    assert least["chip"] < least["panel"]
 
 
 def test_row_groups_that_do_not_gather_cost_little(gpu_device, monkeypatch):
