@@ -459,7 +459,9 @@ __global__ __launch_bounds__(64 * W) void ring_chip_fwd_kernel(RingChipArgs c) {
     __builtin_amdgcn_raw_buffer_store_b32(EMPTY, rsrc, (int)xoff, (int)old, ST_THROUGH);
     __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, rn), hr, (int)hoff, 0, 0);
     if constexpr (DEPTH == 1) {
-      if (c.nt == 1) lds_barrier();        // (the first waves' polling would hold up the last ones' stores)
+      // (the first waves' polling would hold up the last ones' stores; also where other groups have two tiles: N = 968, 6 channels,
+      // B = 69, T = 40 265 -> 199 us a call)
+      if (my_nt == 1) lds_barrier();
       ask(nx);
     }
     ++it;
