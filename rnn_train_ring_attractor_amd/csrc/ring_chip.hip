@@ -687,10 +687,10 @@ ChipPlan chip_plan(int N, int k, int T, int B) {
     const size_t xbytes = (size_t)slots * nbt * KC * CHUNK_BYTES;
     if (xbytes >= ((size_t)1 << 30)) continue;           // (offsets past the buffer say 'nowhere')
     // The deepest prefetch that registers and LDS have room for and the tiles can use: an operand is the state that the group made
-    // its tiles' number of items ago, and asked for as soon as the item behind that, it is not there.  What is asked again then
-    // holds up the stores it waits for (us a call of T = 40, three, two and one item ahead): one tile per group behind, N = 1021, 3
-    // channels, B = 377 539, 261, 279, N = 896, 16 channels, B = 89 404, 239, 266, N = 768, 6 channels, B = 121 two and one 225, 150;
-    // two behind, N = 896, B = 121 280, 294, 347.  A group that is a tile short decides for all from four tiles on: B = 107 368, 303.
+    // its tiles' number of items ago, and asked for right behind that item it is not there.  Asking again then holds up the stores it
+    // waits for.  us a call of T = 40 with three, two and one operands on their way: three tiles per group, N = 1021, 3 channels,
+    // B = 377 539, 261, 279, N = 896, 16 channels, B = 89 404, 239, 266; two tiles, N = 768, 6 channels, B = 121 two and one 225, 150;
+    // four, N = 896, B = 121 280, 294, 347.  Where four tiles are the most, a group with three decides for all: B = 107 368, 303.
     const int fewest = nbt / nrg;
     int depth = fewest >= 4 ? 3 : (nt >= 3 ? 2 : 1);
     while (depth > 1 && (depth == 3 ? r.parked[2] > 0 : chip_lds(r.npw, r.mats, r.parked[1], nt).total > CHIP_LDS)) --depth;

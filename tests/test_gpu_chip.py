@@ -125,7 +125,8 @@ WIDTHS = {3: (517, 764), 4: (771, 1024), 6: (1031, 1536), 8: (1541, 2048)}      
 @pytest.mark.parametrize("npw,kpw,ct,fewest,most,depth", KERNELS)
 def test_every_kernel(npw, kpw, ct, fewest, most, depth, gpu_device, monkeypatch):
     """One to five tiles per row group, the last group's one short: the oracle for rows of the first, a middle and the last tile, every
-    row the bits of the way without slots and of every other batch.  An operand is asked for one item ahead of its group's tiles at most."""
+    row the bits of the way without slots and of every other batch.  With one or two tiles an operand is asked for behind the item
+    before, with three one item ahead, two only where every group has four."""
     T = 12
     for N, k in zip(WIDTHS[kpw], (fewest, most)):
         groups = 8
