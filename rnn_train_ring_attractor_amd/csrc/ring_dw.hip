@@ -73,13 +73,165 @@ __device__ __forceinline__ bf16x8 gate_frag(bf16x8 x, const f32x4 (&g8)[2]) {
   return o;
 }
 
+// ------------------------------------------------------------------------------------------------
+// Short contractions: the four waves of a workgroup share out its K chunks instead of its rows.
+// ------------------------------------------------------------------------------------------------
+// What bounds a few hundred chunks is not the products: with a 128 x 128 block per workgroup the chip is only filled by many
+// K splits, and a split's partial sums (64 KiB a matrix and block) are written and read once more.  Here a workgroup has a
+// 32 x 128 block (a quarter of it), its wave w every fourth chunk from the w-th on, and the waves' sums are added in LDS: for
+// the same number of workgroups a quarter of the splits and of the partial sums.  Blocks past the ring's own tiles are not
+// there at all, and a launch takes up to four matrices (256 accumulation registers).  No barrier and no LDS stage: each wave
+// loads its ten fragments of a chunk, DWS_DEPTH chunks ahead; the gates go from lane to lane through a wave's own LDS.
+// us of contraction and reduction, with 128 x 128 blocks and here: N = 120, 2 channels, 240 chunks 19.9 -> 13.4; N = 256, 2 channels,
+// 400 chunks 25.0 -> 17.8; N = 360, 3 channels, 266 chunks (two launches there) 48.6 -> 22.7.
+constexpr int DWS_DEPTH = 3;
+
+template <int NG>
+struct DwChunk {
+  bf16x8 a[DW_WI], b[DW_WJ];
+  float gate[NG > 2 ? 2 : 1];           // (matrix, row, step) number lane (+ 64) of the chunk
+};
+
+// Tiles per side that hold neurons of the ring.
+__host__ __device__ __forceinline__ int dw_tiles(const RingDwArgs& p, int NT) {
+  const int group = p.linear_tiles ? 1 : NT / 4;          // (NT / 4 consecutive tiles share 4 NT neurons)
+  return (p.N + 16 * group - 1) / (16 * group) * group;
+}
+
+template <int NMAT, bool FIRST>
+__device__ __forceinline__ void dw_chunk_waves(const RingDwArgs& p, int m0, int NT) {
+  constexpr int NG = NMAT - (FIRST ? 1 : 0), NLD = NG > 2 ? 2 : 1;
+  __shared__ __attribute__((aligned(16))) f32x4 sums[4][DW_WJ][64];
+  __shared__ __attribute__((aligned(16))) float gates[4][DWS_DEPTH][4][16][2];     // [wave][stage][gated matrix][row][step]
+  const int tid = threadIdx.x, wv = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+  const int tiles = dw_tiles(p, NT), ni = (tiles + DW_WI - 1) / DW_WI, nb = ni * ((tiles + DW_WJ - 1) / DW_WJ);
+  // The workgroups of a K split read the same chunks: in the order in which the XCDs (dealt out round robin) hold consecutive
+  // workgroups, so that a split is on as few as can be.
+  const int at = (blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3), z = at / nb, block = at % nb;
+  if (z >= p.nz) return;
+  const int it0 = (block % ni) * DW_WI, jt0 = (block / ni) * DW_WJ;
+  const int T = p.T, k = p.k, nbt = p.nbt;
+  const int nchunk = nbt * ((T + 1) / 2);                 // (the host checked that it fits an int)
+  const int ch0 = (int)((long)nchunk * z / p.nz) + wv, ch1 = (int)((long)nchunk * (z + 1) / p.nz);
+  const int n = ch0 < ch1 ? (ch1 - ch0 + 3) / 4 : 0;
+
+  f32x4 acc[NMAT][DW_WI][DW_WJ];
+#pragma unroll
+  for (int a = 0; a < NMAT; ++a)
+#pragma unroll
+    for (int ii = 0; ii < DW_WI; ++ii)
+#pragma unroll
+      for (int u = 0; u < DW_WJ; ++u) {
+        acc[a][ii][u] = f32x4{0.f, 0.f, 0.f, 0.f};
+        asm volatile("" : "+a"(acc[a][ii][u]));
+      }
+
+  // the fetch cursor parks on the wave's last chunk, as above (a wave without any: on some chunk)
+  const int first = ch0 < nchunk ? ch0 : nchunk - 1;
+  const size_t step = (size_t)4 * NT * 64;
+  const bf16x8* ga = reinterpret_cast<const bf16x8*>(p.gfrag) + ((size_t)first * NT + it0) * 64 + lane;
+  const bf16x8* rb = reinterpret_cast<const bf16x8*>(p.rfrag) + ((size_t)first * NT + jt0) * 64 + lane;
+  int left = n, fb = first % nbt, ft = first / nbt;
+  const int db = 4 % nbt, dt = 4 / nbt;
+  const int row = (lane >> 1) & 15, tt = lane & 1;
+  auto fetch = [&](DwChunk<NG>& s) {
+#pragma unroll
+    for (int u = 0; u < DW_WI; ++u) s.a[u] = ga[u * 64];
+#pragma unroll
+    for (int u = 0; u < DW_WJ; ++u) s.b[u] = rb[u * 64];
+    // rows past B and the missing second step of an odd-length sequence meet zero g fragments: any gate will do there
+    const int b = 16 * fb + row, bc = b < p.B ? b : p.B - 1, tg = 2 * ft + tt < T ? 2 * ft + tt : 2 * ft;
+#pragma unroll
+    for (int v = 0; v < NLD; ++v) {
+      const int gm = 2 * v + (lane >> 5), ch = m0 + (gm < NG ? gm : 0) - (FIRST ? 0 : 1);
+      s.gate[v] = NG > 0 ? p.A[((size_t)bc * T + tg) * k + ch] : 0.f;
+    }
+    const int adv = left > 1 ? 1 : 0;
+    left -= adv;
+    ga += adv ? step : 0;
+    rb += adv ? step : 0;
+    fb += adv ? db : 0;
+    ft += adv ? dt : 0;
+    const int wrap = fb >= nbt ? 1 : 0;
+    fb -= wrap ? nbt : 0;
+    ft += wrap;
+  };
+  auto publish = [&](const DwChunk<NG>& s, int buf) {
+    if constexpr (NG > 0)
+#pragma unroll
+      for (int v = 0; v < NLD; ++v) (&gates[wv][buf][0][0][0])[64 * v + lane] = s.gate[v];
+  };
+  auto compute = [&](const DwChunk<NG>& s, int buf) {
+    f32x4 g8[NG > 0 ? NG : 1][2];
+#pragma unroll
+    for (int a = 0; a < NG; ++a) {
+      const f32x4* gp = reinterpret_cast<const f32x4*>(&gates[wv][buf][a][4 * (lane >> 4)][0]);
+      g8[a][0] = gp[0];
+      g8[a][1] = gp[1];
+    }
+#pragma unroll
+    for (int a = 0; a < NMAT; ++a)
+#pragma unroll
+      for (int ii = 0; ii < DW_WI; ++ii) {
+        const bf16x8 gg = (FIRST && a == 0) ? s.a[ii] : gate_frag(s.a[ii], g8[a - (FIRST ? 1 : 0)]);
+#pragma unroll
+        for (int u = 0; u < DW_WJ; ++u) acc[a][ii][u] = mfma16(gg, s.b[u], acc[a][ii][u]);
+      }
+  };
+  DwChunk<NG> st[DWS_DEPTH];
+#pragma unroll
+  for (int d = 0; d < DWS_DEPTH; ++d) {
+    fetch(st[d]);
+    __builtin_amdgcn_sched_barrier(0);
+  }
+  publish(st[0], 0);
+  int i = 0;
+#pragma unroll 1
+  for (; i + DWS_DEPTH <= n; i += DWS_DEPTH)
+#pragma unroll
+    for (int d = 0; d < DWS_DEPTH; ++d) {
+      compute(st[d], d);
+      __builtin_amdgcn_sched_barrier(0);
+      fetch(st[d]);
+      __builtin_amdgcn_sched_barrier(0);
+      publish(st[(d + 1) % DWS_DEPTH], (d + 1) % DWS_DEPTH);
+    }
+#pragma unroll
+  for (int d = 0; d < DWS_DEPTH - 1; ++d) {              // what is left: in stages 0 ...
+    if (i + d >= n) break;
+    compute(st[d], d);
+    publish(st[d + 1], d + 1);
+  }
+
+  // the waves' sums, in wave order; wave w writes out columns 2w and 2w + 1
+#pragma unroll
+  for (int a = 0; a < NMAT; ++a)
+#pragma unroll
+    for (int ii = 0; ii < DW_WI; ++ii) {
+      lds_barrier();
+#pragma unroll
+      for (int u = 0; u < DW_WJ; ++u) sums[wv][u][lane] = acc[a][ii][u];
+      lds_barrier();
+#pragma unroll
+      for (int uu = 0; uu < 2; ++uu) {
+        const int u = 2 * wv + uu;
+        const f32x4 s = ((sums[0][u][lane] + sums[1][u][lane]) + sums[2][u][lane]) + sums[3][u][lane];
+        p.partial[((((size_t)z * (k + 1) + m0 + a) * NT + it0 + ii) * NT + jt0 + u) * 64 + lane] = s;
+      }
+    }
+}
+
 }  // namespace
 
 // seg_begin / seg_end: the launch covers K chunks [seg_begin, seg_end) of the sequence (chunk = time-step pair *
 // batch tiles + batch tile, so a range of chunks is a range of time steps); add != 0: the wave adds its result
-// to the partial sums an earlier launch left.
+// to the partial sums an earlier launch left.  NC = 0: dw_chunk_waves, of matrices mg ... at NT = seg_begin tiles a side.
 template <int NC, int NMAT, bool FIRST>
 __global__ __launch_bounds__(256) void ring_dw_direct_kernel(RingDwArgs p, int mg, int seg_begin, int seg_end, int add) {
+  if constexpr (NC == 0) {
+    dw_chunk_waves<NMAT, FIRST>(p, mg, seg_begin);
+    return;
+  } else {
   constexpr int NT = 4 * NC;
   constexpr int NB = NT / 8;             // 128-neuron blocks per side
   constexpr int NG = NMAT - (FIRST ? 1 : 0);
@@ -221,6 +373,7 @@ __global__ __launch_bounds__(256) void ring_dw_direct_kernel(RingDwArgs p, int m
         *dst = add ? *dst + acc[a][ii][u] : acc[a][ii][u];
       }
   }
+  }
 }
 
 // N <= 128: a launch per three matrices, of a few workgroups where there is little to contract, against one launch for all
@@ -329,6 +482,71 @@ hipError_t ring_launch_dw_tiled(const RingDwArgs& a, int NC, hipStream_t st) {
       }
       if (e != hipSuccess) return e;
     }
+  }
+  return hipSuccess;
+}
+
+// Which of the two kernels contracts: us of either with its reduction, from the chunks a workgroup walks.  Fitted to 60 shapes
+// (N = 120 to 2048, 2 to 16 channels, 1 to 131072 chunks): a chunk of three matrices takes 0.75 us here and 1.1 times that in
+// dw_chunk_waves (both sides near the matrix rate), a launch's start and end 4 and 5 us a round of 256 workgroups, partial sums are
+// written and read at 5 TB/s.  So long contractions of whole 128 x 128 blocks stay here (contraction and reduction, us, here and
+// there: N = 1024, 2 channels, 7680 chunks 1320 and 1470; N = 256, 15360 chunks 195 and 199; N = 512, 131072 chunks 5500 and
+// 5860) and the others go there: N = 256, 2 channels, 100 chunks 18 less; 3 channels (one launch instead of two) 20 less at 100
+// chunks, 92 at 15360; N = 640 (padded to 1024 here), 2 channels, 7680 chunks 690 less.
+// Returns the K splits of dw_chunk_waves, 0: not that kernel.
+int ring_dw_short_nz(int N, int NC, int k, int nbt, int T, int tiled_nz) {
+  if (getenv("RINGATTR_DW_SEGMENT")) return 0;             // (asks for the kernel that is cut)
+  RingDwArgs a = {};
+  a.N = N;
+  const int NB = 4 * NC / 8, tiles = dw_tiles(a, 4 * NC), groups = (k + 4) / 4;
+  const long nb = (long)((tiles + DW_WI - 1) / DW_WI) * ((tiles + DW_WJ - 1) / DW_WJ), nchunk = (long)nbt * ((T + 1) / 2);
+  // as many as fill the chip, each with two chunks a wave at least
+  long nz = 256 / nb;
+  if (nz > nchunk / 8) nz = nchunk / 8;
+  if (nz > tiled_nz) nz = tiled_nz;
+  if (nz < 1) nz = 1;
+  constexpr float CHUNK = 0.75f, BYTES = 5e6f, tiled_share[4] = {0.f, 0.6f, 0.8f, 1.f}, short_share[5] = {0.f, 0.6f, 0.85f, 1.1f, 1.28f};
+  auto chunks = [&](long parts) { return (float)((nchunk + parts - 1) / parts) * CHUNK; };
+  const float tiled_rounds = (float)(((long)NB * NB * tiled_nz + 255) / 256), short_rounds = (float)((nb * nz + 255) / 256);
+  float tiled = 8.f * tiled_nz * (1 + k) * (64.f * NC) * (64.f * NC) / BYTES, here = 8.f * nz * (1 + k) * (16.f * tiles) * (16.f * tiles) / BYTES;
+  for (int m = 0; m <= k; m += 3) tiled += tiled_rounds * (chunks(tiled_nz) * tiled_share[k + 1 - m < 3 ? k + 1 - m : 3] + 4.f);
+  for (int m = 0, left = groups; left > 0; --left) {
+    const int nm = (k + 1 - m + left - 1) / left;
+    here += short_rounds * (chunks(4 * nz) * short_share[nm] + 5.f);
+    m += nm;
+  }
+  return here < tiled ? (int)nz : 0;
+}
+
+// Through dw_chunk_waves where that is the faster one; its K splits (no more than there were) go into a.nz.
+hipError_t ring_launch_dw_short(RingDwArgs& a, int NC, hipStream_t st) {
+  const int nz = ring_dw_short_nz(a.N, NC, a.k, a.nbt, a.T, a.nz);
+  if (nz == 0) return ring_launch_dw_tiled(a, NC, st);
+  a.nz = nz;
+  const int NT = 4 * NC, tiles = dw_tiles(a, NT);
+  const int nb = ((tiles + DW_WI - 1) / DW_WI) * ((tiles + DW_WJ - 1) / DW_WJ);
+  const dim3 grid((unsigned)(8 * ((nb * nz + 7) / 8)));
+  for (int m0 = 0, groups = (a.k + 4) / 4; m0 <= a.k; --groups) {
+    const int nm = (a.k + 1 - m0 + groups - 1) / groups;          // matrices shared out evenly
+    auto go = [&](auto kern) { RING_LAUNCH(kern, grid, dim3(256), 0, st, a, m0, NT, 0, 0); };
+    if (m0 == 0) {
+      switch (nm) {
+        case 4: go(ring_dw_direct_kernel<0, 4, true>); break;
+        case 3: go(ring_dw_direct_kernel<0, 3, true>); break;
+        case 2: go(ring_dw_direct_kernel<0, 2, true>); break;
+        default: go(ring_dw_direct_kernel<0, 1, true>); break;
+      }
+    } else {
+      switch (nm) {
+        case 4: go(ring_dw_direct_kernel<0, 4, false>); break;
+        case 3: go(ring_dw_direct_kernel<0, 3, false>); break;
+        case 2: go(ring_dw_direct_kernel<0, 2, false>); break;
+        default: go(ring_dw_direct_kernel<0, 1, false>); break;
+      }
+    }
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+    m0 += nm;
   }
   return hipSuccess;
 }

@@ -980,17 +980,6 @@ __global__ __launch_bounds__(256) void ring_dw_reduce_kernel(RingDwArgs p, int N
   const size_t per_z = (size_t)(p.k + 1) * NT * NT * 64;
   const size_t u = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (u >= per_z) return;
-  // fixed summation order z = 0, 1, 2, ...; the loads of sixteen slices are issued together
-  f32x4 s = {0.f, 0.f, 0.f, 0.f};
-  int z = 0;
-  for (; z + 16 <= p.nz; z += 16) {
-    f32x4 v[16];
-#pragma unroll
-    for (int i = 0; i < 16; ++i) v[i] = __builtin_nontemporal_load(&p.partial[(size_t)(z + i) * per_z + u]);
-#pragma unroll
-    for (int i = 0; i < 16; ++i) s += v[i];
-  }
-  for (; z < p.nz; ++z) s += p.partial[(size_t)z * per_z + u];
   const int lane = (int)(u & 63);
   size_t v = u >> 6;
   const int jt = (int)(v % NT);
@@ -999,12 +988,29 @@ __global__ __launch_bounds__(256) void ring_dw_reduce_kernel(RingDwArgs p, int N
   const int mm = (int)(v / NT);
   const int q = lane >> 4, n = lane & 15;
   const int j = p.linear_tiles ? 16 * jt + n : 16 * NC * (jt / NC) + NC * n + (jt % NC);
-  if (j >= p.N) return;
+  const int i0 = p.linear_tiles ? 16 * it + 4 * q : 16 * NC * (it / NC) + NC * 4 * q + (it % NC);
+  if (j >= p.N || i0 >= p.N) return;                       // (also tiles past the ring, which have no partial sums)
+  // fixed summation order z = 0, 1, 2, ...; the loads of sixteen slices (where there are as many) are issued together
+  f32x4 s = {0.f, 0.f, 0.f, 0.f};
+  int z = 0;
+  auto some = [&](auto count) {
+    constexpr int COUNT = decltype(count)::value;
+    f32x4 v[COUNT];
+#pragma unroll
+    for (int i = 0; i < COUNT; ++i) v[i] = __builtin_nontemporal_load(&p.partial[(size_t)(z + i) * per_z + u]);
+#pragma unroll
+    for (int i = 0; i < COUNT; ++i) s += v[i];
+    z += COUNT;
+  };
+  while (z + 16 <= p.nz) some(std::integral_constant<int, 16>{});
+  if (z + 8 <= p.nz) some(std::integral_constant<int, 8>{});
+  if (z + 4 <= p.nz) some(std::integral_constant<int, 4>{});
+  for (; z < p.nz; ++z) s += p.partial[(size_t)z * per_z + u];
   float* out = (mm == 0) ? p.grad_Wo : p.grad_Wa + (size_t)(mm - 1) * p.N * p.N;
   const float scale = (mm == 0) ? p.J1 : 1.f;
 #pragma unroll
   for (int e = 0; e < 4; ++e) {
-    const int i = p.linear_tiles ? 16 * it + 4 * q + e : 16 * NC * (it / NC) + NC * (4 * q + e) + (it % NC);
+    const int i = i0 + (p.linear_tiles ? e : NC * e);
     if (i < p.N) {
       float* o = out + (size_t)i * p.N + j;
       *o = p.accumulate ? *o + scale * s[e] : scale * s[e];
@@ -1420,7 +1426,8 @@ hipError_t ring_launch_bptt(const RingBpttArgs& a, int NCv, hipStream_t st) {
   return e;
 }
 
-hipError_t ring_launch_dw(const RingDwArgs& a, int NCv, hipStream_t st) {
+hipError_t ring_launch_dw(const RingDwArgs& args, int NCv, hipStream_t st) {
+  RingDwArgs a = args;
   const int NT = 4 * NCv;
   const long waves = (long)(NT / 2) * ((a.k + 3) / 3) * a.nz;
   const int blocks = (int)((waves + 3) / 4);
@@ -1428,7 +1435,7 @@ hipError_t ring_launch_dw(const RingDwArgs& a, int NCv, hipStream_t st) {
   {
   ProfScope prof(4, st);
   if (ring_dw_tiled_applicable(NCv, a.k, (long)a.nbt * ((a.T + 1) / 2))) {
-    e = ring_launch_dw_tiled(a, NCv, st);   // every group's launch status, first failure wins
+    e = ring_launch_dw_short(a, NCv, st);   // every group's launch status, first failure wins
   } else {
     if (NCv == 1) RING_LAUNCH((ring_dw_kernel<1, 4>), dim3(blocks), dim3(256), 0, st, a);
     else if (NCv == 2) RING_LAUNCH((ring_dw_kernel<2, 8>), dim3(blocks), dim3(256), 0, st, a);

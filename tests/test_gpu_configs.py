@@ -973,3 +973,33 @@ def test_weight_gradient_kernels_of_narrow_rings_on_either_side_of_their_line(B,
     for got, name in ((Wa.grad, "grad_Wa"), (Wo.grad, "grad_Wo")):
         x = got.cpu().numpy()
         assert O.cosine(x, g[name]) >= GRAD_COS and O.max_rel_err(x, g[name]) <= GRAD_TOL, name
+
+
+# Short contractions: one chunk, fewer chunks than waves, remainders; one to four matrices a launch and several launches; K splits on
+# one XCD and on several; widths whose last block is not full, in both tile orders; odd numbers of steps, rows past the batch.
+@pytest.mark.parametrize("N,B,T,k", [(120, 32, 8, 2), (256, 16, 1, 3), (128, 70, 37, 2), (130, 40, 21, 1), (200, 33, 25, 3), (256, 64, 51, 2), (256, 100, 7, 4),
+                                     (360, 100, 15, 3), (360, 50, 20, 7), (512, 16, 3, 6), (640, 48, 12, 2), (761, 20, 6, 5), (1100, 40, 5, 2)])
+def test_short_weight_gradients_against_the_tiled_kernel_and_the_oracle(N, B, T, k, gpu_device, monkeypatch):
+    from rnn_train_ring_attractor_amd import ring_rnn_cuda_func, _lib
+    print(f"[case] short weight gradients N={N} B={B} T={T} k={k}", flush=True)
+    p = make_problem(95, B, T, k, N, action="dense")
+
+    def run():
+        Wa, Wo = _t(p["Wa"], gpu_device).requires_grad_(True), _t(p["Wo"], gpu_device).requires_grad_(True)
+        h = ring_rnn_cuda_func(_t(p["A"], gpu_device), Wa, -0.3 / N, 0.4, Wo, _t(p["r0"], gpu_device), 0.15, "tanh")
+        h.backward(_t(p["G"], gpu_device))
+        return Wo.grad.cpu().numpy(), Wa.grad.cpu().numpy(), _lib.last_kernel_names()["dw"]
+
+    short, again = run(), run()
+    assert short[2].startswith("ring_dw_direct_kernel<0,")
+    assert np.array_equal(short[0], again[0]) and np.array_equal(short[1], again[1])
+    monkeypatch.setenv("RINGATTR_DW_SEGMENT", "0")            # the kernel that can be cut, uncut
+    tiled = run()
+    assert not tiled[2].startswith("ring_dw_direct_kernel<0,")
+    # the same bf16 products, summed in fp32 in another order: at most 37 * 70 of them, error about sqrt(2590) * 2^-24 of a typical sum
+    for got, want in zip(short[:2], tiled[:2]):
+        assert O.max_rel_err(got, want) <= 1e-5
+    ref, _ = O.forward_dense(p["A"], p["Wa"], -0.3 / N, 0.4, p["Wo"], p["r0"], 0.15, "tanh")
+    g = O.backward_dense(p["G"], p["A"], p["Wa"], -0.3 / N, 0.4, p["Wo"], ref, p["r0"], 0.15, "tanh")
+    for got, name in zip(short[:2], ("grad_Wo", "grad_Wa")):
+        assert O.cosine(got, g[name]) >= GRAD_COS and O.max_rel_err(got, g[name]) <= GRAD_TOL, name
