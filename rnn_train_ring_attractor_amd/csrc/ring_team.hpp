@@ -420,7 +420,28 @@ __device__ __forceinline__ void team_products(const TeamCompute<KPW, C16, MR, WK
     }
     if (GA && m <= c.k) row_put(d, m);
   }
-  auto lds_matrix = [&](int m, float gm) {
+  // The matrices in LDS.  Where their number is known and registers are left (not beside 24 and more fragments: with 13 matrices in
+  // registers the reads spill, forward N = 512, 16 channels, B = 256, T = 20 92.6 -> 180 us a call), a matrix's first fragments are read
+  // while the one before it is multiplied, the first matrix's behind the registers' products: an LDS read's latency less a matrix.  us a
+  // call of T = 40, forward: N = 300, 9 channels, B = 800 278 -> 260; N = 700, 4 channels, B = 500 218 -> 203; N = 360, 3 channels,
+  // B = 1000 150 -> 140; N = 144, 3 channels, B = 900 73 -> 68.  Any number of matrices: reads ahead cost what they gain (N = 112, 16
+  // channels, B = 200, T = 60 144 -> 151).
+  constexpr bool AHEAD = EX != TEAM_MORE && MR * C16 * KPW <= 18;
+  bf16x8 f[KPW];
+  auto fetch = [&](int m) {
+    if constexpr (!AHEAD) return;
+    const bf16x8* src = wl + ((size_t)(m - MR) * C16 * c.KC + w) * 64 + lane;
+#pragma unroll
+    for (int kk = 0; kk < KPW; ++kk)
+      if (kk + 1 < KPW || w + WK * kk < c.KC) f[kk] = src[(size_t)WK * kk * 64];
+  };
+  auto lds_matrix = [&](int m, float gm, int next) {
+    bf16x8 f0[KPW];
+    if constexpr (AHEAD) {
+#pragma unroll
+      for (int kk = 0; kk < KPW; ++kk) f0[kk] = f[kk];
+      if (next) fetch(next);
+    }
     // a channel that is zero for all 16 rows contributes nothing (zero-padded action signals); dL/dA needs every product
     if (!GA && __ballot(gm != 0.f) == 0) return;
     float d = 0.f;
@@ -430,7 +451,7 @@ __device__ __forceinline__ void team_products(const TeamCompute<KPW, C16, MR, WK
       const bf16x8* src = wl + ((size_t)((m - MR) * C16 + cc) * c.KC + w) * 64 + lane;
 #pragma unroll
       for (int kk = 0; kk < KPW; ++kk)
-        if (kk + 1 < KPW || w + WK * kk < c.KC) P = mfma16(src[(size_t)WK * kk * 64], x[kk], P);
+        if (kk + 1 < KPW || w + WK * kk < c.KC) P = mfma16(AHEAD && cc == 0 ? f0[kk] : src[(size_t)WK * kk * 64], x[kk], P);
 #pragma unroll
       for (int i = 0; i < 4; ++i) acc[cc][i] = fmaf(gm, P[i], acc[cc][i]);
       row_dot(d, P, cc);
@@ -440,17 +461,19 @@ __device__ __forceinline__ void team_products(const TeamCompute<KPW, C16, MR, WK
   if constexpr (EX == TEAM_MORE) {
     // (gates are read a matrix ahead: forward N = 512, 16 channels, B = 256, T = 20 95.5 -> 93.2 us, N = 168, B = 223, T = 76 158.7 -> 152.3)
     float gn = gates[(MR - 1) * 16 + b];
+    if (last >= MR) fetch(MR);
     for (int m = MR; m <= last; ++m) {
       const float gm = gn;
       gn = gates[(m < c.k ? m : c.k - 1) * 16 + b];
-      lds_matrix(m, gm);
+      lds_matrix(m, gm, m < last ? m + 1 : m);
     }
   } else if constexpr (EX > 0) {
     float g[EX];
 #pragma unroll
     for (int i = 0; i < EX; ++i) g[i] = gates[(MR - 1 + i) * 16 + b];
+    fetch(MR);
 #pragma unroll
-    for (int i = 0; i < EX; ++i) lds_matrix(MR + i, g[i]);
+    for (int i = 0; i < EX; ++i) lds_matrix(MR + i, g[i], i + 1 < EX ? MR + i + 1 : 0);
   }
 }
 
