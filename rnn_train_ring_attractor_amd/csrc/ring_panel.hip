@@ -105,32 +105,64 @@ __device__ __forceinline__ void panel_pass(const PanelPass& p, const unsigned (&
 #pragma unroll
     for (int cur = 0; cur < 2; ++cur) {
       const int s = s0 + cur, nxt = cur ^ 1;
-      // (the barrier of the stage before: nobody reads that buffer any more)
-#pragma unroll
-      for (int i = 0; i < R; ++i) *stage(nxt, i, wv) = xr[i];
       const int sx = s + 2 < nst ? s + 2 : nst - 1;       // past the end: a re-read, unused
+      // Memory and LDS instructions go out a few at a time behind the matrix instructions of a column: a burst of them, in all four
+      // waves at once, keeps the one wave of a SIMD from issuing anything else (of 33 us of products at N = 2048, 16 channels,
+      // B = 256 the matrix instructions alone take 20, the LDS reads 5 more, the loads 7).  us a call, T = 20, in bursts and so:
+      // N = 2048, 16 channels, B = 256 913 -> 883, two of them driven 528 -> 497; T = 40: N = 1100, 8 channels, B = 600 1430 -> 1373,
+      // N = 1500, 2 channels, B = 1000 1293 -> 1250.  One or two row tiles have too few instructions to hide behind (N = 2048, two of
+      // 16 driven, B = 16, T = 40 408 -> 415): their loads go out together.
+      constexpr bool SPREAD = R >= 4;
+      auto next_x = [&](int i) {                          // (the barrier of the stage before: nobody reads that buffer any more)
+        *stage(nxt, i, wv) = xr[i];
+        xr[i] = panel_load(p.x, xrow[i] + (PANEL_S * sx + wv) * 1024, lane);
+      };
+      if constexpr (!SPREAD) {
 #pragma unroll
-      for (int i = 0; i < R; ++i) xr[i] = panel_load(p.x, xrow[i] + (PANEL_S * sx + wv) * 1024, lane);
-      __builtin_amdgcn_sched_barrier(0);
+        for (int i = 0; i < R; ++i) *stage(nxt, i, wv) = xr[i];
+#pragma unroll
+        for (int i = 0; i < R; ++i) xr[i] = panel_load(p.x, xrow[i] + (PANEL_S * sx + wv) * 1024, lane);
+        __builtin_amdgcn_sched_barrier(0);
+      }
 #pragma unroll
       for (int d = 0; d < PANEL_S; ++d) {
-        if (d + 1 < PANEL_S) {
+        if (d + 1 == PANEL_S) lds_barrier();              // the next stage is in LDS; all reads of this one have landed
+        auto next_xa = [&](int i) { xa[(d + 1) & 1][i] = d + 1 < PANEL_S ? *stage(cur, i, d + 1) : *stage(nxt, i, 0); };
+        if constexpr (!SPREAD) {
 #pragma unroll
-          for (int i = 0; i < R; ++i) xa[(d + 1) & 1][i] = *stage(cur, i, d + 1);
-        } else {
-          lds_barrier();                                  // the next stage is in LDS; all reads of this one have landed
-#pragma unroll
-          for (int i = 0; i < R; ++i) xa[(d + 1) & 1][i] = *stage(nxt, i, 0);
+          for (int i = 0; i < R; ++i) next_xa(i);
         }
         __builtin_amdgcn_sched_barrier(0);
         bf16x8(&w)[NV] = wf[PANEL_S * cur + d];
+        // (past the end: re-reads, unused.  With eight row tiles not all of one chunk, whose lines would be waited for one after the
+        // other: as a share of the time in bursts N = 1024, 16 channels, B = 256, T = 40 1.00 so, 0.97 with the last stage's chunks,
+        // N = 1500, two of 16 driven, B = 130 0.95 and 0.935; with four the other way round: N = 2000, 12 channels, B = 60 1.00 and 1.01)
+        const int kp = R == 8 ? PANEL_S * sx + d : PANEL_S * (s + 2) + d < KCH ? PANEL_S * (s + 2) + d : KCH - 1;
+        auto next_w = [&](int v) { w[v] = panel_load(p.w, p.wat[v] + kp * 1024, lane); };
 #pragma unroll
-        for (int v = 0; v < NV; ++v)
+        for (int v = 0; v < NV; ++v) {
+          if constexpr (SPREAD) {
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int i = v * R / NV; i < (v + 1) * R / NV; ++i) next_xa(i);
+            __builtin_amdgcn_sched_barrier(0);
+          }
 #pragma unroll
           for (int i = 0; i < R; ++i) acc[v][i] = mfma16(xa[d & 1][i], w[v], acc[v][i]);
-        const int kp = PANEL_S * (s + 2) + d < KCH ? PANEL_S * (s + 2) + d : KCH - 1;
+          if constexpr (SPREAD) {
+            __builtin_amdgcn_sched_barrier(0);
+            next_w(v);
+            if (d < 2) {
+              const int at = d * NV + v;
 #pragma unroll
-        for (int v = 0; v < NV; ++v) w[v] = panel_load(p.w, p.wat[v] + kp * 1024, lane);
+              for (int i = at * R / (2 * NV); i < (at + 1) * R / (2 * NV); ++i) next_x(i);
+            }
+          }
+        }
+        if constexpr (!SPREAD) {
+#pragma unroll
+          for (int v = 0; v < NV; ++v) next_w(v);
+        }
         __builtin_amdgcn_sched_barrier(0);
       }
     }
