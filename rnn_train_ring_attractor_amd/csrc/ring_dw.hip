@@ -23,6 +23,8 @@
 
 #include <stdlib.h>
 
+#include <utility>
+
 namespace {
 
 constexpr int DW_WI = 2;      // MFMA row tiles per wave (32 neurons of g)
@@ -36,6 +38,26 @@ struct DwStage {
   f32x4 bpart[2];                     // this thread's two fragments of the chunk's r_prev block (LDS stage)
   float gate;                         // one action gate of the chunk: matrix tid/32 % 4, row (tid/2) % 16, step tid % 2
 };
+
+// The order of a chunk's instructions around its N matrix instructions.  A SIMD has one wave here, and what that wave issues in a row
+// (twelve LDS reads, the fifteen vector instructions of a gated fragment, five loads, the LDS stage) keeps its matrix pipe waiting: 1575
+// cycles a chunk for 768 of products.  So a matrix instruction is followed by at most one of READS LDS reads, WRITES LDS writes, LOADS
+// loads (behind the last uses of what they replace) and two vector instructions, which cost it nothing.  us of contraction, left to the
+// compiler and so (same bits): N = 256, 15360 chunks 229 -> 194; N = 512, 12800 chunks 622 -> 517; N = 1024, 3840 chunks 690 -> 610.
+// By vector instructions behind each: N = 512 three 560, two and three in turn 543 to 552, two 521 to 530, one 615.
+template <int N, int READS, int WRITES, int LOADS, int I>
+__device__ __forceinline__ void dw_spread_one() {
+  constexpr int MFMA = 0x008, VALU = 0x002, VMEM_READ = 0x020, DS_READ = 0x100, DS_WRITE = 0x200, LATE = N - LOADS - 3;
+  __builtin_amdgcn_sched_group_barrier(MFMA, 1, 0);
+  if constexpr (I < READS) __builtin_amdgcn_sched_group_barrier(DS_READ, 1, 0);
+  if constexpr (I >= READS + 2 && I < READS + 2 + WRITES) __builtin_amdgcn_sched_group_barrier(DS_WRITE, 1, 0);
+  __builtin_amdgcn_sched_group_barrier(VALU, 2, 0);
+  if constexpr (I >= LATE && I < LATE + LOADS) __builtin_amdgcn_sched_group_barrier(VMEM_READ, 1, 0);
+}
+template <int READS, int WRITES, int LOADS, int... I>
+__device__ __forceinline__ void dw_spread(std::integer_sequence<int, I...>) {
+  (dw_spread_one<(int)sizeof...(I), READS, WRITES, LOADS, I>(), ...);
+}
 
 // NMAT matrices in this launch's group, the first of them ungated (Wo) when FIRST.
 // ga points at this lane's fragment of the wave's first row tile, rb at fragment `tid` of the block's
@@ -82,8 +104,8 @@ __device__ __forceinline__ bf16x8 gate_frag(bf16x8 x, const f32x4 (&g8)[2]) {
 // the same number of workgroups a quarter of the splits and of the partial sums.  Blocks past the ring's own tiles are not
 // there at all, and a launch takes up to four matrices (256 accumulation registers).  No barrier and no LDS stage: each wave
 // loads its ten fragments of a chunk, DWS_DEPTH chunks ahead; the gates go from lane to lane through a wave's own LDS.
-// us of contraction and reduction, with 128 x 128 blocks and here: N = 120, 2 channels, 240 chunks 19.9 -> 13.4; N = 256, 2 channels,
-// 400 chunks 25.0 -> 17.8; N = 360, 3 channels, 266 chunks (two launches there) 48.6 -> 22.7.
+// us of contraction and reduction, with 128 x 128 blocks and here: N = 120, 2 channels, 240 chunks 20.2 -> 13.4; N = 256, 2 channels,
+// 400 chunks 25.8 -> 16.4; N = 360, 3 channels, 266 chunks (two launches there) 48.9 -> 22.9.
 constexpr int DWS_DEPTH = 3;
 
 template <int NG>
@@ -148,12 +170,12 @@ __device__ __forceinline__ void dw_chunk_waves(const RingDwArgs& p, int m0, int 
     }
     const int adv = left > 1 ? 1 : 0;
     left -= adv;
-    ga += adv ? step : 0;
-    rb += adv ? step : 0;
-    fb += adv ? db : 0;
-    ft += adv ? dt : 0;
+    ga += adv * step;                                    // (products: a select of all of these would become a branch)
+    rb += adv * step;
+    fb += adv * db;
+    ft += adv * dt;
     const int wrap = fb >= nbt ? 1 : 0;
-    fb -= wrap ? nbt : 0;
+    fb -= wrap * nbt;
     ft += wrap;
   };
   auto publish = [&](const DwChunk<NG>& s, int buf) {
@@ -191,10 +213,10 @@ __device__ __forceinline__ void dw_chunk_waves(const RingDwArgs& p, int m0, int 
 #pragma unroll
     for (int d = 0; d < DWS_DEPTH; ++d) {
       compute(st[d], d);
-      __builtin_amdgcn_sched_barrier(0);
       fetch(st[d]);
-      __builtin_amdgcn_sched_barrier(0);
       publish(st[(d + 1) % DWS_DEPTH], (d + 1) % DWS_DEPTH);
+      dw_spread<2 * NG, (NG > 0 ? NLD : 0), DW_WI + DW_WJ + NLD>(std::make_integer_sequence<int, NMAT * DW_WI * DW_WJ>{});
+      __builtin_amdgcn_sched_barrier(0);
     }
 #pragma unroll
   for (int d = 0; d < DWS_DEPTH - 1; ++d) {              // what is left: in stages 0 ...
@@ -236,7 +258,7 @@ __global__ __launch_bounds__(256) void ring_dw_direct_kernel(RingDwArgs p, int m
   constexpr int NB = NT / 8;             // 128-neuron blocks per side
   constexpr int NG = NMAT - (FIRST ? 1 : 0);
   __shared__ __attribute__((aligned(16))) f32x4 lds_b[DW_LDS][DW_WJ * 64];
-  __shared__ __attribute__((aligned(16))) float lds_g[DW_LDS][4][16][2];   // [buffer][gated matrix][row][step]
+  __shared__ __attribute__((aligned(16))) float lds_g[DW_LDS][8][16][2];   // [buffer][gated matrix, twice][row][step]
   const int tid = threadIdx.x, wv = tid >> 6, lane = tid & 63;
   const int tiles = NB * NB;
   // keep the workgroups that share a K split on one XCD (workgroup ids are dealt round-robin to
@@ -321,7 +343,7 @@ __global__ __launch_bounds__(256) void ring_dw_direct_kernel(RingDwArgs p, int m
   auto publish = [&](const DwStage<NG>& s, int buf) {
     lds_b[buf][tid] = s.bpart[0];
     lds_b[buf][tid + 256] = s.bpart[1];
-    if (tid < 128) (&lds_g[buf][0][0][0])[tid] = s.gate;
+    (&lds_g[buf][0][0][0])[tid] = s.gate;               // (no branch: the loop is one block to schedule)
   };
 
   if (ch0 < ch1) {
@@ -341,10 +363,10 @@ __global__ __launch_bounds__(256) void ring_dw_direct_kernel(RingDwArgs p, int m
 #pragma unroll
       for (int d = 0; d < DW_DEPTH; ++d) {
         lds_read(op[(d + 1) & 1], (d + 1) % DW_LDS);
-        __builtin_amdgcn_sched_barrier(0);          // issue the reads first: left alone they sink below the MFMAs
         compute(st[d], op[d & 1]);
         fetch_next(st[d]);                          // refill DW_DEPTH chunks ahead
         publish(st[(d + 2) % DW_DEPTH], (d + 2) % DW_LDS);
+        dw_spread<DW_WJ + 2 * NG, 3, 5>(std::make_integer_sequence<int, NMAT * DW_WI * DW_WJ>{});
         lds_barrier();
         // keep the refill of stage d where it is: the scheduler would otherwise sink all refills of
         // a trip to its end and drain the whole queue once per trip
@@ -486,18 +508,19 @@ hipError_t ring_launch_dw_tiled(const RingDwArgs& a, int NC, hipStream_t st) {
   return hipSuccess;
 }
 
-// Which of the two kernels contracts: us of either with its reduction, from the chunks a workgroup walks.  Fitted to 60 shapes
-// (N = 120 to 2048, 2 to 16 channels, 1 to 131072 chunks): a chunk of three matrices takes 0.75 us here and 1.1 times that in
+// Which of the two kernels contracts: us of either with its reduction, from the chunks a workgroup walks.  Fitted to 30 shapes
+// (N = 120 to 2048, 2 to 7 channels, 40 to 15360 chunks): a chunk of three matrices takes 0.65 us here and 1.13 times that in
 // dw_chunk_waves (both sides near the matrix rate), a launch's start and end 4 and 5 us a round of 256 workgroups, partial sums are
-// written and read at 5 TB/s.  So long contractions of whole 128 x 128 blocks stay here (contraction and reduction, us, here and
-// there: N = 1024, 2 channels, 7680 chunks 1320 and 1470; N = 256, 15360 chunks 195 and 199; N = 512, 131072 chunks 5500 and
-// 5860) and the others go there: N = 256, 2 channels, 100 chunks 18 less; 3 channels (one launch instead of two) 20 less at 100
-// chunks, 92 at 15360; N = 640 (padded to 1024 here), 2 channels, 7680 chunks 690 less.
+// written and read at 5 TB/s.  So long contractions of whole 128 x 128 blocks stay here and the others go there; us of contraction and
+// reduction, here and there: N = 1024, 2 channels, 3840 chunks 616 and 669; N = 256, 15360 chunks 203 and 224; N = 2048, 160 chunks
+// 178 and 194; N = 256, 945 chunks 29 and 21; N = 360 (padded to 512 here), 1890 chunks 87 and 60; N = 256, 3 channels (two launches
+// here), 15360 chunks 325 and 240.
 // Returns the K splits of dw_chunk_waves, 0: not that kernel.
-int ring_dw_short_nz(int N, int NC, int k, int nbt, int T, int tiled_nz) {
+int ring_dw_short_nz(int N, int NC, int k, int nbt, int T, int tiled_nz, int linear_tiles) {
   if (getenv("RINGATTR_DW_SEGMENT")) return 0;             // (asks for the kernel that is cut)
   RingDwArgs a = {};
   a.N = N;
+  a.linear_tiles = linear_tiles;
   const int NB = 4 * NC / 8, tiles = dw_tiles(a, 4 * NC), groups = (k + 4) / 4;
   const long nb = (long)((tiles + DW_WI - 1) / DW_WI) * ((tiles + DW_WJ - 1) / DW_WJ), nchunk = (long)nbt * ((T + 1) / 2);
   // as many as fill the chip, each with two chunks a wave at least
@@ -505,7 +528,7 @@ int ring_dw_short_nz(int N, int NC, int k, int nbt, int T, int tiled_nz) {
   if (nz > nchunk / 8) nz = nchunk / 8;
   if (nz > tiled_nz) nz = tiled_nz;
   if (nz < 1) nz = 1;
-  constexpr float CHUNK = 0.75f, BYTES = 5e6f, tiled_share[4] = {0.f, 0.6f, 0.8f, 1.f}, short_share[5] = {0.f, 0.6f, 0.85f, 1.1f, 1.28f};
+  constexpr float CHUNK = 0.65f, BYTES = 5e6f, tiled_share[4] = {0.f, 0.7f, 0.85f, 1.f}, short_share[5] = {0.f, 0.65f, 0.85f, 1.13f, 1.42f};
   auto chunks = [&](long parts) { return (float)((nchunk + parts - 1) / parts) * CHUNK; };
   const float tiled_rounds = (float)(((long)NB * NB * tiled_nz + 255) / 256), short_rounds = (float)((nb * nz + 255) / 256);
   float tiled = 8.f * tiled_nz * (1 + k) * (64.f * NC) * (64.f * NC) / BYTES, here = 8.f * nz * (1 + k) * (16.f * tiles) * (16.f * tiles) / BYTES;
@@ -520,7 +543,7 @@ int ring_dw_short_nz(int N, int NC, int k, int nbt, int T, int tiled_nz) {
 
 // Through dw_chunk_waves where that is the faster one; its K splits (no more than there were) go into a.nz.
 hipError_t ring_launch_dw_short(RingDwArgs& a, int NC, hipStream_t st) {
-  const int nz = ring_dw_short_nz(a.N, NC, a.k, a.nbt, a.T, a.nz);
+  const int nz = ring_dw_short_nz(a.N, NC, a.k, a.nbt, a.T, a.nz, a.linear_tiles);
   if (nz == 0) return ring_launch_dw_tiled(a, NC, st);
   a.nz = nz;
   const int NT = 4 * NC, tiles = dw_tiles(a, NT);

@@ -141,7 +141,7 @@ bool ring_dw_tiled_applicable(int NC, int k, long nchunk);      // nchunk: batch
 int ring_dw_tiled_nz(int NC, int k, long nchunk);
 hipError_t ring_launch_dw_tiled(const RingDwArgs& a, int NC, hipStream_t st);
 hipError_t ring_launch_dw_short(RingDwArgs& a, int NC, hipStream_t st);   // or the kernel for short contractions, with fewer splits (a.nz)
-int ring_dw_short_nz(int N, int NC, int k, int nbt, int T, int tiled_nz);   // that many; 0: not that kernel
+int ring_dw_short_nz(int N, int NC, int k, int nbt, int T, int tiled_nz, int linear_tiles);   // that many; 0: not that kernel
 
 // Fused decode + loss head over the state history (ring_loss.hip).  loss_total: null, or where loss_out[0] goes as well.
 size_t ring_loss_workspace_bytes(int T, int B);

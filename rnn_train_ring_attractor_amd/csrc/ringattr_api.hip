@@ -924,7 +924,9 @@ int ringattr_profile_enable(int on) {
 int ringattr_dw_segments(int N, int a_dim, int seq_len, int batch_size) {
   Geo g;
   if (make_geo(N, a_dim, seq_len, batch_size, g) != RINGATTR_OK) return -1;
-  if (!ring_dw_tiled_applicable(g.NC, g.k, (long)g.nbt * ((g.T + 1) / 2)) || ring_dw_short_nz(N, g.NC, g.k, g.nbt, seq_len, g.nz) > 0) return 1;
+  if (!ring_dw_tiled_applicable(g.NC, g.k, (long)g.nbt * ((g.T + 1) / 2)) ||
+      ring_dw_short_nz(N, g.NC, g.k, g.nbt, seq_len, g.nz, ring_uses_team(N, a_dim, seq_len, batch_size) ? 1 : 0) > 0)
+    return 1;
   return ring_dw_tiled_segments(g.nbt, seq_len, g.nz);
 }
 
