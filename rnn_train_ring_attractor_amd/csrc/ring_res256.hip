@@ -913,17 +913,13 @@ __global__ __launch_bounds__(256) void ring_bptt_res256_kernel(RingBpttArgs p) {
       if constexpr (GA) {
         // the other parity's buffer is being read by this step's flush; this one was read one step ago, before
         // the barrier above
-        // Four chains of additions at a time, without a branch between them: one by one, each with a branch around its store, they
-        // waited for themselves (with the loss fused in, N = 256, B = 4096, T = 240 660 -> 638 us).  Not all eight, and not among the
-        // products: the registers are full, and what is put away for them costs more (860 us).
 #pragma unroll
-        for (int ch = 0; ch < 2; ++ch) {
-          __builtin_amdgcn_sched_barrier(0);
-          f32x4 tot;
+        for (int ch = 0; ch < 2; ++ch)
 #pragma unroll
-          for (int e = 0; e < 4; ++e) tot[e] = row16_sum_dpp(ga[ch][e]);
-          if (n == 0) *reinterpret_cast<f32x4*>(&gabuf[((cur * 2 + ch) * 4 + w) * 16 + 4 * q]) = tot;
-        }
+          for (int e = 0; e < 4; ++e) {
+            const float tot = row16_sum_dpp(ga[ch][e]);
+            if (n == 0) gabuf[((cur * 2 + ch) * 4 + w) * 16 + 4 * q + e] = tot;
+          }
         bptt_stage_load_r<FULL>(p, t - DEPTH, bt, w, lane, S);
       }
       // the next iteration overwrites the other operand buffer and, every R_GCH steps, the other
