@@ -271,6 +271,7 @@ struct RingTeamArgs {
   int c16, mr, wk;       // the shape, for the single workgroups that take over
   int rows;              // non-zero: one wave sums the whole contraction, in the weight-resident order (ring_team_rows.hip);
                          // 2: the record rounded as the whole-tile kernel does (ActRecord)
+  int look;              // one tile a team: how long behind a step's products the next state is first looked for (team_look); -1: before them
 };
 struct RingTeamShape { int kpw, c16, mr, wk, lds_mats, grid; };
 struct RingTeamPlan {

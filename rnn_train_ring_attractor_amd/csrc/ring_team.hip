@@ -226,6 +226,7 @@ static hipError_t team_args(const RingTeamPlan& p, const float* Wo, const float*
   c.mr = p.shape.mr;
   c.wk = p.shape.wk;
   c.rows = 0;
+  c.look = p.nt == 1 && team_may_look_late(p.shape.mr, p.shape.wk, p.shape.lds_mats) ? (p.shape.kpw >= 3 ? 12 : 8) : -1;
   return ring_team_fill(ws, p.xchg_bytes, p.gather_bytes, st);
 }
 
@@ -264,6 +265,7 @@ hipError_t ring_team_rows(const RingFwdArgs& a, const float* Wo, const float* Wa
   hipError_t e = team_args(p, Wo, Wa, a.A, a.J0, a.J1, true, a.N, a.k, a.T, a.B, 16, ws, c, st);
   if (e != hipSuccess) return e;
   c.wk = 1;
+  c.look = a.B <= 4 ? 8 : 10;
   c.rows = a.N == 256 && a.B % 16 == 0 ? 2 : 1;
   e = ring_launch_team_rows(a, c, p.shape, st);
   if (e == hipSuccess) e = ring_launch_team_solo_fwd(a, c, st);
@@ -277,6 +279,7 @@ hipError_t ring_team_rows_bptt(const RingBpttArgs& a, const float* Wo, const flo
   hipError_t e = team_args(p, Wo, Wa, a.A, a.J0, a.J1, true, a.N, a.k, a.T, a.B, 16, ws, c, st);
   if (e != hipSuccess) return e;
   c.wk = c.rows = 1;
+  c.look = a.B <= 4 ? 8 : 10;
   e = ring_launch_team_rows_bptt(a, c, p.shape, st);
   if (e == hipSuccess) e = ring_launch_team_solo_bptt(a, c, st);
   return e == hipSuccess && a.grad_A ? ring_launch_team_rows_ga(c.ga_part, a.grad_A, a.T, a.B, st) : e;

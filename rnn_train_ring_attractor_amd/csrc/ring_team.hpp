@@ -523,9 +523,28 @@ __device__ __forceinline__ bool team_go(const char* lds, const LdsPlan& L) {
   return __builtin_amdgcn_readfirstlane(*reinterpret_cast<const int*>(lds + L.gathered)) != 0;
 }
 
+// When a wave first looks for the next state where a team has one tile.  The state is there some 900 cycles behind the barrier that
+// ends the products (sums, activation, a store on its way), a look takes some 450, and one that comes back too early holds up the
+// next by as much: looked for before the products, or at once behind them, a step waited up to a whole look too long, the same in every
+// step.  So the first look goes out `look` times 64 cycles behind the barrier.  us a call, looking before the products, at once behind
+// the barrier, and 4, 8, 10 and 12 times 64 cycles later:
+//   rows kernels, T = 100: forward N = 256, B = 1, gelu 91.5  81.9  91.0  83.6  83.9  86.1  relu (there) 82.7  84.2  78.9  81.3  86.9
+//     forward N = 256, B = 128, gelu 103.6  94.9  102.7  95.6  94.4  93.5        training 260  235  251  248  234  233
+//   forward N = 360, 3 channels, B = 100, T = 75 97.3  96.1  92.5  90.9  95.5  98.3        training 262  229  229  221  229  235
+//   forward N = 1024, 2 channels, B = 64, T = 60 140.0  141.8  139.6  133.6  130.0  127.2
+//   forward N = 512, 2 channels, B = 64, T = 100 129.8  127.2  130.8  120.9  120.3  125.2      training 313  297  306  287  288  297
+// With many matrices the compute waves are what is waited for, and they look before the products as with several tiles: forward
+// N = 512, 16 channels, B = 128, T = 40 108.6  108.1  109.7  111.5; N = 120, 12 channels, B = 30, T = 100 189  192  196  192.
+// (lds_mats: or TEAM_MORE.)  Kernels of their own: a second loop in the others', or a branch around their loads, costs those that look
+// early (forward N = 400, 9 channels, B = 200, T = 60 132 -> 137 us; training N = 1024, B = 512, T = 40 547 -> 840).
+__host__ __device__ constexpr bool team_may_look_late(int mr, int wk, int lds_mats) { return mr == 3 && wk == 8 && lds_mats <= 4; }
+__device__ __forceinline__ void team_look(int look) {
+  for (int i = 0; i < look; ++i) __builtin_amdgcn_s_sleep(1);
+}
+
 // The compute waves' loop: `steps` rounds over the team's my_nt tiles, operand number s of round s.
 // (TR: with the transposed matrices)
-template <bool TR, int KPW, int C16, int MR, int WK, int EX, bool GA>
+template <bool TR, int KPW, int C16, int MR, int WK, int EX, bool GA, bool LATE>
 __device__ __forceinline__ void team_compute_loop(const RingTeamArgs& c, const LdsPlan& L, char* lds,
                                                   __amdgpu_buffer_rsrc_t rsrc, int mem, int team, int my_nt, int steps, int w,
                                                   int lane) {
@@ -568,6 +587,12 @@ __device__ __forceinline__ void team_compute_loop(const RingTeamArgs& c, const L
       tail = *reinterpret_cast<const u32x4*>(gates + (it & 1) * c.k * 16 + (first < c.k * 16 ? first : (MR - 1) * 16));
     }
     int spins = 0;
+    if constexpr (LATE) {                                  // (one tile per team)
+      if (s > 0) {
+        team_look(c.look);
+        op.template issue<WK>(rsrc, tc, (unsigned)slot * slot_bytes + (unsigned)team * tile_bytes);
+      }
+    }
     // Wide rings: the operand is nearly always there when several tiles share a team, and with the polling loop out of the
     // way the path straight on is shorter: N = 700, B = 500 11.55 -> 11.1 us per step forward and backward, N = 1024,
     // B = 2048 51.2 -> 50.3.  Up to N = 512 it gains nothing (and N = 120, B = 64 in teams of eight loses 2 %).
@@ -594,7 +619,7 @@ __device__ __forceinline__ void team_compute_loop(const RingTeamArgs& c, const L
     __builtin_amdgcn_s_waitcnt(0x0F70);    // vmcnt(0), for the compiler's books: this operand has landed on every path
     const bool wrap = j + 1 == my_nt;
     const int jn = wrap ? 0 : j + 1, sn = !wrap ? slot : (slot + 1 == c.slots ? 0 : slot + 1);
-    nx.template issue<WK>(rsrc, tc, (unsigned)sn * slot_bytes + (unsigned)(team + c.nteams * jn) * tile_bytes);
+    if constexpr (!LATE) nx.template issue<WK>(rsrc, tc, (unsigned)sn * slot_bytes + (unsigned)(team + c.nteams * jn) * tile_bytes);
     f32x4 acc[C16];
     const bool padding = PADS && __ballot(((tail[0] | tail[1] | tail[2] | tail[3]) & 0x7FFFFFFFu) != 0) == 0;
     team_products<KPW, C16, MR, WK, EX, GA>(tc, op, c, wl, gate, gates + (it & 1) * c.k * 16, rows + (it & 1) * C16 * 64,

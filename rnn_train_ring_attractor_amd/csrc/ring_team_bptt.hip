@@ -3,12 +3,6 @@
 
 hipError_t ring_launch_team_bptt(const RingBpttArgs& a, const RingTeamArgs& c, const RingTeamShape& sh, hipStream_t st) {
   constexpr bool GA = false;
-#define RING_TEAM_RUN(KPW, C16, MR, WK, EX)                                                                           \
-  return ring_team_start(reinterpret_cast<const void*>(&ring_team_bptt_kernel<KPW, C16, MR, WK, EX, GA>), sh, c.G,         \
-                         lds_plan<C16, WK>(c.k, c.nt, sh.lds_mats, c.KC, parked_bytes(KPW, C16, MR, WK), true, GA).total, st,                         \
-                         [&](dim3 g, dim3 b, unsigned lds) {                                                          \
-                           RING_LAUNCH((ring_team_bptt_kernel<KPW, C16, MR, WK, EX, GA>), g, b, lds, st, a, c);       \
-                         })
 #define RING_TEAM_CASE(KPW, C16, MR, WK, FEW, MORE)                                                                   \
   if (sh.kpw == KPW && sh.c16 == C16 && sh.mr == MR && sh.wk == WK) {                                                 \
     if (sh.lds_mats == 0) RING_TEAM_RUN(KPW, C16, MR, WK, 0);                                                         \
@@ -20,6 +14,5 @@ hipError_t ring_launch_team_bptt(const RingBpttArgs& a, const RingTeamArgs& c, c
   }
   RING_TEAM_SHAPES(RING_TEAM_CASE)
 #undef RING_TEAM_CASE
-#undef RING_TEAM_RUN
   return hipErrorInvalidValue;
 }

@@ -6,7 +6,7 @@
 // BPTT, reverse time.  Operand number s is g of step T - 1 - s; the products of round s give the carry into step
 // T - 2 - s (the last round, which only grad_r_init needs, is left out when that is not asked for).
 // ------------------------------------------------------------------------------------------------
-template <int KPW, int C16, int MR, int WK, int EX, bool GA>
+template <int KPW, int C16, int MR, int WK, int EX, bool GA, bool LATE>
 __global__ __launch_bounds__(64 * (WK + AUX)) void ring_team_bptt_kernel(RingBpttArgs p, RingTeamArgs c) {
   extern __shared__ __attribute__((aligned(16))) char lds[];
   int team, mem;
@@ -19,7 +19,7 @@ __global__ __launch_bounds__(64 * (WK + AUX)) void ring_team_bptt_kernel(RingBpt
   const int steps = (p.grad_r_init || GA) ? T : T - 1;
 
   if (w < WK) {
-    team_compute_loop<true, KPW, C16, MR, WK, EX, GA>(c, L, lds, rsrc, mem, team, my_nt, steps, w, lane);
+    team_compute_loop<true, KPW, C16, MR, WK, EX, GA, LATE>(c, L, lds, rsrc, mem, team, my_nt, steps, w, lane);
     return;
   }
 
@@ -242,3 +242,16 @@ __global__ __launch_bounds__(64 * (WK + AUX)) void ring_team_bptt_kernel(RingBpt
   }
 }
 
+template <int KPW, int C16, int MR, int WK, int EX, bool GA, bool LATE>
+hipError_t team_bptt_start(const RingBpttArgs& a, const RingTeamArgs& c, const RingTeamShape& sh, hipStream_t st) {
+  auto kern = ring_team_bptt_kernel<KPW, C16, MR, WK, EX, GA, LATE>;
+  return ring_team_start(reinterpret_cast<const void*>(kern), sh, c.G,
+                         lds_plan<C16, WK>(c.k, c.nt, sh.lds_mats, c.KC, parked_bytes(KPW, C16, MR, WK), true, GA).total, st,
+                         [&](dim3 g, dim3 b, unsigned lds) { RING_LAUNCH(kern, g, b, lds, st, a, c); });
+}
+#define RING_TEAM_RUN(KPW, C16, MR, WK, EX)                                                                           \
+  do {                                                                                                                \
+    if constexpr (team_may_look_late(MR, WK, EX))                                                                     \
+      if (c.look >= 0) return team_bptt_start<KPW, C16, MR, WK, EX, GA, true>(a, c, sh, st);                          \
+    return team_bptt_start<KPW, C16, MR, WK, EX, GA, false>(a, c, sh, st);                                            \
+  } while (0)

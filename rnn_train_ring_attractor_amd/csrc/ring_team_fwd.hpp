@@ -5,7 +5,7 @@
 // ------------------------------------------------------------------------------------------------
 // Forward.  p.dfrag / p.rfrag may be null together (inference).
 // ------------------------------------------------------------------------------------------------
-template <int KPW, int C16, int MR, int WK, int EX, int ACT>
+template <int KPW, int C16, int MR, int WK, int EX, int ACT, bool LATE>
 __global__ __launch_bounds__(64 * (WK + AUX)) void ring_team_fwd_kernel(RingFwdArgs p, RingTeamArgs c) {
   extern __shared__ __attribute__((aligned(16))) char lds[];
   int team, mem;
@@ -17,7 +17,7 @@ __global__ __launch_bounds__(64 * (WK + AUX)) void ring_team_fwd_kernel(RingFwdA
   const int T = p.T;
 
   if (w < WK) {
-    team_compute_loop<false, KPW, C16, MR, WK, EX, false>(c, L, lds, rsrc, mem, team, my_nt, T, w, lane);
+    team_compute_loop<false, KPW, C16, MR, WK, EX, false, LATE>(c, L, lds, rsrc, mem, team, my_nt, T, w, lane);
     return;
   }
 
@@ -111,12 +111,17 @@ __global__ __launch_bounds__(64 * (WK + AUX)) void ring_team_fwd_kernel(RingFwdA
   }
 }
 
+template <int KPW, int C16, int MR, int WK, int EX, int ACT, bool LATE>
+hipError_t team_fwd_start(const RingFwdArgs& a, const RingTeamArgs& c, const RingTeamShape& sh, hipStream_t st) {
+  auto kern = ring_team_fwd_kernel<KPW, C16, MR, WK, EX, ACT, LATE>;
+  return ring_team_start(reinterpret_cast<const void*>(kern), sh, c.G,
+                         lds_plan<C16, WK>(c.k, c.nt, sh.lds_mats, c.KC, parked_bytes(KPW, C16, MR, WK), false, false).total, st,
+                         [&](dim3 g, dim3 b, unsigned lds) { RING_LAUNCH(kern, g, b, lds, st, a, c); });
+}
 #define RING_TEAM_ACT(KPW, C16, MR, WK, EX, ACT)                                                                    \
-  return ring_team_start(reinterpret_cast<const void*>(&ring_team_fwd_kernel<KPW, C16, MR, WK, EX, ACT>), sh, c.G,       \
-                         lds_plan<C16, WK>(c.k, c.nt, sh.lds_mats, c.KC, parked_bytes(KPW, C16, MR, WK), false, false).total, st,               \
-                         [&](dim3 g, dim3 b, unsigned lds) {                                                    \
-                           RING_LAUNCH((ring_team_fwd_kernel<KPW, C16, MR, WK, EX, ACT>), g, b, lds, st, a, c);     \
-                         })
+  if constexpr (team_may_look_late(MR, WK, EX))                                                                     \
+    if (c.look >= 0) return team_fwd_start<KPW, C16, MR, WK, EX, ACT, true>(a, c, sh, st);                          \
+  return team_fwd_start<KPW, C16, MR, WK, EX, ACT, false>(a, c, sh, st)
 #define RING_TEAM_ACTS(KPW, C16, MR, WK, EX)                                  \
   switch (a.act) {                                                            \
     case ACT_RELU: RING_TEAM_ACT(KPW, C16, MR, WK, EX, ACT_RELU);             \

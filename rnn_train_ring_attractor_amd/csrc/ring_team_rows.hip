@@ -7,7 +7,7 @@
 // whole contraction in the resident kernel's order (forward: its K chunks first the even and then the odd ones; BPTT: one
 // after the other, the ungated sum starting from (1 - alpha) G), every matrix in an accumulator of its own, the gates
 // afterwards.  One batch tile per team, so up to 32 tiles.
-// us per call, T = 100, weight-resident kernels -> here.  With a record: N = 256, B = 128, gelu: forward 143 -> 117, BPTT
+// us per call, T = 100, weight-resident kernels -> here, with two column tiles a member and before team_look.  With a record: N = 256, B = 128, gelu: forward 143 -> 117, BPTT
 // 138 -> 130; N = 200, B = 64: 156 -> 110 and 245 -> 120; N = 256, B = 128, relu, with the loss's gradient and dL/dA:
 // 165 -> 114 (its row sums by a pass of their own included) and 222 -> 149.  Without: N = 256, B = 1: 142 -> 99.
 // What bounds it is the hand-over's latency and the chain of 24 products (some 400 cycles).
@@ -15,9 +15,18 @@
 
 namespace {
 
-constexpr int ROWS_TILES = 2, ROWS_CHUNKS = 8, ROWS_MATS = 3, ROWS_SLOTS = 8;
-// (the plan has room for one column tile's dL/dA shares, behind everything else)
-constexpr unsigned ROWS_GA_MORE = 2 * 2 * (ROWS_TILES - 1) * 16 * sizeof(float);
+constexpr int ROWS_CHUNKS = 8, ROWS_MATS = 3, ROWS_SLOTS = 8;
+// Two column tiles a member and a compute wave for the 24 products of each, or one column tile and a compute wave for the eight of
+// each matrix (the gates then follow in the auxiliary waves, in the same order): the chain a step waits for is 250 cycles shorter, but
+// takes twice the compute units and half as much more of the operand into each.  So one where sixteen members find room for every batch
+// tile (B <= 256).  us a call, T = 100, two and one, before team_look: forward N = 256, B = 16, relu 96.3 and 86.6, tanh 99.2 and 94.1,
+// B = 1, gelu 93.2 and 90.9, B = 256, gelu 105.2 and 103.8; training N = 200, B = 64, tanh 245 and 232.
+template <int TILES>
+struct RowsSplit {
+  static constexpr int SHARES = TILES == 1 ? ROWS_MATS : 1, WAVES = TILES * SHARES;     // shares of a column tile, compute waves
+  // (the plan has room for the dL/dA shares of one column tile a share, behind everything else)
+  static constexpr unsigned GA_MORE = 2 * 2 * (TILES - 1) * 16 * sizeof(float);
+};
 
 struct RowsOperand {
   u32x4 x[ROWS_CHUNKS];
@@ -36,15 +45,17 @@ struct RowsOperand {
 };
 
 // The weight fragments of one column tile, K chunk number i in the direction's order.
-template <bool TR>
-__device__ __forceinline__ void rows_weights(const RingTeamArgs& c, int out, int q, bf16x8 (&wt)[ROWS_MATS][ROWS_CHUNKS]) {
+// (MATS matrices from `first` on)
+template <bool TR, int MATS>
+__device__ __forceinline__ void rows_weights(const RingTeamArgs& c, int first, int out, int q, bf16x8 (&wt)[MATS][ROWS_CHUNKS]) {
   auto load = [&](auto how) {
     constexpr int HOW = decltype(how)::value, BATCH = HOW == WEIGHT_ROWS4 ? 8 : 4;
 #pragma unroll
-    for (int m = 0; m < ROWS_MATS; ++m)
+    for (int mm = 0; mm < MATS; ++mm)
 #pragma unroll
       for (int i0 = 0; i0 < ROWS_CHUNKS; i0 += BATCH) {
         WeightLoad l[BATCH];
+        const int m = first + mm;
         const float* W = m == 0 ? c.Wo : c.Wa + (size_t)(m - 1) * c.N * c.N;
 #pragma unroll
         for (int i = 0; i < BATCH; ++i) weight_load<HOW>(l[i], W, c.N, out, 32 * (TR ? i0 + i : rows_chunk(i0 + i)) + 8 * q);
@@ -53,7 +64,7 @@ __device__ __forceinline__ void rows_weights(const RingTeamArgs& c, int out, int
         for (int i = 0; i < BATCH; ++i) {
           bf16x8 f = weight_fragment(l[i], c.N, out, 32 * (TR ? i0 + i : rows_chunk(i0 + i)) + 8 * q, m == 0 ? c.scale0 : 1.f, m == 0 ? c.shift0 : 0.f);
           asm volatile("" : "+v"(f));              // (here, not at its first use: twice the registers until then)
-          wt[m][i0 + i] = f;
+          wt[mm][i0 + i] = f;
         }
         __builtin_amdgcn_sched_barrier(0);
       }
@@ -93,11 +104,12 @@ __device__ __forceinline__ void rows_wait(RowsOperand& op, const RingTeamArgs& c
 struct RowsRecord {
   unsigned d_off, p_off;
   bool row_ok;
-  __device__ __forceinline__ RowsRecord(const TeamAux<ROWS_TILES>& aux, int rows) {
+  template <int TILES>
+  __device__ __forceinline__ RowsRecord(const TeamAux<TILES>& aux, int rows) {
     const int lane = aux.lane, j = aux.j0 + (lane & 1), rq = aux.map.b >> 2, w = j >> 6, n = (j & 63) >> 2, cc = j & 3;
-    d_off = (lane & 2) ? NOWHERE : (unsigned)((w * 64 + rq * 16 + n) * 32 + cc * 8);
-    p_off = (unsigned)(((w * 4 + cc) * 64 + rq * 16 + n) * 16 + (lane & 2) * 4);
-    row_ok = aux.map.b < rows;
+    d_off = (lane & 2) || !aux.map.active ? NOWHERE : (unsigned)((w * 64 + rq * 16 + n) * 32 + cc * 8);
+    p_off = aux.map.active ? (unsigned)(((w * 4 + cc) * 64 + rq * 16 + n) * 16 + (lane & 2) * 4) : NOWHERE;
+    row_ok = aux.map.active && aux.map.b < rows;
   }
   __device__ __forceinline__ void dact_store(_Float16* base, int t, int nbt, int bt, int lane, unsigned d) const {
     const u32x2 x = quad_rows2(d, lane);
@@ -110,14 +122,33 @@ struct RowsRecord {
   }
 };
 
-template <int ACT, bool SAVE>
+// An auxiliary thread's two sums: of the one share, or of the matrices' with the gates g1 and g2 of its row.
+template <int TILES>
+__device__ __forceinline__ void rows_sums(const TeamAux<TILES>& aux, const float* share, const float* gates, int buf, float (&x)[2]) {
+  if constexpr (TILES == 1) {
+    using AM = AuxMap<1>;
+    const float* src = share + (size_t)buf * ROWS_MATS * AM::SHARE + aux.map.q * AM::QS + aux.map.b * 4 + 2 * aux.map.p;
+    f32x2 P[ROWS_MATS];
+#pragma unroll
+    for (int m = 0; m < ROWS_MATS; ++m) P[m] = *reinterpret_cast<const f32x2*>(src + m * AM::SHARE);
+    const float g1 = gates[aux.map.b], g2 = gates[16 + aux.map.b];
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int i = 0; i < 2; ++i) x[i] = fmaf(g2, P[2][i], fmaf(g1, P[1][i], P[0][i]));
+  } else {
+    aux.template sum_shares<1>(share, buf, x);
+  }
+}
+
+template <int ACT, bool SAVE, int TILES>
 __device__ __forceinline__ void rows_forward(const RingFwdArgs& p, const RingTeamArgs& c, char* lds) {
-  using TA = TeamAux<ROWS_TILES>;
+  using TA = TeamAux<TILES>;
+  using RS = RowsSplit<TILES>;
   using AM = typename TA::AM;
   constexpr int NPT = TA::NPT;
   int team, mem;
   if (!team_coords(c, team, mem)) return;
-  const LdsPlan L = lds_plan<ROWS_TILES, 1>(c.k, 1, 0, c.KC, 0, false, false);
+  const LdsPlan L = lds_plan<TILES, RS::SHARES>(c.k, 1, 0, c.KC, 0, false, false);
   const int tid = threadIdx.x, w = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
   const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(c.xchg, 0, (int)c.xchg_bytes, 0x00020000);
   const unsigned tile_bytes = (unsigned)c.KC * CHUNK_BYTES, slot_bytes = tile_bytes * (unsigned)c.nbt;
@@ -126,12 +157,13 @@ __device__ __forceinline__ void rows_forward(const RingFwdArgs& p, const RingTea
   float* const gl = reinterpret_cast<float*>(lds + L.gates);
   const int T = p.T, rows = p.B - 16 * team;
 
-  if (w < ROWS_TILES) {
+  if (w < RS::WAVES) {
     const int q = lane >> 4, b = lane & 15;
     unsigned at[ROWS_CHUNKS];
     rows_places<false>(c, lane, rows, at);
-    bf16x8 wt[ROWS_MATS][ROWS_CHUNKS];
-    rows_weights<false>(c, 16 * (mem * ROWS_TILES + w) + b, q, wt);
+    constexpr int MATS = ROWS_MATS / RS::SHARES;
+    bf16x8 wt[MATS][ROWS_CHUNKS];
+    rows_weights<false>(c, TILES == 1 ? w : 0, 16 * (mem * TILES + (TILES == 1 ? 0 : w)) + b, q, wt);
     lds_barrier();                                        // the first gates are in LDS
     if (!team_go(lds, L)) return;
     float* const dst = share + w * AM::SHARE + q * AM::QS + b * 4;
@@ -144,27 +176,33 @@ __device__ __forceinline__ void rows_forward(const RingFwdArgs& p, const RingTea
       const float* g = gl + (t & 1) * c.k * 16 + b;
       const float g1 = g[0], g2 = g[16];
       rows_wait(op, c, rsrc, at, (unsigned)slot * slot_bytes + tile_at, dead, lane);
-      f32x4 P0 = {0.f, 0.f, 0.f, 0.f}, P1 = P0, P2 = P0;
+      f32x4 P0 = {0.f, 0.f, 0.f, 0.f}, P1 = P0, P2 = P0, v;
 #pragma unroll
       for (int i = 0; i < ROWS_CHUNKS; ++i) {
         const bf16x8 x = __builtin_bit_cast(bf16x8, op.x[i]);
-        P1 = mfma16(wt[1][i], x, P1);
-        P2 = mfma16(wt[2][i], x, P2);
+        if constexpr (TILES == 2) {
+          P1 = mfma16(wt[1][i], x, P1);
+          P2 = mfma16(wt[2][i], x, P2);
+        }
         P0 = mfma16(wt[0][i], x, P0);
       }
-      f32x4 v;
+      if constexpr (TILES == 2) {
 #pragma unroll
-      for (int i = 0; i < 4; ++i) v[i] = fmaf(g2, P2[i], fmaf(g1, P1[i], P0[i]));
-      *reinterpret_cast<f32x4*>(dst + (t & 1) * (ROWS_TILES * AM::SHARE)) = v;
+        for (int i = 0; i < 4; ++i) v[i] = fmaf(g2, P2[i], fmaf(g1, P1[i], P0[i]));
+      } else {
+        v = P0;
+      }
+      *reinterpret_cast<f32x4*>(dst + (t & 1) * (RS::WAVES * AM::SHARE)) = v;
       slot = slot + 1 == ROWS_SLOTS ? 0 : slot + 1;
-      op.issue(rsrc, at, (unsigned)slot * slot_bytes + tile_at);      // (the first look at the next state)
       lds_barrier();
+      team_look(c.look);
+      op.issue(rsrc, at, (unsigned)slot * slot_bytes + tile_at);      // (the first look at the next state)
     }
     return;
   }
 
   __builtin_amdgcn_s_setprio(3);
-  TA aux(c, mem, tid - 64 * ROWS_TILES);
+  TA aux(c, mem, tid - 64 * RS::WAVES);
   team_arrive(c, team, aux.at);
   const RowsRecord rec(aux, rows);
   const int N = p.N, B = p.B;
@@ -191,7 +229,7 @@ __device__ __forceinline__ void rows_forward(const RingFwdArgs& p, const RingTea
     tg.put(gl + ((t + 1) & 1) * c.k * 16, g);               // the next step's gates, fetched two steps ago
     lds_barrier();                                          // the step's products are complete
     float x[NPT], rn[NPT], aF[NPT];
-    aux.template sum_shares<1>(share, t & 1, x);
+    rows_sums<TILES>(aux, share, gl + (t & 1) * c.k * 16, t & 1, x);
     ActRecord<ACT> rd[NPT];
 #pragma unroll
     for (int i = 0; i < NPT; ++i) aF[i] = rd[i].apply(x[i], asc);
@@ -222,17 +260,17 @@ __device__ __forceinline__ void rows_forward(const RingFwdArgs& p, const RingTea
 
 }  // namespace
 
-template <int ACT>
-__global__ __launch_bounds__(64 * (ROWS_TILES + AUX)) void ring_team_rows_kernel(RingFwdArgs p, RingTeamArgs c) {
+template <int ACT, int TILES>
+__global__ __launch_bounds__(64 * (RowsSplit<TILES>::WAVES + AUX)) __attribute__((amdgpu_waves_per_eu(2, 2))) void ring_team_rows_kernel(RingFwdArgs p, RingTeamArgs c) {
   extern __shared__ __attribute__((aligned(16))) char lds[];
-  rows_forward<ACT, false>(p, c, lds);
+  rows_forward<ACT, false, TILES>(p, c, lds);
 }
 
 // With the weight-resident kernels' record.
-template <int ACT>
-__global__ __launch_bounds__(64 * (ROWS_TILES + AUX)) void ring_team_res256_fwd_kernel(RingFwdArgs p, RingTeamArgs c) {
+template <int ACT, int TILES>
+__global__ __launch_bounds__(64 * (RowsSplit<TILES>::WAVES + AUX)) __attribute__((amdgpu_waves_per_eu(2, 2))) void ring_team_res256_fwd_kernel(RingFwdArgs p, RingTeamArgs c) {
   extern __shared__ __attribute__((aligned(16))) char lds[];
-  rows_forward<ACT, true>(p, c, lds);
+  rows_forward<ACT, true, TILES>(p, c, lds);
 }
 
 // ------------------------------------------------------------------------------------------------
@@ -240,15 +278,16 @@ __global__ __launch_bounds__(64 * (ROWS_TILES + AUX)) void ring_team_res256_fwd_
 // sum starts from (1 - alpha) G: the auxiliary waves leave it in LDS before they publish g, so a wave that has seen all of g
 // finds it there.
 // ------------------------------------------------------------------------------------------------
-template <bool GA>
-__global__ __launch_bounds__(64 * (ROWS_TILES + AUX)) void ring_team_res256_bptt_kernel(RingBpttArgs p, RingTeamArgs c) {
+template <bool GA, int TILES>
+__global__ __launch_bounds__(64 * (RowsSplit<TILES>::WAVES + AUX)) __attribute__((amdgpu_waves_per_eu(2, 2))) void ring_team_res256_bptt_kernel(RingBpttArgs p, RingTeamArgs c) {
   extern __shared__ __attribute__((aligned(16))) char lds[];
-  using TA = TeamAux<ROWS_TILES>;
+  using TA = TeamAux<TILES>;
+  using RS = RowsSplit<TILES>;
   using AM = typename TA::AM;
   constexpr int NPT = TA::NPT;
   int team, mem;
   if (!team_coords(c, team, mem)) return;
-  const LdsPlan L = lds_plan<ROWS_TILES, 1>(c.k, 1, 0, c.KC, 0, true, GA);
+  const LdsPlan L = lds_plan<TILES, RS::SHARES>(c.k, 1, 0, c.KC, 0, true, GA);
   const int tid = threadIdx.x, w = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
   const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(c.xchg, 0, (int)c.xchg_bytes, 0x00020000);
   const unsigned tile_bytes = (unsigned)c.KC * CHUNK_BYTES, slot_bytes = tile_bytes * (unsigned)c.nbt;
@@ -261,12 +300,14 @@ __global__ __launch_bounds__(64 * (ROWS_TILES + AUX)) void ring_team_res256_bptt
   const int T = p.T, rows = p.B - 16 * team;
   const int steps = (p.grad_r_init || GA) ? T : T - 1;
 
-  if (w < ROWS_TILES) {
+  if (w < RS::WAVES) {
     const int q = lane >> 4, b = lane & 15;
     unsigned at[ROWS_CHUNKS];
     rows_places<true>(c, lane, rows, at);
-    bf16x8 wt[ROWS_MATS][ROWS_CHUNKS];
-    rows_weights<true>(c, 16 * (mem * ROWS_TILES + w) + b, q, wt);
+    constexpr int MATS = ROWS_MATS / RS::SHARES;
+    const int tile = TILES == 1 ? 0 : w;
+    bf16x8 wt[MATS][ROWS_CHUNKS];
+    rows_weights<true>(c, TILES == 1 ? w : 0, 16 * (mem * TILES + tile) + b, q, wt);
     lds_barrier();                                        // the first gates (and r_prev) are in LDS
     if (!team_go(lds, L)) return;
     float* const dst = share + w * AM::SHARE + q * AM::QS + b * 4;
@@ -280,45 +321,53 @@ __global__ __launch_bounds__(64 * (ROWS_TILES + AUX)) void ring_team_res256_bptt
       const float g1 = g[0], g2 = g[16];
       rows_wait(op, c, rsrc, at, (unsigned)slot * slot_bytes + tile_at, dead, lane);
       asm volatile("" ::: "memory");                       // (what follows is read behind the wait)
-      f32x4 P0 = *reinterpret_cast<const f32x4*>(keep + (w * 64 + lane) * 4);
-      f32x4 P1 = {0.f, 0.f, 0.f, 0.f}, P2 = P1;
+      f32x4 P0 = *reinterpret_cast<const f32x4*>(keep + (tile * 64 + lane) * 4);
+      f32x4 P1 = {0.f, 0.f, 0.f, 0.f}, P2 = P1, v;
+      if (TILES == 1 && w > 0) P0 = P1;                    // (this wave's matrix is a gated one)
+      if constexpr (TILES == 2) {
 #pragma unroll
-      for (int i = 0; i < ROWS_CHUNKS; ++i) {
-        const bf16x8 x = __builtin_bit_cast(bf16x8, op.x[i]);
-        P1 = mfma16(wt[1][i], x, P1);
-        P2 = mfma16(wt[2][i], x, P2);
+        for (int i = 0; i < ROWS_CHUNKS; ++i) {
+          const bf16x8 x = __builtin_bit_cast(bf16x8, op.x[i]);
+          P1 = mfma16(wt[1][i], x, P1);
+          P2 = mfma16(wt[2][i], x, P2);
+        }
       }
 #pragma unroll
       for (int i = 0; i < ROWS_CHUNKS; ++i) P0 = mfma16(wt[0][i], __builtin_bit_cast(bf16x8, op.x[i]), P0);
-      slot = slot + 1 == ROWS_SLOTS ? 0 : slot + 1;
-      op.issue(rsrc, at, (unsigned)slot * slot_bytes + tile_at);      // (the first look at the next one)
-      f32x4 v;
+      if constexpr (TILES == 2) {
 #pragma unroll
-      for (int i = 0; i < 4; ++i) v[i] = fmaf(g2, P2[i], fmaf(g1, P1[i], P0[i]));
-      *reinterpret_cast<f32x4*>(dst + (s & 1) * (ROWS_TILES * AM::SHARE)) = v;
+        for (int i = 0; i < 4; ++i) v[i] = fmaf(g2, P2[i], fmaf(g1, P1[i], P0[i]));
+      } else {
+        v = P0;
+      }
+      *reinterpret_cast<f32x4*>(dst + (s & 1) * (RS::WAVES * AM::SHARE)) = v;
       if constexpr (GA) {
-        const f32x4 rp = *reinterpret_cast<const f32x4*>(prev + ((s & 1) * ROWS_TILES * 64 + w * 64 + lane) * 4);
-        float d1 = 0.f, d2 = 0.f;
+        const f32x4 rp = *reinterpret_cast<const f32x4*>(prev + ((s & 1) * TILES * 64 + tile * 64 + lane) * 4);
+        float* const gp = ga + ((s & 1) * 2 * TILES + tile) * 16 + b;
+        auto dot = [&](const f32x4& P, int ch) {
+          float d = 0.f;
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          d1 = fmaf(P1[i], rp[i], d1);
-          d2 = fmaf(P2[i], rp[i], d2);
-        }
-        d1 = sum_bits45(d1);
-        d2 = sum_bits45(d2);
-        float* const gp = ga + ((s & 1) * 2 * ROWS_TILES + w) * 16 + b;
-        if (lane < 16) {
-          gp[0] = d1;
-          gp[ROWS_TILES * 16] = d2;
+          for (int i = 0; i < 4; ++i) d = fmaf(P[i], rp[i], d);
+          d = sum_bits45(d);
+          if (lane < 16) gp[ch * TILES * 16] = d;
+        };
+        if constexpr (TILES == 2) {
+          dot(P1, 0);
+          dot(P2, 1);
+        } else if (w > 0) {
+          dot(P0, w - 1);
         }
       }
       lds_barrier();
+      slot = slot + 1 == ROWS_SLOTS ? 0 : slot + 1;
+      team_look(c.look);
+      op.issue(rsrc, at, (unsigned)slot * slot_bytes + tile_at);      // (the first look at the next one)
     }
     return;
   }
 
   __builtin_amdgcn_s_setprio(3);
-  TA aux(c, mem, tid - 64 * ROWS_TILES);
+  TA aux(c, mem, tid - 64 * RS::WAVES);
   team_arrive(c, team, aux.at);
   const RowsRecord rec(aux, rows);
   const int N = p.N, B = p.B, nbt = p.nbt;
@@ -366,7 +415,7 @@ __global__ __launch_bounds__(64 * (ROWS_TILES + AUX)) void ring_team_res256_bptt
       float v[NPT] = {in.rp[0], in.rp[1]};
       aux.align(N, v);
 #pragma unroll
-      for (int i = 0; i < NPT; ++i) prev[buf * ROWS_TILES * 256 + at4 + i] = rec.row_ok && j + i < N ? (float)(__bf16)v[i] : 0.f;
+      for (int i = 0; i < NPT; ++i) if (aux.map.active) prev[buf * TILES * 256 + at4 + i] = rec.row_ok && j + i < N ? (float)(__bf16)v[i] : 0.f;
     }
   };
   const bool ok[NPT] = {rec.row_ok && j < N, rec.row_ok && j + 1 < N};
@@ -381,7 +430,7 @@ __global__ __launch_bounds__(64 * (ROWS_TILES + AUX)) void ring_team_res256_bptt
       const float r = gin[i], of_loss = fmaf(kc, cs[i], fmaf(ks, sn[i], r > 0.f ? beta : (r < 0.f ? -beta : 0.f)));
       const float all = (loss ? of_loss : r) + carry[i];
       const float G = ok[i] ? all : 0.f, g = (float)in.d[i] * G;
-      keep[at4 + i] = oma * G;
+      if (aux.map.active) keep[at4 + i] = oma * G;
       gg[i] = ok[i] ? g : 0.f;                    // the record carries alpha
     }
     const unsigned x = pack_bf16(gg[0], gg[1]);
@@ -391,11 +440,11 @@ __global__ __launch_bounds__(64 * (ROWS_TILES + AUX)) void ring_team_res256_bptt
   // dL/dA of round s: one partial per column tile
   auto flush = [&](int s) {
     if constexpr (GA) {
-      const int at = aux.at, tile = at >> 5 & 1, ch = at >> 4 & 1, row = at & 15, t = T - 1 - s;
-      const float v = ga[((s & 1) * 2 * ROWS_TILES + (ch * ROWS_TILES + tile)) * 16 + row];
-      const __amdgpu_buffer_rsrc_t r = team_buffer(c.ga_part + ((size_t)mem * ROWS_TILES * T + t) * 2 * B, ((size_t)T + 1) * 2 * B * 4);
+      const int at = aux.at, tile = TILES == 1 ? 0 : at >> 5 & 1, ch = at >> 4 & 1, row = at & 15, t = T - 1 - s;
+      const float v = ga[((s & 1) * 2 * TILES + (ch * TILES + tile)) * 16 + row];
+      const __amdgpu_buffer_rsrc_t r = team_buffer(c.ga_part + ((size_t)mem * TILES * T + t) * 2 * B, ((size_t)T + 1) * 2 * B * 4);
       __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, v), r,
-                                            (int)(at < 64 && row < rows ? (unsigned)((tile * T * 2 + ch) * B + 16 * team + row) * 4 : NOWHERE), 0, 0);
+                                            (int)(at < 32 * TILES && row < rows ? (unsigned)((tile * T * 2 + ch) * B + 16 * team + row) * 4 : NOWHERE), 0, 0);
     }
   };
 
@@ -423,7 +472,7 @@ __global__ __launch_bounds__(64 * (ROWS_TILES + AUX)) void ring_team_res256_bptt
     put_side((s + 1) & 1, in);                               // the gates (and r_prev) of the next round, which is this set's step's
     lds_barrier();                                          // the round's products are complete
     float carry[NPT];
-    aux.template sum_shares<1>(share, s & 1, carry);
+    rows_sums<TILES>(aux, share, gl + (s & 1) * c.k * 16, s & 1, carry);
 #pragma unroll
     for (int i = 0; i < NPT; ++i) carry[i] = ok[i] ? carry[i] : 0.f;
     const int t = T - 2 - s, tt = t < 0 ? 0 : t, next_slot = slot + 1 == ROWS_SLOTS ? 0 : slot + 1;
@@ -467,12 +516,13 @@ RingTeamPlan ring_team_rows_plan(int N, int k, int B, bool record) {
   RingTeamPlan p{};
   if (!ring_res256_applicable(N, k)) return p;
   p.KC = record ? ROWS_CHUNKS : (N + 31) / 32;
-  p.G = (2 * p.KC + ROWS_TILES - 1) / ROWS_TILES;
   p.nteams = (B + 15) / 16;
+  const int one = 2 * p.KC, tiles = p.nteams <= 8 * (32 / one) ? 1 : 2;
+  p.G = (one + tiles - 1) / tiles;
   p.nt = 1;
   p.slots = ROWS_SLOTS;
   p.ok = p.nteams <= 8 * (32 / p.G);                       // (8 XCDs of 32 compute units)
-  p.shape = RingTeamShape{ROWS_CHUNKS, ROWS_TILES, ROWS_MATS, ROWS_TILES, 0, 8 * p.G * ((p.nteams + 7) / 8)};
+  p.shape = RingTeamShape{ROWS_CHUNKS, tiles, ROWS_MATS, tiles == 1 ? RowsSplit<1>::WAVES : RowsSplit<2>::WAVES, 0, 8 * p.G * ((p.nteams + 7) / 8)};
   p.xchg_bytes = (size_t)ROWS_SLOTS * p.nteams * p.KC * CHUNK_BYTES;
   p.gather_bytes = (size_t)p.nteams * RING_TEAM_WORD * sizeof(unsigned long long);
   return p;
@@ -480,28 +530,36 @@ RingTeamPlan ring_team_rows_plan(int N, int k, int B, bool record) {
 
 size_t ring_team_rows_ga_bytes(int T, int B) { return (size_t)16 * T * 2 * B * sizeof(float); }
 
-hipError_t ring_launch_team_rows(const RingFwdArgs& a, const RingTeamArgs& c, const RingTeamShape& sh, hipStream_t st) {
-  const unsigned lds = lds_plan<ROWS_TILES, 1>(c.k, 1, 0, c.KC, 0, false, false).total;
-  auto go = [&](auto kern) {
-    return ring_team_start(reinterpret_cast<const void*>(kern), sh, c.G, lds, st,
-                           [&](dim3 g, dim3 b, unsigned bytes) { RING_LAUNCH(kern, g, b, bytes, st, a, c); });
-  };
+template <int TILES, typename Args, typename Kernel>
+static hipError_t rows_start(Kernel kern, const Args& a, const RingTeamArgs& c, const RingTeamShape& sh, bool bptt, bool ga, hipStream_t st) {
+  const unsigned lds = lds_plan<TILES, RowsSplit<TILES>::SHARES>(c.k, 1, 0, c.KC, 0, bptt, ga).total + (ga ? RowsSplit<TILES>::GA_MORE : 0);
+  return ring_team_start(reinterpret_cast<const void*>(kern), sh, c.G, lds, st,
+                         [&](dim3 g, dim3 b, unsigned bytes) { RING_LAUNCH(kern, g, b, bytes, st, a, c); });
+}
+
+template <int TILES>
+static hipError_t launch_rows(const RingFwdArgs& a, const RingTeamArgs& c, const RingTeamShape& sh, hipStream_t st) {
+  auto go = [&](auto kern) { return rows_start<TILES>(kern, a, c, sh, false, false, st); };
   switch (a.act) {
-    case ACT_RELU: return a.dfrag ? go(ring_team_res256_fwd_kernel<ACT_RELU>) : go(ring_team_rows_kernel<ACT_RELU>);
-    case ACT_GELU: return a.dfrag ? go(ring_team_res256_fwd_kernel<ACT_GELU>) : go(ring_team_rows_kernel<ACT_GELU>);
-    case ACT_TANH: return a.dfrag ? go(ring_team_res256_fwd_kernel<ACT_TANH>) : go(ring_team_rows_kernel<ACT_TANH>);
-    case ACT_SILU: return a.dfrag ? go(ring_team_res256_fwd_kernel<ACT_SILU>) : go(ring_team_rows_kernel<ACT_SILU>);
+    case ACT_RELU: return a.dfrag ? go(ring_team_res256_fwd_kernel<ACT_RELU, TILES>) : go(ring_team_rows_kernel<ACT_RELU, TILES>);
+    case ACT_GELU: return a.dfrag ? go(ring_team_res256_fwd_kernel<ACT_GELU, TILES>) : go(ring_team_rows_kernel<ACT_GELU, TILES>);
+    case ACT_TANH: return a.dfrag ? go(ring_team_res256_fwd_kernel<ACT_TANH, TILES>) : go(ring_team_rows_kernel<ACT_TANH, TILES>);
+    case ACT_SILU: return a.dfrag ? go(ring_team_res256_fwd_kernel<ACT_SILU, TILES>) : go(ring_team_rows_kernel<ACT_SILU, TILES>);
     default: return hipErrorInvalidValue;
   }
 }
 
+hipError_t ring_launch_team_rows(const RingFwdArgs& a, const RingTeamArgs& c, const RingTeamShape& sh, hipStream_t st) {
+  return sh.c16 == 1 ? launch_rows<1>(a, c, sh, st) : launch_rows<2>(a, c, sh, st);
+}
+
 hipError_t ring_launch_team_rows_bptt(const RingBpttArgs& a, const RingTeamArgs& c, const RingTeamShape& sh, hipStream_t st) {
-  const unsigned lds = lds_plan<ROWS_TILES, 1>(c.k, 1, 0, c.KC, 0, true, a.grad_A != nullptr).total + (a.grad_A ? ROWS_GA_MORE : 0);
-  auto go = [&](auto kern) {
-    return ring_team_start(reinterpret_cast<const void*>(kern), sh, c.G, lds, st,
-                           [&](dim3 g, dim3 b, unsigned bytes) { RING_LAUNCH(kern, g, b, bytes, st, a, c); });
-  };
-  return a.grad_A ? go(ring_team_res256_bptt_kernel<true>) : go(ring_team_res256_bptt_kernel<false>);
+  const bool ga = a.grad_A != nullptr;
+  if (sh.c16 == 1)
+    return ga ? rows_start<1>(ring_team_res256_bptt_kernel<true, 1>, a, c, sh, true, true, st)
+              : rows_start<1>(ring_team_res256_bptt_kernel<false, 1>, a, c, sh, true, false, st);
+  return ga ? rows_start<2>(ring_team_res256_bptt_kernel<true, 2>, a, c, sh, true, true, st)
+            : rows_start<2>(ring_team_res256_bptt_kernel<false, 2>, a, c, sh, true, false, st);
 }
 
 hipError_t ring_launch_team_rows_ga(const float* part, float* grad_A, int T, int B, hipStream_t st) {

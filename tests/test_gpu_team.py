@@ -574,3 +574,33 @@ def test_few_matrices_in_lds(B, k, N, gpu_device, teams, monkeypatch):
         assert all(torch.equal(got[x], want[x]) for x in want), [x for x in want if not torch.equal(got[x], want[x])]
     ref, _ = O.forward_dense(A[:9], p["Wa"], -1.0 / N, 0.6, p["Wo"], p["r0"][:9], 0.15, "gelu")
     assert O.max_rel_err(want["hist"][:, :9].cpu().numpy(), ref) <= TRAJ_TOL
+
+
+# Teams for the weight-resident widths: sixteen members of one column tile up to 256 rows, eight of two past that.
+@pytest.mark.parametrize("N,T,act", [(256, 9, "gelu"), (200, 8, "relu"), (131, 5, "silu")])
+def test_rows_on_either_side_of_the_line_between_one_and_two_column_tiles(N, T, act, gpu_device, monkeypatch):
+    from rnn_train_ring_attractor_amd import ring_rnn_cuda_func, _lib
+    p = make_problem(31, 257, T, 2, N)
+    t = lambda x: torch.as_tensor(x, dtype=torch.float32, device=gpu_device)
+    A, Wa, Wo, r0, G = (t(p[n]) for n in ("A", "Wa", "Wo", "r0", "G"))
+
+    def run(B, **env):
+        for name in ("RINGATTR_TEAM", "RINGATTR_TEAM_GATHER_US"):
+            monkeypatch.delenv(name, raising=False)
+        for name, value in env.items():
+            monkeypatch.setenv(name, value)
+        a, ra = A[:B].clone().requires_grad_(True), r0[:B].clone()
+        with torch.no_grad():
+            plain = ring_rnn_cuda_func(a.detach(), Wa, -1.0 / N, 0.5, Wo, ra, 0.15, act)
+        wo, wa = Wo.clone().requires_grad_(True), Wa.clone().requires_grad_(True)
+        h = ring_rnn_cuda_func(a, wa, -1.0 / N, 0.5, wo, ra, 0.15, act)
+        h.backward(G[:, :B].contiguous())
+        assert torch.equal(plain, h)
+        return h.detach(), a.grad, wo.grad, wa.grad, _lib.last_kernel_names()["bptt"]
+
+    for B in (1, 16, 256, 257):
+        teams = run(B)
+        assert teams[4].startswith("ring_team_res256_bptt")
+        for other in (run(B, RINGATTR_TEAM="0"), run(B, RINGATTR_TEAM_GATHER_US="-1")):      # one workgroup a tile; teams that give up
+            for got, want in zip(teams[:4], other[:4]):
+                assert torch.equal(got, want), (B, other[4])
