@@ -122,19 +122,27 @@ struct RowsRecord {
   }
 };
 
-// An auxiliary thread's two sums: of the one share, or of the matrices' with the gates g1 and g2 of its row.
+// The two gates of an auxiliary thread's row, where its matrices' sums come apart.  They are read before the barrier that ends the step's
+// products, as the compute waves with two tiles do: behind it the first auxiliary wave may already be putting the gates of two steps on
+// into the same buffer.
 template <int TILES>
-__device__ __forceinline__ void rows_sums(const TeamAux<TILES>& aux, const float* share, const float* gates, int buf, float (&x)[2]) {
+__device__ __forceinline__ f32x2 rows_gates(const TeamAux<TILES>& aux, const float* gates) {
+  if constexpr (TILES == 1) return f32x2{gates[aux.map.b], gates[16 + aux.map.b]};
+  return f32x2{0.f, 0.f};
+}
+
+// An auxiliary thread's two sums: of the one share, or of the matrices' with its row's gates.
+template <int TILES>
+__device__ __forceinline__ void rows_sums(const TeamAux<TILES>& aux, const float* share, f32x2 g, int buf, float (&x)[2]) {
   if constexpr (TILES == 1) {
     using AM = AuxMap<1>;
     const float* src = share + (size_t)buf * ROWS_MATS * AM::SHARE + aux.map.q * AM::QS + aux.map.b * 4 + 2 * aux.map.p;
     f32x2 P[ROWS_MATS];
 #pragma unroll
     for (int m = 0; m < ROWS_MATS; ++m) P[m] = *reinterpret_cast<const f32x2*>(src + m * AM::SHARE);
-    const float g1 = gates[aux.map.b], g2 = gates[16 + aux.map.b];
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int i = 0; i < 2; ++i) x[i] = fmaf(g2, P[2][i], fmaf(g1, P[1][i], P[0][i]));
+    for (int i = 0; i < 2; ++i) x[i] = fmaf(g[1], P[2][i], fmaf(g[0], P[1][i], P[0][i]));
   } else {
     aux.template sum_shares<1>(share, buf, x);
   }
@@ -173,8 +181,8 @@ __device__ __forceinline__ void rows_forward(const RingFwdArgs& p, const RingTea
     if (dead && lane == 0) *c.host_err = RING_CLUSTER_ERR_WAIT;
     op.issue(rsrc, at, tile_at);
     for (int t = 0; t < T; ++t) {
-      const float* g = gl + (t & 1) * c.k * 16 + b;
-      const float g1 = g[0], g2 = g[16];
+      const float* g = gl + (t & 1) * c.k * 16 + b;        // (two tiles; with one the auxiliary waves apply the gates)
+      const float g1 = TILES == 2 ? g[0] : 0.f, g2 = TILES == 2 ? g[16] : 0.f;
       rows_wait(op, c, rsrc, at, (unsigned)slot * slot_bytes + tile_at, dead, lane);
       f32x4 P0 = {0.f, 0.f, 0.f, 0.f}, P1 = P0, P2 = P0, v;
 #pragma unroll
@@ -226,10 +234,11 @@ __device__ __forceinline__ void rows_forward(const RingFwdArgs& p, const RingTea
 
   int slot = 0, t = 0;
   auto step = [&](bool even, float& g) {
+    const f32x2 row_gates = rows_gates<TILES>(aux, gl + (t & 1) * c.k * 16);
     tg.put(gl + ((t + 1) & 1) * c.k * 16, g);               // the next step's gates, fetched two steps ago
     lds_barrier();                                          // the step's products are complete
     float x[NPT], rn[NPT], aF[NPT];
-    rows_sums<TILES>(aux, share, gl + (t & 1) * c.k * 16, t & 1, x);
+    rows_sums<TILES>(aux, share, row_gates, t & 1, x);
     ActRecord<ACT> rd[NPT];
 #pragma unroll
     for (int i = 0; i < NPT; ++i) aF[i] = rd[i].apply(x[i], asc);
@@ -318,7 +327,7 @@ __global__ __launch_bounds__(64 * (RowsSplit<TILES>::WAVES + AUX)) __attribute__
     op.issue(rsrc, at, tile_at);
     for (int s = 0; s < steps; ++s) {
       const float* g = gl + (s & 1) * c.k * 16 + b;
-      const float g1 = g[0], g2 = g[16];
+      const float g1 = TILES == 2 ? g[0] : 0.f, g2 = TILES == 2 ? g[16] : 0.f;
       rows_wait(op, c, rsrc, at, (unsigned)slot * slot_bytes + tile_at, dead, lane);
       asm volatile("" ::: "memory");                       // (what follows is read behind the wait)
       f32x4 P0 = *reinterpret_cast<const f32x4*>(keep + (tile * 64 + lane) * 4);
@@ -469,10 +478,11 @@ __global__ __launch_bounds__(64 * (RowsSplit<TILES>::WAVES + AUX)) __attribute__
   const __amdgpu_buffer_rsrc_t rinit = team_buffer(p.grad_r_init + (size_t)16 * team * N, p.grad_r_init ? (size_t)(rows < 16 ? rows : 16) * N * 4 : 0);
   int slot = 0, s = 0;
   auto round = [&](In& in) {
+    const f32x2 row_gates = rows_gates<TILES>(aux, gl + (s & 1) * c.k * 16);
     put_side((s + 1) & 1, in);                               // the gates (and r_prev) of the next round, which is this set's step's
     lds_barrier();                                          // the round's products are complete
     float carry[NPT];
-    rows_sums<TILES>(aux, share, gl + (s & 1) * c.k * 16, s & 1, carry);
+    rows_sums<TILES>(aux, share, row_gates, s & 1, carry);
 #pragma unroll
     for (int i = 0; i < NPT; ++i) carry[i] = ok[i] ? carry[i] : 0.f;
     const int t = T - 2 - s, tt = t < 0 ? 0 : t, next_slot = slot + 1 == ROWS_SLOTS ? 0 : slot + 1;

@@ -274,3 +274,37 @@ def test_cluster_kernels_use_no_scratch(cluster_asm):
             m = re.search(r"ScratchSize \[bytes/lane\]: (\d+)", b)
             assert int(m.group(1)) == 0, f"{name} spills {m.group(1)} bytes per lane"
     assert seen == 10
+
+
+# ------------------------------------------------------------------------------------------------
+# Teams for the weight-resident widths with one column tile a member: the auxiliary waves apply the gates, which the first of them puts
+# into two buffers in turn with one barrier a step.  Behind the barrier of step t that wave may be as far as the gates of step t + 2,
+# which go where those of step t are: nobody may still have to read them there.
+# ------------------------------------------------------------------------------------------------
+def test_one_tile_teams_read_a_steps_gates_before_its_barrier(tmp_path):
+    out = tmp_path / "rows.s"
+    proc = subprocess.run([HIPCC, "--offload-arch=gfx950", "-O3", "-std=c++17", "-S", "--cuda-device-only", f"-I{ROOT}/include", f"-I{CSRC}",
+                           "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops", *PER_SOURCE_FLAGS.get("ring_team_rows.hip", []),
+                           os.path.join(CSRC, "ring_team_rows.hip"), "-o", str(out)], capture_output=True, text=True)
+    assert proc.returncode == 0, proc.stderr[-2000:]
+    asm = out.read_text()
+    names = re.findall(r"^(_Z21ring_team_rows_kernelILi\dELi1E\w*|_Z27ring_team_res256_fwd_kernelILi\dELi1E\w*|"
+                       r"_Z28ring_team_res256_bptt_kernelILb[01]ELi1E\w*):", asm, re.M)
+    assert len(names) == 10
+    for name in names:
+        ins = [t for _, t in _instructions(_function_body(asm, name))]
+        barriers = [i for i, t in enumerate(ins) if t.startswith("s_barrier")]
+        steps = 0
+        for before, at in zip(barriers, barriers[1:]):
+            behind = []                                # LDS reads between the barrier and what the step publishes
+            for t in ins[at + 1:]:
+                if t.startswith(("s_barrier", "buffer_store", "s_endpgm")):
+                    break
+                behind += [t] if t.startswith("ds_read") else []
+            # an auxiliary wave's step reads the shares of the three matrices, two neurons each: 64 bits
+            if sum(2 if "read2" in t else 1 for t in behind if "_b64" in t) != 3:
+                continue
+            steps += 1
+            assert all("_b64" in t for t in behind), f"{name}: {behind}"
+            assert any(t.startswith("ds_read2_b32") for t in ins[before + 1:at]), f"{name}: no gates read ahead of the barrier"
+        assert steps == 2, name                        # (two steps a trip, the gates' buffers in turn)
