@@ -183,6 +183,12 @@ __device__ __forceinline__ void dw_chunk_waves(const RingDwArgs& p, int m0, int 
 #pragma unroll
       for (int v = 0; v < NLD; ++v) (&gates[wv][buf][0][0][0])[64 * v + lane] = s.gate[v];
   };
+  // What a wave's lanes put into its LDS, other lanes of it read behind this.  (No instruction: a wave's LDS accesses are carried out in
+  // order; it is the compiler that must not move one past the other.)
+  auto handed_over = [] {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+  };
   auto compute = [&](const DwChunk<NG>& s, int buf) {
     f32x4 g8[NG > 0 ? NG : 1][2];
 #pragma unroll
@@ -207,6 +213,7 @@ __device__ __forceinline__ void dw_chunk_waves(const RingDwArgs& p, int m0, int 
     __builtin_amdgcn_sched_barrier(0);
   }
   publish(st[0], 0);
+  handed_over();
   int i = 0;
 #pragma unroll 1
   for (; i + DWS_DEPTH <= n; i += DWS_DEPTH)
@@ -216,6 +223,7 @@ __device__ __forceinline__ void dw_chunk_waves(const RingDwArgs& p, int m0, int 
       fetch(st[d]);
       publish(st[(d + 1) % DWS_DEPTH], (d + 1) % DWS_DEPTH);
       dw_spread<2 * NG, (NG > 0 ? NLD : 0), DW_WI + DW_WJ + NLD>(std::make_integer_sequence<int, NMAT * DW_WI * DW_WJ>{});
+      handed_over();
       __builtin_amdgcn_sched_barrier(0);
     }
 #pragma unroll
@@ -223,6 +231,7 @@ __device__ __forceinline__ void dw_chunk_waves(const RingDwArgs& p, int m0, int 
     if (i + d >= n) break;
     compute(st[d], d);
     publish(st[d + 1], d + 1);
+    handed_over();
   }
 
   // the waves' sums, in wave order; wave w writes out columns 2w and 2w + 1

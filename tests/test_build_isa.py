@@ -308,3 +308,27 @@ def test_one_tile_teams_read_a_steps_gates_before_its_barrier(tmp_path):
             assert all("_b64" in t for t in behind), f"{name}: {behind}"
             assert any(t.startswith("ds_read2_b32") for t in ins[before + 1:at]), f"{name}: no gates read ahead of the barrier"
         assert steps == 2, name                        # (two steps a trip, the gates' buffers in turn)
+
+
+def test_short_weight_gradients_hand_gates_from_lane_to_lane_behind_a_fence(tmp_path):
+    """dw_chunk_waves: a wave's lanes put a chunk's gates into the wave's own LDS and other lanes of it read them.  LDS carries a wave's
+    accesses out in order, so what is to be kept is the order of the instructions: a wave barrier (no instruction) between the two."""
+    out = tmp_path / "dw.s"
+    proc = subprocess.run([HIPCC, "--offload-arch=gfx950", "-O3", "-std=c++17", "-S", "--cuda-device-only", f"-I{ROOT}/include", f"-I{CSRC}",
+                           "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops", *PER_SOURCE_FLAGS.get("ring_dw.hip", []),
+                           os.path.join(CSRC, "ring_dw.hip"), "-o", str(out)], capture_output=True, text=True)
+    assert proc.returncode == 0, proc.stderr[-2000:]
+    asm = out.read_text()
+    names = re.findall(r"^(_Z21ring_dw_direct_kernelILi0E\w*):", asm, re.M)
+    assert len(names) == 8
+    for name in names:
+        body, written, writes = _function_body(asm, name), False, 0
+        for ln in body + body:                         # (the second pass is the loop's way back)
+            t = ln.strip()
+            if t.startswith(("ds_write_b32", "ds_write2")):
+                written, writes = True, writes + 1
+            elif "wave barrier" in t or t.startswith("s_barrier"):
+                written = False
+            elif t.startswith("ds_read"):
+                assert not written, f"{name}: {t}"
+        assert writes >= 2 * 4 or name.startswith("_Z21ring_dw_direct_kernelILi0ELi1ELb1E"), name      # (one matrix, ungated: no gates)
