@@ -517,13 +517,22 @@ hipError_t ring_launch_dw_tiled(const RingDwArgs& a, int NC, hipStream_t st) {
   return hipSuccess;
 }
 
-// Which of the two kernels contracts: us of either with its reduction, from the chunks a workgroup walks.  Fitted to 30 shapes
-// (N = 120 to 2048, 2 to 7 channels, 40 to 15360 chunks): a chunk of three matrices takes 0.65 us here and 1.13 times that in
-// dw_chunk_waves (both sides near the matrix rate), a launch's start and end 4 and 5 us a round of 256 workgroups, partial sums are
-// written and read at 5 TB/s.  So long contractions of whole 128 x 128 blocks stay here and the others go there; us of contraction and
-// reduction, here and there: N = 1024, 2 channels, 3840 chunks 616 and 669; N = 256, 15360 chunks 203 and 224; N = 2048, 160 chunks
-// 178 and 194; N = 256, 945 chunks 29 and 21; N = 360 (padded to 512 here), 1890 chunks 87 and 60; N = 256, 3 channels (two launches
-// here), 15360 chunks 325 and 240.
+// Which of the two kernels contracts: us of either with its reduction, from the chunks a workgroup walks.  A chunk of three matrices
+// takes 0.65 us here and 1.13 times that in dw_chunk_waves, where one of two takes hardly less: a wave loads ten fragments a chunk there
+// whatever their number.  A launch's start and end take 4 and 5 us a round of 256 workgroups, partial sums are written and read at 5 TB/s.
+// Held against 715 shapes, N = 70 to 2048, 1 to 16 channels, 5 to 65536 chunks: the kernel it takes is at most 13 % and 26 us slower
+// than the other where it is dw_chunk_waves (N = 200: one channel, 3840 chunks 51 against 45 us, five, 15360 chunks 359 against 340);
+// where it stays here some wide rings with many channels would gain from the other (N = 565, seven channels, 43095 chunks 20.8 against
+// 15.8 ms; N = 700, 16, 15360 chunks 15.9 against 13.8; most 0).  So long contractions of whole 128 x 128 blocks and those of one channel stay here; us, here and there:
+//   one channel: N = 512, 15360 chunks 444 and 629, 945 chunks 44 and 42; N = 1024, 3840 chunks 430 and 609; N = 360, 15360 chunks 440
+//     and 388
+//   two: N = 512, 65536 chunks 2480 and 2810; N = 1024, 3840 chunks 573 and 638; N = 256, 15360 chunks 181 and 214; N = 2048, 160 chunks
+//     178 and 194; N = 256, 945 chunks 34 and 25; N = 360 (padded to 512 here), 1890 chunks 87 and 60
+//   three (two launches here): N = 256, 15360 chunks 289 and 212
+// No launch of dw_chunk_waves is cut in time, however long: the waves of its workgroups drift apart as the others do, and it is ahead all
+// the same where it is taken.  us of contraction, cut here and there: N = 360, two channels, 131072 chunks 4810 and 3320, three, 65536
+// chunks 4280 and 2020; N = 640, two, 65536 chunks 10270 and 5570; N = 512, three, 131072 chunks 9300 and 7690; N = 200, three 2380 and
+// 1560; N = 120, six 2970 and 1210.
 // Returns the K splits of dw_chunk_waves, 0: not that kernel.
 int ring_dw_short_nz(int N, int NC, int k, int nbt, int T, int tiled_nz, int linear_tiles) {
   if (getenv("RINGATTR_DW_SEGMENT")) return 0;             // (asks for the kernel that is cut)
@@ -537,7 +546,7 @@ int ring_dw_short_nz(int N, int NC, int k, int nbt, int T, int tiled_nz, int lin
   if (nz > nchunk / 8) nz = nchunk / 8;
   if (nz > tiled_nz) nz = tiled_nz;
   if (nz < 1) nz = 1;
-  constexpr float CHUNK = 0.65f, BYTES = 5e6f, tiled_share[4] = {0.f, 0.7f, 0.85f, 1.f}, short_share[5] = {0.f, 0.65f, 0.85f, 1.13f, 1.42f};
+  constexpr float CHUNK = 0.65f, BYTES = 5e6f, tiled_share[4] = {0.f, 0.7f, 0.75f, 1.f}, short_share[5] = {0.f, 0.65f, 1.1f, 1.13f, 1.42f};
   auto chunks = [&](long parts) { return (float)((nchunk + parts - 1) / parts) * CHUNK; };
   const float tiled_rounds = (float)(((long)NB * NB * tiled_nz + 255) / 256), short_rounds = (float)((nb * nz + 255) / 256);
   float tiled = 8.f * tiled_nz * (1 + k) * (64.f * NC) * (64.f * NC) / BYTES, here = 8.f * nz * (1 + k) * (16.f * tiles) * (16.f * tiles) / BYTES;

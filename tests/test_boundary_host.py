@@ -207,3 +207,15 @@ def test_weight_gradient_segment_count(monkeypatch):
     monkeypatch.setenv("RINGATTR_DW_SEGMENT", "1")
     assert lib.ringattr_dw_segments(256, 2, 33, 256) == 5            # 64 splits x 1 chunk = 4 of the 17 time-step pairs per segment
     assert lib.ringattr_dw_segments(4096, 2, 8, 16) == -1
+
+
+def test_weight_gradients_of_one_channel_stay_with_the_blocks_that_are_cut(monkeypatch):
+    """Which contraction kernel a shape takes shows in its time segments: the one for short contractions is never cut.  Two matrices a
+    launch gain nothing there (half as long again at N = 512 and 1024) unless the ring's width is padded."""
+    from rnn_train_ring_attractor_amd import _lib
+    lib = _lib.load()
+    monkeypatch.delenv("RINGATTR_DW_SEGMENT", raising=False)
+    assert lib.ringattr_dw_segments(512, 1, 512, 8192) == 13
+    assert lib.ringattr_dw_segments(256, 1, 512, 8192) == 4
+    assert lib.ringattr_dw_segments(1024, 1, 120, 2048) == 3
+    assert lib.ringattr_dw_segments(512, 3, 512, 8192) == 1
