@@ -194,8 +194,14 @@ hipError_t ring_team_fill(void* ws, size_t xchg_bytes, size_t gather_bytes, hipS
   return hipGetLastError();
 }
 
+// RingTeamArgs::look (measured: team_look).
+static int first_look(const RingTeamPlan& p, bool bptt) {
+  if (p.nt != 1 || !team_may_look_late(p.shape.mr, p.shape.wk, p.shape.lds_mats)) return -1;
+  return p.shape.kpw < 3 ? 8 : bptt ? 10 : 12;
+}
+
 static hipError_t team_args(const RingTeamPlan& p, const float* Wo, const float* Wa, const float* A, float J0, float J1,
-                            bool folded, int N, int k, int T, int B, int cts, void* ws, RingTeamArgs& c,
+                            bool folded, int N, int k, int T, int B, int cts, int look, void* ws, RingTeamArgs& c,
                             hipStream_t st) {
   hipError_t e = ring_cluster_host_err(&c.host_err);
   if (e != hipSuccess) return e;
@@ -226,7 +232,7 @@ static hipError_t team_args(const RingTeamPlan& p, const float* Wo, const float*
   c.mr = p.shape.mr;
   c.wk = p.shape.wk;
   c.rows = 0;
-  c.look = p.nt == 1 && team_may_look_late(p.shape.mr, p.shape.wk, p.shape.lds_mats) ? (p.shape.kpw >= 3 ? 12 : 8) : -1;
+  c.look = look;
   return ring_team_fill(ws, p.xchg_bytes, p.gather_bytes, st);
 }
 
@@ -251,7 +257,7 @@ hipError_t ring_team_fwd(const RingFwdArgs& a, const float* Wo, const float* Wa,
   const RingTeamPlan p = ring_team_plan(a.N, a.k, a.T, a.B, false, false);
   if (!p.ok || !ws || (a.dfrag != nullptr) != (a.rfrag != nullptr)) return hipErrorInvalidValue;
   RingTeamArgs c;
-  hipError_t e = team_args(p, Wo, Wa, a.A, a.J0, a.J1, folded, a.N, a.k, a.T, a.B, cts, ws, c, st);
+  hipError_t e = team_args(p, Wo, Wa, a.A, a.J0, a.J1, folded, a.N, a.k, a.T, a.B, cts, first_look(p, false), ws, c, st);
   if (e != hipSuccess) return e;
   e = ring_launch_team_fwd(a, c, p.shape, st);
   return e == hipSuccess ? ring_launch_team_solo_fwd(a, c, st) : e;
@@ -262,10 +268,9 @@ hipError_t ring_team_rows(const RingFwdArgs& a, const float* Wo, const float* Wa
   const RingTeamPlan p = ring_team_rows_plan(a.N, a.k, a.B, record);
   if (!p.ok || !ws || !a.hist || record != (a.rfrag != nullptr)) return hipErrorInvalidValue;
   RingTeamArgs c;
-  hipError_t e = team_args(p, Wo, Wa, a.A, a.J0, a.J1, true, a.N, a.k, a.T, a.B, 16, ws, c, st);
+  hipError_t e = team_args(p, Wo, Wa, a.A, a.J0, a.J1, true, a.N, a.k, a.T, a.B, 16, a.B <= 8 ? 8 : 10, ws, c, st);
   if (e != hipSuccess) return e;
   c.wk = 1;
-  c.look = a.B <= 4 ? 8 : 10;
   c.rows = a.N == 256 && a.B % 16 == 0 ? 2 : 1;
   e = ring_launch_team_rows(a, c, p.shape, st);
   if (e == hipSuccess) e = ring_launch_team_solo_fwd(a, c, st);
@@ -276,10 +281,9 @@ hipError_t ring_team_rows_bptt(const RingBpttArgs& a, const float* Wo, const flo
   const RingTeamPlan p = ring_team_rows_plan(a.N, a.k, a.B, true);
   if (!p.ok || !ws) return hipErrorInvalidValue;
   RingTeamArgs c;
-  hipError_t e = team_args(p, Wo, Wa, a.A, a.J0, a.J1, true, a.N, a.k, a.T, a.B, 16, ws, c, st);
+  hipError_t e = team_args(p, Wo, Wa, a.A, a.J0, a.J1, true, a.N, a.k, a.T, a.B, 16, 8, ws, c, st);
   if (e != hipSuccess) return e;
   c.wk = c.rows = 1;
-  c.look = a.B <= 4 ? 8 : 10;
   e = ring_launch_team_rows_bptt(a, c, p.shape, st);
   if (e == hipSuccess) e = ring_launch_team_solo_bptt(a, c, st);
   return e == hipSuccess && a.grad_A ? ring_launch_team_rows_ga(c.ga_part, a.grad_A, a.T, a.B, st) : e;
@@ -305,7 +309,7 @@ hipError_t ring_team_bptt(const RingBpttArgs& a, const float* Wo, const float* W
   const RingTeamPlan p = ring_team_plan(a.N, a.k, a.T, a.B, true, ga);
   if (!p.ok || !ws) return hipErrorInvalidValue;
   RingTeamArgs c;
-  hipError_t e = team_args(p, Wo, Wa, a.A, a.J0, a.J1, folded, a.N, a.k, a.T, a.B, cts, ws, c, st);
+  hipError_t e = team_args(p, Wo, Wa, a.A, a.J0, a.J1, folded, a.N, a.k, a.T, a.B, cts, first_look(p, true), ws, c, st);
   if (e != hipSuccess) return e;
   e = ga ? ring_launch_team_bptt_ga(a, c, p.shape, st) : ring_launch_team_bptt(a, c, p.shape, st);
   if (e == hipSuccess) e = ring_launch_team_solo_bptt(a, c, st);

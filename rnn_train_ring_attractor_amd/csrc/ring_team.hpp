@@ -526,13 +526,32 @@ __device__ __forceinline__ bool team_go(const char* lds, const LdsPlan& L) {
 // When a wave first looks for the next state where a team has one tile.  The state is there some 900 cycles behind the barrier that
 // ends the products (sums, activation, a store on its way), a look takes some 450, and one that comes back too early holds up the
 // next by as much: looked for before the products, or at once behind them, a step waited up to a whole look too long, the same in every
-// step.  So the first look goes out `look` times 64 cycles behind the barrier.  us a call, looking before the products, at once behind
-// the barrier, and 4, 8, 10 and 12 times 64 cycles later:
-//   rows kernels, T = 100: forward N = 256, B = 1, gelu 91.5  81.9  91.0  83.6  83.9  86.1  relu (there) 82.7  84.2  78.9  81.3  86.9
-//     forward N = 256, B = 128, gelu 103.6  94.9  102.7  95.6  94.4  93.5        training 260  235  251  248  234  233
-//   forward N = 360, 3 channels, B = 100, T = 75 97.3  96.1  92.5  90.9  95.5  98.3        training 262  229  229  221  229  235
-//   forward N = 1024, 2 channels, B = 64, T = 60 140.0  141.8  139.6  133.6  130.0  127.2
-//   forward N = 512, 2 channels, B = 64, T = 100 129.8  127.2  130.8  120.9  120.3  125.2      training 313  297  306  287  288  297
+// step.  So the first look goes out `look` times 64 cycles behind the barrier.  (The time does not fall and rise once with `look`: later
+// looks follow the first at fixed distances, and what counts is when the one that finds the state went out.)  us a call, gelu unless
+// said, looking before the products (teams of several tiles' way), at once behind the barrier, and 4, 8, 10 and 12 times 64 cycles later:
+//   rows kernels, forward, T = 100        0      4      8     10     12        BPTT     0      4      8     10     12
+//     N = 256, B = 1                     83.8   92.8   83.7   84.5   88.0             106.4  117.0  104.7  108.7  114.5
+//       relu                             82.5   80.1   77.9   82.0   86.9
+//     N = 256, B = 8                     89.2   95.7   88.3   89.0   89.5    (4 rows) 107.6  119.2  105.5  108.8  114.5
+//     N = 200, B = 8, tanh               84.4   90.0   81.5   83.2   86.9
+//     N = 256, B = 16                    94.2  101.8   94.3   93.4   92.3             127.1  139.5  124.3  124.8  125.1
+//       relu                             91.5   89.4   86.0   85.3   88.4             124.9  137.4  123.7  123.2  124.8
+//     N = 256, B = 128                   95.0  102.6   95.2   93.8   92.8             135.1  147.6  132.6  133.9  133.7
+//     N = 200, B = 128                   90.3   98.8   91.4   90.5   90.0             127.5  139.1  126.6  127.1  127.1
+//     N = 131, B = 384, tanh             91.3   99.3   89.1   88.9   90.5
+//     N = 200, B = 512, tanh (two tiles) 100.0  99.5   96.6   96.0  101.1  (400 rows) 139.3  147.0  136.8  137.7  137.2
+//   So 8, and 10 in a forward of more than eight rows.
+//   others, T = 60               before   0      4      8     10     12      BPTT before   0      4      8     10     12
+//     N = 300, B = 60             71.7   67.8   70.9   66.7   66.5   70.1           98.9   95.5   99.0   94.2   96.6   99.2
+//     N = 360, 3 channels, B = 60 80.4   77.7   81.0   75.5   75.4   78.7          109.7  107.6  112.0  106.3  107.8  111.5
+//     N = 512, B = 60             81.8   79.1   81.4   75.0   74.4   77.5          115.4  113.1  115.3  109.4  110.3  112.3
+//       tanh                      78.5   77.5   74.2   71.0   74.4   77.5
+//     N = 600, B = 60            101.4  100.9  102.9   95.7   94.0   93.8          132.2  130.6  132.8  123.4  123.5  123.9
+//     N = 800, 3 channels, B = 1 141.2  142.4  141.1  132.7  130.6  130.1          179.3  182.9  183.7  175.2  174.1  178.7
+//     N = 1024, B = 60           140.0  141.0  138.1  131.9  128.3  125.1          193.2  189.8  187.9  179.0  178.3  178.7
+//       tanh                     135.4  135.0  133.1  123.9  121.6  124.0
+//   So 8 up to two chunks a compute wave, past that 12 forward and 10 backward.  (N = 800, 3 channels: the late BPTT spills 92 registers
+//   a lane, the other 79, and is ahead all the same: B = 128 223.2, 221.3 with 12 and 219.2 with 10.)
 // With many matrices the compute waves are what is waited for, and they look before the products as with several tiles: forward
 // N = 512, 16 channels, B = 128, T = 40 108.6  108.1  109.7  111.5; N = 120, 12 channels, B = 30, T = 100 189  192  196  192.
 // (lds_mats: or TEAM_MORE.)  Kernels of their own: a second loop in the others', or a branch around their loads, costs those that look
