@@ -196,7 +196,7 @@ hipError_t ring_team_fill(void* ws, size_t xchg_bytes, size_t gather_bytes, hipS
 
 // RingTeamArgs::look (measured: team_look).
 static int first_look(const RingTeamPlan& p, bool bptt) {
-  if (p.nt != 1 || !team_may_look_late(p.shape.mr, p.shape.wk, p.shape.lds_mats)) return -1;
+  if (p.nt != 1 || !team_may_look_late(p.shape.kpw, p.shape.c16, p.shape.mr, p.shape.wk, p.shape.lds_mats)) return -1;
   return p.shape.kpw < 3 ? 8 : bptt ? 10 : 12;
 }
 

@@ -461,11 +461,10 @@ __device__ __forceinline__ void team_products(const TeamCompute<KPW, C16, MR, WK
   if constexpr (EX == TEAM_MORE) {
     // (gates are read a matrix ahead: forward N = 512, 16 channels, B = 256, T = 20 95.5 -> 93.2 us, N = 168, B = 223, T = 76 158.7 -> 152.3)
     float gn = gates[(MR - 1) * 16 + b];
-    if (last >= MR) fetch(MR);
     for (int m = MR; m <= last; ++m) {
       const float gm = gn;
       gn = gates[(m < c.k ? m : c.k - 1) * 16 + b];
-      lds_matrix(m, gm, m < last ? m + 1 : m);
+      lds_matrix(m, gm, 0);
     }
   } else if constexpr (EX > 0) {
     float g[EX];
@@ -556,7 +555,10 @@ __device__ __forceinline__ bool team_go(const char* lds, const LdsPlan& L) {
 // N = 512, 16 channels, B = 128, T = 40 108.6  108.1  109.7  111.5; N = 120, 12 channels, B = 30, T = 100 189  192  196  192.
 // (lds_mats: or TEAM_MORE.)  Kernels of their own: a second loop in the others', or a branch around their loads, costs those that look
 // early (forward N = 400, 9 channels, B = 200, T = 60 132 -> 137 us; training N = 1024, B = 512, T = 40 547 -> 840).
-__host__ __device__ constexpr bool team_may_look_late(int mr, int wk, int lds_mats) { return mr == 3 && wk == 8 && lds_mats <= 4; }
+// Four column tiles a member, and two where one fits the matrices as well, are only taken where teams have several tiles.
+__host__ __device__ constexpr bool team_may_look_late(int kpw, int c16, int mr, int wk, int lds_mats) {
+  return mr == 3 && wk == 8 && lds_mats <= 4 && (c16 == 1 || kpw >= 3 || (c16 == 2 && (kpw == 1 ? lds_mats <= 1 : lds_mats >= 3)));
+}
 __device__ __forceinline__ void team_look(int look) {
   for (int i = 0; i < look; ++i) __builtin_amdgcn_s_sleep(1);
 }
@@ -587,8 +589,8 @@ __device__ __forceinline__ void team_compute_loop(const RingTeamArgs& c, const L
   if (dead && lane == 0) *c.host_err = RING_CLUSTER_ERR_WAIT;
   opA.template issue<WK>(rsrc, tc, (unsigned)team * tile_bytes);
   // One item.  The operand of the next one is fetched meanwhile: with several tiles per team it usually is published
-  // already (its state was formed a round ago), with one tile this is the first poll for it.  Whether it was there is
-  // checked when it is used.
+  // already (its state was formed a round ago), with one tile and many matrices this is the first poll for it.  Whether it was there is
+  // checked when it is used.  (LATE: one tile, and the next item's operand is asked for at its start.)
   auto item = [&](TeamOperand<KPW>& op, TeamOperand<KPW>& nx) {
     float gate[MR];                  // (in LDS since the last barrier; read while the operand is on its way)
 #pragma unroll

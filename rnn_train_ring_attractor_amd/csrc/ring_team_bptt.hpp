@@ -251,7 +251,7 @@ hipError_t team_bptt_start(const RingBpttArgs& a, const RingTeamArgs& c, const R
 }
 #define RING_TEAM_RUN(KPW, C16, MR, WK, EX)                                                                           \
   do {                                                                                                                \
-    if constexpr (team_may_look_late(MR, WK, EX))                                                                     \
+    if constexpr (team_may_look_late(KPW, C16, MR, WK, EX))                                                           \
       if (c.look >= 0) return team_bptt_start<KPW, C16, MR, WK, EX, GA, true>(a, c, sh, st);                          \
     return team_bptt_start<KPW, C16, MR, WK, EX, GA, false>(a, c, sh, st);                                            \
   } while (0)

@@ -119,7 +119,7 @@ hipError_t team_fwd_start(const RingFwdArgs& a, const RingTeamArgs& c, const Rin
                          [&](dim3 g, dim3 b, unsigned lds) { RING_LAUNCH(kern, g, b, lds, st, a, c); });
 }
 #define RING_TEAM_ACT(KPW, C16, MR, WK, EX, ACT)                                                                    \
-  if constexpr (team_may_look_late(MR, WK, EX))                                                                     \
+  if constexpr (team_may_look_late(KPW, C16, MR, WK, EX))                                                           \
     if (c.look >= 0) return team_fwd_start<KPW, C16, MR, WK, EX, ACT, true>(a, c, sh, st);                          \
   return team_fwd_start<KPW, C16, MR, WK, EX, ACT, false>(a, c, sh, st)
 #define RING_TEAM_ACTS(KPW, C16, MR, WK, EX)                                  \
