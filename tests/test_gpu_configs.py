@@ -996,10 +996,38 @@ def test_short_weight_gradients_against_the_tiled_kernel_and_the_oracle(N, B, T,
     monkeypatch.setenv("RINGATTR_DW_SEGMENT", "0")            # the kernel that can be cut, uncut
     tiled = run()
     assert not tiled[2].startswith("ring_dw_direct_kernel<0,")
-    # the same bf16 products, summed in fp32 in another order: at most 37 * 70 of them, error about sqrt(2590) * 2^-24 of a typical sum
+    # the same bf16 products, summed in fp32 in another order: at most 51 * 64 of them, error about sqrt(3264) * 2^-24 = 3.4e-6 of a typical sum
     for got, want in zip(short[:2], tiled[:2]):
         assert O.max_rel_err(got, want) <= 1e-5
     ref, _ = O.forward_dense(p["A"], p["Wa"], -0.3 / N, 0.4, p["Wo"], p["r0"], 0.15, "tanh")
     g = O.backward_dense(p["G"], p["A"], p["Wa"], -0.3 / N, 0.4, p["Wo"], ref, p["r0"], 0.15, "tanh")
     for got, name in zip(short[:2], ("grad_Wo", "grad_Wa")):
         assert O.cosine(got, g[name]) >= GRAD_COS and O.max_rel_err(got, g[name]) <= GRAD_TOL, name
+
+
+# The pipeline of the kernel for short contractions: 9 to 15 chunks a wave, i.e. stages that are loaded again, gate buffers that are written
+# again, all remainders behind a trip of three; two to four matrices a launch, with the ungated one and without; numbers of batch tiles
+# that are neither one nor a multiple of the waves; both tile orders.
+@pytest.mark.parametrize("N,B,T,k", [(360, 100, 81, 2), (360, 100, 85, 3), (360, 100, 89, 6), (360, 100, 101, 7), (360, 40, 190, 1), (360, 72, 157, 4),
+                                     (200, 100, 181, 2)])
+def test_short_weight_gradients_over_many_chunks_a_wave(N, B, T, k, gpu_device, monkeypatch):
+    from rnn_train_ring_attractor_amd import ring_rnn_cuda_func, _lib
+    print(f"[case] short weight gradients, many chunks a wave N={N} B={B} T={T} k={k}", flush=True)
+    p = make_problem(96, B, T, k, N, action="dense")
+    Wa, Wo = _t(p["Wa"], gpu_device).requires_grad_(True), _t(p["Wo"], gpu_device).requires_grad_(True)
+    h = ring_rnn_cuda_func(_t(p["A"], gpu_device), Wa, -0.3 / N, 0.4, Wo, _t(p["r0"], gpu_device), 0.15, "tanh")
+    G = _t(p["G"], gpu_device)
+
+    def run():
+        grads = torch.autograd.grad(h, (Wo, Wa), G, retain_graph=True)
+        return [x.cpu().numpy() for x in grads], _lib.last_kernel_names()["dw"]
+
+    (short, name), (again, _) = run(), run()
+    assert name.startswith("ring_dw_direct_kernel<0,")
+    assert all(np.array_equal(a, b) for a, b in zip(short, again))
+    monkeypatch.setenv("RINGATTR_DW_SEGMENT", "0")            # the kernel that can be cut, uncut
+    tiled, name = run()
+    assert not name.startswith("ring_dw_direct_kernel<0,")
+    # the same chunks' products added up in fp32 in two orders: up to 637 additions, about sqrt(637) * 2^-24 = 1.5e-6 of a typical sum each
+    for got, want in zip(short, tiled):
+        assert O.max_rel_err(got, want) <= 1e-5
