@@ -576,7 +576,8 @@ def test_few_matrices_in_lds(B, k, N, gpu_device, teams, monkeypatch):
     assert O.max_rel_err(want["hist"][:, :9].cpu().numpy(), ref) <= TRAJ_TOL
 
 
-# Teams for the weight-resident widths: sixteen members of one column tile up to 256 rows, eight of two past that.
+# Teams for the weight-resident widths: members of one column tile while every batch tile finds room for a team of them, two past that:
+# 256 rows with a record, up to 384 without (five chunks are ten members).
 @pytest.mark.parametrize("N,T,act", [(256, 9, "gelu"), (200, 8, "relu"), (131, 5, "silu")])
 def test_rows_on_either_side_of_the_line_between_one_and_two_column_tiles(N, T, act, gpu_device, monkeypatch):
     from rnn_train_ring_attractor_amd import ring_rnn_cuda_func, _lib
@@ -604,3 +605,26 @@ def test_rows_on_either_side_of_the_line_between_one_and_two_column_tiles(N, T, 
         for other in (run(B, RINGATTR_TEAM="0"), run(B, RINGATTR_TEAM_GATHER_US="-1")):      # one workgroup a tile; teams that give up
             for got, want in zip(teams[:4], other[:4]):
                 assert torch.equal(got, want), (B, other[4])
+
+
+# Without a record a team has as many members as the ring has column tiles: ten up to N = 160, three teams an XCD, 384 rows; twelve up to
+# N = 192 and more up to 256, two teams an XCD, 256 rows.  With one always sixteen.
+@pytest.mark.parametrize("N,rows", [(131, 384), (160, 384), (161, 256), (256, 256)])
+def test_members_have_one_column_tile_as_far_as_there_is_room(N, rows, gpu_device, monkeypatch):
+    from rnn_train_ring_attractor_amd import ring_rnn_cuda_func, _lib
+    p = make_problem(32, 385, 4, 2, N)
+    t = lambda x: torch.as_tensor(x, dtype=torch.float32, device=gpu_device)
+    A, Wa, Wo, r0 = (t(p[n]) for n in ("A", "Wa", "Wo", "r0"))
+
+    def run(B, record):
+        a, r, wo = A[:B].clone(), r0[:B].clone(), Wo.clone().requires_grad_(record)
+        return ring_rnn_cuda_func(a, Wa, -1.0 / N, 0.5, wo, r, 0.15, "tanh").detach(), _lib.last_kernel_names()["fwd"]
+
+    for record, kernel, limit in ((False, "ring_team_rows_kernel", rows), (True, "ring_team_res256_fwd_kernel", 256)):
+        monkeypatch.delenv("RINGATTR_TEAM", raising=False)
+        (one, name_one), (two, name_two) = run(limit, record), run(limit + 1, record)
+        assert (name_one, name_two) == (kernel + "<2,1>", kernel + "<2,2>")
+        monkeypatch.setenv("RINGATTR_TEAM", "0")
+        whole, name = run(limit + 1, record)
+        assert not name.startswith("ring_team")
+        assert torch.equal(two, whole) and torch.equal(one, whole[:, :limit])
