@@ -293,7 +293,7 @@ hipError_t ring_team_fwd(const RingFwdArgs& a, const float* Wo, const float* Wa,
 hipError_t ring_team_bptt(const RingBpttArgs& a, const float* Wo, const float* Wa, bool folded, int cts, void* ws, hipStream_t st);
 // small batches of 128 < N <= 256 with two channels, in the weight-resident kernels' order (ring_team_rows.hip); record: with
 // a record, and the BPTT
-RingTeamPlan ring_team_rows_plan(int N, int k, int B, bool record);
+RingTeamPlan ring_team_rows_plan(int N, int k, int B, bool record, int launches = 1);   // beside launches - 1 others (sizes do not depend on it)
 bool ring_uses_team_rows(int N, int k, int B, bool record);
 size_t ring_team_rows_bytes(int N, int k, int B, bool record);
 size_t ring_team_rows_bptt_bytes(int N, int k, int T, int B, bool ga);

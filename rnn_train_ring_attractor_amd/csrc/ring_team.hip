@@ -263,9 +263,15 @@ hipError_t ring_team_fwd(const RingFwdArgs& a, const float* Wo, const float* Wa,
   return e == hipSuccess ? ring_launch_team_solo_fwd(a, c, st) : e;
 }
 
+// The split that leaves room for the launches of other streams that have not finished; under capture for one beside this one.
+static RingTeamPlan rows_plan_on(hipStream_t st, int N, int k, int B, bool record) {
+  const int others = ring_launch_guard().beside(st);
+  return ring_team_rows_plan(N, k, B, record, others < 0 ? 2 : others + 1);
+}
+
 hipError_t ring_team_rows(const RingFwdArgs& a, const float* Wo, const float* Wa, void* ws, hipStream_t st) {
   const bool record = a.dfrag != nullptr;
-  const RingTeamPlan p = ring_team_rows_plan(a.N, a.k, a.B, record);
+  const RingTeamPlan p = rows_plan_on(st, a.N, a.k, a.B, record);
   if (!p.ok || !ws || !a.hist || record != (a.rfrag != nullptr)) return hipErrorInvalidValue;
   RingTeamArgs c;
   hipError_t e = team_args(p, Wo, Wa, a.A, a.J0, a.J1, true, a.N, a.k, a.T, a.B, 16, a.B <= 8 ? 8 : 10, ws, c, st);
@@ -278,7 +284,7 @@ hipError_t ring_team_rows(const RingFwdArgs& a, const float* Wo, const float* Wa
 }
 
 hipError_t ring_team_rows_bptt(const RingBpttArgs& a, const float* Wo, const float* Wa, void* ws, hipStream_t st) {
-  const RingTeamPlan p = ring_team_rows_plan(a.N, a.k, a.B, true);
+  const RingTeamPlan p = rows_plan_on(st, a.N, a.k, a.B, true);
   if (!p.ok || !ws) return hipErrorInvalidValue;
   RingTeamArgs c;
   hipError_t e = team_args(p, Wo, Wa, a.A, a.J0, a.J1, true, a.N, a.k, a.T, a.B, 16, 8, ws, c, st);

@@ -18,9 +18,19 @@ namespace {
 constexpr int ROWS_CHUNKS = 8, ROWS_MATS = 3, ROWS_SLOTS = 8;
 // Two column tiles a member and a compute wave for the 24 products of each, or one column tile and a compute wave for the eight of
 // each matrix (the gates then follow in the auxiliary waves, in the same order): the chain a step waits for is 250 cycles shorter, but
-// takes twice the compute units and half as much more of the operand into each.  So one where sixteen members find room for every batch
-// tile (B <= 256).  us a call, T = 100, two and one, before team_look: forward N = 256, B = 16, relu 96.3 and 86.6, tanh 99.2 and 94.1,
-// B = 1, gelu 93.2 and 90.9, B = 256, gelu 105.2 and 103.8; training N = 200, B = 64, tanh 245 and 232.
+// takes twice the compute units and half as much more of the operand into each.  us a call, T = 100, two and one, before team_look:
+// forward N = 256, B = 16, relu 96.3 and 86.6, tanh 99.2 and 94.1, B = 1, gelu 93.2 and 90.9, B = 256, gelu 105.2 and 103.8; training
+// N = 200, B = 64, tanh 245 and 232.  So one where members of one find room for every batch tile (256 rows; 384 at N <= 160 without a
+// record, where a team has ten members instead of sixteen), beside as many launches as are under way on other streams: two tiles let
+// twice as many of them run at once.  Under capture, where nobody knows what a graph will be replayed beside, as if there were one
+// other.  us a call, gelu, T = 100, always one tile, always two, and so:
+//   eager, streams         1                    2                    3                    4
+//     N = 256, B = 1      83.6   94.0   83.6   45.5   50.3   45.4   70.0   34.1   34.2   74.9   33.0   32.6
+//     N = 256, B = 128    93.6  102.6   94.0   51.3   55.0   51.2  103.5   38.0   38.1  109.2   55.0   55.4
+//     N = 256, B = 200    95.5  103.2   95.9   93.8   56.1   55.9  105.6   52.4   52.3  110.7   50.7   50.9
+//   graphs, replayed on a stream each (B = 200: four that want all compute units starve each other until they give up)
+//     N = 256, B = 128   101.4  109.5  101.2   53.1   56.7   52.7   49.4   39.3   49.4   46.3   37.8   48.9
+//     N = 256, B = 200   103.5  111.3  110.9   96.8   57.2   57.2   99.0   75.0   75.1   2659   52.7   52.8
 template <int TILES>
 struct RowsSplit {
   static constexpr int SHARES = TILES == 1 ? ROWS_MATS : 1, WAVES = TILES * SHARES;     // shares of a column tile, compute waves
@@ -522,12 +532,12 @@ __global__ __launch_bounds__(256) void ring_team_res256_ga_reduce_kernel(const f
 }
 
 // record: with one, or a BPTT; then all 256 neurons have a member (the padding's part of the record is zero)
-RingTeamPlan ring_team_rows_plan(int N, int k, int B, bool record) {
+RingTeamPlan ring_team_rows_plan(int N, int k, int B, bool record, int launches) {
   RingTeamPlan p{};
   if (!ring_res256_applicable(N, k)) return p;
   p.KC = record ? ROWS_CHUNKS : (N + 31) / 32;
   p.nteams = (B + 15) / 16;
-  const int one = 2 * p.KC, tiles = p.nteams <= 8 * (32 / one) ? 1 : 2;
+  const int one = 2 * p.KC, tiles = p.nteams <= 8 * (32 / (launches * one)) ? 1 : 2;
   p.G = (one + tiles - 1) / tiles;
   p.nt = 1;
   p.slots = ROWS_SLOTS;

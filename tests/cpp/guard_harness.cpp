@@ -148,6 +148,45 @@ int main() {
     launch(g, 2, 31);
     expect(Fake::order.empty(), "a stream that is gone is forgotten");
   }
+  reset();
+  {
+    Guard g(32);
+    expect(g.beside(1) == 0, "nobody is beside the first launch");
+    launch(g, 1, 15);
+    expect(g.beside(1) == 0 && Fake::records == 0, "a stream is not beside itself");
+    expect(g.beside(2) == 1, "an unfinished launch of another stream is");
+    launch(g, 2, 7);
+    expect(g.beside(1) == 1 && g.beside(3) == 2, "streams are counted, not launches");
+    launch(g, 2, 15);
+    expect(g.beside(1) == 1 && g.beside(3) == 2, "however many units their launches hold");
+    Fake::finished[1] = 1;
+    expect(g.beside(3) == 1 && g.beside(2) == 0, "finished launches are not");
+    Fake::capture.insert(3);
+    const int n = Fake::records;
+    expect(g.beside(3) == -1 && Fake::records == n, "a capturing stream does not know");
+  }
+  reset();
+  {
+    Guard g(32);
+    launch(g, 1, 15);
+    launch(g, 1, 7);
+    launch(g, 1, 15);
+    expect(Fake::records == 0, "one stream records nothing, whatever its launches hold");
+  }
+  reset();
+  {
+    Guard g(32);
+    launch(g, 1, 15);
+    launch(g, 2, 15);
+    Fake::order.clear();
+    for (int i = 0; i < 3; ++i) launch(g, 1, 7), launch(g, 2, 7);
+    expect(Fake::order.empty(), "a narrow launch runs beside a wide one");
+    launch(g, 3, 7);
+    expect(waits(3, 1), "what is queued holds what its widest launch does");
+    Fake::finished[1] = Fake::finished[2] = 1;
+    launch(g, 4, 7);
+    expect(Fake::order.empty(), "until that one has finished");
+  }
   std::printf("guard ok: %d\n", checks);
   return 0;
 }

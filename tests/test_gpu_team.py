@@ -628,3 +628,64 @@ def test_members_have_one_column_tile_as_far_as_there_is_room(N, rows, gpu_devic
         whole, name = run(limit + 1, record)
         assert not name.startswith("ring_team")
         assert torch.equal(two, whole) and torch.equal(one, whole[:, :limit])
+
+
+# One column tile a member takes twice the compute units two do.  So only while the launches of other streams that have not finished leave
+# room for it (two side by side up to 128 rows), and under capture, where nobody knows what the graph will be replayed beside, as if there
+# were one other.  The same bits either way.
+@pytest.mark.parametrize("B", [40, 128, 129, 200])
+def test_members_have_two_column_tiles_beside_other_streams(B, gpu_device, monkeypatch):
+    from rnn_train_ring_attractor_amd import ring_rnn_cuda_func, rnn_cuda, _lib
+    monkeypatch.delenv("RINGATTR_TEAM", raising=False)
+    N, T = 256, 6
+    print(f"[case] rows kernels beside other streams B={B}", flush=True)
+    p = make_problem(47, B, T, 2, N)
+    t = lambda x: torch.as_tensor(x, dtype=torch.float32, device=gpu_device)
+    A, Wa, Wo, r0 = (t(p[n]) for n in ("A", "Wa", "Wo", "r0"))
+    long_A = torch.zeros(16, 10000, 2, device=gpu_device)
+    long_r = r0[:16].clone()
+
+    def infer():
+        with torch.no_grad():
+            return ring_rnn_cuda_func(A, Wa, -1.0 / N, 0.5, Wo, r0, 0.15, "gelu"), _lib.last_kernel_names()["fwd"][-4:]
+
+    def train():
+        wo = Wo.clone().requires_grad_(True)
+        h = ring_rnn_cuda_func(A, Wa, -1.0 / N, 0.5, wo, r0, 0.15, "gelu")
+        names = _lib.last_kernel_names()["fwd"][-4:]
+        h.backward(torch.ones_like(h))
+        return h.detach(), wo.grad, names, _lib.last_kernel_names()["bptt"]
+
+    def beside(streams, call):
+        torch.cuda.synchronize()
+        for s in streams:
+            with torch.cuda.stream(s), torch.no_grad():          # some eight milliseconds each
+                ring_rnn_cuda_func(long_A, Wa, -1.0 / N, 0.5, Wo, long_r, 0.15, "gelu")
+        out = call()
+        torch.cuda.synchronize()
+        return out
+
+    others = [torch.cuda.Stream(device=gpu_device) for _ in range(3)]
+    alone_i, alone_t = beside([], infer), beside([], train)
+    assert alone_i[1] == "1,1>" and alone_t[2] == "1,1>" and alone_t[3].endswith("<false,1>")
+    for n in (1, 2, 3):
+        one = n == 1 and B <= 128
+        got_i, got_t = beside(others[:n], infer), beside(others[:n], train)
+        assert got_i[1] == ("1,1>" if one else "1,2>") and got_t[2] == ("1,1>" if one else "1,2>")
+        assert got_t[3].endswith("<false,1>" if one else "<false,2>")
+        assert torch.equal(got_i[0], alone_i[0]) and torch.equal(got_t[0], alone_t[0]) and torch.equal(got_t[1], alone_t[1])
+    again = beside([], infer)
+    assert again[1] == "1,1>" and torch.equal(again[0], alone_i[0])
+
+    out = torch.empty_like(alone_i[0])
+    graph = torch.cuda.CUDAGraph()
+    torch.cuda.synchronize()
+    with torch.cuda.graph(graph):
+        rnn_cuda.fwd_cuda.fwd(A=A, Wa=Wa, J0=-1.0 / N, J1=0.5, Wo=Wo, r_init=r0, bump_history=out, alpha=0.15, activation_type=1)
+    assert _lib.last_kernel_names()["fwd"][-4:] == ("1,1>" if B <= 128 else "1,2>")
+    for _ in range(3):
+        out.fill_(float("nan"))
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, alone_i[0])
