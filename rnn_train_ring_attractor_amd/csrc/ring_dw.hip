@@ -42,7 +42,8 @@ struct DwStage {
 // The order of a chunk's instructions around its N matrix instructions.  A SIMD has one wave here, and what that wave issues in a row
 // (twelve LDS reads, the fifteen vector instructions of a gated fragment, five loads, the LDS stage) keeps its matrix pipe waiting: 1575
 // cycles a chunk for 768 of products.  So a matrix instruction is followed by at most one of READS LDS reads, WRITES LDS writes, LOADS
-// loads (behind the last uses of what they replace) and two vector instructions, which cost it nothing.  us of contraction, left to the
+// loads (behind the last uses of what they replace) and two vector instructions, which cost it nothing: 1345 cycles a chunk (N = 256,
+// 15360 chunks; vector beside matrix instructions in 66.8 instead of 28.6 million of 189 million matrix cycles).  us of contraction, left to the
 // compiler and so (same bits): N = 256, 15360 chunks 229 -> 194; N = 512, 12800 chunks 622 -> 517; N = 1024, 3840 chunks 690 -> 610.
 // By vector instructions behind each: N = 512 three 560, two and three in turn 543 to 552, two 521 to 530, one 615.
 template <int N, int READS, int WRITES, int LOADS, int I>
@@ -466,7 +467,8 @@ static hipError_t launch_group(const RingDwArgs& a, int mg, unsigned blocks, int
 // long walk they drift apart and every one fetches its operands from memory for itself: at N = 512, B = 8192 the
 // kernel reads 1.02 x its operands over 512 chunks per workgroup, 1.45 x over 2048 and 2.47 x over 8192.  A long
 // sequence is therefore cut into segments in time, one launch each (a launch boundary re-aligns the workgroups);
-// the launches after the first add to the partial sums.  RINGATTR_DW_SEGMENT overrides the length (0: no cut).
+// the launches after the first add to the partial sums.  RINGATTR_DW_SEGMENT overrides the length (0: no cut) and keeps every
+// contraction with the kernel that is cut (ring_dw_short_nz).
 static int dw_segment_chunks() {
   const char* e = getenv("RINGATTR_DW_SEGMENT");   // read at every call: tests switch it between calls
   return e ? atoi(e) : 640;
@@ -530,9 +532,10 @@ hipError_t ring_launch_dw_tiled(const RingDwArgs& a, int NC, hipStream_t st) {
 //     178 and 194; N = 256, 945 chunks 34 and 25; N = 360 (padded to 512 here), 1890 chunks 87 and 60
 //   three (two launches here): N = 256, 15360 chunks 289 and 212
 // No launch of dw_chunk_waves is cut in time, however long: the waves of its workgroups drift apart as the others do, and it is ahead all
-// the same where it is taken.  us of contraction, cut here and there: N = 360, two channels, 131072 chunks 4810 and 3320, three, 65536
-// chunks 4280 and 2020; N = 640, two, 65536 chunks 10270 and 5570; N = 512, three, 131072 chunks 9300 and 7690; N = 200, three 2380 and
-// 1560; N = 120, six 2970 and 1210.
+// the same where it is taken, by the products that padding and a last launch of one matrix cost the other.  us of contraction (GB
+// fetched), cut here and there: N = 360, two channels, 131072 chunks 4710 (9.5) and 3290 (10.4), three, 65536 chunks 4280 and 2020;
+// N = 640, two, 65536 chunks 10270 and 5570; N = 512, three, 131072 chunks 8630 (18.6) and 7150 (33.7); N = 200, three 2380 and 1560;
+// N = 120, six 2970 and 1210.
 // Returns the K splits of dw_chunk_waves, 0: not that kernel.
 int ring_dw_short_nz(int N, int NC, int k, int nbt, int T, int tiled_nz, int linear_tiles) {
   if (getenv("RINGATTR_DW_SEGMENT")) return 0;             // (asks for the kernel that is cut)

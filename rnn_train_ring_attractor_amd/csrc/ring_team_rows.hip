@@ -3,14 +3,16 @@
 // family's backward reads either one's record.
 //
 // Those kernels give one compute unit the whole ring, 24 products for each of its 16 column tiles, and B = 1 pays the same
-// step as B = 4096.  Here a member of a team has two column tiles and a compute wave the 24 products of one: it sums the
-// whole contraction in the resident kernel's order (forward: its K chunks first the even and then the odd ones; BPTT: one
-// after the other, the ungated sum starting from (1 - alpha) G), every matrix in an accumulator of its own, the gates
-// afterwards.  One batch tile per team, so up to 32 tiles.
-// us per call, T = 100, weight-resident kernels -> here, with two column tiles a member and before team_look.  With a record: N = 256, B = 128, gelu: forward 143 -> 117, BPTT
-// 138 -> 130; N = 200, B = 64: 156 -> 110 and 245 -> 120; N = 256, B = 128, relu, with the loss's gradient and dL/dA:
-// 165 -> 114 (its row sums by a pass of their own included) and 222 -> 149.  Without: N = 256, B = 1: 142 -> 99.
-// What bounds it is the hand-over's latency and the chain of 24 products (some 400 cycles).
+// step as B = 4096.  Here a member of a team has one column tile and a compute wave for the eight products of each matrix, or
+// two and one for all 24 of each (RowsSplit).  A wave sums the whole contraction in the resident kernel's order (forward: its
+// K chunks first the even and then the odd ones; BPTT: one after the other, the ungated sum starting from (1 - alpha) G), every
+// matrix in an accumulator of its own, the gates afterwards.  One batch tile per team, so up to 32 tiles.
+// us per call, T = 100, weight-resident kernels -> here with two column tiles and before team_look -> now with one.  With a record:
+// N = 256, B = 128, gelu: forward 143 -> 117 -> 100, BPTT 138 -> 130 -> 113; N = 200, B = 64: 156 -> 110 and 245 -> 120; N = 256,
+// B = 128, relu, with the loss's gradient and dL/dA: 165 -> 114 (its row sums by a pass of their own included) and 222 -> 149.
+// Without: N = 256, B = 1: 142 -> 99 -> 80.
+// What bounds it is the hand-over's latency, a chain of eight products (24 with two tiles, some 400 cycles) and the sums and the
+// activation behind a barrier, one after the other.
 #include "ring_team.hpp"
 
 namespace {
