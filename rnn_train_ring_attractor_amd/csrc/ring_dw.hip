@@ -525,7 +525,8 @@ hipError_t ring_launch_dw_tiled(const RingDwArgs& a, int NC, hipStream_t st) {
 // Held against 715 shapes, N = 70 to 2048, 1 to 16 channels, 5 to 65536 chunks: the kernel it takes is at most 13 % and 26 us slower
 // than the other where it is dw_chunk_waves (N = 200: one channel, 3840 chunks 51 against 45 us, five, 15360 chunks 359 against 340);
 // where it stays here some wide rings with many channels would gain from the other (N = 565, seven channels, 43095 chunks 20.8 against
-// 15.8 ms; N = 700, 16, 15360 chunks 15.9 against 13.8; most 0).  So long contractions of whole 128 x 128 blocks and those of one channel stay here; us, here and there:
+// 15.8 ms; N = 700, 16, 15360 chunks 15.9 against 13.8; most gain nothing).  So long contractions of whole 128 x 128 blocks and those of
+// one channel stay here; us, here and there:
 //   one channel: N = 512, 15360 chunks 444 and 629, 945 chunks 44 and 42; N = 1024, 3840 chunks 430 and 609; N = 360, 15360 chunks 440
 //     and 388
 //   two: N = 512, 65536 chunks 2480 and 2810; N = 1024, 3840 chunks 573 and 638; N = 256, 15360 chunks 181 and 214; N = 2048, 160 chunks
